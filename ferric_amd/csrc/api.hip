@@ -15,7 +15,7 @@ namespace {
 // object, so each device the library runs on holds its own copy (512 KiB) from load to process exit and no call has to
 // allocate. Host code never uses the array's name as an address: fhip_init asks the runtime for the device address of the
 // current device's copy and keeps it per device.
-constexpr size_t WEIGHT_SLACK = 256;   // readable bytes every weight has behind its last block
+using fhip::WEIGHT_SLACK;
 constexpr size_t NOALLOC_FLOATS = 131072;
 static __device__ __align__(256) float scratch[NOALLOC_FLOATS];
 constexpr int MAX_DEVICES = 64;
@@ -175,7 +175,7 @@ int lib_workspace(hipStream_t s, size_t need, void** out, const char* who) {
     size_t n = 1 << 20;
     while (n < need) n <<= 1;
     void* p = nullptr;
-    int rc = check_hip(hipMalloc(&p, n), "hipMalloc (library workspace)");
+    int rc = fhip::device_malloc(&p, n, "hipMalloc (library workspace)");
     if (rc) return rc;
     if (!e) { g_ws.push_back(StreamWs{s, nullptr, 0, {}}); e = &g_ws.back(); }
     if (e->cur) e->retired.push_back(e->cur);
@@ -327,9 +327,9 @@ int fhip_malloc(void** d_ptr, size_t nbytes) {
     *d_ptr = nullptr;
     // 256 bytes more than asked for: a weight wrapped at the end of such a buffer (fhip_weight_wrap_device) keeps the slack
     // behind its last block that fhip_weight_create gives its own allocations
-    return check_hip(hipMalloc(d_ptr, nbytes + WEIGHT_SLACK), "hipMalloc");
+    return fhip::pool_malloc(d_ptr, nbytes);
 }
-int fhip_free(void* d_ptr) { return d_ptr ? check_hip(hipFree(d_ptr), "hipFree") : FHIP_OK; }
+int fhip_free(void* d_ptr) { return d_ptr ? fhip::pool_free(d_ptr) : FHIP_OK; }
 int fhip_memcpy_h2d(void* d, const void* h, size_t n, void* s) {
     if (n == 0) return FHIP_OK;
     if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_memcpy_h2d: NULL pointer");
@@ -394,11 +394,16 @@ int fhip_graph_capture_begin(void* s) {
     int rc = need_init();
     if (rc) return rc;
     if (!s) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_begin: needs a stream from fhip_stream_create");
-    return check_hip(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    rc = check_hip(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    if (!rc) fhip::pool_capture_depth(1);
+    return rc;
 }
 int fhip_graph_capture_end(void* s, void** graph_exec) {
     if (!s || !graph_exec) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_end: NULL argument");
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)s, &st) != hipSuccess) (void)hipGetLastError();
     *graph_exec = nullptr;
+    if (st != hipStreamCaptureStatusNone) fhip::pool_capture_depth(-1);
     hipGraph_t g = nullptr;
     int rc = check_hip(hipStreamEndCapture((hipStream_t)s, &g), "hipStreamEndCapture");
     if (rc) return rc;
@@ -426,7 +431,7 @@ int fhip_weight_create(uint32_t ty, const uint8_t* h_raw, size_t nbytes, size_t 
     if (nbytes && !h_raw) return set_error(FHIP_ERR_ARG, "fhip_weight_create: NULL bytes");
     void* d = nullptr;
     // slack past the stream: a wide load that starts inside the last block may end behind it
-    if ((rc = check_hip(hipMalloc(&d, nbytes + WEIGHT_SLACK), "hipMalloc(weight)"))) return rc;
+    if ((rc = fhip::device_malloc(&d, nbytes + WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
     if (nbytes && (rc = check_hip(hipMemcpy(d, h_raw, nbytes, hipMemcpyHostToDevice), "hipMemcpy(weight)"))) { (void)hipFree(d); return rc; }
     if ((rc = check_hip(hipMemset((uint8_t*)d + nbytes, 0, WEIGHT_SLACK), "hipMemset(weight tail)"))) { (void)hipFree(d); return rc; }
     w.d_raw = (const uint8_t*)d;
@@ -450,7 +455,7 @@ int fhip_weight_create_parts(uint32_t ty, const uint8_t* const* h_parts, const s
     fhip_weight w;
     if ((rc = make_weight(ty, nbytes, rows, cols, w))) return rc;
     void* d = nullptr;
-    if ((rc = check_hip(hipMalloc(&d, nbytes + 256), "hipMalloc(weight)"))) return rc;
+    if ((rc = fhip::device_malloc(&d, nbytes + WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
     size_t at = 0;
     for (size_t i = 0; i < n_parts && !rc; i++) {
         if (part_bytes[i]) rc = check_hip(hipMemcpy((uint8_t*)d + at, h_parts[i], part_bytes[i], hipMemcpyHostToDevice), "hipMemcpy(weight)");
@@ -474,13 +479,17 @@ int fhip_weight_wrap_device(uint32_t ty, const uint8_t* d_raw, size_t nbytes, si
     if (nbytes && !d_raw) return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: NULL bytes");
     if (((uintptr_t)d_raw & 15) != 0) return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: bytes must be 16-byte aligned");
     if (nbytes) {   // the allocation has to reach WEIGHT_SLACK bytes past the last block, as the library's own weights do
-        hipDeviceptr_t base = nullptr;
-        size_t size = 0;
-        if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)d_raw) != hipSuccess) {
-            (void)hipGetLastError();
-            return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: not a device allocation");
+        uintptr_t start = 0, end = 0;
+        if (!fhip::pool_range(d_raw, &start, &end)) {
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)d_raw) != hipSuccess) {
+                (void)hipGetLastError();
+                return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: not a device allocation");
+            }
+            end = (uintptr_t)base + size;
         }
-        const uintptr_t end = (uintptr_t)base + size, need = (uintptr_t)d_raw + nbytes + WEIGHT_SLACK;
+        const uintptr_t need = (uintptr_t)d_raw + nbytes + WEIGHT_SLACK;
         if (need > end)
             return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: the allocation must extend %zu bytes past the weight's last block "
                              "(it ends %zu bytes behind it); buffers from fhip_malloc always do", WEIGHT_SLACK, (size_t)(end - ((uintptr_t)d_raw + nbytes)));
@@ -752,7 +761,10 @@ size_t fhip_workspace_bytes_coop(const fhip_weight* w, const fhip_weight* down, 
     return a > b ? a : b;
 }
 
-void fhip_workspace_release(void* stream) { release_workspace((hipStream_t)stream); }
+void fhip_workspace_release(void* stream) {
+    release_workspace((hipStream_t)stream);
+    fhip::pool_trim();
+}
 
 int fhip_gemm_q_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, void* stream) {
     int rc = need_init();

@@ -1,0 +1,189 @@
+// Device memory of the library (fhip_malloc / fhip_free): freed blocks are kept for the next allocation of their size class.
+//
+// hipFree waits for the device, and a block of more than a few megabytes is mapped and unmapped on every call. An operator that
+// allocates its output (and perhaps scratch) per call therefore paid a full drain of the queue per call, and the large ones the
+// page tables of hundreds of megabytes: a 2048-row feed-forward block of 1.1 ms of kernels took 10.6 ms, a 5 us mat-vec 20 us.
+//
+// What hipFree's wait gave callers is kept: a freed block may still be in use by work enqueued on any stream, this library's or
+// another's, so it is not handed out again before the device has been idle once since the free. Freed blocks collect on a `dirty`
+// list; when an allocation finds no clean block and its class already holds keep_blocks() dirty ones, one hipDeviceSynchronize
+// turns every dirty block of the device clean. Until then the class grows, so the wait comes once in up to 64 calls for small
+// blocks and once in two for the largest, instead of at every free.
+#include "common.hpp"
+
+#include <map>
+#include <mutex>
+#include <vector>
+
+namespace {
+
+constexpr size_t WEIGHT_SLACK = fhip::WEIGHT_SLACK;
+constexpr size_t POOL_BLOCK_MAX = (size_t)768 << 20;   // larger blocks (weights, mostly) are freed at once
+constexpr size_t POOL_CACHED_MAX = (size_t)2 << 30;    // cached bytes per device; beyond it the classes unused longest are freed
+constexpr int MAX_DEVICES = 64;
+
+struct Live { size_t asked, cls; int dev; };
+struct SizeClass {
+    std::vector<void*> clean, dirty;
+    uint64_t last_use = 0;
+};
+struct Pool {
+    std::mutex mu;
+    std::map<uintptr_t, Live> live;                    // by address: fhip_weight_wrap_device looks up ranges
+    std::map<size_t, SizeClass> classes[MAX_DEVICES];
+    size_t cached[MAX_DEVICES] = {};
+    uint64_t clock = 0;
+};
+// never destroyed: objects of a host program may be freed after static destructors have begun to run
+Pool& pool() { static Pool* p = new Pool(); return *p; }
+
+thread_local int t_capturing = 0;   // captures this thread has open: no wait and no free may happen inside one
+
+// Eight classes per power of two: at most an eighth of a block is not asked for.
+size_t size_class(size_t n) {
+    if (n <= 1024) return 1024;
+    const int top = 63 - __builtin_clzll((unsigned long long)n - 1);   // 2^top < n <= 2^(top + 1)
+    const size_t step = (size_t)1 << (top - 3);
+    return (n + step - 1) / step * step;
+}
+
+// Dirty blocks a class may hold before an allocation waits for the device: 128 MiB of them, 2 to 64. A wait costs about 10 us and
+// the gap behind it about as much, so a caller of microsecond kernels wants tens of calls between waits, while a class of
+// hundreds of megabytes belongs to calls of a millisecond.
+size_t keep_blocks(size_t cls) {
+    const size_t k = ((size_t)128 << 20) / cls;
+    return k < 2 ? 2 : (k > 64 ? 64 : k);
+}
+
+// Under p.mu: blocks out of the classes of `dev` that were unused longest, until at most `target` bytes stay cached.
+void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
+    auto& cs = p.classes[dev];
+    while (p.cached[dev] > target) {
+        SizeClass* oldest = nullptr;
+        size_t bytes = 0;
+        for (auto& c : cs)
+            if ((!c.second.clean.empty() || !c.second.dirty.empty()) && (!oldest || c.second.last_use < oldest->last_use)) {
+                oldest = &c.second;
+                bytes = c.first;
+            }
+        if (!oldest) return;
+        for (auto* list : {&oldest->clean, &oldest->dirty})
+            while (!list->empty() && p.cached[dev] > target) {
+                out.push_back(list->back());
+                list->pop_back();
+                p.cached[dev] -= bytes;
+            }
+    }
+}
+
+}  // namespace
+
+namespace fhip {
+
+void pool_capture_depth(int delta) { t_capturing += delta; }
+
+void pool_trim() {
+    Pool& p = pool();
+    std::vector<void*> out;
+    {
+        std::lock_guard<std::mutex> lock(p.mu);
+        for (int d = 0; d < MAX_DEVICES; d++) take_oldest(p, d, 0, out);
+    }
+    for (void* q : out) (void)hipFree(q);   // hipFree waits for whatever still uses the block
+}
+
+int device_malloc(void** out, size_t n, const char* what) {
+    hipError_t e = hipMalloc(out, n);
+    if (e == hipErrorOutOfMemory) {         // what the pool holds back may be what is missing
+        (void)hipGetLastError();
+        pool_trim();
+        e = hipMalloc(out, n);
+    }
+    return check_hip(e, what);
+}
+
+int pool_malloc(void** out, size_t nbytes) {
+    *out = nullptr;
+    const size_t need = nbytes + WEIGHT_SLACK, cls = size_class(need);
+    int dev = 0;
+    int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
+    if (rc) return rc;
+    if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) return device_malloc(out, need, "hipMalloc");
+    Pool& p = pool();
+    for (bool waited = false;;) {
+        std::vector<std::pair<size_t, std::vector<void*>>> dirty;
+        {
+            std::lock_guard<std::mutex> lock(p.mu);
+            SizeClass& c = p.classes[dev][cls];
+            c.last_use = ++p.clock;
+            if (!c.clean.empty()) {
+                *out = c.clean.back();
+                c.clean.pop_back();
+                p.cached[dev] -= cls;
+                p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
+                return FHIP_OK;
+            }
+            if (waited || t_capturing || c.dirty.size() < keep_blocks(cls)) break;
+            // every dirty block of the device leaves its list while the lock is given up for the wait: another thread that
+            // comes for one of them meanwhile makes a new block
+            for (auto& k : p.classes[dev])
+                if (!k.second.dirty.empty()) {
+                    dirty.emplace_back(k.first, std::vector<void*>());
+                    dirty.back().second.swap(k.second.dirty);
+                }
+        }
+        rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+        std::lock_guard<std::mutex> lock(p.mu);
+        for (auto& d : dirty) {
+            SizeClass& c = p.classes[dev][d.first];
+            auto& to = rc ? c.dirty : c.clean;
+            to.insert(to.end(), d.second.begin(), d.second.end());
+        }
+        if (rc) return rc;
+        waited = true;
+    }
+    if ((rc = device_malloc(out, cls, "hipMalloc"))) return rc;
+    std::lock_guard<std::mutex> lock(p.mu);
+    p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
+    return FHIP_OK;
+}
+
+int pool_free(void* ptr) {
+    Pool& p = pool();
+    std::vector<void*> over;
+    {
+        std::lock_guard<std::mutex> lock(p.mu);
+        auto it = p.live.find((uintptr_t)ptr);
+        if (it == p.live.end()) {
+            over.push_back(ptr);            // a block too large for the pool
+        } else {
+            const Live b = it->second;
+            p.live.erase(it);
+            SizeClass& c = p.classes[b.dev][b.cls];
+            c.dirty.push_back(ptr);
+            c.last_use = ++p.clock;
+            p.cached[b.dev] += b.cls;
+            if (!t_capturing && p.cached[b.dev] > POOL_CACHED_MAX) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
+        }
+    }
+    int rc = FHIP_OK;
+    for (void* q : over) {
+        const int r = check_hip(hipFree(q), "hipFree");
+        if (r) rc = r;
+    }
+    return rc;
+}
+
+bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end) {
+    Pool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mu);
+    auto it = p.live.upper_bound((uintptr_t)ptr);
+    if (it == p.live.begin()) return false;
+    --it;
+    if ((uintptr_t)ptr >= it->first + it->second.cls) return false;
+    *base = it->first;
+    *end = it->first + it->second.asked + WEIGHT_SLACK;
+    return true;
+}
+
+}  // namespace fhip

@@ -86,8 +86,6 @@ def rope(x, n_heads, head_dim, base, offset=0, positions=None, freq_scale=None, 
     _check(_lib.load().fhip_rope(x.buf.ptr, 0, t, n_heads, head_dim, n_rot, base, pos_t.buf.ptr if pos_t is not None else None, offset,
                                  freq_scale.buf.ptr if freq_scale is not None else None, int(interleaved), out.buf.ptr,
                                  _stream_handle(stream)))
-    if pos_t is not None and not isinstance(positions, Tensor):
-        _check(_lib.load().fhip_stream_sync(_stream_handle(stream)))     # the temporary position buffer is freed on return
     return out
 
 
@@ -122,15 +120,12 @@ def decode_attention(q, cache, n_heads, n_kv_heads, length=None, last_pos=None, 
     assert cache.width == n_kv_heads * dh
     lib = _lib.load()
     need = lib.fhip_decode_attention_ws_bytes(n_heads, n_kv_heads, dh, length)
-    own = None
     if need and ws is None:
-        own = ws = DeviceBuffer(need)
+        ws = DeviceBuffer(need)
     out = Tensor.empty((1, n_heads * dh))
     _check(lib.fhip_decode_attention_ex(q.buf.ptr, cache.k.buf.ptr, cache.v.buf.ptr, n_heads, n_kv_heads, dh, length,
                                         last_pos.buf.ptr if last_pos is not None else None, window, softcap,
                                         ws.ptr if ws is not None else None, out.buf.ptr, _stream_handle(stream)))
-    if own is not None:
-        _check(lib.fhip_stream_sync(_stream_handle(stream)))   # the scratch is freed on return
     return out
 
 
@@ -156,15 +151,12 @@ def decode_attention_kvq(q, kcache, vcache, n_heads, n_kv_heads, length=None, la
     assert 1 <= length <= min(kcache.cap, vcache.cap), f"decode_attention: length {length} outside the caches"
     lib = _lib.load()
     need = lib.fhip_decode_attention_ws_bytes(n_heads, n_kv_heads, dh, length)
-    own = None
     if need and ws is None:
-        own = ws = DeviceBuffer(need)
+        ws = DeviceBuffer(need)
     out = Tensor.empty((1, n_heads * dh))
     _check(lib.fhip_decode_attention_kvq(kcache.fmt, q.buf.ptr, kcache.codes.ptr, kcache.scales.ptr, vcache.codes.ptr, vcache.scales.ptr,
                                          n_heads, n_kv_heads, dh, length, last_pos.buf.ptr if last_pos is not None else None, window, softcap,
                                          ws.ptr if ws is not None else None, out.buf.ptr, _stream_handle(stream)))
-    if own is not None:
-        _check(lib.fhip_stream_sync(_stream_handle(stream)))   # the scratch is freed on return
     return out
 
 

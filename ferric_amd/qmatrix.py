@@ -13,6 +13,7 @@ Names, argument meaning and error behaviour follow the reference (paths relative
 the GPU through libferric_hip.so; nothing here does arithmetic on the host.
 """
 import ctypes as C
+import math
 
 import numpy as np
 
@@ -23,6 +24,9 @@ Q4_0, Q4_1, Q5_0, Q5_1, Q5_K = 2, 3, 6, 7, 13   # further formats: unpackers, ma
 IQ4_NL, IQ4_XS, MXFP4 = 20, 23, 39             # codebook / microscaling formats, same coverage
 BATCH_AUTO, BATCH_F32_MATVEC, BATCH_ORDERED = 0, 1, 2   # QMatrix.batch_policy
 F32, F16, BF16 = 0, 1, 30                      # unquantized tensor types: type_size and deq_raw only (lib.rs:473-475, 499-501)
+
+
+_F32 = np.dtype(np.float32)
 
 
 def _vp(a):
@@ -87,7 +91,8 @@ def _stream_handle(stream):
 
 
 class DeviceBuffer:
-    """nbytes of device memory, freed with the object."""
+    """nbytes of device memory, freed with the object. Work enqueued on any stream may still use it then: the library does not hand
+    the memory out again before the device has been idle once (fhip_free), so scratch can be dropped without a synchronisation."""
 
     def __init__(self, nbytes):
         lib = _lib.init()
@@ -108,7 +113,7 @@ class Tensor:
     """A contiguous row-major device tensor (f32 unless made with from_bf16_bits)."""
 
     def __init__(self, buf, shape, dtype=np.float32):
-        self.buf, self.shape, self.dtype = buf, tuple(int(s) for s in shape), np.dtype(dtype)
+        self.buf, self.shape, self.dtype = buf, tuple(map(int, shape)), _F32 if dtype is np.float32 else np.dtype(dtype)
 
     # -- construction / readback (crates/ferric-tensor/src/lib.rs: Tensor::from_vec, to_vec) --
     @staticmethod
@@ -134,11 +139,11 @@ class Tensor:
 
     @staticmethod
     def empty(shape, dtype=np.float32):
-        n = int(np.prod(shape))
-        return Tensor(DeviceBuffer(n * np.dtype(dtype).itemsize), shape, dtype)
+        n = math.prod(map(int, shape))
+        return Tensor(DeviceBuffer(n * (4 if dtype is np.float32 else np.dtype(dtype).itemsize)), shape, dtype)
 
     def numel(self):
-        return int(np.prod(self.shape))
+        return math.prod(self.shape)
 
     def to_vec(self, stream=None):
         """Device -> host; the only synchronising call (the reference's readback)."""
@@ -258,7 +263,6 @@ class Tensor:
         out = Tensor.empty((rows, down.rows()))
         _lib.check(_lib.load().fhip_ffn(gate_up.handle, down.handle, self.buf.ptr, rows, out.buf.ptr, ws.buf.ptr,
                                         _stream_handle(stream)))
-        out._keepalive = ws  # scratch must outlive the enqueued work
         return out
 
     # -- mixture-of-experts decode (dtype.rs:1582-1780) -----------------------------------------
@@ -328,10 +332,6 @@ class Tensor:
         ws = Tensor.empty((t * k, out_pe))
         _lib.check(_lib.load().fhip_matmul_q_id_wsum(w.handle, self.buf.ptr, t, selw.buf.ptr, k, out_pe, out.buf.ptr, ws.buf.ptr,
                                                      _stream_handle(stream)))
-        if stream is not None:
-            stream.synchronize()      # ws is freed on return
-        else:
-            _lib.check(_lib.load().fhip_stream_sync(None))
         return out
 
     def matmul_q6_k_id_wsum(self, w, selw, out_pe, stream=None):
@@ -371,10 +371,6 @@ class Tensor:
         out = Tensor.empty((rows, w.rows()))
         ws = DeviceBuffer(max(16, rows * inn * 2))
         _lib.check(_lib.load().fhip_matmul_q_coop(w.handle, self.buf.ptr, rows, out.buf.ptr, ws.ptr, _stream_handle(stream)))
-        if stream is not None:
-            stream.synchronize()      # ws is freed on return
-        else:
-            _lib.check(_lib.load().fhip_stream_sync(None))
         return out
 
     def matmul_q4_k_coop(self, w, stream=None):
@@ -402,10 +398,6 @@ class Tensor:
         ws = DeviceBuffer(max(256, lib.fhip_matmul_q_f16x2_ws_bytes(w.handle, rows)))
         out = Tensor.empty((rows, w.rows()))
         _lib.check(lib.fhip_matmul_q_f16x2(w.handle, self.buf.ptr, rows, out.buf.ptr, ws.ptr, _stream_handle(stream)))
-        if stream is not None:
-            stream.synchronize()      # ws is freed on return
-        else:
-            _lib.check(lib.fhip_stream_sync(None))
         return out
 
     def ffn_f16x2(self, gate_up, down, stream=None):
@@ -416,10 +408,6 @@ class Tensor:
         ws = DeviceBuffer(max(256, lib.fhip_ffn_f16x2_ws_bytes(gate_up.handle, down.handle, rows)))
         out = Tensor.empty((rows, down.rows()))
         _lib.check(lib.fhip_ffn_f16x2(gate_up.handle, down.handle, self.buf.ptr, rows, out.buf.ptr, ws.ptr, _stream_handle(stream)))
-        if stream is not None:
-            stream.synchronize()      # ws is freed on return
-        else:
-            _lib.check(lib.fhip_stream_sync(None))
         return out
 
     def ffn_coop(self, gate_up, down, stream=None):
@@ -430,10 +418,6 @@ class Tensor:
         ws = DeviceBuffer(max(256, lib.fhip_ffn_coop_ws_bytes(gate_up.handle, down.handle, rows)))
         out = Tensor.empty((rows, down.rows()))
         _lib.check(lib.fhip_ffn_coop(gate_up.handle, down.handle, self.buf.ptr, rows, out.buf.ptr, ws.ptr, _stream_handle(stream)))
-        if stream is not None:
-            stream.synchronize()      # ws is freed on return
-        else:
-            _lib.check(lib.fhip_stream_sync(None))
         return out
 
     def gemm_q_bf16(self, w, stream=None):
@@ -459,6 +443,8 @@ class QMatrix:
         rc = _lib.load().fhip_block_bytes(ggml_type, C.byref(v), C.byref(b))
         return (v.value, b.value) if rc == _lib.OK else None
 
+        lib = _lib.load()
+        self._rows, self._cols = lib.fhip_weight_rows(handle), lib.fhip_weight_cols(handle)    # fixed when the handle is made
     @staticmethod
     def from_bytes(data, ggml_type, rows, cols):
         """dtype.rs:893. Unknown type -> ValueError; cols not a block multiple or a wrong byte
@@ -492,10 +478,10 @@ class QMatrix:
         return QMatrix(h, ggml_type, keepalive=buf)
 
     def rows(self):
-        return _lib.load().fhip_weight_rows(self.handle)
+        return self._rows
 
     def cols(self):
-        return _lib.load().fhip_weight_cols(self.handle)
+        return self._cols
 
     def nbytes(self):
         return _lib.load().fhip_weight_nbytes(self.handle)

@@ -84,6 +84,9 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
 /* ---- device memory, streams, events (plumbing the binding needs to own tensors) ------------- */
 /* These stand where the reference's Tensor creates/reads wgpu buffers
  * (crates/ferric-tensor/src/lib.rs:1481 empty(), :141 to_vec(), :1816 readback). */
+/* Freed blocks are kept (up to 2 GiB a device, none above 768 MiB; fhip_workspace_release gives them back, as does an allocation
+ * that finds no memory) for later fhip_malloc calls. A block may be freed while work that uses it is still enqueued, on any stream:
+ * it is not handed out again before the device has been idle once since the free. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
 int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream); /* async on stream */
@@ -417,7 +420,7 @@ int fhip_batch_policy(int policy);
 
 /* The library's workspace of a stream (NULL: the default stream): device memory the batched paths of fhip_matmul_q,
  * fhip_matmul_q_swiglu and fhip_ffn use for prepared activations and intermediates. It is allocated on first need, only
- * grows (to a power of two), is shared by the calls enqueued on that stream, and is freed by fhip_workspace_release or
+ * grows (to a power of two), is shared by the calls enqueued on that stream, and is freed by fhip_workspace_release (with the blocks fhip_free has kept) or
  * fhip_stream_destroy (both wait for the stream first). fhip_workspace_bytes: what a call with these weights (down may be
  * NULL) and rows_x rows needs at most, 0 when it takes the mat-vec kernel. fhip_workspace_reserve: grow it to nbytes now,
  * e.g. before a graph capture, during which it cannot grow. A buffer that was outgrown stays allocated until the release,
