@@ -21,6 +21,7 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
 UNITS = {
     "api.hip": [],
     "memory.hip": [],
+    "transfer.hip": [],
     "dequant.hip": ["-ffp-contract=off"],
     "kvquant.hip": ["-ffp-contract=off"],       # the reference multiplies, then adds: no fused multiply-add
     "gemv.hip": ["-DFHIP_GEMV_PLANES=2"],

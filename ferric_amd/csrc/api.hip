@@ -333,14 +333,12 @@ int fhip_free(void* d_ptr) { return d_ptr ? fhip::pool_free(d_ptr) : FHIP_OK; }
 int fhip_memcpy_h2d(void* d, const void* h, size_t n, void* s) {
     if (n == 0) return FHIP_OK;
     if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_memcpy_h2d: NULL pointer");
-    return check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, (hipStream_t)s), "hipMemcpyAsync H2D");
+    return fhip::copy_h2d(d, h, n, (hipStream_t)s);
 }
 int fhip_memcpy_d2h(void* h, const void* d, size_t n, void* s) {
     if (n == 0) return FHIP_OK;
     if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_memcpy_d2h: NULL pointer");
-    int rc = check_hip(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, (hipStream_t)s), "hipMemcpyAsync D2H");
-    if (rc) return rc;
-    return check_hip(hipStreamSynchronize((hipStream_t)s), "hipStreamSynchronize");
+    return fhip::copy_d2h(h, d, n, (hipStream_t)s);
 }
 int fhip_memcpy_d2d(void* dst, const void* src, size_t n, void* s) {
     if (n == 0) return FHIP_OK;
@@ -400,12 +398,12 @@ int fhip_graph_capture_begin(void* s) {
 }
 int fhip_graph_capture_end(void* s, void** graph_exec) {
     if (!s || !graph_exec) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_end: NULL argument");
+    *graph_exec = nullptr;
+    hipGraph_t g = nullptr;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing((hipStream_t)s, &st) != hipSuccess) (void)hipGetLastError();
-    *graph_exec = nullptr;
-    if (st != hipStreamCaptureStatusNone) fhip::pool_capture_depth(-1);
-    hipGraph_t g = nullptr;
     int rc = check_hip(hipStreamEndCapture((hipStream_t)s, &g), "hipStreamEndCapture");
+    if (st != hipStreamCaptureStatusNone) fhip::pool_capture_depth(-1);
     if (rc) return rc;
     hipGraphExec_t ge = nullptr;
     rc = check_hip(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0), "hipGraphInstantiate");
@@ -563,17 +561,7 @@ int fhip_deq_raw(const uint8_t* h_raw, size_t nbytes, size_t n, uint32_t ty, flo
     // pushes whole blocks only and so returns a shorter vector (lib.rs:609-614).
     size_t produced = ty == FHIP_Q8_0 ? nb * vals : n;
     if (n_written) *n_written = produced;
-    if (nb) {
-        void *d_in = nullptr, *d_out = nullptr;
-        if ((rc = check_hip(hipMalloc(&d_in, nb * bytes), "hipMalloc"))) return rc;
-        if ((rc = check_hip(hipMalloc(&d_out, nb * vals * sizeof(float)), "hipMalloc"))) { (void)hipFree(d_in); return rc; }
-        rc = check_hip(hipMemcpy(d_in, h_raw, nb * bytes, hipMemcpyHostToDevice), "hipMemcpy H2D");
-        if (!rc) rc = fhip::launch_dequant(ty, (const uint8_t*)d_in, nb, (float*)d_out, nullptr);
-        if (!rc) rc = check_hip(hipMemcpy(h_out, d_out, nb * vals * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy D2H");
-        (void)hipFree(d_in);
-        (void)hipFree(d_out);
-        if (rc) return rc;
-    }
+    if (nb && (rc = fhip::dequant_host(ty, h_raw, nb, vals, bytes, h_out))) return rc;
     for (size_t i = nb * vals; i < produced; i++) h_out[i] = 0.0f;
     return FHIP_OK;
 }

@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from .qmatrix import DeviceBuffer, Graph, Tensor, _stream_handle, _vp
+from .qmatrix import DeviceBuffer, Graph, Tensor, _stream_handle, _upload
 
 
 def _check(rc):
@@ -22,8 +22,8 @@ def _check(rc):
 def _u32_tensor(values):
     a = np.ascontiguousarray(values, dtype=np.uint32)
     t = Tensor(DeviceBuffer(max(a.nbytes, 4)), a.shape, np.uint32)
-    _check(_lib.load().fhip_memcpy_h2d(t.buf.ptr, _vp(a), a.nbytes, None))
-    _check(_lib.load().fhip_stream_sync(None))
+    _upload(t.buf, a)
+    _check(_lib.load().fhip_stream_sync(None))     # the words are read on streams that do not wait for this one
     return t
 
 
@@ -255,8 +255,7 @@ class Qwen3Decoder:
     # -- state ------------------------------------------------------------------------------------
     def set_pos(self, pos):
         a = np.array([pos], np.uint32)
-        _check(_lib.load().fhip_memcpy_h2d(self.pos.buf.ptr, _vp(a), 4, _stream_handle(self.stream)))
-        _check(_lib.load().fhip_stream_sync(_stream_handle(self.stream)))
+        _upload(self.pos.buf, a, self.stream)
         for c in self._all_caches():
             c.len = pos
 
@@ -266,8 +265,7 @@ class Qwen3Decoder:
     def set_input(self, x_host):
         a = np.ascontiguousarray(x_host, dtype=np.float32).reshape(-1)
         assert a.size == self.cfg.d_model
-        _check(_lib.load().fhip_memcpy_h2d(self.xa.buf.ptr, _vp(a), a.nbytes, _stream_handle(self.stream)))
-        _check(_lib.load().fhip_stream_sync(_stream_handle(self.stream)))
+        _upload(self.xa.buf, a, self.stream)
 
     # -- one step ---------------------------------------------------------------------------------
     def _norm_matmul(self, w, cur, alt, resid, norm_w, y, swiglu):
@@ -364,8 +362,9 @@ class Qwen3Decoder:
         pos0 = self._all_caches()[0].len
         assert pos0 + t <= self.max_len, f"prefill: {pos0} + {t} rows exceed the capacity {self.max_len}"
         E = Tensor.empty
-        X = Tensor.from_vec(x, x.shape, self.stream)
-        positions = _u32_tensor(np.arange(pos0, pos0 + t))
+        X, positions = E(x.shape), E((t,), np.uint32)
+        _upload(X.buf, x, self.stream)
+        _upload(positions.buf, np.arange(pos0, pos0 + t, dtype=np.uint32), self.stream)
         h, qkv, q, att = E((t, c.d_model)), E((t, self.q_out + 2 * self.kv_out)), E((t, self.q_out)), E((t, self.q_out))
         o, x1, y = E((t, c.d_model)), E((t, c.d_model)), E((t, c.d_model))
         normed = E((t, c.d_model)) if self.on is not None else None                   # a post-normed branch output

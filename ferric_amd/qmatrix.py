@@ -90,6 +90,17 @@ def _stream_handle(stream):
     return stream.handle if stream is not None else None
 
 
+H2D_STAGED = 640 << 10      # fhip_memcpy_h2d: a source of up to this many bytes has been read when the call returns
+
+
+def _upload(buf, a, stream=None):
+    """A contiguous host array into a DeviceBuffer, in stream order; the array may go away afterwards."""
+    lib, s = _lib.load(), _stream_handle(stream)
+    _lib.check(lib.fhip_memcpy_h2d(buf.ptr, a.ctypes.data, a.nbytes, s))
+    if a.nbytes > H2D_STAGED:
+        _lib.check(lib.fhip_stream_sync(s))
+
+
 class DeviceBuffer:
     """nbytes of device memory, freed with the object. Work enqueued on any stream may still use it then: the library does not hand
     the memory out again before the device has been idle once (fhip_free), so scratch can be dropped without a synchronisation."""
@@ -121,11 +132,8 @@ class Tensor:
         a = np.ascontiguousarray(data, dtype=np.float32)
         assert a.size == int(np.prod(shape)), "from_vec: data does not match shape"
         t = Tensor(DeviceBuffer(a.nbytes), shape)
-        _lib.check(_lib.load().fhip_memcpy_h2d(t.buf.ptr, _vp(a), a.nbytes, _stream_handle(stream)))
-        if stream is None:
-            _lib.check(_lib.load().fhip_stream_sync(None))
-        else:
-            stream.synchronize()  # the host array may go away
+        _upload(t.buf, a, stream)
+        _lib.check(_lib.load().fhip_stream_sync(_stream_handle(stream)))    # a new tensor may be used on any stream
         return t
 
     @staticmethod
@@ -133,7 +141,7 @@ class Tensor:
         a = np.ascontiguousarray(bits, dtype=np.uint16)
         assert a.size == int(np.prod(shape))
         t = Tensor(DeviceBuffer(a.nbytes), shape, np.uint16)
-        _lib.check(_lib.load().fhip_memcpy_h2d(t.buf.ptr, _vp(a), a.nbytes, None))
+        _upload(t.buf, a)
         _lib.check(_lib.load().fhip_stream_sync(None))
         return t
 
@@ -148,7 +156,7 @@ class Tensor:
     def to_vec(self, stream=None):
         """Device -> host; the only synchronising call (the reference's readback)."""
         out = np.empty(self.numel(), dtype=self.dtype)
-        _lib.check(_lib.load().fhip_memcpy_d2h(_vp(out), self.buf.ptr, out.nbytes, _stream_handle(stream)))
+        _lib.check(_lib.load().fhip_memcpy_d2h(out.ctypes.data, self.buf.ptr, out.nbytes, _stream_handle(stream)))
         return out
 
     def cat(self, other, dim, stream=None):
@@ -435,6 +443,8 @@ class QMatrix:
 
     def __init__(self, handle, ggml_type, keepalive=None):
         self.handle, self.ggml_type, self._keepalive = handle, ggml_type, keepalive
+        lib = _lib.load()
+        self._rows, self._cols = lib.fhip_weight_rows(handle), lib.fhip_weight_cols(handle)    # fixed when the handle is made
 
     @staticmethod
     def block_bytes(ggml_type):
@@ -443,8 +453,6 @@ class QMatrix:
         rc = _lib.load().fhip_block_bytes(ggml_type, C.byref(v), C.byref(b))
         return (v.value, b.value) if rc == _lib.OK else None
 
-        lib = _lib.load()
-        self._rows, self._cols = lib.fhip_weight_rows(handle), lib.fhip_weight_cols(handle)    # fixed when the handle is made
     @staticmethod
     def from_bytes(data, ggml_type, rows, cols):
         """dtype.rs:893. Unknown type -> ValueError; cols not a block multiple or a wrong byte

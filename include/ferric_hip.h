@@ -89,7 +89,8 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
  * it is not handed out again before the device has been idle once since the free. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
-int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream); /* async on stream */
+/* async on stream; a source of up to 640 KiB has been read when the call returns (not in a stream capture) */
+int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream);
 int fhip_memcpy_d2h(void* h_dst, const void* d_src, size_t nbytes, void* stream); /* synchronises stream before returning */
 int fhip_memcpy_d2d(void* d_dst, const void* d_src, size_t nbytes, void* stream);
 /* `height` rows of `width` bytes between two pitched device arrays, async on stream (what Tensor::cat along the last
