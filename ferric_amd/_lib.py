@@ -185,3 +185,20 @@ def init(device=0):
         check(lib.fhip_init(device))
         _inited = True
     return lib
+
+
+def _host_first_use():
+    init()
+    _host.bind(SO_PATH)
+
+
+try:
+    from ferric_amd import _host        # the device memory object, an extension module built with the library
+    _host.setup(_host_first_use, check)
+    DeviceBuffer, matmul_q = _host.DeviceBuffer, _host.matmul_q
+except (ImportError, AttributeError) as _e:      # not built, or built from older source
+    _why = str(_e)
+
+    class DeviceBuffer:
+        def __init__(self, nbytes):
+            raise ImportError(f"ferric_amd._host is missing: build it with `python -m ferric_amd.build` ({_why})")

@@ -4,16 +4,20 @@
 
 Every translation unit is compiled for gfx950 with packed-FP32 instruction selection switched
 off; dequant.hip and kvquant.hip additionally with -ffp-contract=off, because their outputs
-must match the reference's separately-rounded f32 arithmetic bit for bit.
+must match the reference's separately-rounded f32 arithmetic bit for bit. The Python side's device memory object
+(csrc/host_py.cpp) is an extension module of its own, built by the host compiler.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libferric_hip.so")
+HOST_OUT = os.path.join(HERE, "_host" + sysconfig.get_config_var("EXT_SUFFIX"))
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
@@ -53,6 +57,13 @@ def _compile(name, flags, objdir, verbose):
     return obj
 
 
+def _build_host():
+    cmd = [CXX, "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "host_py.cpp"), "-o", HOST_OUT, "-ldl"]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on host_py.cpp:\n" + r.stdout)
+
+
 def build(verbose=False):
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
@@ -62,6 +73,7 @@ def build(verbose=False):
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout)
+    _build_host()
     return OUT
 
 

@@ -1,6 +1,6 @@
 // The extern "C" surface of libferric_hip (declared in include/ferric_hip.h): argument checks with
 // the reference's error behaviour, weight handles, and thin dispatch into the kernel launchers.
-#include "common.hpp"
+#include "hostmem.hpp"
 
 #include <stdarg.h>
 #include <stdio.h>

@@ -71,21 +71,6 @@ int check_hip(hipError_t e, const char* what);
 int device_cus();
 size_t device_lds_bytes();  // LDS one workgroup may use
 
-// memory.hip: the library's device memory
-constexpr size_t WEIGHT_SLACK = 256;   // readable bytes every weight and every block of fhip_malloc has behind its last byte
-int pool_malloc(void** out, size_t nbytes);
-int pool_free(void* ptr);
-void pool_trim();                      // gives every cached block back
-void pool_capture_depth(int delta);    // the calling thread opens (+1) or ends (-1) a stream capture
-bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the live block of pool_malloc that ptr lies in, as far as it was asked for
-int device_malloc(void** out, size_t n, const char* what);           // hipMalloc; with no memory left, once more after pool_trim
-
-// transfer.hip: copies through pinned memory of the library's own; both directions and the host-to-host unpackers
-constexpr size_t H2D_STAGED = (size_t)640 << 10;   // up to here copy_h2d has read its source when it returns
-int copy_h2d(void* d, const void* h, size_t n, hipStream_t s);
-int copy_d2h(void* h, const void* d, size_t n, hipStream_t s);   // synchronises
-int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nblocks, size_t block_values, size_t block_bytes, float* h_out);   // synchronises
-
 // dequant.hip
 int launch_f16_to_f32(const uint16_t* d_bits, size_t n, float* d_out, hipStream_t s);
 int launch_bf16_to_f32(const uint16_t* d_bits, size_t n, float* d_out, hipStream_t s);

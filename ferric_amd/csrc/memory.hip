@@ -8,9 +8,11 @@
 // another's, so it is not handed out again before the device has been idle once since the free. Freed blocks collect on a `dirty`
 // list; when an allocation finds no clean block and its class already holds keep_blocks() dirty ones, one hipDeviceSynchronize
 // turns every dirty block of the device clean. Until then the class grows, so the wait comes once in up to 64 calls for small
-// blocks and once in two for the largest, instead of at every free.
-#include "common.hpp"
+// blocks and once in two for the largest, instead of at every free. A class of large blocks whose last free lies a millisecond back
+// is drained at once instead of grown: the queue has most likely run empty since, and a new block would have to be mapped.
+#include "hostmem.hpp"
 
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -20,12 +22,14 @@ namespace {
 constexpr size_t WEIGHT_SLACK = fhip::WEIGHT_SLACK;
 constexpr size_t POOL_BLOCK_MAX = (size_t)768 << 20;   // larger blocks (weights, mostly) are freed at once
 constexpr size_t POOL_CACHED_MAX = (size_t)2 << 30;    // cached bytes per device; beyond it the classes unused longest are freed
+constexpr size_t LARGE = (size_t)1 << 20;              // blocks whose mapping costs more than a wait for an idle device
 constexpr int MAX_DEVICES = 64;
 
 struct Live { size_t asked, cls; int dev; };
 struct SizeClass {
     std::vector<void*> clean, dirty;
     uint64_t last_use = 0;
+    std::chrono::steady_clock::time_point last_free;
 };
 struct Pool {
     std::mutex mu;
@@ -123,7 +127,9 @@ int pool_malloc(void** out, size_t nbytes) {
                 p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
                 return FHIP_OK;
             }
-            if (waited || t_capturing || c.dirty.size() < keep_blocks(cls)) break;
+            if (waited || t_capturing || c.dirty.empty()) break;
+            if (c.dirty.size() < keep_blocks(cls) &&
+                (cls < LARGE || std::chrono::steady_clock::now() - c.last_free < std::chrono::milliseconds(1))) break;
             // every dirty block of the device leaves its list while the lock is given up for the wait: another thread that
             // comes for one of them meanwhile makes a new block
             for (auto& k : p.classes[dev])
@@ -162,6 +168,7 @@ int pool_free(void* ptr) {
             SizeClass& c = p.classes[b.dev][b.cls];
             c.dirty.push_back(ptr);
             c.last_use = ++p.clock;
+            if (b.cls >= LARGE) c.last_free = std::chrono::steady_clock::now();
             p.cached[b.dev] += b.cls;
             if (!t_capturing && p.cached[b.dev] > POOL_CACHED_MAX) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
         }

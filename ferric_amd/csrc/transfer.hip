@@ -8,7 +8,7 @@
 //   to the host     one kernel and one wait; more than a slot is cut into chunks, each copied out of its slot by a worker thread
 //                   while the next ones cross the bus (page faults of the destination included, which is why there are several)
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms.
-#include "common.hpp"
+#include "hostmem.hpp"
 
 #include <string.h>
 

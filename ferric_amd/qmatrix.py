@@ -18,6 +18,7 @@ import math
 import numpy as np
 
 from . import _lib
+from ._lib import DeviceBuffer
 
 Q8_0, Q4_K, Q6_K = 8, 12, 14
 Q4_0, Q4_1, Q5_0, Q5_1, Q5_K = 2, 3, 6, 7, 13   # further formats: unpackers, mat-vec / small batch, "_id" variants
@@ -27,6 +28,7 @@ F32, F16, BF16 = 0, 1, 30                      # unquantized tensor types: type_
 
 
 _F32 = np.dtype(np.float32)
+_new, _prod = object.__new__, math.prod
 
 
 def _vp(a):
@@ -101,25 +103,6 @@ def _upload(buf, a, stream=None):
         _lib.check(lib.fhip_stream_sync(s))
 
 
-class DeviceBuffer:
-    """nbytes of device memory, freed with the object. Work enqueued on any stream may still use it then: the library does not hand
-    the memory out again before the device has been idle once (fhip_free), so scratch can be dropped without a synchronisation."""
-
-    def __init__(self, nbytes):
-        lib = _lib.init()
-        p = C.c_void_p()
-        _lib.check(lib.fhip_malloc(C.byref(p), nbytes))
-        self.ptr, self.nbytes = p, nbytes
-
-    def __del__(self):
-        try:
-            if self.ptr:
-                _lib.load().fhip_free(self.ptr)
-                self.ptr = None
-        except Exception:
-            pass
-
-
 class Tensor:
     """A contiguous row-major device tensor (f32 unless made with from_bf16_bits)."""
 
@@ -146,12 +129,15 @@ class Tensor:
         return t
 
     @staticmethod
-    def empty(shape, dtype=np.float32):
-        n = math.prod(map(int, shape))
-        return Tensor(DeviceBuffer(n * (4 if dtype is np.float32 else np.dtype(dtype).itemsize)), shape, dtype)
+    def empty(shape, dtype=_F32):
+        t = _new(Tensor)
+        t.shape = shape = tuple(map(int, shape))
+        t.dtype = dtype = dtype if dtype is _F32 else np.dtype(dtype)
+        t.buf = DeviceBuffer(_prod(shape) * (4 if dtype is _F32 else dtype.itemsize))
+        return t
 
     def numel(self):
-        return math.prod(self.shape)
+        return _prod(self.shape)
 
     def to_vec(self, stream=None):
         """Device -> host; the only synchronising call (the reference's readback)."""
@@ -190,10 +176,11 @@ class Tensor:
     def matmul_q(self, w, stream=None):
         """y = x . W^T for a packed weight of any supported format -- dtype.rs:935."""
         rows, inn = self._rows_inner()
-        assert inn == w.cols(), f"inner dim mismatch: x[..,{inn}] vs W[..,{w.cols()}]"
-        out = Tensor.empty((rows, w.rows()))
-        _lib.check(_lib.load().fhip_matmul_q(w.handle, self.buf.ptr, rows, out.buf.ptr, _stream_handle(stream)))
-        return out
+        assert inn == w._cols, f"inner dim mismatch: x[..,{inn}] vs W[..,{w._cols}]"
+        y = _new(Tensor)
+        y.shape, y.dtype = (rows, w._rows), _F32
+        y.buf = _lib.matmul_q(self.buf, w.handle, rows, w._rows, None if stream is None else stream.handle)
+        return y
 
     def _matmul_typed(self, w, ty, stream):
         assert w.ggml_type == ty, f"weight is ggml type {w.ggml_type}, not {ty}"
