@@ -1,6 +1,7 @@
 // The extern "C" surface of libferric_hip (declared in include/ferric_hip.h): argument checks with
 // the reference's error behaviour, weight handles, and thin dispatch into the kernel launchers.
 #include "hostmem.hpp"
+#include "prompt.hpp"
 
 #include <stdarg.h>
 #include <stdio.h>
@@ -15,7 +16,6 @@ namespace {
 // object, so each device the library runs on holds its own copy (512 KiB) from load to process exit and no call has to
 // allocate. Host code never uses the array's name as an address: fhip_init asks the runtime for the device address of the
 // current device's copy and keeps it per device.
-using fhip::WEIGHT_SLACK;
 constexpr size_t NOALLOC_FLOATS = 131072;
 static __device__ __align__(256) float scratch[NOALLOC_FLOATS];
 constexpr int MAX_DEVICES = 64;
@@ -429,9 +429,9 @@ int fhip_weight_create(uint32_t ty, const uint8_t* h_raw, size_t nbytes, size_t 
     if (nbytes && !h_raw) return set_error(FHIP_ERR_ARG, "fhip_weight_create: NULL bytes");
     void* d = nullptr;
     // slack past the stream: a wide load that starts inside the last block may end behind it
-    if ((rc = fhip::device_malloc(&d, nbytes + WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
+    if ((rc = fhip::device_malloc(&d, nbytes + fhip::WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
     if (nbytes && (rc = check_hip(hipMemcpy(d, h_raw, nbytes, hipMemcpyHostToDevice), "hipMemcpy(weight)"))) { (void)hipFree(d); return rc; }
-    if ((rc = check_hip(hipMemset((uint8_t*)d + nbytes, 0, WEIGHT_SLACK), "hipMemset(weight tail)"))) { (void)hipFree(d); return rc; }
+    if ((rc = check_hip(hipMemset((uint8_t*)d + nbytes, 0, fhip::WEIGHT_SLACK), "hipMemset(weight tail)"))) { (void)hipFree(d); return rc; }
     w.d_raw = (const uint8_t*)d;
     w.owns = true;
     *out = new fhip_weight(w);
@@ -453,7 +453,7 @@ int fhip_weight_create_parts(uint32_t ty, const uint8_t* const* h_parts, const s
     fhip_weight w;
     if ((rc = make_weight(ty, nbytes, rows, cols, w))) return rc;
     void* d = nullptr;
-    if ((rc = fhip::device_malloc(&d, nbytes + WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
+    if ((rc = fhip::device_malloc(&d, nbytes + fhip::WEIGHT_SLACK, "hipMalloc(weight)"))) return rc;
     size_t at = 0;
     for (size_t i = 0; i < n_parts && !rc; i++) {
         if (part_bytes[i]) rc = check_hip(hipMemcpy((uint8_t*)d + at, h_parts[i], part_bytes[i], hipMemcpyHostToDevice), "hipMemcpy(weight)");
@@ -476,7 +476,7 @@ int fhip_weight_wrap_device(uint32_t ty, const uint8_t* d_raw, size_t nbytes, si
     if ((rc = make_weight(ty, nbytes, rows, cols, w))) return rc;
     if (nbytes && !d_raw) return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: NULL bytes");
     if (((uintptr_t)d_raw & 15) != 0) return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: bytes must be 16-byte aligned");
-    if (nbytes) {   // the allocation has to reach WEIGHT_SLACK bytes past the last block, as the library's own weights do
+    if (nbytes) {   // the allocation has to reach fhip::WEIGHT_SLACK bytes past the last block, as the library's own weights do
         uintptr_t start = 0, end = 0;
         if (!fhip::pool_range(d_raw, &start, &end)) {
             hipDeviceptr_t base = nullptr;
@@ -487,10 +487,10 @@ int fhip_weight_wrap_device(uint32_t ty, const uint8_t* d_raw, size_t nbytes, si
             }
             end = (uintptr_t)base + size;
         }
-        const uintptr_t need = (uintptr_t)d_raw + nbytes + WEIGHT_SLACK;
+        const uintptr_t need = (uintptr_t)d_raw + nbytes + fhip::WEIGHT_SLACK;
         if (need > end)
             return set_error(FHIP_ERR_ARG, "fhip_weight_wrap_device: the allocation must extend %zu bytes past the weight's last block "
-                             "(it ends %zu bytes behind it); buffers from fhip_malloc always do", WEIGHT_SLACK, (size_t)(end - ((uintptr_t)d_raw + nbytes)));
+                             "(it ends %zu bytes behind it); buffers from fhip_malloc always do", fhip::WEIGHT_SLACK, (size_t)(end - ((uintptr_t)d_raw + nbytes)));
     }
     w.d_raw = d_raw;
     w.owns = false;
@@ -745,8 +745,9 @@ size_t fhip_workspace_bytes(const fhip_weight* gu, const fhip_weight* down, size
 }
 
 size_t fhip_workspace_bytes_coop(const fhip_weight* w, const fhip_weight* down, size_t rows_x) {
-    const size_t a = fhip::gemm_bf16_ws_bytes(w, rows_x), b = fhip::gemm_bf16_ws_bytes(down, rows_x);
-    return a > b ? a : b;
+    const size_t a = fhip::gemm_bf16_ws_bytes(w, rows_x), b = fhip::gemm_bf16_ws_bytes(down, rows_x), c = fhip::gemm_bf16_swiglu_ws_bytes(w, rows_x);
+    const size_t ab = a > b ? a : b;
+    return ab > c ? ab : c;
 }
 
 void fhip_workspace_release(void* stream) {
@@ -1159,10 +1160,12 @@ int fhip_matmul_q_coop(const fhip_weight* w, const float* d_x, size_t rows_x, fl
     return gemm_bf16_lib_ws(w, d_ws_bf16, rows_x, d_y, (hipStream_t)stream, "fhip_matmul_q_coop");
 }
 
+// the tiled GEMM applies SwiGLU itself; up to 32 rows the gate|up matrix is small and stays in f32 between two launches
+static bool ffn_coop_fused(size_t rows_x) { return rows_x > 32; }
 
 size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gu, const fhip_weight* down, size_t rows_x) {
     if (!gu || !down) return 0;
-    return align256(rows_x * gu->cols * 2) + align256(rows_x * gu->rows * 4) + align256(rows_x * down->cols * 2);
+    return align256(rows_x * gu->cols * 2) + (ffn_coop_fused(rows_x) ? 0 : align256(rows_x * gu->rows * 4)) + align256(rows_x * down->cols * 2);
 }
 
 int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
@@ -1178,12 +1181,20 @@ int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d
     if (((uintptr_t)d_ws & 255) != 0) return set_error(FHIP_ERR_ARG, "fhip_ffn_coop: workspace must be 256-byte aligned");
     // an empty inner dimension on either side: gate and up are 0, silu(0) * 0 = 0, and so is every output
     if (gu->cols == 0 || n_ff == 0) return zero_outputs(rows_x, down->rows, d_y, (hipStream_t)stream);
+    const bool fused = ffn_coop_fused(rows_x);
     uint8_t* ws = (uint8_t*)d_ws;
     uint16_t* xb = (uint16_t*)ws;
     float* g = (float*)(ws + align256(rows_x * gu->cols * 2));
-    uint16_t* hb = (uint16_t*)((uint8_t*)g + align256(rows_x * gu->rows * 4));
+    uint16_t* hb = (uint16_t*)((uint8_t*)g + (fused ? 0 : align256(rows_x * gu->rows * 4)));
     hipStream_t s = (hipStream_t)stream;
     if ((rc = fhip::launch_cvt_bf16(d_x, rows_x * gu->cols, xb, s))) return rc;
+    if (fused) {
+        const size_t need = fhip::gemm_bf16_swiglu_ws_bytes(gu, rows_x);
+        void* split = nullptr;
+        if (need && (rc = lib_workspace(s, need, &split, "fhip_ffn_coop"))) return rc;
+        if ((rc = fhip::launch_gemm_bf16_swiglu(gu, xb, rows_x, hb, s, (float*)split, need))) return rc;
+        return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, "fhip_ffn_coop");
+    }
     if ((rc = gemm_bf16_lib_ws(gu, xb, rows_x, g, s, "fhip_ffn_coop"))) return rc;
     if ((rc = fhip::launch_swiglu_bf16(g, rows_x, n_ff, hb, s))) return rc;
     return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, "fhip_ffn_coop");

@@ -27,7 +27,7 @@
 // (256 or 128 rows) for output widths that 160 deals to the chip's workgroups exactly, and one for up to 32 rows; the
 // launcher picks by a cost estimate. A launch that cuts output tiles along K sums the partial tiles in a fixed order: the same inputs give the
 // same bits on every run.
-#include "common.hpp"
+#include "prompt.hpp"
 #include "loads.hpp"
 
 #include <hip/hip_fp16.h>
@@ -313,7 +313,31 @@ struct GemmParams {
     int per;             // of those, units per workgroup
     float* ws;           // partial tiles of the left-over tiles that several runs share: [left-over tile][contributor][BM x 256]
     int kmax;            // contributor slots per left-over tile
+    uint16_t* H;         // SwiGLU launches: bf16 [T, ff] in place of Y
+    int ff;
 };
+
+// A SwiGLU launch computes H[t, n] = bf16(silu(gate) * up) with gate row n and up row ff + n of W. Its columns are dealt to the
+// matrix instructions so that both meet in one lane: of every 32 columns the first 16 are gate rows, the other 16 the up rows of the
+// same outputs (N counts these columns: 2 x ff rounded up to 16). The f32 pair of an output then lies 16 lanes apart, and one
+// v_permlane16_swap of two accumulator registers (rows r and r + 1 of the tile) leaves every lane with gate and up of one output.
+// Measured: the f32 gate|up matrix of 2048 x 34816 and the kernel that read it back took 100 us behind a 783 us GEMM.
+__device__ __forceinline__ int swiglu_row(int v, int ff) {
+    const int n = 16 * (v >> 5) + (v & 15);
+    return (n < ff ? n : ff - 1) + (v & 16 ? ff : 0);
+}
+__device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
+// the 32 x 32 accumulator of rows t0 .. and columns v0 ..: outputs 16 * (v0 / 32) + (c & 15)
+__device__ __forceinline__ void store_swiglu(const GemmParams& p, const f32x16& acc, int t0, int v0, int h, int c) {
+    const int n = 16 * (v0 >> 5) + (c & 15);
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+        const auto gu = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[r]), __float_as_uint(acc[r + 1]), false, false);
+        const int t = t0 + 8 * (r >> 2) + 4 * h + (r & 3) + (c >> 4);
+        if (t < p.T && n < p.ff)
+            p.H[(size_t)t * p.ff + n] = (uint16_t)(pk_bf16(silu_mul(__uint_as_float(gu[0]), __uint_as_float(gu[1])), 0.f) & 0xFFFFu);
+    }
+}
 
 template <int I, int N, class Fn>
 __device__ __forceinline__ void static_for(Fn&& f) {
@@ -344,7 +368,7 @@ __device__ __forceinline__ void static_for(Fn&& f) {
 // block of 32 weight rows, both waves carry its raw bytes and each unpacks two of a step's four slices, so that at 128
 // activation rows (MI = 2) every weight is unpacked once (the 64 x 256 tile unpacks it twice, once per tile row) with the
 // same partial-tile bytes per workgroup.
-template <class F, int MI, int NI>
+template <class F, int MI, int NI, bool SWIGLU>
 __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
     constexpr int BM = 64 * MI, BN = 128 * NI;
     constexpr int FRAG = 512;                                   // bf16 per published fragment (64 lanes x 8)
@@ -381,7 +405,8 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
     const uint8_t* wrow;
     {
         int n = n0 + (NI == 2 ? 32 * wm : 0) + c;
-        wrow = p.W + (size_t)(n < p.N ? n : p.N - 1) * p.row_bytes;
+        n = n < p.N ? n : p.N - 1;
+        wrow = p.W + (size_t)(SWIGLU ? swiglu_row(n, p.ff) : n) * p.row_bytes;
     }
     const int b_wr = ((NI == 2 ? 2 * wn + wm : wn) * 4) * FRAG + lane * 8;    // + t * FRAG
     const int b_rd = ((NI * wn) * 4) * FRAG + lane * 8;                        // + (4 * j + t) * FRAG
@@ -513,6 +538,10 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
 #pragma unroll
         for (int j = 0; j < NI; j++) {
             const int n = n0 + 32 * j + c;
+            if (SWIGLU && whole) {
+                store_swiglu(p, acc[i][j], t0 + 32 * i, n0 + 32 * j, h, c);
+                continue;
+            }
             if (n >= p.N) continue;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -543,7 +572,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
 // 75.7 -> 68.9, Q6_K 5120 x 17408 at 128 rows 64.6 -> 59.0, Q8_0 12288 x 4096 at 128 rows 57.8 -> 52.3; at 512 rows of
 // 5120 x 5120 (128 tiles cut in two instead of 64 cut in four) it is level, 49.2 against 48.0.
 // ------------------------------------------------------------------------------------------------
-template <class F, int MI>
+template <class F, int MI, bool SWIGLU>
 __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
     constexpr int NB = 5;
     constexpr int BM = 64 * MI, BN = 32 * NB;
@@ -585,7 +614,8 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
     const uint8_t* wrow;
     {
         int n = n0 + 32 * (unpacker ? wave : 0) + c;
-        wrow = p.W + (size_t)(n < p.N ? n : p.N - 1) * p.row_bytes;
+        n = n < p.N ? n : p.N - 1;
+        wrow = p.W + (size_t)(SWIGLU ? swiglu_row(n, p.ff) : n) * p.row_bytes;
     }
     const int b_wr = (wave * 4) * FRAG + lane * 8;              // + t * FRAG (unpackers)
     const int b_rd = (4 * j0) * FRAG + lane * 8;                // + (4 * j + t) * FRAG
@@ -729,7 +759,12 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 #pragma unroll
     for (int j = 0; j < NBW; j++) {
         const int n = n0 + 32 * (j0 + j) + c;
-        if (j >= nj || n >= p.N) continue;
+        if (j >= nj) continue;
+        if (SWIGLU && whole) {
+            store_swiglu(p, acc[j], t0, n0 + 32 * (j0 + j), h, c);
+            continue;
+        }
+        if (n >= p.N) continue;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int t = t0 + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -776,6 +811,48 @@ __global__ void __launch_bounds__(256) sum_split_tiles_kernel(float* __restrict_
         if (col + 1 < N) y[1] = a.y;
         if (col + 2 < N) y[2] = a.z;
         if (col + 3 < N) y[3] = a.w;
+    }
+}
+
+// The same for a SwiGLU launch: a thread adds the gate columns and the up columns of four adjacent outputs of one row.
+__global__ void __launch_bounds__(256) sum_split_swiglu_kernel(uint16_t* __restrict__ H, const float* __restrict__ ws, int T, int ff, int BM, int BN,
+                                                             int tiles_n, int nchunks, int per, int kmax, int first_tile) {
+    const int rt = blockIdx.x, tile = first_tile + rt;
+    const long long u0 = (long long)rt * nchunks;
+    const int nk = (int)((u0 + nchunks - 1) / per) - (int)(u0 / per) + 1;
+    if (nk == 1) return;
+    const int tile_y = tile / tiles_n, tile_x = tile - tile_y * tiles_n;
+    const int item = blockIdx.y * 256 + threadIdx.x, bn8 = BN >> 3;
+    const int lt = item / bn8, c4 = (item - lt * bn8) * 4;         // output column of the tile
+    const int t = tile_y * BM + lt, col = tile_x * (BN >> 1) + c4;
+    if (lt >= BM || t >= T || col >= ff) return;
+    const size_t slot = (size_t)BM * BN;
+    const float* q = ws + (size_t)rt * kmax * slot + (size_t)lt * BN + 32 * (c4 >> 4) + (c4 & 15);
+    float4 g = {0.f, 0.f, 0.f, 0.f}, u = g;
+    for (int k0 = 0; k0 < nk; k0 += 4) {
+        float4 vg[4], vu[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float* s = q + (size_t)(k0 + j < nk ? k0 + j : 0) * slot;
+            vg[j] = *(const float4*)s;
+            vu[j] = *(const float4*)(s + 16);
+        }
+        if (k0 == 0) { g = vg[0]; u = vu[0]; }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k0 + j > 0 && k0 + j < nk) {
+                g.x += vg[j].x; g.y += vg[j].y; g.z += vg[j].z; g.w += vg[j].w;
+                u.x += vu[j].x; u.y += vu[j].y; u.z += vu[j].z; u.w += vu[j].w;
+            }
+    }
+    const uint32_t lo = pk_bf16(silu_mul(g.x, u.x), silu_mul(g.y, u.y)), hi = pk_bf16(silu_mul(g.z, u.z), silu_mul(g.w, u.w));
+    uint16_t* out = H + (size_t)t * ff + col;
+    if ((ff & 3) == 0) *(uint2*)out = make_uint2(lo, hi);
+    else {
+        out[0] = (uint16_t)(lo & 0xFFFFu);
+        if (col + 1 < ff) out[1] = (uint16_t)(lo >> 16);
+        if (col + 2 < ff) out[2] = (uint16_t)(hi & 0xFFFFu);
+        if (col + 3 < ff) out[3] = (uint16_t)(hi >> 16);
     }
 }
 
@@ -1053,15 +1130,19 @@ static size_t plan_ws_bytes(const TilePlan& q) {
     return q.split_wgs > 0 ? (size_t)q.left * q.kmax * (size_t)(64 * q.mi * q.bn) * sizeof(float) : 0;
 }
 
-template <class F, int MI, int BN>
-int launch_cfg(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, const TilePlan& q, long long cus, float* d_ws,
+// columns of a SwiGLU launch (see swiglu_row)
+static size_t swiglu_columns(size_t ff) { return (ff + 15) / 16 * 32; }
+
+template <class F, int MI, int BN, bool SWIGLU>
+int launch_cfg(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out, hipStream_t s, const TilePlan& q, long long cus, float* d_ws,
                size_t ws_bytes) {
     GemmParams p;
-    p.W = w->d_raw; p.X = d_x; p.Y = d_y;
-    p.T = (int)t; p.N = (int)w->rows; p.K = (int)w->cols; p.row_bytes = w->row_bytes;
+    const size_t columns = SWIGLU ? swiglu_columns(w->rows / 2) : w->rows;
+    p.W = w->d_raw; p.X = d_x; p.Y = SWIGLU ? nullptr : (float*)d_out; p.H = SWIGLU ? (uint16_t*)d_out : nullptr; p.ff = (int)(w->rows / 2);
+    p.T = (int)t; p.N = (int)columns; p.K = (int)w->cols; p.row_bytes = w->row_bytes;
     p.nblk = (int)(w->row_bytes / F::BLOCK);
     p.nchunks = F::chunks(p.K);
-    p.tiles_n = (int)((w->rows + BN - 1) / BN);
+    p.tiles_n = (int)((columns + BN - 1) / BN);
     // one workgroup per CU (its LDS tiles take most of a CU's 160 KB)
     p.whole_rounds = q.whole_rounds;
     p.units = q.units;
@@ -1069,11 +1150,14 @@ int launch_cfg(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, 
     p.ws = d_ws; p.kmax = q.kmax;
     if (q.split_wgs > 0 && (!d_ws || ws_bytes < plan_ws_bytes(q)))
         return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: the launch cuts tiles along K and needs %zu bytes of workspace", plan_ws_bytes(q));
-    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 2>), dim3(q.grid), dim3(512), 0, s, p);
-    else if constexpr (BN == 128) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 1>), dim3(q.grid), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<F, MI>), dim3(q.grid), dim3(512), 0, s, p);
-    if (q.split_wgs > 0)
-        hipLaunchKernelGGL(sum_split_tiles_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 4 + 255) / 256)), dim3(256), 0, s, d_y, (const float*)d_ws, p.T, p.N, 64 * MI,
+    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 2, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    else if constexpr (BN == 128) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 1, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<F, MI, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    if (q.split_wgs > 0 && SWIGLU)
+        hipLaunchKernelGGL(sum_split_swiglu_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 8 + 255) / 256)), dim3(256), 0, s, p.H, (const float*)d_ws, p.T, p.ff, 64 * MI,
+                           BN, p.tiles_n, p.nchunks, p.per, p.kmax, (int)(p.whole_rounds * cus));
+    else if (q.split_wgs > 0)
+        hipLaunchKernelGGL(sum_split_tiles_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 4 + 255) / 256)), dim3(256), 0, s, p.Y, (const float*)d_ws, p.T, p.N, 64 * MI,
                            BN, p.tiles_n, p.nchunks, p.per, p.kmax, (int)(p.whole_rounds * cus));
     return fhip::check_hip(hipGetLastError(), "gemm_q_bf16 launch");
 }
@@ -1082,7 +1166,7 @@ int g_force_tile = -1;   // tests: 0..3 = 64, 128, 256 rows x 256 columns, 256 x
 
 // the tile the estimate picks for this launch (one of the seven the loop lists) with its plan
 template <class F>
-static void choose_plan(const fhip_weight* w, size_t t, TilePlan& out) {
+static void choose_plan(const fhip_weight* w, size_t columns, size_t t, TilePlan& out) {
     const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     const int nchunks = F::chunks((int)w->cols);
     float best_cost = 0.f;
@@ -1090,23 +1174,22 @@ static void choose_plan(const fhip_weight* w, size_t t, TilePlan& out) {
         constexpr int MI_OF[7] = {1, 2, 4, 4, 2, 1, 2}, BN_OF[7] = {256, 256, 256, 160, 128, 128, 160};
         const int mi = MI_OF[i], bn = BN_OF[i];
         if (g_force_tile >= 0 && g_force_tile <= 6 && i != g_force_tile) continue;
-        const TilePlan q = plan_tiles((long long)((w->rows + bn - 1) / bn), nchunks, t, mi, cus, bn);
+        const TilePlan q = plan_tiles((long long)((columns + bn - 1) / bn), nchunks, t, mi, cus, bn);
         const float c = plan_cost_us<F>(q, nchunks, cus);
         if (best_cost == 0.f || c < 0.98f * best_cost) { best_cost = c; out = q; }
     }
 }
 
 template <class F>
-static size_t ws_bytes_fmt(const fhip_weight* w, size_t t) {
+static size_t ws_bytes_fmt(const fhip_weight* w, size_t columns, size_t t) {
     if (t <= 32) return skinny_ws_bytes(plan_skinny(w->rows, F::chunks((int)w->cols), t, fhip::device_cus() > 0 ? fhip::device_cus() : 256));
     TilePlan q;
-    choose_plan<F>(w, t, q);
+    choose_plan<F>(w, columns, t, q);
     return plan_ws_bytes(q);
 }
 
-template <class F>
-int launch_fmt(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
-    if (t <= 32) return launch_skinny<F>(w, d_x, t, d_y, s, d_ws, ws_bytes);
+template <class F, bool SWIGLU>
+int launch_tiled(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
     // Which tile. The 256 x 256 tile unpacks each weight once per 256 activation rows, but when there is no whole round of
     // such tiles for the chip every tile is cut along K, each workgroup writes a whole partial tile for a few chunks of
     // work, and a lower tile (twice the tiles, half the fix-up, longer runs), the 256 x 160 tile (whose count divides the
@@ -1118,14 +1201,20 @@ int launch_fmt(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, 
     // 4096 x 4096 T = 128 35 / 33 / 37 / 32 / 31 / 40.
     const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     TilePlan q;
-    choose_plan<F>(w, t, q);
-    if (q.bn == 160) return q.mi == 4 ? launch_cfg<F, 4, 160>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
-                                      : launch_cfg<F, 2, 160>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.bn == 128) return q.mi == 2 ? launch_cfg<F, 2, 128>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
-                                      : launch_cfg<F, 1, 128>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.mi == 4) return launch_cfg<F, 4, 256>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.mi == 2) return launch_cfg<F, 2, 256>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    return launch_cfg<F, 1, 256>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    choose_plan<F>(w, SWIGLU ? swiglu_columns(w->rows / 2) : w->rows, t, q);
+    if (q.bn == 160) return q.mi == 4 ? launch_cfg<F, 4, 160, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
+                                      : launch_cfg<F, 2, 160, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    if (q.bn == 128) return q.mi == 2 ? launch_cfg<F, 2, 128, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
+                                      : launch_cfg<F, 1, 128, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    if (q.mi == 4) return launch_cfg<F, 4, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    if (q.mi == 2) return launch_cfg<F, 2, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    return launch_cfg<F, 1, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+}
+
+template <class F>
+int launch_fmt(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
+    if (t <= 32) return launch_skinny<F>(w, d_x, t, d_y, s, d_ws, ws_bytes);
+    return launch_tiled<F, false>(w, d_x, t, d_y, s, d_ws, ws_bytes);
 }
 
 // f32 -> bf16 (round to nearest even), 8 values per thread, the tail one by one
@@ -1148,7 +1237,7 @@ __global__ void __launch_bounds__(256) swiglu_bf16_kernel(const float* __restric
     if (i >= n) return;
     const size_t row = i / d, col = i % d;
     const float g = gu[row * 2 * d + col], u = gu[row * 2 * d + d + col];
-    out[i] = (uint16_t)(pk_bf16((g / (1.0f + expf(-g))) * u, 0.f) & 0xFFFFu);
+    out[i] = (uint16_t)(pk_bf16(silu_mul(g, u), 0.f) & 0xFFFFu);
 }
 
 }  // namespace
@@ -1178,10 +1267,10 @@ int gemm_bf16_force_tile(int tile) {
 size_t gemm_bf16_ws_bytes(const fhip_weight* w, size_t t) {
     if (!w || t == 0 || w->rows == 0) return 0;
     switch (w->type) {
-        case FHIP_Q4_K: return ws_bytes_fmt<Q4K>(w, t);
-        case FHIP_Q6_K: return ws_bytes_fmt<Q6K>(w, t);
-        case FHIP_Q8_0: return ws_bytes_fmt<Q80>(w, t);
-        case FHIP_Q5_K: return ws_bytes_fmt<Q5K>(w, t);
+        case FHIP_Q4_K: return ws_bytes_fmt<Q4K>(w, w->rows, t);
+        case FHIP_Q6_K: return ws_bytes_fmt<Q6K>(w, w->rows, t);
+        case FHIP_Q8_0: return ws_bytes_fmt<Q80>(w, w->rows, t);
+        case FHIP_Q5_K: return ws_bytes_fmt<Q5K>(w, w->rows, t);
         default: return 0;
     }
 }
@@ -1196,6 +1285,33 @@ int launch_gemm_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float*
         case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_x, t, d_y, s, d_ws, ws_bytes);
         case FHIP_Q8_0: return launch_fmt<Q80>(w, d_x, t, d_y, s, d_ws, ws_bytes);
         case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_x, t, d_y, s, d_ws, ws_bytes);
+        default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "QMatrix: no native matmul for ggml type %u", w->type);
+    }
+}
+
+// H [t, rows / 2] = bf16(silu(gate) * up) of the stacked [gate | up] weight, for more than 32 rows (fewer: launch_gemm_bf16 and
+// launch_swiglu_bf16)
+size_t gemm_bf16_swiglu_ws_bytes(const fhip_weight* w, size_t t) {
+    if (!w || t <= 32 || w->rows == 0 || w->rows % 2 != 0) return 0;
+    const size_t columns = swiglu_columns(w->rows / 2);
+    switch (w->type) {
+        case FHIP_Q4_K: return ws_bytes_fmt<Q4K>(w, columns, t);
+        case FHIP_Q6_K: return ws_bytes_fmt<Q6K>(w, columns, t);
+        case FHIP_Q8_0: return ws_bytes_fmt<Q80>(w, columns, t);
+        case FHIP_Q5_K: return ws_bytes_fmt<Q5K>(w, columns, t);
+        default: return 0;
+    }
+}
+
+int launch_gemm_bf16_swiglu(const fhip_weight* w, const uint16_t* d_x, size_t t, uint16_t* d_h, hipStream_t s, float* d_ws, size_t ws_bytes) {
+    if (((uintptr_t)d_x & 15) != 0) return set_error(FHIP_ERR_ARG, "gemm_q_bf16: x must be 16-byte aligned");
+    if ((unsigned long long)t * w->cols >= (1ull << 31))
+        return set_error(FHIP_ERR_SHAPE, "gemm_q_bf16: t * cols must be below 2^31 (got %zu x %zu)", t, w->cols);
+    switch (w->type) {
+        case FHIP_Q4_K: return launch_tiled<Q4K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q6_K: return launch_tiled<Q6K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q8_0: return launch_tiled<Q80, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q5_K: return launch_tiled<Q5K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "QMatrix: no native matmul for ggml type %u", w->type);
     }
 }

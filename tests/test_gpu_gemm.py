@@ -220,6 +220,26 @@ def test_batched_decode_ffn_on_the_matrix_cores(F, O):
         assert np.abs(y1 - y).max() <= 2e-5 * np.abs(y).max()
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6, -1])
+def test_swiglu_inside_the_tiled_gemm(F, tile):
+    # ffn_coop over 32 rows applies SwiGLU in the gate|up launch (or in the launch that sums a cut tile): the same f32 sums, one f32
+    # expression and one rounding to bf16, so the block equals its steps bit for bit. Rows that end inside a tile, widths whose
+    # tiles are whole, cut and ragged (n_ff = 96: tiles of mostly nothing; 1312: no multiple of any tile's columns).
+    from ferric_amd.synth import synth_weights
+    lib = F._lib.load()
+    before = lib.fhip_debug_gemm_tile(tile)
+    try:
+        for i, (tg, td, t, d, n_ff) in enumerate([(Q4_K, Q8_0, 33, 512, 96), (Q4_K, Q8_0, 300, 1024, 1312), (Q6_K, Q4_K, 65, 768, 512), (Q8_0, Q6_K, 257, 288, 768),
+                                                  (Q5_K, Q8_0, 130, 1024, 1312), (Q4_K, Q6_K, 520, 256, 9984)]):
+            gu = F.QMatrix.from_bytes(synth_weights(tg, 2 * n_ff, d, 900 + i), tg, 2 * n_ff, d)
+            dn = F.QMatrix.from_bytes(synth_weights(td, 256, n_ff, 950 + i), td, 256, n_ff)
+            x = F.Tensor.from_vec(np.random.default_rng(i).standard_normal(t * d).astype(np.float32), (t, d))
+            want = x.matmul_q_coop(gu).swiglu(n_ff).matmul_q_coop(dn).to_vec()
+            assert np.array_equal(x.ffn_coop(gu, dn).to_vec().view(np.uint32), want.view(np.uint32)), (tile, tg, t, n_ff)
+    finally:
+        lib.fhip_debug_gemm_tile(before)
+
+
 def test_gemm_errors(F):
     qm = F.QMatrix.from_bytes(np.zeros(144, np.uint8), Q4_K, 1, 256)
     with pytest.raises(AssertionError, match="inner dim mismatch"):
