@@ -2,34 +2,50 @@
 //
 // A pageable hipMemcpyAsync costs a staging copy inside the runtime and a switch between the compute queue and a DMA engine: behind
 // a kernel, 20 KB to the device took 16 us with the synchronisation that lets the source go, 608 KB to the host 38 us, and 84 MB
-// to fresh host memory 12.5 ms (a single thread taking page faults one by one). Here a copy goes through a slot of pinned memory
-// that a small kernel on the caller's own stream reads or writes directly:
-//   to the device   the source is in the slot when the call returns, so nobody waits (3 us of host time)
-//   to the host     one kernel and one wait; more than a slot is cut into chunks, each copied out of its slot by a worker thread
-//                   while the next ones cross the bus (page faults of the destination included, which is why there are several)
+// to fresh host memory 12.5 ms (a single thread taking page faults one by one). Here a copy goes through slots of pinned memory
+// that a small kernel on the caller's own stream reads or writes directly; the kernel's workgroups confirm in pinned words of
+// their own, which a host thread polls without a call into the runtime.
+//   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time)
+//   to the host     up to a slot in one or two kernels, the host copying the first part out while the second crosses the bus
+//                   (608 KB, idle device: 37 us with one kernel and a stream synchronisation); more is cut into chunks, each
+//                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
+//                   included, which is why there are several workers)
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms.
 #include "hostmem.hpp"
 
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <vector>
 
 namespace {
 
-constexpr size_t OUT_BYTES = (size_t)2 << 20;    // a slot's part for data on its way to the host ...
-constexpr size_t IN_BYTES = fhip::H2D_STAGED;    // ... and to the device (OUT_BYTES of floats are at most 557 056 block bytes, Q8_0)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr size_t OUT_BYTES = (size_t)1 << 20;    // a slot's part for data on its way to the host ...
+constexpr size_t IN_BYTES = fhip::H2D_STAGED;    // ... and to the device (a chunk of floats is at most 278 528 block bytes, Q8_0)
+constexpr size_t CHUNK = OUT_BYTES;              // of a long copy
 constexpr size_t SLOT_BYTES = OUT_BYTES + IN_BYTES;
-constexpr int SLOTS = 12, JOB_SLOTS = 8;         // a chunked copy takes up to JOB_SLOTS and leaves the others to small copies
-constexpr int MAX_WG = 32, THREADS = 512;        // workgroups of a small copy (each confirms its part in a word of its own)
-constexpr int WORKERS = 6;
+constexpr int SLOTS = 16, JOB_SLOTS = 12;        // a chunked copy takes up to JOB_SLOTS and leaves the others to small copies
+constexpr int MAX_WG = 64, THREADS = 512;        // workgroups of a copy (each confirms its part in a word of its own)
+constexpr size_t TWO_PARTS = (size_t)96 << 10;   // copies to the host from here on go in two parts: a launch costs less than the copy it hides
+constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
 // n bytes, each workgroup a strided share; U = 16, 4 or 1 bytes, what the addresses allow. done (may be null): workgroup w stores seq
-// in done[w] once everything it reads has been read.
+// in done[w] once everything it reads has been read and everything it writes has arrived.
+// A confirmation is one store behind a wait, not a release: a release at system scope writes back the whole L2 (5 us of a 4 KB copy).
+// The stores it stands for go through to memory themselves (sc0 sc1), and s_waitcnt holds the wave until they have arrived.
+template <class U>
+__device__ __forceinline__ void store_through(U* p, U v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+template <>
+__device__ __forceinline__ void store_through(u32x4* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory"); }
+
 template <class U>
 __global__ __launch_bounds__(THREADS) void copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t n, uint32_t* done,
                                                        uint32_t seq) {
@@ -39,14 +55,15 @@ __global__ __launch_bounds__(THREADS) void copy_kernel(const uint8_t* __restrict
     size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     for (; i + 3 * step < units; i += 4 * step) {       // four loads in flight: a load from host memory takes over a microsecond
         const U a = s[i], b = s[i + step], c = s[i + 2 * step], e = s[i + 3 * step];
-        d[i] = a; d[i + step] = b; d[i + 2 * step] = c; d[i + 3 * step] = e;
+        store_through(d + i, a); store_through(d + i + step, b); store_through(d + i + 2 * step, c); store_through(d + i + 3 * step, e);
     }
-    for (; i < units; i += step) d[i] = s[i];
+    for (; i < units; i += step) store_through(d + i, s[i]);
     if (sizeof(U) > 1 && blockIdx.x == 0)
-        for (size_t k = units * sizeof(U) + threadIdx.x; k < n; k += THREADS) dst[k] = src[k];
+        for (size_t k = units * sizeof(U) + threadIdx.x; k < n; k += THREADS) store_through(dst + k, src[k]);
     if (done) {
-        __syncthreads();                                // every wave's stores, and so the loads in front of them, are issued
-        if (threadIdx.x == 0) __hip_atomic_store(&done[blockIdx.x], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(&done[blockIdx.x], seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -58,7 +75,7 @@ int launch_copy(const void* src, void* dst, size_t n, int max_wg, uint32_t* done
     *wgs = (int)g;
     const uint8_t* from = (const uint8_t*)src;
     uint8_t* to = (uint8_t*)dst;
-    if (unit == 16) copy_kernel<uint4><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
+    if (unit == 16) copy_kernel<u32x4><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
     else if (unit == 4) copy_kernel<uint32_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
     else copy_kernel<uint8_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
     return fhip::check_hip(hipGetLastError(), "copy kernel");
@@ -66,19 +83,32 @@ int launch_copy(const void* src, void* dst, size_t n, int max_wg, uint32_t* done
 
 struct Slot {
     uint8_t* host = nullptr;     // SLOT_BYTES pinned: [OUT_BYTES][IN_BYTES]
-    uint8_t* dev = nullptr;      // IN_BYTES of device memory (dequantization only)
+    uint8_t* dev = nullptr;      // as much device memory (dequantization only)
     uint32_t* done = nullptr;    // MAX_WG pinned words
     uint32_t seq = 0;
     int wgs = 0;                 // words of `done` that have to reach seq before the GPU has read the slot
     bool held = false;
-    hipEvent_t ev = nullptr;
 
-    bool read_by_gpu() const {
-        for (int i = 0; i < wgs; i++)
-            if (__atomic_load_n(&done[i], __ATOMIC_ACQUIRE) != seq) return false;
+    bool read_by_gpu() const { return confirmed(seq, wgs); }
+    bool confirmed(uint32_t want, int n) const {
+        for (int i = 0; i < n; i++)
+            if (__atomic_load_n(&done[i], __ATOMIC_ACQUIRE) != want) return false;
         return true;
     }
 };
+
+// Until the first n words of the slot hold `want`: polled for two milliseconds (a decode step), then left to the runtime.
+int await_words(const Slot* q, uint32_t want, int n, hipStream_t s) {
+    const auto start = std::chrono::steady_clock::now();
+    for (unsigned i = 0; !q->confirmed(want, n); i++) {
+#if defined(__x86_64__)
+        __builtin_ia32_pause();
+#endif
+        if ((i & 255) == 255 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2))
+            return fhip::check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+    }
+    return FHIP_OK;
+}
 
 struct Ring {                    // one per device
     std::mutex mu;
@@ -130,40 +160,55 @@ Ring* ring(int* rc) {
     return &all[dev];
 }
 
-// ---- chunks on their way to the host, copied out of their slots by worker threads ----------------------------------------------
+// ---- chunks whose host side worker threads copy -------------------------------------------------------------------------------
+// Task k of a job: the first n_slots are the ways up of chunks 0 .. n_slots - 1, then the way down of chunk c and the way up of chunk
+// c + n_slots take turns. A job that goes one way only has the other kind as empty tasks.
 struct Job {
-    uint8_t* dst;
-    size_t bytes, chunk, count;               // the destination, cut into `count` chunks of `chunk` bytes (the last: what is left)
+    size_t count;                             // chunks; chunk c is [c * chunk, ..) of each side it has
+    const uint8_t* up;                        // the caller's memory on the way up (may be null) ...
+    size_t up_bytes, up_chunk, up_at;         // ... and where its chunks lie in a slot
+    uint8_t* down;                            // and on the way down (may be null)
+    size_t down_bytes, down_chunk;
     Slot** slots;
     size_t n_slots;
-    int dev;
-    std::atomic<size_t> launched{0}, next{0}, copied{0};
-    std::atomic<uint8_t>* out;                // [count] chunk has left its slot
+    std::atomic<size_t> launched{0}, next{0}, left{0};
+    std::atomic<uint8_t>*filled, *emptied;    // [count] the chunk is in its slot / out of it
+    uint32_t* want;                           // [count] what the slot's words hold once the device is done with the chunk ...
+    int* words;                               // ... and how many do
     std::atomic<int> abort{0};
-    std::atomic<int> err{0};                  // hipError_t of an event
-};
 
+    bool device_done(size_t c) const { return launched.load(std::memory_order_acquire) > c && slots[c % n_slots]->confirmed(want[c], words[c]); }
+};
+size_t part(size_t bytes, size_t chunk, size_t c) { return bytes - c * chunk < chunk ? bytes - c * chunk : chunk; }
+
+// false: the job was aborted
+bool go_up(Job* j, size_t c) {
+    if (c >= j->count || !j->up) return true;
+    while (c >= j->n_slots && !(j->down ? j->emptied[c - j->n_slots].load(std::memory_order_acquire) != 0 : j->device_done(c - j->n_slots))) {
+        if (j->abort.load()) return false;
+        std::this_thread::yield();
+    }
+    memcpy(j->slots[c % j->n_slots]->host + j->up_at, j->up + c * j->up_chunk, part(j->up_bytes, j->up_chunk, c));
+    j->filled[c].store(1, std::memory_order_release);
+    return true;
+}
+bool go_down(Job* j, size_t c) {
+    if (c >= j->count || !j->down) return true;
+    while (!j->device_done(c)) {
+        if (j->abort.load()) return false;
+        std::this_thread::yield();
+    }
+    memcpy(j->down + c * j->down_chunk, j->slots[c % j->n_slots]->host, part(j->down_bytes, j->down_chunk, c));
+    j->emptied[c].store(1, std::memory_order_release);
+    j->left.fetch_add(1);
+    return true;
+}
 void work_on(Job* j) {
-    (void)hipSetDevice(j->dev);
     for (;;) {
-        const size_t c = j->next.fetch_add(1);
-        if (c >= j->count) return;
-        while (j->launched.load(std::memory_order_acquire) <= c) {
-            if (j->abort.load()) return;
-            std::this_thread::yield();
-        }
-        Slot* q = j->slots[c % j->n_slots];
-        hipError_t e;
-        while ((e = hipEventQuery(q->ev)) == hipErrorNotReady) {
-            (void)hipGetLastError();
-            if (j->abort.load()) return;
-            std::this_thread::yield();
-        }
-        if (e != hipSuccess) { j->err.store((int)e); j->abort.store(1); return; }
-        const size_t at = c * j->chunk, n = j->bytes - at < j->chunk ? j->bytes - at : j->chunk;
-        memcpy(j->dst + at, q->host, n);
-        j->out[c].store(1, std::memory_order_release);
-        j->copied.fetch_add(1);
+        const size_t k = j->next.fetch_add(1);
+        if (k >= 2 * j->count + j->n_slots) return;
+        const size_t m = k - j->n_slots;
+        if (!(k < j->n_slots ? go_up(j, k) : m % 2 ? go_up(j, m / 2 + j->n_slots) : go_down(j, m / 2))) return;
     }
 }
 
@@ -217,50 +262,62 @@ struct Workers {
 };
 Workers& workers() { static Workers* w = new Workers(); return *w; }
 
-// fill(c, slot, stream, n): enqueue what puts chunk c (n bytes) into slot->host; streams are taken in turn
-template <class Fill>
-int run_chunks(Ring* r, uint8_t* dst, size_t bytes, size_t chunk, hipStream_t* streams, size_t n_streams, Fill fill) {
+// launch(c, slot, stream, &words): enqueue what the device does with chunk c in slot->host, the last kernel confirming slot->seq + 1 in
+// the slot's words; streams are taken in turn. The caller sets the sides of `j` and its count.
+template <class Launch>
+int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Launch launch) {
     Workers& w = workers();
     std::lock_guard<std::mutex> one(w.one);
     int rc = FHIP_OK;
-    Job j;
-    j.dst = dst; j.bytes = bytes; j.chunk = chunk; j.count = (bytes + chunk - 1) / chunk;
     Slot* slots[JOB_SLOTS];
     j.slots = slots;
     j.n_slots = 0;
-    if ((rc = fhip::check_hip(hipGetDevice(&j.dev), "hipGetDevice"))) return rc;
     while (j.n_slots < JOB_SLOTS && j.n_slots < j.count) {
         Slot* q = j.n_slots ? r->take(&rc) : r->need(&rc);
         if (!q) break;
         slots[j.n_slots++] = q;
-        if (!q->ev && (rc = fhip::check_hip(hipEventCreateWithFlags(&q->ev, hipEventDisableTiming), "hipEventCreate"))) { q->ev = nullptr; break; }
     }
-    std::atomic<uint8_t>* out = nullptr;
     if (!rc) {
-        out = new std::atomic<uint8_t>[j.count]();
-        j.out = out;
+        std::vector<std::atomic<uint8_t>> flags(2 * j.count);
+        std::vector<uint32_t> want(j.count);
+        std::vector<int> words(j.count);
+        j.filled = flags.data(); j.emptied = flags.data() + j.count; j.want = want.data(); j.words = words.data();
         const bool helped = w.post(&j);
+        auto wait_for = [&](auto ready) {       // also looks for a device error every few milliseconds: what waits here would wait for ever
+            auto look = std::chrono::steady_clock::now();
+            for (unsigned i = 1; !ready() && !rc; i++) {
+                std::this_thread::yield();
+                if (i % 1024 || std::chrono::steady_clock::now() - look < std::chrono::milliseconds(5)) continue;
+                look = std::chrono::steady_clock::now();
+                for (size_t k = 0; k < n_streams && !rc; k++) {
+                    const hipError_t e = hipStreamQuery(streams[k]);
+                    if (e == hipErrorNotReady) (void)hipGetLastError();
+                    else rc = fhip::check_hip(e, "hipStreamQuery");
+                }
+            }
+        };
         for (size_t c = 0; c < j.count && !rc; c++) {
-            if (c >= j.n_slots && helped)
-                while (!out[c - j.n_slots].load(std::memory_order_acquire) && !j.abort.load()) std::this_thread::yield();
-            if (j.abort.load()) break;
             Slot* q = slots[c % j.n_slots];
             hipStream_t s = streams[c % n_streams];
-            const size_t at = c * chunk, n = bytes - at < chunk ? bytes - at : chunk;
-            if (!(rc = fill(c, q, s, n))) rc = fhip::check_hip(hipEventRecord(q->ev, s), "hipEventRecord");
-            if (!rc && !helped && !(rc = fhip::check_hip(hipEventSynchronize(q->ev), "hipEventSynchronize"))) {
-                memcpy(dst + at, q->host, n);
-                j.copied.fetch_add(1);
+            if (!helped) {                       // without threads the chunks go one by one
+                if (c >= j.n_slots) wait_for([&] { return j.device_done(c - j.n_slots); });
+                if (!rc) (void)go_up(&j, c);
+            } else if (j.up) {
+                wait_for([&] { return j.filled[c].load(std::memory_order_acquire) != 0; });
+            } else if (c >= j.n_slots) {
+                wait_for([&] { return j.emptied[c - j.n_slots].load(std::memory_order_acquire) != 0; });
             }
-            if (!rc) j.launched.store(c + 1, std::memory_order_release);
+            int wgs = 0;
+            if (rc || (rc = launch(c, q, s, &wgs))) break;
+            want[c] = ++q->seq; words[c] = q->wgs = wgs;
+            j.launched.store(c + 1, std::memory_order_release);
+            if (!helped && !(rc = await_words(q, want[c], wgs, s))) (void)go_down(&j, c);
         }
+        if (j.down && !rc) wait_for([&] { return j.left.load() >= j.count; });
         if (rc) j.abort.store(1);
-        while (!j.abort.load() && j.copied.load() < j.count) std::this_thread::yield();
         w.finish();
-        if (!rc && j.err.load()) rc = fhip::check_hip((hipError_t)j.err.load(), "hipEventQuery");
-        if (rc)                                // an enqueued chunk may still write into a slot
+        if (rc)                                 // an enqueued chunk may still use a slot
             for (size_t i = 0; i < n_streams; i++) (void)hipStreamSynchronize(streams[i]);
-        delete[] out;
     }
     for (size_t i = 0; i < j.n_slots; i++) r->release(slots[i]);
     return rc;
@@ -276,13 +333,15 @@ bool capturing(hipStream_t s) {
 
 namespace fhip {
 
-// Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime (35 GB/s, and
-// it returns when the source has been read or is known to be pinned). A copy in a stream capture stays a copy node.
+// Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime (10 MB in 285 us;
+// chunks of it copied into slots by workers and pulled over the bus by kernels took 300 - 360), and it returns when the source has
+// been read or is known to be pinned. A copy in a stream capture stays a copy node.
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     if (n > IN_BYTES || capturing(s)) return check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
     int rc;
     Ring* r = ring(&rc);
-    Slot* q = r ? r->need(&rc) : nullptr;
+    if (!r) return rc;
+    Slot* q = r->need(&rc);
     if (!q) return rc;
     memcpy(q->host, h, n);
     int wgs = 0;
@@ -296,23 +355,36 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     int rc, wgs = 0;
     Ring* r = ring(&rc);
     if (!r) return rc;
+    const uint8_t* from = (const uint8_t*)d;
     if (n > OUT_BYTES) {
-        const uint8_t* from = (const uint8_t*)d;
-        return run_chunks(r, (uint8_t*)h, n, OUT_BYTES, &s, 1, [&](size_t c, Slot* q, hipStream_t st, size_t bytes) {
-            return launch_copy(from + c * OUT_BYTES, q->host, bytes, 64, nullptr, 0, st, &wgs);
+        Job j{};
+        j.count = (n + CHUNK - 1) / CHUNK;
+        j.down = (uint8_t*)h; j.down_bytes = n; j.down_chunk = CHUNK;
+        return run_chunks(r, j, &s, 1, [&](size_t c, Slot* q, hipStream_t st, int* w) {
+            return launch_copy(from + c * CHUNK, q->host, part(n, CHUNK, c), MAX_WG, q->done, q->seq + 1, st, w);
         });
     }
-    Slot* q = r->need(&rc);
-    if (!q) return rc;
-    if (!(rc = launch_copy(d, q->host, n, MAX_WG, nullptr, 0, s, &wgs)) && !(rc = check_hip(hipStreamSynchronize(s), "hipStreamSynchronize")))
-        memcpy(h, q->host, n);
-    r->release(q);
+    // one part, or two thirds and the rest (where a second slot is free: nobody waits for one while holding one)
+    Slot* half[2] = {r->need(&rc), nullptr};
+    if (!half[0]) return rc;
+    if (n >= TWO_PARTS && !(half[1] = r->take(&rc)) && rc) { r->release(half[0]); return rc; }
+    const size_t first = half[1] ? (n / 3 * 2 + 255) & ~(size_t)255 : n;
+    int words[2] = {0, 0};
+    for (int i = 0; i < (first < n ? 2 : 1) && !rc; i++) {
+        Slot* q = half[i];
+        if (!(rc = launch_copy(from + (i ? first : 0), q->host, i ? n - first : first, MAX_WG, q->done, q->seq + 1, s, &wgs))) { q->seq++; q->wgs = words[i] = wgs; }
+    }
+    for (int i = 0; i < 2 && half[i] && !rc; i++)
+        if (!(rc = await_words(half[i], half[i]->seq, words[i], s))) memcpy((uint8_t*)h + (i ? first : 0), half[i]->host, i ? n - first : first);
+    for (Slot* q : half)
+        if (q) r->release(q);
     return rc;
 }
 
-// nb blocks (bytes each, vals values) of host memory to nb * vals floats of host memory: chunk by chunk the bytes go up, the
-// unpacker writes its floats straight into the slot and a worker copies them out. Two streams, so that the way up of one chunk
-// runs beside the way down of the one before it.
+// nb blocks (bytes each, vals values) of host memory to nb * vals floats of host memory: chunk by chunk the bytes go up, are unpacked
+// on the device, go down into the slot and out of it by a worker. Two streams, so that the way up of one chunk and its unpacking run
+// beside the way down of the one before it. (The unpacker wrote into the slot itself once; the way over device memory costs a chunk
+// 5 of its 40 us, beside the bus, and lets the copy kernel confirm the chunk instead of an event that the workers had to query.)
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, size_t bytes, float* h_out) {
     int rc;
     Ring* r = ring(&rc);
@@ -322,21 +394,31 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
         for (auto& st : r->stream)
             if (!st && (rc = check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate"))) { st = nullptr; return rc; }
     }
-    const size_t per = OUT_BYTES / sizeof(float) / vals;   // blocks of a chunk
-    auto fill = [&](size_t c, Slot* q, hipStream_t s, size_t out_bytes) {
-        const size_t blocks = out_bytes / sizeof(float) / vals, in = blocks * bytes;
-        int err, wgs;
-        if (!q->dev && (err = device_malloc((void**)&q->dev, IN_BYTES, "hipMalloc"))) { q->dev = nullptr; return err; }
-        uint8_t* up = q->host + OUT_BYTES;
-        memcpy(up, h_raw + c * per * bytes, in);
-        if ((err = launch_copy(up, q->dev, in, MAX_WG, nullptr, 0, s, &wgs))) return err;
-        return launch_dequant(type, q->dev, blocks, (float*)q->host, s);
+    const size_t per = CHUNK / sizeof(float) / vals, out_chunk = per * vals * sizeof(float);   // blocks of a chunk, and their floats
+    const size_t n = nb * vals * sizeof(float);
+    auto launch = [&](size_t c, Slot* q, hipStream_t s, int* wgs) {
+        const size_t blocks = nb - c * per < per ? nb - c * per : per;
+        int err;
+        if (!q->dev && (err = device_malloc((void**)&q->dev, SLOT_BYTES, "hipMalloc"))) { q->dev = nullptr; return err; }
+        if ((err = launch_copy(q->host + OUT_BYTES, q->dev + OUT_BYTES, blocks * bytes, MAX_WG, nullptr, 0, s, wgs))) return err;
+        if ((err = launch_dequant(type, q->dev + OUT_BYTES, blocks, (float*)q->dev, s))) return err;
+        return launch_copy(q->dev, q->host, blocks * vals * sizeof(float), MAX_WG, q->done, q->seq + 1, s, wgs);
     };
-    if (nb > per) return run_chunks(r, (uint8_t*)h_out, nb * vals * sizeof(float), OUT_BYTES, r->stream, 2, fill);
+    if (nb > per) {
+        Job j{};
+        j.count = (nb + per - 1) / per;
+        j.up = h_raw; j.up_bytes = nb * bytes; j.up_chunk = per * bytes; j.up_at = OUT_BYTES;
+        j.down = (uint8_t*)h_out; j.down_bytes = n; j.down_chunk = out_chunk;
+        return run_chunks(r, j, r->stream, 2, launch);
+    }
     Slot* q = r->need(&rc);
     if (!q) return rc;
-    const size_t n = nb * vals * sizeof(float);
-    if (!(rc = fill(0, q, r->stream[0], n)) && !(rc = check_hip(hipStreamSynchronize(r->stream[0]), "hipStreamSynchronize"))) memcpy(h_out, q->host, n);
+    int wgs = 0;
+    memcpy(q->host + OUT_BYTES, h_raw, nb * bytes);
+    if (!(rc = launch(0, q, r->stream[0], &wgs))) {
+        q->seq++; q->wgs = wgs;
+        if (!(rc = await_words(q, q->seq, wgs, r->stream[0]))) memcpy(h_out, q->host, n);
+    }
     r->release(q);
     return rc;
 }

@@ -12,9 +12,9 @@ pytestmark = pytest.mark.gpu
 KIB, MIB = 1 << 10, 1 << 20
 
 
-# one byte, tails of the 16-byte units, a slot's way up (640 KiB) and way down (2 MiB) and one byte on either side, more chunks
-# than a copy holds slots (8)
-@pytest.mark.parametrize("n", [1, 3, 15, 17, 4096, 64 * KIB + 5, 640 * KIB - 1, 640 * KIB, 640 * KIB + 1, 2 * MIB - 16, 2 * MIB, 2 * MIB + 1,
+# one byte, tails of the 16-byte units, a slot's way up (640 KiB) and way down (1 MiB) and one byte on either side, more chunks
+# than a copy holds slots (12); a copy back is made in two parts from 96 KiB on (64 + offset bytes are added to n)
+@pytest.mark.parametrize("n", [1, 3, 15, 17, 4096, 64 * KIB + 5, 96 * KIB - 65, 96 * KIB - 64, 96 * KIB + 1, 640 * KIB - 1, 640 * KIB, 640 * KIB + 1, MIB - 65, MIB - 64, MIB - 63, 2 * MIB + 1,
                                6 * MIB + 7, 21 * MIB + 4])
 @pytest.mark.parametrize("offset", [0, 1, 4])
 def test_round_trip(F, n, offset):
@@ -33,7 +33,7 @@ def test_round_trip(F, n, offset):
 
 
 @pytest.mark.parametrize("ty,block", [(8, 32), (12, 256), (14, 256), (7, 32), (39, 32)])
-@pytest.mark.parametrize("values", [32 * 8, 2 * MIB // 4 - 256, 2 * MIB // 4, 2 * MIB // 4 + 256, 9 * 2 * MIB // 4 + 512])
+@pytest.mark.parametrize("values", [32 * 8, MIB // 4 - 256, MIB // 4, MIB // 4 + 256, 2 * MIB // 4 + 256, 17 * MIB // 4 + 512])
 def test_host_dequantization_in_chunks(F, O, ty, block, values):
     from ferric_amd.synth import synth_weights
     raw = synth_weights(ty, 1, values // block * block, values)
