@@ -597,18 +597,21 @@ struct MXF4S {
             hi[j] = lut16x4((D.q[j] >> 4) & 0x0F0F0F0Fu, T0, T1, T2, T3);
         }
         if (D.e >= 252u) {   // a weight of this block may be +-inf: the reference's per-element products
-#pragma unroll 1
+            // (indexed by unrolled loops only: a run-time index would keep the planes of every block in scratch memory)
+#pragma unroll
             for (int m = 0; m < M; m++) {
                 float a = 0.f;
-#pragma unroll 1
-                for (int el = 0; el < 32; el++) {
-                    const int i = el >> 2, sh = 8 * (el & 3);
-                    int v = 0;
 #pragma unroll
-                    for (int p = 0; p < NP; p++) v = v * 256 + (int)(int8_t)(xp[m][0][p][i] >> sh);
-                    const uint32_t kw = el < 16 ? lo[el >> 2] : hi[(el - 16) >> 2];
-                    const float w = (float)(int)(int8_t)(kw >> sh) * d;
-                    a = fmaf(xs[m][0] * (float)v, w, a);
+                for (int i = 0; i < 8; i++) {
+                    const uint32_t kw = i < 4 ? lo[i & 3] : hi[i & 3];
+#pragma unroll 1
+                    for (int sh = 0; sh < 32; sh += 8) {
+                        int v = 0;
+#pragma unroll
+                        for (int p = 0; p < NP; p++) v = v * 256 + (int)(int8_t)(xp[m][0][p][i] >> sh);
+                        const float w = (float)(int)(int8_t)(kw >> sh) * d;
+                        a = fmaf(xs[m][0] * (float)v, w, a);
+                    }
                 }
                 out[m] = a;
             }
@@ -680,6 +683,7 @@ struct GemvParams {
 // row in flight; 151936 x 5120 133 -> 120).
 // (With three activation planes both spill at 168 registers, 152 and 64 bytes a lane: that build keeps eight waves.)
 template <class F> constexpr int max_threads(int M) {
+    if (F::WPL == 32) return M <= 2 ? 1024 : 640;            // (32 weights a lane: two rows fit 108 registers, four 158)
     return M == 1 ? 1024 : (NP == 2 && (F::TYPE == FHIP_Q4_K || F::TYPE == FHIP_Q6_K) ? 640 : 512);
 }
 // Rows in flight per wave, sized so the prefetched rows plus the resident activation planes fit 128 VGPRs
@@ -687,6 +691,18 @@ template <class F> constexpr int max_threads(int M) {
 template <class F> constexpr int rows_in_flight(int M) { return M == 1 ? F::U1 : (NP == 2 && F::TYPE == FHIP_Q6_K ? 1 : 2); }
 // Activation rows one pass can hold in registers.
 template <class F> constexpr int max_m() { return F::WPL == 64 ? 2 : 4; }
+int waves_per_row_group(int NG, int maxw);
+// Waves a workgroup may have, of those its registers allow. A batch of the 32-value formats used eight whatever the row length,
+// which left one row group of five waves on a CU for 2560 or 5120 columns; now as many as fit: us at 24 bits, two | four rows,
+// MXFP4 9728 x 2560 11.4 -> 8.9 | 16.3 -> 13.8, Q4_0 5120 x 5120 9.8 -> 8.9 | 16.6 -> 13.0, Q5_1 30000 x 4096 21.5 -> 19.9 | 41.9 ->
+// 38.9. Eight still where more lose: rows of more than 8192 columns, whose staging every further wave waits for (Q4_0 4096 x 14336
+// 15.5 | 30.8, with sixteen 18.4 | 36.8), and Q8_0 from 28 MB on (30000 x 4096 30.2, with sixteen 35.3).
+template <class F> int wave_limit(int M, size_t cols, size_t wbytes) {
+    const int most = max_threads<F>(M) / 64;
+    if (F::WPL != 32 || M == 1 || most <= 8) return most;
+    if (cols <= 8192 && !(F::TYPE == FHIP_Q8_0 && wbytes >= ((size_t)28 << 20))) return most;
+    return waves_per_row_group((int)((cols / F::WPL + 15) / 16), 8) <= 8 ? 8 : most;
+}
 
 __device__ __forceinline__ uint32_t div_magic(uint32_t n, uint32_t magic) { return magic ? __umulhi(n, magic) : n; }
 
@@ -1201,7 +1217,7 @@ int launch_one_u(const fhip_weight* w, const float* d_x, float* d_y, size_t out_
     p.sel = sel ? *sel : fhip::SelParams{nullptr, 0, 0, 0, 0, 0, 1, 0};
     p.units = (int)(w->cols / F::WPL);
     p.NG = (p.units + 15) / 16;
-    constexpr int MAXW = max_threads<F>(M) / 64;
+    const int MAXW = wave_limit<F>(M, w->cols, wbytes);
     p.RF = full_wave_replicas(p.NG, MAXW);
     int WPR = waves_per_row_group(p.NG, MAXW);
     // Rows per row group (rpg) and row groups per workgroup (G). A CU holds Gcap row groups at once (one
@@ -1229,13 +1245,13 @@ int launch_one_u(const fhip_weight* w, const float* d_x, float* d_y, size_t out_
     // cold weights, one activation row: Q6_K is fastest with 5 - 7 waves per workgroup at every size (5120 columns, 5120 /
     // 20480 / 151936 rows: 8.65 -> 7.83, 19.7 -> 18.5, 118.5 -> 107.0 us; 128256 x 4096: 82.1 -> 73.7 us with six row groups),
     // Q4_K with the fewest whole row groups that make 8 waves (8 - 14) once the weight has 28 MB or more (20480 x 5120 13.9 -> 12.6 us, fused gate|up 34816 x 5120
-    // 20.9 -> 20.2, 28672 x 4096 15.3 -> 14.6) and with all 15 - 16 below that (5120 x 5120: 5.95 us against 6.39). A small
+    // 20.9 -> 20.2, 28672 x 4096 15.3 -> 14.6; Q8_0 likewise, 30000 x 4096 34.3 -> 28.8) and with all 15 - 16 below that (5120 x 5120: 5.95 us against 6.39). A small
     // Q6_K weight whose later rows are requested behind the barrier keeps all its waves (5120 x 5120: 7.08 us against 7.98;
     // twelve of the sixteen one-wave row groups of 4096 columns: 4096 x 4096 5.49 us against 5.98).
     if (M == 1 && p.sel.npairs <= 1) {
         int want = Gcap;
         if (F::TYPE == FHIP_Q6_K) want = late && small ? (WPR == 1 ? 12 : Gcap) : 6 / WPR;
-        else if (F::TYPE == FHIP_Q4_K && !small) want = (8 + WPR - 1) / WPR;
+        else if ((F::TYPE == FHIP_Q4_K || F::TYPE == FHIP_Q8_0) && !small) want = (8 + WPR - 1) / WPR;
         if (want < 1) want = 1;
         // the fused norm holds one 8-value piece of the row per thread
         if (norm) {
@@ -1335,16 +1351,21 @@ int launch_one(const fhip_weight* w, const float* d_x, float* d_y, size_t out_ro
     return launch_one_u<F, M, SWIGLU, rows_in_flight<F>(M)>(w, d_x, d_y, out_rows, s, sel, norm);
 }
 
-// Largest batch width (4, 2, 1, or 0 = shape not covered) whose workgroup fits the wave and LDS limits.
+// Largest batch width (4, 2, 1, 3 for what is left of a batch, or 0 = shape not covered) whose workgroup fits the wave and LDS limits.
 template <class F, bool SWIGLU>
 int max_batch(const fhip_weight* w, size_t left) {
     if (w->cols % F::WPL != 0 || g_force_generic) return 0;
     const int NG = (int)((w->cols / F::WPL + 15) / 16);
-    auto WPRm = [&](int m) { return waves_per_row_group(NG, max_threads<F>(m) / 64); };
     const size_t cap = fhip::device_lds_bytes();
-    if (left >= 4 && max_m<F>() >= 4 && WPRm(4) * 64 <= max_threads<F>(4) && lds_bytes<F, 4, SWIGLU>(w->cols, NG, max_threads<F>(4) / 64 / WPRm(4), 256) <= cap) return 4;
-    if (left >= 2 && WPRm(2) * 64 <= max_threads<F>(2) && lds_bytes<F, 2, SWIGLU>(w->cols, NG, max_threads<F>(2) / 64 / WPRm(2), 256) <= cap) return 2;
-    if (WPRm(1) * 64 <= max_threads<F>(1) && lds_bytes<F, 1, SWIGLU>(w->cols, NG, max_threads<F>(1) / 64 / WPRm(1), 256) <= cap) return 1;
+    auto fits = [&](auto Mc) {
+        constexpr int M = decltype(Mc)::value;
+        const int maxw = wave_limit<F>(M, w->cols, w->nbytes), wpr = waves_per_row_group(NG, maxw);
+        return left >= M && max_m<F>() >= M && wpr <= maxw && lds_bytes<F, M, SWIGLU>(w->cols, NG, maxw / wpr, 256) <= cap;
+    };
+    if (fits(std::integral_constant<int, 4>{})) return 4;
+    if (left == 3 && fits(std::integral_constant<int, 3>{})) return 3;
+    if (fits(std::integral_constant<int, 2>{})) return 2;
+    if (fits(std::integral_constant<int, 1>{})) return 1;
     return 0;
 }
 
@@ -1360,6 +1381,7 @@ int launch_fmt(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y
         int mb = max_batch<F, SWIGLU>(w, rows_x - m0), rc;
         if constexpr (max_m<F>() >= 4) {
             if (mb == 4) { rc = launch_one<F, 4, SWIGLU>(w, x, y, out_rows, s); if (rc != FHIP_OK) return rc; m0 += 4; continue; }
+            if (mb == 3) { rc = launch_one<F, 3, SWIGLU>(w, x, y, out_rows, s); if (rc != FHIP_OK) return rc; m0 += 3; continue; }
         }
         if (mb == 2) rc = launch_one<F, 2, SWIGLU>(w, x, y, out_rows, s);
         else rc = launch_one<F, 1, SWIGLU>(w, x, y, out_rows, s);

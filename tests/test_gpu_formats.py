@@ -284,3 +284,20 @@ def test_the_shape_complete_f32_kernel_still_agrees(F, O):
             assert np.abs(got - want).max() <= dot_bar() * np.abs(want).max(), ty
     finally:
         F._lib.check(lib.fhip_debug_generic_matvec(0))
+
+
+@pytest.mark.parametrize("ty", [8] + [t for t in NEW if t != 13])
+@pytest.mark.parametrize("rows,cols", [(130, 2560), (37, 8192), (21, 8448), (9, 17408)])
+def test_batches_of_the_32_value_formats_have_the_bits_of_single_rows(F, ty, rows, cols):
+    # passes of four, three (what is left of a batch), two and one activation rows, on either side of the row length (8192) from
+    # which a workgroup keeps eight waves; the mat-vec policy keeps Q8_0 off the f16 kernels
+    from ferric_amd.synth import synth_weights
+    w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 77), ty, rows, cols)
+    w.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(5).standard_normal((7, cols)).astype(np.float32)
+    for bits_ in (24, 16):
+        w.matvec_precision(bits_)
+        one = np.concatenate([F.Tensor.from_vec(r, (1, cols)).matmul_q(w).to_vec() for r in x]).reshape(7, rows)
+        for m in (2, 3, 4, 7):
+            got = F.Tensor.from_vec(x[:m].reshape(-1), (m, cols)).matmul_q(w).to_vec().reshape(m, rows)
+            assert np.array_equal(got.view(np.uint32), one[:m].view(np.uint32)), (ty, bits_, m)
