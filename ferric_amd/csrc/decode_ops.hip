@@ -303,33 +303,34 @@ __device__ __forceinline__ RawDims<FMT, DPL> fetch_dims_q(const uint32_t* __rest
     }
     return r;
 }
+// one code word's four dims, scale and minimum as f32
+template <int FMT>
+__device__ __forceinline__ void expand_dims_f(uint32_t code, int shift, float d, float m, float (&r)[4]) {   // shift: 0 or 4, the 4-bit formats' half
+#pragma clang fp contract(off)
+    if constexpr (FMT == FHIP_KVQ_Q8_0) {
+        r[0] = (float)(int8_t)(code & 255u) * d;
+        r[1] = (float)(int8_t)((code >> 8) & 255u) * d;
+        r[2] = (float)(int8_t)((code >> 16) & 255u) * d;
+        r[3] = (float)(int8_t)(code >> 24) * d;
+    } else {
+        const uint32_t word = code >> shift;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float n = (float)((word >> (8 * i)) & 15u);
+            if constexpr (FMT == FHIP_KVQ_Q4_0) r[i] = (n - 8.0f) * d;
+            else { const float t = n * d; r[i] = t + m; }
+        }
+    }
+}
 template <int FMT, int DPL>
 __device__ __forceinline__ void expand_dims_q(const RawDims<FMT, DPL>& raw, int col, float (&r)[DPL]) {
-#pragma clang fp contract(off)
-    const int j = col & 31;
-    if constexpr (FMT == FHIP_KVQ_Q8_0) {
-        const float d = __half2float(__ushort_as_half(raw.d));
+    const float d = __half2float(__ushort_as_half(raw.d)), m = __half2float(__ushort_as_half(raw.m));
 #pragma unroll
-        for (int w = 0; w < DPL / 4; w++) {
-            const uint32_t word = raw.w[w];
-            r[4 * w] = (float)(int8_t)(word & 255u) * d;
-            r[4 * w + 1] = (float)(int8_t)((word >> 8) & 255u) * d;
-            r[4 * w + 2] = (float)(int8_t)((word >> 16) & 255u) * d;
-            r[4 * w + 3] = (float)(int8_t)(word >> 24) * d;
-        }
-    } else {
-        const int shift = j < 16 ? 0 : 4;
-        const float d = __half2float(__ushort_as_half(raw.d)), m = __half2float(__ushort_as_half(raw.m));
+    for (int w = 0; w < DPL / 4; w++) {
+        float v[4];
+        expand_dims_f<FMT>(raw.w[w], ((col + 4 * w) & 31) < 16 ? 0 : 4, d, m, v);
 #pragma unroll
-        for (int w = 0; w < DPL / 4; w++) {
-            const uint32_t word = raw.w[w] >> shift;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float n = (float)((word >> (8 * i)) & 15u);
-                if constexpr (FMT == FHIP_KVQ_Q4_0) r[4 * w + i] = (n - 8.0f) * d;
-                else { const float t = n * d; r[4 * w + i] = t + m; }
-            }
-        }
+        for (int i = 0; i < 4; i++) r[4 * w + i] = v[i];
     }
 }
 
@@ -623,6 +624,253 @@ __global__ __launch_bounds__(COMBINE_THREADS) void attn_combine_kernel(const flo
     }
 }
 
+// ---------------------------------------------------------------- the same over a long block-quantized cache, on the matrix cores
+// All gq query heads of a KV head at once. A wave takes 32 keys at a time, in two tiles of 16.
+//   Scores: v_mfma_f32_16x16x32_bf16 with the codes of one block of 32 dims as the A operand (16 keys; whole numbers of at most eight
+//   bits, exact in bf16) and the query's 32 dims as the B operand (16 queries, gq of them real), cut into three bf16 values whose sum
+//   is the f32 query. Three instructions give the block's sum in f32; the block's scale multiplies it. Lane n + 16 g ends up with keys
+//   4 g .. 4 g + 3 of query n, so a query's maximum and sum are register operations and two exchanges.
+//   Values: f32 on v_mfma_f32_16x16x4: register r of a tile's probabilities is a B operand as it stands (four keys, 4 g + r, of query n);
+//   the A operand is dim 4 n + i of those keys, from a lane's four dims of a row of 64, dequantized as above.
+// Scales come one row a lane and go round through LDS (the wave's own part of it), the cut queries are shared there. The next round's
+// key codes are requested when the scores are done. The waves of a workgroup meet in LDS as above. A launch costs the same for any
+// number of query heads up to the eight taken (an instruction has room for 16).
+// What bounds it: three waves per SIMD at head size 128 (168 registers), each waiting for its rows and then issuing 24 + 64 matrix and
+// some 450 other instructions a round, about 7 us a round of the 3 at 32768 keys. With the combine launch, us, this | the kernel above,
+// 8 KV heads, 32768 Q8_0 keys: head size 128 (71 MB), 8 query heads each 39.5 | 59.4; head size 64, 5: 25.2 | 33.2, 8: 24.5 | 45.4.
+// Error against f64 (2-norm, relative, six draws) at those shapes 2.7e-7 | 2.8e-7, 2.4e-7 .. 2.6e-7 | 2.5e-7 .. 2.7e-7. Q4_1 is left to the kernel
+// above: the minimum as a product of its own cost 2 % more error. Tried: values on the 4 x 4 x 1 instruction (the same times, an
+// instantiation per group size), scores on it as well (slower by 2 us: it issues once in some 20 cycles), 64 keys a round (spills, +17 us).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+union Frag { uint32_t w[4]; bf16x8 v; };
+// the upper halves of two f32: two bf16 (exact where the lower halves are zero)
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
+
+// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16 (4-bit formats: less 8)
+template <int FMT>
+__device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) {
+    Frag f;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        float v[4];
+        if constexpr (FMT == FHIP_KVQ_Q8_0) {
+            v[0] = (float)(int8_t)(w[i] & 255u); v[1] = (float)(int8_t)((w[i] >> 8) & 255u);
+            v[2] = (float)(int8_t)((w[i] >> 16) & 255u); v[3] = (float)(int8_t)(w[i] >> 24);
+        } else {
+            const uint32_t x = (w[i] >> shift) & 0x0F0F0F0Fu;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = (float)((x >> (8 * j)) & 255u) - 8.0f;
+        }
+        f.w[2 * i] = upper_halves(v[0], v[1]);
+        f.w[2 * i + 1] = upper_halves(v[2], v[3]);
+    }
+    return f.v;
+}
+
+constexpr int LONG_WAVES = 6, LONG_KEYS = 32;   // waves of a workgroup, keys a wave takes at a time
+template <int HD, int FMT>
+__global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
+                                                                           const uint32_t* __restrict__ len_dev, float scale, int splits,
+                                                                           uint32_t window, float softcap, float* __restrict__ part, int gq) {   // gq: query heads per KV head, at most 8
+    constexpr int NB = HD / 32, NT = LONG_KEYS / 16, NH = HD / 64;      // blocks of a row, tiles of 16 keys, 64-dim parts of a row
+    constexpr int CW = FMT == FHIP_KVQ_Q8_0 ? 8 : 4;                    // code words of a block
+    static_assert(FMT == FHIP_KVQ_Q8_0 || FMT == FHIP_KVQ_Q4_0, "");
+    __shared__ float sm_m[LONG_WAVES][8], sm_l[LONG_WAVES][8];
+    __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][8][HD + 4];    // rows four banks apart
+    __shared__ __attribute__((aligned(16))) float sm_d[LONG_WAVES][NB][64];   // rows 0 .. 31 the keys' scales, 32 .. 63 the values'
+    __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of query n at lane n + 16 g, three bf16 each
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int kvh = blockIdx.x, split = blockIdx.y, head0 = kvh * gq;
+    uint32_t len = len_dev ? *len_dev + 1u : len_host;
+    if (len > len_host) len = len_host;
+    const uint32_t first = (window > 0 && window < len) ? len - window : 0u;
+    const uint32_t per = (len - first + splits - 1) / splits;
+    const uint32_t k0 = first + (uint32_t)split * per, k1 = min(len, k0 + per);
+    const int nblk = n_kv * NB;
+
+    uint32_t kw[NT][NB][2], sc[NB / 2];
+    auto request_k = [&](uint32_t kt) {
+        const uint32_t last = k1 - 1u - kt;                             // rows past the split re-read its last row and count nothing
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const size_t b = (size_t)(kt + min((uint32_t)(16 * t + n), last)) * nblk + (size_t)kvh * NB;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const uint2 v = *(const uint2*)(qc.k_codes + (b + j) * CW + 2 * (g & (CW / 2 - 1)));
+                kw[t][j][0] = v.x; kw[t][j][1] = v.y;
+            }
+        }
+        const size_t b = ((size_t)(kt + min((uint32_t)(lane & 31), last)) * nblk + (size_t)kvh * NB);
+        const uint32_t* sp = (const uint32_t*)((lane < 32 ? qc.k_scales : qc.v_scales) + b);
+#pragma unroll
+        for (int i = 0; i < NB / 2; i++) sc[i] = sp[i];
+    };
+    uint32_t kt = k0 + (uint32_t)(LONG_KEYS * wave);
+    if (kt < k1) request_k(kt);
+
+    if (wave < NB) {                                                    // wave j cuts the queries' block j up for all
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = 0.f;
+        if (n < gq) load_dims<8>(q + ((size_t)head0 + n) * HD + 32 * wave + 8 * g, x);
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            sm_q[wave][t][lane] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);   // exact
+        }
+    }
+    __syncthreads();
+
+    const int vblk = n >> 3, word = n & (CW - 1), shift = (n & 7) < 4 ? 0 : 4;               // of dims 4 n .. 4 n + 3 of a 64-dim part
+    const uint32_t vrow = (uint32_t)(4 * g) * (uint32_t)nblk + (uint32_t)vblk;              // blocks from a tile's first to the lane's
+    const uint32_t vco = (vrow * CW + (uint32_t)word) * 4u;
+
+    f32x4 run[NH][4];                       // [part][i]: dims 64 part + 16 g + 4 r + i of query n
+    float m = -3.0e38f, l = 0.f;            // of query n
+#pragma unroll
+    for (int h = 0; h < NH; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) run[h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (; kt < k1; kt += LONG_KEYS * LONG_WAVES) {
+        const uint32_t last = k1 - 1u - kt;
+        uint32_t vw[NT][4][NH];                 // [tile][r][part]: dims 4 n .. + 3 of the part, key 16 t + 4 g + r
+        if (last >= LONG_KEYS - 1u) {
+            // a lane's own part of the address is the same for every row (and fits 32 bits); the rest is the wave's
+            const char* vc = (const char*)(qc.v_codes + ((size_t)kt * nblk + (size_t)kvh * NB) * CW);
+#pragma unroll
+            for (int i = 0; i < NT * 4 * NH; i++) {
+                const int t = i / (4 * NH), r = i / NH % 4, h = i % NH;
+                vw[t][r][h] = *(const uint32_t*)(vc + ((size_t)(16 * t + r) * nblk + 2 * h) * (CW * 4) + vco);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NT * 4; i++) {
+                uint32_t mine = (uint32_t)(4 * g);
+                asm volatile("" : "+v"(mine));                          // worked out here: kept from round to round these are eight more registers
+                const size_t b = (size_t)(kt + min(mine + (uint32_t)(16 * (i / 4) + i % 4), last)) * nblk + (size_t)kvh * NB + (size_t)vblk;
+#pragma unroll
+                for (int h = 0; h < NH; h++) vw[i / 4][i % 4][h] = qc.v_codes[(b + 2 * h) * CW + word];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NB / 2; i++) {
+            const float lo = __half2float(__ushort_as_half((uint16_t)sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(sc[i] >> 16)));
+            sm_d[wave][2 * i][lane] = lo;
+            sm_d[wave][2 * i + 1][lane] = hi;
+        }
+        asm volatile("" ::: "memory");          // a wave's LDS accesses complete in order; this keeps the compiler's in order too
+
+        float p[NT][4];                         // [tile][r]: key 16 t + 4 g + r of query n
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[t][r] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            Frag qf[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) { const uint4 w = sm_q[j][i][lane]; qf[i].w[0] = w.x; qf[i].w[1] = w.y; qf[i].w[2] = w.z; qf[i].w[3] = w.w; }
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const bf16x8 c = codes_bf16<FMT>(kw[t][j], 4 * (g >> 1));
+                f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 2; i >= 0; i--) a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, qf[i].v, a, 0, 0, 0);
+                const f32x4 d = *(const f32x4*)&sm_d[wave][j][16 * t + 4 * g];
+#pragma unroll
+                for (int r = 0; r < 4; r++) p[t][r] = fmaf(d[r], a[r], p[t][r]);
+            }
+            asm volatile("" ::: "memory");      // a block at a time: the operands of all of them do not fit the registers
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kt + LONG_KEYS * LONG_WAVES < k1) request_k(kt + LONG_KEYS * LONG_WAVES);
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[t][r] *= scale;
+        if (softcap > 0.f) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) p[t][r] = softcap * tanhf(p[t][r] / softcap);
+        }
+        const int lim = (int)min(last, (uint32_t)LONG_KEYS);
+        float top = -3.0e38f;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (4 * g > lim - (16 * t + r)) p[t][r] = -3.0e38f;
+                top = fmaxf(top, p[t][r]);
+            }
+        top = fmaxf(top, __shfl_xor(top, 16));
+        top = fmaxf(top, __shfl_xor(top, 32));
+        const float m_new = fmaxf(m, top), corr = __expf(m - m_new);
+        float ps[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[t][r] = 4 * g > lim - (16 * t + r) ? 0.f : __expf(p[t][r] - m_new);
+            ps[t] = (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
+        }
+        l = fmaf(l, corr, ps[0] + ps[1]);
+        m = m_new;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int h = 0; h < NH; h++) {
+                const f32x4 d = *(const f32x4*)&sm_d[wave][2 * h + vblk][32 + 16 * t + 4 * g];
+                f32x4 acc[4];                   // the tile's sums start at zero: chains of 16 keys, then one addition
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float v[4];
+                    expand_dims_f<FMT>(vw[t][r][h], shift, d[r], 0.f, v);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], p[t][r], acc[i], 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) run[h][i][r] = t == 0 ? fmaf(run[h][i][r], corr, acc[i][r]) : run[h][i][r] + acc[i][r];
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (lane < gq) { sm_m[wave][lane] = m; sm_l[wave][lane] = l; }
+    if (n < gq) {
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                *(f32x4*)&sm_acc[wave][n][64 * h + 16 * g + 4 * r] = f32x4{run[h][0][r], run[h][1][r], run[h][2][r], run[h][3][r]};
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < gq * HD; idx += 64 * LONG_WAVES) {
+        const int h = idx / HD, d = idx % HD;
+        float M = sm_m[0][h];
+#pragma unroll
+        for (int w = 1; w < LONG_WAVES; w++) M = fmaxf(M, sm_m[w][h]);
+        float L = 0.f, A = 0.f;
+#pragma unroll
+        for (int w = 0; w < LONG_WAVES; w++) {
+            const float f = __expf(sm_m[w][h] - M);
+            L = fmaf(sm_l[w][h], f, L);
+            A = fmaf(sm_acc[w][h][d], f, A);
+        }
+        float* pp = part + ((size_t)(head0 + h) * splits + split) * (HD + 2);
+        pp[d] = A;
+        if (d == 0) { pp[HD] = M; pp[HD + 1] = L; }
+    }
+}
+
 template <int G>
 int launch_attn_g(int hd, dim3 grid, hipStream_t s, const float* q, const float* K, const float* V, int n_kv, uint32_t len, const uint32_t* d_len,
                   float scale, int splits, uint32_t window, float softcap, float* part, float* out, int gq = G) {
@@ -658,6 +906,22 @@ int launch_attn_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, con
         case 8: return launch_attn_kvq_g<8, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
         default: return fhip::set_error(FHIP_ERR_SHAPE, "decode_attention: %d query heads per KV head (1..=8 supported)", g);
     }
+}
+
+// Which launches take it: the kernel above costs less for few query heads a KV head. A decode step of four layers (d 2048), four tokens, us,
+// this | that: 8 KV heads, head size 128, 32768 keys, 8 query heads each Q8_0 1393 | 1596, 5: 1364 | 1337, Q4_0 1420 | 1371; 4 KV heads, 8, 9000 keys
+// Q4_0 1012 | 1044; head size 64, 8: 32768 keys Q4_0 1079 | 1350, 5: 10000 keys Q8_0 848 | 881, 4 KV heads, 4: 6000 keys 837 | 840.
+// Key codes are read eight bytes at a time; a lane's offset inside a round's rows is kept in 32 bits (n_kv).
+bool attn_long_takes(int fmt, int g, int hd, int n_kv, const uint32_t* k_codes) {
+    if (fmt == FHIP_KVQ_Q4_1 || g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
+    return g >= (hd == 64 ? 5 : 6);
+}
+template <int FMT>
+void launch_attn_long_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, const QCache& qc, int n_kv, uint32_t len, const uint32_t* d_len,
+                          float scale, int splits, uint32_t window, float softcap, float* part) {
+    const dim3 wg(64 * LONG_WAVES);
+    if (hd == 64) hipLaunchKernelGGL((attn_long_kvq_kernel<64, FMT>), grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g);
+    else hipLaunchKernelGGL((attn_long_kvq_kernel<128, FMT>), grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g);
 }
 
 template <int G>
@@ -870,7 +1134,14 @@ int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes
     const int splits = mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "decode_attention: this cache length needs the workspace");
     const dim3 grid((unsigned)n_kv, (unsigned)splits);
-    if (mid) {
+    if (!mid && splits > 1 && attn_long_takes(fmt, g, hd, n_kv, k_codes)) {
+        rc = FHIP_OK;
+        switch (fmt) {
+            case FHIP_KVQ_Q8_0: launch_attn_long_kvq<FHIP_KVQ_Q8_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws); break;
+            case FHIP_KVQ_Q4_0: launch_attn_long_kvq<FHIP_KVQ_Q4_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws); break;
+            default: return set_error(FHIP_ERR_ARG, "decode_attention: unknown KV format %d", fmt);
+        }
+    } else if (mid) {
         const dim3 lin((unsigned)((n_kv * splits + 7) / 8 * 8 * g), 1);
         switch (fmt) {
             case FHIP_KVQ_Q8_0: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q8_0>(hd, lin, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out, -g); break;

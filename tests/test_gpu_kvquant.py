@@ -213,6 +213,35 @@ def test_attention_over_the_blocks_is_attention_over_the_dequantized_rows(F, Q, 
     assert b"head_dim must be 64 or 128" in lib.fhip_last_error()
 
 
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("nh,nkv,hd,rows,lengths", [
+    (5, 1, 64, 5121, (5121, 97, 1)),              # the smallest group and cache that take the kernel; splits of a few keys, of one, of none
+    (16, 2, 64, 6150, (6150, 5000)), (10, 2, 64, 5200, (5200,)), (6, 1, 128, 5121, (5121, 33)), (8, 1, 128, 7000, (7000, 6999)),
+    (7, 1, 128, 16384, (16384, 9001))])
+def test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, hd, rows, lengths):
+    """Group sizes and lengths at the edges of the long-cache kernel's rounds (32 keys a wave, six waves, 64 or 256 splits), with the
+    length on the device, a window and a softcap, against the oracle over the oracle's dequantized rows: the f32 attention's 1e-5
+    of the largest output. Large scores (a query of magnitude 4) sharpen the softmax, where an error in a score would show."""
+    from ferric_amd import decode as X
+    from oracle import decode_oracle as D
+    rng = np.random.default_rng(90 + fmt)
+    width = nkv * hd
+    k = (rng.standard_normal((rows, width)) + 0.5).astype(np.float32)
+    v = rng.standard_t(3, (rows, width)).astype(np.float32)
+    q = (rng.standard_normal((1, nh * hd)) * np.where(np.arange(nh * hd) < hd, 4.0, 1.0)).astype(np.float32)
+    kq, vq = (Q.QKvCache.from_tensor(F.Tensor.from_vec(x, x.shape), fmt) for x in (k, v))
+    kr, vr = K.roundtrip(k, rows, width, fmt), K.roundtrip(v, rows, width, fmt)
+    qt = F.Tensor.from_vec(q, q.shape)
+    word = F.Tensor(F.DeviceBuffer(4), (1,), np.uint32)
+    for n in lengths:
+        last = np.array([n - 1], np.uint32)
+        F._lib.check(F._lib.load().fhip_memcpy_h2d(word.buf.ptr, last.ctypes.data, 4, None))
+        for window, cap in ((0, 0.0), (301, 20.0)):
+            got = X.decode_attention_kvq(qt, kq, vq, nh, nkv, length=rows, last_pos=word, window=window, softcap=cap).to_vec()
+            want = D.decode_attention(q[0], kr[:n], vr[:n], nh, nkv, window, cap).reshape(-1)
+            assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max(), (n, window)
+
+
 def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
     rng = np.random.default_rng(80)
     t, width, cap = 5, 256, 16
