@@ -138,12 +138,14 @@ __global__ void geglu_kernel(const float* __restrict__ gu, size_t n, size_t d, f
 // Pair c of a head rotates by angle pos * base^(-2c / n_rot) (times freq_scale[c]); partners are (c, c + n_rot/2) in the
 // split-half layout and (2c, 2c + 1) interleaved; dims >= n_rot pass through (lib.rs:2118-2162, 2094-2116). The inverse
 // frequency is evaluated in f64 and rounded to f32 once, the angle is the f32 product the reference forms.
-__device__ __forceinline__ float rope_inv_freq(int c, int n_rot, float base, const float* freq_scale) {
-    float inv = (float)exp(-2.0 * (double)c / (double)n_rot * log((double)base));
+// rate = -2 / n_rot * log(base) is the host's: the division and the logarithm in f64 were most of what a lane did for its pair.
+__device__ __forceinline__ float rope_inv_freq(int c, double rate, const float* freq_scale) {
+    const float inv = (float)exp((double)c * rate);
     return freq_scale ? inv * freq_scale[c] : inv;
 }
+inline double rope_rate(int n_rot, float base) { return n_rot > 0 ? -2.0 / (double)n_rot * log((double)base) : 0.0; }
 
-__global__ void rope_kernel(const float* __restrict__ x, size_t src_row_stride, int t, int heads, int hd, int n_rot, float base,
+__global__ void rope_kernel(const float* __restrict__ x, size_t src_row_stride, int t, int heads, int hd, int n_rot, double rate,
                             const uint32_t* __restrict__ pos, uint32_t pos_off, const float* __restrict__ freq_scale, int interleaved,
                             float* __restrict__ out) {
     const int half = n_rot / 2, per_head = hd - half;   // work items per head: the pairs, then the pass-through tail
@@ -155,7 +157,7 @@ __global__ void rope_kernel(const float* __restrict__ x, size_t src_row_stride, 
     if (w >= half) { const int c = n_rot + (w - half); oi[c] = xi[c]; return; }
     const int c = w;
     const float p = (float)(pos ? pos[i] : pos_off + (uint32_t)i);
-    const float ang = p * rope_inv_freq(c, n_rot, base, freq_scale);
+    const float ang = p * rope_inv_freq(c, rate, freq_scale);
     float sn, cs;
     sincosf(ang, &sn, &cs);
     const int p0 = interleaved ? 2 * c : c, p1 = interleaved ? 2 * c + 1 : c + half;
@@ -181,7 +183,8 @@ struct QkvPostParams {
     float* v_cache;
     int t, n_head, n_kv, hd, n_rot, interleaved;
     uint32_t cap;
-    float eps, base;
+    float eps;
+    double rate;             // rope_rate(n_rot, base)
     int kv_packed;           // != 0: k_cache / v_cache are packed [t, n_kv * hd] outputs, row i for token i (cap is not looked at)
 };
 
@@ -218,7 +221,7 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvPostParams p) {
     auto val = [&](int j) { float v = bias ? x[j] + bias[j] : x[j]; return nw ? v * inv * nw[j] : v; };
     const int half = p.n_rot / 2;
     for (int c = lane; c < half; c += 64) {
-        const float ang = (float)pos * rope_inv_freq(c, p.n_rot, p.base, p.freq_scale);
+        const float ang = (float)pos * rope_inv_freq(c, p.rate, p.freq_scale);
         float sn, cs;
         sincosf(ang, &sn, &cs);
         const int p0 = p.interleaved ? 2 * c : c, p1 = p.interleaved ? 2 * c + 1 : c + half;
@@ -227,6 +230,65 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvPostParams p) {
         dst[p1] = x2 * cs + x1 * sn;
     }
     for (int j = p.n_rot + lane; j < p.hd; j += 64) dst[j] = val(j);
+}
+
+// The same operations for heads of 128 dims rotated whole in the split-half layout, the common case: a lane's two values are a pair,
+// so a head is read once and nothing is read again. A wave takes HPW consecutive heads of a token, requests them all before the first
+// is worked on, and works the token's angles out once for them. The one-head form above paid, per head, three round trips in a row (the
+// squares, the pair again, the weights) and the f64 exponential: 509 rows of 40 + 8 + 8 heads (29 MB) 19.2 -> 10.2 us.
+template <int HPW>
+__global__ __launch_bounds__(256) void qkv_post128_kernel(QkvPostParams p) {
+    const int lane = threadIdx.x & 63;
+    const int per_tok = p.n_head + 2 * p.n_kv, waves_per_tok = (per_tok + HPW - 1) / HPW;
+    const size_t wid = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wid >= (size_t)p.t * waves_per_tok) return;
+    const int i = (int)(wid / waves_per_tok), h0 = (int)(wid % waves_per_tok) * HPW;
+    const float* x = p.qkv + ((size_t)i * per_tok + h0) * 128 + lane;
+    float a[HPW], b[HPW];
+#pragma unroll
+    for (int j = 0; j < HPW; j++) {
+        const int o = h0 + j < per_tok ? 128 * j : 0;
+        a[j] = x[o];
+        b[j] = x[o + 64];
+    }
+    const uint32_t pos = p.pos[i];
+    float wq[2] = {1.f, 1.f}, wk[2] = {1.f, 1.f};
+    if (p.q_norm) { wq[0] = p.q_norm[lane]; wq[1] = p.q_norm[lane + 64]; }
+    if (p.k_norm) { wk[0] = p.k_norm[lane]; wk[1] = p.k_norm[lane + 64]; }
+    if (p.bias) {
+        const float* bias = p.bias + (size_t)h0 * 128 + lane;
+#pragma unroll
+        for (int j = 0; j < HPW; j++) {
+            const int o = h0 + j < per_tok ? 128 * j : 0;
+            a[j] += bias[o];
+            b[j] += bias[o + 64];
+        }
+    }
+    float sn = 0.f, cs = 1.f;
+    if (h0 < p.n_head + p.n_kv) sincosf((float)pos * rope_inv_freq(lane, p.rate, p.freq_scale), &sn, &cs);
+    const bool stored = p.kv_packed || pos < p.cap;              // a position past the cache is dropped, never written out of bounds
+    const size_t kv_row = (p.kv_packed ? (size_t)i : (size_t)pos) * p.n_kv;
+#pragma unroll
+    for (int j = 0; j < HPW; j++) {
+        const int h = h0 + j;
+        if (h >= per_tok || (h >= p.n_head && !stored)) return;
+        const bool value = h >= p.n_head + p.n_kv, key = !value && h >= p.n_head;
+        float* dst = value ? p.v_cache + (kv_row + (h - p.n_head - p.n_kv)) * 128
+                           : key ? p.k_cache + (kv_row + (h - p.n_head)) * 128 : p.q_out + ((size_t)i * p.n_head + h) * 128;
+        float x1 = a[j], x2 = b[j];
+        if (!value) {
+            if (key ? p.k_norm : p.q_norm) {
+                const float inv = 1.0f / sqrtf(wave_sum(fmaf(x2, x2, x1 * x1)) / 128.0f + p.eps);
+                x1 = x1 * inv * (key ? wk[0] : wq[0]);
+                x2 = x2 * inv * (key ? wk[1] : wq[1]);
+            }
+            const float y1 = x1 * cs - x2 * sn, y2 = x2 * cs + x1 * sn;
+            x1 = y1;
+            x2 = y2;
+        }
+        dst[lane] = x1;
+        dst[lane + 64] = x2;
+    }
 }
 
 // K and V rows of t tokens into their caches at the tokens' positions, one launch (lib.rs:1379-1398).
@@ -458,7 +520,7 @@ __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typ
             }
             auto val = [&](int e) { float v = bias ? x[e] + bias[e] : x[e]; return nw ? v * inv * nw[e] : v; };
             for (int c = lane; c < half; c += 64) {
-                const float ang = (float)pos * rope_inv_freq(c, fp.n_rot, fp.base, fp.freq_scale);
+                const float ang = (float)pos * rope_inv_freq(c, fp.rate, fp.freq_scale);
                 float sn, cs;
                 sincosf(ang, &sn, &cs);
                 const int p0 = fp.interleaved ? 2 * c : c, p1 = fp.interleaved ? 2 * c + 1 : c + half;
@@ -992,7 +1054,7 @@ int launch_rope(const float* x, size_t src_row_stride, size_t t, int heads, int 
     size_t n = t * (size_t)heads * (size_t)(hd - n_rot / 2);
     size_t grid = (n + 255) / 256;
     if (t > 0x7FFFFFFFull || grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rope: too many rows for one launch");
-    hipLaunchKernelGGL(rope_kernel, dim3((unsigned)grid), dim3(256), 0, s, x, src_row_stride, (int)t, heads, hd, n_rot, base, d_pos, pos_off,
+    hipLaunchKernelGGL(rope_kernel, dim3((unsigned)grid), dim3(256), 0, s, x, src_row_stride, (int)t, heads, hd, n_rot, rope_rate(n_rot, base), d_pos, pos_off,
                        freq_scale, interleaved, out);
     return check_hip(hipGetLastError(), "rope launch");
 }
@@ -1005,10 +1067,18 @@ int launch_qkv_post(const float* qkv, const float* bias, const float* q_norm, co
     p.qkv = qkv; p.bias = bias; p.q_norm = q_norm; p.k_norm = k_norm; p.pos = d_pos; p.freq_scale = freq_scale;
     p.q_out = q_out; p.k_cache = k_cache; p.v_cache = v_cache;
     p.t = (int)t; p.n_head = n_head; p.n_kv = n_kv; p.hd = hd; p.n_rot = n_rot; p.interleaved = interleaved;
-    p.cap = (uint32_t)cap; p.eps = eps; p.base = base; p.kv_packed = kv_packed ? 1 : 0;
-    size_t waves = t * (size_t)(n_head + 2 * n_kv), grid = (waves + 3) / 4;
-    if (t > 0x7FFFFFFFull || grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post: too many rows for one launch");
-    hipLaunchKernelGGL(qkv_post_kernel, dim3((unsigned)grid), dim3(256), 0, s, p);
+    p.cap = (uint32_t)cap; p.eps = eps; p.rate = rope_rate(n_rot, base); p.kv_packed = kv_packed ? 1 : 0;
+    const size_t per_tok = (size_t)(n_head + 2 * n_kv);
+    if (t > 0x7FFFFFFFull || (t * per_tok + 3) / 4 > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post: too many rows for one launch");
+    // eight heads a wave once that leaves the CUs some four waves each; a token or two needs all the waves it can have
+    const size_t hpw = t * ((per_tok + 7) / 8) >= 4 * (size_t)device_cus() ? 8 : 1;
+    if (hd == 128 && n_rot == 128 && !interleaved) {
+        const dim3 grid((unsigned)((t * ((per_tok + hpw - 1) / hpw) + 3) / 4));
+        if (hpw == 8) hipLaunchKernelGGL(qkv_post128_kernel<8>, grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL(qkv_post128_kernel<1>, grid, dim3(256), 0, s, p);
+    } else {
+        hipLaunchKernelGGL(qkv_post_kernel, dim3((unsigned)((t * per_tok + 3) / 4)), dim3(256), 0, s, p);
+    }
     return check_hip(hipGetLastError(), "qkv_post launch");
 }
 
@@ -1182,7 +1252,7 @@ int launch_qkv_post_attention(const float* qkv, const float* bias, const float* 
     fp.qkv = qkv; fp.bias = bias; fp.q_norm = q_norm; fp.k_norm = k_norm; fp.pos = d_pos; fp.freq_scale = freq_scale;
     fp.q_out = nullptr; fp.k_cache = k_cache; fp.v_cache = v_cache;
     fp.t = 1; fp.n_head = n_head; fp.n_kv = n_kv; fp.hd = hd; fp.n_rot = n_rot; fp.interleaved = interleaved ? 1 : 0;
-    fp.cap = (uint32_t)cap; fp.eps = eps; fp.base = base; fp.kv_packed = 0;
+    fp.cap = (uint32_t)cap; fp.eps = eps; fp.rate = rope_rate(n_rot, base); fp.kv_packed = 0;
     const float scale = 1.0f / sqrtf((float)hd);
     const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;
     if (g > 8) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention: %d query heads per KV head (1..=8 supported)", g);

@@ -202,6 +202,34 @@ def test_attention_properties_at_a_32k_context(F, X):
     assert np.abs(flat - want).max() <= 1e-5 * np.abs(want).max() + 1e-6
 
 
+@pytest.mark.parametrize("t,nh,nkv,norms", [(513, 10, 2, True), (1100, 5, 1, False), (205, 32, 4, True)])
+def test_qkv_post_of_many_rows_has_the_bits_of_single_rows(F, X, D, t, nh, nkv, norms):
+    """Eight heads a wave (a last group that is not full; groups that hold query, key and value heads at once) against one head a wave,
+    with positions past the cache among the rows: they are dropped by both. One row also against the oracle."""
+    rng = np.random.default_rng(t)
+    lib, hd, cap = F._lib.load(), 128, 700
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    qkv = rng.standard_normal((t, (nh + 2 * nkv) * hd)).astype(np.float32)
+    bias, qn, kn = (rng.standard_normal(n).astype(np.float32) for n in ((nh + 2 * nkv) * hd, hd, hd))
+    pos = (rng.permutation(t) + max(0, cap - t + 3)).astype(np.uint32)                # distinct; some at or past the capacity
+    bt, qnt, knt = (T(bias), T(qn), T(kn)) if norms else (None, None, None)
+    P = lambda x: x.buf.ptr if x is not None else None
+    pt, qt = F.Tensor(F.DeviceBuffer(4 * t), (t,), np.uint32), T(qkv)
+    F._lib.check(lib.fhip_memcpy_h2d(pt.buf.ptr, pos.ctypes.data, 4 * t, None))
+    out = []
+    for rows in (t, 1):
+        qo, kc, vc = (T(np.full(sh, 7.0, np.float32)) for sh in ((t, nh * hd), (cap, nkv * hd), (cap, nkv * hd)))
+        for i in range(0, t, rows):
+            F._lib.check(lib.fhip_qkv_post(qt.buf.ptr.value + 4 * i * qkv.shape[1], P(bt), P(qnt), P(knt), pt.buf.ptr.value + 4 * i, None, rows, nh, nkv, hd, hd, 0,
+                                           1e-6, 1e6, qo.buf.ptr.value + 4 * i * nh * hd, kc.buf.ptr, vc.buf.ptr, cap, None))
+        out.append([x.to_vec() for x in (qo, kc, vc)])
+    for a, b in zip(*out):
+        assert np.array_equal(bits(a), bits(b))
+    i = t // 2
+    wq, _, _ = D.qkv_post(qkv[i:i + 1], bias if norms else None, qn if norms else None, kn if norms else None, pos[i:i + 1], nh, nkv, hd, 1e-6, 1e6, interleaved=False)
+    assert close(out[0][0].reshape(t, nh * hd)[i], wq.reshape(-1), 1e-5)
+
+
 def test_qkv_post_fuses_bias_norm_rope_and_append(F, X, D):
     rng = np.random.default_rng(3)
     lib = F._lib.load()
