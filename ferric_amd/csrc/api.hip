@@ -786,6 +786,15 @@ int fhip_add_rmsnorm(const float* d_a, const float* d_b, const float* d_weight, 
     return fhip::launch_rmsnorm(d_a, d_b, d_weight, rows, d, eps, d_sum, d_norm, (hipStream_t)stream);
 }
 
+int fhip_add_rmsnorm_bf16(const float* d_a, const float* d_b, const float* d_weight, size_t rows, size_t d, float eps, float* d_sum,
+                          uint16_t* d_norm_bf16, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (rows == 0 || d == 0) return FHIP_OK;
+    if (!d_a || !d_weight || !d_norm_bf16 || (d_b && !d_sum)) return set_error(FHIP_ERR_ARG, "fhip_add_rmsnorm_bf16: NULL pointer");
+    return fhip::launch_rmsnorm_bf16(d_a, d_b, d_weight, rows, d, eps, d_b ? d_sum : nullptr, d_norm_bf16, (hipStream_t)stream);
+}
+
 int fhip_add(const float* d_a, const float* d_b, size_t n, float* d_out, void* stream) {
     int rc = need_init();
     if (rc) return rc;
@@ -935,16 +944,30 @@ int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_cod
                                              (int)n_kv, (int)head_dim, len, d_last_pos, window, softcap, d_ws, d_out, (hipStream_t)stream);
 }
 
+static int check_causal(const char* who, const void* d_q, const void* d_k, const void* d_v, const void* d_out, size_t n_head, size_t n_kv) {
+    if (!d_q || !d_k || !d_v || !d_out) return set_error(FHIP_ERR_ARG, "%s: NULL pointer", who);
+    if ((((uintptr_t)d_q | (uintptr_t)d_k | (uintptr_t)d_v | (uintptr_t)d_out) & 15) != 0)
+        return set_error(FHIP_ERR_ARG, "%s: pointers must be 16-byte aligned", who);
+    if (n_head > 0x7FFFFFFFull || n_kv > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "%s: too many heads", who);
+    return FHIP_OK;
+}
+
 int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
                           size_t window, float softcap, float* d_out, void* stream) {
     int rc = need_init();
     if (rc) return rc;
     if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
-    if (!d_q || !d_k || !d_v || !d_out) return set_error(FHIP_ERR_ARG, "fhip_causal_attention: NULL pointer");
-    if ((((uintptr_t)d_q | (uintptr_t)d_k | (uintptr_t)d_v | (uintptr_t)d_out) & 15) != 0)
-        return set_error(FHIP_ERR_ARG, "fhip_causal_attention: pointers must be 16-byte aligned");
-    if (n_head > 0x7FFFFFFFull || n_kv > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "fhip_causal_attention: too many heads");
+    if ((rc = check_causal("fhip_causal_attention", d_q, d_k, d_v, d_out, n_head, n_kv))) return rc;
     return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, d_out, (hipStream_t)stream);
+}
+
+int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
+                               size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
+    if ((rc = check_causal("fhip_causal_attention_bf16", d_q, d_k, d_v, d_out_bf16, n_head, n_kv))) return rc;
+    return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, d_out_bf16, (hipStream_t)stream);
 }
 
 size_t fhip_decode_attention_ws_bytes(size_t n_head, size_t n_kv, size_t head_dim, size_t len) {
@@ -1168,36 +1191,48 @@ size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gu, const fhip_weight* down, si
     return align256(rows_x * gu->cols * 2) + (ffn_coop_fused(rows_x) ? 0 : align256(rows_x * gu->rows * 4)) + align256(rows_x * down->cols * 2);
 }
 
-int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
-                  void* d_ws, void* stream) {
+// d_x f32 (converted into the workspace first), or already bf16 in d_xb
+static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* down, const float* d_x, const uint16_t* d_xb, size_t rows_x, float* d_y,
+                    void* d_ws, hipStream_t s) {
     int rc = need_init();
     if (rc) return rc;
-    if (!gu || !down) return set_error(FHIP_ERR_ARG, "fhip_ffn_coop: NULL weight");
-    if (gu->rows % 2 != 0) return set_error(FHIP_ERR_SHAPE, "fhip_ffn_coop: gate_up rows must be even");
+    if (!gu || !down) return set_error(FHIP_ERR_ARG, "%s: NULL weight", who);
+    if (gu->rows % 2 != 0) return set_error(FHIP_ERR_SHAPE, "%s: gate_up rows must be even", who);
     const size_t n_ff = gu->rows / 2;
     if (down->cols != n_ff) return set_error(FHIP_ERR_SHAPE, "down in dim must equal n_ff");
     if (rows_x == 0) return FHIP_OK;
-    if (!d_x || !d_y || !d_ws) return set_error(FHIP_ERR_ARG, "fhip_ffn_coop: NULL pointer");
-    if (((uintptr_t)d_ws & 255) != 0) return set_error(FHIP_ERR_ARG, "fhip_ffn_coop: workspace must be 256-byte aligned");
+    if ((!d_x && !d_xb) || !d_y || !d_ws) return set_error(FHIP_ERR_ARG, "%s: NULL pointer", who);
+    if (((uintptr_t)d_ws & 255) != 0) return set_error(FHIP_ERR_ARG, "%s: workspace must be 256-byte aligned", who);
     // an empty inner dimension on either side: gate and up are 0, silu(0) * 0 = 0, and so is every output
-    if (gu->cols == 0 || n_ff == 0) return zero_outputs(rows_x, down->rows, d_y, (hipStream_t)stream);
+    if (gu->cols == 0 || n_ff == 0) return zero_outputs(rows_x, down->rows, d_y, s);
     const bool fused = ffn_coop_fused(rows_x);
     uint8_t* ws = (uint8_t*)d_ws;
     uint16_t* xb = (uint16_t*)ws;
     float* g = (float*)(ws + align256(rows_x * gu->cols * 2));
     uint16_t* hb = (uint16_t*)((uint8_t*)g + (fused ? 0 : align256(rows_x * gu->rows * 4)));
-    hipStream_t s = (hipStream_t)stream;
-    if ((rc = fhip::launch_cvt_bf16(d_x, rows_x * gu->cols, xb, s))) return rc;
+    if (!d_xb) {
+        if ((rc = fhip::launch_cvt_bf16(d_x, rows_x * gu->cols, xb, s))) return rc;
+        d_xb = xb;
+    }
     if (fused) {
         const size_t need = fhip::gemm_bf16_swiglu_ws_bytes(gu, rows_x);
         void* split = nullptr;
-        if (need && (rc = lib_workspace(s, need, &split, "fhip_ffn_coop"))) return rc;
-        if ((rc = fhip::launch_gemm_bf16_swiglu(gu, xb, rows_x, hb, s, (float*)split, need))) return rc;
-        return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, "fhip_ffn_coop");
+        if (need && (rc = lib_workspace(s, need, &split, who))) return rc;
+        if ((rc = fhip::launch_gemm_bf16_swiglu(gu, d_xb, rows_x, hb, s, (float*)split, need))) return rc;
+        return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, who);
     }
-    if ((rc = gemm_bf16_lib_ws(gu, xb, rows_x, g, s, "fhip_ffn_coop"))) return rc;
+    if ((rc = gemm_bf16_lib_ws(gu, d_xb, rows_x, g, s, who))) return rc;
     if ((rc = fhip::launch_swiglu_bf16(g, rows_x, n_ff, hb, s))) return rc;
-    return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, "fhip_ffn_coop");
+    return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, who);
+}
+
+int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
+                  void* d_ws, void* stream) {
+    return ffn_coop("fhip_ffn_coop", gu, down, d_x, nullptr, rows_x, d_y, d_ws, (hipStream_t)stream);
+}
+
+int fhip_ffn_bf16(const fhip_weight* gu, const fhip_weight* down, const uint16_t* d_x_bf16, size_t rows_x, float* d_y, void* d_ws, void* stream) {
+    return ffn_coop("fhip_ffn_bf16", gu, down, nullptr, d_x_bf16, rows_x, d_y, d_ws, (hipStream_t)stream);
 }
 
 size_t fhip_matmul_q_f16x2_ws_bytes(const fhip_weight* w, size_t rows_x) {

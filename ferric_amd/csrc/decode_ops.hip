@@ -10,6 +10,7 @@
 // All of this is f32 arithmetic on small vectors: the kernels are launch- and latency-bound (a decode step has one row),
 // except attention, which streams the layer's K and V rows once (HBM-bound: 2 * len * n_kv * head_dim * 4 bytes).
 #include "common.hpp"
+#include "prompt.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -37,10 +38,19 @@ __device__ __forceinline__ float wave_sum(float v) {
 // ---------------------------------------------------------------- RMSNorm, optionally of a + b
 // out[r, j] = x[r, j] * (1 / sqrt(mean_j x^2 + eps)) * weight[j]   (lib.rs:2018-2033); with b: x = a + b, and the sum is
 // written too (lib.rs:2057-2074). TPR threads share a row (a fixed-shape tree sum, so results do not depend on scheduling).
-template <int TPR>
+// Out = uint16_t: the normed rows as bf16, rounded as fhip_cvt_f32_bf16 rounds them -- what the matrix cores read, for a prompt: a
+// launch and a trip of the f32 rows through memory less per matmul.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2)); }
+__device__ __forceinline__ void store_norm(float* out, size_t j, float4 v) { ((float4*)out)[j] = v; }
+__device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float4 v) { ((uint2*)out)[j] = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
+__device__ __forceinline__ void store_norm(float* out, size_t j, float v) { out[j] = v; }
+__device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float v) { out[j] = (uint16_t)(pk_bf16(v, 0.f) & 0xFFFFu); }
+template <int TPR, typename Out>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const float* __restrict__ b,
                                                       const float* __restrict__ weight, size_t rows, int d, float eps,
-                                                      float* sum_out, float* __restrict__ norm_out) {   // sum_out may be a
+                                                      float* sum_out, Out* __restrict__ norm_out) {   // sum_out may be a
     constexpr int RPW = 256 / TPR;   // rows per workgroup
     constexpr int NV = 8;            // float4 per thread held in registers: rows up to 4 * NV * TPR values
     __shared__ float red[4];
@@ -79,7 +89,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
             if (j < nv) {
                 const float4 w = ((const float4*)weight)[j];
                 if (sum_out) ((float4*)(sum_out + base))[j] = r[i];
-                ((float4*)(norm_out + base))[j] = make_float4(r[i].x * inv * w.x, r[i].y * inv * w.y, r[i].z * inv * w.z, r[i].w * inv * w.w);
+                store_norm(norm_out + base, (size_t)j, make_float4(r[i].x * inv * w.x, r[i].y * inv * w.y, r[i].z * inv * w.z, r[i].w * inv * w.w));
             }
         }
         return;
@@ -101,7 +111,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
     if (!live) return;
     for (int j = t; j < d; j += TPR) {   // the same thread wrote sum_out[.., j] above, so reading it back is ordered
         float v = sum_out ? sum_out[base + j] : (xb ? xa[j] + xb[j] : xa[j]);
-        norm_out[base + j] = v * inv * weight[j];
+        store_norm(norm_out, base + j, v * inv * weight[j]);
     }
 }
 
@@ -1001,19 +1011,29 @@ int launch_attn_fused_g(int hd, dim3 grid, hipStream_t s, const QkvPostParams& f
 
 namespace fhip {
 
-int launch_rmsnorm(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, float* norm_out,
-                   hipStream_t s) {
+template <typename Out>
+static int launch_rmsnorm_out(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, Out* norm_out,
+                              hipStream_t s) {
     if (rows == 0 || d == 0) return FHIP_OK;
     if (d > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: row length exceeds 2^31");
     if (d <= 512) {
         size_t grid = (rows + 3) / 4;
         if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<64>), dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
+        hipLaunchKernelGGL((rmsnorm_kernel<64, Out>), dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
     } else {
         if (rows > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<256>), dim3((unsigned)rows), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
+        hipLaunchKernelGGL((rmsnorm_kernel<256, Out>), dim3((unsigned)rows), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
     }
     return check_hip(hipGetLastError(), "rmsnorm launch");
+}
+
+int launch_rmsnorm(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, float* norm_out,
+                   hipStream_t s) {
+    return launch_rmsnorm_out(a, b, weight, rows, d, eps, sum_out, norm_out, s);
+}
+int launch_rmsnorm_bf16(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, uint16_t* norm_out,
+                        hipStream_t s) {
+    return launch_rmsnorm_out(a, b, weight, rows, d, eps, sum_out, norm_out, s);
 }
 
 int launch_u32_add(uint32_t* w, size_t n, uint32_t delta, hipStream_t s) {

@@ -32,6 +32,7 @@
 // banks apart), shared by the 8 waves (128 queries) of a workgroup; workgroups of the same KV head read the same rows out of
 // L2. Query blocks are issued longest first across all heads.
 #include "common.hpp"
+#include "prompt.hpp"
 
 #include <math.h>
 
@@ -39,11 +40,18 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// Output rows as f32, or as bf16 (rounded as fhip_cvt_f32_bf16 rounds them) for a matmul on the matrix cores.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2)); }
+__device__ __forceinline__ void store_out(float* p, float4 v) { *(float4*)p = v; }
+__device__ __forceinline__ void store_out(uint16_t* p, float4 v) { *(uint2*)p = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
+
 // NW: waves (16 query rows each) per workgroup.
-template <int HD, int NW>
+template <int HD, int NW, typename Out>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
                                                               int S, int n_head, int n_kv, float scale, int window, float softcap,
-                                                              float* __restrict__ out) {
+                                                              Out* __restrict__ out) {
     constexpr int KS = HD + 4;              // floats per K row in LDS
     constexpr int QD = HD / 4;              // dims per quarter
     constexpr int NDT = HD / 16;            // output tiles of 16 rows
@@ -191,13 +199,13 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
     if (!wave_live || i0 + c >= T) return;
     const float inv = 1.0f / l;
     // register r of output tile d is row m = 4 ks + r, i.e. dim NDT m + d
-    float* op = out + ((size_t)i * n_head + head) * HD;
+    Out* op = out + ((size_t)i * n_head + head) * HD;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        float* dst = op + NDT * (4 * ks + r);
+        Out* dst = op + NDT * (4 * ks + r);
 #pragma unroll
         for (int d = 0; d < NDT; d += 4)
-            *(float4*)(dst + d) = float4{oacc[d][r] * inv, oacc[d + 1][r] * inv, oacc[d + 2][r] * inv, oacc[d + 3][r] * inv};
+            store_out(dst + d, float4{oacc[d][r] * inv, oacc[d + 1][r] * inv, oacc[d + 2][r] * inv, oacc[d + 3][r] * inv});
     }
 }
 
@@ -205,8 +213,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
 
 namespace fhip {
 
-int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                            float softcap, float* out, hipStream_t st) {
+template <typename Out>
+static int launch_causal_out(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
+                             float softcap, Out* out, hipStream_t st) {
     if (t == 0 || n_head == 0 || hd == 0) return FHIP_OK;
     if (s < t) return set_error(FHIP_ERR_SHAPE, "cache (%zu) cannot be shorter than the query block (%zu)", s, t);   // nn.rs:73, :249
     if (n_kv <= 0 || n_head % n_kv != 0) return set_error(FHIP_ERR_SHAPE, "causal_attention: n_heads must be a multiple of n_kv_heads");
@@ -221,11 +230,20 @@ int launch_causal_attention(const float* q, const float* K, const float* V, size
     const dim3 grid((unsigned)n_head, (unsigned)qblocks), wg(64 * nw);
     const float scale = 1.0f / sqrtf((float)hd);
     const int win = window == 0 || window >= s ? 0 : (int)window;     // a window that covers the cache is no window
-    if (hd == 128 && nw == 8) hipLaunchKernelGGL((causal_attn_kernel<128, 8>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else if (hd == 128) hipLaunchKernelGGL((causal_attn_kernel<128, 4>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else if (nw == 8) hipLaunchKernelGGL((causal_attn_kernel<64, 8>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else hipLaunchKernelGGL((causal_attn_kernel<64, 4>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
+    if (hd == 128 && nw == 8) hipLaunchKernelGGL((causal_attn_kernel<128, 8, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
+    else if (hd == 128) hipLaunchKernelGGL((causal_attn_kernel<128, 4, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
+    else if (nw == 8) hipLaunchKernelGGL((causal_attn_kernel<64, 8, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
+    else hipLaunchKernelGGL((causal_attn_kernel<64, 4, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
     return check_hip(hipGetLastError(), "causal_attention launch");
+}
+
+int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
+                            float softcap, float* out, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, out, st);
+}
+int launch_causal_attention_bf16(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
+                                 float softcap, uint16_t* out, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, out, st);
 }
 
 }  // namespace fhip

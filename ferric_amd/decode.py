@@ -365,7 +365,10 @@ class Qwen3Decoder:
         X, positions = E(x.shape), E((t,), np.uint32)
         _upload(X.buf, x, self.stream)
         _upload(positions.buf, np.arange(pos0, pos0 + t, dtype=np.uint32), self.stream)
-        h, qkv, q, att = E((t, c.d_model)), E((t, self.q_out + 2 * self.kv_out)), E((t, self.q_out)), E((t, self.q_out))
+        # the projections' input rows: normed (and, ungated, attended) straight to bf16 where the projections read that
+        rows = np.float32 if precise else np.uint16
+        h, qkv, q = E((t, c.d_model), rows), E((t, self.q_out + 2 * self.kv_out)), E((t, self.q_out))
+        att = E((t, self.q_out), np.float32 if self.gate is not None else rows)
         o, x1, y = E((t, c.d_model)), E((t, c.d_model)), E((t, c.d_model))
         normed = E((t, c.d_model)) if self.on is not None else None                   # a post-normed branch output
         f, gu = E((t, c.n_ff)), (E((t, 2 * c.n_ff)) if c.geglu else None)
@@ -380,8 +383,19 @@ class Qwen3Decoder:
         def matmul(w, a, out):
             if precise:
                 _check(lib.fhip_matmul_q(w.handle, a.buf.ptr, t, out.buf.ptr, s))
+            elif a.dtype == np.uint16:
+                _check(lib.fhip_gemm_q_bf16(w.handle, a.buf.ptr, t, out.buf.ptr, s))
             else:
                 _check(lib.fhip_matmul_q_coop(w.handle, a.buf.ptr, t, out.buf.ptr, ws16.ptr, s))
+
+        def norm(a, b, w, total):
+            """h = rmsnorm(a [+ b]); with b, total = a + b."""
+            if not precise:
+                _check(lib.fhip_add_rmsnorm_bf16(a.buf.ptr, b.buf.ptr if b is not None else None, w.buf.ptr, t, c.d_model, c.eps, total.buf.ptr, h.buf.ptr, s))
+            elif b is None:
+                _check(lib.fhip_rmsnorm(a.buf.ptr, w.buf.ptr, t, c.d_model, c.eps, h.buf.ptr, s))
+            else:
+                _check(lib.fhip_add_rmsnorm(a.buf.ptr, b.buf.ptr, w.buf.ptr, t, c.d_model, c.eps, total.buf.ptr, h.buf.ptr, s))
 
         def ffn(l, a, out):
             if c.geglu:
@@ -394,10 +408,11 @@ class Qwen3Decoder:
                 need = lib.fhip_ffn_coop_ws_bytes(l.ffn_gate_up.handle, l.ffn_down.handle, t)
                 if wsf[0] is None or wsf[0].nbytes < need:
                     wsf[0] = DeviceBuffer(max(need, 256))
-                _check(lib.fhip_ffn_coop(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, t, out.buf.ptr, wsf[0].ptr, s))
+                _check(lib.fhip_ffn_bf16(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, t, out.buf.ptr, wsf[0].ptr, s))
 
+        pending = None                                   # the previous layer's FFN branch: joins the residual in the next norm's launch
         for l, kv in zip(self.layers, self.caches):
-            _check(lib.fhip_rmsnorm(X.buf.ptr, l.attn_norm.buf.ptr, t, c.d_model, c.eps, h.buf.ptr, s))
+            norm(x1 if pending is not None else X, pending, l.attn_norm, X)
             matmul(l.wqkv, h, qkv)
             bias = l.qkv_bias.buf.ptr if l.qkv_bias is not None else None
             qn = l.q_norm.buf.ptr if l.q_norm is not None else None
@@ -418,8 +433,8 @@ class Qwen3Decoder:
                     _check(lib.fhip_kvq_dequantize_rows(self.kv_fmt, cache.codes.ptr, cache.scales.ptr, 0, pos0 + t, self.kv_out, None,
                                                         dst.buf.ptr, s))
                 kp, vp = kd.buf.ptr, vd.buf.ptr
-            _check(lib.fhip_causal_attention(q.buf.ptr, kp, vp, t, pos0 + t, c.n_head, c.n_head_kv, c.head_dim, l.window, c.attn_softcap,
-                                             att.buf.ptr, s))
+            attend = lib.fhip_causal_attention if att.dtype == np.float32 else lib.fhip_causal_attention_bf16
+            _check(attend(q.buf.ptr, kp, vp, t, pos0 + t, c.n_head, c.n_head_kv, c.head_dim, l.window, c.attn_softcap, att.buf.ptr, s))
             if l.attn_gate is not None:
                 matmul(l.attn_gate, h, gate)
                 _check(lib.fhip_mul_sigmoid(att.buf.ptr, gate.buf.ptr, t * self.q_out, att.buf.ptr, s))
@@ -428,13 +443,14 @@ class Qwen3Decoder:
             if l.post_attn_norm is not None:
                 _check(lib.fhip_rmsnorm(o.buf.ptr, l.post_attn_norm.buf.ptr, t, c.d_model, c.post_norm_eps, normed.buf.ptr, s))
                 branch = normed
-            _check(lib.fhip_add_rmsnorm(X.buf.ptr, branch.buf.ptr, l.ffn_norm.buf.ptr, t, c.d_model, c.eps, x1.buf.ptr, h.buf.ptr, s))
+            norm(X, branch, l.ffn_norm, x1)
             ffn(l, h, y)
-            branch = y
+            pending = y
             if l.post_ffn_norm is not None:
                 _check(lib.fhip_rmsnorm(y.buf.ptr, l.post_ffn_norm.buf.ptr, t, c.d_model, c.post_norm_eps, normed.buf.ptr, s))
-                branch = normed
-            _check(lib.fhip_add(x1.buf.ptr, branch.buf.ptr, t * c.d_model, X.buf.ptr, s))
+                pending = normed
+        if pending is not None:
+            _check(lib.fhip_add(x1.buf.ptr, pending.buf.ptr, t * c.d_model, X.buf.ptr, s))
         _check(lib.fhip_u32_add(self.pos.buf.ptr, 1, t, s))
         out = X.to_vec(self.stream).reshape(t, c.d_model)      # synchronises: the temporaries may go
         for cache in self._all_caches():

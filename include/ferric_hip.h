@@ -259,6 +259,10 @@ int fhip_rmsnorm(const float* d_x, const float* d_weight, size_t rows, size_t d,
  * (the residual updated in place). */
 int fhip_add_rmsnorm(const float* d_a, const float* d_b, const float* d_weight, size_t rows, size_t d, float eps, float* d_sum,
                      float* d_norm, void* stream);
+/* The same with the normed rows as bf16 (each value the one fhip_cvt_f32_bf16 makes of d_norm's), for fhip_gemm_q_bf16 and
+ * fhip_ffn_bf16; d_b NULL: rmsnorm of d_a alone (d_sum is not looked at). */
+int fhip_add_rmsnorm_bf16(const float* d_a, const float* d_b, const float* d_weight, size_t rows, size_t d, float eps, float* d_sum,
+                          uint16_t* d_norm_bf16, void* stream);
 
 /* lib.rs:279 Tensor::add, same shapes: out = a + b, n elements. */
 int fhip_add(const float* d_a, const float* d_b, size_t n, float* d_out, void* stream);
@@ -329,7 +333,8 @@ int fhip_kvq_append2(int fmt, const float* d_k, const float* d_v, size_t src_row
  * is loaded (the use the reference chose the block layout for and left unbuilt, kvquant.rs:30-37, qwen3.rs:897-905: it
  * materialises `dequantize()` of the whole history per layer and step and attends over that). The values that enter the
  * softmax are exactly fhip_kvq_dequantize_rows', so the result has the bits of fhip_decode_attention_ex over the dequantized
- * rows, at 8.5 / 4.5 / 5 bits per value of traffic instead of 32 + 32 written and read back. */
+ * rows -- behind more than 5120 rows of a Q8_0 or Q4_0 cache with six or more query heads per KV head (five of 64 dims) its
+ * value to f32 rounding, the sums being formed on the matrix cores in another order -- at 8.5 / 4.5 / 5 bits per value of traffic instead of 32 + 32 written and read back. */
 int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_codes, const uint32_t* d_k_scales, const uint32_t* d_v_codes,
                               const uint32_t* d_v_scales, size_t n_head, size_t n_kv, size_t head_dim, size_t len, const uint32_t* d_last_pos,
                               size_t window, float softcap, float* d_ws, float* d_out, void* stream);
@@ -343,6 +348,9 @@ int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_cod
  * matrix instructions), out [t, n_head * head_dim]; pointers 16-byte aligned. */
 int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
                           size_t window, float softcap, float* d_out, void* stream);
+/* The same with the output rows as bf16, each value the one fhip_cvt_f32_bf16 makes of the f32 result. */
+int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
+                               size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream);
 
 /* fhip_qkv_post with the key and value heads written to packed outputs [t, n_kv * head_dim] (row i for token i) instead of
  * cache rows: for callers that store them themselves, as the quantized arm of qwen3.rs:906-912 does. */
@@ -470,6 +478,8 @@ int fhip_matmul_q_coop(const fhip_weight* w, const float* d_x, size_t rows_x, fl
 size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gate_up, const fhip_weight* down, size_t rows_x);
 int fhip_ffn_coop(const fhip_weight* gate_up, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
                   void* d_ws, void* stream);
+/* The same on rows that are bf16 already (16-byte aligned); the same workspace, the same bits. */
+int fhip_ffn_bf16(const fhip_weight* gate_up, const fhip_weight* down, const uint16_t* d_x_bf16, size_t rows_x, float* d_y, void* d_ws, void* stream);
 
 /* crates/ferric-tensor/src/dtype.rs:935-944 Tensor::matmul_q for 1..32 activation rows in ONE pass over the weights
  * with f32-grade results (the reference's kernels, :2995-3051 and :3423-3469, walk the weight row once per activation

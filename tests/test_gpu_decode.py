@@ -667,3 +667,47 @@ def test_prefill_of_a_prompt_block_then_decode(F, X, O, D, name, arms, cfg_kw, k
             assert np.median(errs) <= 5e-3 and (errs <= bar).mean() >= 0.75, (name, np.sort(errs)[-4:])
     with pytest.raises(AssertionError, match="exceed the capacity"):
         dec.prefill(xs[:2])
+
+
+def test_rows_rounded_to_bf16_by_their_producer(F, X):
+    """fhip_add_rmsnorm_bf16 and fhip_causal_attention_bf16 store the bits fhip_cvt_f32_bf16 makes of their f32 forms (both row kernels, a
+    width that is not a multiple of four, NaN and infinities; both head sizes and workgroup shapes); fhip_ffn_bf16 on converted rows has
+    the bits of fhip_ffn_coop."""
+    rng = np.random.default_rng(3)
+    lib, chk = F._lib.load(), F._lib.check
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    E = F.Tensor.empty
+    raw = lambda t: t.to_vec().view(np.uint16 if t.dtype == np.uint16 else np.uint32)
+    for rows, d in ((3, 5120), (7, 130), (5, 512), (2, 9001), (1, 3)):
+        a, b, w = (rng.standard_normal(n).astype(np.float32) for n in ((rows, d), (rows, d), (d,)))
+        a[0, 0], w[-1] = np.inf, np.nan
+        at, bt, wt = T(a), T(b), T(w)
+        for resid in (None, bt):
+            f, s0, s1, h = E((rows, d)), E((rows, d)), E((rows, d)), E((rows, d), np.uint16)
+            if resid is None:
+                chk(lib.fhip_rmsnorm(at.buf.ptr, wt.buf.ptr, rows, d, 1e-6, f.buf.ptr, None))
+                chk(lib.fhip_add_rmsnorm_bf16(at.buf.ptr, None, wt.buf.ptr, rows, d, 1e-6, None, h.buf.ptr, None))
+            else:
+                chk(lib.fhip_add_rmsnorm(at.buf.ptr, bt.buf.ptr, wt.buf.ptr, rows, d, 1e-6, s0.buf.ptr, f.buf.ptr, None))
+                chk(lib.fhip_add_rmsnorm_bf16(at.buf.ptr, bt.buf.ptr, wt.buf.ptr, rows, d, 1e-6, s1.buf.ptr, h.buf.ptr, None))
+                assert np.array_equal(raw(s0), raw(s1))
+            assert np.array_equal(raw(f.cvt_bf16()), raw(h)), (rows, d)
+    for t, s, nh, nkv, hd in ((33, 70, 10, 2, 128), (100, 100, 4, 4, 64), (512, 512, 136, 8, 64), (520, 520, 104, 8, 128)):
+        q, k, v = (T(rng.standard_normal(n).astype(np.float32)) for n in ((t, nh * hd), (s, nkv * hd), (s, nkv * hd)))
+        f, h = E((t, nh * hd)), E((t, nh * hd), np.uint16)
+        chk(lib.fhip_causal_attention(q.buf.ptr, k.buf.ptr, v.buf.ptr, t, s, nh, nkv, hd, 0, 0.0, f.buf.ptr, None))
+        chk(lib.fhip_causal_attention_bf16(q.buf.ptr, k.buf.ptr, v.buf.ptr, t, s, nh, nkv, hd, 0, 0.0, h.buf.ptr, None))
+        assert np.array_equal(raw(f.cvt_bf16()), raw(h)), (t, hd)
+    from ferric_amd.synth import synth_weights
+    d, ff = 512, 768
+    gu, down = (F.QMatrix.from_bytes(synth_weights(Q4_K, r, c, 1), Q4_K, r, c) for r, c in ((2 * ff, d), (d, ff)))
+    for t in (7, 32, 33, 200):
+        x = T(rng.standard_normal((t, d)).astype(np.float32))
+        ws, y = F.DeviceBuffer(lib.fhip_ffn_coop_ws_bytes(gu.handle, down.handle, t)), E((t, d))
+        xb = x.cvt_bf16()
+        chk(lib.fhip_ffn_bf16(gu.handle, down.handle, xb.buf.ptr, t, y.buf.ptr, ws.ptr, None))
+        assert np.array_equal(raw(x.ffn_coop(gu, down)), raw(y)), t
+    one = E((1, 8), np.uint16)
+    assert lib.fhip_add_rmsnorm_bf16(wt.buf.ptr, bt.buf.ptr, wt.buf.ptr, 1, 2, 1e-6, None, one.buf.ptr, None) != 0       # a sum asked for and no place for it
+    assert lib.fhip_causal_attention_bf16(q.buf.ptr, k.buf.ptr, v.buf.ptr, 1, 1, 1, 1, 64, 0, 0.0, one.buf.ptr.value + 8, None) != 0
+    assert b"16-byte aligned" in lib.fhip_last_error()
