@@ -266,6 +266,7 @@ int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_i
     const bool ordered = w->batch_policy == FHIP_BATCH_ORDERED;
     float* part = ordered && fhip::gemm_f16x2_part_bytes(w, t) ? (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))) : nullptr;
     const bool clr = !part && fhip::gemm_f16x2_adds_into_y(w, t);   // then the split clears y on the side
+    if (!swiglu_in && !src && !clr && fhip::gemm_f16x2_own_x(w, d_x, t)) return fhip::launch_gemm_f16x2(w, nullptr, t, d_y, s, false, part, deferred, d_x);
     int rc = fhip::launch_xsplit_f16(w, d_x, t, swiglu_in, xp, s, clr ? d_y : nullptr, clr ? t * w->rows : 0, src);
     if (rc) return rc;
     return fhip::launch_gemm_f16x2(w, xp, t, d_y, s, clr, part, deferred);

@@ -23,7 +23,7 @@
 //     mantissa of the f16 constant 1024 or, for the high nibble, 16 positions up) and 4 packed f16 fma that remove the
 //     constant and apply the sub-block scale: 9 VALU for 8 weights, against ~30 for the bf16 path's f32 arithmetic.
 //     The k order inside an MFMA is free as long as both operands agree, so the activations are laid out in the
-//     order the nibbles come out (xsplit_f16_kernel does that once per call).
+//     order the nibbles come out (xsplit_f16_kernel does that once per call, or each workgroup for its own chunks).
 //
 // Lane (g4 = lane / 16, c = lane % 16) of a wave works on weight row c of a 16-row set and on k-group g4 of each
 // 32-wide MFMA slice; a wave carries two row sets (32 weight rows), a workgroup four waves (128 rows; the row-streaming
@@ -454,6 +454,19 @@ __device__ __forceinline__ float act(const float* __restrict__ x, int t, int K, 
     return x_at(x, t, k, src);
 }
 
+// A chunk's scale out of the largest magnitude of its columns: the factor, and the one that takes it out again
+__device__ __forceinline__ void chunk_scale(float m, float& sc, float& inv) {
+    sc = 1.0f;
+    inv = 1.0f;
+    if (m > 0.f && m < INFINITY) {
+        int ex;
+        (void)frexpf(m, &ex);            // m < 2^ex
+        ex = ex < -111 ? -111 : ex;      // the scale stays a finite f32; chunks below 2^-111 keep fewer bits
+        sc = ldexpf(1.0f, 15 - ex);      // scaled maximum in [2^14, 2^15)
+        inv = ldexpf(1.0f, ex - 15);
+    }
+}
+
 // one workgroup per (chunk, operand row of a group of 8): thread k of it converts column k of the chunk
 template <class F, bool SWIGLU>
 __global__ void __launch_bounds__(256) xsplit_f16_kernel(const float* __restrict__ X, int T, int K, int NT, uint16_t* __restrict__ Xp,
@@ -474,14 +487,8 @@ __global__ void __launch_bounds__(256) xsplit_f16_kernel(const float* __restrict
     if (lane == 0) red[tid >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    float sc = 1.0f, inv = 1.0f;
-    if (m > 0.f && m < INFINITY) {
-        int ex;
-        (void)frexpf(m, &ex);            // m < 2^ex
-        ex = ex < -111 ? -111 : ex;      // the scale stays a finite f32; chunks below 2^-111 keep fewer bits
-        sc = ldexpf(1.0f, 15 - ex);      // scaled maximum in [2^14, 2^15)
-        inv = ldexpf(1.0f, ex - 15);
-    }
+    float sc, inv;
+    chunk_scale(m, sc, inv);
     const size_t row = ((size_t)(ck * NT + (t >> 3)) * 16 + (t & 7)) * XR;
     auto put = [&](int col, float v) {
         const _Float16 h = (_Float16)v;
@@ -509,6 +516,8 @@ __global__ void __launch_bounds__(256) xsplit_f16_kernel(const float* __restrict
 struct F16Params {
     const uint8_t* W;
     const uint16_t* Xp;   // prepared activations: [nchunks][16 NT][XR] f16
+    const float* X;       // or the rows as they are, [T, K], for a kernel that prepares a chunk's operand rows itself
+    int K;
     float* Y;             // [T, N]
     int T, N, nchunks;
     int nblk;             // Q8_0: blocks in a weight row (the last chunk may hold fewer than 8)
@@ -680,7 +689,9 @@ __global__ void __launch_bounds__(256, F::occupancy(NT)) gemm_q_f16x2_kernel(F16
 // on bytes it has not seen) this takes 34 us for a 34816 x 5120 Q4_K weight and 27 us for 5120 x 17408 Q6_K, the kernel
 // above 39 and 35.5 us: its one-row-per-lane loads ask for every cache line two or three times, 16 bytes at a time.
 // ------------------------------------------------------------------------------------------------
-template <class F, int NT, int WAVES>
+// OWN_X: the workgroup makes the operand rows of its chunks itself out of the f32 rows, the bits of xsplit_f16_kernel's: a wave takes
+// 8 NT / WAVES rows, a lane four columns (their four positions are one aligned run of eight bytes in every format's order).
+template <class F, int NT, int WAVES, bool OWN_X>
 __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROWS_OCCUPANCY : 2)) gemm_q_f16x2_rows_kernel(F16Params p) {
     // WAVES = 8 (up to 8 activation rows on the large K-split weights of the FFN block): ONE workgroup of eight waves (256 weight
     // rows) per CU. Three workgroups of four waves, each with its own staged activations, ended far apart -- the younger a workgroup on its CU the later (ends of the first / second / third
@@ -701,17 +712,72 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROW
     long long u = (long long)blockIdx.x * p.units / gridDim.x;
     const long long u_end = (long long)(blockIdx.x + 1) * p.units / gridDim.x;
 
-    u32x4 stage[NP];
+    constexpr int RPW = 8 * NT / WAVES;      // OWN_X: activation rows per wave
+    u32x4 stage[OWN_X ? 1 : NP];
+    f32x4 xrow[OWN_X ? RPW : 1];
     auto load_x = [&](int ck) {
-        const u32x4* src = (const u32x4*)(p.Xp + (size_t)ck * 16 * NT * XR);
+        if constexpr (OWN_X) {
+            const int k = ck * CHUNK + 4 * lane;
 #pragma unroll
-        for (int q = 0; q < NP; q++)
-            if (tid + NTHR * q < PIECES) stage[q] = src[tid + NTHR * q];
+            for (int r = 0; r < RPW; r++) {
+                const int t = wave * RPW + r;
+                xrow[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                if (t < p.T && k < p.K) xrow[r] = *(const f32x4*)(p.X + (size_t)t * p.K + k);
+            }
+        } else {
+            const u32x4* src = (const u32x4*)(p.Xp + (size_t)ck * 16 * NT * XR);
+#pragma unroll
+            for (int q = 0; q < NP; q++)
+                if (tid + NTHR * q < PIECES) stage[q] = src[tid + NTHR * q];
+        }
     };
     auto store_x = [&](int buf) {
+        if constexpr (OWN_X) {
+            const int pos = F::pos_of(4 * lane);
 #pragma unroll
-        for (int q = 0; q < NP; q++)
-            if (tid + NTHR * q < PIECES) ((u32x4*)Xs[buf])[tid + NTHR * q] = stage[q];
+            for (int r = 0; r < RPW; r++) {
+                const int t = wave * RPW + r;
+                uint16_t* const hi = Xs[buf] + (16 * (t >> 3) + (t & 7)) * XR;
+                uint16_t* const lo = hi + 8 * XR;
+                // (a NaN is not the largest magnitude: it reaches the operands as it is)
+                float m = fmaxf(fmaxf(fabsf(xrow[r][0]), fabsf(xrow[r][1])), fmaxf(fabsf(xrow[r][2]), fabsf(xrow[r][3])));
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+                float sc, inv;
+                chunk_scale(m, sc, inv);
+                uint32_t h[4], l[4];
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    v[j] = xrow[r][j] * sc;
+                    const _Float16 a = (_Float16)v[j];
+                    h[F::pos_of(j)] = __builtin_bit_cast(uint16_t, a);
+                    l[F::pos_of(j)] = __builtin_bit_cast(uint16_t, (_Float16)(v[j] - (float)a));
+                }
+                *(u32x2*)(hi + pos) = (u32x2){h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+                *(u32x2*)(lo + pos) = (u32x2){l[0] | (l[1] << 16), l[2] | (l[3] << 16)};
+                if constexpr (F::HAS_MIN) {
+                    // the sums of 32 columns in the order of xsplit's exchanges: columns 16, 8, 4, 2, 1 apart
+#pragma unroll
+                    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) v[j] += __shfl_xor(v[j], o);
+                    const float sum = ((v[0] + v[2]) + (v[1] + v[3])) * 0.015625f;
+                    if ((lane & 7) == 0) {
+                        const _Float16 a = (_Float16)sum;
+                        hi[CHUNK + (lane >> 3)] = __builtin_bit_cast(uint16_t, a);
+                        lo[CHUNK + (lane >> 3)] = __builtin_bit_cast(uint16_t, (_Float16)(sum - (float)a));
+                    }
+                    if (lane == 1) *(u32x4*)(hi + CHUNK + 8) = (u32x4){0u, 0u, 0u, 0u};
+                    if (lane == 2) *(u32x4*)(lo + CHUNK + 8) = (u32x4){0u, 0u, 0u, 0u};
+                }
+                if (lane == 0) { *(float*)(hi + XSCALE) = inv; *(float*)(lo + XSCALE) = inv; }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < NP; q++)
+                if (tid + NTHR * q < PIECES) ((u32x4*)Xs[buf])[tid + NTHR * q] = stage[q];
+        }
     };
     const int a_rd = c * XR + 8 * g4;
     const int m_rd = c * XR + CHUNK + (g4 ? 8 : 0);
@@ -962,6 +1028,16 @@ Plan make_plan(const fhip_weight* w, size_t t) {
     return q;
 }
 
+// Whether the launch makes its operand rows itself: the same bits, a launch and a trip of the rows through memory less, but every
+// workgroup that holds a chunk converts it (two rows of 256 values a wave, between a chunk's products and the next barrier). Ordered
+// sums, 8 rows, us, itself | prepared: one unit a workgroup Q8_0 4096 x 4096 12.4 | 14.2, Q4_K 1024 x 5120 9.3 | 11.4, Q6_K 2048 x 9728 14.2 | 16.3;
+// two, 12288 x 4096 Q8_0 22.0 | 22.8, Q4_K 16.5 | 16.9, Q6_K 20.4 | 20.4; more, 5120 x 17408 Q8_0 34.5 | 35.5, Q4_K 25.8 | 24.2, 34816 x 5120 Q4_K
+// 38.9 | 34.2. At 16 rows: 4096 x 4096 Q8_0 15.3 | 16.4, Q6_K 14.1 | 15.2, 12288 x 4096 (three) Q6_K 26.2 | 25.7.
+bool own_x(const fhip_weight* w, const Plan& q, const float* d_x) {
+    const bool rows_kernel = (q.nt == 1 && q.group == 128) || (q.nt == 2 && (w->type == FHIP_Q8_0 || w->type == FHIP_Q6_K));
+    return rows_kernel && d_x && ((uintptr_t)d_x & 15) == 0 && q.units <= 2 * (long long)q.grid;
+}
+
 template <class F>
 int launch_xsplit_fmt(const float* d_x, size_t t, size_t k, bool swiglu, const Plan& q, uint16_t* d_xp, hipStream_t s, float* zero,
                       size_t zero_n, const fhip::F16Parts& src) {
@@ -972,10 +1048,11 @@ int launch_xsplit_fmt(const float* d_x, size_t t, size_t k, bool swiglu, const P
 }
 
 template <class F>
-int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y, hipStream_t s, bool y_cleared, float* d_part, fhip::F16Parts* deferred) {
+int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, hipStream_t s, bool y_cleared, float* d_part,
+               fhip::F16Parts* deferred) {
     const Plan q = make_plan(w, t);
     F16Params p;
-    p.W = w->d_raw; p.Xp = d_xp; p.Y = d_y;
+    p.W = w->d_raw; p.Xp = d_xp; p.X = d_x; p.K = (int)w->cols; p.Y = d_y;
     p.part = q.split ? d_part : nullptr; p.kmax = q.kmax;
     p.T = (int)t; p.N = (int)w->rows; p.nchunks = q.nchunks; p.row_bytes = w->row_bytes;
     p.nblk = (int)(w->cols / 32);
@@ -984,10 +1061,18 @@ int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y,
         const size_t n = t * w->rows;
         hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_y, n);
     }
+    const bool own = d_x != nullptr;
     if (q.nt == 1 && q.group == 256) {
-        if constexpr (F::ROW_PER_LANE) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 1, 8>), dim3(q.grid), dim3(512), 0, s, p);
-    } else if (q.nt == 1) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 1, 4>), dim3(q.grid), dim3(256), 0, s, p);
-    else if (q.nt == 2 && F::ROWS_AT_16) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 2, 4>), dim3(q.grid), dim3(256), 0, s, p);
+        if constexpr (F::ROW_PER_LANE) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 1, 8, false>), dim3(q.grid), dim3(512), 0, s, p);
+    } else if (q.nt == 1) {
+        if (own) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 1, 4, true>), dim3(q.grid), dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 1, 4, false>), dim3(q.grid), dim3(256), 0, s, p);
+    } else if (q.nt == 2 && F::ROWS_AT_16) {
+        if constexpr (F::ROWS_AT_16) {
+            if (own) hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 2, 4, true>), dim3(q.grid), dim3(256), 0, s, p);
+            else hipLaunchKernelGGL((gemm_q_f16x2_rows_kernel<F, 2, 4, false>), dim3(q.grid), dim3(256), 0, s, p);
+        }
+    }
     else if constexpr (F::ROW_PER_LANE) {
         if (q.nt == 2) hipLaunchKernelGGL((gemm_q_f16x2_kernel<F, 2>), dim3(q.grid), dim3(256), 0, s, p);
         else hipLaunchKernelGGL((gemm_q_f16x2_kernel<F, 4>), dim3(q.grid), dim3(256), 0, s, p);
@@ -1043,13 +1128,15 @@ int launch_xsplit_f16(const fhip_weight* w, const float* d_x, size_t t, bool swi
     }
 }
 
+bool gemm_f16x2_own_x(const fhip_weight* w, const float* d_x, size_t t) { return own_x(w, make_plan(w, t), d_x); }
+
 int launch_gemm_f16x2(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y, hipStream_t s, bool y_cleared, float* d_part,
-                      F16Parts* deferred) {
+                      F16Parts* deferred, const float* d_x) {
     switch (w->type) {
-        case FHIP_Q4_K: return launch_fmt<Q4K>(w, d_xp, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_xp, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_xp, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q8_0: return launch_fmt<Q80>(w, d_xp, t, d_y, s, y_cleared, d_part, deferred);
+        case FHIP_Q4_K: return launch_fmt<Q4K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
+        case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
+        case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
+        case FHIP_Q8_0: return launch_fmt<Q80>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "f16x2 matmul: no kernel for ggml type %u", w->type);
     }
 }

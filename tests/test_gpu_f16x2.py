@@ -343,3 +343,30 @@ def test_ordered_policy_gives_the_same_bits_on_every_run(F, O):
         assert np.array_equal(xt.try_matmul_swiglu(wgu).matmul_q(wdn).to_vec(), xt.ffn(wgu, wdn).to_vec())
     finally:
         lib.fhip_batch_policy(before)
+
+
+@pytest.mark.parametrize("ty,rows,cols", [(8, 130, 32), (8, 33, 288), (8, 600, 512), (12, 40, 256), (12, 1100, 512), (13, 300, 512), (14, 600, 256), (14, 129, 512)])
+def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows, cols):
+    """A small weight's ordered launch converts its chunks itself; fhip_matmul_q_f16x2 prepares them by a launch of its own. Up to two chunks
+    (sums of two terms, whose order does not matter) both have the same bits, for every number of rows the kernel takes, a last
+    chunk that is not full, an odd number of weight rows, rows of zeros, chunks of tiny, huge and non-finite values."""
+    from conftest import bits
+    from ferric_amd.synth import synth_weights
+    rng = np.random.default_rng(rows + cols)
+    lib = F._lib.load()
+    w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 1), ty, rows, cols)
+    w.batch_policy(F.BATCH_ORDERED)
+    for t in (5, 7, 8, 9, 13, 16):
+        x = (rng.standard_normal((t, cols)) * np.exp2(rng.integers(-20, 20, (t, 1)))).astype(np.float32)
+        x[0, :30], x[1], x[2, 7], x[3, -1], x[4, 20] = 1e-41, 0.0, 3e38, -np.inf, np.nan
+        xt, ws, ys = F.Tensor.from_vec(x, x.shape), F.DeviceBuffer(lib.fhip_matmul_q_f16x2_ws_bytes(w.handle, t)), []
+        for prepared in (False, True):
+            y = F.Tensor.empty((t, rows))
+            if prepared:
+                F._lib.check(lib.fhip_matmul_q_f16x2(w.handle, xt.buf.ptr, t, y.buf.ptr, ws.ptr, None))
+            else:
+                F._lib.check(lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, None))
+            ys.append(y.to_vec())
+        nan = np.isnan(ys[0])
+        assert np.array_equal(nan, np.isnan(ys[1])) and nan.any(), t
+        assert np.array_equal(bits(ys[0])[~nan], bits(ys[1])[~nan]), t
