@@ -931,6 +931,23 @@ int fhip_kvq_append2(int fmt, const float* d_k, const float* d_v, size_t src_row
                                    (hipStream_t)stream, d_v, d_v_codes, (uint16_t*)d_v_scales);
 }
 
+int fhip_qkv_post_kvq(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
+                      const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                      float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
+                      void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if ((rc = kvq_checks("fhip_qkv_post_kvq", fmt, n_kv * head_dim)) || (rc = rope_checks("fhip_qkv_post_kvq", n_head + 2 * n_kv, head_dim, n_rot))) return rc;
+    if (t == 0 || head_dim == 0 || n_head + n_kv == 0) return FHIP_OK;
+    if (!fhip::qkv_post_kvq_takes((int)head_dim)) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_kvq: head_dim must be a multiple of 32 up to 256, got %zu", head_dim);
+    if (!d_qkv || !d_positions || !d_q_out || !d_k_codes || !d_k_scales || !d_v_codes || !d_v_scales)
+        return set_error(FHIP_ERR_ARG, "fhip_qkv_post_kvq: NULL pointer");
+    if (cap > 0xFFFFFFFFull) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_kvq: too large for one launch");
+    return fhip::launch_qkv_post_kvq(fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_positions, d_freq_scale, t, (int)n_head, (int)n_kv, (int)head_dim, (int)n_rot,
+                                     interleaved != 0, eps, base, d_q_out, d_k_codes, (uint16_t*)d_k_scales, d_v_codes, (uint16_t*)d_v_scales, cap,
+                                     (hipStream_t)stream);
+}
+
 int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_codes, const uint32_t* d_k_scales, const uint32_t* d_v_codes,
                               const uint32_t* d_v_scales, size_t n_head, size_t n_kv, size_t head_dim, size_t len, const uint32_t* d_last_pos,
                               size_t window, float softcap, float* d_ws, float* d_out, void* stream) {

@@ -178,6 +178,10 @@ int launch_rope(const float* x, size_t src_row_stride, size_t t, int heads, int 
 int launch_qkv_post(const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos, const float* freq_scale,
                     size_t t, int n_head, int n_kv, int hd, int n_rot, int interleaved, float eps, float base, float* q_out, float* k_cache,
                     float* v_cache, size_t cap, hipStream_t s, bool kv_packed = false);   // kv_packed: K / V rows to packed [t, n_kv * hd] outputs
+bool qkv_post_kvq_takes(int hd);
+int launch_qkv_post_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos,
+                        const float* freq_scale, size_t t, int n_head, int n_kv, int hd, int n_rot, int interleaved, float eps, float base, float* q_out,
+                        uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes, uint16_t* v_scales, size_t cap, hipStream_t s);
 int launch_kv_append(const float* k, const float* v, size_t t, size_t width, const uint32_t* d_pos, uint32_t pos_off, size_t cap, float* kc,
                      float* vc, hipStream_t s);
 int attn_splits(size_t len, int n_kv);

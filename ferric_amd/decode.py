@@ -199,7 +199,7 @@ class Qwen3Decoder:
     A gated layer adds two launches (the gate's mat-vec on the same normed input, the sigmoid product), post-norms two (the
     RMSNorm of each branch output; the add happens inside the next mat-vec as before), GEGLU one (the activation on its own).
     kv_fmt: the caches are block-quantized (kvquant.QKvCache pairs of fixed capacity): the token's K and V rows are quantized by
-    one launch and attention reads the blocks in place, 8 launches per layer; no f32 copy of the history exists.
+    the post-processing's launch and attention reads the blocks in place, 7 launches per layer; no f32 copy of the history exists.
     """
 
     def __init__(self, cfg, layers, max_len, stream=None, output_norm=None, lm_head=None, fuse_norm=True, fuse_attn=None, kv_fmt=None):
@@ -216,8 +216,7 @@ class Qwen3Decoder:
         else:
             from .kvquant import QKvCache
             self.caches = [(QKvCache(kv_fmt, max_len, self.kv_out), QKvCache(kv_fmt, max_len, self.kv_out)) for _ in layers]
-            self.k1, self.v1 = Tensor.empty((1, self.kv_out)), Tensor.empty((1, self.kv_out))     # the new token's rows before they are stored
-            fuse_attn = self.fuse_attn = False            # the rows are quantized by a launch of their own
+            fuse_attn = self.fuse_attn = False            # the rows are quantized in the post-processing's launch, in front of attention's
         self.pos = _u32_tensor([0])                       # device word: the position of the token being decoded
         self.xa = Tensor.empty((1, c.d_model))            # residual stream: the step's input is written here ...
         self.xb = Tensor.empty((1, c.d_model))            # ... and the residual alternates between the two buffers
@@ -244,8 +243,7 @@ class Qwen3Decoder:
         self.fuse_attn = bool(self.fuse_attn)
         # a default-arm layer; caches of up to 256 rows under grouped query heads need no combine launch behind the attention
         short = self.max_len <= 256 and c.n_head > c.n_head_kv
-        self.launches_per_layer = ((7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) + (1 if kv_fmt is not None else 0)
-                                   - (1 if short else 0))
+        self.launches_per_layer = (7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) - (1 if short else 0)
         # per token beside the layers: the position word's increment and the head (final norm inside the head's mat-vec; a head of
         # 128 MB and more takes the norm as a launch of its own, which costs less than the wider workgroups the fused norm needs)
         big_head = lm_head is not None and lm_head.nbytes() >= (128 << 20)
@@ -304,12 +302,11 @@ class Qwen3Decoder:
             kn = l.k_norm.buf.ptr if l.k_norm is not None else None
             ws = self.ws.ptr if self.ws is not None else None
             if self.kv_fmt is not None:
-                # the quantized arm (qwen3.rs:906-912): post-process, store the token's rows as blocks, attend over the blocks
+                # the quantized arm (qwen3.rs:906-912): post-process and store the token's rows as blocks, attend over the blocks
                 kq, vq = kv
-                _check(lib.fhip_qkv_post_packed(self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, 1, c.n_head, c.n_head_kv, c.head_dim, n_rot,
-                                                int(c.rope_interleaved), c.eps, base, self.q.buf.ptr, self.k1.buf.ptr, self.v1.buf.ptr, s))
-                _check(lib.fhip_kvq_append2(self.kv_fmt, self.k1.buf.ptr, self.v1.buf.ptr, 0, 1, self.kv_out, self.pos.buf.ptr, 0, kq.cap,
-                                            kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, s))
+                _check(lib.fhip_qkv_post_kvq(self.kv_fmt, self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, 1, c.n_head, c.n_head_kv, c.head_dim, n_rot,
+                                             int(c.rope_interleaved), c.eps, base, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr,
+                                             vq.scales.ptr, kq.cap, s))
                 _check(lib.fhip_decode_attention_kvq(self.kv_fmt, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, c.n_head,
                                                      c.n_head_kv, c.head_dim, self.max_len, self.pos.buf.ptr, l.window, c.attn_softcap, ws,
                                                      self.att.buf.ptr, s))

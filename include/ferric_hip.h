@@ -357,6 +357,12 @@ int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* 
 int fhip_qkv_post_packed(const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
                          const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved,
                          float eps, float base, float* d_q_out, float* d_k_out, float* d_v_out, void* stream);
+/* fhip_qkv_post_packed and fhip_kvq_append2 of its key and value rows in one launch, the same bytes: row i goes to cache row
+ * d_positions[i] of caches of `cap` rows (a position past them is dropped). head_dim a multiple of 32 up to 256. */
+int fhip_qkv_post_kvq(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
+                      const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                      float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
+                      void* stream);
 
 /* crates/ferric-tensor/src/nn.rs:140 decode_attention -> lib.rs:762 fused_decode_attention (kernels :2675, :2740 ff.):
  * one query row q [n_head * head_dim] against the cache rows [0, len) of K and V [., n_kv * head_dim];

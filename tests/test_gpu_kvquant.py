@@ -260,3 +260,54 @@ def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
             got = cache.dequantize().to_vec().reshape(cap, width)
             for i, r in enumerate(where):
                 assert np.array_equal(bits(got[r]), bits(K.roundtrip(x[i], 1, width, fmt)[0])), (fmt, i)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("nh,nkv,hd,n_rot,inter,norms", [(10, 2, 128, 128, 0, True), (4, 4, 64, 64, 1, True), (6, 3, 32, 16, 0, False), (5, 1, 96, 64, 0, True),
+                                                         (2, 1, 256, 256, 0, True), (8, 2, 64, 0, 0, True)])
+def test_post_processing_and_quantized_stores_in_one_launch(F, Q, fmt, nh, nkv, hd, n_rot, inter, norms):
+    """fhip_qkv_post_kvq against fhip_qkv_post_packed followed by fhip_kvq_append2: the same query bits, codes and scales, for heads of one, one
+    and a half and four halves of a wave; blocks of zeros of both signs, equal magnitudes, NaN and infinities; a position past the cache."""
+    rng = np.random.default_rng(nh * hd + fmt)
+    lib, t, cap, width = F._lib.load(), 5, 9, nkv * hd
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    qkv = (rng.standard_normal((t, (nh + 2 * nkv) * hd)) * 3).astype(np.float32)
+    v = qkv[:, (nh + nkv) * hd:]
+    v[0, :32] = np.where(np.arange(32) % 2, 0.0, -0.0)
+    v[1, :32] = np.where(np.arange(32) % 3, 2.5, -2.5)
+    v[2, 3], v[2, 20], v[3, 5] = np.nan, np.inf, 1e-42
+    v[3, 6:32] = np.abs(v[3, 6:32])
+    bias, qn, kn = (rng.standard_normal(n).astype(np.float32) for n in (qkv.shape[1], hd, hd))
+    bias[(nh + nkv) * hd:] = 0
+    bt, qnt, knt = (T(bias), T(qn), T(kn)) if norms else (None, None, None)
+    P = lambda x: x.buf.ptr if x is not None else None
+    qt, pt = T(qkv), F.Tensor(F.DeviceBuffer(4 * t), (t,), np.uint32)
+    where = np.array([3, 0, 8, 7, cap + 2], np.uint32)
+    F._lib.check(lib.fhip_memcpy_h2d(pt.buf.ptr, where.ctypes.data, 4 * t, None))
+    got = []
+    for one in (True, False):
+        kq, vq, qo = Q.QKvCache(fmt, cap, width), Q.QKvCache(fmt, cap, width), T(np.full((t, nh * hd), 7.0, np.float32))
+        for c in (kq, vq):
+            for b in (c.codes, c.scales):
+                fill = np.full(b.nbytes, 0x5A, np.uint8)
+                F._lib.check(lib.fhip_memcpy_h2d(b.ptr, fill.ctypes.data, b.nbytes, None))
+        if one:
+            F._lib.check(lib.fhip_qkv_post_kvq(fmt, qt.buf.ptr, P(bt), P(qnt), P(knt), pt.buf.ptr, None, t, nh, nkv, hd, n_rot, inter, 1e-6, 1e6, qo.buf.ptr,
+                                               kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, cap, None))
+        else:
+            k1, v1 = F.Tensor.empty((t, width)), F.Tensor.empty((t, width))
+            F._lib.check(lib.fhip_qkv_post_packed(qt.buf.ptr, P(bt), P(qnt), P(knt), pt.buf.ptr, None, t, nh, nkv, hd, n_rot, inter, 1e-6, 1e6, qo.buf.ptr,
+                                                  k1.buf.ptr, v1.buf.ptr, None))
+            F._lib.check(lib.fhip_kvq_append2(fmt, k1.buf.ptr, v1.buf.ptr, 0, t, width, pt.buf.ptr, 0, cap, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr,
+                                              vq.scales.ptr, None))
+        raw = [bits(qo.to_vec())]
+        for b in (kq.codes, kq.scales, vq.codes, vq.scales):
+            h = np.empty(b.nbytes, np.uint8)
+            F._lib.check(lib.fhip_memcpy_d2h(h.ctypes.data, b.ptr, b.nbytes, None))
+            raw.append(h)
+        got.append(raw)
+    for name, a, b in zip(("q", "k codes", "k scales", "v codes", "v scales"), *got):
+        assert np.array_equal(a, b), (name, np.flatnonzero(a != b)[:8])
+    c = kq
+    assert lib.fhip_qkv_post_kvq(fmt, qt.buf.ptr, None, None, None, pt.buf.ptr, None, 1, 1, 1, 288, 0, 0, 1e-6, 1e6, qt.buf.ptr, c.codes.ptr, c.scales.ptr, c.codes.ptr,
+                                 c.scales.ptr, cap, None) != 0 and b"multiple of 32" in lib.fhip_last_error()
