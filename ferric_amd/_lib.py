@@ -92,7 +92,7 @@ SYMBOLS = {
     "fhip_add_rmsnorm": (C.c_int, [_vp, _vp, _vp, _sz, _sz, C.c_float, _vp, _vp, _vp]),
     "fhip_add_rmsnorm_bf16": (C.c_int, [_vp, _vp, _vp, _sz, _sz, C.c_float, _vp, _vp, _vp]),
     "fhip_causal_attention_bf16": (C.c_int, [_vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, _sz, C.c_float, _vp, _vp]),
-    "fhip_ffn_bf16": (C.c_int, [_vp, _vp, _vp, _sz, _vp, _vp, _vp]),
+    "fhip_ffn_bf16": (C.c_int, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp]),
     "fhip_add": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
     "fhip_mul_sigmoid": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
     "fhip_kvq_sizes": (C.c_int, [C.c_int, _sz, _sz, C.POINTER(_sz), C.POINTER(_sz)]),

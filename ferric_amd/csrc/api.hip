@@ -1209,9 +1209,9 @@ size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gu, const fhip_weight* down, si
     return align256(rows_x * gu->cols * 2) + (ffn_coop_fused(rows_x) ? 0 : align256(rows_x * gu->rows * 4)) + align256(rows_x * down->cols * 2);
 }
 
-// d_x f32 (converted into the workspace first), or already bf16 in d_xb
-static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* down, const float* d_x, const uint16_t* d_xb, size_t rows_x, float* d_y,
-                    void* d_ws, hipStream_t s) {
+// d_x f32 (converted into the workspace first), or already bf16 in d_xb; d_gu: null, or where gate|up goes in f32 between two launches
+static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* down, const float* d_x, const uint16_t* d_xb, float* d_gu, size_t rows_x,
+                    float* d_y, void* d_ws, hipStream_t s) {
     int rc = need_init();
     if (rc) return rc;
     if (!gu || !down) return set_error(FHIP_ERR_ARG, "%s: NULL weight", who);
@@ -1223,11 +1223,12 @@ static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* d
     if (((uintptr_t)d_ws & 255) != 0) return set_error(FHIP_ERR_ARG, "%s: workspace must be 256-byte aligned", who);
     // an empty inner dimension on either side: gate and up are 0, silu(0) * 0 = 0, and so is every output
     if (gu->cols == 0 || n_ff == 0) return zero_outputs(rows_x, down->rows, d_y, s);
-    const bool fused = ffn_coop_fused(rows_x);
+    const bool in_tile = ffn_coop_fused(rows_x), fused = in_tile && !d_gu;
     uint8_t* ws = (uint8_t*)d_ws;
     uint16_t* xb = (uint16_t*)ws;
     float* g = (float*)(ws + align256(rows_x * gu->cols * 2));
-    uint16_t* hb = (uint16_t*)((uint8_t*)g + (fused ? 0 : align256(rows_x * gu->rows * 4)));
+    uint16_t* hb = (uint16_t*)((uint8_t*)g + (in_tile ? 0 : align256(rows_x * gu->rows * 4)));
+    if (d_gu) g = d_gu;
     if (!d_xb) {
         if ((rc = fhip::launch_cvt_bf16(d_x, rows_x * gu->cols, xb, s))) return rc;
         d_xb = xb;
@@ -1246,11 +1247,12 @@ static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* d
 
 int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
                   void* d_ws, void* stream) {
-    return ffn_coop("fhip_ffn_coop", gu, down, d_x, nullptr, rows_x, d_y, d_ws, (hipStream_t)stream);
+    return ffn_coop("fhip_ffn_coop", gu, down, d_x, nullptr, nullptr, rows_x, d_y, d_ws, (hipStream_t)stream);
 }
 
-int fhip_ffn_bf16(const fhip_weight* gu, const fhip_weight* down, const uint16_t* d_x_bf16, size_t rows_x, float* d_y, void* d_ws, void* stream) {
-    return ffn_coop("fhip_ffn_bf16", gu, down, nullptr, d_x_bf16, rows_x, d_y, d_ws, (hipStream_t)stream);
+int fhip_ffn_bf16(const fhip_weight* gu, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
+                  void* stream) {
+    return ffn_coop("fhip_ffn_bf16", gu, down, nullptr, d_x_bf16, d_gate_up, rows_x, d_y, d_ws, (hipStream_t)stream);
 }
 
 size_t fhip_matmul_q_f16x2_ws_bytes(const fhip_weight* w, size_t rows_x) {

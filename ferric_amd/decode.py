@@ -368,7 +368,9 @@ class Qwen3Decoder:
         att = E((t, self.q_out), np.float32 if self.gate is not None else rows)
         o, x1, y = E((t, c.d_model)), E((t, c.d_model)), E((t, c.d_model))
         normed = E((t, c.d_model)) if self.on is not None else None                   # a post-normed branch output
-        f, gu = E((t, c.n_ff)), (E((t, 2 * c.n_ff)) if c.geglu else None)
+        # On a quantized cache gate|up is formed apart from SwiGLU: a code follows every rounding in front of it, and a sum that the fused launch
+        # cuts elsewhere along K would move a tenth of the codes that later layers store.
+        f, gu = E((t, c.n_ff)), (E((t, 2 * c.n_ff)) if c.geglu or (self.kv_fmt is not None and not precise) else None)
         gate = E((t, self.q_out)) if self.gate is not None else None
         ws16 = DeviceBuffer(2 * t * max(c.d_model, self.q_out, c.n_ff) + 256)          # bf16 copies of the coop matmuls' inputs
         k1 = v1 = kd = vd = None
@@ -405,7 +407,8 @@ class Qwen3Decoder:
                 need = lib.fhip_ffn_coop_ws_bytes(l.ffn_gate_up.handle, l.ffn_down.handle, t)
                 if wsf[0] is None or wsf[0].nbytes < need:
                     wsf[0] = DeviceBuffer(max(need, 256))
-                _check(lib.fhip_ffn_bf16(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, t, out.buf.ptr, wsf[0].ptr, s))
+                _check(lib.fhip_ffn_bf16(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, gu.buf.ptr if gu is not None else None, t, out.buf.ptr,
+                                         wsf[0].ptr, s))
 
         pending = None                                   # the previous layer's FFN branch: joins the residual in the next norm's launch
         for l, kv in zip(self.layers, self.caches):

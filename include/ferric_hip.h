@@ -484,8 +484,12 @@ int fhip_matmul_q_coop(const fhip_weight* w, const float* d_x, size_t rows_x, fl
 size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gate_up, const fhip_weight* down, size_t rows_x);
 int fhip_ffn_coop(const fhip_weight* gate_up, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
                   void* d_ws, void* stream);
-/* The same on rows that are bf16 already (16-byte aligned); the same workspace, the same bits. */
-int fhip_ffn_bf16(const fhip_weight* gate_up, const fhip_weight* down, const uint16_t* d_x_bf16, size_t rows_x, float* d_y, void* d_ws, void* stream);
+/* The same on rows that are bf16 already (16-byte aligned); the same workspace. d_gate_up NULL: the same bits. Else f32 scratch
+ * [rows_x, gate_up rows], 16-byte aligned: gate|up is formed there as fhip_gemm_q_bf16 forms it and SwiGLU follows in a launch of its own
+ * -- above 32 rows the launch that applies SwiGLU itself may cut an output's sum along K elsewhere, a last-bit difference before
+ * the rounding to bf16. */
+int fhip_ffn_bf16(const fhip_weight* gate_up, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
+                  void* stream);
 
 /* crates/ferric-tensor/src/dtype.rs:935-944 Tensor::matmul_q for 1..32 activation rows in ONE pass over the weights
  * with f32-grade results (the reference's kernels, :2995-3051 and :3423-3469, walk the weight row once per activation

@@ -705,8 +705,16 @@ def test_rows_rounded_to_bf16_by_their_producer(F, X):
         x = T(rng.standard_normal((t, d)).astype(np.float32))
         ws, y = F.DeviceBuffer(lib.fhip_ffn_coop_ws_bytes(gu.handle, down.handle, t)), E((t, d))
         xb = x.cvt_bf16()
-        chk(lib.fhip_ffn_bf16(gu.handle, down.handle, xb.buf.ptr, t, y.buf.ptr, ws.ptr, None))
+        chk(lib.fhip_ffn_bf16(gu.handle, down.handle, xb.buf.ptr, None, t, y.buf.ptr, ws.ptr, None))
         assert np.array_equal(raw(x.ffn_coop(gu, down)), raw(y)), t
+        # gate|up in memory: the bits of the steps one by one
+        g, y2 = E((t, 2 * ff)), E((t, d))
+        chk(lib.fhip_ffn_bf16(gu.handle, down.handle, xb.buf.ptr, g.buf.ptr, t, y2.buf.ptr, ws.ptr, None))
+        h2 = xb.gemm_q_bf16(gu)
+        assert np.array_equal(raw(h2), raw(g)), t
+        f = E((t, ff))
+        chk(lib.fhip_swiglu(h2.buf.ptr, t, ff, f.buf.ptr, None))
+        assert np.array_equal(raw(f.cvt_bf16().gemm_q_bf16(down)), raw(y2)), t
     one = E((1, 8), np.uint16)
     assert lib.fhip_add_rmsnorm_bf16(wt.buf.ptr, bt.buf.ptr, wt.buf.ptr, 1, 2, 1e-6, None, one.buf.ptr, None) != 0       # a sum asked for and no place for it
     assert lib.fhip_causal_attention_bf16(q.buf.ptr, k.buf.ptr, v.buf.ptr, 1, 1, 1, 1, 64, 0, 0.0, one.buf.ptr.value + 8, None) != 0
