@@ -369,6 +369,7 @@ int fhip_stream_create(void** s) {
 int fhip_stream_destroy(void* s) {
     if (!s) return FHIP_OK;
     release_workspace((hipStream_t)s);   // the library's buffer for this stream goes with it
+    fhip::capture_ended((hipStream_t)s, true);
     return check_hip(hipStreamDestroy((hipStream_t)s), "hipStreamDestroy");
 }
 int fhip_stream_sync(void* s) { return check_hip(hipStreamSynchronize((hipStream_t)s), "hipStreamSynchronize"); }
@@ -394,17 +395,15 @@ int fhip_graph_capture_begin(void* s) {
     if (rc) return rc;
     if (!s) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_begin: needs a stream from fhip_stream_create");
     rc = check_hip(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    if (!rc) fhip::pool_capture_depth(1);
+    if (!rc) fhip::capture_begun((hipStream_t)s);
     return rc;
 }
 int fhip_graph_capture_end(void* s, void** graph_exec) {
     if (!s || !graph_exec) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_end: NULL argument");
     *graph_exec = nullptr;
     hipGraph_t g = nullptr;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)s, &st) != hipSuccess) (void)hipGetLastError();
     int rc = check_hip(hipStreamEndCapture((hipStream_t)s, &g), "hipStreamEndCapture");
-    if (st != hipStreamCaptureStatusNone) fhip::pool_capture_depth(-1);
+    fhip::capture_ended((hipStream_t)s, false);          // whatever came of it: the thread's capture is over
     if (rc) return rc;
     hipGraphExec_t ge = nullptr;
     rc = check_hip(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0), "hipGraphInstantiate");

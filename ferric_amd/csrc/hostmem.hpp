@@ -9,7 +9,9 @@ constexpr size_t WEIGHT_SLACK = 256;   // readable bytes every weight and every 
 int pool_malloc(void** out, size_t nbytes);
 int pool_free(void* ptr);
 void pool_trim();                      // gives every cached block back
-void pool_capture_depth(int delta);    // the calling thread opens (+1) or ends (-1) a stream capture
+void capture_begun(hipStream_t s);                       // the calling thread has opened a capture of s ...
+void capture_ended(hipStream_t s, bool destroyed);       // ... and has ended it, or (any thread) the stream is gone; nothing if it is another thread's
+bool thread_captures();                                  // the calling thread has a capture open
 bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the live block of pool_malloc that ptr lies in, as far as it was asked for
 int device_malloc(void** out, size_t n, const char* what);           // hipMalloc; with no memory left, once more after pool_trim
 

@@ -12,6 +12,7 @@
 // is drained at once instead of grown: the queue has most likely run empty since, and a new block would have to be mapped.
 #include "hostmem.hpp"
 
+#include <atomic>
 #include <chrono>
 #include <map>
 #include <mutex>
@@ -41,7 +42,20 @@ struct Pool {
 // never destroyed: objects of a host program may be freed after static destructors have begun to run
 Pool& pool() { static Pool* p = new Pool(); return *p; }
 
-thread_local int t_capturing = 0;   // captures this thread has open: no wait and no free may happen inside one
+// The captures that fhip_graph_capture_begin opened and that have not ended, each with the thread it belongs to (the runtime lets no
+// other thread end it). A thread that captures may not wait for the device nor map or unmap memory: the runtime refuses and
+// invalidates the capture, and the stream then takes no work until it has been through another capture.
+struct Captures {
+    std::mutex mu;
+    std::map<hipStream_t, uint64_t> owner;
+    std::atomic<size_t> open{0};                       // = owner.size(), for threads that only want to know that there is none
+};
+Captures& captures() { static Captures* c = new Captures(); return *c; }
+uint64_t this_thread() {
+    static std::atomic<uint64_t> last{0};
+    thread_local const uint64_t id = ++last;
+    return id;
+}
 
 // Eight classes per power of two: at most an eighth of a block is not asked for.
 size_t size_class(size_t n) {
@@ -84,7 +98,38 @@ void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
 
 namespace fhip {
 
-void pool_capture_depth(int delta) { t_capturing += delta; }
+void capture_begun(hipStream_t s) {
+    Captures& c = captures();
+    std::lock_guard<std::mutex> lock(c.mu);
+    c.owner[s] = this_thread();
+    c.open = c.owner.size();
+}
+
+void capture_ended(hipStream_t s, bool destroyed) {
+    Captures& c = captures();
+    std::lock_guard<std::mutex> lock(c.mu);
+    auto it = c.owner.find(s);
+    if (it == c.owner.end() || (!destroyed && it->second != this_thread())) return;
+    c.owner.erase(it);
+    c.open = c.owner.size();
+}
+
+bool thread_captures() {
+    Captures& c = captures();
+    if (c.open.load(std::memory_order_relaxed) == 0) return false;
+    std::lock_guard<std::mutex> lock(c.mu);
+    bool any = false;
+    for (auto it = c.owner.begin(); it != c.owner.end();) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (it->second != this_thread()) { ++it; continue; }
+        if (hipStreamIsCapturing(it->first, &st) != hipSuccess) (void)hipGetLastError();
+        if (st == hipStreamCaptureStatusNone) { it = c.owner.erase(it); continue; }   // ended or destroyed through the runtime itself
+        any = true;
+        ++it;
+    }
+    c.open = c.owner.size();
+    return any;
+}
 
 void pool_trim() {
     Pool& p = pool();
@@ -114,6 +159,7 @@ int pool_malloc(void** out, size_t nbytes) {
     if (rc) return rc;
     if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) return device_malloc(out, need, "hipMalloc");
     Pool& p = pool();
+    const bool capturing = thread_captures();
     for (bool waited = false;;) {
         std::vector<std::pair<size_t, std::vector<void*>>> dirty;
         {
@@ -127,7 +173,7 @@ int pool_malloc(void** out, size_t nbytes) {
                 p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
                 return FHIP_OK;
             }
-            if (waited || t_capturing || c.dirty.empty()) break;
+            if (waited || capturing || c.dirty.empty()) break;
             if (c.dirty.size() < keep_blocks(cls) &&
                 (cls < LARGE || std::chrono::steady_clock::now() - c.last_free < std::chrono::milliseconds(1))) break;
             // every dirty block of the device leaves its list while the lock is given up for the wait: another thread that
@@ -170,7 +216,7 @@ int pool_free(void* ptr) {
             c.last_use = ++p.clock;
             if (b.cls >= LARGE) c.last_free = std::chrono::steady_clock::now();
             p.cached[b.dev] += b.cls;
-            if (!t_capturing && p.cached[b.dev] > POOL_CACHED_MAX) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
+            if (p.cached[b.dev] > POOL_CACHED_MAX && !thread_captures()) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
         }
     }
     int rc = FHIP_OK;
