@@ -94,6 +94,19 @@ void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
     }
 }
 
+// Whether hipMalloc would give the calling thread memory now. A cached block must not go where a new one could not: a thread that captures
+// a stream through the runtime itself would have a graph go on using scratch that its operator has freed. The thread's mode is
+// thread-local meanwhile, so that the question does not invalidate a global capture of another thread.
+bool runtime_allocates() {
+    hipStreamCaptureMode mode = hipStreamCaptureModeThreadLocal;
+    void* none = nullptr;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipMalloc(&none, 0);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
 }  // namespace
 
 namespace fhip {
@@ -153,14 +166,17 @@ int device_malloc(void** out, size_t n, const char* what) {
 
 int pool_malloc(void** out, size_t nbytes) {
     *out = nullptr;
+    if (thread_captures())
+        return set_error(FHIP_ERR_HIP, "fhip_malloc: not while the thread captures a stream (the graph would go on using the memory after it is freed): allocate "
+                         "before the capture begins");
     const size_t need = nbytes + WEIGHT_SLACK, cls = size_class(need);
     int dev = 0;
     int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
     if (rc) return rc;
     if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) return device_malloc(out, need, "hipMalloc");
     Pool& p = pool();
-    const bool capturing = thread_captures();
-    for (bool waited = false;;) {
+    const bool cached = runtime_allocates();           // otherwise the runtime is asked for a new block, and says why not
+    for (bool waited = false; cached;) {
         std::vector<std::pair<size_t, std::vector<void*>>> dirty;
         {
             std::lock_guard<std::mutex> lock(p.mu);
@@ -173,7 +189,7 @@ int pool_malloc(void** out, size_t nbytes) {
                 p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
                 return FHIP_OK;
             }
-            if (waited || capturing || c.dirty.empty()) break;
+            if (waited || c.dirty.empty()) break;
             if (c.dirty.size() < keep_blocks(cls) &&
                 (cls < LARGE || std::chrono::steady_clock::now() - c.last_free < std::chrono::milliseconds(1))) break;
             // every dirty block of the device leaves its list while the lock is given up for the wait: another thread that

@@ -86,7 +86,8 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
  * (crates/ferric-tensor/src/lib.rs:1481 empty(), :141 to_vec(), :1816 readback). */
 /* Freed blocks are kept (up to 2 GiB a device, none above 768 MiB; fhip_workspace_release gives them back, as does an allocation
  * that finds no memory) for later fhip_malloc calls. A block may be freed while work that uses it is still enqueued, on any stream:
- * it is not handed out again before the device has been idle once since the free. */
+ * it is not handed out again before the device has been idle once since the free. fhip_malloc fails (FHIP_ERR_HIP) while the calling
+ * thread captures a stream: what a captured call uses has to outlive the graph, so it is allocated before the capture begins. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
 /* async on stream; a source of up to 640 KiB has been read when the call returns (not in a stream capture) */

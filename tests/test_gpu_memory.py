@@ -48,3 +48,69 @@ def test_a_stream_destroyed_while_it_captures_ends_the_capture(F):
     handle, s.handle = s.handle, None
     F._lib.check(F._lib.load().fhip_stream_destroy(handle))
     assert blocks_in_turn(F, 11000) <= 64
+
+
+def _allocating_calls(F):
+    """Operators that allocate (their result, most of them scratch of their own too), each as a call on a stream."""
+    from ferric_amd import decode, kvquant
+    from ferric_amd.synth import synth_weights
+    rng = np.random.default_rng(0)
+    t = lambda *shape: F.Tensor.from_vec(rng.standard_normal(shape).astype(np.float32), shape)
+    w = lambda ty, rows, cols: F.QMatrix.from_bytes(synth_weights(ty, rows, cols, rows), ty, rows, cols)
+    x, x40, gu, down = t(8, 512), t(40, 512), w(F.Q4_K, 1024, 512), w(F.Q6_K, 512, 512)
+    slab, sel, slots = w(F.Q4_K, 4 * 256, 512), F.Tensor.from_vec(np.array([[0.5, 0.5, 1, 3]], np.float32), (1, 4)), t(1, 2, 512)
+    q, cache = t(1, 512), decode.KvCache(3000, 256).append2(t(3000, 256), t(3000, 256))
+    kvq = [kvquant.QKvCache(kvquant.Q8_0, 3000, 256).append(t(3000, 256)) for _ in range(2)]
+    return {
+        "a buffer": lambda s: F.DeviceBuffer(5000),
+        "matmul_q": lambda s: x.matmul_q(gu, s),
+        "matmul_q_coop": lambda s: x40.matmul_q_coop(gu, s),
+        "matmul_q_f16x2": lambda s: x.matmul_q_f16x2(gu, s),
+        "ffn": lambda s: x.ffn(gu, down, s),
+        "ffn_f16x2": lambda s: x.ffn_f16x2(gu, down, s),
+        "ffn_coop": lambda s: x40.ffn_coop(gu, down, s),
+        "matmul_q_id_wsum": lambda s: slots.matmul_q_id_wsum(slab, sel, 256, s),
+        "rope": lambda s: decode.rope(q, 4, 128, 1e6, positions=[7], stream=s),
+        "decode_attention": lambda s: decode.decode_attention(q, cache, 4, 2, stream=s),
+        "decode_attention_kvq": lambda s: decode.decode_attention_kvq(q, *kvq, 4, 2, stream=s),
+    }
+
+
+@pytest.fixture(scope="module")
+def allocating_calls(F):
+    return _allocating_calls(F)
+
+
+@pytest.mark.parametrize("name", ["a buffer", "matmul_q", "matmul_q_coop", "matmul_q_f16x2", "ffn", "ffn_f16x2", "ffn_coop", "matmul_q_id_wsum", "rope", "decode_attention",
+                                  "decode_attention_kvq"])
+def test_nothing_is_allocated_inside_a_capture(F, allocating_calls, name):
+    """The graph would use the scratch again after the pool has given it to somebody else. The calls have run before, so that the pool
+    holds blocks for all of it; the capture goes on after the refusal."""
+    s, call = F.Stream(), allocating_calls[name]
+    word = F.Tensor.from_vec(np.zeros(4, np.float32), (4,))
+    for _ in range(2):
+        call(s)
+        blocks_in_turn(F, 13000)                 # has waited for the device: what the call freed can be handed out
+    g = F.Graph.begin(s)
+    with pytest.raises(F._lib.FerricHipError, match="captures a stream"):
+        call(s)
+    F._lib.check(F._lib.load().fhip_u32_add(word.buf.ptr, 1, 1, s.handle))
+    g.end()
+    for _ in range(3):
+        g.launch()
+        s.synchronize()
+    assert word.to_vec(s).view(np.uint32)[0] == 3
+    call(s)
+
+
+def test_nothing_is_allocated_inside_a_capture_through_the_runtime(F):
+    """hipMalloc refuses such a thread, and so does the pool, though it holds blocks of the size."""
+    hip = C.CDLL("libamdhip64.so.7")
+    s, graph = F.Stream(), C.c_void_p()
+    blocks_in_turn(F, 15000)
+    assert hip.hipStreamBeginCapture(s.handle, 1) == 0
+    with pytest.raises(F._lib.FerricHipError):
+        F.DeviceBuffer(15000)
+    assert hip.hipStreamEndCapture(s.handle, C.byref(graph)) != 0       # the runtime invalidates what it refuses
+    hip.hipGetLastError()                                               # (or the next launch would report it)
+    F.DeviceBuffer(15000)
