@@ -362,15 +362,14 @@ int fhip_stream_create(void** s) {
     int rc = need_init();
     if (rc) return rc;
     hipStream_t st;
-    rc = check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
+    rc = fhip::stream_create(&st);
     *s = rc ? nullptr : (void*)st;
     return rc;
 }
 int fhip_stream_destroy(void* s) {
     if (!s) return FHIP_OK;
     release_workspace((hipStream_t)s);   // the library's buffer for this stream goes with it
-    fhip::capture_ended((hipStream_t)s, true);
-    return check_hip(hipStreamDestroy((hipStream_t)s), "hipStreamDestroy");
+    return fhip::stream_destroy((hipStream_t)s);
 }
 int fhip_stream_sync(void* s) { return check_hip(hipStreamSynchronize((hipStream_t)s), "hipStreamSynchronize"); }
 int fhip_event_create(void** e) {

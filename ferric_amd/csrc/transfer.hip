@@ -141,7 +141,7 @@ struct Ring {                    // one per device
         for (int tries = 0; tries < 1 << 20; tries++) {
             if (Slot* q = take(rc)) return q;
             if (*rc) return nullptr;
-            if (tries == 1 << 14 && (*rc = fhip::check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize"))) return nullptr;
+            if (tries == 1 << 14 && (*rc = fhip::device_wait())) return nullptr;
             std::this_thread::yield();
         }
         *rc = fhip::set_error(FHIP_ERR_HIP, "transfer: no pinned slot came free");

@@ -114,3 +114,21 @@ def test_nothing_is_allocated_inside_a_capture_through_the_runtime(F):
     assert hip.hipStreamEndCapture(s.handle, C.byref(graph)) != 0       # the runtime invalidates what it refuses
     hip.hipGetLastError()                                               # (or the next launch would report it)
     F.DeviceBuffer(15000)
+
+
+def test_other_threads_allocate_and_copy_while_one_captures(F):
+    """Their waits for the device must leave the capture alone (hipDeviceSynchronize would fail and invalidate it)."""
+    lib, check = F._lib.load(), F._lib.check
+    s, word = F.Stream(), F.Tensor.from_vec(np.zeros(4, np.float32), (4,))
+    g = F.Graph.begin(s)
+    check(lib.fhip_u32_add(word.buf.ptr, 1, 1, s.handle))
+    with ThreadPoolExecutor(1) as other:
+        assert other.submit(blocks_in_turn, F, 17000).result() <= 64
+        a = np.arange(3 * MIB, dtype=np.float32)
+        assert np.array_equal(other.submit(lambda: F.Tensor.from_vec(a, a.shape).to_vec()).result(), a)
+    check(lib.fhip_u32_add(word.buf.ptr, 1, 1, s.handle))
+    g.end()
+    for _ in range(3):
+        g.launch()
+        s.synchronize()
+    assert word.to_vec(s).view(np.uint32)[0] == 6
