@@ -12,7 +12,7 @@ void pool_trim();                      // gives every cached block back
 void capture_begun(hipStream_t s);                       // the calling thread has opened a capture of s ...
 void capture_ended(hipStream_t s, bool destroyed);       // ... and has ended it, or (any thread) the stream is gone; nothing if it is another thread's
 bool thread_captures();                                  // the calling thread has a capture open
-bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the live block of pool_malloc that ptr lies in, as far as it was asked for
+bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the block in use that ptr lies in, as far as it was asked for
 int stream_create(hipStream_t* s);      // a stream of the library's own ...
 int stream_destroy(hipStream_t s);     // ... and its end (any stream is taken)
 int device_wait();                     // until all work enqueued on the current device has ended; captures of other threads go on

@@ -27,15 +27,22 @@ constexpr size_t POOL_CACHED_MAX = (size_t)2 << 30;    // cached bytes per devic
 constexpr size_t LARGE = (size_t)1 << 20;              // blocks whose mapping costs more than a wait for an idle device
 constexpr int MAX_DEVICES = 64;
 
-struct Live { size_t asked, cls; int dev; };
+// Every block fhip_malloc has from the runtime, in use or cached: a free has to know the ones that are free already.
+struct Block {
+    size_t asked, cls;                                 // cls: bytes there are
+    int dev;
+    bool pooled, live;
+};
+typedef std::map<uintptr_t, Block> Blocks;             // by address: fhip_weight_wrap_device looks up ranges
+typedef std::vector<Blocks::iterator> Cached;
 struct SizeClass {
-    std::vector<void*> clean, dirty;
+    Cached clean, dirty;
     uint64_t last_use = 0;
     std::chrono::steady_clock::time_point last_free;
 };
 struct Pool {
     std::mutex mu;
-    std::map<uintptr_t, Live> live;                    // by address: fhip_weight_wrap_device looks up ranges
+    Blocks blocks;
     std::map<size_t, SizeClass> classes[MAX_DEVICES];
     size_t cached[MAX_DEVICES] = {};
     uint64_t clock = 0;
@@ -88,7 +95,8 @@ size_t keep_blocks(size_t cls) {
     return k < 2 ? 2 : (k > 64 ? 64 : k);
 }
 
-// Under p.mu: blocks out of the classes of `dev` that were unused longest, until at most `target` bytes stay cached.
+// Under p.mu: blocks out of the classes of `dev` that were unused longest, until at most `target` bytes stay cached. They are no blocks
+// of the pool any more.
 void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
     auto& cs = p.classes[dev];
     while (p.cached[dev] > target) {
@@ -102,7 +110,8 @@ void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
         if (!oldest) return;
         for (auto* list : {&oldest->clean, &oldest->dirty})
             while (!list->empty() && p.cached[dev] > target) {
-                out.push_back(list->back());
+                out.push_back((void*)list->back()->first);
+                p.blocks.erase(list->back());
                 list->pop_back();
                 p.cached[dev] -= bytes;
             }
@@ -232,20 +241,27 @@ int pool_malloc(void** out, size_t nbytes) {
     int dev = 0;
     int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
     if (rc) return rc;
-    if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) return device_malloc(out, need, "hipMalloc");
     Pool& p = pool();
+    if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) {
+        if ((rc = device_malloc(out, need, "hipMalloc"))) return rc;
+        std::lock_guard<std::mutex> lock(p.mu);
+        p.blocks[(uintptr_t)*out] = Block{nbytes, need, dev, false, true};
+        return FHIP_OK;
+    }
     const bool cached = runtime_allocates();           // otherwise the runtime is asked for a new block, and says why not
     for (bool waited = false; cached;) {
-        std::vector<std::pair<size_t, std::vector<void*>>> dirty;
+        std::vector<std::pair<size_t, Cached>> dirty;
         {
             std::lock_guard<std::mutex> lock(p.mu);
             SizeClass& c = p.classes[dev][cls];
             c.last_use = ++p.clock;
             if (!c.clean.empty()) {
-                *out = c.clean.back();
+                Blocks::iterator b = c.clean.back();
                 c.clean.pop_back();
                 p.cached[dev] -= cls;
-                p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
+                b->second.asked = nbytes;
+                b->second.live = true;
+                *out = (void*)b->first;
                 return FHIP_OK;
             }
             if (waited || c.dirty.empty()) break;
@@ -255,7 +271,7 @@ int pool_malloc(void** out, size_t nbytes) {
             // comes for one of them meanwhile makes a new block
             for (auto& k : p.classes[dev])
                 if (!k.second.dirty.empty()) {
-                    dirty.emplace_back(k.first, std::vector<void*>());
+                    dirty.emplace_back(k.first, Cached());
                     dirty.back().second.swap(k.second.dirty);
                 }
         }
@@ -271,7 +287,7 @@ int pool_malloc(void** out, size_t nbytes) {
     }
     if ((rc = device_malloc(out, cls, "hipMalloc"))) return rc;
     std::lock_guard<std::mutex> lock(p.mu);
-    p.live[(uintptr_t)*out] = Live{nbytes, cls, dev};
+    p.blocks[(uintptr_t)*out] = Block{nbytes, cls, dev, true, true};
     return FHIP_OK;
 }
 
@@ -280,14 +296,19 @@ int pool_free(void* ptr) {
     std::vector<void*> over;
     {
         std::lock_guard<std::mutex> lock(p.mu);
-        auto it = p.live.find((uintptr_t)ptr);
-        if (it == p.live.end()) {
-            over.push_back(ptr);            // a block too large for the pool
+        auto it = p.blocks.find((uintptr_t)ptr);
+        if (it == p.blocks.end()) {
+            over.push_back(ptr);            // not of fhip_malloc: the runtime knows it, or says that it does not
+        } else if (!it->second.live) {
+            return set_error(FHIP_ERR_ARG, "fhip_free: the block has been freed already");
+        } else if (!it->second.pooled) {
+            p.blocks.erase(it);
+            over.push_back(ptr);
         } else {
-            const Live b = it->second;
-            p.live.erase(it);
+            Block& b = it->second;
+            b.live = false;
             SizeClass& c = p.classes[b.dev][b.cls];
-            c.dirty.push_back(ptr);
+            c.dirty.push_back(it);
             c.last_use = ++p.clock;
             if (b.cls >= LARGE) c.last_free = std::chrono::steady_clock::now();
             p.cached[b.dev] += b.cls;
@@ -305,10 +326,10 @@ int pool_free(void* ptr) {
 bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end) {
     Pool& p = pool();
     std::lock_guard<std::mutex> lock(p.mu);
-    auto it = p.live.upper_bound((uintptr_t)ptr);
-    if (it == p.live.begin()) return false;
+    auto it = p.blocks.upper_bound((uintptr_t)ptr);
+    if (it == p.blocks.begin()) return false;
     --it;
-    if ((uintptr_t)ptr >= it->first + it->second.cls) return false;
+    if (!it->second.live || (uintptr_t)ptr >= it->first + it->second.cls) return false;
     *base = it->first;
     *end = it->first + it->second.asked + WEIGHT_SLACK;
     return true;

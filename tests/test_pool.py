@@ -1,0 +1,92 @@
+"""The device memory pool (ferric_amd/csrc/memory.hip) on the CPU, over a runtime that only hands out addresses: what has to be refused, what may
+be handed out again, and what a capture on one thread means for the others."""
+import ctypes as C
+import os
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+from conftest import ROOT
+
+KIB, MIB, GIB = 1 << 10, 1 << 20, 1 << 30
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    d = tmp_path_factory.mktemp("pool")
+    obj = str(d / "pool.o")
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "--offload-arch=gfx950", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-c",
+                    os.path.join(ROOT, "tests", "pool_harness.cpp"), "-o", obj], check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    return obj
+
+
+class Pool:
+    def __init__(self, obj, path):
+        subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", path, obj, "-lpthread"], check=True)
+        self.c = C.CDLL(path)
+        for name, res, args in (("h_malloc", C.c_int, [C.c_size_t, C.c_void_p]), ("h_free", C.c_int, [C.c_void_p]), ("h_range", C.c_size_t, [C.c_void_p]),
+                                ("h_stream", C.c_void_p, []), ("h_stream_destroy", C.c_int, [C.c_void_p]), ("h_begin", None, [C.c_void_p, C.c_int]),
+                                ("h_end", C.c_int, [C.c_void_p]), ("h_bytes", C.c_size_t, []), ("h_text", C.c_char_p, []), ("h_trim", None, [])):
+            getattr(self.c, name).restype, getattr(self.c, name).argtypes = res, args
+
+    def malloc(self, n):
+        """(return code, address)"""
+        p = C.c_void_p(1)
+        rc = self.c.h_malloc(n, C.byref(p))
+        return rc, p.value
+
+    def new(self, n):
+        rc, p = self.malloc(n)
+        assert rc == 0 and p
+        return p
+
+
+@pytest.fixture
+def pool(library, tmp_path):
+    return Pool(library, str(tmp_path / "pool.so"))       # a copy of its own: the pool is as old as the library
+
+
+@pytest.mark.parametrize("n", [0, 100, 5000, 3 * MIB, 900 * MIB])
+def test_a_second_free_is_refused(pool, n):
+    """Also of a block that has been clean for a while, and of one too large to be kept. Nothing is given to two owners afterwards."""
+    p = pool.new(n)
+    assert pool.c.h_range(p) == n + 256
+    assert pool.c.h_free(p) == 0 and pool.c.h_range(p) == 0
+    held = pool.c.h_bytes()
+    assert pool.c.h_free(p) != 0
+    for _ in range(80):
+        assert pool.c.h_free(pool.new(n + 8)) == 0        # of the same class; has waited for the device meanwhile
+    assert pool.c.h_free(p) != 0 and pool.c.h_bytes() >= held
+    mine = [pool.new(n) for _ in range(5)]
+    assert len(set(mine)) == 5 and all(pool.c.h_range(q) == n + 256 for q in mine)
+    assert [pool.c.h_free(q) for q in mine] == [0] * 5
+
+
+def test_a_block_is_handed_out_again_only_after_the_device_was_idle(pool):
+    for n in (2000, 700 * KIB, 300 * MIB):
+        freed_under_work = set()
+        for _ in range(300):
+            p = pool.new(n)
+            if not pool.c.h_busy():
+                freed_under_work.clear()
+            assert p not in freed_under_work
+            pool.c.h_work()
+            freed_under_work.add(p)
+            pool.c.h_free(p)
+        assert pool.c.h_waits() > 0
+
+
+def test_cached_memory_is_bounded_and_given_back(pool):
+    blocks = [pool.new(100 * MIB + k) for k in range(40)]
+    for p in blocks:
+        assert pool.c.h_free(p) == 0
+    assert pool.c.h_bytes() <= 2 * GIB
+    assert all(pool.c.h_free(p) != 0 for p in blocks)     # the cached ones and those the runtime has back
+    pool.c.h_trim()
+    assert pool.c.h_bytes() == 0
+    big = [pool.new(6 * GIB), pool.new(GIB)]               # what the pool holds back is not what is missing
+    pool.c.h_free(big[0])
+    pool.new(500 * MIB)
+    pool.c.h_free(pool.new(700 * MIB))
+    pool.new(6 * GIB)
