@@ -79,7 +79,7 @@ struct OwnStreams {
 };
 OwnStreams& own_streams() { static OwnStreams* o = new OwnStreams(); return *o; }
 
-// Eight classes per power of two: at most an eighth of a block is not asked for.
+// Eight classes per power of two: at most an eighth of a block is not asked for. n: up to POOL_BLOCK_MAX, which is a class of its own.
 size_t size_class(size_t n) {
     if (n <= 1024) return 1024;
     const int top = 63 - __builtin_clzll((unsigned long long)n - 1);   // 2^top < n <= 2^(top + 1)
@@ -237,17 +237,19 @@ int pool_malloc(void** out, size_t nbytes) {
     if (thread_captures())
         return set_error(FHIP_ERR_HIP, "fhip_malloc: not while the thread captures a stream (the graph would go on using the memory after it is freed): allocate "
                          "before the capture begins");
-    const size_t need = nbytes + WEIGHT_SLACK, cls = size_class(need);
+    if (nbytes > SIZE_MAX - WEIGHT_SLACK) return check_hip(hipErrorOutOfMemory, "fhip_malloc");
+    const size_t need = nbytes + WEIGHT_SLACK;
     int dev = 0;
     int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
     if (rc) return rc;
     Pool& p = pool();
-    if (need < nbytes || cls > POOL_BLOCK_MAX || dev >= MAX_DEVICES) {
+    if (need > POOL_BLOCK_MAX || dev >= MAX_DEVICES) {
         if ((rc = device_malloc(out, need, "hipMalloc"))) return rc;
         std::lock_guard<std::mutex> lock(p.mu);
         p.blocks[(uintptr_t)*out] = Block{nbytes, need, dev, false, true};
         return FHIP_OK;
     }
+    const size_t cls = size_class(need);
     const bool cached = runtime_allocates();           // otherwise the runtime is asked for a new block, and says why not
     for (bool waited = false; cached;) {
         std::vector<std::pair<size_t, Cached>> dirty;

@@ -90,3 +90,18 @@ def test_cached_memory_is_bounded_and_given_back(pool):
     pool.new(500 * MIB)
     pool.c.h_free(pool.new(700 * MIB))
     pool.new(6 * GIB)
+
+
+@pytest.mark.parametrize("n", [9 * GIB, 1 << 60, (1 << 63) + 5, (1 << 64) - (1 << 60), (1 << 64) - (1 << 60) - 256, (1 << 64) - 1000, (1 << 64) - 257, (1 << 64) - 256, (1 << 64) - 1])
+def test_a_size_that_no_device_has_is_refused(pool, n):
+    """Among them negative counts cast to size_t; none may come out as a small class or a null pointer."""
+    for _ in range(2):
+        rc, p = pool.malloc(n)
+        assert rc != 0 and not p and pool.c.h_bytes() == 0
+
+
+@pytest.mark.parametrize("n", [0, 1, 768, 769, 1024, 1025, 64 * KIB - 256, 64 * KIB - 255, MIB, 512 * MIB - 256, 512 * MIB - 255, 768 * MIB - 257, 768 * MIB - 256, 768 * MIB - 255])
+def test_a_block_holds_what_was_asked_for(pool, n):
+    p = pool.new(n)
+    assert n + 256 <= pool.c.h_bytes() <= max(1024, (n + 256) * 9 // 8) and pool.c.h_range(p) == n + 256
+    assert pool.c.h_range(p + n + 255) == 1
