@@ -165,6 +165,7 @@ bool thread_captures() {
 }
 
 void pool_trim() {
+    if (thread_captures() || !runtime_allocates()) return;   // hipFree would refuse, and the blocks would be nobody's
     Pool& p = pool();
     std::vector<void*> out;
     {
@@ -314,7 +315,7 @@ int pool_free(void* ptr) {
             c.last_use = ++p.clock;
             if (b.cls >= LARGE) c.last_free = std::chrono::steady_clock::now();
             p.cached[b.dev] += b.cls;
-            if (p.cached[b.dev] > POOL_CACHED_MAX && !thread_captures()) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
+            if (p.cached[b.dev] > POOL_CACHED_MAX && !thread_captures() && runtime_allocates()) take_oldest(p, b.dev, POOL_CACHED_MAX, over);
         }
     }
     int rc = FHIP_OK;

@@ -105,3 +105,45 @@ def test_a_block_holds_what_was_asked_for(pool, n):
     p = pool.new(n)
     assert n + 256 <= pool.c.h_bytes() <= max(1024, (n + 256) * 9 // 8) and pool.c.h_range(p) == n + 256
     assert pool.c.h_range(p + n + 255) == 1
+
+
+@pytest.mark.parametrize("through_library", [0, 1])
+def test_a_thread_that_captures_gets_no_memory_and_loses_none(pool, through_library):
+    """Cached blocks of the size or not. What it frees stays with the pool, past the bound too, and is given back later. A capture that
+    the pool knows of stays valid."""
+    cached, big = [pool.new(3000) for _ in range(3)], [pool.new(300 * MIB) for _ in range(9)]
+    for p in cached:
+        pool.c.h_free(p)
+    for _ in range(70):
+        pool.c.h_free(pool.new(9000))                      # has waited: the three are clean
+    s = pool.c.h_stream()
+    pool.c.h_begin(s, through_library)
+    held = pool.c.h_bytes()
+    for n in (3000, 300 * MIB, GIB):
+        assert pool.malloc(n)[0] != 0
+    for p in big:
+        assert pool.c.h_free(p) == 0
+    pool.c.h_trim()
+    assert pool.c.h_bytes() == held
+    assert pool.c.h_end(s) == (0 if through_library else 1)
+    pool.c.h_free(pool.new(300 * MIB))
+    assert pool.c.h_bytes() <= 2 * GIB
+    pool.c.h_trim()
+    assert pool.c.h_bytes() == 0
+    assert pool.c.h_stream_destroy(s) == 0
+
+
+def test_a_capture_ends_with_its_thread_or_its_stream(pool):
+    a, b = pool.c.h_stream(), pool.c.h_stream()
+    with ThreadPoolExecutor(1) as other:
+        pool.c.h_begin(a, 1)
+        assert other.submit(pool.c.h_end, a).result() == 2
+        assert pool.malloc(100)[0] != 0 and other.submit(pool.malloc, 100).result()[0] == 0
+        for _ in range(200):                               # the other thread's waits
+            assert other.submit(pool.c.h_free, other.submit(pool.new, 5000).result()).result() == 0
+        assert pool.c.h_waits() > 0 and pool.c.h_end(a) == 0
+        pool.c.h_begin(a, 1)
+        pool.c.h_begin(b, 1)
+        assert pool.c.h_end(a) == 0 and pool.malloc(100)[0] != 0
+        pool.c.h_stream_destroy(b)
+        pool.new(100)
