@@ -25,6 +25,7 @@ SYMBOLS = {
     "fhip_malloc": (C.c_int, [C.POINTER(_vp), _sz]),
     "fhip_free": (C.c_int, [_vp]),
     "fhip_memcpy_h2d": (C.c_int, [_vp, _vp, _sz, _vp]),
+    "fhip_upload": (C.c_int, [_vp, _vp, _sz, _vp]),
     "fhip_memcpy_d2h": (C.c_int, [_vp, _vp, _sz, _vp]),
     "fhip_memcpy_d2d": (C.c_int, [_vp, _vp, _sz, _vp]),
     "fhip_memcpy_2d_d2d": (C.c_int, [_vp, _sz, _vp, _sz, _sz, _sz, _vp]),

@@ -336,6 +336,11 @@ int fhip_memcpy_h2d(void* d, const void* h, size_t n, void* s) {
     if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_memcpy_h2d: NULL pointer");
     return fhip::copy_h2d(d, h, n, (hipStream_t)s);
 }
+int fhip_upload(void* d, const void* h, size_t n, void* s) {
+    if (n == 0) return FHIP_OK;
+    if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_upload: NULL pointer");
+    return fhip::upload(d, h, n, (hipStream_t)s);
+}
 int fhip_memcpy_d2h(void* h, const void* d, size_t n, void* s) {
     if (n == 0) return FHIP_OK;
     if (!d || !h) return set_error(FHIP_ERR_ARG, "fhip_memcpy_d2h: NULL pointer");

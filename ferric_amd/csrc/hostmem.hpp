@@ -11,7 +11,8 @@ int pool_free(void* ptr);
 void pool_trim();                      // gives every cached block back
 void capture_begun(hipStream_t s);                       // the calling thread has opened a capture of s ...
 void capture_ended(hipStream_t s, bool destroyed);       // ... and has ended it, or (any thread) the stream is gone; nothing if it is another thread's
-bool thread_captures();                                  // the calling thread has a capture open
+bool thread_captures();                                  // the calling thread has a capture open (of those)
+bool runtime_allocates();                                // the runtime permits the calling thread to allocate and to wait: it has no capture open at all
 bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the block in use that ptr lies in, as far as it was asked for
 int stream_create(hipStream_t* s);      // a stream of the library's own ...
 int stream_destroy(hipStream_t s);     // ... and its end (any stream is taken)
@@ -21,7 +22,8 @@ int device_malloc(void** out, size_t n, const char* what);           // hipMallo
 // transfer.hip: copies through pinned memory of the library's own; both directions and the host-to-host unpackers
 constexpr size_t H2D_STAGED = (size_t)640 << 10;   // up to here copy_h2d has read its source when it returns
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s);
-int copy_d2h(void* h, const void* d, size_t n, hipStream_t s);   // synchronises
+int upload(void* d, const void* h, size_t n, hipStream_t s);     // copy_h2d that has read its source when it returns; refused in a capture
+int copy_d2h(void* h, const void* d, size_t n, hipStream_t s);   // synchronises; refused in a capture
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nblocks, size_t block_values, size_t block_bytes, float* h_out);   // synchronises
 
 }  // namespace fhip

@@ -118,15 +118,6 @@ void take_oldest(Pool& p, int dev, size_t target, std::vector<void*>& out) {
     }
 }
 
-// Whether hipMalloc would give the calling thread memory now. A cached block must not go where a new one could not: a thread that captures
-// a stream through the runtime itself would have a graph go on using scratch that its operator has freed. (70 ns)
-bool runtime_allocates() {
-    void* none = nullptr;
-    if (hipMalloc(&none, 0) == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
-}
-
 }  // namespace
 
 namespace fhip {
@@ -221,6 +212,15 @@ int device_wait() {
     if (e != hipErrorOutOfMemory) return check_hip(e, "waiting for the device");
     (void)hipGetLastError();
     return check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+}
+
+// A cached block must not go where a new one could not: a thread that captures a stream through the runtime itself would have a graph go
+// on using scratch that its operator has freed. (70 ns)
+bool runtime_allocates() {
+    void* none = nullptr;
+    if (hipMalloc(&none, 0) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 int device_malloc(void** out, size_t n, const char* what) {

@@ -329,15 +329,23 @@ bool capturing(hipStream_t s) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// A call that returns what the device has made of it has no place in a capture, where nothing runs: the host would go on with memory that
+// nobody has written, and each replay would write to it, or read it, after it is gone. The runtime refuses such a thread its waits.
+int may_wait(hipStream_t s, const char* who) {
+    if (!fhip::thread_captures() && fhip::runtime_allocates() && !(s && capturing(s))) return FHIP_OK;
+    return fhip::set_error(FHIP_ERR_HIP, "%s: waits for the device, which is not permitted while the stream is, or the thread has a stream, in a capture", who);
+}
+
 }  // namespace
 
 namespace fhip {
 
 // Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime (10 MB in 285 us;
 // chunks of it copied into slots by workers and pulled over the bus by kernels took 300 - 360), and it returns when the source has
-// been read or is known to be pinned. A copy in a stream capture stays a copy node.
+// been read or is known to be pinned. A copy in a stream capture stays a copy node; on another stream than the captured one it goes
+// through the runtime too, since a slot may have to be made.
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
-    if (n > IN_BYTES || capturing(s)) return check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+    if (n > IN_BYTES || capturing(s) || thread_captures()) return check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
     int rc;
     Ring* r = ring(&rc);
     if (!r) return rc;
@@ -350,9 +358,15 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     return rc;
 }
 
+int upload(void* d, const void* h, size_t n, hipStream_t s) {
+    if (int rc = may_wait(s, "fhip_upload")) return rc;
+    const int rc = copy_h2d(d, h, n, s);
+    return rc || n <= IN_BYTES ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+}
+
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
-    if (capturing(s)) return check_hip(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
     int rc, wgs = 0;
+    if ((rc = may_wait(s, "fhip_memcpy_d2h"))) return rc;
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;
@@ -387,6 +401,7 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
 // 5 of its 40 us, beside the bus, and lets the copy kernel confirm the chunk instead of an event that the workers had to query.)
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, size_t bytes, float* h_out) {
     int rc;
+    if ((rc = may_wait(nullptr, "fhip_deq_raw"))) return rc;
     Ring* r = ring(&rc);
     if (!r) return rc;
     {

@@ -96,11 +96,9 @@ H2D_STAGED = 640 << 10      # fhip_memcpy_h2d: a source of up to this many bytes
 
 
 def _upload(buf, a, stream=None):
-    """A contiguous host array into a DeviceBuffer, in stream order; the array may go away afterwards."""
-    lib, s = _lib.load(), _stream_handle(stream)
-    _lib.check(lib.fhip_memcpy_h2d(buf.ptr, a.ctypes.data, a.nbytes, s))
-    if a.nbytes > H2D_STAGED:
-        _lib.check(lib.fhip_stream_sync(s))
+    """A contiguous host array into a DeviceBuffer, in stream order; the array may go away afterwards (not inside a capture, whose
+    replays would read it again)."""
+    _lib.check(_lib.load().fhip_upload(buf.ptr, a.ctypes.data, a.nbytes, _stream_handle(stream)))
 
 
 class Tensor:

@@ -90,9 +90,14 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
  * thread captures a stream: what a captured call uses has to outlive the graph, so it is allocated before the capture begins. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
-/* async on stream; a source of up to 640 KiB has been read when the call returns (not in a stream capture) */
+/* async on stream; a source of up to 640 KiB has been read when the call returns, unless the thread captures a stream: on a captured
+ * stream the copy is recorded, and every replay reads the source */
 int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream);
-int fhip_memcpy_d2h(void* h_dst, const void* d_src, size_t nbytes, void* stream); /* synchronises stream before returning */
+/* The same with a source that has been read when the call returns, whatever its size (the copy itself is in stream order). FHIP_ERR_HIP while the
+ * stream, or any stream by the calling thread, is captured. */
+int fhip_upload(void* d_dst, const void* h_src, size_t nbytes, void* stream);
+/* synchronises stream before returning; FHIP_ERR_HIP while the stream, or any stream by the calling thread, is captured */
+int fhip_memcpy_d2h(void* h_dst, const void* d_src, size_t nbytes, void* stream);
 int fhip_memcpy_d2d(void* d_dst, const void* d_src, size_t nbytes, void* stream);
 /* `height` rows of `width` bytes between two pitched device arrays, async on stream (what Tensor::cat along the last
  * dim of a matrix comes to, crates/ferric-tensor/src/lib.rs:201-221: each side is copied into its columns of the result) */

@@ -132,3 +132,69 @@ def test_other_threads_allocate_and_copy_while_one_captures(F):
         g.launch()
         s.synchronize()
     assert word.to_vec(s).view(np.uint32)[0] == 6
+
+
+def _small_decoder(F, stream):
+    from ferric_amd import decode
+    from ferric_amd.synth import synth_weights
+    d, heads, kv, hd, ff = 512, 4, 2, 64, 1024
+    rng = np.random.default_rng(1)
+    w = lambda ty, rows, cols, seed: F.QMatrix.from_bytes(synth_weights(ty, rows, cols, seed), ty, rows, cols)
+    n = lambda k: F.Tensor.from_vec(rng.uniform(0.5, 1.5, k).astype(np.float32), (k,))
+    layer = decode.Qwen3Layer(n(d), w(F.Q4_K, (heads + 2 * kv) * hd, d, 1), w(F.Q8_0, d, heads * hd, 2), n(d), w(F.Q4_K, 2 * ff, d, 3), w(F.Q6_K, d, ff, 4), n(hd), n(hd))
+    return decode.Qwen3Decoder(decode.Qwen3Cfg(d, heads, kv, hd, ff), [layer], max_len=64, stream=stream)
+
+
+def test_host_copies_are_refused_inside_a_capture(F):
+    """Reading back, setting a decoder's input or position, dequantizing to the host: on the captured stream and on others. The capture goes on, and so
+    does what the refused calls would have set."""
+    s, elsewhere = F.Stream(), F.Stream()
+    dec = _small_decoder(F, s)
+    x = np.random.default_rng(2).standard_normal((3, 512)).astype(np.float32)
+    dec.set_pos(0)
+    dec.set_input(x[0])
+    dec.step()
+    want, before = dec.hidden(), [c.len for c in dec.caches]
+    t, big, raw = F.Tensor.from_vec(x, x.shape), np.zeros(1 << 20, np.float32), np.zeros(34 * 64, np.uint8)
+    room = F.Tensor.empty(big.shape)
+    assert F.deq_raw(raw, 32 * 64, F.Q8_0).size == 32 * 64
+    dec.set_pos(0)
+    g = F.Graph.begin(s)
+    dec._enqueue_step()
+    refused = [lambda: t.to_vec(s), lambda: t.to_vec(elsewhere), lambda: t.to_vec(), lambda: dec.hidden(), lambda: dec.set_pos(7), lambda: dec.set_input(x[1]),
+               lambda: F.qmatrix._upload(room.buf, big, s), lambda: F.qmatrix._upload(room.buf, big, elsewhere), lambda: F.deq_raw(raw, 32 * 64, F.Q8_0),
+               lambda: dec.prefill(x)]
+    for call in refused:
+        with pytest.raises(F._lib.FerricHipError, match="captur"):
+            call()
+    g.end()
+    assert [c.len for c in dec.caches] == [0] != before
+    for _ in range(3):
+        dec.set_pos(0)
+        dec.set_input(x[0])
+        g.launch()
+        assert np.array_equal(dec.hidden(), want)
+    assert np.array_equal(t.to_vec(), x.reshape(-1))
+
+
+def test_a_recorded_upload_reads_its_source_at_every_replay(F):
+    lib, check = F._lib.load(), F._lib.check
+    s, t, src = F.Stream(), F.Tensor.empty((1000,)), np.zeros(1000, np.float32)
+    g = F.Graph.begin(s)
+    check(lib.fhip_memcpy_h2d(t.buf.ptr, src.ctypes.data, src.nbytes, s.handle))
+    g.end()
+    for k in range(3):
+        src[:] = k + 1
+        g.launch()
+        assert (t.to_vec(s) == k + 1).all()
+
+
+def test_an_upload_has_read_its_source_whatever_its_size(F):
+    lib, check, s = F._lib.load(), F._lib.check, F.Stream()
+    for n in (1, 640 * KIB, 640 * KIB + 4, 40 * MIB):
+        want = np.random.default_rng(n).integers(0, 256, n, np.uint8)
+        d, src, got = F.DeviceBuffer(n), want.copy(), np.empty(n, np.uint8)
+        check(lib.fhip_upload(d.ptr, src.ctypes.data, n, s.handle))
+        src[:] = 0
+        check(lib.fhip_memcpy_d2h(got.ctypes.data, d.ptr, n, s.handle))
+        assert np.array_equal(got, want)
