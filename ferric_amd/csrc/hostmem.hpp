@@ -17,6 +17,10 @@ bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the bloc
 int stream_create(hipStream_t* s);      // a stream of the library's own ...
 int stream_destroy(hipStream_t s);     // ... and its end (any stream is taken)
 int device_wait();                     // until all work enqueued on the current device has ended; captures of other threads go on
+// n bytes from ptr on: inside one block in use of device dev; outside: they start in a block of fhip_malloc, but it is free, or they run past what was
+// asked for (and the slack); elsewhere: nothing of fhip_malloc's, or another device's
+enum class Place { inside, outside, elsewhere };
+Place pool_place(const void* ptr, size_t n, int dev);
 int device_malloc(void** out, size_t n, const char* what);           // hipMalloc; with no memory left, once more after pool_trim
 
 // transfer.hip: copies through pinned memory of the library's own; both directions and the host-to-host unpackers

@@ -338,4 +338,16 @@ bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end) {
     return true;
 }
 
+Place pool_place(const void* ptr, size_t n, int dev) {
+    Pool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mu);
+    auto it = p.blocks.upper_bound((uintptr_t)ptr);
+    if (it == p.blocks.begin()) return Place::elsewhere;
+    const Block& b = (--it)->second;
+    const size_t at = (uintptr_t)ptr - it->first, size = b.asked + WEIGHT_SLACK;
+    if (at >= b.cls) return Place::elsewhere;
+    if (!b.live || at > size || n > size - at) return Place::outside;
+    return b.dev == dev ? Place::inside : Place::elsewhere;
+}
+
 }  // namespace fhip

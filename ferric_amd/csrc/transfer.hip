@@ -329,6 +329,22 @@ bool capturing(hipStream_t s) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// Whether the copy kernels, which look nothing up, may take this copy (*yes): the device side inside one block of the library's on the current device,
+// the host side no device memory. Other memory is the runtime's, to copy or to refuse; what leaves one of the library's blocks is refused
+// here, since the runtime knows the block of the pool and not what was asked for. (0.15 us)
+int for_kernels(const void* d, size_t n, const void* h, const char* who, bool* yes) {
+    int dev = 0;
+    hipPointerAttribute_t a;
+    *yes = false;
+    if (const int rc = fhip::check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
+    const fhip::Place at = fhip::pool_place(d, n, dev);
+    if (at == fhip::Place::outside) return fhip::set_error(FHIP_ERR_HIP, "%s: %zu bytes at %p are not within one allocation", who, n, d);
+    if (at == fhip::Place::elsewhere) return FHIP_OK;
+    if (hipPointerGetAttributes(&a, h) == hipSuccess) *yes = a.type != hipMemoryTypeDevice && a.type != hipMemoryTypeArray;
+    else { (void)hipGetLastError(); *yes = true; }       // to some versions of the runtime, plain host memory is no pointer of its own
+    return FHIP_OK;
+}
+
 // A call that returns what the device has made of it has no place in a capture, where nothing runs: the host would go on with memory that
 // nobody has written, and each replay would write to it, or read it, after it is gone. The runtime refuses such a thread its waits.
 int may_wait(hipStream_t s, const char* who) {
@@ -345,8 +361,14 @@ namespace fhip {
 // been read or is known to be pinned. A copy in a stream capture stays a copy node; on another stream than the captured one it goes
 // through the runtime too, since a slot may have to be made.
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
-    if (n > IN_BYTES || capturing(s) || thread_captures()) return check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
     int rc;
+    bool kernels;
+    if ((rc = for_kernels(d, n, h, "fhip_memcpy_h2d", &kernels))) return rc;
+    const bool in_capture = capturing(s) || thread_captures();
+    if (n > IN_BYTES || in_capture || !kernels) {
+        rc = check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+        return rc || n > IN_BYTES || in_capture ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+    }
     Ring* r = ring(&rc);
     if (!r) return rc;
     Slot* q = r->need(&rc);
@@ -367,6 +389,12 @@ int upload(void* d, const void* h, size_t n, hipStream_t s) {
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     int rc, wgs = 0;
     if ((rc = may_wait(s, "fhip_memcpy_d2h"))) return rc;
+    bool kernels;
+    if ((rc = for_kernels(d, n, h, "fhip_memcpy_d2h", &kernels))) return rc;
+    if (!kernels) {
+        if ((rc = check_hip(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H"))) return rc;
+        return check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+    }
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;

@@ -90,7 +90,9 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
  * thread captures a stream: what a captured call uses has to outlive the graph, so it is allocated before the capture begins. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
-/* async on stream; a source of up to 640 KiB has been read when the call returns, unless the thread captures a stream: on a captured
+/* Host and device memory of any kind; a device range that starts in a block of fhip_malloc has to lie within what was asked for (and the 256 bytes
+ * behind it), FHIP_ERR_HIP otherwise.
+ * async on stream; a source of up to 640 KiB has been read when the call returns, unless the thread captures a stream: on a captured
  * stream the copy is recorded, and every replay reads the source */
 int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream);
 /* The same with a source that has been read when the call returns, whatever its size (the copy itself is in stream order). FHIP_ERR_HIP while the

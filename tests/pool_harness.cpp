@@ -80,6 +80,7 @@ size_t h_range(void* p) {            // bytes from p to the end of the block in 
     uintptr_t base = 0, end = 0;
     return fhip::pool_range(p, &base, &end) ? end - (uintptr_t)p : 0;
 }
+int h_place(void* p, size_t n, int dev) { return (int)fhip::pool_place(p, n, dev); }
 void* h_stream() { hipStream_t s = nullptr; (void)fhip::stream_create(&s); return s; }
 int h_stream_destroy(void* s) { return fhip::stream_destroy((hipStream_t)s); }
 void h_begin(void* s, int through_library) {

@@ -198,3 +198,29 @@ def test_an_upload_has_read_its_source_whatever_its_size(F):
         src[:] = 0
         check(lib.fhip_memcpy_d2h(got.ctypes.data, d.ptr, n, s.handle))
         assert np.array_equal(got, want)
+
+
+# ---- copies of what the library does not own -------------------------------------------------------------------------------------------
+
+def test_copies_outside_the_librarys_blocks_go_to_the_runtime(F):
+    """Device memory of somebody else's, device memory in the host's place, more bytes than a block has: copied by the runtime, which looks its
+    pointers up, or refused, and never reached by a kernel that does not look."""
+    lib, hip, s = F._lib.load(), C.CDLL("libamdhip64.so.7"), F.Stream()
+    rng = np.random.default_rng(5)
+    for n in (7, 100 * KIB, 640 * KIB, 3 * MIB):
+        a, got = rng.integers(0, 256, n, np.uint8), np.zeros(n, np.uint8)
+        foreign, own = C.c_void_p(), F.DeviceBuffer(n)
+        assert hip.hipMalloc(C.byref(foreign), C.c_size_t(n)) == 0
+        src = a.copy()
+        F._lib.check(lib.fhip_upload(foreign, src.ctypes.data, n, s.handle))
+        src[:] = 0
+        F._lib.check(lib.fhip_memcpy_d2h(got.ctypes.data, foreign, n, s.handle))
+        assert np.array_equal(got, a)
+        F._lib.check(lib.fhip_upload(own.ptr, foreign, n, s.handle))               # device memory as the source
+        got[:] = 0
+        F._lib.check(lib.fhip_memcpy_d2h(got.ctypes.data, own.ptr, n, s.handle))
+        assert np.array_equal(got, a)
+        for name, call in (("to", lambda d, m: lib.fhip_memcpy_h2d(d, (C.c_char * m)(), m, s.handle)), ("from", lambda d, m: lib.fhip_memcpy_d2h((C.c_char * m)(), d, m, s.handle))):
+            for at, m in ((0, n + 257), (n, 257), (0, n + 64 * MIB)):                 # past what was asked for, and its slack
+                assert call(C.c_void_p(own.ptr.value + at), m) == F._lib.ERR_HIP, (name, at, m)
+        assert hip.hipFree(foreign) == 0

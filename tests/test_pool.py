@@ -147,3 +147,16 @@ def test_a_capture_ends_with_its_thread_or_its_stream(pool):
         assert pool.c.h_end(a) == 0 and pool.malloc(100)[0] != 0
         pool.c.h_stream_destroy(b)
         pool.new(100)
+
+
+@pytest.mark.parametrize("n", [0, 1000, 900 * MIB])
+def test_a_copy_belongs_into_one_block_in_use(pool, n):
+    """As far as it was asked for (and the slack behind it), whatever the class holds beyond; on its own device; not after the free."""
+    p, place = pool.new(n), pool.c.h_place
+    place.argtypes = [C.c_void_p, C.c_size_t, C.c_int]
+    inside, outside, elsewhere = 0, 1, 2
+    assert [place(*a) for a in ((p, n + 256, 0), (p + 100, n + 156, 0), (p + n + 255, 1, 0))] == [inside] * 3
+    assert [place(*a) for a in ((p, n + 257, 0), (p + 100, n + 157, 0), (p + n + 255, 2, 0), (p, (1 << 64) - 1, 0), (p + 8, (1 << 64) - 8, 0))] == [outside] * 5
+    assert [place(*a) for a in ((p - 1, 2, 0), (p, 1, 1), (4096, 1, 0), (p + 2 * GIB, 1, 0))] == [elsewhere] * 4
+    pool.c.h_free(p)
+    assert place(p, 1, 0) == (outside if n < GIB // 2 else elsewhere)       # still the pool's, or the runtime's again
