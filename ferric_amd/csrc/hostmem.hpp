@@ -16,7 +16,6 @@ bool runtime_allocates();                                // the runtime permits 
 bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the block in use that ptr lies in, as far as it was asked for
 int stream_create(hipStream_t* s);      // a stream of the library's own ...
 int stream_destroy(hipStream_t s);     // ... and its end (any stream is taken)
-int device_wait();                     // until all work enqueued on the current device has ended; captures of other threads go on
 // n bytes from ptr on: inside one block in use of device dev; outside: they start in a block of fhip_malloc, but it is free, or they run past what was
 // asked for (and the slack); elsewhere: nothing of fhip_malloc's, or another device's
 enum class Place { inside, outside, elsewhere };

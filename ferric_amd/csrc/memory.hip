@@ -190,7 +190,7 @@ int stream_destroy(hipStream_t s) {
 // hipFree's own wait, and not hipDeviceSynchronize: that one fails while any thread of the process captures, and invalidates the capture.
 // On an idle device it takes 0.73 us, but where there is work it comes back some 50 us after the end of it (61 4.4 us mat-vecs: 104 - 108 us against
 // 52 - 54). So the null stream and the library's own are waited for first, which is as quick (56 - 59 us in all) and harms no capture.
-int device_wait() {
+static int device_wait() {
     int dev = 0;
     std::vector<std::shared_ptr<OwnStream>> held;
     if (const int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;

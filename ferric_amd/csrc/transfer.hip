@@ -115,6 +115,8 @@ struct Ring {                    // one per device
     Slot slot[SLOTS];
     uint32_t* words = nullptr;
     hipStream_t stream[2] = {nullptr, nullptr};   // of dequantizations
+    std::mutex spare_mu;
+    uint8_t* spare = nullptr;    // SLOT_BYTES of device memory for a dequantization without a slot
 
     // The lowest slot that neither the host holds nor the GPU still reads: low slots stay warm in the CPU's caches. A slot's
     // pinned memory is made when it is first taken. null: all are taken.
@@ -136,16 +138,15 @@ struct Ring {                    // one per device
         }
         return nullptr;
     }
-    // take() until there is one; the device is waited for when none comes free by itself
-    Slot* need(int* rc) {
-        for (int tries = 0; tries < 1 << 20; tries++) {
+    // take(), for some milliseconds where all are taken. null without an error: copies that wait for other streams' work hold them, and
+    // this one is better left to the runtime than made to wait for that work too
+    Slot* get(int* rc) {
+        const auto start = std::chrono::steady_clock::now();
+        for (;;) {
             if (Slot* q = take(rc)) return q;
-            if (*rc) return nullptr;
-            if (tries == 1 << 14 && (*rc = fhip::device_wait())) return nullptr;
+            if (*rc || std::chrono::steady_clock::now() - start > std::chrono::milliseconds(4)) return nullptr;
             std::this_thread::yield();
         }
-        *rc = fhip::set_error(FHIP_ERR_HIP, "transfer: no pinned slot came free");
-        return nullptr;
     }
     void release(Slot* q) {
         std::lock_guard<std::mutex> lock(mu);
@@ -179,25 +180,30 @@ struct Job {
 
     bool device_done(size_t c) const { return launched.load(std::memory_order_acquire) > c && slots[c % n_slots]->confirmed(want[c], words[c]); }
 };
+// A wait's pause: the core is given away, and after a millisecond slept away
+struct Pause {
+    const std::chrono::steady_clock::time_point start = std::chrono::steady_clock::now();
+    void operator()() const {
+        if (std::chrono::steady_clock::now() - start < std::chrono::milliseconds(1)) std::this_thread::yield();
+        else std::this_thread::sleep_for(std::chrono::microseconds(50));
+    }
+};
 size_t part(size_t bytes, size_t chunk, size_t c) { return bytes - c * chunk < chunk ? bytes - c * chunk : chunk; }
 
 // false: the job was aborted
 bool go_up(Job* j, size_t c) {
     if (c >= j->count || !j->up) return true;
-    while (c >= j->n_slots && !(j->down ? j->emptied[c - j->n_slots].load(std::memory_order_acquire) != 0 : j->device_done(c - j->n_slots))) {
+    auto free = [&] { return c < j->n_slots || (j->down ? j->emptied[c - j->n_slots].load(std::memory_order_acquire) != 0 : j->device_done(c - j->n_slots)); };
+    for (Pause pause; !free(); pause())
         if (j->abort.load()) return false;
-        std::this_thread::yield();
-    }
     memcpy(j->slots[c % j->n_slots]->host + j->up_at, j->up + c * j->up_chunk, part(j->up_bytes, j->up_chunk, c));
     j->filled[c].store(1, std::memory_order_release);
     return true;
 }
 bool go_down(Job* j, size_t c) {
     if (c >= j->count || !j->down) return true;
-    while (!j->device_done(c)) {
+    for (Pause pause; !j->device_done(c); pause())
         if (j->abort.load()) return false;
-        std::this_thread::yield();
-    }
     memcpy(j->down + c * j->down_chunk, j->slots[c % j->n_slots]->host, part(j->down_bytes, j->down_chunk, c));
     j->emptied[c].store(1, std::memory_order_release);
     j->left.fetch_add(1);
@@ -263,7 +269,9 @@ struct Workers {
 Workers& workers() { static Workers* w = new Workers(); return *w; }
 
 // launch(c, slot, stream, &words): enqueue what the device does with chunk c in slot->host, the last kernel confirming slot->seq + 1 in
-// the slot's words; streams are taken in turn. The caller sets the sides of `j` and its count.
+// the slot's words; streams are taken in turn, and have no other work to finish first: a job is every other chunked copy's turn too. The
+// caller sets the sides of `j` and its count. NO_SLOT: nothing was done.
+constexpr int NO_SLOT = 1;
 template <class Launch>
 int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Launch launch) {
     Workers& w = workers();
@@ -273,10 +281,11 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Launch l
     j.slots = slots;
     j.n_slots = 0;
     while (j.n_slots < JOB_SLOTS && j.n_slots < j.count) {
-        Slot* q = j.n_slots ? r->take(&rc) : r->need(&rc);
+        Slot* q = j.n_slots ? r->take(&rc) : r->get(&rc);
         if (!q) break;
         slots[j.n_slots++] = q;
     }
+    if (!rc && !j.n_slots) return NO_SLOT;
     if (!rc) {
         std::vector<std::atomic<uint8_t>> flags(2 * j.count);
         std::vector<uint32_t> want(j.count);
@@ -285,9 +294,9 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Launch l
         const bool helped = w.post(&j);
         auto wait_for = [&](auto ready) {       // also looks for a device error every few milliseconds: what waits here would wait for ever
             auto look = std::chrono::steady_clock::now();
-            for (unsigned i = 1; !ready() && !rc; i++) {
-                std::this_thread::yield();
-                if (i % 1024 || std::chrono::steady_clock::now() - look < std::chrono::milliseconds(5)) continue;
+            for (Pause pause; !ready() && !rc;) {
+                pause();
+                if (std::chrono::steady_clock::now() - look < std::chrono::milliseconds(5)) continue;
                 look = std::chrono::steady_clock::now();
                 for (size_t k = 0; k < n_streams && !rc; k++) {
                     const hipError_t e = hipStreamQuery(streams[k]);
@@ -365,14 +374,13 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     bool kernels;
     if ((rc = for_kernels(d, n, h, "fhip_memcpy_h2d", &kernels))) return rc;
     const bool in_capture = capturing(s) || thread_captures();
-    if (n > IN_BYTES || in_capture || !kernels) {
+    Ring* r = n > IN_BYTES || in_capture || !kernels ? nullptr : ring(&rc);
+    Slot* q = r ? r->get(&rc) : nullptr;
+    if (rc) return rc;
+    if (!q) {
         rc = check_hip(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
         return rc || n > IN_BYTES || in_capture ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
     }
-    Ring* r = ring(&rc);
-    if (!r) return rc;
-    Slot* q = r->need(&rc);
-    if (!q) return rc;
     memcpy(q->host, h, n);
     int wgs = 0;
     if (!(rc = launch_copy(q->host, d, n, MAX_WG, q->done, q->seq + 1, s, &wgs))) { q->seq++; q->wgs = wgs; }
@@ -386,15 +394,18 @@ int upload(void* d, const void* h, size_t n, hipStream_t s) {
     return rc || n <= IN_BYTES ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 
+// by the runtime: pointers that are not for kernels, or no slot
+static int copy_d2h_plain(void* h, const void* d, size_t n, hipStream_t s) {
+    const int rc = check_hip(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
+    return rc ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+}
+
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     int rc, wgs = 0;
     if ((rc = may_wait(s, "fhip_memcpy_d2h"))) return rc;
     bool kernels;
     if ((rc = for_kernels(d, n, h, "fhip_memcpy_d2h", &kernels))) return rc;
-    if (!kernels) {
-        if ((rc = check_hip(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H"))) return rc;
-        return check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-    }
+    if (!kernels) return copy_d2h_plain(h, d, n, s);
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;
@@ -402,13 +413,16 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
         Job j{};
         j.count = (n + CHUNK - 1) / CHUNK;
         j.down = (uint8_t*)h; j.down_bytes = n; j.down_chunk = CHUNK;
-        return run_chunks(r, j, &s, 1, [&](size_t c, Slot* q, hipStream_t st, int* w) {
+        // what the stream still has to do is waited for here, not by the workers and not in front of other copies
+        if ((rc = check_hip(hipStreamSynchronize(s), "hipStreamSynchronize"))) return rc;
+        rc = run_chunks(r, j, &s, 1, [&](size_t c, Slot* q, hipStream_t st, int* w) {
             return launch_copy(from + c * CHUNK, q->host, part(n, CHUNK, c), MAX_WG, q->done, q->seq + 1, st, w);
         });
+        return rc == NO_SLOT ? copy_d2h_plain(h, d, n, s) : rc;
     }
     // one part, or two thirds and the rest (where a second slot is free: nobody waits for one while holding one)
-    Slot* half[2] = {r->need(&rc), nullptr};
-    if (!half[0]) return rc;
+    Slot* half[2] = {r->get(&rc), nullptr};
+    if (!half[0]) return rc ? rc : copy_d2h_plain(h, d, n, s);
     if (n >= TWO_PARTS && !(half[1] = r->take(&rc)) && rc) { r->release(half[0]); return rc; }
     const size_t first = half[1] ? (n / 3 * 2 + 255) & ~(size_t)255 : n;
     int words[2] = {0, 0};
@@ -420,6 +434,21 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
         if (!(rc = await_words(half[i], half[i]->seq, words[i], s))) memcpy((uint8_t*)h + (i ? first : 0), half[i]->host, i ? n - first : first);
     for (Slot* q : half)
         if (q) r->release(q);
+    return rc;
+}
+
+// dequant_host with no slot to be had: a slot's worth of device memory kept for it, `per` blocks at a time, and the runtime's copies
+static int dequant_plain(Ring* r, uint32_t type, const uint8_t* h_raw, size_t nb, size_t per, size_t vals, size_t bytes, float* h_out) {
+    std::lock_guard<std::mutex> one(r->spare_mu);
+    hipStream_t s = r->stream[0];
+    int rc = FHIP_OK;
+    if (!r->spare && (rc = device_malloc((void**)&r->spare, SLOT_BYTES, "hipMalloc"))) { r->spare = nullptr; return rc; }
+    for (size_t b = 0; b < nb && !rc; b += per) {
+        const size_t n = nb - b < per ? nb - b : per;
+        if ((rc = check_hip(hipMemcpyAsync(r->spare + OUT_BYTES, h_raw + b * bytes, n * bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D"))) break;
+        if ((rc = launch_dequant(type, r->spare + OUT_BYTES, n, (float*)r->spare, s))) break;
+        rc = copy_d2h_plain(h_out + b * vals, r->spare, n * vals * sizeof(float), s);
+    }
     return rc;
 }
 
@@ -452,10 +481,11 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
         j.count = (nb + per - 1) / per;
         j.up = h_raw; j.up_bytes = nb * bytes; j.up_chunk = per * bytes; j.up_at = OUT_BYTES;
         j.down = (uint8_t*)h_out; j.down_bytes = n; j.down_chunk = out_chunk;
-        return run_chunks(r, j, r->stream, 2, launch);
+        rc = run_chunks(r, j, r->stream, 2, launch);
+        return rc == NO_SLOT ? dequant_plain(r, type, h_raw, nb, per, vals, bytes, h_out) : rc;
     }
-    Slot* q = r->need(&rc);
-    if (!q) return rc;
+    Slot* q = r->get(&rc);
+    if (!q) return rc ? rc : dequant_plain(r, type, h_raw, nb, per, vals, bytes, h_out);
     int wgs = 0;
     memcpy(q->host + OUT_BYTES, h_raw, nb * bytes);
     if (!(rc = launch(0, q, r->stream[0], &wgs))) {

@@ -1,6 +1,7 @@
 """Device memory and host copies of the library where they have to say no: stream captures, blocks freed twice, sizes and ranges that
 no allocation has; and what they do beside each other on several threads and streams."""
 import ctypes as C
+import time
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -224,3 +225,74 @@ def test_copies_outside_the_librarys_blocks_go_to_the_runtime(F):
             for at, m in ((0, n + 257), (n, 257), (0, n + 64 * MIB)):                 # past what was asked for, and its slack
                 assert call(C.c_void_p(own.ptr.value + at), m) == F._lib.ERR_HIP, (name, at, m)
         assert hip.hipFree(foreign) == 0
+
+
+# ---- copies beside each other ------------------------------------------------------------------------------------------------------------
+
+class Work:
+    """Something for a stream to do for about the given time, in launches of some milliseconds that leave room on every CU."""
+
+    def __init__(self, F):
+        self.lib, self.check, self.sink, self.iters = F._lib.load(), F._lib.check, F.DeviceBuffer(64), 20000
+        self.s = F.Stream()
+        self.launch(self.s)
+        self.s.synchronize()
+        start = time.perf_counter()
+        self.launch(self.s)
+        self.s.synchronize()
+        self.each = time.perf_counter() - start
+
+    def launch(self, s):
+        self.check(self.lib.fhip_debug_mfma_probe(self.iters, self.sink.ptr, None, s.handle))
+
+    def enqueue(self, s, seconds):
+        for _ in range(max(1, int(seconds / self.each))):
+            self.launch(s)
+
+
+@pytest.fixture(scope="module")
+def work(F):
+    return Work(F)
+
+
+def _read(F, t, s):
+    return F.Tensor.to_vec(t, s)
+
+
+def test_a_long_readback_behind_work_holds_nobody_up(F, work):
+    """2 MB behind half a second of work on one stream; 5 MB on an idle one and a dequantization in chunks come back meanwhile, and the wait costs one
+    core at most."""
+    busy, idle = F.Stream(), F.Stream()
+    a = np.random.default_rng(3).standard_normal(5 << 18).astype(np.float32)
+    t, raw = F.Tensor.from_vec(a, a.shape), np.zeros(34 << 16, np.uint8)
+    small = F.Tensor.from_vec(a[:1 << 19], (1 << 19,))
+    _read(F, t, idle), F.deq_raw(raw, 32 << 16, F.Q8_0)          # the slots and the workers are there
+    with ThreadPoolExecutor(1) as other:
+        work.enqueue(busy, 0.5)
+        wall, cpu = time.perf_counter(), time.process_time()
+        waiting = other.submit(_read, F, small, busy)
+        time.sleep(0.02)
+        assert np.array_equal(_read(F, t, idle), a) and not F.deq_raw(raw, 32 << 16, F.Q8_0).any()
+        assert not waiting.done()
+        assert np.array_equal(waiting.result(), a[:1 << 19])
+        wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall > 0.2 and cpu < 2 * wall, (wall, cpu)
+
+
+def test_many_readbacks_behind_work_leave_the_others_their_way(F, work):
+    """More of them than there are pinned slots, behind half a second of work; copies in both directions of other streams come back meanwhile."""
+    from ferric_amd.synth import synth_weights
+    busy, idle = F.Stream(), F.Stream()
+    a = np.random.default_rng(4).standard_normal(60000).astype(np.float32)
+    t, long = F.Tensor.from_vec(a, a.shape), F.Tensor.from_vec(np.tile(a, 20), (1200000,))
+    raw = synth_weights(F.Q8_0, 1, 32 << 16, 6)
+    dense = F.deq_raw(raw, 32 << 16, F.Q8_0)
+    with ThreadPoolExecutor(20) as other:
+        work.enqueue(busy, 0.5)
+        waiting = [other.submit(_read, F, t, busy) for _ in range(20)]
+        time.sleep(0.02)
+        assert np.array_equal(_read(F, t, idle), a) and np.array_equal(_read(F, long, idle)[-60000:], a)
+        F.qmatrix._upload(t.buf, a, idle)
+        assert np.array_equal(F.deq_raw(raw, 32 << 16, F.Q8_0), dense) and np.array_equal(F.deq_raw(raw[:3400], 3200, F.Q8_0), dense[:3200])
+        assert not any(w.done() for w in waiting)
+        assert all(np.array_equal(w.result(), a) for w in waiting)
