@@ -9,6 +9,7 @@
 #include <Python.h>
 #include <dlfcn.h>
 #include <stddef.h>
+#include <structmember.h>
 
 namespace {
 
@@ -26,6 +27,8 @@ struct Buffer {
     void* mem;
     PyObject* nbytes;                // as it was given
     PyObject* ptr;                   // c_void_p of mem, made when it is first asked for
+    PyObject* dict;                  // attributes a user hangs on the object, made when there are some
+    PyObject* weak;
 };
 
 // the exception for a return code of the library
@@ -69,8 +72,20 @@ int buffer_init(Buffer* self, PyObject* args, PyObject* kw) {
     return rc;
 }
 
+int buffer_traverse(Buffer* self, visitproc visit, void* arg) {
+    Py_VISIT(Py_TYPE(self));
+    Py_VISIT(self->dict);
+    return 0;
+}
+int buffer_clear(Buffer* self) {
+    Py_CLEAR(self->dict);
+    return 0;
+}
+
 void buffer_dealloc(Buffer* self) {
     PyTypeObject* type = Py_TYPE(self);
+    PyObject_GC_UnTrack(self);
+    if (self->weak) PyObject_ClearWeakRefs((PyObject*)self);
     if (self->mem) {
         void* mem = self->mem;
         self->mem = nullptr;
@@ -80,6 +95,7 @@ void buffer_dealloc(Buffer* self) {
     }
     Py_CLEAR(self->nbytes);
     Py_CLEAR(self->ptr);
+    Py_CLEAR(self->dict);
     type->tp_free((PyObject*)self);
     Py_DECREF(type);
 }
@@ -98,30 +114,46 @@ PyObject* buffer_nbytes(Buffer* self, void*) {
 PyGetSetDef buffer_getset[] = {
     {"ptr", (getter)buffer_ptr, nullptr, "device address (ctypes.c_void_p)", nullptr},
     {"nbytes", (getter)buffer_nbytes, nullptr, "bytes asked for", nullptr},
+    {"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr},
     {nullptr, nullptr, nullptr, nullptr, nullptr},
+};
+PyMemberDef buffer_members[] = {
+    {"__dictoffset__", T_PYSSIZET, offsetof(Buffer, dict), READONLY, nullptr},
+    {"__weaklistoffset__", T_PYSSIZET, offsetof(Buffer, weak), READONLY, nullptr},
+    {nullptr, 0, 0, 0, nullptr},
 };
 PyType_Slot buffer_slots[] = {
     {Py_tp_init, (void*)buffer_init},
     {Py_tp_new, (void*)PyType_GenericNew},
     {Py_tp_dealloc, (void*)buffer_dealloc},
+    {Py_tp_traverse, (void*)buffer_traverse},
+    {Py_tp_clear, (void*)buffer_clear},
     {Py_tp_getset, (void*)buffer_getset},
+    {Py_tp_members, (void*)buffer_members},
     {Py_tp_doc, (void*)"DeviceBuffer(nbytes)\n\nnbytes of device memory, freed with the object. Work enqueued on any stream may still use it "
                        "then: the library does not hand\nthe memory out again before the device has been idle once (fhip_free), so scratch can be "
                        "dropped without a synchronisation."},
     {0, nullptr},
 };
-PyType_Spec buffer_spec = {"ferric_amd._host.DeviceBuffer", sizeof(Buffer), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE, buffer_slots};
+PyType_Spec buffer_spec = {"ferric_amd._host.DeviceBuffer", sizeof(Buffer), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC, buffer_slots};
 
 // matmul_q(x buffer, weight handle, rows, output columns, stream) -> buffer of rows x columns f32: fhip_malloc and fhip_matmul_q.
-// The handle and the stream are ctypes pointers; the stream may be None.
+// The handle and the stream are ctypes pointers or addresses; the stream may be None. NotImplemented for a buffer of another type: the caller goes through
+// ctypes, which takes whatever `ptr` such an object has.
 PyObject* matmul_q(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 5 || !PyObject_TypeCheck(a[0], g_buffer_type)) { PyErr_SetString(PyExc_TypeError, "matmul_q(DeviceBuffer, handle, rows, columns, stream)"); return nullptr; }
+    if (n != 5) { PyErr_SetString(PyExc_TypeError, "matmul_q(DeviceBuffer, handle, rows, columns, stream)"); return nullptr; }
+    if (!PyObject_TypeCheck(a[0], g_buffer_type)) Py_RETURN_NOTIMPLEMENTED;
     const size_t rows = PyLong_AsSize_t(a[2]), cols = PyLong_AsSize_t(a[3]);
     if (PyErr_Occurred()) return nullptr;
     void* handle[2] = {nullptr, nullptr};
     for (int i = 0; i < 2; i++) {
         PyObject* h = a[i ? 4 : 1];
         if (h == Py_None) continue;
+        if (PyLong_Check(h)) {
+            handle[i] = PyLong_AsVoidPtr(h);
+            if (PyErr_Occurred()) return nullptr;
+            continue;
+        }
         PyObject* v = PyObject_GetAttr(h, g_value);
         if (!v) return nullptr;
         if (v != Py_None) handle[i] = PyLong_AsVoidPtr(v);

@@ -178,6 +178,9 @@ class Tensor:
         y = _new(Tensor)
         y.shape, y.dtype = (rows, w._rows), _F32
         y.buf = _lib.matmul_q(self.buf, w.handle, rows, w._rows, None if stream is None else stream.handle)
+        if y.buf is NotImplemented:      # a tensor over another object with a `ptr`
+            y.buf = DeviceBuffer(4 * rows * w._rows)
+            _lib.check(_lib.load().fhip_matmul_q(w.handle, self.buf.ptr, rows, y.buf.ptr, _stream_handle(stream)))
         return y
 
     def _matmul_typed(self, w, ty, stream):

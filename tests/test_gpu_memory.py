@@ -1,7 +1,9 @@
 """Device memory and host copies of the library where they have to say no: stream captures, blocks freed twice, sizes and ranges that
 no allocation has; and what they do beside each other on several threads and streams."""
 import ctypes as C
+import gc
 import time
+import weakref
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -296,3 +298,47 @@ def test_many_readbacks_behind_work_leave_the_others_their_way(F, work):
         assert np.array_equal(F.deq_raw(raw, 32 << 16, F.Q8_0), dense) and np.array_equal(F.deq_raw(raw[:3400], 3200, F.Q8_0), dense[:3200])
         assert not any(w.done() for w in waiting)
         assert all(np.array_equal(w.result(), a) for w in waiting)
+
+
+# ---- the Python object ---------------------------------------------------------------------------------------------------------------------
+
+def test_a_device_buffer_takes_attributes_and_weak_references(F):
+    b = F.DeviceBuffer(100)
+    b.owner, gone = "me", []
+    ref = weakref.ref(b, gone.append)
+    assert b.owner == "me" and vars(b) == {"owner": "me"} and ref() is b and b.nbytes == 100
+    del b.owner
+    with pytest.raises(AttributeError):
+        b.owner
+    assert weakref.WeakValueDictionary({1: b})[1] is b
+    del b
+    assert ref() is None and gone == [ref]
+
+    class Mine(F.DeviceBuffer):
+        pass
+    cycle = [F.DeviceBuffer(100), Mine(100)]
+    refs = [weakref.ref(c) for c in cycle]
+    cycle[0].other, cycle[1].other = cycle[1], cycle[0]
+    del cycle
+    gc.collect()
+    assert [r() for r in refs] == [None, None]
+
+
+def test_matmul_q_takes_any_buffer_and_stream_with_an_address(F):
+    """Objects that are not the library's own: a `ptr` and a `handle`, as ctypes pointers or as numbers, as the other operators take them."""
+    from ferric_amd.synth import synth_weights
+
+    class Address:
+        def __init__(self, **kw):
+            self.__dict__.update(kw)
+    w = F.QMatrix.from_bytes(synth_weights(F.Q4_K, 256, 512, 3), F.Q4_K, 256, 512)
+    x, s = F.Tensor.from_vec(np.random.default_rng(0).standard_normal((3, 512)).astype(np.float32), (3, 512)), F.Stream()
+    want = x.matmul_q(w).to_vec()
+    for ptr in (x.buf.ptr, x.buf.ptr.value):
+        for handle in (s.handle, s.handle.value):
+            other = F.Tensor(Address(ptr=ptr, nbytes=x.buf.nbytes), x.shape)
+            for t in (other, x):
+                assert np.array_equal(t.matmul_q(w, Address(handle=handle)).to_vec(s), want)
+        assert np.array_equal(other.matmul_q(w).to_vec(), want)
+    with pytest.raises(AttributeError):
+        F.Tensor(Address(), x.shape).matmul_q(w)
