@@ -40,9 +40,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // written too (lib.rs:2057-2074). TPR threads share a row (a fixed-shape tree sum, so results do not depend on scheduling).
 // Out = uint16_t: the normed rows as bf16, rounded as fhip_cvt_f32_bf16 rounds them -- what the matrix cores read, for a prompt: a
 // launch and a trip of the f32 rows through memory less per matmul.
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2)); }
+using fhip::pk_bf16;
 __device__ __forceinline__ void store_norm(float* out, size_t j, float4 v) { ((float4*)out)[j] = v; }
 __device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float4 v) { ((uint2*)out)[j] = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
 __device__ __forceinline__ void store_norm(float* out, size_t j, float v) { out[j] = v; }

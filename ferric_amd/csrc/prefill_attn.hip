@@ -41,9 +41,7 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Output rows as f32, or as bf16 (rounded as fhip_cvt_f32_bf16 rounds them) for a matmul on the matrix cores.
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2)); }
+using fhip::pk_bf16;
 __device__ __forceinline__ void store_out(float* p, float4 v) { *(float4*)p = v; }
 __device__ __forceinline__ void store_out(uint16_t* p, float4 v) { *(uint2*)p = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
 

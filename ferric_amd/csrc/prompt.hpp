@@ -4,6 +4,11 @@
 
 namespace fhip {
 
+// two floats rounded to bf16 (to nearest, ties to even): v_cvt_pk_bf16_f32, a in the low half
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2)); }
+
 // gemm_mfma.hip
 int launch_gemm_bf16_swiglu(const fhip_weight* w, const uint16_t* d_x, size_t t, uint16_t* d_h, hipStream_t s, float* d_ws, size_t ws_bytes);
 size_t gemm_bf16_swiglu_ws_bytes(const fhip_weight* w, size_t t);
