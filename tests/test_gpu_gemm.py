@@ -222,9 +222,11 @@ def test_batched_decode_ffn_on_the_matrix_cores(F, O):
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6, -1])
 def test_swiglu_inside_the_tiled_gemm(F, tile):
-    # ffn_coop over 32 rows applies SwiGLU in the gate|up launch (or in the launch that sums a cut tile): the same f32 sums, one f32
-    # expression and one rounding to bf16, so the block equals its steps bit for bit. Rows that end inside a tile, widths whose
-    # tiles are whole, cut and ragged (n_ff = 96: tiles of mostly nothing; 1312: no multiple of any tile's columns).
+    # ffn_coop over 32 rows applies SwiGLU in the gate|up launch (or in the launch that sums a cut tile): one f32 expression and one rounding to
+    # bf16 on sums that are the same f32 sums as those of its steps where both launches cut the same outputs along K. They do on these
+    # shapes, whose tiles are all whole or all cut, and the block equals its steps bit for bit; where a launch has whole tiles and cut ones the
+    # fused launch cuts other outputs (test_swiglu_beside_whole_and_cut_tiles). Rows that end inside a tile, widths whose tiles are
+    # ragged (n_ff = 96: tiles of mostly nothing; 1312: no multiple of any tile's columns).
     from ferric_amd.synth import synth_weights
     lib = F._lib.load()
     before = lib.fhip_debug_gemm_tile(tile)
@@ -238,6 +240,35 @@ def test_swiglu_inside_the_tiled_gemm(F, tile):
             assert np.array_equal(x.ffn_coop(gu, dn).to_vec().view(np.uint32), want.view(np.uint32)), (tile, tg, t, n_ff)
     finally:
         lib.fhip_debug_gemm_tile(before)
+
+
+# 272 tiles of 64 x 128, 312 of 64 x 256 and of 128 x 256, and the launcher's choice: 256 workgroups take a whole one each and the rest is cut along K
+@pytest.mark.parametrize("tile,t,d,n_ff", [(5, 40, 512, 17408), (0, 130, 512, 13312), (1, 270, 768, 13312), (-1, 520, 512, 17408)])
+def test_swiglu_beside_whole_and_cut_tiles(F, O, tile, t, d, n_ff):
+    # The fused launch deals columns of gate and up in turn to a tile and so cuts other outputs than a launch over the stacked rows does:
+    # their sums are added in another order, and a last bit in front of the rounding of h to bf16 may move. Against f64 the block is as exact as
+    # its steps. Bound of both: an operand's rounding to bf16 is at most 2^-9 of it; x and the weights of gate and up enter silu(g) u twice (its two
+    # factors), h and the weights of down once, so 6 * 2^-9 of the norm if every rounding were its largest and all of them added up.
+    from ferric_amd.synth import synth_weights
+    lib = F._lib.load()
+    before = lib.fhip_debug_gemm_tile(tile)
+    try:
+        raw = synth_weights(Q4_K, 2 * n_ff, d, 31), synth_weights(Q6_K, 256, n_ff, 32)
+        gu, dn = F.QMatrix.from_bytes(raw[0], Q4_K, 2 * n_ff, d), F.QMatrix.from_bytes(raw[1], Q6_K, 256, n_ff)
+        x = np.random.default_rng(33).standard_normal((t, d)).astype(np.float32)
+        x /= np.float32(np.linalg.norm(O.deq_raw(raw[0], 2 * n_ff * d, Q4_K).reshape(2 * n_ff, d), axis=1).mean())     # gate and up of order one
+        X = F.Tensor.from_vec(x, x.shape)
+        fused, again = (X.ffn_coop(gu, dn).to_vec().reshape(t, -1) for _ in range(2))
+        steps = X.matmul_q_coop(gu).swiglu(n_ff).matmul_q_coop(dn).to_vec().reshape(t, -1)
+    finally:
+        lib.fhip_debug_gemm_tile(before)
+    g = x.astype(np.float64) @ O.deq_raw(raw[0], 2 * n_ff * d, Q4_K).reshape(2 * n_ff, d).astype(np.float64).T
+    h = g[:, :n_ff] / (1 + np.exp(-g[:, :n_ff])) * g[:, n_ff:]
+    want = h @ O.deq_raw(raw[1], 256 * n_ff, Q6_K).reshape(256, n_ff).astype(np.float64).T
+    err = lambda y: np.linalg.norm(y - want) / np.linalg.norm(want)
+    assert np.array_equal(fused.view(np.uint32), again.view(np.uint32))
+    assert err(fused) < 6 * 2.0 ** -9 and err(fused) < 1.01 * err(steps), (err(fused), err(steps))
+    assert np.linalg.norm(fused - steps) < 2e-4 * np.linalg.norm(want), np.linalg.norm(fused - steps) / np.linalg.norm(want)
 
 
 def test_gemm_errors(F):
