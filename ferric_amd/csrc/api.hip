@@ -367,14 +367,15 @@ int fhip_stream_create(void** s) {
     int rc = need_init();
     if (rc) return rc;
     hipStream_t st;
-    rc = fhip::stream_create(&st);
+    rc = check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
     *s = rc ? nullptr : (void*)st;
     return rc;
 }
 int fhip_stream_destroy(void* s) {
     if (!s) return FHIP_OK;
     release_workspace((hipStream_t)s);   // the library's buffer for this stream goes with it
-    return fhip::stream_destroy((hipStream_t)s);
+    fhip::capture_ended((hipStream_t)s, true);
+    return check_hip(hipStreamDestroy((hipStream_t)s), "hipStreamDestroy");
 }
 int fhip_stream_sync(void* s) { return check_hip(hipStreamSynchronize((hipStream_t)s), "hipStreamSynchronize"); }
 int fhip_event_create(void** e) {
@@ -398,8 +399,11 @@ int fhip_graph_capture_begin(void* s) {
     int rc = need_init();
     if (rc) return rc;
     if (!s) return set_error(FHIP_ERR_ARG, "fhip_graph_capture_begin: needs a stream from fhip_stream_create");
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)s, &st) != hipSuccess) (void)hipGetLastError();
+    if (st != hipStreamCaptureStatusActive) fhip::capture_begun((hipStream_t)s);   // (begun twice: the runtime says so, and the first one stays)
     rc = check_hip(hipStreamBeginCapture((hipStream_t)s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    if (!rc) fhip::capture_begun((hipStream_t)s);
+    if (rc && st != hipStreamCaptureStatusActive) fhip::capture_ended((hipStream_t)s, false);
     return rc;
 }
 int fhip_graph_capture_end(void* s, void** graph_exec) {

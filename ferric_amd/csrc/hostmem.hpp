@@ -9,13 +9,11 @@ constexpr size_t WEIGHT_SLACK = 256;   // readable bytes every weight and every 
 int pool_malloc(void** out, size_t nbytes);
 int pool_free(void* ptr);
 void pool_trim();                      // gives every cached block back
-void capture_begun(hipStream_t s);                       // the calling thread has opened a capture of s ...
-void capture_ended(hipStream_t s, bool destroyed);       // ... and has ended it, or (any thread) the stream is gone; nothing if it is another thread's
+void capture_begun(hipStream_t s);                       // the calling thread is about to open a capture of s ...
+void capture_ended(hipStream_t s, bool destroyed);       // ... and has ended it or failed to, or (any thread) the stream goes; nothing if it is another thread's
 bool thread_captures();                                  // the calling thread has a capture open (of those)
 bool runtime_allocates();                                // the runtime permits the calling thread to allocate and to wait: it has no capture open at all
 bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the block in use that ptr lies in, as far as it was asked for
-int stream_create(hipStream_t* s);      // a stream of the library's own ...
-int stream_destroy(hipStream_t s);     // ... and its end (any stream is taken)
 // n bytes from ptr on: inside one block in use of device dev; outside: they start in a block of fhip_malloc, but it is free, or they run past what was
 // asked for (and the slack); elsewhere: nothing of fhip_malloc's, or another device's
 enum class Place { inside, outside, elsewhere };

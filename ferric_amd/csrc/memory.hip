@@ -15,7 +15,6 @@
 #include <atomic>
 #include <chrono>
 #include <map>
-#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -50,6 +49,13 @@ struct Pool {
 // never destroyed: objects of a host program may be freed after static destructors have begun to run
 Pool& pool() { static Pool* p = new Pool(); return *p; }
 
+// the calling thread's device; a process that sees one only is not asked every time (50 ns)
+hipError_t current_device(int* dev) {
+    static const bool one = [] { int n = 0; return hipGetDeviceCount(&n) == hipSuccess && n == 1; }();
+    *dev = 0;
+    return one ? hipSuccess : hipGetDevice(dev);
+}
+
 // The captures that fhip_graph_capture_begin opened and that have not ended, each with the thread it belongs to (the runtime lets no
 // other thread end it). A thread that captures may not wait for the device nor map or unmap memory: the runtime refuses and
 // invalidates the capture, and the stream then takes no work until it has been through another capture.
@@ -64,20 +70,6 @@ uint64_t this_thread() {
     thread_local const uint64_t id = ++last;
     return id;
 }
-
-// The streams of fhip_stream_create. Who waits for one holds it: a stream destroyed meanwhile goes with the last holder.
-struct OwnStream {
-    const hipStream_t s;
-    const int dev;
-    OwnStream(hipStream_t stream, int device) : s(stream), dev(device) {}
-    OwnStream(const OwnStream&) = delete;
-    ~OwnStream() { (void)hipStreamDestroy(s); }
-};
-struct OwnStreams {
-    std::mutex mu;
-    std::map<hipStream_t, std::shared_ptr<OwnStream>> all;
-};
-OwnStreams& own_streams() { static OwnStreams* o = new OwnStreams(); return *o; }
 
 // Eight classes per power of two: at most an eighth of a block is not asked for. n: up to POOL_BLOCK_MAX, which is a class of its own.
 size_t size_class(size_t n) {
@@ -131,6 +123,7 @@ void capture_begun(hipStream_t s) {
 
 void capture_ended(hipStream_t s, bool destroyed) {
     Captures& c = captures();
+    if (c.open.load() == 0) return;
     std::lock_guard<std::mutex> lock(c.mu);
     auto it = c.owner.find(s);
     if (it == c.owner.end() || (!destroyed && it->second != this_thread())) return;
@@ -166,54 +159,24 @@ void pool_trim() {
     for (void* q : out) (void)hipFree(q);   // hipFree waits for whatever still uses the block
 }
 
-int stream_create(hipStream_t* s) {
-    int dev = 0, rc;
-    if ((rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) || (rc = check_hip(hipStreamCreateWithFlags(s, hipStreamNonBlocking), "hipStreamCreate"))) return rc;
-    OwnStreams& o = own_streams();
-    std::lock_guard<std::mutex> lock(o.mu);
-    o.all[*s] = std::make_shared<OwnStream>(*s, dev);
-    return FHIP_OK;
-}
-
-int stream_destroy(hipStream_t s) {
-    std::shared_ptr<OwnStream> held;
-    OwnStreams& o = own_streams();
-    {
-        std::lock_guard<std::mutex> lock(o.mu);
-        auto it = o.all.find(s);
-        if (it != o.all.end()) { held = std::move(it->second); o.all.erase(it); }
-    }
-    capture_ended(s, true);
-    return held ? FHIP_OK : check_hip(hipStreamDestroy(s), "hipStreamDestroy");
-}
-
-// hipFree's own wait, and not hipDeviceSynchronize: that one fails while any thread of the process captures, and invalidates the capture.
-// On an idle device it takes 0.73 us, but where there is work it comes back some 50 us after the end of it (61 4.4 us mat-vecs: 104 - 108 us against
-// 52 - 54). So the null stream and the library's own are waited for first, which is as quick (56 - 59 us in all) and harms no capture. Under the older
-// runtime that torch brings along hipFree still takes 34 - 45 us then, until that runtime has retired the launches: 0.4 us a call, one wait
-// in 64, of a 5 us mat-vec that allocates its output.
+// Until all work enqueued on the device has ended. hipDeviceSynchronize fails while any thread of the process captures, and invalidates the
+// capture: it is called where the library knows of none, and none can begin under the lock. Beside a capture it is hipFree's own wait, which
+// the runtime permits, but which comes back only when the runtime has retired every launch (61 mat-vecs of 4.4 us: 52 us with the one, 104 - 110
+// with the other; taken everywhere it cost 5 - 10 % of calls of 6 - 22 us that allocate their output).
 static int device_wait() {
-    int dev = 0;
-    std::vector<std::shared_ptr<OwnStream>> held;
-    if (const int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
     {
-        OwnStreams& o = own_streams();
-        std::lock_guard<std::mutex> lock(o.mu);
-        for (auto& s : o.all)
-            if (s.second->dev == dev) held.push_back(s.second);
+        Captures& c = captures();
+        std::lock_guard<std::mutex> lock(c.mu);
+        if (c.owner.empty()) {
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipErrorStreamCaptureUnsupported) return check_hip(e, "hipDeviceSynchronize");
+            (void)hipGetLastError();                   // another thread captures through the runtime
+        }
     }
-    hipError_t quick = hipStreamSynchronize(nullptr);
-    for (auto& own : held) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (quick == hipSuccess && (quick = hipStreamIsCapturing(own->s, &st)) == hipSuccess && st == hipStreamCaptureStatusNone) quick = hipStreamSynchronize(own->s);
-    }
-    if (quick != hipSuccess) (void)hipGetLastError();    // hipFree says what is wrong
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, 256);
     if (e == hipSuccess) e = hipFree(p);
-    if (e != hipErrorOutOfMemory) return check_hip(e, "waiting for the device");
-    (void)hipGetLastError();
-    return check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    return check_hip(e, "waiting for the device");
 }
 
 // A cached block must not go where a new one could not: a thread that captures a stream through the runtime itself would have a graph go
@@ -243,7 +206,7 @@ int pool_malloc(void** out, size_t nbytes) {
     if (nbytes > SIZE_MAX - WEIGHT_SLACK) return check_hip(hipErrorOutOfMemory, "fhip_malloc");
     const size_t need = nbytes + WEIGHT_SLACK;
     int dev = 0;
-    int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
+    int rc = check_hip(current_device(&dev), "hipGetDevice");
     if (rc) return rc;
     Pool& p = pool();
     if (need > POOL_BLOCK_MAX || dev >= MAX_DEVICES) {

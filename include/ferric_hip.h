@@ -87,7 +87,9 @@ int fhip_block_bytes(uint32_t ggml_type, size_t* values, size_t* bytes);
 /* Freed blocks are kept (up to 2 GiB a device, none above 768 MiB; fhip_workspace_release gives them back, as does an allocation
  * that finds no memory) for later fhip_malloc calls. A block may be freed while work that uses it is still enqueued, on any stream:
  * it is not handed out again before the device has been idle once since the free. fhip_malloc fails (FHIP_ERR_HIP) while the calling
- * thread captures a stream: what a captured call uses has to outlive the graph, so it is allocated before the capture begins. */
+ * thread captures a stream: what a captured call uses has to outlive the graph, so it is allocated before the capture begins. It may wait for
+ * the device: beside a capture of fhip_graph_capture_begin on another thread in a way that leaves the capture alone, otherwise with
+ * hipDeviceSynchronize, at which the runtime invalidates captures that other threads began through the runtime itself. */
 int fhip_malloc(void** d_ptr, size_t nbytes);
 int fhip_free(void* d_ptr);
 /* Host and device memory of any kind; a device range that starts in a block of fhip_malloc has to lie within what was asked for (and the 256 bytes

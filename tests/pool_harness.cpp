@@ -57,19 +57,13 @@ hipError_t hipDeviceSynchronize() {
     rt.idle();
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t s) {
-    std::lock_guard<std::mutex> lock(rt.mu);
-    if (rt.refuse() || rt.capture.count(s)) return hipErrorStreamCaptureUnsupported;
-    return hipSuccess;
-}
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
     std::lock_guard<std::mutex> lock(rt.mu);
     auto it = rt.capture.find(s);
     *st = it == rt.capture.end() ? hipStreamCaptureStatusNone : it->second.second ? hipStreamCaptureStatusActive : hipStreamCaptureStatusInvalidated;
     return hipSuccess;
 }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { static uintptr_t n = 4096; *s = (hipStream_t)(n += 16); return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { std::lock_guard<std::mutex> lock(rt.mu); rt.capture.erase(s); return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 
@@ -81,11 +75,17 @@ size_t h_range(void* p) {            // bytes from p to the end of the block in 
     return fhip::pool_range(p, &base, &end) ? end - (uintptr_t)p : 0;
 }
 int h_place(void* p, size_t n, int dev) { return (int)fhip::pool_place(p, n, dev); }
-void* h_stream() { hipStream_t s = nullptr; (void)fhip::stream_create(&s); return s; }
-int h_stream_destroy(void* s) { return fhip::stream_destroy((hipStream_t)s); }
+void* h_stream() { static uintptr_t n = 4096; return (void*)(n += 16); }
+int h_stream_destroy(void* s) {
+    fhip::capture_ended((hipStream_t)s, true);
+    std::lock_guard<std::mutex> lock(rt.mu);
+    rt.capture.erase((hipStream_t)s);
+    return 0;
+}
 void h_begin(void* s, int through_library) {
-    { std::lock_guard<std::mutex> lock(rt.mu); rt.capture[(hipStream_t)s] = {std::this_thread::get_id(), true}; }
     if (through_library) fhip::capture_begun((hipStream_t)s);
+    std::lock_guard<std::mutex> lock(rt.mu);
+    rt.capture[(hipStream_t)s] = {std::this_thread::get_id(), true};
 }
 int h_end(void* s) {                 // 0: a valid graph, 1: an invalidated one, 2: another thread's capture, or none
     std::unique_lock<std::mutex> lock(rt.mu);

@@ -11,6 +11,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 KIB, MIB = 1 << 10, 1 << 20
+KEPT = 64                 # freed blocks that a small class collects before an allocation waits for the device
 
 
 def blocks_in_turn(F, nbytes, times=200):
@@ -41,8 +42,8 @@ def test_a_capture_is_its_own_threads_whoever_tries_to_end_it(F):
     for _ in range(3):
         g.launch()
     assert word.to_vec(s).view(np.uint32)[0] == 6
-    assert other.submit(blocks_in_turn, F, 9000).result() <= 64
-    assert blocks_in_turn(F, 9000) <= 64
+    assert other.submit(blocks_in_turn, F, 9000).result() <= KEPT
+    assert blocks_in_turn(F, 9000) <= KEPT
 
 
 def test_a_stream_destroyed_while_it_captures_ends_the_capture(F):
@@ -50,7 +51,7 @@ def test_a_stream_destroyed_while_it_captures_ends_the_capture(F):
     F.Graph.begin(s)
     handle, s.handle = s.handle, None
     F._lib.check(F._lib.load().fhip_stream_destroy(handle))
-    assert blocks_in_turn(F, 11000) <= 64
+    assert blocks_in_turn(F, 11000) <= KEPT
 
 
 def _allocating_calls(F):
@@ -126,7 +127,7 @@ def test_other_threads_allocate_and_copy_while_one_captures(F):
     g = F.Graph.begin(s)
     check(lib.fhip_u32_add(word.buf.ptr, 1, 1, s.handle))
     with ThreadPoolExecutor(1) as other:
-        assert other.submit(blocks_in_turn, F, 17000).result() <= 64
+        assert other.submit(blocks_in_turn, F, 17000).result() <= KEPT
         a = np.arange(3 * MIB, dtype=np.float32)
         assert np.array_equal(other.submit(lambda: F.Tensor.from_vec(a, a.shape).to_vec()).result(), a)
     check(lib.fhip_u32_add(word.buf.ptr, 1, 1, s.handle))
