@@ -270,18 +270,18 @@ Workers& workers() { static Workers* w = new Workers(); return *w; }
 
 // launch(c, slot, stream, &words): enqueue what the device does with chunk c in slot->host, the last kernel confirming slot->seq + 1 in
 // the slot's words; streams are taken in turn, and have no other work to finish first: a job is every other chunked copy's turn too. The
-// caller sets the sides of `j` and its count. begun: null, or the slot chunk 0 has crossed into (it is released with the others). NO_SLOT:
-// nothing was done.
-constexpr int NO_SLOT = 1;
+// caller sets the sides of `j` and its count. begun: the slots of the first n_begun chunks, which have been launched (they are released with the
+// others). NO_SLOT: nothing was done.
+constexpr int NO_SLOT = 1, BEGUN = 3;
 template <class Launch>
-int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* begun, Launch launch) {
+int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* const* begun, size_t n_begun, Launch launch) {
     Workers& w = workers();
     std::lock_guard<std::mutex> one(w.one);
     int rc = FHIP_OK;
     Slot* slots[JOB_SLOTS];
     j.slots = slots;
     j.n_slots = 0;
-    if (begun) slots[j.n_slots++] = begun;
+    while (j.n_slots < n_begun) { slots[j.n_slots] = begun[j.n_slots]; j.n_slots++; }
     while (j.n_slots < JOB_SLOTS && j.n_slots < j.count) {
         Slot* q = j.n_slots ? r->take(&rc) : r->get(&rc);
         if (!q) break;
@@ -293,9 +293,11 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* be
         std::vector<uint32_t> want(j.count);
         std::vector<int> words(j.count);
         j.filled = flags.data(); j.emptied = flags.data() + j.count; j.want = want.data(); j.words = words.data();
-        if (begun) { want[0] = begun->seq; words[0] = begun->wgs; j.launched.store(1); }
+        for (size_t c = 0; c < n_begun; c++) { want[c] = begun[c]->seq; words[c] = begun[c]->wgs; }
+        j.launched.store(n_begun);
         const bool helped = w.post(&j);
-        if (begun && !helped) (void)go_down(&j, 0);
+        for (size_t c = 0; c < n_begun && !helped && !rc; c++)
+            if (!(rc = await_words(begun[c], want[c], words[c], streams[0]))) (void)go_down(&j, c);
         auto wait_for = [&](auto ready) {       // also looks for a device error every few milliseconds: what waits here would wait for ever
             auto look = std::chrono::steady_clock::now();
             for (Pause pause; !ready() && !rc;) {
@@ -309,7 +311,7 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* be
                 }
             }
         };
-        for (size_t c = begun ? 1 : 0; c < j.count && !rc; c++) {
+        for (size_t c = n_begun; c < j.count && !rc; c++) {
             Slot* q = slots[c % j.n_slots];
             hipStream_t s = streams[c % n_streams];
             if (!helped) {                       // without threads the chunks go one by one
@@ -417,15 +419,25 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
         Job j{};
         j.count = (n + CHUNK - 1) / CHUNK;
         j.down = (uint8_t*)h; j.down_bytes = n; j.down_chunk = CHUNK;
-        // what the stream still has to do is waited for here, with the first chunk, and not by the workers and in front of other copies
-        // (hipStreamSynchronize in its place: 8 us more of a 1.6 MB copy from an idle stream's 86)
-        Slot* q = r->get(&rc);
-        if (!q) return rc ? rc : copy_d2h_plain(h, d, n, s);
-        if (!(rc = launch_copy(from, q->host, CHUNK, MAX_WG, q->done, q->seq + 1, s, &wgs))) { q->seq++; q->wgs = wgs; rc = await_words(q, q->seq, wgs, s); }
-        if (rc) { r->release(q); return rc; }
-        return run_chunks(r, j, &s, 1, q, [&](size_t c, Slot* to, hipStream_t st, int* w) {
+        auto launch = [&](size_t c, Slot* to, hipStream_t st, int* w) {
             return launch_copy(from + c * CHUNK, to->host, part(n, CHUNK, c), MAX_WG, to->done, to->seq + 1, st, w);
-        });
+        };
+        // what the stream still has to do is waited for here, with the first chunk, and not by the workers and in front of other copies (hipStreamSynchronize in
+        // its place: 8 us more of a 1.6 MB copy from an idle stream's 86); two more are on their way meanwhile, or the bus would wait too
+        Slot* begun[BEGUN];
+        size_t n_begun = 0;
+        while (n_begun < BEGUN && n_begun < j.count && !rc) {
+            Slot* q = n_begun ? r->take(&rc) : r->get(&rc);
+            if (!q) break;
+            begun[n_begun] = q;
+            if (!(rc = launch(n_begun++, q, s, &wgs))) { q->seq++; q->wgs = wgs; }
+        }
+        if (!rc && !n_begun) return copy_d2h_plain(h, d, n, s);
+        if (!rc) rc = await_words(begun[0], begun[0]->seq, begun[0]->wgs, s);
+        if (!rc) return run_chunks(r, j, &s, 1, begun, n_begun, launch);
+        (void)hipStreamSynchronize(s);              // an enqueued chunk may still use a slot
+        for (size_t i = 0; i < n_begun; i++) r->release(begun[i]);
+        return rc;
     }
     // one part, or two thirds and the rest (where a second slot is free: nobody waits for one while holding one)
     Slot* half[2] = {r->get(&rc), nullptr};
@@ -488,7 +500,7 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
         j.count = (nb + per - 1) / per;
         j.up = h_raw; j.up_bytes = nb * bytes; j.up_chunk = per * bytes; j.up_at = OUT_BYTES;
         j.down = (uint8_t*)h_out; j.down_bytes = n; j.down_chunk = out_chunk;
-        rc = run_chunks(r, j, r->stream, 2, nullptr, launch);
+        rc = run_chunks(r, j, r->stream, 2, nullptr, 0, launch);
         return rc == NO_SLOT ? dequant_plain(r, type, h_raw, nb, per, vals, bytes, h_out) : rc;
     }
     Slot* q = r->get(&rc);
