@@ -38,23 +38,29 @@ int raise_rc(int rc) {
     return -1;
 }
 
+int ready() {
+    if (p_malloc) return 0;
+    if (!g_first_use) { PyErr_SetString(PyExc_RuntimeError, "ferric_amd._host: setup() has not been called"); return -1; }
+    PyObject* r = PyObject_CallNoArgs(g_first_use);
+    if (!r) return -1;
+    Py_DECREF(r);
+    if (!p_malloc) { PyErr_SetString(PyExc_RuntimeError, "ferric_amd._host: bind() has not been called"); return -1; }
+    return 0;
+}
+void buffer_holds(Buffer* self, void* mem, PyObject* n) {
+    self->mem = mem;
+    Py_INCREF(n);
+    Py_XSETREF(self->nbytes, n);
+}
 int buffer_allocate(Buffer* self, size_t bytes, PyObject* n) {
-    if (!p_malloc) {
-        if (!g_first_use) { PyErr_SetString(PyExc_RuntimeError, "ferric_amd._host: setup() has not been called"); return -1; }
-        PyObject* r = PyObject_CallNoArgs(g_first_use);
-        if (!r) return -1;
-        Py_DECREF(r);
-        if (!p_malloc) { PyErr_SetString(PyExc_RuntimeError, "ferric_amd._host: bind() has not been called"); return -1; }
-    }
+    if (ready()) return -1;
     int rc;
     void* mem = nullptr;
     Py_BEGIN_ALLOW_THREADS           // may wait for the device
     rc = p_malloc(&mem, bytes);
     Py_END_ALLOW_THREADS
     if (rc) return raise_rc(rc);
-    self->mem = mem;
-    Py_INCREF(n);
-    Py_XSETREF(self->nbytes, n);
+    buffer_holds(self, mem, n);
     return 0;
 }
 
@@ -162,15 +168,16 @@ PyObject* matmul_q(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     PyObject* nbytes = PyLong_FromSize_t(rows * cols * sizeof(float));
     if (!nbytes) return nullptr;
-    Buffer* out = (Buffer*)g_buffer_type->tp_alloc(g_buffer_type, 0);
-    const int bad = out ? buffer_allocate(out, rows * cols * sizeof(float), nbytes) : -1;
-    Py_DECREF(nbytes);
-    if (bad) { Py_XDECREF(out); return nullptr; }
-    void *x = ((Buffer*)a[0])->mem, *y = out->mem;
+    Buffer* out = ready() ? nullptr : (Buffer*)g_buffer_type->tp_alloc(g_buffer_type, 0);
+    if (!out) { Py_DECREF(nbytes); return nullptr; }
+    void *x = ((Buffer*)a[0])->mem, *y = nullptr;
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = p_matmul_q(handle[0], x, rows, y, handle[1]);
+    Py_BEGIN_ALLOW_THREADS           // once for both: giving the interpreter away and taking it back is 0.1 us
+    rc = p_malloc(&y, rows * cols * sizeof(float));
+    if (!rc) rc = p_matmul_q(handle[0], x, rows, y, handle[1]);
     Py_END_ALLOW_THREADS
+    if (y) buffer_holds(out, y, nbytes);
+    Py_DECREF(nbytes);
     if (rc) { raise_rc(rc); Py_DECREF(out); return nullptr; }
     return (PyObject*)out;
 }
