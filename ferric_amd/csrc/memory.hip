@@ -2,7 +2,7 @@
 //
 // hipFree waits for the device, and a block of more than a few megabytes is mapped and unmapped on every call. An operator that
 // allocates its output (and perhaps scratch) per call therefore paid a full drain of the queue per call, and the large ones the
-// page tables of hundreds of megabytes: a 2048-row feed-forward block of 1.1 ms of kernels took 10.6 ms, a 5 us mat-vec 20 us.
+// page tables of hundreds of megabytes: a 2048-row feed-forward block of 1.1 ms of kernels took 4.8 to 10.6 ms, a 5 us mat-vec 20 us.
 //
 // What hipFree's wait gave callers is kept: a freed block may still be in use by work enqueued on any stream, this library's or
 // another's, so it is not handed out again before the device has been idle once since the free. Freed blocks collect on a `dirty`
@@ -163,20 +163,19 @@ void pool_trim() {
 // capture: it is called where the library knows of none, and none can begin under the lock. Beside a capture it is hipFree's own wait, which
 // the runtime permits, but which comes back only when the runtime has retired every launch (61 mat-vecs of 4.4 us: 52 us with the one, 104 - 110
 // with the other; taken everywhere it cost 5 - 10 % of calls of 6 - 22 us that allocate their output).
-static int device_wait() {
+static hipError_t device_wait() {
     {
         Captures& c = captures();
         std::lock_guard<std::mutex> lock(c.mu);
         if (c.owner.empty()) {
             const hipError_t e = hipDeviceSynchronize();
-            if (e != hipErrorStreamCaptureUnsupported) return check_hip(e, "hipDeviceSynchronize");
+            if (e != hipErrorStreamCaptureUnsupported) return e;
             (void)hipGetLastError();                   // another thread captures through the runtime
         }
     }
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, 256);
-    if (e == hipSuccess) e = hipFree(p);
-    return check_hip(e, "waiting for the device");
+    const hipError_t e = hipMalloc(&p, 256);
+    return e == hipSuccess ? hipFree(p) : e;
 }
 
 // A cached block must not go where a new one could not: a thread that captures a stream through the runtime itself would have a graph go
@@ -243,14 +242,15 @@ int pool_malloc(void** out, size_t nbytes) {
                     dirty.back().second.swap(k.second.dirty);
                 }
         }
-        rc = device_wait();
+        const hipError_t e = device_wait();
         std::lock_guard<std::mutex> lock(p.mu);
         for (auto& d : dirty) {
             SizeClass& c = p.classes[dev][d.first];
-            auto& to = rc ? c.dirty : c.clean;
+            auto& to = e != hipSuccess ? c.dirty : c.clean;
             to.insert(to.end(), d.second.begin(), d.second.end());
         }
-        if (rc) return rc;
+        if (e == hipErrorOutOfMemory) { (void)hipGetLastError(); break; }   // device_malloc gives back what is cached
+        if (e != hipSuccess) return check_hip(e, "waiting for the device");
         waited = true;
     }
     if ((rc = device_malloc(out, cls, "hipMalloc"))) return rc;

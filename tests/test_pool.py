@@ -77,6 +77,19 @@ def test_a_block_is_handed_out_again_only_after_the_device_was_idle(pool):
         assert pool.c.h_waits() > 0
 
 
+def test_cached_memory_is_found_beside_a_capture(pool):
+    """With nothing left to allocate (8 GiB: eleven blocks of 704 MiB and one of 448), not even what the wait needs."""
+    s = pool.c.h_stream()
+    blocks = [pool.new(704 * MIB - 256) for _ in range(11)] + [pool.new(448 * MIB - 256)]
+    assert pool.c.h_bytes() == 8 * GIB
+    with ThreadPoolExecutor(1) as other:
+        pool.c.h_begin(s, 1)
+        for p in blocks[:2]:
+            pool.c.h_free(p)
+        assert other.submit(pool.malloc, 704 * MIB - 256).result()[0] == 0
+        assert pool.c.h_end(s) == 0
+
+
 def test_cached_memory_is_bounded_and_given_back(pool):
     blocks = [pool.new(100 * MIB + k) for k in range(40)]
     for p in blocks:
