@@ -53,7 +53,7 @@ impl DeviceF32 {
     pub fn from_slice(v: &[f32]) -> Result<Self, String> {
         let mut p: *mut c_void = ptr::null_mut();
         check(unsafe { ffi::fhip_malloc(&mut p, v.len().max(1) * 4) })?;
-        check(unsafe { ffi::fhip_memcpy_h2d(p, v.as_ptr() as *const c_void, v.len() * 4, ptr::null_mut()) })?;
+        check(unsafe { ffi::fhip_upload(p, v.as_ptr() as *const c_void, v.len() * 4, ptr::null_mut()) })?; // the slice is only borrowed
         Ok(Self { ptr: p as *mut f32, len: v.len() })
     }
     pub fn to_vec(&self) -> Result<Vec<f32>, String> {
