@@ -63,6 +63,7 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
     *st = it == rt.capture.end() ? hipStreamCaptureStatusNone : it->second.second ? hipStreamCaptureStatusActive : hipStreamCaptureStatusInvalidated;
     return hipSuccess;
 }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) { static thread_local hipStreamCaptureMode now = hipStreamCaptureModeGlobal; std::swap(*m, now); return hipSuccess; }
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }

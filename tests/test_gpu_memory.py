@@ -120,6 +120,20 @@ def test_nothing_is_allocated_inside_a_capture_through_the_runtime(F):
     F.DeviceBuffer(15000)
 
 
+def test_cached_memory_and_copies_leave_a_global_capture_of_another_thread_alone(F):
+    """The runtime invalidates such a capture when any thread calls hipMalloc; a block that the pool holds already needs no such call."""
+    hip, s, graph = C.CDLL("libamdhip64.so.7"), F.Stream(), C.c_void_p()
+    t = F.Tensor.from_vec(np.arange(5000, dtype=np.float32), (5000,))
+    t.to_vec()
+    blocks_in_turn(F, 19000)                     # the last wait was a few blocks ago: some are clean
+    with ThreadPoolExecutor(1) as other:
+        assert other.submit(hip.hipStreamBeginCapture, s.handle, 0).result() == 0
+        F.DeviceBuffer(19000)
+        assert np.array_equal(t.to_vec(), np.arange(5000, dtype=np.float32))
+        assert other.submit(hip.hipStreamEndCapture, s.handle, C.byref(graph)).result() == 0
+    hip.hipGraphDestroy(graph)
+
+
 def test_other_threads_allocate_and_copy_while_one_captures(F):
     """Their waits for the device must leave the capture alone (hipDeviceSynchronize would fail and invalidate it)."""
     lib, check = F._lib.load(), F._lib.check
