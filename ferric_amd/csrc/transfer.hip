@@ -347,19 +347,24 @@ bool capturing(hipStream_t s) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// no device memory: the host may touch it (0.1 us)
+bool plain_host(const void* h) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, h) == hipSuccess) return a.type != hipMemoryTypeDevice && a.type != hipMemoryTypeArray;
+    (void)hipGetLastError();                             // to some versions of the runtime, plain host memory is no pointer of its own
+    return true;
+}
+
 // Whether the copy kernels, which look nothing up, may take this copy (*yes): the device side inside one block of the library's on the current device,
 // the host side no device memory. Other memory is the runtime's, to copy or to refuse; what leaves one of the library's blocks is refused
 // here, since the runtime knows the block of the pool and not what was asked for. (0.15 us)
 int for_kernels(const void* d, size_t n, const void* h, const char* who, bool* yes) {
     int dev = 0;
-    hipPointerAttribute_t a;
     *yes = false;
     if (const int rc = fhip::check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
     const fhip::Place at = fhip::pool_place(d, n, dev);
     if (at == fhip::Place::outside) return fhip::set_error(FHIP_ERR_HIP, "%s: %zu bytes at %p are not within one allocation", who, n, d);
-    if (at == fhip::Place::elsewhere) return FHIP_OK;
-    if (hipPointerGetAttributes(&a, h) == hipSuccess) *yes = a.type != hipMemoryTypeDevice && a.type != hipMemoryTypeArray;
-    else { (void)hipGetLastError(); *yes = true; }       // to some versions of the runtime, plain host memory is no pointer of its own
+    *yes = at == fhip::Place::inside && plain_host(h);
     return FHIP_OK;
 }
 
@@ -459,7 +464,7 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     return rc;
 }
 
-// dequant_host with no slot to be had: a slot's worth of device memory kept for it, `per` blocks at a time, and the runtime's copies
+// dequant_host with no slot to be had, or with device memory for a host side: a slot's worth of device memory kept for it, `per` blocks at a time, and the runtime's copies
 static int dequant_plain(Ring* r, uint32_t type, const uint8_t* h_raw, size_t nb, size_t per, size_t vals, size_t bytes, float* h_out) {
     std::lock_guard<std::mutex> one(r->spare_mu);
     hipStream_t s = r->stream[0];
@@ -490,6 +495,7 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
     }
     const size_t per = CHUNK / sizeof(float) / vals, out_chunk = per * vals * sizeof(float);   // blocks of a chunk, and their floats
     const size_t n = nb * vals * sizeof(float);
+    if (!plain_host(h_raw) || !plain_host(h_out)) return dequant_plain(r, type, h_raw, nb, per, vals, bytes, h_out);
     auto launch = [&](size_t c, Slot* q, hipStream_t s, int* wgs) {
         const size_t blocks = nb - c * per < per ? nb - c * per : per;
         int err;

@@ -244,6 +244,18 @@ def test_copies_outside_the_librarys_blocks_go_to_the_runtime(F):
         assert hip.hipFree(foreign) == 0
 
 
+@pytest.mark.parametrize("values", [32 * 40, 5 << 18])
+def test_host_dequantization_takes_device_memory_on_either_side(F, values):
+    from ferric_amd.synth import synth_weights
+    lib, raw = F._lib.load(), synth_weights(F.Q8_0, 1, values, 8)
+    want, t, got = F.deq_raw(raw, values, F.Q8_0), F.Tensor.empty((values,)), C.c_size_t()
+    d = F.DeviceBuffer(raw.size)
+    F._lib.check(lib.fhip_upload(d.ptr, raw.ctypes.data, raw.size, None))
+    F._lib.check(lib.fhip_stream_sync(None))
+    F._lib.check(lib.fhip_deq_raw(d.ptr, raw.size, values, F.Q8_0, t.buf.ptr, C.byref(got)))
+    assert got.value == values and np.array_equal(t.to_vec(), want)
+
+
 # ---- copies beside each other ------------------------------------------------------------------------------------------------------------
 
 class Work:
