@@ -103,12 +103,38 @@ int device_cus() { return g_cus; }
 size_t device_lds_bytes() { return g_lds; }
 
 // The streaming mat-vec exists in two copies, one per activation precision; these forward to the one the weight names.
-// From three rows on, Q4_K, Q5_K and Q6_K batches go four rows at a time through the kernel that multiplies on the 4 x 4 x 4 int8
+// From three rows on, Q4_K, Q5_K, Q6_K and Q8_0 batches go four rows at a time through the kernel that multiplies on the 4 x 4 x 4 int8
 // matrix instruction (gemv_quad.hip: the same arithmetic and the same bits per row, one pass over the weight for four rows);
-// what is left of a batch, one or two rows, and every other format take the dot-product kernel.
+// what is left of a batch, one or two rows, takes the dot-product kernel.
+// Batches of the 32-value formats from here on go up to sixteen rows at a time through the kernel that multiplies on the 16 x 16 x 32
+// int8 matrix instruction (gemv_wide.hip: the same bits per row). Its cost is the quantiser's, per activation row and workgroup,
+// plus the weight once; the dot-product kernel's is a launch and the weight per four rows. us, cold, dot-product | wide, three rows:
+// IQ4_NL 1024 x 5120 7.8 | 10.1, 4096 x 4096 9.6 | 10.1, 9728 x 2560 11.7 | 10.8, 34816 x 5120 43 | 30.5; four: Q4_0 1024 x 5120 9.4 | 10.3,
+// 1946 x 1504 6.8 | 7.7, 4096 x 4096 12.8 | 9.8, 34816 x 5120 43 | 29.7; five: 1024 x 1024 9.7 | 8.0, 1024 x 5120 13.8 | 11.8, 34816 x 5120
+// 60 | 38; sixteen: 1467 x 1760 38.8 | 15.8, 4096 x 4096 50 | 23, 34816 x 5120 171 | 61. Q8_0 has the four-row kernel (gemv_quad.hip) at three
+// and four rows of up to 5120 columns (4096 x 4096 9.5 | 11.5).
+bool takes_wide(const fhip_weight* w, size_t t) {
+    const size_t weights = w->rows * w->cols;
+    if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
+    if (t < 3 || (t == 3 && weights < ((size_t)24 << 20)) || (t == 4 && weights < ((size_t)8 << 20))) return false;
+    return w->planes == 3 ? gemv_wide_supports_p3(w, t < 16 ? t : 16) : gemv_wide_supports_p2(w, t < 16 ? t : 16);
+}
 bool g_quad_matvec = true, g_generic_forced = false;
 int launch_gemv(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, size_t n_ff, hipStream_t s) {
     const bool p3 = w->planes == 3;
+    if (!n_ff && g_quad_matvec && !g_generic_forced && d_x && d_y && takes_wide(w, rows_x)) {
+        for (size_t m0 = 0; m0 < rows_x;) {
+            const size_t t = rows_x - m0 < 16 ? rows_x - m0 : 16;
+            const float* x = d_x + m0 * w->cols;
+            float* y = d_y + m0 * w->rows;
+            int rc;
+            if (takes_wide(w, t)) rc = p3 ? launch_gemv_wide_p3(w, x, t, y, s) : launch_gemv_wide_p2(w, x, t, y, s);
+            else rc = p3 ? launch_gemv_p3(w, x, t, y, 0, s) : launch_gemv_p2(w, x, t, y, 0, s);
+            if (rc) return rc;
+            m0 += t;
+        }
+        return FHIP_OK;
+    }
     if (rows_x >= 3 && g_quad_matvec && !g_generic_forced && d_x && d_y &&
         (p3 ? gemv_quad_supports_p3(w, 4, n_ff) : gemv_quad_supports_p2(w, 4, n_ff))) {
         const size_t out_rows = n_ff ? n_ff : w->rows;

@@ -92,7 +92,9 @@ int launch_gemv(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_
     void gemv_force_generic##sfx(bool on);                                                                                         \
     bool gemv_streams##sfx(const fhip_weight* w, size_t n_ff);                                                                      \
     bool gemv_quad_supports##sfx(const fhip_weight* w, size_t rows_x, size_t n_ff);                                                 \
-    int launch_gemv_quad##sfx(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, size_t n_ff, hipStream_t s);
+    int launch_gemv_quad##sfx(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, size_t n_ff, hipStream_t s);       \
+    bool gemv_wide_supports##sfx(const fhip_weight* w, size_t t);                                                                   \
+    int launch_gemv_wide##sfx(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s);
 FHIP_GEMV_COPY(_p2)
 FHIP_GEMV_COPY(_p3)
 #undef FHIP_GEMV_COPY

@@ -1,0 +1,67 @@
+"""Batches of the 32-value formats on the kernel that multiplies through the 16 x 16 x 32 int8 matrix instruction (gemv_wide.hip)
+against single rows on the dot-product mat-vec it restates: the same bits for every row, whatever the batch a row sits in
+(crates/ferric-tensor/src/cpu_simd.rs:175-200); the entry points' own tests hold both to the oracle."""
+import numpy as np
+import pytest
+
+from conftest import bits
+
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("precision")]
+Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, IQ4_NL, IQ4_XS, MXFP4 = 2, 3, 6, 7, 8, 20, 23, 39
+# rows x cols: one block; whole tiles and groups; cut tiles and a last group of 1, 4 and 8 blocks; several passes over K (17408
+# columns); several tiles a workgroup
+SHAPES = [(1, 32), (16, 512), (37, 1056), (130, 2560), (9, 17408), (4200, 768)]
+
+
+def singles_of(F, qm, x):
+    return np.stack([F.Tensor.from_vec(r, (1, x.shape[1])).matmul_q(qm).to_vec() for r in x])
+
+
+def same(got, want):
+    ok = ~np.isnan(want)
+    return np.array_equal(np.isnan(got), ~ok) and np.array_equal(bits(got)[ok], bits(want)[ok])
+
+
+@pytest.mark.parametrize("ty", [Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, IQ4_NL, IQ4_XS, MXFP4])
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_same_bits_as_single_rows(F, ty, rows, cols):
+    from ferric_amd.synth import synth_weights
+    cols = max(256, cols // 256 * 256) if ty == IQ4_XS else cols
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, rows + cols), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(cols).standard_normal((18, cols)).astype(np.float32)
+    x[1] *= np.float32(300.0)
+    x[2, ::7] = 0
+    # runs block fixed point cannot hold: tiny, huge, infinite and NaN members, in rows of every accumulator
+    x[4, :32] *= np.float32(1e-36)
+    x[7, -32:] = np.float32(1e30)
+    x[9, cols // 2], x[14, 5] = np.inf, np.nan
+    one = singles_of(F, qm, x)
+    for m in (5, 8, 9, 16, 18):
+        got = F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows)
+        assert same(got, one[:m]), m
+
+
+@pytest.mark.parametrize("ty,rows,cols,m", [(Q5_1, 12300, 2080, 3), (IQ4_NL, 12289, 2048, 4), (Q8_0, 1200, 7040, 4)])
+def test_three_and_four_rows_of_large_weights(F, ty, rows, cols, m):
+    from ferric_amd.synth import synth_weights
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(4).standard_normal((m, cols)).astype(np.float32)
+    assert same(F.Tensor.from_vec(x, x.shape).matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
+
+
+def test_mxfp4_blocks_that_may_overflow(F):
+    """Scale bytes from 252 on: inf weights, and finite ones near the top of f32, beside ordinary blocks."""
+    rng = np.random.default_rng(21)
+    rows, cols = 40, 544
+    blk = rng.integers(0, 256, (rows, cols // 32, 17), dtype=np.uint8)
+    blk[:, :, 0] = rng.integers(0x70, 0x80, (rows, cols // 32), dtype=np.uint8)
+    blk[3, 5, 0], blk[7, 0, 0], blk[7, 9, 0], blk[11, 15, 0], blk[12, 2, 0], blk[33, 16, 0] = 255, 254, 253, 252, 251, 253
+    qm = F.QMatrix.from_bytes(blk.reshape(-1), MXFP4, rows, cols)
+    x = rng.standard_normal((16, cols)).astype(np.float32)
+    x[5, 160:168] = 0.0
+    one = singles_of(F, qm, x)
+    assert not np.isfinite(one[:, 7]).any()
+    for m in (5, 16):
+        assert same(F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows), one[:m]), m
