@@ -801,40 +801,65 @@ __global__ __launch_bounds__(256) void attn_split_fused_kernel(QkvPostParams fp,
     attn_split_body<G, DPL, true>(nullptr, fp.k_cache, fp.v_cache, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, fp, gq);
 }
 
-// One workgroup per query head: weights exp(m_s - max m) of the splits once (through LDS), then every output dim is a
-// weighted sum of the splits' accumulators over the weighted sum of their sums. splits <= 256. Always launched with
-// COMBINE_THREADS threads, whatever the head size: the loops below stride by that constant.
-constexpr int COMBINE_THREADS = 128;
-__global__ __launch_bounds__(COMBINE_THREADS) void attn_combine_kernel(const float* __restrict__ part, int hd, int splits, float* __restrict__ out) {
-    __shared__ float w[256], lw[256];
-    const int head = blockIdx.x, tid = threadIdx.x;
+// One workgroup per query head: weights exp(m_s - max m) of the splits once (each wave reduces them for itself; through LDS to
+// the threads that need one), then every output dim is a weighted sum of the splits' accumulators over the weighted sum of their
+// sums. splits <= 256. Thread (group, dim): group i of COMBINE_GROUPS takes splits i, i + COMBINE_GROUPS, ..., the groups meet in LDS.
+// Nothing but latency: with one thread a dim the splits came in six trips to memory one after the other, now in one (up to 64 splits;
+// 128 in two): 40 heads of 128, 64 splits 5.0 us, 20 heads, 128 splits 8.4.
+constexpr int COMBINE_GROUPS = 8;
+__global__ __launch_bounds__(128 * COMBINE_GROUPS) void attn_combine_kernel(const float* __restrict__ part, int hd, int splits, float* __restrict__ out) {
+    __shared__ float w[256];
+    __shared__ float red[COMBINE_GROUPS][128];
+    const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, grp = tid / hd, d = tid - grp * hd;   // (hd: 64 or 128)
     const float* pp = part + (size_t)head * splits * (hd + 2);
-    // this thread's output dim of the first splits is requested together with the splits' maxima and sums: one memory round
-    // trip instead of two in a row for the short caches, where this kernel is nothing but latency
-    constexpr int EARLY = 16;
+    // the first eight of the thread's splits are requested together with the splits' maxima and sums
+    constexpr int EARLY = 8;
     float pv[EARLY];
 #pragma unroll
-    for (int s = 0; s < EARLY; s++) pv[s] = (s < splits && tid < hd) ? pp[(size_t)s * (hd + 2) + tid] : 0.f;
-    for (int s = tid; s < splits; s += COMBINE_THREADS) { w[s] = pp[(size_t)s * (hd + 2) + hd]; lw[s] = pp[(size_t)s * (hd + 2) + hd + 1]; }
-    __syncthreads();
-    float M = -3.0e38f;
-    for (int s = 0; s < splits; s++) M = fmaxf(M, w[s]);
-    __syncthreads();
-    for (int s = tid; s < splits; s += COMBINE_THREADS) { const float f = __expf(w[s] - M); w[s] = f; lw[s] *= f; }
-    __syncthreads();
-    float L = 0.f;
-    for (int s = 0; s < splits; s++) L += lw[s];
-    for (int d = tid; d < hd; d += COMBINE_THREADS) {
-        float A = 0.f;
-        if (d == tid) {
-#pragma unroll
-            for (int s = 0; s < EARLY; s++)
-                if (s < splits) A = fmaf(pv[s], w[s], A);
-        }
-#pragma unroll 8
-        for (int s = d == tid ? EARLY : 0; s < splits; s++) A = fmaf(pp[(size_t)s * (hd + 2) + d], w[s], A);
-        out[(size_t)head * hd + d] = A / L;
+    for (int i = 0; i < EARLY; i++) {
+        const int s = grp + COMBINE_GROUPS * i;
+        pv[i] = s < splits ? pp[(size_t)s * (hd + 2) + d] : 0.f;
     }
+    float mv[4], lv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int s = lane + 64 * i;
+        mv[i] = -3.0e38f; lv[i] = 0.f;
+        if (s < splits) { mv[i] = pp[(size_t)s * (hd + 2) + hd]; lv[i] = pp[(size_t)s * (hd + 2) + hd + 1]; }
+    }
+    float M = fmaxf(fmaxf(mv[0], mv[1]), fmaxf(mv[2], mv[3]));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+    float L = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int s = lane + 64 * i;
+        const float f = s < splits ? __expf(mv[i] - M) : 0.f;
+        L = fmaf(lv[i], f, L);
+        if (tid < 64) w[s] = f;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
+    __syncthreads();
+    float A = 0.f;
+#pragma unroll
+    for (int i = 0; i < EARLY; i++) A = fmaf(pv[i], w[grp + COMBINE_GROUPS * i], A);   // (0 past the last split)
+    for (int s0 = grp + COMBINE_GROUPS * EARLY; s0 < splits; s0 += COMBINE_GROUPS * EARLY) {
+        float v[EARLY];
+#pragma unroll
+        for (int i = 0; i < EARLY; i++) {
+            const int s = s0 + COMBINE_GROUPS * i;
+            v[i] = s < splits ? pp[(size_t)s * (hd + 2) + d] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < EARLY; i++) A = fmaf(v[i], w[s0 + COMBINE_GROUPS * i], A);
+    }
+    red[grp][d] = A;
+    __syncthreads();
+    if (grp != 0) return;
+#pragma unroll
+    for (int i = 1; i < COMBINE_GROUPS; i++) A += red[i][d];
+    out[(size_t)head * hd + d] = A / L;
 }
 
 // ---------------------------------------------------------------- the same over a long block-quantized cache, on the matrix cores
@@ -1354,7 +1379,7 @@ int launch_decode_attention(const float* q, const float* K, const float* V, int 
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "decode_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3(COMBINE_THREADS), 0, s, ws, hd, splits, out);
+        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
         rc = check_hip(hipGetLastError(), "decode_attention combine launch");
     }
     return rc;
@@ -1412,7 +1437,7 @@ int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "decode_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3(COMBINE_THREADS), 0, s, ws, hd, splits, out);
+        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
         rc = check_hip(hipGetLastError(), "decode_attention combine launch");
     }
     return rc;
@@ -1465,7 +1490,7 @@ int launch_qkv_post_attention(const float* qkv, const float* bias, const float* 
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "qkv_post_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3(COMBINE_THREADS), 0, s, ws, hd, splits, out);
+        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
         rc = check_hip(hipGetLastError(), "qkv_post_attention combine launch");
     }
     return rc;
