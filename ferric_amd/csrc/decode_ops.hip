@@ -863,22 +863,27 @@ __global__ __launch_bounds__(128 * COMBINE_GROUPS) void attn_combine_kernel(cons
 }
 
 // ---------------------------------------------------------------- the same over a long block-quantized cache, on the matrix cores
-// All gq query heads of a KV head at once. A wave takes 32 keys at a time, in two tiles of 16.
-//   Scores: v_mfma_f32_16x16x32_bf16 with the codes of one block of 32 dims as the A operand (16 keys; whole numbers of at most eight
-//   bits, exact in bf16) and the query's 32 dims as the B operand (16 queries, gq of them real), cut into three bf16 values whose sum
-//   is the f32 query. Three instructions give the block's sum in f32; the block's scale multiplies it. Lane n + 16 g ends up with keys
-//   4 g .. 4 g + 3 of query n, so a query's maximum and sum are register operations and two exchanges.
-//   Values: f32 on v_mfma_f32_16x16x4: register r of a tile's probabilities is a B operand as it stands (four keys, 4 g + r, of query n);
-//   the A operand is dim 4 n + i of those keys, from a lane's four dims of a row of 64, dequantized as above.
-// Scales come one row a lane and go round through LDS (the wave's own part of it), the cut queries are shared there. The next round's
-// key codes are requested when the scores are done. The waves of a workgroup meet in LDS as above. A launch costs the same for any
-// number of query heads up to the eight taken (an instruction has room for 16).
-// What bounds it: three waves per SIMD at head size 128 (168 registers), each waiting for its rows and then issuing 24 + 64 matrix and
-// some 450 other instructions a round, about 7 us a round of the 3 at 32768 keys. With the combine launch, us, this | the kernel above,
-// 8 KV heads, 32768 Q8_0 keys: head size 128 (71 MB), 8 query heads each 39.5 | 59.4; head size 64, 5: 25.2 | 33.2, 8: 24.5 | 45.4.
-// Error against f64 (2-norm, relative, six draws) at those shapes 2.7e-7 | 2.8e-7, 2.4e-7 .. 2.6e-7 | 2.5e-7 .. 2.7e-7. Q4_1 is left to the kernel
-// above: the minimum as a product of its own cost 2 % more error. Tried: values on the 4 x 4 x 1 instruction (the same times, an
-// instantiation per group size), scores on it as well (slower by 2 us: it issues once in some 20 cycles), 64 keys a round (spills, +17 us).
+// All gq query heads of a KV head at once. A wave takes 32 keys at a time, in two tiles of 16, everything on v_mfma_f32_16x16x32_bf16 with
+// the codes (whole numbers of at most eight bits, exact in bf16) as the A operand and an f32 cut into three bf16 values, whose sum it is, as
+// the B operand: products are exact, sums f32.
+//   Scores: A = one block of 32 dims of 16 keys, B = the query's 32 dims. Three instructions give the block's sum in f32; the block's scale
+//   multiplies it. Lane n + 16 g ends up with keys 4 g .. 4 g + 3 of column n's query, so a query's maximum and sum are register operations
+//   and two exchanges.
+//   Values: A = 16 dims of one block of 32 keys, B = probability times the block's scale at that key (one rounding) of column n's query: the
+//   eight keys of k-group g are the ones whose probabilities the lane holds. Two instructions a block and cut; the sums stay in the
+//   accumulators, the running maximum's correction is skipped where no maximum moved.
+// Up to five query heads a KV head (SPL): the 16 columns hold every query three times and column n takes cut n / gq of its query's products
+// (the three sums meet at the end), a third of the values' instructions. Six to eight: a column a query, three instructions.
+// Scales come one row a lane and go round through LDS (the wave's own part of it), the cut queries are shared there. At head size 64 the next
+// round's key codes are requested when the scores are done; at 128 they would not fit the 128 registers that let four waves share a
+// SIMD, and the other waves' arithmetic runs under the request. The waves of a workgroup meet in LDS as above.
+// What bounds it: instruction issue. A wave's round is some 700 vector instructions (a fifth each: codes to bf16, probabilities times scales
+// and their cuts) and 32 matrix instructions of 16 cycles (SPL; 48 otherwise); the rows' bytes (71 MB at 8 KV heads of 128, 32768 Q8_0 keys) would take 13 us.
+// At that shape, us, before (values on f32 matrix instructions for six query heads and more, the dot-product kernel for fewer) -> now: 5 query
+// heads a KV head 38.3 -> 27.0, 8: 33.9 -> 26.4; head size 64, 4: 23.0 -> 17.2. Error against f64 (2-norm, relative, eighteen shapes) no larger in any:
+// 2.2e-7 .. 2.5e-7 before, 1.4e-7 .. 1.8e-7 with the combine launch's present order. Tried: the codes requested as consecutive
+// 16-byte pieces and turned through LDS (31 us at head size 128, level at 64: what the address unit saves goes into LDS reads and spills).
+// Q4_1 is left to the kernel above: the minimum as a product of its own cost 2 % more error.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 union Frag { uint32_t w[4]; bf16x8 v; };
@@ -906,20 +911,22 @@ __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) 
     return f.v;
 }
 
-constexpr int LONG_WAVES = 6, LONG_KEYS = 32;   // waves of a workgroup, keys a wave takes at a time
-template <int HD, int FMT>
-__global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
+constexpr int LONG_WAVES = 8, LONG_KEYS = 32;   // waves of a workgroup, keys a wave takes at a time
+template <int HD, int FMT, bool SPL>
+__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
                                                                            const uint32_t* __restrict__ len_dev, float scale, int splits,
-                                                                           uint32_t window, float softcap, float* __restrict__ part, int gq) {   // gq: query heads per KV head, at most 8
-    constexpr int NB = HD / 32, NT = LONG_KEYS / 16, NH = HD / 64;      // blocks of a row, tiles of 16 keys, 64-dim parts of a row
-    constexpr int CW = FMT == FHIP_KVQ_Q8_0 ? 8 : 4;                    // code words of a block
+                                                                           uint32_t window, float softcap, float* __restrict__ part, int gq) {   // gq: query heads per KV head, at most 8 (SPL: 5)
+    constexpr int NB = HD / 32, NT = LONG_KEYS / 16;                    // blocks of a row, tiles of 16 keys
+    constexpr bool Q8 = FMT == FHIP_KVQ_Q8_0, PRE = HD == 64;             // PRE: keys requested a round ahead
+    constexpr int CW = Q8 ? 8 : 4;                                      // code words of a block
     static_assert(FMT == FHIP_KVQ_Q8_0 || FMT == FHIP_KVQ_Q4_0, "");
     __shared__ float sm_m[LONG_WAVES][8], sm_l[LONG_WAVES][8];
     __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][8][HD + 4];    // rows four banks apart
     __shared__ __attribute__((aligned(16))) float sm_d[LONG_WAVES][NB][64];   // rows 0 .. 31 the keys' scales, 32 .. 63 the values'
-    __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of query n at lane n + 16 g, three bf16 each
+    __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of column n's query at lane n + 16 g, three bf16 each
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
+    const int cut = SPL ? n / gq : 0, qn = SPL ? n - cut * gq : n;     // the column's query and, SPL, its cut (3: a column without one)
     const int kvh = blockIdx.x, split = blockIdx.y, head0 = kvh * gq;
     uint32_t len = len_dev ? *len_dev + 1u : len_host;
     if (len > len_host) len = len_host;
@@ -946,13 +953,13 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const
         for (int i = 0; i < NB / 2; i++) sc[i] = sp[i];
     };
     uint32_t kt = k0 + (uint32_t)(LONG_KEYS * wave);
-    if (kt < k1) request_k(kt);
+    if (PRE && kt < k1) request_k(kt);
 
     if (wave < NB) {                                                    // wave j cuts the queries' block j up for all
         float x[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) x[i] = 0.f;
-        if (n < gq) load_dims<8>(q + ((size_t)head0 + n) * HD + 32 * wave + 8 * g, x);
+        if (qn < gq) load_dims<8>(q + ((size_t)head0 + qn) * HD + 32 * wave + 8 * g, x);
 #pragma unroll
         for (int t = 0; t < 3; t++) {
             sm_q[wave][t][lane] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
@@ -962,37 +969,48 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const
     }
     __syncthreads();
 
-    const int vblk = n >> 3, word = n & (CW - 1), shift = (n & 7) < 4 ? 0 : 4;               // of dims 4 n .. 4 n + 3 of a 64-dim part
-    const uint32_t vrow = (uint32_t)(4 * g) * (uint32_t)nblk + (uint32_t)vblk;              // blocks from a tile's first to the lane's
-    const uint32_t vco = (vrow * CW + (uint32_t)word) * 4u;
+    // The lane's A row of a block's two tiles: dims 2 n and 2 n + 1 (Q8_0, the two bytes of a half word), n and 16 + n (4-bit formats, the two
+    // nibbles of a byte).
+    const uint32_t row_b = (uint32_t)nblk * (CW * 4);                   // bytes from a row's codes to the next row's
+    const uint32_t vco = (uint32_t)(4 * g) * row_b + (uint32_t)(Q8 ? 2 * n : n);
+    auto load_code = [&](const char* p) -> uint32_t { return Q8 ? (uint32_t)*(const uint16_t*)p : (uint32_t)*(const uint8_t*)p; };
+    const uint32_t cut1 = cut >= 1 ? 0xFFFF0000u : 0u, cut2 = cut >= 2 ? 0xFFFF0000u : 0u;
 
-    f32x4 run[NH][4];                       // [part][i]: dims 64 part + 16 g + 4 r + i of query n
-    float m = -3.0e38f, l = 0.f;            // of query n
+    f32x4 run[NB][2];                       // [block][tile]: A rows 4 g + r of column n
+    float m = -3.0e38f, l = 0.f;            // of column n's query
 #pragma unroll
-    for (int h = 0; h < NH; h++)
+    for (int j = 0; j < NB; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) run[h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 2; i++) run[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (; kt < k1; kt += LONG_KEYS * LONG_WAVES) {
         const uint32_t last = k1 - 1u - kt;
-        uint32_t vw[NT][4][NH];                 // [tile][r][part]: dims 4 n .. + 3 of the part, key 16 t + 4 g + r
+        if (!PRE) request_k(kt);
+        uint32_t vw[NB][NT][2];                 // [block][tile of keys]: the codes of keys 16 t + 4 g + (0, 1) and + (2, 3), a half word each
+        const char* vc = (const char*)(qc.v_codes + ((size_t)kt * nblk + (size_t)kvh * NB) * CW);
         if (last >= LONG_KEYS - 1u) {
             // a lane's own part of the address is the same for every row (and fits 32 bits); the rest is the wave's
-            const char* vc = (const char*)(qc.v_codes + ((size_t)kt * nblk + (size_t)kvh * NB) * CW);
 #pragma unroll
-            for (int i = 0; i < NT * 4 * NH; i++) {
-                const int t = i / (4 * NH), r = i / NH % 4, h = i % NH;
-                vw[t][r][h] = *(const uint32_t*)(vc + ((size_t)(16 * t + r) * nblk + 2 * h) * (CW * 4) + vco);
-            }
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r += 2)
+#pragma unroll
+                    for (int j = 0; j < NB; j++) {
+                        const char* p = vc + (size_t)(16 * t + r) * row_b + j * (CW * 4);
+                        vw[j][t][r >> 1] = load_code(p + vco) | load_code(p + row_b + vco) << 16;
+                    }
         } else {
 #pragma unroll
-            for (int i = 0; i < NT * 4; i++) {
-                uint32_t mine = (uint32_t)(4 * g);
-                asm volatile("" : "+v"(mine));                          // worked out here: kept from round to round these are eight more registers
-                const size_t b = (size_t)(kt + min(mine + (uint32_t)(16 * (i / 4) + i % 4), last)) * nblk + (size_t)kvh * NB + (size_t)vblk;
+            for (int t = 0; t < NT; t++)
 #pragma unroll
-                for (int h = 0; h < NH; h++) vw[i / 4][i % 4][h] = qc.v_codes[(b + 2 * h) * CW + word];
-            }
+                for (int r = 0; r < 4; r += 2) {
+                    uint32_t mine = (uint32_t)(4 * g);
+                    asm volatile("" : "+v"(mine));                      // worked out here: kept from round to round these are eight more registers
+                    const char* p0 = vc + (size_t)min(mine + (uint32_t)(16 * t + r), last) * row_b + (Q8 ? 2 * n : n);
+                    const char* p1 = vc + (size_t)min(mine + (uint32_t)(16 * t + r + 1), last) * row_b + (Q8 ? 2 * n : n);
+#pragma unroll
+                    for (int j = 0; j < NB; j++) vw[j][t][r >> 1] = load_code(p0 + j * (CW * 4)) | load_code(p1 + j * (CW * 4)) << 16;
+                }
         }
 #pragma unroll
         for (int i = 0; i < NB / 2; i++) {
@@ -1002,7 +1020,7 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const
         }
         asm volatile("" ::: "memory");          // a wave's LDS accesses complete in order; this keeps the compiler's in order too
 
-        float p[NT][4];                         // [tile][r]: key 16 t + 4 g + r of query n
+        float p[NT][4];                         // [tile][r]: key 16 t + 4 g + r of column n's query
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -1025,7 +1043,7 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const
             asm volatile("" ::: "memory");      // a block at a time: the operands of all of them do not fit the registers
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (kt + LONG_KEYS * LONG_WAVES < k1) request_k(kt + LONG_KEYS * LONG_WAVES);
+        if (PRE && kt + LONG_KEYS * LONG_WAVES < k1) request_k(kt + LONG_KEYS * LONG_WAVES);
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -1056,39 +1074,86 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 3) void attn_long_kvq_kernel(const
             ps[t] = (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
         }
         l = fmaf(l, corr, ps[0] + ps[1]);
+        if (__builtin_amdgcn_ballot_w64(m_new != m) != 0) {
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) run[j][i] *= corr;
+        }
         m = m_new;
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int j = 0; j < NB; j++) {
+            float x[2 * 4];                     // probability times the block's scale, key 16 t + 4 g + r at 4 t + r
 #pragma unroll
-            for (int h = 0; h < NH; h++) {
-                const f32x4 d = *(const f32x4*)&sm_d[wave][2 * h + vblk][32 + 16 * t + 4 * g];
-                f32x4 acc[4];                   // the tile's sums start at zero: chains of 16 keys, then one addition
+            for (int t = 0; t < NT; t++) {
+                const f32x4 d = *(const f32x4*)&sm_d[wave][j][32 + 16 * t + 4 * g];
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    float v[4];
-                    expand_dims_f<FMT>(vw[t][r][h], shift, d[r], 0.f, v);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], p[t][r], acc[i], 0, 0, 0);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) run[h][i][r] = t == 0 ? fmaf(run[h][i][r], corr, acc[i][r]) : run[h][i][r] + acc[i][r];
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < 4; r++) x[4 * t + r] = p[t][r] * d[r];
             }
+            Frag a[2];                          // the codes of the block's two tiles of dims
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t w = vw[j][e >> 1][e & 1];
+                    float lo, hi;
+                    if constexpr (Q8) { lo = (float)(int8_t)(w >> (8 * i)); hi = (float)(int8_t)(w >> (16 + 8 * i)); }
+                    else { lo = (float)((w >> (4 * i)) & 15u) - 8.0f; hi = (float)((w >> (16 + 4 * i)) & 15u) - 8.0f; }
+                    a[i].w[e] = upper_halves(lo, hi);
+                }
+            if constexpr (SPL) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    x[e] -= __uint_as_float(__float_as_uint(x[e]) & cut1);
+                    x[e] -= __uint_as_float(__float_as_uint(x[e]) & cut2);
+                }
+                Frag f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) f.w[e] = upper_halves(x[2 * e], x[2 * e + 1]);
+#pragma unroll
+                for (int i = 0; i < 2; i++) run[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].v, f.v, run[j][i], 0, 0, 0);
+            } else {
+                Frag f[3];
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        f[k].w[e] = upper_halves(x[2 * e], x[2 * e + 1]);
+                        x[2 * e] -= __uint_as_float(__float_as_uint(x[2 * e]) & 0xFFFF0000u);
+                        x[2 * e + 1] -= __uint_as_float(__float_as_uint(x[2 * e + 1]) & 0xFFFF0000u);
+                    }
+#pragma unroll
+                for (int k = 2; k >= 0; k--)    // (smallest cut first)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) run[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].v, f[k].v, run[j][i], 0, 0, 0);
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
+    if constexpr (SPL) {                        // column n < gq takes its other two cuts
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float v = run[j][i][r];
+                    run[j][i][r] = v + (__shfl(v, (lane & 48) | ((n + gq) & 15)) + __shfl(v, (lane & 48) | ((n + 2 * gq) & 15)));
+                }
+    }
     if (lane < gq) { sm_m[wave][lane] = m; sm_l[wave][lane] = l; }
     if (n < gq) {
 #pragma unroll
-        for (int h = 0; h < NH; h++)
+        for (int j = 0; j < NB; j++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                *(f32x4*)&sm_acc[wave][n][64 * h + 16 * g + 4 * r] = f32x4{run[h][0][r], run[h][1][r], run[h][2][r], run[h][3][r]};
+            for (int r = 0; r < 4; r++) {
+                const int mrow = 4 * g + r;     // A row: dims 2 mrow, 2 mrow + 1 (Q8_0), mrow, 16 + mrow
+                sm_acc[wave][n][32 * j + (Q8 ? 2 * mrow : mrow)] = run[j][0][r];
+                sm_acc[wave][n][32 * j + (Q8 ? 2 * mrow + 1 : 16 + mrow)] = run[j][1][r];
+            }
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < gq * HD; idx += 64 * LONG_WAVES) {
@@ -1146,20 +1211,22 @@ int launch_attn_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, con
     }
 }
 
-// Which launches take it: the kernel above costs less for few query heads a KV head. A decode step of four layers (d 2048), four tokens, us,
-// this | that: 8 KV heads, head size 128, 32768 keys, 8 query heads each Q8_0 1393 | 1596, 5: 1364 | 1337, Q4_0 1420 | 1371; 4 KV heads, 8, 9000 keys
-// Q4_0 1012 | 1044; head size 64, 8: 32768 keys Q4_0 1079 | 1350, 5: 10000 keys Q8_0 848 | 881, 4 KV heads, 4: 6000 keys 837 | 840.
+// Which launches take it: its cost does not depend on the number of query heads a KV head, the kernel above costs less for one and two. us, this | that
+// without the combine launch, 8 KV heads, head size 128, 32768 Q8_0 keys: 2 query heads each 26.4 | 23.1, 3: 26.7 | 27.6, 4: 26.8 | 32.2, 5: 27.0 | 38.3;
+// Q4_0, 3: 26.3 | 30.1, 5: 25.7 | 38.8; 8000 keys Q8_0, 3: 11.4 | 12.0, 4: 11.3 | 13.6; head size 64, 32768 keys, 3: 16.8 | 19.5, 4: 17.2 | 23.0; 8000 keys,
+// 3: 8.8 | 9.2; 4 KV heads of 128, 9000 keys, 3: 10.6 | 9.8, 5: 10.9 | 13.5.
 // Key codes are read eight bytes at a time; a lane's offset inside a round's rows is kept in 32 bits (n_kv).
-bool attn_long_takes(int fmt, int g, int hd, int n_kv, const uint32_t* k_codes) {
+bool attn_long_takes(int fmt, int g, int n_kv, const uint32_t* k_codes) {
     if (fmt == FHIP_KVQ_Q4_1 || g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
-    return g >= (hd == 64 ? 5 : 6);
+    return g >= 3;
 }
 template <int FMT>
 void launch_attn_long_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, const QCache& qc, int n_kv, uint32_t len, const uint32_t* d_len,
                           float scale, int splits, uint32_t window, float softcap, float* part) {
     const dim3 wg(64 * LONG_WAVES);
-    if (hd == 64) hipLaunchKernelGGL((attn_long_kvq_kernel<64, FMT>), grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g);
-    else hipLaunchKernelGGL((attn_long_kvq_kernel<128, FMT>), grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g); };
+    if (hd == 64) { if (g <= 5) go(attn_long_kvq_kernel<64, FMT, true>); else go(attn_long_kvq_kernel<64, FMT, false>); }
+    else { if (g <= 5) go(attn_long_kvq_kernel<128, FMT, true>); else go(attn_long_kvq_kernel<128, FMT, false>); }
 }
 
 template <int G>
@@ -1412,7 +1479,7 @@ int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes
     const int splits = mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "decode_attention: this cache length needs the workspace");
     const dim3 grid((unsigned)n_kv, (unsigned)splits);
-    if (!mid && splits > 1 && attn_long_takes(fmt, g, hd, n_kv, k_codes)) {
+    if (!mid && splits > 1 && attn_long_takes(fmt, g, n_kv, k_codes)) {
         rc = FHIP_OK;
         switch (fmt) {
             case FHIP_KVQ_Q8_0: launch_attn_long_kvq<FHIP_KVQ_Q8_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws); break;

@@ -242,6 +242,14 @@ def test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, h
             assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max(), (n, window)
 
 
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("nh,nkv,hd,rows,lengths", [
+    (3, 1, 64, 5121, (5121, 257)), (4, 1, 128, 5377, (5377, 256)), (10, 2, 128, 9001, (9001, 33)), (15, 3, 64, 7001, (7001,)), (21, 3, 128, 5200, (5200,))])
+def test_long_caches_by_cut_columns_and_by_query_columns(F, Q, K, fmt, nh, nkv, hd, rows, lengths):
+    """Three to five query heads a KV head (a column holds one cut of a query's products) and seven, at the edges of eight waves' rounds."""
+    test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, hd, rows, lengths)
+
+
 def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
     rng = np.random.default_rng(80)
     t, width, cap = 5, 256, 16
