@@ -76,6 +76,7 @@ __device__ __forceinline__ constexpr int kcol(int t, int h) { return 32 * (t >> 
 // ------------------------------------------------------------------------------------------------
 
 struct Q4K {
+    using Eager = Q4K;
     static constexpr int BLOCK = 144;
     static constexpr float UNPACK_US = 1.4f;   // unpack of a 256 x 256 chunk by one workgroup
     // one chunk of a workgroup tile of 64 x 256, 128 x 256, 256 x 256, 256 x 160, 128 x 128, 64 x 128, 128 x 160, in us (fitted, see plan_cost_us)
@@ -104,7 +105,7 @@ struct Q4K {
         }
     }
     template <int G>
-    static __device__ __forceinline__ void begin(Raw& r, int, int, int, Ctx& x) {
+    static __device__ __forceinline__ void begin(Raw& r, const uint8_t*, int, int, int, Ctx& x) {
         if (G == 0) r.hd = r.hdn;
         const float d = f16_bits(r.hd[0] & 0xFFFFu), dmin = f16_bits(r.hd[0] >> 16);
         float s0, m0, s1, m1;
@@ -135,6 +136,7 @@ struct Q4K {
 // step G takes bit 2G + (T >> 1) of them. The high nibbles are shifted down (with the fifth bit on top they do not fit a
 // byte in place), so both sub-block scales are plain d * sc.
 struct Q5K {
+    using Eager = Q5K;
     static constexpr int BLOCK = 176;
     static constexpr float UNPACK_US = 1.8f;
     static constexpr float CHUNK_US[7] = {3.83f, 5.16f, 9.41f, 6.12f, 3.17f, 2.26f, 3.78f};
@@ -152,7 +154,7 @@ struct Q5K {
         for (int g = 0; g < 4; g++) r.q[g] = *(const u32x4*)(blk + 48 + 32 * g + 16 * h);
     }
     template <int G>
-    static __device__ __forceinline__ void begin(Raw& r, int, int, int, Ctx& x) {
+    static __device__ __forceinline__ void begin(Raw& r, const uint8_t*, int, int, int, Ctx& x) {
         if (G == 0) { r.hd = r.hdn; r.qh = r.qhn; }
         const float d = f16_bits(r.hd[0] & 0xFFFFu), dmin = f16_bits(r.hd[0] >> 16);
         float s0, m0, s1, m1;
@@ -182,6 +184,7 @@ struct Q5K {
 };
 
 struct Q6K {
+    using Eager = Q6K;
     // Step G covers half hf = G >> 1 of the super-block and its groups g0 = 2(G & 1), g0 + 1 (low nibbles of
     // ql for G even, high nibbles for G odd); slice T is group g = g0 + (T >> 1), l = 16h + 8(T & 1) + [0, 8),
     // whose scale is sc[8hf + 2g + h]  (crates/ferric-gguf/src/lib.rs:833-851).
@@ -207,7 +210,7 @@ struct Q6K {
         r.d = r.dn;
     }
     template <int G>
-    static __device__ __forceinline__ void begin(Raw& r, int, int h, int, Ctx& x) {
+    static __device__ __forceinline__ void begin(Raw& r, const uint8_t*, int, int h, int, Ctx& x) {
         if (G == 0) {
             // byte h of every 16-bit pair is this lane half's scale: shift it down once per chunk
 #pragma unroll
@@ -247,16 +250,26 @@ struct Q6K {
     }
 };
 
-struct Q80 {
+// LATE: a piece stays as it was loaded until the step that reads it shifts it into place (loads.hpp). Shifted beside its load it is
+// waited for right there. At 64 and 128 rows a step is too short to hide that behind the other wave of a SIMD; at 256 rows it is not, and
+// the registers of the unshifted pieces cost more (Eager). Measured, us, shifted at once -> late: 128 x 160 tiles of 5120 x 13824 at 64 /
+// 128 / 256 rows 53.8 / 57.8 / 91.9 -> 47.4 / 50.7 / 80.2, of 4096 x 4096 29.4 -> 27.7 at 128; 64 x 256 78.8 -> 75.9, 64 x 128 109.8 ->
+// 105.3, 128 x 128 63.1 -> 61.6 at 128 rows; 256 x 256 at 2048 rows 379 -> 383, 256 x 160 on 17408 x 4096 387 -> 393. Q6_K, whose pieces
+// are shifted once for four steps but unpacked by more arithmetic, lost 2 ... 7 % in every tile and shifts at once. With CHUNK_US for what
+// a chunk takes now, 14 % of shapes change their tile, to 128 x 160: 1280 x 8704 at 378 rows 44.5 -> 36.8, 1616 x 2304 at 874 40.1 -> 27.9,
+// 9392 x 11776 at 40 69.7 -> 58.5, 9328 x 2304 at 267 50.3 -> 41.4 (worst of fourteen: 4424 x 5120 at 35 rows 28.0 -> 29.3).
+template <bool LATE>
+struct Q80T {
+    using Eager = Q80T<false>;
     // A chunk is 8 blocks of 34 bytes; step G covers blocks 2G, 2G+1; slice T is block 2G + (T >> 1),
     // elements 16h + 8(T & 1) + [0, 8). A trailing partial chunk is allowed: blocks past the row's end are
     // read from the last valid block's address and given scale 0 (their activations are staged as 0 too).
     static constexpr int BLOCK = 34;
     static constexpr float UNPACK_US = 5.1f;
-    static constexpr float CHUNK_US[7] = {9.51f, 9.88f, 11.93f, 6.86f, 7.16f, 6.65f, 5.76f};
+    static constexpr float CHUNK_US[7] = {9.40f, 9.88f, 11.93f, 6.86f, 7.00f, 6.50f, 5.05f};
     static constexpr bool PARTIAL = true;   // a row may end inside a chunk
     static __host__ __device__ int chunks(int K) { return (K + 255) / 256; }
-    struct Raw { u32x4 q[4][2]; uint32_t d[4][2]; };
+    struct Raw { fhip::Un16 q[4][2]; uint32_t d[4][2]; };
     struct Ctx { float d[2]; };
     static __device__ __forceinline__ const uint8_t* blk(const uint8_t* row, int c, int i, int nblk) {
         int bi = 8 * c + i;
@@ -270,19 +283,24 @@ struct Q80 {
             for (int u = 0; u < 2; u++) {
                 const uint8_t* p = blk(row, c, 2 * g + u, nblk);
                 r.d[g][u] = *(const uint16_t*)p;
-                r.q[g][u] = fhip::load16_a2(p + 2 + 16 * h);
+                r.q[g][u] = fhip::load16_un<LATE>(p + 2 + 16 * h);
             }
     }
     template <int G>
-    static __device__ __forceinline__ void begin(Raw& r, int c, int, int nblk, Ctx& x) {
+    static __device__ __forceinline__ void begin(Raw& r, const uint8_t* row, int c, int, int nblk, Ctx& x) {
 #pragma unroll
-        for (int u = 0; u < 2; u++) x.d[u] = (8 * c + 2 * G + u) < nblk ? f16_bits(r.d[G][u]) : 0.0f;
+        for (int u = 0; u < 2; u++) {
+            const int i = 8 * c + 2 * G + u, bi = i < nblk ? i : nblk - 1;
+            // the quants' address modulo 4: blocks are 34 bytes apart, the quants 2 behind the block's start
+            if (LATE) fhip::shift_in_place(r.q[G][u], ((uint32_t)(uintptr_t)row + 2u * (uint32_t)(bi & 1) + 2u) & 2u);
+            x.d[u] = i < nblk ? f16_bits(r.d[G][u]) : 0.0f;
+        }
     }
     template <int G, int T>
     static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
         // q = (q ^ 0x80) - 128 with the biased byte unsigned: d*q = d*u - 128*d, every term exact in f32
         const float d = x.d[T >> 1];
-        return frag8(r.q[G][T >> 1][2 * (T & 1)] ^ 0x80808080u, r.q[G][T >> 1][2 * (T & 1) + 1] ^ 0x80808080u, d, -128.0f * d);
+        return frag8(r.q[G][T >> 1].w[2 * (T & 1)] ^ 0x80808080u, r.q[G][T >> 1].w[2 * (T & 1) + 1] ^ 0x80808080u, d, -128.0f * d);
     }
     template <int G>
     static __device__ __forceinline__ void refill(Raw& r, const uint8_t* row, int nc, int h, int nblk) {
@@ -290,10 +308,12 @@ struct Q80 {
         for (int u = 0; u < 2; u++) {
             const uint8_t* p = blk(row, nc, 2 * G + u, nblk);
             r.d[G][u] = *(const uint16_t*)p;
-            r.q[G][u] = fhip::load16_a2(p + 2 + 16 * h);
+            r.q[G][u] = fhip::load16_un<LATE>(p + 2 + 16 * h);
         }
     }
 };
+
+using Q80 = Q80T<true>;
 
 struct GemmParams {
     const uint8_t* W;
@@ -455,7 +475,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
     {
         const int nc = c_begin + 1 < c_last ? c_begin + 1 : c_last;
         typename F::Ctx x;
-        F::template begin<0>(raw, c_begin, h, p.nblk, x);
+        F::template begin<0>(raw, wrow, c_begin, h, p.nblk, x);
         static_for<0, 4>([&](auto T) {
             if (mine(T.value)) *(bf16x8*)(&Bs[0][b_wr + T.value * FRAG]) = F::template frag<0, T.value>(raw, x);
         });
@@ -487,7 +507,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
         };
         read_ops(0, a[0], b[0]);
         load_a(4 * ck + G + 1);
-        F::template begin<GN>(raw, pc, h, p.nblk, ctx);
+        F::template begin<GN>(raw, wrow, pc, h, p.nblk, ctx);
         __builtin_amdgcn_sched_barrier(0);
         static_for<0, 4>([&](auto S) {
             constexpr int t = decltype(S)::value;
@@ -676,7 +696,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
         F::prime(raw, wrow, c_begin, h, p.nblk);
         const int nc = c_begin + 1 < c_last ? c_begin + 1 : c_last;
         typename F::Ctx x;
-        F::template begin<0>(raw, c_begin, h, p.nblk, x);
+        F::template begin<0>(raw, wrow, c_begin, h, p.nblk, x);
         static_for<0, 4>([&](auto T) {
             *(bf16x8*)(&Bs[0][b_wr + T.value * FRAG]) = F::template frag<0, T.value>(raw, x);
         });
@@ -705,7 +725,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
         };
         read_ops(0, a[0], b[0]);
         if constexpr (!(UNPACK && SPLIT)) load_a(4 * ck + G + 1);
-        if constexpr (UNPACK) F::template begin<GN>(raw, pc, h, p.nblk, ctx);
+        if constexpr (UNPACK) F::template begin<GN>(raw, wrow, pc, h, p.nblk, ctx);
         __builtin_amdgcn_sched_barrier(0);
         static_for<0, 4>([&](auto S) {
             constexpr int t = decltype(S)::value;
@@ -936,7 +956,7 @@ __global__ void __launch_bounds__(256, TP == 8 ? 4 : 2) gemm_q_bf16_skinny_kerne
         store_x(0);
         {
             typename F::Ctx x;
-            F::template begin<0>(raw, c_begin, h, p.nblk, x);
+            F::template begin<0>(raw, wrow, c_begin, h, p.nblk, x);
             static_for<0, 4>([&](auto T) { b[T.value] = F::template frag<0, T.value>(raw, x); });
         }
         __syncthreads();
@@ -953,7 +973,7 @@ __global__ void __launch_bounds__(256, TP == 8 ? 4 : 2) gemm_q_bf16_skinny_kerne
                 constexpr int GN = (G + 1) & 3;
                 typename F::Ctx x;
                 if constexpr (G == 3) {
-                    F::template begin<0>(nxt, cn, h, p.nblk, x);
+                    F::template begin<0>(nxt, wrow, cn, h, p.nblk, x);
                     static_for<0, 4>([&](auto T) {
                         constexpr int t = decltype(T)::value;
                         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t], b[t], acc, 0, 0, 0);
@@ -964,7 +984,7 @@ __global__ void __launch_bounds__(256, TP == 8 ? 4 : 2) gemm_q_bf16_skinny_kerne
 #pragma unroll
                     for (int t = 0; t < 4; t++) a[t] = *(const bf16x8*)(&Xs[buf ^ 1][a_rd + kcol(t, 0)]);
                 } else {
-                    F::template begin<GN>(raw, ck, h, p.nblk, x);
+                    F::template begin<GN>(raw, wrow, ck, h, p.nblk, x);
                     static_for<0, 4>([&](auto T) {
                         constexpr int t = decltype(T)::value;
                         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t], b[t], acc, 0, 0, 0);
@@ -1051,7 +1071,7 @@ int launch_skinny(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_
     p.ws = d_ws; p.kmax = q.kmax;
     if (q.split && (!d_ws || ws_bytes < skinny_ws_bytes(q)))
         return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: the launch cuts row groups along K and needs %zu bytes of workspace", skinny_ws_bytes(q));
-    if (t <= 8) hipLaunchKernelGGL((gemm_q_bf16_skinny_kernel<F, 8>), dim3(q.grid), dim3(256), 0, s, p);
+    if (t <= 8) hipLaunchKernelGGL((gemm_q_bf16_skinny_kernel<typename F::Eager, 8>), dim3(q.grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((gemm_q_bf16_skinny_kernel<F, 32>), dim3(q.grid), dim3(256), 0, s, p);
     if (q.split)
         hipLaunchKernelGGL(sum_split_groups_kernel, dim3((unsigned)q.groups, (unsigned)((t + 1) / 2)), dim3(256), 0, s, d_y, (const float*)d_ws, p.T, p.N, q.tp, p.nchunks,
@@ -1146,9 +1166,10 @@ int launch_cfg(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out,
     p.ws = d_ws; p.kmax = q.kmax;
     if (q.split_wgs > 0 && (!d_ws || ws_bytes < plan_ws_bytes(q)))
         return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: the launch cuts tiles along K and needs %zu bytes of workspace", plan_ws_bytes(q));
-    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 2, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
-    else if constexpr (BN == 128) hipLaunchKernelGGL((gemm_q_bf16_kernel<F, MI, 1, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<F, MI, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    using W = std::conditional_t<MI == 4, typename F::Eager, F>;
+    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<W, MI, 2, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    else if constexpr (BN == 128) hipLaunchKernelGGL((gemm_q_bf16_kernel<W, MI, 1, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<W, MI, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
     if (q.split_wgs > 0 && SWIGLU)
         hipLaunchKernelGGL(sum_split_swiglu_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 8 + 255) / 256)), dim3(256), 0, s, p.H, (const float*)d_ws, p.T, p.ff, 64 * MI,
                            BN, p.tiles_n, p.nchunks, p.per, p.kmax, (int)(p.whole_rounds * cus));

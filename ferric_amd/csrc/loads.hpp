@@ -30,4 +30,19 @@ __device__ __forceinline__ ld_u32x2 load8_a2(const uint8_t* p) {
     return (ld_u32x2){__builtin_amdgcn_alignbyte(w[1], w[0], m), __builtin_amdgcn_alignbyte(e, w[1], m)};
 }
 
+// The same in two halves, for loops that ask for a piece long before they read it. The shift needs the loaded dwords: beside the load
+// it is a wait for memory however far the first use is, since the compiler does not carry it over a barrier. So the piece is kept as
+// it came and shifted where it is read, by the address modulo 4 (0 or 2). LATE = false shifts at once,
+// in registers of the plain size.
+struct Un16 { ld_u32x4 w; uint32_t e; };
+template <bool LATE>
+__device__ __forceinline__ Un16 load16_un(const uint8_t* p) {
+    if (!LATE) return Un16{load16_a2(p), 0u};
+    return Un16{((const LdU4A4*)(p - ((uint32_t)(uintptr_t)p & 2u)))->v, *(const uint16_t*)(p + 14)};
+}
+__device__ __forceinline__ void shift_in_place(Un16& u, uint32_t m) {
+    u.w = (ld_u32x4){__builtin_amdgcn_alignbyte(u.w[1], u.w[0], m), __builtin_amdgcn_alignbyte(u.w[2], u.w[1], m),
+                     __builtin_amdgcn_alignbyte(u.w[3], u.w[2], m), __builtin_amdgcn_alignbyte(u.e, u.w[3], m)};
+}
+
 }  // namespace fhip
