@@ -6,9 +6,17 @@
 // than `window` masked), chunked_attention (:239-265, T query rows against S >= T cached rows, query i at position off + i)
 // and flash_attention_prefill (crates/ferric-llama/src/qwen3.rs:925: "all three are the same math"), with the Gemma-2 score
 // softcap (:59-61). The reference composes it from permutes, two batched matmuls and a masked softmax over a [nh, T, S] score
-// tensor (or a WGSL flash kernel up to its shared-memory limit); here it is one flash-style launch on the matrix cores in f32.
+// tensor (or a WGSL flash kernel up to its shared-memory limit); here it is one flash-style launch on the matrix cores, at f32's grade.
 //
-// Why f32 matrix instructions. v_mfma_f32_16x16x4_f32 multiplies f32 operands exactly and accumulates in f32: results have the
+// Two kernels: causal_attn_cut_kernel, on bf16 matrix instructions with every f32 operand cut into three bf16 values, is what a caller gets;
+// causal_attn_kernel, on f32 matrix instructions, is what fhip_causal_attention_f32_products gives (prompts on a block-quantized cache:
+// the header says why). Measured, us, f32 -> cut, 40 query and 8 KV heads of 128: 509 rows x 809 keys 102.9 -> 71.7, 2048 x 2048 432 ->
+// 266, 512 x 8192 1163 -> 783; few workgroups: 39 x 929, 8 heads 85.7 -> 69.3; heads of 64: 512 x 512, 32 heads 31.7 -> 27.5, 49 x 49 7.0 ->
+// 6.3. Relative error against f64, same shapes: 5.6e-7 -> 4.5e-7, 4.5e-7 -> 3.7e-7, 1.65e-6 -> 1.41e-6, 6.8e-7 -> 5.6e-7, 2.7e-7 -> 2.0e-7,
+// 1.7e-7 -> 1.2e-7. What bounds the cut kernel: the chain of a tile (cut and store 32 keys, products, statistics, products: 2.2 us a wave
+// alone on its SIMD, of which 0.65 are MFMA) at one or two waves a SIMD.
+//
+// Why f32 matrix instructions (the second kernel, and the first one's tiling). v_mfma_f32_16x16x4_f32 multiplies f32 operands exactly and accumulates in f32: results have the
 // grade of the reference's f32 arithmetic (the tests hold them to 1e-5 of the largest output against an f64 evaluation), where
 // bf16 operands would leave three digits. It runs at the chip's f32 matrix rate (157 TFLOP/s), a sixteenth of bf16's.
 //
@@ -207,13 +215,217 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
     }
 }
 
+// ------------------------------------------------------------------------------------------------------------------------------
+// The same on bf16 matrix instructions. An f32 value is three bf16 values exactly (the nearest to it, the nearest to what is left, and
+// what is left then), and a product of two f32 values is, to 2^-25, the six products of their cuts of which one factor at least is the
+// first or both the second: six v_mfma_f32_16x16x32_bf16 of 16 cycles for 32 columns of k, where v_mfma_f32_16x16x4_f32 needs eight of 32.
+// Every operand keeps its 24 bits, sums are f32.
+//
+// Tiles, masks and statistics are the f32 kernel's: a wave owns 16 query rows of one head, lane (c, ks), key tiles of 32 rows. K and V are
+// cut once a tile by the workgroup as they go to LDS, K as [plane][key][dim], V as [plane][dim][slot]: slot 8 ks + 4 u + i is key
+// 16 u + 4 ks + i, the key whose probability register i of S^T_u holds in lane group ks, so the second product takes the probabilities
+// from their registers and a lane's A operand, eight slots of one dim, is one 16-byte read. K rows are padded by 16 bytes and V rows
+// (64 bytes) too: 16 lanes then cover the 64 banks once, in the reads and in the 8-byte writes of four keys x four dims a thread.
+// ------------------------------------------------------------------------------------------------------------------------------
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// two values into their three cuts, packed in pairs
+struct Cuts2 { uint32_t w[3]; };
+__device__ __forceinline__ Cuts2 cut2(float a, float b) {
+    Cuts2 r;
+    r.w[0] = pk_bf16(a, b);
+    a -= __uint_as_float(r.w[0] << 16);
+    b -= __uint_as_float(r.w[0] & 0xFFFF0000u);
+    r.w[1] = pk_bf16(a, b);
+    a -= __uint_as_float(r.w[1] << 16);
+    b -= __uint_as_float(r.w[1] & 0xFFFF0000u);
+    r.w[2] = pk_bf16(a, b);
+    return r;
+}
+// N accumulators' six products, the smallest first; the accumulators take turns, so that none waits for its last product
+template <int N>
+__device__ __forceinline__ void mfma_cuts(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3], f32x4* acc) {
+    constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int x = 0; x < 6; x++)
+#pragma unroll
+        for (int n = 0; n < N; n++) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n][A[x]], b[B[x]], acc[n], 0, 0, 0);
+}
+
+template <int HD, int NW, typename Out>
+__global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
+                                                                     int S, int n_head, int n_kv, float scale, int window, float softcap,
+                                                                     Out* __restrict__ out) {
+    constexpr int KROW = HD + 8;            // bf16 per K row and plane
+    constexpr int VROW = 32 + 8;            // bf16 per V dim and plane
+    constexpr int KP = 32 * KROW, VP = HD * VROW;   // bf16 per plane
+    constexpr int NK = HD / 32;             // k-steps of the first product
+    constexpr int ND = HD / 16;             // output tiles of 16 dims
+    constexpr int UNITS = 8 * (HD / 4);     // blocks of four keys x four dims in a K (or V) tile
+    constexpr int NU = (2 * UNITS + 64 * NW - 1) / (64 * NW);   // of those of K and V together, per thread
+    __shared__ __attribute__((aligned(16))) uint16_t Ks[3 * KP];
+    __shared__ __attribute__((aligned(16))) uint16_t Vs[3 * VP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, ks = lane >> 4;
+    const int head = blockIdx.x, kvh = head / (n_head / n_kv);
+    const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;        // longest first, as in the f32 kernel
+    const int off = S - T;
+    const int wg_first = qb * 16 * NW, wg_last = min(T - 1, wg_first + 16 * NW - 1);
+    const int i0 = wg_first + wave * 16;
+    const bool wave_live = i0 < T;
+    const int i_last = min(i0 + 15, T - 1);
+    const int i = min(i0 + c, T - 1), qpos = off + i;
+    const int kt_hi = (off + wg_last) / 32;
+    const int kt_lo = window > 0 ? max(0, off + wg_first - window + 1) / 32 : 0;
+    const int my_hi = wave_live ? (off + i_last) / 32 : -1;
+    const int my_lo = window > 0 ? max(0, off + i0 - window + 1) / 32 : 0;
+
+    bf16x8 qf[NK][3];                       // query c, dims 32 n + 8 ks + [0, 8)
+    {
+        const float* qp = q + ((size_t)i * n_head + head) * HD + 8 * ks;
+#pragma unroll
+        for (int n = 0; n < NK; n++) {
+            const f32x4 a = *(const f32x4*)(qp + 32 * n), b = *(const f32x4*)(qp + 32 * n + 4);
+            const Cuts2 w0 = cut2(a[0], a[1]), w1 = cut2(a[2], a[3]), w2 = cut2(b[0], b[1]), w3 = cut2(b[2], b[3]);
+#pragma unroll
+            for (int y = 0; y < 3; y++) qf[n][y] = __builtin_bit_cast(bf16x8, (u32x4){w0.w[y], w1.w[y], w2.w[y], w3.w[y]});
+        }
+    }
+    f32x4 oacc[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++) oacc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -3.0e38f, l = 0.f;
+    const size_t kv_stride = (size_t)n_kv * HD;
+
+    // Unit x of a thread: number tid + 64 NW x, K's first (wave-uniform which). Keys 4 g .. 4 g + 3, dims 4 dq .. 4 dq + 3; of K a
+    // wave takes whole rows (dq fastest), of V all eight key groups of eight dims' quads (g fastest).
+    f32x4 piece[NU][4];
+    int dst[NU];                            // of K: bf16 offset of (key 4 g, dim 4 dq); of V: of (dim 4 dq, slot of key 4 g)
+    int key0[NU], dim0[NU];
+#pragma unroll
+    for (int x = 0; x < NU; x++) {
+        const int n = tid + 64 * NW * x, v = n - UNITS;
+        const int g = v < 0 ? n / (HD / 4) : v & 7, dq = v < 0 ? n % (HD / 4) : v >> 3;
+        key0[x] = 4 * g;
+        dim0[x] = 4 * dq;
+        dst[x] = v < 0 ? 4 * g * KROW + 4 * dq : 4 * dq * VROW + 8 * (g & 3) + 4 * (g >> 2);
+    }
+    auto mine = [&](int x) { return 2 * UNITS % (64 * NW) == 0 || wave + NW * x < 2 * UNITS / 64; };
+    auto is_k = [&](int x) { return UNITS % (64 * NW) == 0 ? x < UNITS / (64 * NW) : wave + NW * x < UNITS / 64; };
+    auto load = [&](int kt) {
+#pragma unroll
+        for (int x = 0; x < NU; x++)
+            if (mine(x)) {
+                const float* src = (is_k(x) ? K : V) + (size_t)kvh * HD + dim0[x];
+                // rows past the cache repeat its last row; they are masked below
+#pragma unroll
+                for (int r = 0; r < 4; r++) piece[x][r] = *(const f32x4*)(src + (size_t)min(kt * 32 + key0[x] + r, S - 1) * kv_stride);
+            }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int x = 0; x < NU; x++)
+            if (mine(x)) {
+                if (is_k(x)) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const Cuts2 w0 = cut2(piece[x][r][0], piece[x][r][1]), w1 = cut2(piece[x][r][2], piece[x][r][3]);
+#pragma unroll
+                        for (int y = 0; y < 3; y++) *(uint2*)(Ks + y * KP + dst[x] + r * KROW) = make_uint2(w0.w[y], w1.w[y]);
+                    }
+                } else {
+#pragma unroll
+                    for (int d = 0; d < 4; d++) {
+                        const Cuts2 w0 = cut2(piece[x][0][d], piece[x][1][d]), w1 = cut2(piece[x][2][d], piece[x][3][d]);
+#pragma unroll
+                        for (int y = 0; y < 3; y++) *(uint2*)(Vs + y * VP + dst[x] + d * VROW) = make_uint2(w0.w[y], w1.w[y]);
+                    }
+                }
+            }
+    };
+    load(kt_lo);
+    for (int kt = kt_lo; kt <= kt_hi; kt++) {
+        __syncthreads();                                        // every wave is done with the previous tile
+        store();
+        __syncthreads();
+        load(min(kt + 1, kt_hi));                               // in flight under this tile's arithmetic
+        if (kt < my_lo || kt > my_hi) continue;                 // wave-uniform; the barriers above are reached by every wave
+
+        f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        const uint16_t* krow = Ks + c * KROW + 8 * ks;
+#pragma unroll
+        for (int n = 0; n < NK; n++) {
+            bf16x8 kf[2][3];
+#pragma unroll
+            for (int y = 0; y < 3; y++)
+#pragma unroll
+                for (int u = 0; u < 2; u++) kf[u][y] = *(const bf16x8*)(krow + y * KP + 16 * u * KROW + 32 * n);
+            mfma_cuts(kf, qf[n], sacc);
+        }
+        const bool whole = kt * 32 + 31 <= off + i0 && (window == 0 || off + i_last - kt * 32 < window);
+        float sc[8];                                            // of this lane's query against its 8 keys of the tile
+#pragma unroll
+        for (int x = 0; x < 8; x++) sc[x] = sacc[x >> 2][x & 3] * scale;
+        if (softcap > 0.f) {
+#pragma unroll
+            for (int x = 0; x < 8; x++) sc[x] = softcap * tanhf(sc[x] / softcap);
+        }
+        if (!whole) {
+#pragma unroll
+            for (int x = 0; x < 8; x++) {
+                const int j = kt * 32 + 16 * (x >> 2) + 4 * ks + (x & 3);
+                sc[x] = j <= qpos && (window == 0 || qpos - j < window) ? sc[x] : -INFINITY;   // nn.rs:128-133
+            }
+        }
+        float mt = -3.0e38f;
+#pragma unroll
+        for (int x = 0; x < 8; x++) mt = fmaxf(mt, sc[x]);
+        mt = fmaxf(mt, __shfl_xor(mt, 16));
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        const float m_new = fmaxf(m, mt);
+        const float corr = __expf(m - m_new);
+        float ps = 0.f;
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            sc[x] = __expf(sc[x] - m_new);                      // 0 of a masked key: m_new is finite
+            ps += sc[x];
+        }
+        l = fmaf(l, corr, ps);
+        m = m_new;
+        const Cuts2 p0 = cut2(sc[0], sc[1]), p1 = cut2(sc[2], sc[3]), p2 = cut2(sc[4], sc[5]), p3 = cut2(sc[6], sc[7]);
+        bf16x8 pf[3];
+#pragma unroll
+        for (int y = 0; y < 3; y++) pf[y] = __builtin_bit_cast(bf16x8, (u32x4){p0.w[y], p1.w[y], p2.w[y], p3.w[y]});
+#pragma unroll
+        for (int d = 0; d < ND; d++) oacc[d] *= corr;
+        const uint16_t* vrow = Vs + c * VROW + 8 * ks;
+#pragma unroll
+        for (int d = 0; d < ND; d += 2) {
+            bf16x8 vf[2][3];
+#pragma unroll
+            for (int y = 0; y < 3; y++)
+#pragma unroll
+                for (int e = 0; e < 2; e++) vf[e][y] = *(const bf16x8*)(vrow + y * VP + (16 * d + 16 * e) * VROW);
+            mfma_cuts(vf, pf, oacc + d);
+        }
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (!wave_live || i0 + c >= T) return;
+    const float inv = 1.0f / l;
+    Out* op = out + ((size_t)i * n_head + head) * HD + 4 * ks;   // register r of output tile d is dim 16 d + 4 ks + r
+#pragma unroll
+    for (int d = 0; d < ND; d++) store_out(op + 16 * d, float4{oacc[d][0] * inv, oacc[d][1] * inv, oacc[d][2] * inv, oacc[d][3] * inv});
+}
+
 }  // namespace
 
 namespace fhip {
 
 template <typename Out>
 static int launch_causal_out(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                             float softcap, Out* out, hipStream_t st) {
+                             float softcap, bool cuts, Out* out, hipStream_t st) {
     if (t == 0 || n_head == 0 || hd == 0) return FHIP_OK;
     if (s < t) return set_error(FHIP_ERR_SHAPE, "cache (%zu) cannot be shorter than the query block (%zu)", s, t);   // nn.rs:73, :249
     if (n_kv <= 0 || n_head % n_kv != 0) return set_error(FHIP_ERR_SHAPE, "causal_attention: n_heads must be a multiple of n_kv_heads");
@@ -228,20 +440,24 @@ static int launch_causal_out(const float* q, const float* K, const float* V, siz
     const dim3 grid((unsigned)n_head, (unsigned)qblocks), wg(64 * nw);
     const float scale = 1.0f / sqrtf((float)hd);
     const int win = window == 0 || window >= s ? 0 : (int)window;     // a window that covers the cache is no window
-    if (hd == 128 && nw == 8) hipLaunchKernelGGL((causal_attn_kernel<128, 8, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else if (hd == 128) hipLaunchKernelGGL((causal_attn_kernel<128, 4, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else if (nw == 8) hipLaunchKernelGGL((causal_attn_kernel<64, 8, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
-    else hipLaunchKernelGGL((causal_attn_kernel<64, 4, Out>), grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out); };
+    if (cuts) {
+        if (hd == 128) nw == 8 ? go(causal_attn_cut_kernel<128, 8, Out>) : go(causal_attn_cut_kernel<128, 4, Out>);
+        else nw == 8 ? go(causal_attn_cut_kernel<64, 8, Out>) : go(causal_attn_cut_kernel<64, 4, Out>);
+    } else {
+        if (hd == 128) nw == 8 ? go(causal_attn_kernel<128, 8, Out>) : go(causal_attn_kernel<128, 4, Out>);
+        else nw == 8 ? go(causal_attn_kernel<64, 8, Out>) : go(causal_attn_kernel<64, 4, Out>);
+    }
     return check_hip(hipGetLastError(), "causal_attention launch");
 }
 
 int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                            float softcap, float* out, hipStream_t st) {
-    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, out, st);
+                            float softcap, bool cuts, float* out, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, st);
 }
 int launch_causal_attention_bf16(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                                 float softcap, uint16_t* out, hipStream_t st) {
-    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, out, st);
+                                 float softcap, bool cuts, uint16_t* out, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, st);
 }
 
 }  // namespace fhip

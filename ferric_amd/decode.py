@@ -434,8 +434,12 @@ class Qwen3Decoder:
                     _check(lib.fhip_kvq_dequantize_rows(self.kv_fmt, cache.codes.ptr, cache.scales.ptr, 0, pos0 + t, self.kv_out, None,
                                                         dst.buf.ptr, s))
                 kp, vp = kd.buf.ptr, vd.buf.ptr
-            attend = lib.fhip_causal_attention if att.dtype == np.float32 else lib.fhip_causal_attention_bf16
-            _check(attend(q.buf.ptr, kp, vp, t, pos0 + t, c.n_head, c.n_head_kv, c.head_dim, l.window, c.attn_softcap, att.buf.ptr, s))
+            shape = (q.buf.ptr, kp, vp, t, pos0 + t, c.n_head, c.n_head_kv, c.head_dim, l.window, c.attn_softcap)
+            if self.kv_fmt is not None:           # the codes of later layers follow every last bit of this one's rows
+                _check(lib.fhip_causal_attention_f32_products(*shape, int(att.dtype != np.float32), att.buf.ptr, s))
+            else:
+                attend = lib.fhip_causal_attention if att.dtype == np.float32 else lib.fhip_causal_attention_bf16
+                _check(attend(*shape, att.buf.ptr, s))
             if l.attn_gate is not None:
                 matmul(l.attn_gate, h, gate)
                 _check(lib.fhip_mul_sigmoid(att.buf.ptr, gate.buf.ptr, t * self.q_out, att.buf.ptr, s))

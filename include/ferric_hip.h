@@ -361,6 +361,11 @@ int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, 
 /* The same with the output rows as bf16, each value the one fhip_cvt_f32_bf16 makes of the f32 result. */
 int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
                                size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream);
+/* The same result from the f32 matrix instructions (d_out f32, or bf16 with out_bf16): slower, no less exact, other last bits. For
+ * stacks on a block-quantized cache, where behind bf16 roundings a last bit decides code bytes of the layers after it, and a block's
+ * codes should not depend on the library's version. */
+int fhip_causal_attention_f32_products(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
+                                       size_t head_dim, size_t window, float softcap, int out_bf16, void* d_out, void* stream);
 
 /* fhip_qkv_post with the key and value heads written to packed outputs [t, n_kv * head_dim] (row i for token i) instead of
  * cache rows: for callers that store them themselves, as the quantized arm of qwen3.rs:906-912 does. */

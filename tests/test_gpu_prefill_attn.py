@@ -1,4 +1,4 @@
-"""fhip_causal_attention (prefill / chunked prefill / windowed / softcapped causal attention on the f32 matrix instructions)
+"""fhip_causal_attention (prefill / chunked prefill / windowed / softcapped causal attention on the matrix instructions)
 through the C ABI against the f64 oracle. Floating point: the bar is 1e-5 of the largest expected output, the bar of the
 single-query attention tests; a row that sees one key only must return that key's value row exactly."""
 import numpy as np
@@ -89,3 +89,34 @@ def test_argument_checks(F, X):
     assert b"head_dim must be 64 or 128" in lib.fhip_last_error()
     assert lib.fhip_causal_attention(None, a.buf.ptr, a.buf.ptr, 4, 4, 4, 4, 64, 0, 0.0, a.buf.ptr, None) != 0
     assert lib.fhip_causal_attention(None, None, None, 0, 0, 4, 4, 64, 0, 0.0, None, None) == 0       # nothing to do
+
+
+@pytest.mark.parametrize("t,s,nh,nkv,hd,w,cap,vscale", [(1, 1, 2, 1, 64, 0, 0.0, 1.0), (33, 70, 10, 2, 128, 0, 0.0, 1e30), (130, 130, 4, 4, 64, 17, 0.0, 1e-30),
+                                                        (65, 300, 5, 1, 128, 0, 30.0, 1.0), (1100, 1100, 64, 8, 64, 0, 0.0, 1.0)])
+def test_f32_products_beside_the_cut_ones(F, X, D, t, s, nh, nkv, hd, w, cap, vscale):
+    # both kernels at the bar of this file, f32 and bf16 rows of the f32 one, and the two beside each other: each is within a few f32
+    # roundings of sums of s terms (4e-6 of the largest output: sums of up to 1100 terms, 2e-6 each at the most). Values far from 1 keep their 24 bits in three cuts; 1100 rows of 64 heads take
+    # the workgroups of eight waves.
+    rng = np.random.default_rng(t + s)
+    q = rng.standard_normal((t, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((s, nkv * hd)).astype(np.float32)
+    v = (rng.standard_normal((s, nkv * hd)) * vscale).astype(np.float32)
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    tq, tk, tv = T(q), T(k), T(v)
+    cut = X.causal_attention(tq, tk, tv, nh, nkv, w, cap).to_vec().reshape(t, nh * hd)
+    lib = F._lib.load()
+    out, half = T(np.zeros((t, nh * hd), np.float32)), T(np.zeros((t, nh * hd), np.float32))
+    args = (tq.buf.ptr, tk.buf.ptr, tv.buf.ptr, t, s, nh, nkv, hd, w, cap)
+    assert lib.fhip_causal_attention_f32_products(*args, 0, out.buf.ptr, None) == 0
+    assert lib.fhip_causal_attention_f32_products(*args, 1, half.buf.ptr, None) == 0
+    f32 = out.to_vec().reshape(t, nh * hd)
+    top = np.abs(f32).max()
+    assert np.abs(cut - f32).max() <= 4e-6 * top
+    if t <= 130:
+        want = D.causal_attention(q, k, v, nh, nkv, w, cap)
+        for got in (cut, f32):
+            assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+    b = f32.view(np.uint32).astype(np.uint64)
+    rounded = ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint16)
+    assert np.array_equal(half.to_vec().view(np.uint16).reshape(-1)[:t * nh * hd], rounded.reshape(-1))
+    assert lib.fhip_causal_attention_f32_products(*args[:3], s + 1, s, *args[5:], 0, out.buf.ptr, None) != 0
