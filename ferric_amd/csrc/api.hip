@@ -1222,6 +1222,13 @@ int fhip_matmul_q_id_wsum(const fhip_weight* w, const float* d_x, size_t t, cons
     if (!d_x || !d_selw || !d_y || !d_ws) return set_error(FHIP_ERR_ARG, "fhip_matmul_q_id_wsum: NULL pointer");
     if (((uintptr_t)d_x & 15) != 0 || (w->cols * 4) % 16 != 0) return set_error(FHIP_ERR_ARG, "fhip_matmul_q_id_wsum: x rows must be 16-byte aligned");
     sel.selw = d_selw; sel.x_per_pair = 1; sel.y_stride = out_pe; sel.npairs = (int)(t * k);
+    // one launch where the kernel covers the rows; it reads the inputs until its end, so an output laid over one of them takes the two launches,
+    // of which only the second writes it
+    auto apart = [&](const float* in, size_t n) { return d_y + t * out_pe <= in || in + n <= d_y; };
+    if (apart(d_x, t * k * w->cols) && apart(d_selw, t * 2 * k) && out_pe > 0 &&
+        (w->planes == 3 ? fhip::launch_gemv_wsum_p3(w, d_x, d_y, out_pe, sel, (hipStream_t)stream, &rc)
+                        : fhip::launch_gemv_wsum_p2(w, d_x, d_y, out_pe, sel, (hipStream_t)stream, &rc)))
+        return rc;
     if ((rc = fhip::launch_gemv_sel(w, d_x, d_ws, out_pe, false, sel, (hipStream_t)stream))) return rc;
     return fhip::launch_moe_wsum(d_ws, d_selw, t, (int)k, out_pe, d_y, (hipStream_t)stream);
 }

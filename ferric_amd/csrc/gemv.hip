@@ -1154,6 +1154,186 @@ __global__ void __launch_bounds__(max_threads<F>(M)) gemv_stream_kernel(GemvPara
         }
 }
 
+// The down projection of routed experts with its weighted sum inside (fhip_matmul_q_id_wsum):
+//   y[t, o] = sum_s selw[t, s] * (W[e(t, s)][o, :] . x[t k + s, :]),   slots added in order.
+// The pairs' launch left [t k, out_pe] products in memory for a launch of its own to add, 4 us of 16 at four tokens of 8 x (2048 x 768). Here a
+// workgroup owns `rows` outputs of one token and all its k slots: waves s wps .. s wps + wps - 1 work on slot s as the streaming
+// kernel's tail waves do (RT = 4 / NG rows at once, U steps in flight), the partial sums meet in LDS and are added slot by slot in the order and with
+// the arithmetic of the two launches, so the bits are theirs. Both launches -> this one, us: Q6_K 2048 x 768, 8 slots, 1 / 2 / 4 / 8 tokens 10.2 / 10.8 /
+// 13.7 / 21.5 -> 6.4 / 8.2 / 10.7 / 17.1; Q8_0 1024 x 1536, 6 slots, 4 tokens 13.8 -> 10.6; Q4_K 4096 x 2048, 2 slots, 1 token 9.8 -> 6.4 (a launch's
+// fixed 5 us and the bytes; the large ones reach 3.8 TB/s of expert bytes).
+struct WsumParams {
+    const uint8_t* W;
+    const float* x;      // [t k, cols]
+    const float* selw;   // [t, 2 k]: weights, then experts
+    float* y;            // [t, out_rows]
+    int out_rows, cols;
+    uint32_t row_bytes;
+    int NG, units, k, n_expert;
+    size_t expert_rows;
+    int wps;             // waves per slot
+    int rows;            // outputs per workgroup
+};
+
+template <class F, int U>
+__global__ void __launch_bounds__(1024) gemv_wsum_kernel(WsumParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    constexpr int RUN = F::RUN, NRUN = F::NRUN, RD = RUN / 4, RC = RD / 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ti = blockIdx.y, s = wave / p.wps, q = wave - s * p.wps;
+    const float* selw = p.selw + (size_t)ti * 2 * p.k;
+    const float* x = p.x + ((size_t)ti * p.k + s) * p.cols;
+    // the slot's activations, pieces q, q + wps, ... of 512: the first two asked for at once
+    const int e0 = (q * 64 + lane) * 8, e_step = p.wps * 512;
+    const float* x0 = x + (e0 < p.cols ? e0 : 0);
+    const float* x1 = x + (e0 + e_step < p.cols ? e0 + e_step : 0);
+    const float4 xa0 = *(const float4*)x0, xb0 = *(const float4*)(x0 + 4), xa1 = *(const float4*)x1, xb1 = *(const float4*)(x1 + 4);
+    int e = (int)selw[p.k + s];
+    e = e < 0 ? 0 : (e >= p.n_expert ? p.n_expert - 1 : e);   // a corrupt index must not leave the slab
+    e = __builtin_amdgcn_readfirstlane(e);
+    const int row0 = blockIdx.x * p.rows;
+    const int nrows = min(p.rows, p.out_rows - row0);
+    const uint8_t* base = p.W + ((size_t)e * p.expert_rows + (size_t)row0) * p.row_bytes;
+
+    // lane -> slot of the row and row of the step; a lane past the row's last unit works on unit 0 and contributes 0
+    const int slot = lane >> 4, l16 = lane & 15;
+    const int rt_log2 = p.NG == 1 ? 2 : p.NG == 2 ? 1 : 0, RT = 1 << rt_log2;
+    const int group = p.NG == 1 ? 0 : p.NG == 2 ? (slot & 1) : (slot < p.NG ? slot : 0);
+    const int row_off = p.NG == 1 ? slot : p.NG == 2 ? (slot >> 1) : 0;
+    const bool lane_ok = p.NG < 3 || slot < p.NG;
+    typename F::Lane L;
+    int run[NRUN];
+    const bool unit_ok = group * 16 + l16 < p.units;
+    const int my_unit = unit_ok ? group * 16 + l16 : 0;
+    F::setup(my_unit, L, run);
+    const uint32_t lane_extra = (uint32_t)row_off * p.row_bytes;
+
+    // step `it` of this wave: rows v(it) + row_off of the workgroup's; the last step may hold fewer than RT
+    auto v_of = [&](int it) { return (it * p.wps + q) << rt_log2; };
+    const int left = nrows - (q << rt_log2), stride = p.wps << rt_log2;
+    const int n_it = left > 0 ? (left + stride - 1) / stride : 0;
+    auto row_base = [&](int it) -> const uint8_t* { return base + (size_t)(uint32_t)v_of(it) * p.row_bytes; };
+    auto lane_eo = [&](int it) { return v_of(it) + row_off < nrows ? lane_extra : 0u; };
+    typename F::Data buf[U];
+    // a wave without rows asks for the workgroup's first row and drops it
+    buf[0] = F::load(n_it > 0 ? row_base(0) : base, L, n_it > 0 ? lane_eo(0) : 0u);
+    asm volatile("" ::: "memory");
+
+    const int nrun = p.cols / RUN;
+    uint8_t* planes = smem + (size_t)s * p.cols * NP;           // planes of every slot | scales, sums of every slot | partial sums
+    float* scales = (float*)(smem + (size_t)p.k * p.cols * NP) + (size_t)s * 2 * nrun;
+    float* sums = scales + nrun;
+    float* part = (float*)(smem + (size_t)p.k * p.cols * NP) + (size_t)p.k * 2 * nrun;   // [k][rows][NG]
+    auto stage = [&](int e8, const float4& a, const float4& b) {
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        uint32_t pl[NP][2];
+        float scale, qsum;
+        quantize8<RUN>(v, pl, scale, qsum);
+        const int within = e8 % RUN;
+        int u, j;
+        F::owner(e8 / RUN, u, j);
+#pragma unroll
+        for (int pp = 0; pp < NP; pp++)
+            *(u32x2*)(planes + ((size_t)((j * NP + pp) * RC + (within >> 4)) * p.units + u) * 16 + (within & 15)) = u32x2{pl[pp][0], pl[pp][1]};
+        if (within == 0) { scales[j * p.units + u] = scale; sums[j * p.units + u] = qsum; }
+    };
+    if (e0 < p.cols) stage(e0, xa0, xb0);
+    if (e0 + e_step < p.cols) stage(e0 + e_step, xa1, xb1);
+    for (int e8 = e0 + 2 * e_step; e8 < p.cols; e8 += e_step) stage(e8, *(const float4*)(x + e8), *(const float4*)(x + e8 + 4));
+#pragma unroll
+    for (int j = 1; j < U; j++)
+        if (j < n_it) buf[j] = F::load(row_base(j), L, lane_eo(j));
+    __syncthreads();
+
+    uint32_t xp[1][NRUN][NP][RD];
+    float xs[1][NRUN], xq[1][NRUN];
+    bool special = false;
+#pragma unroll
+    for (int j = 0; j < NRUN; j++) {
+        xs[0][j] = scales[j * p.units + my_unit];
+        xq[0][j] = sums[j * p.units + my_unit];
+        special = special || xs[0][j] != xs[0][j];
+#pragma unroll
+        for (int pp = 0; pp < NP; pp++)
+#pragma unroll
+            for (int i = 0; i < RD; i += 4) {
+                const u32x4 t = *(const u32x4*)(planes + ((size_t)((j * NP + pp) * RC + (i >> 2)) * p.units + my_unit) * 16);
+                xp[0][j][pp][i] = t[0]; xp[0][j][pp][i + 1] = t[1]; xp[0][j][pp][i + 2] = t[2]; xp[0][j][pp][i + 3] = t[3];
+            }
+    }
+    special = special && unit_ok;
+
+    float* mypart = part + (size_t)s * p.rows * p.NG;
+    const bool bit0 = (lane & 1) != 0, bit1 = (lane & 2) != 0;
+    const int my_j = slot_of<U>(l16);
+    const bool store_lane = lane_ok && l16 < (U == 1 ? 1 : 4) && my_j < U && (U != 2 || (l16 & 1) == 0);
+    const bool contributes = unit_ok && !special;
+    auto consume = [&](typename F::Data& cur, float& out) {
+        cur.pin_all();
+        float acc[1];
+        F::template dot<1>(cur, L, xp, xs, xq, acc);
+        out = contributes ? acc[0] : 0.f;
+    };
+    auto store_step = [&](const float (&outs)[U], int it0) {
+        const float t = slot_sum_many<U>(outs, bit0, bit1);
+        const int v = v_of(it0 + my_j) + row_off;
+        if (store_lane && it0 + my_j < n_it && v < nrows) mypart[(size_t)v * p.NG + group] = t;
+    };
+    __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0): a clean state at the loop head, as in the streaming kernel
+    int i0 = 0;
+    float outs[U];
+#pragma unroll 1
+    for (; i0 + 2 * U <= n_it; i0 += U) {                       // every step of this round and of the next one exists
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            consume(buf[j], outs[j]);
+            buf[j] = F::load(row_base(i0 + j + U), L, lane_eo(i0 + j + U));
+        }
+        store_step(outs, i0);
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {                               // drain: the last round or two, the second perhaps not full
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int it = i0 + r * U + j;
+            outs[j] = 0.f;
+            if (it < n_it) {
+                consume(buf[j], outs[j]);
+                if (r == 0 && it + U < n_it) buf[j] = F::load(row_base(it + U), L, lane_eo(it + U));
+            }
+        }
+        if (i0 + r * U < n_it) store_step(outs, i0 + r * U);
+    }
+    // lanes whose activations block fixed point cannot hold, element by element, as in the streaming kernel
+    if (__builtin_amdgcn_ballot_w64(special) != 0) {
+#pragma unroll 1
+        for (int it = 0; it < n_it; it++) {
+            const uint8_t* rowp = row_base(it) + lane_eo(it);
+            const int v = v_of(it) + row_off;
+            float a = 0.f;
+            if (special) {
+#pragma unroll 1
+                for (int j = 0; j < NRUN; j++)
+#pragma unroll 1
+                    for (int i = 0; i < RUN; i++) a += x[run[j] * RUN + i] * fhip::deq_at<F::TYPE>(rowp, run[j] * RUN + i);
+            }
+            a = slot_sum(a);
+            if (lane_ok && l16 == 0 && v < nrows) mypart[(size_t)v * p.NG + group] += a;
+        }
+    }
+    __syncthreads();
+    for (int r = tid; r < nrows; r += blockDim.x) {
+        float total = 0.f;
+        for (int sl = 0; sl < p.k; sl++) {
+            const float* g = part + ((size_t)sl * p.rows + r) * p.NG;
+            float a = 0.f;
+            for (int n = 0; n < p.NG; n++) a += g[n];
+            total = total + selw[sl] * a;
+        }
+        p.y[(size_t)ti * p.out_rows + row0 + r] = total;
+    }
+}
+
 // Un-fused SwiGLU, crates/ferric-tensor/src/lib.rs:2603-2618: gu [t, 2d] = [gate | up] per row.
 __global__ void swiglu_kernel(const float* __restrict__ gu, size_t n, size_t d, float* __restrict__ out) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1502,6 +1682,50 @@ int GEMV_EXPORT(launch_gemv_sel)(const fhip_weight* w, const float* d_x, float* 
         case FHIP_MXFP4:
             return swiglu ? launch_gemv_generic_sel(w, d_x, d_y, out_rows, swiglu, sel, s) : launch_sel_plain<MXF4S>(w, d_x, d_y, out_rows, sel, s);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "QMatrix: no native matmul for ggml type %u", w->type);
+    }
+}
+
+// Rows of up to four slots (4096 columns, 2048 of the 32-value formats) whose planes for all k slots fit LDS; false: nothing launched,
+// the pairs' launch and the summing one do it.
+template <class F>
+bool launch_wsum_fmt(const fhip_weight* w, const float* d_x, float* d_y, size_t out_rows, const SelParams& sel, hipStream_t st, int* rc) {
+    if (max_batch<F, false>(w, 1) == 0) return false;
+    WsumParams p;
+    p.W = w->d_raw; p.x = d_x; p.selw = sel.selw; p.y = d_y;
+    p.out_rows = (int)out_rows; p.cols = (int)w->cols; p.row_bytes = (uint32_t)w->row_bytes;
+    p.units = (int)(w->cols / F::WPL);
+    p.NG = (p.units + 15) / 16;
+    p.k = sel.k; p.n_expert = sel.n_expert; p.expert_rows = sel.expert_rows;
+    const size_t t = (size_t)sel.npairs / sel.k;
+    if (p.NG > 4 || t > 65535) return false;
+    // outputs per workgroup: one workgroup per CU over the tokens, at most 256 (their partial sums lie in LDS), in whole steps of a wave
+    const size_t cus = device_cus() > 0 ? device_cus() : 256, per_token = cus / t > 0 ? cus / t : 1;
+    const int RT = p.NG == 1 ? 4 : p.NG == 2 ? 2 : 1;
+    size_t rows = (out_rows + per_token - 1) / per_token;
+    rows = rows > 256 ? 256 : (rows + RT - 1) / RT * RT;
+    p.rows = (int)rows;
+    const int steps = p.rows / RT;
+    p.wps = 16 / p.k < steps ? 16 / p.k : steps;
+    const size_t lds = (size_t)p.k * (w->cols * NP + 2 * (w->cols / F::RUN) * sizeof(float) + rows * p.NG * sizeof(float));
+    if (lds > device_lds_bytes()) return false;
+    void (*kernel)(WsumParams) = gemv_wsum_kernel<F, F::U1>;
+    static bool lds_raised = false;
+    if (!lds_raised) {
+        (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)device_lds_bytes());
+        (void)hipGetLastError();
+        lds_raised = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((out_rows + rows - 1) / rows), (unsigned)t), dim3(64 * p.wps * p.k), lds, st, p);
+    *rc = check_hip(hipGetLastError(), "matmul_q_id_wsum launch");
+    return true;
+}
+
+bool GEMV_EXPORT(launch_gemv_wsum)(const fhip_weight* w, const float* d_x, float* d_y, size_t out_rows, const SelParams& sel, hipStream_t s, int* rc) {
+    switch (w->type) {
+        case FHIP_Q4_K: return launch_wsum_fmt<Q4K>(w, d_x, d_y, out_rows, sel, s, rc);
+        case FHIP_Q6_K: return launch_wsum_fmt<Q6K>(w, d_x, d_y, out_rows, sel, s, rc);
+        case FHIP_Q8_0: return launch_wsum_fmt<Q80>(w, d_x, d_y, out_rows, sel, s, rc);
+        default: return false;
     }
 }
 

@@ -112,7 +112,8 @@ __global__ void __launch_bounds__(64) moe_topk_kernel(const float* __restrict__ 
     }
 }
 
-// out[ti, o] = sum_s selw[ti, s] * parts[ti*k + s, o], slots added in order (dtype.rs:2555-2567)
+// out[ti, o] = sum_s selw[ti, s] * parts[ti*k + s, o], slots added in order (dtype.rs:2555-2567); where gemv.hip's gemv_wsum_kernel does not
+// cover the rows (launch_wsum_fmt)
 __global__ void __launch_bounds__(256) moe_wsum_kernel(const float* __restrict__ parts, const float* __restrict__ selw, size_t n, int k,
                                                         size_t out_pe, float* __restrict__ y) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -149,6 +149,32 @@ def test_id_wsum(F, O, ty, name, cols):
     assert np.array_equal(one.view(np.uint32), got[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("ty,cols,t,k,out_pe,bits16", [(Q6_K, 768, 4, 8, 2048, False), (Q4_K, 2048, 1, 6, 999, False), (Q4_K, 2304, 3, 1, 37, True), (Q6_K, 4096, 2, 3, 130, False),
+                                                       (Q8_0, 96, 5, 7, 4099, True), (Q8_0, 1152, 2, 4, 1, False), (Q8_0, 2048, 1, 8, 515, False), (Q6_K, 4352, 2, 2, 64, False),
+                                                       (Q8_0, 512, 300, 2, 300, False)])
+def test_id_wsum_in_one_launch_gives_the_bits_of_two(F, ty, cols, t, k, out_pe, bits16):
+    # An output laid over the activations takes the pairs' launch and the summing one: same bits as the one launch. One to four slots of a row, partly
+    # filled ones, rows and workgroups that end inside a step, more rows than a workgroup holds, more tokens than CUs; 4352 columns go to the two launches
+    # either way. One activation is infinite and one run too large for fixed point (element by element).
+    rng = np.random.default_rng(cols + t)
+    n_expert = 9
+    raw, w = slab(F, ty, n_expert, out_pe, cols, 7)
+    if bits16:
+        w.matvec_precision(16)
+    x = rng.standard_normal((t, k, cols)).astype(np.float32)
+    x[0, 0, 5] = np.inf
+    x[t - 1, k - 1, cols - 3] = 3e30
+    sel = selection(rng, t, k, n_expert)
+    st = F.Tensor.from_vec(sel.reshape(-1), (t, 2 * k))
+    one = F.Tensor.from_vec(x.reshape(-1), (t, k, cols)).matmul_q_id_wsum(w, st, out_pe).to_vec()
+    n = max(x.size, t * out_pe)
+    both = F.Tensor.from_vec(np.concatenate([x.reshape(-1), np.zeros(n - x.size, np.float32)]), (n,))
+    ws = F.Tensor.empty((t * k * out_pe,))
+    assert F._lib.load().fhip_matmul_q_id_wsum(w.handle, both.buf.ptr, t, st.buf.ptr, k, out_pe, both.buf.ptr, ws.buf.ptr, None) == 0
+    two = both.to_vec()[:t * out_pe]
+    assert np.array_equal(one.view(np.uint32).reshape(-1), two.view(np.uint32))
+
+
 def test_indices_outside_the_slab_are_clamped_and_shapes_are_checked(F, O):
     rng = np.random.default_rng(24)
     cols, out_pe, n_expert, k = 256, 32, 3, 2
