@@ -1071,6 +1071,25 @@ int fhip_qkv_post_attention(const float* d_qkv, const float* d_bias, const float
                                            (hipStream_t)stream);
 }
 
+int fhip_qkv_post_attention_kvq(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_pos,
+                                const float* d_freq_scale, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                                float base, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap, size_t len,
+                                size_t window, float softcap, float* d_ws, float* d_out, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if ((rc = kvq_checks("fhip_qkv_post_attention_kvq", fmt, n_kv * head_dim)) || (rc = rope_checks("fhip_qkv_post_attention_kvq", n_head + 2 * n_kv, head_dim, n_rot)))
+        return rc;
+    if (n_head == 0 || head_dim == 0) return FHIP_OK;
+    if (!d_qkv || !d_pos || !d_k_codes || !d_k_scales || !d_v_codes || !d_v_scales || !d_out)
+        return set_error(FHIP_ERR_ARG, "fhip_qkv_post_attention_kvq: NULL pointer");
+    if (n_head > 0x7FFFFFFFull || n_kv > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_attention_kvq: too many heads");
+    if (cap > 0xFFFFFFFFull) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_attention_kvq: capacity exceeds 2^32 rows");
+    if (!(softcap >= 0.f)) return set_error(FHIP_ERR_ARG, "fhip_qkv_post_attention_kvq: softcap must be >= 0");
+    return fhip::launch_qkv_post_attention_kvq(fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_pos, d_freq_scale, (int)n_head, (int)n_kv, (int)head_dim, (int)n_rot, interleaved != 0,
+                                               eps, base, d_k_codes, (uint16_t*)d_k_scales, d_v_codes, (uint16_t*)d_v_scales, cap, len, window, softcap, d_ws, d_out,
+                                               (hipStream_t)stream);
+}
+
 int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
                        float* d_h_scratch, int swiglu, float* d_y, void* stream) {
     int rc = need_init();

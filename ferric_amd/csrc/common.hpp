@@ -171,6 +171,9 @@ int launch_kvq_append(int fmt, const float* src, size_t src_row_stride, size_t t
 int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes, const uint16_t* k_scales, const uint32_t* v_codes,
                                 const uint16_t* v_scales, int n_head, int n_kv, int hd, size_t len, const uint32_t* d_len, size_t window,
                                 float softcap, float* ws, float* out, hipStream_t s);
+int launch_qkv_post_attention_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos, const float* freq_scale,
+                                  int n_head, int n_kv, int hd, int n_rot, bool interleaved, float eps, float base, uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes,
+                                  uint16_t* v_scales, size_t cap, size_t len, size_t window, float softcap, float* ws, float* out, hipStream_t s);
 int launch_kvq_dequantize(int fmt, const uint32_t* codes, const uint16_t* scales, size_t row0, size_t rows, size_t width, const uint32_t* d_last_pos,
                           float* out, hipStream_t s);
 int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,

@@ -10,6 +10,8 @@
 // All of this is f32 arithmetic on small vectors: the kernels are launch- and latency-bound (a decode step has one row),
 // except attention, which streams the layer's K and V rows once (HBM-bound: 2 * len * n_kv * head_dim * 4 bytes).
 #include "common.hpp"
+
+#include <type_traits>
 #include "prompt.hpp"
 
 #include <hip/hip_fp16.h>
@@ -463,7 +465,6 @@ __global__ void kv_append_kernel(const float* __restrict__ k, const float* __res
 // row with 4 DPP adds. The 4 streams of a wave are merged by lane exchange, the 4 waves through LDS, the splits by
 // attn_combine_kernel: always the same rescale, exp(m_part - m_all).
 constexpr int ATT_KB = 2;         // keys in flight per stream
-constexpr int ATT_STREAMS = 16;   // per workgroup of 256 threads
 
 __device__ __forceinline__ float row16_sum(float v) {   // all 16 lanes of a DPP row get the row's sum
     v = dpp_add<0xB1, 0xF>(v);
@@ -547,25 +548,71 @@ __device__ __forceinline__ void expand_dims_q(const RawDims<FMT, DPL>& raw, int 
     }
 }
 
+// One head of the newest token's raw QKV row as a wave takes it through qkv_post_kernel's arithmetic: the values (+ bias) and the norm's
+// weights in one trip to memory, lane + 64 i each ...
+template <int HD>
+struct PostHead {
+    float x[HD / 64], w[HD / 64];
+};
+template <int HD>
+__device__ __forceinline__ PostHead<HD> post_request(const QkvPostParams& fp, int src, const float* nw, int lane) {
+    PostHead<HD> p;
+    const float* x = fp.qkv + (size_t)src * HD;
+    const float* bias = fp.bias ? fp.bias + (size_t)src * HD : nullptr;
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++) {
+        p.x[i] = bias ? x[lane + 64 * i] + bias[lane + 64 * i] : x[lane + 64 * i];
+        p.w[i] = nw ? nw[lane + 64 * i] : 1.f;
+    }
+    return p;
+}
+// ... then normed (through `row`, the wave's own HD floats of LDS) and rotated by the lane's pair's angle into dst, LDS or memory.
+template <int HD>
+__device__ __forceinline__ void post_rotate(const QkvPostParams& fp, const PostHead<HD>& p, bool norm, float cs, float sn, int lane, float* row, float* dst) {
+    static_assert(HD <= 128, "a lane rotates one pair");
+    float inv = 1.f;
+    if (norm) {
+        float ms = 0.f;
+#pragma unroll
+        for (int i = 0; i < HD / 64; i++) ms = fmaf(p.x[i], p.x[i], ms);
+        ms = wave_sum(ms);
+        inv = 1.0f / sqrtf(ms / (float)HD + fp.eps);
+    }
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++) row[lane + 64 * i] = norm ? p.x[i] * inv * p.w[i] : p.x[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");      // the wave's own row: its accesses complete in order
+    const int half = fp.n_rot / 2;
+    if (lane < half) {
+        const int p0 = fp.interleaved ? 2 * lane : lane, p1 = fp.interleaved ? 2 * lane + 1 : lane + half;
+        const float x1 = row[p0], x2 = row[p1];
+        dst[p0] = rot_lo(x1, x2, cs, sn);
+        dst[p1] = rot_hi(x1, x2, cs, sn);
+    }
+    for (int e = fp.n_rot + lane; e < HD; e += 64) dst[e] = row[e];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // FUSED: the query heads do not come from memory but are formed here from the raw QKV row of the newest token -- bias, per-head
 // RMSNorm, rotation, exactly qkv_post_kernel's arithmetic -- by every workgroup for its own G heads, into LDS; and the
 // workgroup whose key range holds the token's position also forms that token's K and V rows for its KV head and appends them
 // to the cache before it starts on the keys (a store, a workgroup barrier, then the ordinary loop reads the row back like any
-// other: no other workgroup's range holds that row). One launch less per layer than post-processing + attention.
+// other: no other workgroup's range holds that row). One launch less per layer than post-processing + attention. On a quantized cache (QF) the
+// two rows go through LDS and quantize_lanes: 8.7 -> 5.8 us at 64 rows, 12.7 -> 9.9 at 1000, 24.7 -> 21.3 at 20000 (40 query and 8 KV heads of 128, Q8_0).
 template <bool FUSED> struct CachePtr { typedef const float* __restrict__ type; };
 template <> struct CachePtr<true> { typedef const float* type; };   // the fused kernel also writes the cache: no promise of no alias
 
 // QF: -1 for an f32 cache (K, V), else the FHIP_KVQ_* format of the block-quantized cache in qc (K and V are null then).
-template <int G, int DPL, bool FUSED, int QF = -1>
+// WV: waves of the workgroup. KvqStore (FUSED on a quantized cache): the cache of qc, to append to.
+template <int G, int DPL, bool FUSED, int QF = -1, int WV = 4>
 __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typename CachePtr<FUSED>::type K, typename CachePtr<FUSED>::type V,
                                                 int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev, float scale, int splits,
                                                 uint32_t window, float softcap, float* __restrict__ part, float* __restrict__ out,
-                                                const QkvPostParams& fp, int gq, const QCache& qc = QCache{}) {
-    static_assert(!(FUSED && QF >= 0), "the fused post-processing appends f32 rows");
-    constexpr int HD = 16 * DPL;
-    __shared__ float sm_m[4][G], sm_l[4][G];
-    __shared__ float sm_acc[4][G][HD];
+                                                const QkvPostParams& fp, int gq, const QCache& qc = QCache{}, const KvqStore& qst = KvqStore{}) {
+    constexpr int HD = 16 * DPL, ATT_STREAMS = 4 * WV;
+    __shared__ float sm_m[WV][G], sm_l[WV][G];
+    __shared__ float sm_acc[WV][G][HD];
     __shared__ float sm_q[FUSED ? G : 1][FUSED ? HD : 1];
+    __shared__ float sm_row[FUSED ? WV : 1][FUSED ? HD : 1], sm_kv[FUSED && QF >= 0 ? 2 : 1][FUSED && QF >= 0 ? HD : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane & 15;
     const int sid = wave * 4 + (lane >> 4);
     // Workgroup blockIdx.x takes the G query heads from head0 on; gq = query heads per KV head. gq == G: one workgroup per KV
@@ -583,20 +630,18 @@ __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typ
     // FUSED: the raw values of every head this wave will post-process (job j = wave + 4 r: query head j of the group, then
     // the key and the value row) are requested before anything else, the length word with them, so that one memory round
     // trip covers what used to be three in a row (the length, the first round's rows, the second round's).
-    constexpr int ROUNDS = FUSED ? (G + 2 + 3) / 4 : 1, EPL = HD / 64;
-    float xr[ROUNDS][EPL];
+    constexpr int ROUNDS = FUSED ? (G + 2 + WV - 1) / WV : 1;
+    PostHead<HD> raw[ROUNDS];
+    float freq = 0.f;
     if constexpr (FUSED) {
 #pragma unroll
         for (int r = 0; r < ROUNDS; r++) {
-            const int j = wave + 4 * r;
-            if (j < G + 2) {
-                const int src = j < G ? head0 + j : (j == G ? fp.n_head + kvh : fp.n_head + n_kv + kvh);
-                const float* x = fp.qkv + (size_t)src * HD;
-                const float* bias = fp.bias ? fp.bias + (size_t)src * HD : nullptr;
-#pragma unroll
-                for (int i = 0; i < EPL; i++) xr[r][i] = bias ? x[lane + 64 * i] + bias[lane + 64 * i] : x[lane + 64 * i];
-            }
+            const int j = wave + WV * r;
+            if (j < G + 2)
+                raw[r] = post_request<HD>(fp, j < G ? head0 + j : (j == G ? fp.n_head + kvh : fp.n_head + n_kv + kvh),
+                                          j < G ? fp.q_norm : (j == G ? fp.k_norm : nullptr), lane);
         }
+        if (wave <= G && lane < fp.n_rot / 2) freq = rope_inv_freq(lane, fp.rate, fp.freq_scale);   // under the loads' latency
     }
     uint32_t len = len_dev ? *len_dev + 1u : len_host;   // the device word is the newest token's position
     asm volatile("" ::: "memory");                       // keeps the loads above in front of the arithmetic on the length
@@ -646,40 +691,30 @@ __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typ
         // inside the cache) is still appended, by the last split, as the separate post-processing launch would
         const bool owner = pos < fp.cap && (pos < len ? (pos >= k0 && pos < k1) : split == splits - 1);
         const int njobs = G + (owner ? 2 : 0);
-        const int kvw = n_kv * HD, half = fp.n_rot / 2;
+        const int kvw = n_kv * HD;
+        float sn = 0.f, cs = 1.f;
+        if (wave <= G) sincosf((float)pos * freq, &sn, &cs);
 #pragma unroll
         for (int r = 0; r < ROUNDS; r++) {                 // job j < G: query head j of the group; G: the K row; G + 1: the V row
-            const int j = wave + 4 * r;
+            const int j = wave + WV * r;
             if (j >= njobs) continue;
-            const int src = j < G ? head0 + j : (j == G ? fp.n_head + kvh : fp.n_head + n_kv + kvh);
-            const float* x = fp.qkv + (size_t)src * HD;
-            const float* bias = fp.bias ? fp.bias + (size_t)src * HD : nullptr;
-            const float* nw = j < G ? fp.q_norm : (j == G ? fp.k_norm : nullptr);
-            float* dst = j < G ? &sm_q[FUSED ? j : 0][0] : (j == G ? fp.k_cache : fp.v_cache) + (size_t)pos * kvw + (size_t)kvh * HD;
-            if (j == G + 1) {
-#pragma unroll
-                for (int i = 0; i < EPL; i++) dst[lane + 64 * i] = xr[r][i];
+            if (j < G) {
+                post_rotate<HD>(fp, raw[r], fp.q_norm != nullptr, cs, sn, lane, &sm_row[FUSED ? wave : 0][0], &sm_q[FUSED ? j : 0][0]);
                 continue;
             }
-            float inv = 1.f;
-            if (nw) {
-                float ms = 0.f;
+            float* dst = QF >= 0 ? &sm_kv[FUSED && QF >= 0 ? j - G : 0][0] : (j == G ? fp.k_cache : fp.v_cache) + (size_t)pos * kvw + (size_t)kvh * HD;
+            if (j == G) post_rotate<HD>(fp, raw[r], fp.k_norm != nullptr, cs, sn, lane, &sm_row[FUSED ? wave : 0][0], dst);
+            else {
 #pragma unroll
-                for (int i = 0; i < EPL; i++) ms = fmaf(xr[r][i], xr[r][i], ms);
-                ms = wave_sum(ms);
-                inv = 1.0f / sqrtf(ms / (float)HD + fp.eps);
+                for (int i = 0; i < HD / 64; i++) dst[lane + 64 * i] = raw[r].x[i];
             }
-            auto val = [&](int e) { float v = bias ? x[e] + bias[e] : x[e]; return nw ? v * inv * nw[e] : v; };
-            for (int c = lane; c < half; c += 64) {
-                const float ang = (float)pos * rope_inv_freq(c, fp.rate, fp.freq_scale);
-                float sn, cs;
-                sincosf(ang, &sn, &cs);
-                const int p0 = fp.interleaved ? 2 * c : c, p1 = fp.interleaved ? 2 * c + 1 : c + half;
-                const float x1 = val(p0), x2 = val(p1);
-                dst[p0] = rot_lo(x1, x2, cs, sn);
-                dst[p1] = rot_hi(x1, x2, cs, sn);
+            if constexpr (QF >= 0) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const size_t b0 = ((size_t)pos * n_kv + kvh) * (HD / 32);
+#pragma unroll
+                for (int e = lane; e < HD; e += 64)
+                    quantize_lanes<QF>(dst[e], lane & 31, true, j == G ? qst.k_codes : qst.v_codes, j == G ? qst.k_scales : qst.v_scales, b0 + (size_t)(e >> 5));
             }
-            for (int e = fp.n_rot + lane; e < HD; e += 64) dst[e] = val(e);
         }
         __syncthreads();
     }
@@ -759,12 +794,14 @@ __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typ
         if (lane == 0) { sm_m[wave][h] = M; sm_l[wave][h] = lv; }
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < G * HD; idx += 256) {
+    for (int idx = threadIdx.x; idx < G * HD; idx += 64 * WV) {
         const int h = idx / HD, d = idx % HD;
-        const float M = fmaxf(fmaxf(sm_m[0][h], sm_m[1][h]), fmaxf(sm_m[2][h], sm_m[3][h]));
+        float M = sm_m[0][h];
+#pragma unroll
+        for (int w = 1; w < WV; w++) M = fmaxf(M, sm_m[w][h]);
         float L = 0.f, A = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
+        for (int w = 0; w < WV; w++) {
             const float f = __expf(sm_m[w][h] - M);
             L = fmaf(sm_l[w][h], f, L);
             A = fmaf(sm_acc[w][h][d], f, A);
@@ -780,25 +817,33 @@ __device__ __forceinline__ void attn_split_body(const float* __restrict__ q, typ
     }
 }
 
-template <int G, int DPL>
-__global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V,
-                                                         int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev, float scale, int splits,
-                                                         uint32_t window, float softcap, float* __restrict__ part, float* __restrict__ out, int gq) {
-    attn_split_body<G, DPL, false>(q, K, V, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, QkvPostParams{}, gq);
+template <int G, int DPL, int WV>
+__global__ __launch_bounds__(64 * WV) void attn_split_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V,
+                                                             int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev, float scale, int splits,
+                                                             uint32_t window, float softcap, float* __restrict__ part, float* __restrict__ out, int gq) {
+    attn_split_body<G, DPL, false, -1, WV>(q, K, V, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, QkvPostParams{}, gq);
 }
 
-template <int G, int DPL, int QF>
-__global__ __launch_bounds__(256) void attn_split_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
-                                                             const uint32_t* __restrict__ len_dev, float scale, int splits, uint32_t window,
-                                                             float softcap, float* __restrict__ part, float* __restrict__ out, int gq) {
-    attn_split_body<G, DPL, false, QF>(q, nullptr, nullptr, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, QkvPostParams{}, gq, qc);
+template <int G, int DPL, int QF, int WV>
+__global__ __launch_bounds__(64 * WV) void attn_split_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
+                                                                 const uint32_t* __restrict__ len_dev, float scale, int splits, uint32_t window,
+                                                                 float softcap, float* __restrict__ part, float* __restrict__ out, int gq) {
+    attn_split_body<G, DPL, false, QF, WV>(q, nullptr, nullptr, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, QkvPostParams{}, gq, qc);
 }
 
-template <int G, int DPL>
-__global__ __launch_bounds__(256) void attn_split_fused_kernel(QkvPostParams fp, int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev,
-                                                               float scale, int splits, uint32_t window, float softcap, float* __restrict__ part,
-                                                               float* __restrict__ out, int gq) {
-    attn_split_body<G, DPL, true>(nullptr, fp.k_cache, fp.v_cache, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, fp, gq);
+template <int G, int DPL, int WV>
+__global__ __launch_bounds__(64 * WV) void attn_split_fused_kernel(QkvPostParams fp, int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev,
+                                                                   float scale, int splits, uint32_t window, float softcap, float* __restrict__ part,
+                                                                   float* __restrict__ out, int gq) {
+    attn_split_body<G, DPL, true, -1, WV>(nullptr, fp.k_cache, fp.v_cache, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, fp, gq);
+}
+
+template <int G, int DPL, int QF, int WV>
+__global__ __launch_bounds__(64 * WV) void attn_split_fused_kvq_kernel(QkvPostParams fp, KvqStore st, int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev,
+                                                                       float scale, int splits, uint32_t window, float softcap, float* __restrict__ part,
+                                                                       float* __restrict__ out, int gq) {
+    attn_split_body<G, DPL, true, QF, WV>(nullptr, nullptr, nullptr, n_kv, len_host, len_dev, scale, splits, window, softcap, part, out, fp, gq,
+                                          QCache{st.k_codes, st.k_scales, st.v_codes, st.v_scales}, st);
 }
 
 // One workgroup per query head: weights exp(m_s - max m) of the splits once (each wave reduces them for itself; through LDS to
@@ -912,10 +957,11 @@ __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) 
 }
 
 constexpr int LONG_WAVES = 8, LONG_KEYS = 32;   // waves of a workgroup, keys a wave takes at a time
-template <int HD, int FMT, bool SPL>
-__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
-                                                                           const uint32_t* __restrict__ len_dev, float scale, int splits,
-                                                                           uint32_t window, float softcap, float* __restrict__ part, int gq) {   // gq: query heads per KV head, at most 8 (SPL: 5)
+// FUSED: q is formed here from the raw QKV row and the workgroup whose keys hold the newest token appends it, as attn_split_body does (fp, st).
+template <int HD, int FMT, bool SPL, bool FUSED>
+__device__ __forceinline__ void attn_long_body(const float* __restrict__ q, const QCache& qc, int n_kv, uint32_t len_host, const uint32_t* __restrict__ len_dev,
+                                               float scale, int splits, uint32_t window, float softcap, float* __restrict__ part, int gq,   // gq: query heads per KV head, at most 8 (SPL: 5)
+                                               const QkvPostParams& fp, const KvqStore& st) {
     constexpr int NB = HD / 32, NT = LONG_KEYS / 16;                    // blocks of a row, tiles of 16 keys
     constexpr bool Q8 = FMT == FHIP_KVQ_Q8_0, PRE = HD == 64;             // PRE: keys requested a round ahead
     constexpr int CW = Q8 ? 8 : 4;                                      // code words of a block
@@ -953,13 +999,57 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const
         for (int i = 0; i < NB / 2; i++) sc[i] = sp[i];
     };
     uint32_t kt = k0 + (uint32_t)(LONG_KEYS * wave);
-    if (PRE && kt < k1) request_k(kt);
+    // the heads' rows, the token's rows and the waves' scratch rows lie where the sums of the waves will
+    float* const sq = FUSED ? &sm_acc[0][0][0] : nullptr;               // [8][HD] | [2][HD] | [LONG_WAVES][HD]
+    static_assert(18 * HD <= LONG_WAVES * 8 * (HD + 4), "");
+    bool owner = false;
+    if constexpr (FUSED) {
+        const uint32_t pos = *len_dev;
+        owner = pos < fp.cap && (pos < len ? (pos >= k0 && pos < k1) : split == splits - 1);
+    }
+    if (PRE && kt < k1 && !owner) request_k(kt);
+    if constexpr (FUSED) {
+        const int njobs = gq + (owner ? 2 : 0);
+        const uint32_t pos = *len_dev;
+        PostHead<HD> raw[2];                                            // up to ten jobs for eight waves
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int j = wave + LONG_WAVES * r;
+            if (j < njobs)
+                raw[r] = post_request<HD>(fp, j < gq ? head0 + j : (j == gq ? fp.n_head + kvh : fp.n_head + n_kv + kvh), j < gq ? fp.q_norm : (j == gq ? fp.k_norm : nullptr), lane);
+        }
+        float sn = 0.f, cs = 1.f;
+        if (lane < fp.n_rot / 2) sincosf((float)pos * rope_inv_freq(lane, fp.rate, fp.freq_scale), &sn, &cs);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int j = wave + LONG_WAVES * r;
+            if (j >= njobs) continue;
+            float* const dst = sq + j * HD + (j < gq ? 0 : (8 - gq) * HD);   // a query row, or rows 8 and 9
+            if (j <= gq) post_rotate<HD>(fp, raw[r], (j < gq ? fp.q_norm : fp.k_norm) != nullptr, cs, sn, lane, sq + (10 + wave) * HD, dst);
+            else {
+#pragma unroll
+                for (int i = 0; i < HD / 64; i++) dst[lane + 64 * i] = raw[r].x[i];
+            }
+            if (j >= gq) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const size_t b0 = ((size_t)pos * n_kv + kvh) * NB;
+#pragma unroll
+                for (int e = 0; e < HD; e += 64)
+                    quantize_lanes<FMT>(dst[e + lane], lane & 31, true, j == gq ? st.k_codes : st.v_codes, j == gq ? st.k_scales : st.v_scales, b0 + (size_t)((e + lane) >> 5));
+            }
+        }
+        __syncthreads();
+        if (PRE && kt < k1 && owner) request_k(kt);
+    }
 
     if (wave < NB) {                                                    // wave j cuts the queries' block j up for all
         float x[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) x[i] = 0.f;
-        if (qn < gq) load_dims<8>(q + ((size_t)head0 + qn) * HD + 32 * wave + 8 * g, x);
+        if (qn < gq) {
+            if constexpr (FUSED) load_dims<8>(sq + qn * HD + 32 * wave + 8 * g, x);
+            else load_dims<8>(q + ((size_t)head0 + qn) * HD + 32 * wave + 8 * g, x);
+        }
 #pragma unroll
         for (int t = 0; t < 3; t++) {
             sm_q[wave][t][lane] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
@@ -1174,39 +1264,82 @@ __global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const
     }
 }
 
+template <int HD, int FMT, bool SPL>
+__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
+                                                                           const uint32_t* __restrict__ len_dev, float scale, int splits,
+                                                                           uint32_t window, float softcap, float* __restrict__ part, int gq) {
+    attn_long_body<HD, FMT, SPL, false>(q, qc, n_kv, len_host, len_dev, scale, splits, window, softcap, part, gq, QkvPostParams{}, KvqStore{});
+}
+template <int HD, int FMT, bool SPL>
+__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_fused_kvq_kernel(QkvPostParams fp, KvqStore st, int n_kv, uint32_t len_host,
+                                                                                 const uint32_t* __restrict__ len_dev, float scale, int splits,
+                                                                                 uint32_t window, float softcap, float* __restrict__ part, int gq) {
+    attn_long_body<HD, FMT, SPL, true>(nullptr, QCache{st.k_codes, st.k_scales, st.v_codes, st.v_scales}, n_kv, len_host, len_dev, scale, splits, window, softcap, part, gq,
+                                       fp, st);
+}
+
+// wide (G = 1): workgroups of ATT_WIDE waves
+constexpr int ATT_WIDE = 16;
+template <int G, class Kernel, class Wide, class... Args>
+void attn_go(dim3 grid, hipStream_t s, bool wide, Kernel kernel, Wide kernel_wide, Args... args) {
+    if (G == 1 && wide) hipLaunchKernelGGL(kernel_wide, grid, dim3(64 * ATT_WIDE), 0, s, args...);
+    else hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, args...);
+}
+
 template <int G>
 int launch_attn_g(int hd, dim3 grid, hipStream_t s, const float* q, const float* K, const float* V, int n_kv, uint32_t len, const uint32_t* d_len,
-                  float scale, int splits, uint32_t window, float softcap, float* part, float* out, int gq = G) {
+                  float scale, int splits, uint32_t window, float softcap, float* part, float* out, int gq = G, bool wide = false) {
     switch (hd) {
-        case 64: hipLaunchKernelGGL((attn_split_kernel<G, 4>), grid, dim3(256), 0, s, q, K, V, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
-        case 128: hipLaunchKernelGGL((attn_split_kernel<G, 8>), grid, dim3(256), 0, s, q, K, V, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
+        case 64: attn_go<G>(grid, s, wide, attn_split_kernel<G, 4, 4>, attn_split_kernel<1, 4, ATT_WIDE>, q, K, V, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
+        case 128: attn_go<G>(grid, s, wide, attn_split_kernel<G, 8, 4>, attn_split_kernel<1, 8, ATT_WIDE>, q, K, V, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
         default: return fhip::set_error(FHIP_ERR_SHAPE, "decode_attention: head_dim must be 64 or 128");
     }
     return FHIP_OK;
 }
 
-template <int G, int QF>
-int launch_attn_kvq_g(int hd, dim3 grid, hipStream_t s, const float* q, const QCache& qc, int n_kv, uint32_t len, const uint32_t* d_len,
-                      float scale, int splits, uint32_t window, float softcap, float* part, float* out, int gq = G) {
-    switch (hd) {
-        case 64: hipLaunchKernelGGL((attn_split_kvq_kernel<G, 4, QF>), grid, dim3(256), 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
-        case 128: hipLaunchKernelGGL((attn_split_kvq_kernel<G, 8, QF>), grid, dim3(256), 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
-        default: return fhip::set_error(FHIP_ERR_SHAPE, "decode_attention: head_dim must be 64 or 128");
-    }
-    return FHIP_OK;
+// What the launches over a quantized cache share; fp: the raw QKV row to post-process and append (null: q holds the queries).
+struct KvqLaunch {
+    hipStream_t s;
+    const float* q;
+    const QkvPostParams* fp;
+    KvqStore cache;
+    int n_kv;
+    uint32_t len;
+    const uint32_t* d_len;
+    float scale;
+    int splits;
+    uint32_t window;
+    float softcap;
+    float *part, *out;
+    QCache qc() const { return QCache{cache.k_codes, cache.k_scales, cache.v_codes, cache.v_scales}; }
+};
+template <int G, int DPL, int QF>
+void launch_attn_kvq_hd(dim3 grid, const KvqLaunch& a, int gq, bool wide) {
+    if (a.fp)
+        attn_go<G>(grid, a.s, wide, attn_split_fused_kvq_kernel<G, DPL, QF, 4>, attn_split_fused_kvq_kernel<1, DPL, QF, ATT_WIDE>, *a.fp, a.cache, a.n_kv, a.len, a.d_len, a.scale,
+                   a.splits, a.window, a.softcap, a.part, a.out, gq);
+    else
+        attn_go<G>(grid, a.s, wide, attn_split_kvq_kernel<G, DPL, QF, 4>, attn_split_kvq_kernel<1, DPL, QF, ATT_WIDE>, a.q, a.qc(), a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window,
+                   a.softcap, a.part, a.out, gq);
 }
+// gq: as attn_split_body's (G, -g, or query heads per KV head with G = 1)
 template <int QF>
-int launch_attn_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, const QCache& qc, int n_kv, uint32_t len, const uint32_t* d_len,
-                    float scale, int splits, uint32_t window, float softcap, float* part, float* out) {
+int launch_attn_kvq(int g, int hd, dim3 grid, const KvqLaunch& a, int gq, bool wide = false) {
+    auto go = [&](auto Gc) {
+        constexpr int G = decltype(Gc)::value;
+        if (hd == 64) launch_attn_kvq_hd<G, 4, QF>(grid, a, gq, wide);
+        else launch_attn_kvq_hd<G, 8, QF>(grid, a, gq, wide);
+        return FHIP_OK;
+    };
     switch (g) {
-        case 1: return launch_attn_kvq_g<1, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 2: return launch_attn_kvq_g<2, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 3: return launch_attn_kvq_g<3, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 4: return launch_attn_kvq_g<4, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 5: return launch_attn_kvq_g<5, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 6: return launch_attn_kvq_g<6, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 7: return launch_attn_kvq_g<7, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
-        case 8: return launch_attn_kvq_g<8, QF>(hd, grid, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, out);
+        case 1: return go(std::integral_constant<int, 1>{});
+        case 2: return go(std::integral_constant<int, 2>{});
+        case 3: return go(std::integral_constant<int, 3>{});
+        case 4: return go(std::integral_constant<int, 4>{});
+        case 5: return go(std::integral_constant<int, 5>{});
+        case 6: return go(std::integral_constant<int, 6>{});
+        case 7: return go(std::integral_constant<int, 7>{});
+        case 8: return go(std::integral_constant<int, 8>{});
         default: return fhip::set_error(FHIP_ERR_SHAPE, "decode_attention: %d query heads per KV head (1..=8 supported)", g);
     }
 }
@@ -1221,20 +1354,26 @@ bool attn_long_takes(int fmt, int g, int n_kv, const uint32_t* k_codes) {
     return g >= 3;
 }
 template <int FMT>
-void launch_attn_long_kvq(int g, int hd, dim3 grid, hipStream_t s, const float* q, const QCache& qc, int n_kv, uint32_t len, const uint32_t* d_len,
-                          float scale, int splits, uint32_t window, float softcap, float* part) {
-    const dim3 wg(64 * LONG_WAVES);
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, s, q, qc, n_kv, len, d_len, scale, splits, window, softcap, part, g); };
-    if (hd == 64) { if (g <= 5) go(attn_long_kvq_kernel<64, FMT, true>); else go(attn_long_kvq_kernel<64, FMT, false>); }
-    else { if (g <= 5) go(attn_long_kvq_kernel<128, FMT, true>); else go(attn_long_kvq_kernel<128, FMT, false>); }
+void launch_attn_long_kvq(int g, int hd, dim3 grid, const KvqLaunch& a) {
+    auto go = [&](auto kernel, auto fused) {
+        if (a.fp) hipLaunchKernelGGL(fused, grid, dim3(64 * LONG_WAVES), 0, a.s, *a.fp, a.cache, a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
+        else hipLaunchKernelGGL(kernel, grid, dim3(64 * LONG_WAVES), 0, a.s, a.q, a.qc(), a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
+    };
+    if (hd == 64) {
+        if (g <= 5) go(attn_long_kvq_kernel<64, FMT, true>, attn_long_fused_kvq_kernel<64, FMT, true>);
+        else go(attn_long_kvq_kernel<64, FMT, false>, attn_long_fused_kvq_kernel<64, FMT, false>);
+    } else {
+        if (g <= 5) go(attn_long_kvq_kernel<128, FMT, true>, attn_long_fused_kvq_kernel<128, FMT, true>);
+        else go(attn_long_kvq_kernel<128, FMT, false>, attn_long_fused_kvq_kernel<128, FMT, false>);
+    }
 }
 
 template <int G>
 int launch_attn_fused_g(int hd, dim3 grid, hipStream_t s, const QkvPostParams& fp, int n_kv, uint32_t len, const uint32_t* d_len, float scale,
-                        int splits, uint32_t window, float softcap, float* part, float* out, int gq = G) {
+                        int splits, uint32_t window, float softcap, float* part, float* out, int gq = G, bool wide = false) {
     switch (hd) {
-        case 64: hipLaunchKernelGGL((attn_split_fused_kernel<G, 4>), grid, dim3(256), 0, s, fp, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
-        case 128: hipLaunchKernelGGL((attn_split_fused_kernel<G, 8>), grid, dim3(256), 0, s, fp, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
+        case 64: attn_go<G>(grid, s, wide, attn_split_fused_kernel<G, 4, 4>, attn_split_fused_kernel<1, 4, ATT_WIDE>, fp, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
+        case 128: attn_go<G>(grid, s, wide, attn_split_fused_kernel<G, 8, 4>, attn_split_fused_kernel<1, 8, ATT_WIDE>, fp, n_kv, len, d_len, scale, splits, window, softcap, part, out, gq); break;
         default: return fhip::set_error(FHIP_ERR_SHAPE, "decode_attention: head_dim must be 64 or 128");
     }
     return FHIP_OK;
@@ -1366,13 +1505,17 @@ int launch_kv_append(const float* k, const float* v, size_t t, size_t width, con
     return check_hip(hipGetLastError(), "kv_append launch");
 }
 
-// Splits of the key range: about two workgroups per CU over all KV heads, at least 64 keys each (two rounds of the
-// workgroup's 16 streams x 2 keys; 16 for caches of up to 256 rows), at most 256 (the combine kernel's LDS tables).
-// Caches of up to ATT_SHORT rows (a launch sized for that many) with several query heads per KV head: one workgroup per query head over the whole key range, no
-// splits, no combine launch. The rows of a KV head are read by each of its query heads' workgroups (a few hundred KB out of the
-// L2), which costs less than the second launch and the trip of the partial results through memory.
-constexpr size_t ATT_SHORT = 256;   // chained 64-layer step, ms per token, this shape | one workgroup per (query head, split): 180 keys 3.87 | 3.92, 248: 3.96 | 3.99, 300: 4.05 | 3.96, 370: 4.11 | 3.97
-bool attn_per_query_head(size_t len, int n_head, int n_kv) { return n_kv > 0 && n_head > n_kv && len <= ATT_SHORT; }
+// Caches of up to ATT_SHORT rows (a launch sized for that many): one workgroup per query head over the whole key range, no splits, no
+// combine launch. The rows of a KV head are read by each of its query heads' workgroups (a few hundred KB out of the L2), which costs less
+// than the second launch and the trip of the partial results through memory. A step of a workgroup's streams is a trip to memory (0.9 us on rows no
+// cache holds), so from ATT_WIDE_FROM rows on it has sixteen waves, 128 keys a step, in place of four; fewer rows leave most of those without a key (48 rows
+// 4.6 -> 5.6 us). Four waves -> sixteen, f32 cache, us: 130 / 200 / 256 rows 6.2 / 6.9 / 7.1 -> 5.8 / 6.2 / 6.5. us a token through four layers (d 2048, 16 and 8 heads of 128), one
+// workgroup a head | per (head, split) and combined: f32 300 rows 153.6 | 159.4, 400 158.0 | 159.4, 490 162.1 | 160.4; Q8_0 300 154.4 | 159.7,
+// 490 160.9 | 159.6; d 5120, 40 heads, f32 300 320.3 | 323.6, 400 326.7 | 322.4, Q8_0 300 313.5 | 326.9, 490 318.3 | 324.2. A head per KV head, f32, 60 rows: 154.3 with
+// splits of 16 keys, 140.5 in one workgroup.
+constexpr size_t ATT_SHORT = 352, ATT_WIDE_FROM = 97;
+bool attn_per_query_head(size_t len) { return len <= ATT_SHORT; }
+bool attn_wide(size_t len) { return len >= ATT_WIDE_FROM; }
 
 // Between ATT_SHORT and ATT_MID rows under grouped query heads: one workgroup per (query head, split of at least ATT_MID_KEYS
 // keys). The kernel that takes all query heads of a KV head at once holds 180 registers a lane (two waves per SIMD) and its
@@ -1389,14 +1532,13 @@ int attn_mid_splits(size_t len, int n_head) {
     return s < 1 ? 1 : (s > 256 ? 256 : s);
 }
 
+// Splits of the key range beyond ATT_SHORT: about two workgroups per CU over all KV heads, at least 64 keys each (two rounds of the
+// workgroup's 16 streams x 2 keys), at most 256 (the combine kernel's LDS tables).
 int attn_splits(size_t len, int n_kv) {
-    if (n_kv <= 0 || len == 0) return 1;
+    if (n_kv <= 0 || attn_per_query_head(len)) return 1;
     constexpr int keys = 64;
     int want = (2 * device_cus() + n_kv - 1) / n_kv;
-    // up to 256 keys a split of 16 (half of the streams, one round) beat one of 64 by 0.1 ms per token of the chained step;
-    // from 512 keys on the larger split count costs more in the combine than it saves
-    const size_t per_split = len <= 256 ? 16 : (size_t)keys;
-    size_t by_keys = (len + per_split - 1) / per_split;
+    size_t by_keys = (len + (size_t)keys - 1) / (size_t)keys;
     int splits = (int)(by_keys < (size_t)want ? by_keys : (size_t)want);
     return splits < 1 ? 1 : (splits > 256 ? 256 : splits);
 }
@@ -1419,8 +1561,8 @@ int launch_decode_attention(const float* q, const float* K, const float* V, int 
     const float scale = 1.0f / sqrtf((float)hd);
     const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;   // a window that large is no window
     if (g > 8) return set_error(FHIP_ERR_SHAPE, "decode_attention: %d query heads per KV head (1..=8 supported)", g);
-    if (attn_per_query_head(len, n_head, n_kv)) {
-        int rc = launch_attn_g<1>(hd, dim3((unsigned)n_head, 1), s, q, K, V, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g);
+    if (attn_per_query_head(len)) {
+        int rc = launch_attn_g<1>(hd, dim3((unsigned)n_head, 1), s, q, K, V, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g, attn_wide(len));
         return rc ? rc : check_hip(hipGetLastError(), "decode_attention launch");
     }
     const bool mid = attn_per_head_splits(len, n_head, n_kv);
@@ -1452,54 +1594,35 @@ int launch_decode_attention(const float* q, const float* K, const float* V, int 
     return rc;
 }
 
-int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes, const uint16_t* k_scales, const uint32_t* v_codes,
-                                const uint16_t* v_scales, int n_head, int n_kv, int hd, size_t len, const uint32_t* d_len, size_t window,
-                                float softcap, float* ws, float* out, hipStream_t s) {
+// One query row over a quantized cache: q, or, with fp, formed from the raw QKV row whose key and value are appended first.
+static int launch_attention_over_kvq(const char* who, int fmt, const float* q, const QkvPostParams* fp, const KvqStore& cache, int n_head, int n_kv, int hd, size_t len,
+                                     const uint32_t* d_len, size_t window, float softcap, float* ws, float* out, hipStream_t s) {
     if (n_head == 0 || hd == 0) return FHIP_OK;
-    if (len == 0) return set_error(FHIP_ERR_SHAPE, "decode_attention: empty cache");
-    if (n_kv <= 0 || n_head % n_kv != 0) return set_error(FHIP_ERR_SHAPE, "decode_attention: n_heads must be a multiple of n_kv_heads");
-    if (hd != 64 && hd != 128) return set_error(FHIP_ERR_SHAPE, "decode_attention: head_dim must be 64 or 128");
-    if (len > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "decode_attention: cache length exceeds 2^31");
+    if (len == 0) return set_error(FHIP_ERR_SHAPE, "%s: empty cache", who);
+    if (n_kv <= 0 || n_head % n_kv != 0) return set_error(FHIP_ERR_SHAPE, "%s: n_heads must be a multiple of n_kv_heads", who);
+    if (hd != 64 && hd != 128) return set_error(FHIP_ERR_SHAPE, "%s: head_dim must be 64 or 128", who);
+    if (len > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "%s: cache length exceeds 2^31", who);
     const int g = n_head / n_kv;
-    const float scale = 1.0f / sqrtf((float)hd);
-    const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;
-    const QCache qc{k_codes, k_scales, v_codes, v_scales};
-    int rc;
-    if (g >= 1 && g <= 8 && attn_per_query_head(len, n_head, n_kv)) {   // as the f32 cache's launch: the same sums, the same bits
-        const dim3 per_head((unsigned)n_head, 1);
-        switch (fmt) {
-            case FHIP_KVQ_Q8_0: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q8_0>(hd, per_head, s, q, qc, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g); break;
-            case FHIP_KVQ_Q4_0: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q4_0>(hd, per_head, s, q, qc, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g); break;
-            case FHIP_KVQ_Q4_1: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q4_1>(hd, per_head, s, q, qc, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g); break;
-            default: return set_error(FHIP_ERR_ARG, "decode_attention: unknown KV format %d", fmt);
-        }
-        return rc ? rc : check_hip(hipGetLastError(), "decode_attention launch");
-    }
+    const bool per_head = g >= 1 && g <= 8 && attn_per_query_head(len);   // as the f32 cache's launch: the same sums, the same bits
     const bool mid = g >= 1 && g <= 8 && attn_per_head_splits(len, n_head, n_kv);
-    const int splits = mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
-    if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "decode_attention: this cache length needs the workspace");
-    const dim3 grid((unsigned)n_kv, (unsigned)splits);
-    if (!mid && splits > 1 && attn_long_takes(fmt, g, n_kv, k_codes)) {
-        rc = FHIP_OK;
-        switch (fmt) {
-            case FHIP_KVQ_Q8_0: launch_attn_long_kvq<FHIP_KVQ_Q8_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws); break;
-            case FHIP_KVQ_Q4_0: launch_attn_long_kvq<FHIP_KVQ_Q4_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws); break;
-            default: return set_error(FHIP_ERR_ARG, "decode_attention: unknown KV format %d", fmt);
-        }
-    } else if (mid) {
-        const dim3 lin((unsigned)((n_kv * splits + 7) / 8 * 8 * g), 1);
-        switch (fmt) {
-            case FHIP_KVQ_Q8_0: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q8_0>(hd, lin, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out, -g); break;
-            case FHIP_KVQ_Q4_0: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q4_0>(hd, lin, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out, -g); break;
-            case FHIP_KVQ_Q4_1: rc = launch_attn_kvq_g<1, FHIP_KVQ_Q4_1>(hd, lin, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out, -g); break;
-            default: return set_error(FHIP_ERR_ARG, "decode_attention: unknown KV format %d", fmt);
-        }
-    } else
+    const int splits = per_head ? 1 : mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
+    if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "%s: this cache length needs the workspace", who);
+    const KvqLaunch a{s, q, fp, cache, n_kv, (uint32_t)len, d_len, 1.0f / sqrtf((float)hd), splits, window > 0x7FFFFFFFull ? 0u : (uint32_t)window, softcap, ws, out};
+    const dim3 grid = per_head ? dim3((unsigned)n_head, 1) : mid ? dim3((unsigned)((n_kv * splits + 7) / 8 * 8 * g), 1) : dim3((unsigned)n_kv, (unsigned)splits);
+    const int G = per_head || mid ? 1 : g, gq = per_head ? g : mid ? -g : g;
+    const bool wide = per_head && attn_wide(len), lng = !per_head && !mid && splits > 1 && attn_long_takes(fmt, g, n_kv, cache.k_codes);
+    int rc = FHIP_OK;
     switch (fmt) {
-        case FHIP_KVQ_Q8_0: rc = launch_attn_kvq<FHIP_KVQ_Q8_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out); break;
-        case FHIP_KVQ_Q4_0: rc = launch_attn_kvq<FHIP_KVQ_Q4_0>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out); break;
-        case FHIP_KVQ_Q4_1: rc = launch_attn_kvq<FHIP_KVQ_Q4_1>(g, hd, grid, s, q, qc, n_kv, (uint32_t)len, d_len, scale, splits, win, softcap, ws, out); break;
-        default: return set_error(FHIP_ERR_ARG, "decode_attention: unknown KV format %d", fmt);
+        case FHIP_KVQ_Q8_0:
+            if (lng) launch_attn_long_kvq<FHIP_KVQ_Q8_0>(g, hd, grid, a);
+            else rc = launch_attn_kvq<FHIP_KVQ_Q8_0>(G, hd, grid, a, gq, wide);
+            break;
+        case FHIP_KVQ_Q4_0:
+            if (lng) launch_attn_long_kvq<FHIP_KVQ_Q4_0>(g, hd, grid, a);
+            else rc = launch_attn_kvq<FHIP_KVQ_Q4_0>(G, hd, grid, a, gq, wide);
+            break;
+        case FHIP_KVQ_Q4_1: rc = launch_attn_kvq<FHIP_KVQ_Q4_1>(G, hd, grid, a, gq, wide); break;
+        default: return set_error(FHIP_ERR_ARG, "%s: unknown KV format %d", who, fmt);
     }
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "decode_attention launch"))) return rc;
@@ -1508,6 +1631,33 @@ int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes
         rc = check_hip(hipGetLastError(), "decode_attention combine launch");
     }
     return rc;
+}
+
+int launch_decode_attention_kvq(int fmt, const float* q, const uint32_t* k_codes, const uint16_t* k_scales, const uint32_t* v_codes,
+                                const uint16_t* v_scales, int n_head, int n_kv, int hd, size_t len, const uint32_t* d_len, size_t window,
+                                float softcap, float* ws, float* out, hipStream_t s) {
+    // (read only: without fp nothing is appended)
+    const KvqStore cache{const_cast<uint32_t*>(k_codes), const_cast<uint16_t*>(k_scales), const_cast<uint32_t*>(v_codes), const_cast<uint16_t*>(v_scales)};
+    return launch_attention_over_kvq("decode_attention", fmt, q, nullptr, cache, n_head, n_kv, hd, len, d_len, window, softcap, ws, out, s);
+}
+
+static QkvPostParams one_token_post(const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos, const float* freq_scale, int n_head,
+                                    int n_kv, int hd, int n_rot, bool interleaved, float eps, float base, size_t cap) {
+    QkvPostParams fp;
+    fp.qkv = qkv; fp.bias = bias; fp.q_norm = q_norm; fp.k_norm = k_norm; fp.pos = d_pos; fp.freq_scale = freq_scale;
+    fp.q_out = nullptr; fp.k_cache = nullptr; fp.v_cache = nullptr;
+    fp.t = 1; fp.n_head = n_head; fp.n_kv = n_kv; fp.hd = hd; fp.n_rot = n_rot; fp.interleaved = interleaved ? 1 : 0;
+    fp.cap = (uint32_t)cap; fp.eps = eps; fp.rate = rope_rate(n_rot, base); fp.kv_packed = 0;
+    return fp;
+}
+
+int launch_qkv_post_attention_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos, const float* freq_scale,
+                                  int n_head, int n_kv, int hd, int n_rot, bool interleaved, float eps, float base, uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes,
+                                  uint16_t* v_scales, size_t cap, size_t len, size_t window, float softcap, float* ws, float* out, hipStream_t s) {
+    if (len > cap) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention_kvq: length outside the cache");
+    const QkvPostParams fp = one_token_post(qkv, bias, q_norm, k_norm, d_pos, freq_scale, n_head, n_kv, hd, n_rot, interleaved, eps, base, cap);
+    return launch_attention_over_kvq("qkv_post_attention_kvq", fmt, nullptr, &fp, KvqStore{k_codes, k_scales, v_codes, v_scales}, n_head, n_kv, hd, len, d_pos, window, softcap, ws,
+                                     out, s);
 }
 
 int launch_qkv_post_attention(const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos,
@@ -1521,20 +1671,17 @@ int launch_qkv_post_attention(const float* qkv, const float* bias, const float* 
     if (len > 0x7FFFFFFFull || len > cap) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention: length outside the cache");
     const int g = n_head / n_kv;
     const bool mid = g <= 8 && attn_per_head_splits(len, n_head, n_kv);
-    const int splits = attn_per_query_head(len, n_head, n_kv) ? 1 : (mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv));
+    const int splits = attn_per_query_head(len) ? 1 : (mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv));
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "qkv_post_attention: this cache length needs the workspace");
-    QkvPostParams fp;
-    fp.qkv = qkv; fp.bias = bias; fp.q_norm = q_norm; fp.k_norm = k_norm; fp.pos = d_pos; fp.freq_scale = freq_scale;
-    fp.q_out = nullptr; fp.k_cache = k_cache; fp.v_cache = v_cache;
-    fp.t = 1; fp.n_head = n_head; fp.n_kv = n_kv; fp.hd = hd; fp.n_rot = n_rot; fp.interleaved = interleaved ? 1 : 0;
-    fp.cap = (uint32_t)cap; fp.eps = eps; fp.rate = rope_rate(n_rot, base); fp.kv_packed = 0;
+    QkvPostParams fp = one_token_post(qkv, bias, q_norm, k_norm, d_pos, freq_scale, n_head, n_kv, hd, n_rot, interleaved, eps, base, cap);
+    fp.k_cache = k_cache; fp.v_cache = v_cache;
     const float scale = 1.0f / sqrtf((float)hd);
     const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;
     if (g > 8) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention: %d query heads per KV head (1..=8 supported)", g);
-    if (attn_per_query_head(len, n_head, n_kv)) {
+    if (attn_per_query_head(len)) {
         // every workgroup of a KV head forms the new token's K and V rows and stores them (the same bits from each) before
         // it reads them back with the other keys
-        int rc = launch_attn_fused_g<1>(hd, dim3((unsigned)n_head, 1), s, fp, n_kv, (uint32_t)len, d_pos, scale, 1, win, softcap, ws, out, g);
+        int rc = launch_attn_fused_g<1>(hd, dim3((unsigned)n_head, 1), s, fp, n_kv, (uint32_t)len, d_pos, scale, 1, win, softcap, ws, out, g, attn_wide(len));
         return rc ? rc : check_hip(hipGetLastError(), "qkv_post_attention launch");
     }
     dim3 grid((unsigned)n_kv, (unsigned)splits);

@@ -216,7 +216,6 @@ class Qwen3Decoder:
         else:
             from .kvquant import QKvCache
             self.caches = [(QKvCache(kv_fmt, max_len, self.kv_out), QKvCache(kv_fmt, max_len, self.kv_out)) for _ in layers]
-            fuse_attn = self.fuse_attn = False            # the rows are quantized in the post-processing's launch, in front of attention's
         self.pos = _u32_tensor([0])                       # device word: the position of the token being decoded
         self.xa = Tensor.empty((1, c.d_model))            # residual stream: the step's input is written here ...
         self.xb = Tensor.empty((1, c.d_model))            # ... and the residual alternates between the two buffers
@@ -241,8 +240,8 @@ class Qwen3Decoder:
             # of its own up to 2048 keys (5.12 -> 5.06 ms/token there, 4.92 -> 4.84 at 128) and is level with it from 4096 on.
             self.fuse_attn = True
         self.fuse_attn = bool(self.fuse_attn)
-        # a default-arm layer; caches of up to 256 rows under grouped query heads need no combine launch behind the attention
-        short = self.max_len <= 256 and c.n_head > c.n_head_kv
+        # a default-arm layer; short caches, whose attention splits nothing, need no combine launch behind it
+        short = self.ws is None
         self.launches_per_layer = (7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) - (1 if short else 0)
         # per token beside the layers: the position word's increment and the head (final norm inside the head's mat-vec; a head of
         # 128 MB and more takes the norm as a launch of its own, which costs less than the wider workgroups the fused norm needs)
@@ -304,12 +303,17 @@ class Qwen3Decoder:
             if self.kv_fmt is not None:
                 # the quantized arm (qwen3.rs:906-912): post-process and store the token's rows as blocks, attend over the blocks
                 kq, vq = kv
-                _check(lib.fhip_qkv_post_kvq(self.kv_fmt, self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, 1, c.n_head, c.n_head_kv, c.head_dim, n_rot,
-                                             int(c.rope_interleaved), c.eps, base, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr,
-                                             vq.scales.ptr, kq.cap, s))
-                _check(lib.fhip_decode_attention_kvq(self.kv_fmt, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, c.n_head,
-                                                     c.n_head_kv, c.head_dim, self.max_len, self.pos.buf.ptr, l.window, c.attn_softcap, ws,
-                                                     self.att.buf.ptr, s))
+                if self.fuse_attn:
+                    _check(lib.fhip_qkv_post_attention_kvq(self.kv_fmt, self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, c.n_head, c.n_head_kv, c.head_dim,
+                                                           n_rot, int(c.rope_interleaved), c.eps, base, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr,
+                                                           vq.scales.ptr, kq.cap, self.max_len, l.window, c.attn_softcap, ws, self.att.buf.ptr, s))
+                else:
+                    _check(lib.fhip_qkv_post_kvq(self.kv_fmt, self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, 1, c.n_head, c.n_head_kv, c.head_dim,
+                                                 n_rot, int(c.rope_interleaved), c.eps, base, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr,
+                                                 vq.scales.ptr, kq.cap, s))
+                    _check(lib.fhip_decode_attention_kvq(self.kv_fmt, self.q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, c.n_head,
+                                                         c.n_head_kv, c.head_dim, self.max_len, self.pos.buf.ptr, l.window, c.attn_softcap, ws,
+                                                         self.att.buf.ptr, s))
             elif self.fuse_attn:
                 _check(lib.fhip_qkv_post_attention(self.qkv.buf.ptr, bias, qn, kn, self.pos.buf.ptr, None, c.n_head, c.n_head_kv, c.head_dim,
                                                    n_rot, int(c.rope_interleaved), c.eps, base, kv.k.buf.ptr, kv.v.buf.ptr, kv.cap,

@@ -406,6 +406,12 @@ int fhip_qkv_post_attention(const float* d_qkv, const float* d_bias, const float
                             const float* d_freq_scale, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
                             float base, float* d_k_cache, float* d_v_cache, size_t cap, size_t len, size_t window, float softcap, float* d_ws,
                             float* d_out, void* stream);
+/* The same on a block-quantized cache: fhip_qkv_post_kvq and fhip_decode_attention_kvq for ONE new token in one launch (two where the
+ * key range is split), the same bytes in the cache and the same results. head_dim 64 or 128. */
+int fhip_qkv_post_attention_kvq(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_pos,
+                                const float* d_freq_scale, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                                float base, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap, size_t len,
+                                size_t window, float softcap, float* d_ws, float* d_out, void* stream);
 
 /* rmsnorm / add_rmsnorm (lib.rs:346, :372) fused into the mat-vec that consumes it, for ONE activation row:
  *   h = rmsnorm(x [+ resid], norm_w, eps);   y = h W^T   (swiglu != 0: y = silu(gate . h) * (up . h), as fhip_matmul_q_swiglu)

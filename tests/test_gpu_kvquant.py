@@ -319,3 +319,53 @@ def test_post_processing_and_quantized_stores_in_one_launch(F, Q, fmt, nh, nkv, 
     c = kq
     assert lib.fhip_qkv_post_kvq(fmt, qt.buf.ptr, None, None, None, pt.buf.ptr, None, 1, 1, 1, 288, 0, 0, 1e-6, 1e6, qt.buf.ptr, c.codes.ptr, c.scales.ptr, c.codes.ptr,
                                  c.scales.ptr, cap, None) != 0 and b"multiple of 32" in lib.fhip_last_error()
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("nh,nkv,hd,cap,pos,norm,bias,inter,n_rot,window,cap_soft", [
+    # one workgroup a query head: four waves, the first of sixteen, full, the last; a head of its own per KV head
+    (10, 2, 128, 1, 0, True, False, False, 128, 0, 0.0), (8, 4, 64, 96, 95, True, True, False, 64, 0, 0.0), (8, 4, 64, 97, 64, False, False, True, 64, 0, 30.0),
+    (40, 8, 128, 352, 351, True, False, False, 128, 100, 0.0), (4, 4, 128, 352, 200, True, True, False, 64, 0, 0.0),
+    # a workgroup a query head and split; all heads of a KV head a workgroup, and the matrix kernel (three heads and more), whose first request waits for the row
+    (8, 4, 128, 353, 352, True, False, False, 128, 0, 0.0), (40, 8, 128, 1500, 1300, True, True, False, 128, 0, 0.0), (4, 4, 64, 700, 699, True, False, False, 64, 0, 0.0),
+    (8, 4, 128, 5300, 5299, True, False, False, 128, 0, 0.0), (10, 2, 64, 5300, 4000, True, True, False, 64, 0, 0.0), (16, 2, 128, 6000, 5999, True, False, True, 128, 300, 0.0),
+    (16, 2, 64, 6000, 17, True, False, False, 32, 0, 20.0), (6, 2, 128, 5200, 5100, False, False, False, 0, 0, 0.0),
+    # a position past the cache is attended up to the cache's end and appended nowhere
+    (8, 4, 128, 300, 300, True, False, False, 128, 0, 0.0), (10, 2, 64, 5300, 6000, True, False, False, 64, 0, 0.0)])
+def test_post_processing_inside_the_attention_launch(F, Q, fmt, nh, nkv, hd, cap, pos, norm, bias, inter, n_rot, window, cap_soft):
+    # the two calls and the one leave the same bytes in the cache and the same outputs, bit for bit
+    from ferric_amd import decode as X
+    lib, rng = F._lib.load(), np.random.default_rng(cap + pos + fmt)
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    width, row = nkv * hd, (nh + 2 * nkv) * hd
+    qkv = T(rng.standard_normal((1, row)).astype(np.float32))
+    b = T(rng.standard_normal(row).astype(np.float32)) if bias else None
+    qn, kn = (T(rng.standard_normal(hd).astype(np.float32)) for _ in range(2)) if norm else (None, None)
+    P = lambda t: t.buf.ptr if t is not None else None
+    rows = [rng.standard_normal((cap, width)).astype(np.float32) for _ in range(2)]
+    p = X._u32_tensor([pos])
+    ws = F.DeviceBuffer(max(256, lib.fhip_decode_attention_ws_bytes(nh, nkv, hd, cap)))
+    got = []
+    for one in (False, True):
+        kc, vc = (Q.QKvCache.from_tensor(T(r), fmt) for r in rows)
+        out, q = T(np.zeros((1, nh * hd), np.float32)), T(np.zeros((1, nh * hd), np.float32))
+        if one:
+            F._lib.check(lib.fhip_qkv_post_attention_kvq(fmt, qkv.buf.ptr, P(b), P(qn), P(kn), p.buf.ptr, None, nh, nkv, hd, n_rot, int(inter), 1e-6, 1e6, kc.codes.ptr,
+                                                         kc.scales.ptr, vc.codes.ptr, vc.scales.ptr, cap, cap, window, cap_soft, ws.ptr, out.buf.ptr, None))
+        else:
+            F._lib.check(lib.fhip_qkv_post_kvq(fmt, qkv.buf.ptr, P(b), P(qn), P(kn), p.buf.ptr, None, 1, nh, nkv, hd, n_rot, int(inter), 1e-6, 1e6, q.buf.ptr, kc.codes.ptr,
+                                               kc.scales.ptr, vc.codes.ptr, vc.scales.ptr, cap, None))
+            F._lib.check(lib.fhip_decode_attention_kvq(fmt, q.buf.ptr, kc.codes.ptr, kc.scales.ptr, vc.codes.ptr, vc.scales.ptr, nh, nkv, hd, cap, p.buf.ptr, window, cap_soft,
+                                                       ws.ptr, out.buf.ptr, None))
+        got.append([out.to_vec().view(np.uint32)] + [x.view(np.uint8) for c in (kc, vc) for x in c.to_host()])
+    for a, c in zip(*got):
+        assert np.array_equal(a, c)
+
+
+def test_post_processing_inside_the_attention_launch_refuses(F, Q):
+    lib = F._lib.load()
+    t = F.Tensor.from_vec(np.zeros(1024, np.float32), (1024,))
+    call = lambda fmt=0, qkv=t.buf.ptr, nh=2, nkv=1, hd=64, cap=4, n=4, soft=0.0, ws=t.buf.ptr: lib.fhip_qkv_post_attention_kvq(
+        fmt, qkv, None, None, None, t.buf.ptr, None, nh, nkv, hd, 64, 0, 1e-6, 1e6, t.buf.ptr, t.buf.ptr, t.buf.ptr, t.buf.ptr, cap, n, 0, soft, ws, t.buf.ptr, None)
+    for bad in (dict(fmt=7), dict(qkv=None), dict(nh=3, nkv=2), dict(nh=9), dict(hd=96), dict(n=5), dict(n=0), dict(soft=-1.0), dict(cap=6000, n=6000, ws=None)):
+        assert call(**bad) != 0, bad
