@@ -6,8 +6,8 @@
 // that a small kernel on the caller's own stream reads or writes directly; the kernel's workgroups confirm in pinned words of
 // their own, which a host thread polls without a call into the runtime.
 //   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time)
-//   to the host     up to a slot in one or two kernels, the host copying the first part out while the second crosses the bus
-//                   (608 KB, idle device: 37 us with one kernel and a stream synchronisation); more is cut into chunks, each
+//   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
+//                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation); more is cut into chunks, each
 //                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
 //                   included, which is why there are several workers)
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms. A whole copy to the host reaches
@@ -36,7 +36,8 @@ constexpr size_t CHUNK = OUT_BYTES;              // of a long copy
 constexpr size_t SLOT_BYTES = OUT_BYTES + IN_BYTES;
 constexpr int SLOTS = 16, JOB_SLOTS = 12;        // a chunked copy takes up to JOB_SLOTS and leaves the others to small copies
 constexpr int MAX_WG = 64, THREADS = 512;        // workgroups of a copy (each confirms its part in a word of its own)
-constexpr size_t TWO_PARTS = (size_t)96 << 10;   // copies to the host from here on go in two parts: a launch costs less than the copy it hides
+constexpr size_t IN_PARTS = (size_t)96 << 10;    // copies to the host from here on go in parts, the host copying one out while the next ones cross
+constexpr int PARTS = 8;                         // at most
 constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
@@ -49,61 +50,77 @@ __device__ __forceinline__ void store_through(U* p, U v) { __hip_atomic_store(p,
 template <>
 __device__ __forceinline__ void store_through(u32x4* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory"); }
 
+// The copy in up to PARTS parts one after the other, each confirmed by itself: part p ends at byte end[p] (a multiple of 16 but for the last one's).
+struct Parts {
+    int count;
+    size_t end[PARTS];
+    uint32_t* done[PARTS];       // MAX_WG words each; null: nobody is told
+};
 template <class U>
-__global__ __launch_bounds__(THREADS) void copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t n, uint32_t* done,
-                                                       uint32_t seq) {
-    const size_t units = n / sizeof(U), step = (size_t)gridDim.x * THREADS;
+__global__ __launch_bounds__(THREADS) void copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, Parts parts, uint32_t seq) {
+    const size_t step = (size_t)gridDim.x * THREADS, n = parts.end[parts.count - 1];
     const U* s = (const U*)src;
     U* d = (U*)dst;
-    size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
-    for (; i + 3 * step < units; i += 4 * step) {       // four loads in flight: a load from host memory takes over a microsecond
-        const U a = s[i], b = s[i + step], c = s[i + 2 * step], e = s[i + 3 * step];
-        store_through(d + i, a); store_through(d + i + step, b); store_through(d + i + 2 * step, c); store_through(d + i + 3 * step, e);
-    }
-    for (; i < units; i += step) store_through(d + i, s[i]);
-    if (sizeof(U) > 1 && blockIdx.x == 0)
-        for (size_t k = units * sizeof(U) + threadIdx.x; k < n; k += THREADS) store_through(dst + k, src[k]);
-    if (done) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (threadIdx.x == 0) __hip_atomic_store(&done[blockIdx.x], seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    size_t begin = 0;
+#pragma unroll 1
+    for (int p = 0; p < parts.count; p++) {
+        const size_t units = parts.end[p] / sizeof(U);
+        size_t i = begin + (size_t)blockIdx.x * THREADS + threadIdx.x;
+        for (; i + 3 * step < units; i += 4 * step) {   // four loads in flight: a load from host memory takes over a microsecond
+            const U a = s[i], b = s[i + step], c = s[i + 2 * step], e = s[i + 3 * step];
+            store_through(d + i, a); store_through(d + i + step, b); store_through(d + i + 2 * step, c); store_through(d + i + 3 * step, e);
+        }
+        for (; i < units; i += step) store_through(d + i, s[i]);
+        if (sizeof(U) > 1 && blockIdx.x == 0 && p == parts.count - 1)
+            for (size_t k = units * sizeof(U) + threadIdx.x; k < n; k += THREADS) store_through(dst + k, src[k]);
+        if (parts.done[p]) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (threadIdx.x == 0) __hip_atomic_store(&parts.done[p][blockIdx.x], seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        begin = units;
     }
 }
 
-int launch_copy(const void* src, void* dst, size_t n, int max_wg, uint32_t* done, uint32_t seq, hipStream_t s, int* wgs) {
+int launch_copy(const void* src, void* dst, const Parts& parts, int max_wg, int units_per_thread, uint32_t seq, hipStream_t s, int* wgs) {
     const uintptr_t a = (uintptr_t)src | (uintptr_t)dst;
-    const size_t unit = a & 3 ? 1 : (a & 15 ? 4 : 16);
-    size_t g = (n / unit + 4 * THREADS - 1) / (4 * THREADS);
+    const size_t unit = a & 3 ? 1 : (a & 15 ? 4 : 16), per_wg = (size_t)units_per_thread * THREADS;
+    size_t g = (parts.end[0] / unit + per_wg - 1) / per_wg;
     g = g < 1 ? 1 : (g > (size_t)max_wg ? (size_t)max_wg : g);
     *wgs = (int)g;
     const uint8_t* from = (const uint8_t*)src;
     uint8_t* to = (uint8_t*)dst;
-    if (unit == 16) copy_kernel<u32x4><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
-    else if (unit == 4) copy_kernel<uint32_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
-    else copy_kernel<uint8_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, n, done, seq);
+    if (unit == 16) copy_kernel<u32x4><<<(unsigned)g, THREADS, 0, s>>>(from, to, parts, seq);
+    else if (unit == 4) copy_kernel<uint32_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, parts, seq);
+    else copy_kernel<uint8_t><<<(unsigned)g, THREADS, 0, s>>>(from, to, parts, seq);
     return fhip::check_hip(hipGetLastError(), "copy kernel");
+}
+int launch_copy(const void* src, void* dst, size_t n, int max_wg, uint32_t* done, uint32_t seq, hipStream_t s, int* wgs) {
+    return launch_copy(src, dst, Parts{1, {n}, {done}}, max_wg, 4, seq, s, wgs);
 }
 
 struct Slot {
     uint8_t* host = nullptr;     // SLOT_BYTES pinned: [OUT_BYTES][IN_BYTES]
     uint8_t* dev = nullptr;      // as much device memory (dequantization only)
-    uint32_t* done = nullptr;    // MAX_WG pinned words
+    uint32_t* done = nullptr;    // MAX_WG pinned words, of a copy in parts the last part's ...
+    uint32_t* early = nullptr;   // ... and (PARTS - 1) * MAX_WG for the parts before it
     uint32_t seq = 0;
     int wgs = 0;                 // words of `done` that have to reach seq before the GPU has read the slot
     bool held = false;
 
     bool read_by_gpu() const { return confirmed(seq, wgs); }
-    bool confirmed(uint32_t want, int n) const {
+    bool confirmed(uint32_t want, int n) const { return confirmed(done, want, n); }
+    static bool confirmed(const uint32_t* words, uint32_t want, int n) {
         for (int i = 0; i < n; i++)
-            if (__atomic_load_n(&done[i], __ATOMIC_ACQUIRE) != want) return false;
+            if (__atomic_load_n(&words[i], __ATOMIC_ACQUIRE) != want) return false;
         return true;
     }
 };
 
-// Until the first n words of the slot hold `want`: polled for two milliseconds (a decode step), then left to the runtime.
-int await_words(const Slot* q, uint32_t want, int n, hipStream_t s) {
+// Until the first n of the words hold `want`: polled for two milliseconds (a decode step), then left to the runtime.
+int await_words(const uint32_t* words, uint32_t want, int n, hipStream_t s) {
     const auto start = std::chrono::steady_clock::now();
-    for (unsigned i = 0; !q->confirmed(want, n); i++) {
+    for (unsigned i = 0; !Slot::confirmed(words, want, n); i++) {
 #if defined(__x86_64__)
         __builtin_ia32_pause();
 #endif
@@ -130,11 +147,12 @@ struct Ring {                    // one per device
             Slot& q = slot[i];
             if (q.held || !q.read_by_gpu()) continue;
             if (!words) {
-                if ((*rc = fhip::check_hip(hipHostMalloc((void**)&words, SLOTS * MAX_WG * sizeof(uint32_t), hipHostMallocPortable), "hipHostMalloc"))) return nullptr;
-                memset(words, 0, SLOTS * MAX_WG * sizeof(uint32_t));
+                if ((*rc = fhip::check_hip(hipHostMalloc((void**)&words, SLOTS * PARTS * MAX_WG * sizeof(uint32_t), hipHostMallocPortable), "hipHostMalloc"))) return nullptr;
+                memset(words, 0, SLOTS * PARTS * MAX_WG * sizeof(uint32_t));
             }
             if (!q.host && (*rc = fhip::check_hip(hipHostMalloc((void**)&q.host, SLOT_BYTES, hipHostMallocPortable), "hipHostMalloc"))) { q.host = nullptr; return nullptr; }
-            q.done = words + i * MAX_WG;
+            q.done = words + i * PARTS * MAX_WG;
+            q.early = q.done + MAX_WG;
             q.held = true;
             q.wgs = 0;
             return &q;
@@ -300,7 +318,7 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* co
         j.launched.store(n_begun);
         const bool helped = w.post(&j);
         for (size_t c = 0; c < n_begun && !helped && !rc; c++)
-            if (!(rc = await_words(begun[c], want[c], words[c], streams[0]))) (void)go_down(&j, c);
+            if (!(rc = await_words(begun[c]->done, want[c], words[c], streams[0]))) (void)go_down(&j, c);
         auto wait_for = [&](auto ready) {       // also looks for a device error every few milliseconds: what waits here would wait for ever
             auto look = std::chrono::steady_clock::now();
             for (Pause pause; !ready() && !rc;) {
@@ -329,7 +347,7 @@ int run_chunks(Ring* r, Job& j, hipStream_t* streams, size_t n_streams, Slot* co
             if (rc || (rc = launch(c, q, s, &wgs))) break;
             want[c] = ++q->seq; words[c] = q->wgs = wgs;
             j.launched.store(c + 1, std::memory_order_release);
-            if (!helped && !(rc = await_words(q, want[c], wgs, s))) (void)go_down(&j, c);
+            if (!helped && !(rc = await_words(q->done, want[c], wgs, s))) (void)go_down(&j, c);
         }
         if (j.down && !rc) wait_for([&] { return j.left.load() >= j.count; });
         if (rc) j.abort.store(1);
@@ -441,26 +459,31 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
             if (!(rc = launch(n_begun++, q, s, &wgs))) { q->seq++; q->wgs = wgs; }
         }
         if (!rc && !n_begun) return copy_d2h_plain(h, d, n, s);
-        if (!rc) rc = await_words(begun[0], begun[0]->seq, begun[0]->wgs, s);
+        if (!rc) rc = await_words(begun[0]->done, begun[0]->seq, begun[0]->wgs, s);
         if (!rc) return run_chunks(r, j, &s, 1, begun, n_begun, launch);
         (void)hipStreamSynchronize(s);              // an enqueued chunk may still use a slot
         for (size_t i = 0; i < n_begun; i++) r->release(begun[i]);
         return rc;
     }
-    // one part, or two thirds and the rest (where a second slot is free: nobody waits for one while holding one)
-    Slot* half[2] = {r->get(&rc), nullptr};
-    if (!half[0]) return rc ? rc : copy_d2h_plain(h, d, n, s);
-    if (n >= TWO_PARTS && !(half[1] = r->take(&rc)) && rc) { r->release(half[0]); return rc; }
-    const size_t first = half[1] ? (n / 3 * 2 + 255) & ~(size_t)255 : n;
-    int words[2] = {0, 0};
-    for (int i = 0; i < (first < n ? 2 : 1) && !rc; i++) {
-        Slot* q = half[i];
-        if (!(rc = launch_copy(from + (i ? first : 0), q->host, i ? n - first : first, MAX_WG, q->done, q->seq + 1, s, &wgs))) { q->seq++; q->wgs = words[i] = wgs; }
+    Slot* q = r->get(&rc);
+    if (!q) return rc ? rc : copy_d2h_plain(h, d, n, s);
+    // The host copies out at 30 GB/s what crosses at 53, so the total is the first part's way over and the host's whole copy: parts of 60 KB, at least four. A
+    // kernel of two thirds and one of the rest | four parts | eight, us on an idle device: 125 KB 15.4 | 13.3 | 16.6, 250 KB 19.3 | 16.5 | 17.7, 432 KB 25.0 |
+    // 22.8 | 21.7, 593 KB 31.5 | 28.4 | 26.1, 976 KB 45.4 | 41.5 | 39.0.
+    const size_t by_size = n / ((size_t)60 << 10);
+    Parts parts{n < IN_PARTS ? 1 : by_size < 4 ? 4 : by_size < PARTS ? (int)by_size : PARTS, {}, {}};
+    for (int p = 0; p < parts.count; p++) {
+        const bool last = p == parts.count - 1;
+        parts.end[p] = last ? n : (n / parts.count * (p + 1) + 255) & ~(size_t)255;
+        parts.done[p] = last ? q->done : q->early + p * MAX_WG;
     }
-    for (int i = 0; i < 2 && half[i] && !rc; i++)
-        if (!(rc = await_words(half[i], half[i]->seq, words[i], s))) memcpy((uint8_t*)h + (i ? first : 0), half[i]->host, i ? n - first : first);
-    for (Slot* q : half)
-        if (q) r->release(q);
+    const uint32_t seq = q->seq + 1;
+    if (!(rc = launch_copy(from, q->host, parts, MAX_WG, 1, seq, s, &wgs))) { q->seq = seq; q->wgs = wgs; }
+    for (int p = 0; p < parts.count && !rc; p++) {
+        const size_t begin = p ? parts.end[p - 1] : 0;
+        if (!(rc = await_words(parts.done[p], seq, wgs, s))) memcpy((uint8_t*)h + begin, q->host + begin, parts.end[p] - begin);
+    }
+    r->release(q);
     return rc;
 }
 
@@ -518,7 +541,7 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
     memcpy(q->host + OUT_BYTES, h_raw, nb * bytes);
     if (!(rc = launch(0, q, r->stream[0], &wgs))) {
         q->seq++; q->wgs = wgs;
-        if (!(rc = await_words(q, q->seq, wgs, r->stream[0]))) memcpy(h_out, q->host, n);
+        if (!(rc = await_words(q->done, q->seq, wgs, r->stream[0]))) memcpy(h_out, q->host, n);
     }
     r->release(q);
     return rc;

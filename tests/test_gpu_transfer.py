@@ -13,7 +13,7 @@ KIB, MIB = 1 << 10, 1 << 20
 
 
 # one byte, tails of the 16-byte units, a slot's way up (640 KiB) and way down (1 MiB) and one byte on either side, more chunks
-# than a copy holds slots (12); a copy back is made in two parts from 96 KiB on (64 + offset bytes are added to n)
+# than a copy holds slots (12); a copy back is made in parts from 96 KiB on (64 + offset bytes are added to n)
 @pytest.mark.parametrize("n", [1, 3, 15, 17, 4096, 64 * KIB + 5, 96 * KIB - 65, 96 * KIB - 64, 96 * KIB + 1, 640 * KIB - 1, 640 * KIB, 640 * KIB + 1, MIB - 65, MIB - 64, MIB - 63, 2 * MIB + 1,
                                6 * MIB + 7, 21 * MIB + 4])
 @pytest.mark.parametrize("offset", [0, 1, 4])
