@@ -288,6 +288,10 @@ size_t f16x2_matmul_ws(const fhip_weight* w, size_t t) {
 // deferred: the ordered sum of K-split groups is left to the reader of y, which gets *deferred as its `src`
 int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
                  fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
+    if (!swiglu_in && !src && fhip::gemm_f16x2_held(w, d_x, t, d_y)) {
+        if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0, 0, 128};
+        return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
+    }
     uint16_t* xp = (uint16_t*)d_ws;
     const bool ordered = w->batch_policy == FHIP_BATCH_ORDERED;
     float* part = ordered && fhip::gemm_f16x2_part_bytes(w, t) ? (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))) : nullptr;

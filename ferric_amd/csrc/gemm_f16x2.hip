@@ -42,6 +42,7 @@
 namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -953,6 +954,247 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROW
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The same arithmetic with a weight row's whole K inside one workgroup: no operand rows prepared by a launch of their own, no partial sums
+// in memory, no launch that adds them. Chunk ck belongs to wave ck % (waves of the workgroup), which makes the chunk's operand rows once
+// (the bits are xsplit_f16_kernel's) and keeps them in registers for all the tiles of 16 weight rows the workgroup goes through; the waves' sums
+// meet in LDS and are added in the waves' order. A wave's weight bytes are fetched as in the row-streaming kernel, contiguous lanes on contiguous
+// bytes into its own LDS image, its chunks of the next tile in flight through all of a tile's arithmetic. Activation rows come in sets of 8 NT,
+// blockIdx.y their number: with few tiles the sets of a batch go to workgroups of their own, which read the weights again, from the caches.
+//
+// What bounds it: at few tiles a chain, the load of the rows, three trips through LDS and the first weights from HBM (4.5 us with one
+// chunk a wave, 9 with 16 waves, 11 with two chunks, of which about 2 are the launch); at many the unpacking, as in the kernels above. Hence as many
+// waves as there are chunks up to 16, and 12 with two chunks each where all are at work at once; and hence no branch and no conditional value among
+// the loads: each one costs a wait for all loads before it (Q4_K 5120 x 2048 at 8 rows with such branches 12.4 us, without 7.6), and rows loaded in
+// fragment order, 16 bytes to a lane from as many lines, cost the address unit 4 us more than rows loaded whole and turned in LDS.
+// 8 rows, cold weights, us, before (two or three launches) | now: Q4_K 2000 x 1024 8.8 | 4.8, 4096 x 4096 13.3 | 9.3, 12000 x 3072 18.7 | 10.8,
+// 34000 x 2048 24.4 | 16.2; Q6_K 4096 x 4096 13.4 | 9.5, 34000 x 3072 38.4 | 27.1; Q8_0 4096 x 4096 13.9 | 9.1, 34000 x 4096 58.1 | 41.8.
+// 16 rows: Q4_K 2000 x 2048 12.9 | 6.4, 4096 x 4096 17.3 | 11.1, Q8_0 12000 x 3072 31.6 | 21.0. 32 rows: Q4_K 4096 x 4096 27.9 | 13.9.
+// NT: sets of eight activation rows in one workgroup; C: chunks a wave holds (32 NT C registers of operands); WV: waves at most; EU: waves to a SIMD.
+// ------------------------------------------------------------------------------------------------
+struct HeldParams {
+    const uint8_t* W;
+    const float* X;       // [T, K]
+    float* Y;             // [T, N]
+    int T, N, K, nchunks, nblk, tiles, nw, like_rows;   // nw: waves of a workgroup
+    size_t row_bytes;
+};
+template <class F, int NT, int C, int WV, int EU>
+__global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldParams p) {
+    const bool like_rows = F::ROWS_AT_16 || p.like_rows;        // a chunk's expression is the row-streaming kernel's, or that of the kernel above it
+    const int t0 = blockIdx.y * (8 * NT);                       // first activation row of the workgroup
+    const float* const X = p.X + (size_t)t0 * p.K;
+    float* const Y = p.Y + (size_t)t0 * p.N;
+    const int T = p.T - t0;
+    constexpr int WP = 16 * F::PARTS, NW = (WP + 63) / 64, NTL = (16 * F::TAILS + 63) / 64;
+    constexpr int XROW = 4 * CHUNK + 16, AROW = 2 * CHUNK + 16; // bytes of a staged activation row and of an operand row: the 16 keep rows on different banks
+    constexpr int IMAGE = 16 * F::LROW > 16 * AROW ? 16 * F::LROW : 16 * AROW;
+    static_assert(8 * XROW <= IMAGE, "eight activation rows fit the image");
+    __shared__ __attribute__((aligned(16))) uint8_t Wl[WV][IMAGE];
+    __shared__ float Ps[2][WV][8 * NT][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = p.nw;                                        // (blockDim is a load from memory, whose wait would be one for all the loads before it)
+    const int g4 = lane >> 4, c = lane & 15;
+    uint8_t* const wl = Wl[wave];
+
+    u32x4 G[C][NW];
+    uint32_t gt[C][NTL ? NTL : 1];
+    auto part = [&](int k) { const int pc = k * 64 + lane; return pc < WP ? pc : WP - 1; };
+    auto tail = [&](int k) { const int tc = k * 64 + lane; return tc < 16 * F::TAILS ? tc : 16 * F::TAILS - 1; };
+    auto load_w = [&](int tile, int i) {                       // rows past the end of the weight repeat its last row
+        // (no branch: behind one, a wait would be for every load. What is past the end loads again what another lane or wave has loaded)
+        const int mine = wave + nw * i, ck = mine < p.nchunks ? mine : p.nchunks - 1, row0 = tile * 16, rmax = p.N - 1 - row0;
+        const uint8_t* b = p.W + (size_t)row0 * p.row_bytes;
+#pragma unroll
+        for (int k = 0; k < NW; k++) {
+            const int pc = part(k), row = pc / F::PARTS;
+            const uint32_t off = (uint32_t)(row < rmax ? row : rmax) * (uint32_t)p.row_bytes + F::piece_off(ck, pc - row * F::PARTS, p.nblk);
+            G[i][k] = F::ldg(b + off);
+        }
+#pragma unroll
+        for (int k = 0; k < NTL; k++) {
+            const int tc = tail(k), row = tc / (F::TAILS ? F::TAILS : 1);
+            bool live;
+            const uint32_t off = (uint32_t)(row < rmax ? row : rmax) * (uint32_t)p.row_bytes + F::tail_off(ck, tc - row * F::TAILS, p.nblk, live);
+            gt[i][k] = *(const uint16_t*)(b + off);
+        }
+    };
+    auto park_w = [&](int i) {
+#pragma unroll
+        for (int k = 0; k < NW; k++) {
+            const int pc = part(k), row = pc / F::PARTS;
+            *(u32x4*)(wl + row * F::LROW + F::piece_lds(pc - row * F::PARTS)) = G[i][k];
+        }
+#pragma unroll
+        for (int k = 0; k < NTL; k++) {
+            const int tc = tail(k), row = tc / (F::TAILS ? F::TAILS : 1);
+            bool live;
+            F::tail_off(wave + nw * i, tc - row * F::TAILS, p.nblk, live);
+            *(uint16_t*)(wl + row * F::LROW + F::tail_lds(tc - row * F::TAILS)) = live ? (uint16_t)gt[i][k] : (uint16_t)0;
+        }
+    };
+    auto mine = [&](int i) { return wave + nw * i < p.nchunks; };   // wave-uniform
+    f32x4 xr[C][NT][8];                                         // a chunk's 256 columns of a row, four to a lane
+#pragma unroll
+    for (int i = 0; i < C; i++)
+#pragma unroll
+        for (int q = 0; q < NT; q++)
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                const int t = 8 * q + r, k = (wave + nw * i) * CHUNK + 4 * lane;
+                xr[i][q][r] = *(const f32x4*)(X + (size_t)(t < T ? t : 0) * p.K + (k < p.K ? k : 0));   // (no branch: one would wait for every load)
+            }
+    asm volatile("" ::: "memory");                              // the rows are waited for first, the weights only once they are due
+#pragma unroll
+    for (int i = 0; i < C; i++) load_w(blockIdx.x, i);
+    asm volatile("" ::: "memory");
+
+    // ---- operand rows of the wave's chunks: row c of a set is the hi (c < 8) or lo part of activation row c & 7
+    f16x8 a[C][NT][8], am[C][NT];
+    float e[C][NT][4];                                          // what takes the chunk's scale out of operand rows 4 g4 + r again
+    const int row = lane >> 3, sub = lane & 7;                  // the 32 columns of an activation row that this lane cuts
+#pragma unroll
+    for (int i = 0; i < C; i++)
+#pragma unroll
+        for (int q = 0; q < NT; q++) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int r = 0; r < 8; r++) {                       // a row's 16-byte pieces, the eight of a sub-block turned by its number
+                const bool in = 8 * q + r < T && (wave + nw * i) * CHUNK + 4 * lane < p.K;
+                *(f32x4*)(wl + r * XROW + 16 * (lane ^ (lane >> 3))) = in ? xr[i][q][r] : (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            f32x4 v[8];
+            float m = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = *(const f32x4*)(wl + row * XROW + 16 * (8 * sub + (j ^ sub)));
+            // (a NaN is not the largest magnitude: it reaches the operands as it is)
+#pragma unroll
+            for (int j = 0; j < 8; j++) m = fmaxf(m, fmaxf(fmaxf(fabsf(v[j][0]), fabsf(v[j][1])), fmaxf(fabsf(v[j][2]), fabsf(v[j][3]))));
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+            float sc, inv;
+            chunk_scale(m, sc, inv);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                f16x8 hi, low;
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const float x = v[j + (k >> 2)][k & 3] *= sc;
+                    hi[k] = (_Float16)x;
+                    low[k] = (_Float16)(x - (float)hi[k]);
+                }
+                *(f16x8*)(wl + row * AROW + 64 * sub + 8 * j) = hi;
+                *(f16x8*)(wl + (row + 8) * AROW + 64 * sub + 8 * j) = low;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const _Float16* ar = (const _Float16*)(wl + c * AROW);
+#pragma unroll
+            for (int I = 0; I < 8; I++) {                       // eight columns in the order of src_k: two fours, each in an order of its own
+                const f16x4 l = *(const f16x4*)(ar + F::src_k((I * 4 + g4) * 8)), u = *(const f16x4*)(ar + F::src_k((I * 4 + g4) * 8 + 4));
+                constexpr int O[8] = {F::src_k(0), F::src_k(1), F::src_k(2), F::src_k(3), F::src_k(4) - F::src_k(4) + 4, F::src_k(5) - F::src_k(4) + 4,
+                                      F::src_k(6) - F::src_k(4) + 4, F::src_k(7) - F::src_k(4) + 4};
+                a[i][q][I] = __builtin_shufflevector(l, u, O[0], O[1], O[2], O[3], O[4], O[5], O[6], O[7]);
+            }
+            if constexpr (F::HAS_MIN) {
+                // the sub-block's sum in the order of xsplit's exchanges: columns 16, 8, 4, 2, 1 apart
+                f32x4 w[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) w[j] = v[j] + v[j + 4];
+                w[0] += w[2]; w[1] += w[3];
+                w[0] += w[1];
+                const float s = ((w[0][0] + w[0][2]) + (w[0][1] + w[0][3])) * 0.015625f;
+                const _Float16 sh = (_Float16)s, sl = (_Float16)(s - (float)sh);
+                const int both = __builtin_bit_cast(unsigned short, sh) | __builtin_bit_cast(unsigned short, sl) << 16;
+#pragma unroll
+                for (int k = 0; k < 8; k++) {                   // k-group 0 holds the eight sums, the others zeros
+                    const unsigned w2 = (unsigned)__shfl(both, 8 * (c & 7) + k);
+                    am[i][q][k] = g4 == 0 ? __builtin_bit_cast(_Float16, (unsigned short)(c >= 8 ? w2 >> 16 : w2)) : (_Float16)0.f;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) e[i][q][r] = __shfl(inv, 8 * ((4 * g4 + r) & 7));
+        }
+
+    int buf = 0;
+    auto one_tile = [&](int tile, auto Next) {                  // Next: there is another tile after this one
+        f32x4 total[NT];
+#pragma unroll
+        for (int q = 0; q < NT; q++) total[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the image is the wave's own: its accesses complete in order
+            park_w(i);
+            if constexpr (decltype(Next)::value) load_w(tile + gridDim.x, i);
+            if (!mine(i)) continue;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            typename F::Raw raw;
+            F::from_lds(raw, wl + c * F::LROW, g4);
+            typename F::Ctx x;
+            f32x4 acc[NT], ct[NT];
+            float dprev = 0.f;
+#pragma unroll
+            for (int q = 0; q < NT; q++) { acc[q] = (f32x4){0.f, 0.f, 0.f, 0.f}; ct[q] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
+            static_for<0, 8>([&](auto Ic) {
+                constexpr int I = decltype(Ic)::value;
+                F::template pre<I>(raw, g4, x);
+                const f16x8 b = F::template frag<I>(raw, x);
+                if constexpr (F::SLICE_SCALE) {                 // as in the row-streaming kernel
+                    f32x4 cur[NT];
+#pragma unroll
+                    for (int q = 0; q < NT; q++) cur[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][q][I], b, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    if constexpr (I > 0) {
+#pragma unroll
+                        for (int q = 0; q < NT; q++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) ct[q][r] = fmaf(dprev, acc[q][r], ct[q][r]);
+                    }
+#pragma unroll
+                    for (int q = 0; q < NT; q++) acc[q] = cur[q];
+                    dprev = x.d;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < NT; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][q][I], b, acc[q], 0, 0, 0);
+                }
+            });
+            if constexpr (F::HAS_MIN) {
+                const f16x8 bm = F::mins(raw, g4);
+#pragma unroll
+                for (int q = 0; q < NT; q++) {
+                    const f32x4 accm = __builtin_amdgcn_mfma_f32_16x16x32_f16(am[i][q], bm, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) ct[q][r] = like_rows ? fmaf(x.dm, accm[r], ct[q][r]) : accm[r];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < NT; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    total[q][r] = fmaf(e[i][q][r], like_rows ? fmaf(x.d, acc[q][r], ct[q][r]) : fmaf(x.dm, ct[q][r], acc[q][r] * x.d), total[q][r]);
+        }
+        // lanes g4 and g4 ^ 2 hold the hi and the lo part of the same output
+#pragma unroll
+        for (int q = 0; q < NT; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float v = total[q][r] + __shfl_xor(total[q][r], 32);
+                if (g4 < 2) Ps[buf][wave][8 * q + 4 * g4 + r][c] = v;
+            }
+        __syncthreads();
+        for (int o = tid; o < 8 * NT * 16; o += 64 * nw) {
+            const int t = o >> 4, n = tile * 16 + (o & 15);
+            float v = Ps[buf][0][t][o & 15];
+            for (int w = 1; w < nw; w++) v += Ps[buf][w][t][o & 15];
+            if (t < T && n < p.N) Y[(size_t)t * p.N + n] = v;
+        }
+        buf ^= 1;
+    };
+    int tile = blockIdx.x;
+    for (; tile + (int)gridDim.x < p.tiles; tile += gridDim.x) one_tile(tile, std::true_type{});
+    one_tile(tile, std::false_type{});
+}
+
 // Ordered mode: group `blockIdx.x` of `group` (128 or 256) outputs, if more than one workgroup held part of its K: Y = slot 0 + slot 1 + ...
 // in that order. Thread = output column (threadIdx.x & 127) of activation row 2 * blockIdx.y + (threadIdx.x >> 7).
 __global__ void __launch_bounds__(256) sum_split_kernel(float* __restrict__ Y, const float* __restrict__ part, int T, int N, int nchunks,
@@ -1086,9 +1328,79 @@ int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, siz
     return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
 }
 
+template <class F>
+int launch_held_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
+    HeldParams p;
+    p.W = w->d_raw; p.X = d_x; p.Y = d_y;
+    p.T = (int)t; p.N = (int)w->rows; p.K = (int)w->cols; p.nblk = (int)(w->cols / 32);
+    p.nchunks = (int)((w->cols + CHUNK - 1) / CHUNK);
+    p.tiles = (int)((w->rows + 15) / 16);
+    p.row_bytes = w->row_bytes;
+    const int cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+    // Both sets of 9..16 rows in one workgroup where the tiles alone fill the chip several times over: 16 rows, us, apart | together:
+    // 34000 x 4096 Q4_K 40.7 | 36.4, Q8_0 64.0 | 50.5, but 12000 x 3072 Q4_K 14.6 | 19.2, 2000 x 4096 Q8_0 9.0 | 14.9
+    const bool two = t > 8 && t <= 16 && p.nchunks <= 16 && p.tiles > 4 * cus;
+    const int sets = two ? 1 : (int)((t + 7) / 8);
+    // waves: one a chunk up to 16 (4096 x 4096 Q8_0 at 8 rows 10.2 us, 11.9 with eight of two chunks each); beyond, 12 with two chunks each while
+    // every workgroup has a CU to itself (2000 x 5120 Q6_K 11.8 us against 12.9), eight with three chunks and no spill where
+    // they go through several tiles (12000 x 6144 Q8_0 25.9 us against 28.0)
+    const int most = two || p.nchunks <= 8 ? 8 : p.nchunks <= 16 ? 16 : p.tiles * sets <= cus ? 12 : 8;
+    const int held = (p.nchunks + most - 1) / most;
+    p.nw = (p.nchunks + held - 1) / held;
+    p.like_rows = t <= 8;
+    // one workgroup a CU; two of eight waves where there are many tiles (34000 x 2048 Q6_K 19.3 us against 21.6, but 5120 x 2048 9.9 against 8.7)
+    int slots = cus * (!two && held == 1 && most == 8 && p.tiles * sets > 4 * cus ? 2 : 1) / sets;
+    if (slots < 1) slots = 1;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles < slots ? p.tiles : slots), (unsigned)sets), dim3(64 * p.nw), 0, s, p); };
+    if (two) {
+        if (held == 1) go(gemm_q_f16x2_held_kernel<F, 2, 1, 8, 2>);
+        else go(gemm_q_f16x2_held_kernel<F, 2, 2, 8, 2>);
+    } else if (most == 16) go(gemm_q_f16x2_held_kernel<F, 1, 1, 16, 4>);
+    else if (most == 12) go(gemm_q_f16x2_held_kernel<F, 1, 2, 12, 3>);
+    else if (held == 1) go(gemm_q_f16x2_held_kernel<F, 1, 1, 8, 4>);
+    else go(gemm_q_f16x2_held_kernel<F, 1, 3, 8, 2>);
+    return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
+}
+
 }  // namespace
 
 namespace fhip {
+
+// Where the held kernel is the faster one, us, the other kernels | it:
+// - up to 16 chunks (4096 columns) nearly always (the figures at the kernel). Not with one chunk and more than two tiles a CU, where the streaming
+//   kernel is one launch as well (8 rows, 12000 x 256 Q4_K 5.3 | 6.3; 8000 x 256 5.3 | 5.2), and at more than 8 rows of a tall weight not
+//   where the other kernels cut nothing along K (34000 x 512 Q4_K at 24 rows 16.8 | 18.3, Q5_K at 16 13.7 | 16.6).
+// - 17 to 24 chunks, two or three of them one after the other in a wave: 8 rows from half a tile a CU on (600 x 5120 Q4_K 9.4 | 11.3, 2000 x 5120
+//   11.9 | 11.8, 4096 x 5120 14.4 | 12.4) but for the first quarter of a second pass (4600 x 5120 14.7 | 15.6, 5120 x 5120 16.4 | 15.4); 9..16
+//   rows from a quarter of a tile a CU (2000 x 5120 16.0 | 12.4) to four (34000 x 5120 54.8 | 56.5); more rows of a format with minima, whose other
+//   kernel is the slower one, to two (600 x 5120 Q4_K at 32 17.8 | 11.8, 8000 41.6 | 30.8, 34000 83.7 | 97.9), of Q6_K while the sets
+//   of all tiles are two and a half a CU (3000 x 5120 at 24 23.5 | 19.4, 4096 22.0 | 22.8).
+bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+    if (!gemm_f16x2_supports(w, t) || !d_x || ((uintptr_t)d_x & 15) != 0 || w->rows > 0x7FFFFF00ull) return false;
+    // (all workgroups read the rows: none may have written over them)
+    if ((uintptr_t)d_y < (uintptr_t)(d_x + t * w->cols) && (uintptr_t)d_x < (uintptr_t)(d_y + t * w->rows)) return false;
+    const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16, sets = (t + 7) / 8;
+    const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+    if (chunks == 1) { if (tiles > 2 * cus) return false; }
+    else if (chunks > 24) return false;
+    else if (chunks > 16) {
+        if (t <= 8) return 2 * tiles >= cus && (tiles <= cus || 4 * tiles >= 5 * cus);
+        if (t <= 16) { if (4 * tiles < cus || tiles > 4 * cus) return false; }
+        else if (w->type == FHIP_Q6_K ? 2 * tiles * sets > 5 * cus : tiles > 2 * cus) return false;
+    }
+    return t <= 8 || tiles <= 4 * cus || make_plan(w, t).split;
+}
+
+int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
+    if (t == 0 || w->rows == 0) return FHIP_OK;
+    switch (w->type) {
+        case FHIP_Q4_K: return launch_held_fmt<Q4K>(w, d_x, t, d_y, s);
+        case FHIP_Q5_K: return launch_held_fmt<Q5K>(w, d_x, t, d_y, s);
+        case FHIP_Q6_K: return launch_held_fmt<Q6K>(w, d_x, t, d_y, s);
+        case FHIP_Q8_0: return launch_held_fmt<Q80>(w, d_x, t, d_y, s);
+        default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "f16x2 matmul: no kernel for ggml type %u", w->type);
+    }
+}
 
 bool gemm_f16x2_supports(const fhip_weight* w, size_t t) {
     if (!w || t < 1 || w->cols == 0 || w->cols > (size_t)MAXW * 1024) return false;
