@@ -60,7 +60,13 @@ __device__ __forceinline__ uint32_t hadd2(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, a) + __builtin_bit_cast(f16x2, b));
 }
 __device__ __forceinline__ uint32_t splat_h(_Float16 h) { return __builtin_bit_cast(uint32_t, (f16x2){h, h}); }
-__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t o) { return (a & m) | o; }
+// (a & m) | o in one instruction, its constants in registers: written out, the compiler takes two with a literal each, and these are
+// a fifth of what a weight costs to unpack (8 rows: Q5_K 12000 x 5120 21.8 -> 20.2 us, Q4_K 34000 x 5120 34.9 -> 33.0, Q6_K 5120 x 17408 32.9 -> 32.2)
+__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t o) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(o));
+    return r;
+}
 
 constexpr uint32_t H1024 = 0x64006400u;      // f16 pair (1024, 1024): mantissa step 1
 constexpr uint32_t H64 = 0x54005400u;        // f16 pair (64, 64): mantissa step 1/16
@@ -243,10 +249,10 @@ struct Q5K {
         const uint32_t w = I < 4 ? r.q0[I & 3] : r.q1[I & 3], w8 = w >> 8;
         const uint32_t hb = (I < 4 ? r.h0[I & 3] : r.h1[I & 3]) >> x.sh;
         u32x4 o;
-        o[0] = hfma2(and_or(w, 0x000F000Fu, H1024) | ((hb << 4) & 0x00100010u), x.s0, x.c0);
-        o[1] = hfma2(and_or(w8, 0x000F000Fu, H1024) | ((hb >> 4) & 0x00100010u), x.s0, x.c0);
-        o[2] = hfma2(and_or(w, 0x00F000F0u, H1024) | ((hb << 7) & 0x01000100u), x.s1, x.c1);
-        o[3] = hfma2(and_or(w8, 0x00F000F0u, H1024) | ((hb >> 1) & 0x01000100u), x.s1, x.c1);
+        o[0] = hfma2(and_or(hb << 4, 0x00100010u, and_or(w, 0x000F000Fu, H1024)), x.s0, x.c0);
+        o[1] = hfma2(and_or(hb >> 4, 0x00100010u, and_or(w8, 0x000F000Fu, H1024)), x.s0, x.c0);
+        o[2] = hfma2(and_or(hb << 7, 0x01000100u, and_or(w, 0x00F000F0u, H1024)), x.s1, x.c1);
+        o[3] = hfma2(and_or(hb >> 1, 0x01000100u, and_or(w8, 0x00F000F0u, H1024)), x.s1, x.c1);
         return __builtin_bit_cast(f16x8, o);
     }
     static __device__ __forceinline__ f16x8 mins(const Raw& r, int g4) {
@@ -1044,9 +1050,11 @@ __global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldPara
                 const int t = 8 * q + r, k = (wave + nw * i) * CHUNK + 4 * lane;
                 xr[i][q][r] = *(const f32x4*)(X + (size_t)(t < T ? t : 0) * p.K + (k < p.K ? k : 0));   // (no branch: one would wait for every load)
             }
+    constexpr bool LATE_W = WV == 12;                           // only once the first chunk's rows have left their registers (1500 x 6144 Q4_K at 16 rows 12.9 us, 13.8 before)
     asm volatile("" ::: "memory");                              // the rows are waited for first, the weights only once they are due
 #pragma unroll
-    for (int i = 0; i < C; i++) load_w(blockIdx.x, i);
+    for (int i = 0; i < C; i++)
+        if (!LATE_W) load_w(blockIdx.x, i);
     asm volatile("" ::: "memory");
 
     // ---- operand rows of the wave's chunks: row c of a set is the hi (c < 8) or lo part of activation row c & 7
@@ -1064,6 +1072,12 @@ __global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldPara
                 *(f32x4*)(wl + r * XROW + 16 * (lane ^ (lane >> 3))) = in ? xr[i][q][r] : (f32x4){0.f, 0.f, 0.f, 0.f};
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (LATE_W && i + q == 0) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < C; j++) load_w(blockIdx.x, j);
+                asm volatile("" ::: "memory");
+            }
             f32x4 v[8];
             float m = 0.f;
 #pragma unroll
