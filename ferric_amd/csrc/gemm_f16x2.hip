@@ -973,9 +973,9 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROW
 // waves as there are chunks up to 16, and 12 with two chunks each where all are at work at once; and hence no branch and no conditional value among
 // the loads: each one costs a wait for all loads before it (Q4_K 5120 x 2048 at 8 rows with such branches 12.4 us, without 7.6), and rows loaded in
 // fragment order, 16 bytes to a lane from as many lines, cost the address unit 4 us more than rows loaded whole and turned in LDS.
-// 8 rows, cold weights, us, before (two or three launches) | now: Q4_K 2000 x 1024 8.8 | 4.8, 4096 x 4096 13.3 | 9.3, 12000 x 3072 18.7 | 10.8,
-// 34000 x 2048 24.4 | 16.2; Q6_K 4096 x 4096 13.4 | 9.5, 34000 x 3072 38.4 | 27.1; Q8_0 4096 x 4096 13.9 | 9.1, 34000 x 4096 58.1 | 41.8.
-// 16 rows: Q4_K 2000 x 2048 12.9 | 6.4, 4096 x 4096 17.3 | 11.1, Q8_0 12000 x 3072 31.6 | 21.0. 32 rows: Q4_K 4096 x 4096 27.9 | 13.9.
+// 8 rows, cold weights, us, before (two or three launches) | now: Q4_K 2000 x 1024 8.8 | 4.6, 4096 x 4096 13.3 | 8.9, 12000 x 3072 18.7 | 10.2,
+// 34000 x 2048 24.4 | 15.8; Q6_K 4096 x 4096 13.4 | 8.9, 34000 x 3072 38.4 | 26.9; Q8_0 4096 x 4096 13.9 | 8.9, 34000 x 4096 58.1 | 41.8.
+// 16 rows: Q4_K 2000 x 2048 12.9 | 6.1, 4096 x 4096 17.3 | 10.3, Q8_0 12000 x 3072 31.6 | 20.8. 32 rows: Q4_K 4096 x 4096 27.9 | 13.4.
 // NT: sets of eight activation rows in one workgroup; C: chunks a wave holds (32 NT C registers of operands); WV: waves at most; EU: waves to a SIMD.
 // ------------------------------------------------------------------------------------------------
 struct HeldParams {
