@@ -10,9 +10,9 @@
 //
 // Two kernels: causal_attn_cut_kernel, on bf16 matrix instructions with every f32 operand cut into three bf16 values, is what a caller gets;
 // causal_attn_kernel, on f32 matrix instructions, is what fhip_causal_attention_f32_products gives (prompts on a block-quantized cache:
-// the header says why). Measured, us, f32 -> cut, 40 query and 8 KV heads of 128: 509 rows x 809 keys 102.9 -> 71.7, 2048 x 2048 432 ->
-// 266, 512 x 8192 1163 -> 783; few workgroups: 39 x 929, 8 heads 85.7 -> 69.3; heads of 64: 512 x 512, 32 heads 31.7 -> 27.5, 49 x 49 7.0 ->
-// 6.3. Relative error against f64, same shapes: 5.6e-7 -> 4.5e-7, 4.5e-7 -> 3.7e-7, 1.65e-6 -> 1.41e-6, 6.8e-7 -> 5.6e-7, 2.7e-7 -> 2.0e-7,
+// the header says why). Measured, us, f32 -> cut, 40 query and 8 KV heads of 128: 509 rows x 809 keys 102.9 -> 72.6, 2048 x 2048 432 ->
+// 274, 512 x 8192 1163 -> 789; few workgroups: 39 x 929, 8 heads 85.7 -> 70.3; heads of 64: 512 x 512, 32 heads 31.7 -> 27.7, 49 x 49 7.0 ->
+// 6.8. Relative error against f64, same shapes: 5.6e-7 -> 4.5e-7, 4.5e-7 -> 3.7e-7, 1.65e-6 -> 1.41e-6, 6.8e-7 -> 5.6e-7, 2.7e-7 -> 2.0e-7,
 // 1.7e-7 -> 1.2e-7. What bounds the cut kernel: the chain of a tile (cut and store 32 keys, products, statistics, products: 2.2 us a wave
 // alone on its SIMD, of which 0.65 are MFMA) at one or two waves a SIMD.
 //
@@ -53,19 +53,18 @@ using fhip::pk_bf16;
 __device__ __forceinline__ void store_out(float* p, float4 v) { *(float4*)p = v; }
 __device__ __forceinline__ void store_out(uint16_t* p, float4 v) { *(uint2*)p = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
 
-// NW: waves (16 query rows each) per workgroup.
-template <int HD, int NW, typename Out>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
-                                                              int S, int n_head, int n_kv, float scale, int window, float softcap,
-                                                              Out* __restrict__ out) {
+// NW: waves (16 query rows each) per workgroup. STAGED: the workgroup's waves call it together and share the tiles in Ks [32][HD + 4] and Vs
+// [32][HD]. Otherwise a wave comes alone, waits for no other and takes its operands from memory: the same instructions on the same
+// values, the same bits, about three times the time.
+template <int HD, int NW, bool STAGED, typename Out>
+__device__ __forceinline__ void f32_body(float* Ks, float* Vs, const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T, int S, int n_head, int n_kv,
+                                         float scale, int window, float softcap, Out* __restrict__ out) {
     constexpr int KS = HD + 4;              // floats per K row in LDS
     constexpr int QD = HD / 4;              // dims per quarter
     constexpr int NDT = HD / 16;            // output tiles of 16 rows
     constexpr int QROWS = 16 * NW;          // query rows per workgroup
     constexpr int NF = 32 * (HD / 4) / (64 * NW);   // 16-byte pieces of a K (and of a V) tile per thread
     static_assert(NF >= 1 && NF * 64 * NW == 32 * (HD / 4), "the tile divides over the threads");
-    __shared__ __attribute__((aligned(16))) float Ks[32 * KS];
-    __shared__ __attribute__((aligned(16))) float Vs[32 * HD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, ks = lane >> 4;
     // Workgroups are handed out x first: all heads' last query blocks (which see the most keys), then all heads' second to
@@ -112,36 +111,36 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
         prow[n] = f / (HD / 4);
         pcol[n] = (f % (HD / 4)) * 4;
     }
-#pragma unroll
-    for (int n = 0; n < NF; n++) {
-        const size_t src = (size_t)min(kt_lo * 32 + prow[n], S - 1) * kv_stride + (size_t)pcol[n];
-        kreg[n] = *(const f32x4*)(Kh + src);
-        vreg[n] = *(const f32x4*)(Vh + src);
-    }
-    for (int kt = kt_lo; kt <= kt_hi; kt++) {
-        __syncthreads();                                        // every wave is done with the previous tile
-#pragma unroll
-        for (int n = 0; n < NF; n++) {
-            *(f32x4*)(Ks + prow[n] * KS + pcol[n]) = kreg[n];
-            *(f32x4*)(Vs + prow[n] * HD + pcol[n]) = vreg[n];
-        }
-        __syncthreads();
-        const int nxt = min(kt + 1, kt_hi);                     // in flight under this tile's arithmetic
+    auto request = [&](int kt) {
 #pragma unroll
         for (int n = 0; n < NF; n++) {
             // rows past the cache repeat its last row; they are masked below
-            const size_t src = (size_t)min(nxt * 32 + prow[n], S - 1) * kv_stride + (size_t)pcol[n];
+            const size_t src = (size_t)min(kt * 32 + prow[n], S - 1) * kv_stride + (size_t)pcol[n];
             kreg[n] = *(const f32x4*)(Kh + src);
             vreg[n] = *(const f32x4*)(Vh + src);
         }
-        if (kt < my_lo || kt > my_hi) continue;                 // wave-uniform; the barriers above are reached by every wave
+    };
+    if (STAGED) request(kt_lo);
+    for (int kt = STAGED ? kt_lo : my_lo; kt <= (STAGED ? kt_hi : my_hi); kt++) {
+        if constexpr (STAGED) {
+            __syncthreads();                                    // every wave is done with the previous tile
+#pragma unroll
+            for (int n = 0; n < NF; n++) {
+                *(f32x4*)(Ks + prow[n] * KS + pcol[n]) = kreg[n];
+                *(f32x4*)(Vs + prow[n] * HD + pcol[n]) = vreg[n];
+            }
+            __syncthreads();
+            request(min(kt + 1, kt_hi));                        // in flight under this tile's arithmetic
+            if (kt < my_lo || kt > my_hi) continue;             // wave-uniform; the barriers above are reached by every wave
+        }
 
         // the two halves' chains alternate, so an instruction does not wait for the result of the one before it
         f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-        const float* krow = Ks + c * KS + ks * QD;
+        const float* krow = STAGED ? Ks + c * KS + ks * QD : Kh + (size_t)min(kt * 32 + c, S - 1) * kv_stride + ks * QD;
+        const float* krow16 = STAGED ? krow + 16 * KS : Kh + (size_t)min(kt * 32 + 16 + c, S - 1) * kv_stride + ks * QD;
 #pragma unroll
         for (int t = 0; t < QD; t += 4) {
-            const float4 k0 = *(const float4*)(krow + t), k1 = *(const float4*)(krow + 16 * KS + t);
+            const float4 k0 = *(const float4*)(krow + t), k1 = *(const float4*)(krow16 + t);
             sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0.x, qf[t], sacc[0], 0, 0, 0);
             sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k1.x, qf[t], sacc[1], 0, 0, 0);
             sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0.y, qf[t + 1], sacc[0], 0, 0, 0);
@@ -189,7 +188,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
         for (int u = 0; u < 2; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float* vrow = Vs + (16 * u + 4 * ks + r) * HD + NDT * c;
+                const int key = 16 * u + 4 * ks + r;
+                const float* vrow = (STAGED ? Vs + key * HD : Vh + (size_t)min(kt * 32 + key, S - 1) * kv_stride) + NDT * c;
                 float va[NDT];
 #pragma unroll
                 for (int d = 0; d < NDT; d += 4) {
@@ -215,11 +215,30 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
     }
 }
 
+template <int HD, int NW, typename Out>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
+                                                              int S, int n_head, int n_kv, float scale, int window, float softcap,
+                                                              Out* __restrict__ out) {
+    __shared__ __attribute__((aligned(16))) float Ks[32 * (HD + 4)];    // floats per K row in LDS: four banks on from row to row
+    __shared__ __attribute__((aligned(16))) float Vs[32 * HD];
+    f32_body<HD, NW, true>(Ks, Vs, q, K, V, T, S, n_head, n_kv, scale, window, softcap, out);
+}
+
 // ------------------------------------------------------------------------------------------------------------------------------
 // The same on bf16 matrix instructions. An f32 value is three bf16 values exactly (the nearest to it, the nearest to what is left, and
 // what is left then), and a product of two f32 values is, to 2^-25, the six products of their cuts of which one factor at least is the
 // first or both the second: six v_mfma_f32_16x16x32_bf16 of 16 cycles for 32 columns of k, where v_mfma_f32_16x16x4_f32 needs eight of 32.
-// Every operand keeps its 24 bits, sums are f32.
+// Sums are f32. Every operand keeps its 24 bits: a third cut is whole down to bf16's smallest value, 2^-133, which values V is multiplied by
+// 2^40 for on the way (any f32 then has its last bit above that; exact, and taken off at the end). A query's or key's member under 2^-110
+// and a probability under 2^-110 lose what lies below 2^-134: nothing to a score that goes into an exponential, nor to a row of a sum over 1.
+//
+// What three cuts cannot carry: an infinite member, or one that rounds to infinity, leaves infinity less infinity in the cuts behind, a NaN
+// score has no weight in the f32 kernel, and sums near f32's limit can overflow in one cut and not in another. All of these leave a NaN or an
+// infinity in a sum of the wave's, or no weight at all, so a wave looks over its sums once at the end, and one that finds such a value does
+// its rows again on the f32 kernel's body: there the result is that kernel's, bit for bit. (A score one of whose partial sums passes f32's
+// limit downwards counts as one of no weight, as any order of an f32 sum may have it.) What the look and V's factor cost, us: 509 x 809 rows 71.6 -> 72.6,
+// 2048 x 2048 272 -> 274, 512 x 8192 777 -> 789, 49 x 49, heads of 64, 6.3 -> 6.8. The largest member kept tile by tile cost twice that (2048 x 2048 275,
+// and thirty-two registers unless forced out before the barrier).
 //
 // Tiles, masks and statistics are the f32 kernel's: a wave owns 16 query rows of one head, lane (c, ks), key tiles of 32 rows. K and V are
 // cut once a tile by the workgroup as they go to LDS, K as [plane][key][dim], V as [plane][dim][slot]: slot 8 ks + 4 u + i is key
@@ -252,6 +271,8 @@ __device__ __forceinline__ void mfma_cuts(const bf16x8 (&a)[N][3], const bf16x8 
 #pragma unroll
         for (int n = 0; n < N; n++) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n][A[x]], b[B[x]], acc[n], 0, 0, 0);
 }
+
+constexpr float V_UP = 0x1p40f;
 
 template <int HD, int NW, typename Out>
 __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
@@ -337,7 +358,7 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
                 } else {
 #pragma unroll
                     for (int d = 0; d < 4; d++) {
-                        const Cuts2 w0 = cut2(piece[x][0][d], piece[x][1][d]), w1 = cut2(piece[x][2][d], piece[x][3][d]);
+                        const Cuts2 w0 = cut2(piece[x][0][d] * V_UP, piece[x][1][d] * V_UP), w1 = cut2(piece[x][2][d] * V_UP, piece[x][3][d] * V_UP);
 #pragma unroll
                         for (int y = 0; y < 3; y++) *(uint2*)(Vs + y * VP + dst[x] + d * VROW) = make_uint2(w0.w[y], w1.w[y]);
                     }
@@ -412,8 +433,18 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    if (!wave_live || i0 + c >= T) return;
-    const float inv = 1.0f / l;
+    if (!wave_live) return;
+    float top = l > 0.f ? l : INFINITY;
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) top = __builtin_elementwise_maximum(top, fabsf(oacc[d][r]));    // a NaN stays
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(top < INFINITY)) != 0, 0)) {
+        f32_body<HD, NW, false>(nullptr, nullptr, q, K, V, T, S, n_head, n_kv, scale, window, softcap, out);
+        return;
+    }
+    if (i0 + c >= T) return;
+    const float inv = 1.0f / l * (1.0f / V_UP);                 // l <= 2^30: no rounding
     Out* op = out + ((size_t)i * n_head + head) * HD + 4 * ks;   // register r of output tile d is dim 16 d + 4 ks + r
 #pragma unroll
     for (int d = 0; d < ND; d++) store_out(op + 16 * d, float4{oacc[d][0] * inv, oacc[d][1] * inv, oacc[d][2] * inv, oacc[d][3] * inv});

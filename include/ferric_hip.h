@@ -356,14 +356,15 @@ int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_cod
  * and chunked prefill) and the flash prefill kernel crates/ferric-llama/src/qwen3.rs:925 picks when it can -- "all three are
  * the same math". s < t -> FHIP_ERR_SHAPE with the reference's message (nn.rs:73). head_dim 64 or 128; f32 grade (every
  * operand as three bf16 values, 24 bits, on the bf16 matrix instructions; f32 sums), out [t, n_head * head_dim]; pointers 16-byte aligned.
- * A member that is infinite, NaN or beyond bf16's range (3.39e38) makes NaN of the outputs it takes part in. */
+ * Members of any magnitude: where a row meets one that three bf16 values do not hold (infinite, NaN, from 1e26 on in V, from 3.39e38 on in q and K) its result is
+ * fhip_causal_attention_f32_products'. */
 int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
                           size_t window, float softcap, float* d_out, void* stream);
 /* The same with the output rows as bf16, each value the one fhip_cvt_f32_bf16 makes of the f32 result. */
 int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
                                size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream);
 /* The same result from the f32 matrix instructions (d_out f32, or bf16 with out_bf16): slower, its error against f64 a fifth larger, other last
- * bits; f32's whole range. For
+ * bits. For
  * stacks on a block-quantized cache, where behind bf16 roundings a last bit decides code bytes of the layers after it, and a block's
  * codes should not depend on the library's version. */
 int fhip_causal_attention_f32_products(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,

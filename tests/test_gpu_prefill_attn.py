@@ -120,3 +120,82 @@ def test_f32_products_beside_the_cut_ones(F, X, D, t, s, nh, nkv, hd, w, cap, vs
     rounded = ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint16)
     assert np.array_equal(half.to_vec().view(np.uint16).reshape(-1)[:t * nh * hd], rounded.reshape(-1))
     assert lib.fhip_causal_attention_f32_products(*args[:3], s + 1, s, *args[5:], 0, out.buf.ptr, None) != 0
+
+
+def both_kernels(F, X, q, k, v, nh, nkv, cap=0.0):
+    """[t, nh * hd] of fhip_causal_attention and of fhip_causal_attention_f32_products, f32; the bf16 form of the first has to be its rounding."""
+    lib, T, t, s, hd = F._lib.load(), (lambda a: F.Tensor.from_vec(a, a.shape)), q.shape[0], k.shape[0], q.shape[1] // nh
+    tq, tk, tv, out, half = T(q), T(k), T(v), T(np.zeros(q.shape, np.float32)), T(np.zeros(q.shape, np.float32))
+    cut = X.causal_attention(tq, tk, tv, nh, nkv, 0, cap).to_vec().reshape(q.shape)
+    args = (tq.buf.ptr, tk.buf.ptr, tv.buf.ptr, t, s, nh, nkv, hd, 0, cap)
+    assert lib.fhip_causal_attention_f32_products(*args, 0, out.buf.ptr, None) == 0
+    assert lib.fhip_causal_attention_bf16(*args, half.buf.ptr, None) == 0
+    b = cut.view(np.uint32).astype(np.uint64)
+    rounded = ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint16)
+    got = half.to_vec().view(np.uint16).reshape(-1)[:cut.size].reshape(cut.shape)
+    assert np.array_equal(got[~np.isnan(cut)], rounded[~np.isnan(cut)])
+    assert ((got[np.isnan(cut)] & 0x7FFF) > 0x7F80).all()
+    return cut, out.to_vec().reshape(q.shape)
+
+
+# four and eight waves a workgroup at both head sizes (eight from 512 workgroups of 128 rows on)
+RANGE_SHAPES = [(70, 130, 10, 2, 128), (70, 130, 4, 4, 64), (200, 200, 256, 32, 128), (1100, 1100, 64, 8, 64)]
+
+
+@pytest.mark.parametrize("shape", RANGE_SHAPES)
+@pytest.mark.parametrize("kind", ["key -inf", "key inf, softcap", "key nan", "scores overflow", "value inf", "value largest", "query nan"])
+def test_members_that_three_cuts_do_not_carry(F, X, D, shape, kind):
+    """Members beyond the range the bf16 cuts hold: a row that sees one is the f32 kernel's, bit for bit (a NaN a NaN); where the result is finite
+    it is the oracle's at the bar of this file; rows that are not computed beside such a one keep their bits."""
+    t, s, nh, nkv, hd = shape
+    rng = np.random.default_rng(hd + s)
+    q = rng.standard_normal((t, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((s, nkv * hd)).astype(np.float32)
+    v = rng.standard_normal((s, nkv * hd)).astype(np.float32)
+    cap, j, off = 0.0, s - 20, s - t
+    first = j - off                                             # the first row that sees key j
+    if kind == "key -inf":
+        q[:, ::hd] = -np.abs(q[:, ::hd]) - 0.1                  # an infinite negative score: weight 0
+    if kind == "key inf, softcap":
+        cap = 30.0                                              # an infinite score is 30 or -30
+    clean, _ = both_kernels(F, X, q, k, v, nh, nkv, cap)
+    if kind in ("key -inf", "key inf, softcap"):
+        k[j, ::hd] = np.inf
+    elif kind == "key nan":
+        k[j, ::hd] = np.nan
+    elif kind == "scores overflow":
+        k[j] *= 1e25
+        q[first:] *= 1e25
+    elif kind == "value inf":
+        v[j, 5::hd] = -np.inf
+    elif kind == "value largest":
+        v[j] = np.where(v[j] > 0, 1, -1) * np.finfo(np.float32).max
+    else:
+        q[first:, 7::hd] = np.nan
+    cut, f32 = both_kernels(F, X, q, k, v, nh, nkv, cap)
+    same = (bits(cut) == bits(f32)) | (np.isnan(cut) & np.isnan(f32))
+    assert same[first:].all(), np.argwhere(~same[first:])[:4]
+    before = first // 16 * 16                                   # the wave that holds row `first` starts there ...
+    while before > 0 and (off + before - 1) // 32 >= j // 32:   # ... and the wave before it reads no key of j's tile
+        before -= 16
+    assert np.array_equal(bits(cut[:before]), bits(clean[:before]))
+    if kind in ("key -inf", "key inf, softcap", "value largest"):
+        for r in (first, t - 1):
+            want = D.decode_attention(q[r], k[:off + r + 1], v[:off + r + 1], nh, nkv, 0, cap)[0]
+            assert np.isfinite(want).all() and np.abs(cut[r] - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("shape", RANGE_SHAPES)
+@pytest.mark.parametrize("scale", [1e-33, 1e-36, 3e-38, 1e-41, 1e16])
+def test_small_and_large_values_keep_their_bits(F, X, D, shape, scale):
+    """V of every magnitude down to f32's subnormals: the cuts hold all of an f32's bits, so the error stays that of f32 sums of up to 1100 terms (4e-6 of
+    the largest output, as above) and, for results that are subnormal themselves, half a unit of their last place."""
+    t, s, nh, nkv, hd = shape
+    rng = np.random.default_rng(hd + s + 1)
+    q = rng.standard_normal((t, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((s, nkv * hd)).astype(np.float32)
+    v = (rng.standard_normal((s, nkv * hd)) * scale).astype(np.float32)
+    cut, _ = both_kernels(F, X, q, k, v, nh, nkv)
+    for r in (0, t // 2, t - 1):
+        want = D.decode_attention(q[r], k[:s - t + r + 1], v[:s - t + r + 1], nh, nkv)[0]
+        assert np.abs(cut[r] - want).max() <= 4e-6 * np.abs(want).max() + 2.0 ** -149, (r, np.abs(cut[r] - want).max() / np.abs(want).max())
