@@ -9,8 +9,8 @@
 // tensor (or a WGSL flash kernel up to its shared-memory limit); here it is one flash-style launch on the matrix cores, at f32's grade.
 //
 // Two kernels: causal_attn_cut_kernel, on bf16 matrix instructions with every f32 operand cut into three bf16 values, is what a caller gets;
-// causal_attn_kernel, on f32 matrix instructions, is what fhip_causal_attention_f32_products gives (prompts on a block-quantized cache:
-// the header says why). Measured, us, f32 -> cut, 40 query and 8 KV heads of 128: 509 rows x 809 keys 102.9 -> 72.6, 2048 x 2048 432 ->
+// causal_attn_kernel, on f32 matrix instructions, is what fhip_causal_attention_f32_products gives (prompts on a block-quantized cache,
+// whose codes would be others and no better ones: the header). Measured, us, f32 -> cut, 40 query and 8 KV heads of 128: 509 rows x 809 keys 102.9 -> 72.6, 2048 x 2048 432 ->
 // 274, 512 x 8192 1163 -> 789; few workgroups: 39 x 929, 8 heads 85.7 -> 70.3; heads of 64: 512 x 512, 32 heads 31.7 -> 27.7, 49 x 49 7.0 ->
 // 6.8. Relative error against f64, same shapes: 5.6e-7 -> 4.5e-7, 4.5e-7 -> 3.7e-7, 1.65e-6 -> 1.41e-6, 6.8e-7 -> 5.6e-7, 2.7e-7 -> 2.0e-7,
 // 1.7e-7 -> 1.2e-7. What bounds the cut kernel: the chain of a tile (cut and store 32 keys, products, statistics, products: 2.2 us a wave

@@ -364,9 +364,8 @@ int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, 
 int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
                                size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream);
 /* The same result from the f32 matrix instructions (d_out f32, or bf16 with out_bf16): slower, its error against f64 a fifth larger, other last
- * bits. For
- * stacks on a block-quantized cache, where behind bf16 roundings a last bit decides code bytes of the layers after it, and a block's
- * codes should not depend on the library's version. */
+ * bits. For stacks on a block-quantized cache, where behind bf16 roundings a last bit decides code bytes of the layers after it: the kernel above
+ * would store other codes (13 .. 16 % of them in a fourth layer), which are no nearer to those of f64 rows. */
 int fhip_causal_attention_f32_products(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
                                        size_t head_dim, size_t window, float softcap, int out_bf16, void* d_out, void* stream);
 
