@@ -1511,10 +1511,17 @@ int launch_kv_append(const float* k, const float* v, size_t t, size_t width, con
 // cache holds), so from ATT_WIDE_FROM rows on it has sixteen waves, 128 keys a step, in place of four; fewer rows leave most of those without a key (48 rows
 // 4.6 -> 5.6 us). Four waves -> sixteen, f32 cache, us: 130 / 200 / 256 rows 6.2 / 6.9 / 7.1 -> 5.8 / 6.2 / 6.5. us a token through four layers (d 2048, 16 and 8 heads of 128), one
 // workgroup a head | per (head, split) and combined: f32 300 rows 153.6 | 159.4, 400 158.0 | 159.4, 490 162.1 | 160.4; Q8_0 300 154.4 | 159.7,
-// 490 160.9 | 159.6; d 5120, 40 heads, f32 300 320.3 | 323.6, 400 326.7 | 322.4, Q8_0 300 313.5 | 326.9, 490 318.3 | 324.2. A head per KV head, f32, 60 rows: 154.3 with
-// splits of 16 keys, 140.5 in one workgroup.
-constexpr size_t ATT_SHORT = 352, ATT_WIDE_FROM = 97;
-bool attn_per_query_head(size_t len) { return len <= ATT_SHORT; }
+// 490 160.9 | 159.6; d 5120, 40 heads, f32 300 320.3 | 323.6, 400 326.7 | 322.4, Q8_0 300 313.5 | 326.9, 490 318.3 | 324.2.
+// A head per KV head shares its rows with no other, and beyond ATT_SHORT_ROWS rows times heads of 128 dims on an f32 cache its workgroup waits for memory
+// where splits of 64 keys bring more workgroups; so there it ends at ATT_SHORT_OWN rows. us a launch on rows no cache holds, one workgroup a head | splits:
+// f32, 16 heads 304 / 352 rows 7.7 | 8.1, 8.6 | 8.5; 24 heads 320 / 352 rows 8.2 | 8.6, 11.6 | 9.4; 32 heads 256 / 288 / 352 rows 8.3 | 9.3, 9.9 | 9.2, 11.6 | 9.9;
+// 40 heads 256 / 352 rows 10.8 | 9.8, 13.1 | 10.4; 4 heads 352 rows 8.1 | 7.9; heads of 64, 64 of them, 352 rows 8.3 | 9.1. A quantized cache takes the f32 one's
+// way, whose bits it promises, though it reads a quarter: Q8_0, 32 heads 288 rows 7.9 | 8.9, 224 rows 7.3 | 8.8. Grouped heads in one workgroup each | per (head, split)
+// at 352 rows: f32 2 heads 8.0 | 8.2, 16 of 4 8.6 | 9.0, 40 of 8 8.9 | 9.3, 64 of 8 9.2 | 9.4, 32 of 8 of 64 dims 6.2 | 8.0; Q8_0 2 heads 7.6 | 8.7.
+constexpr size_t ATT_SHORT = 352, ATT_SHORT_OWN = 256, ATT_SHORT_ROWS = 8192, ATT_WIDE_FROM = 97;
+bool attn_per_query_head(size_t len, int n_head, int n_kv, int hd, bool ws = true) {   // ws: splits have a workspace to go to
+    return len <= (ws && n_head == n_kv && hd == 128 && len * (size_t)n_kv > ATT_SHORT_ROWS ? ATT_SHORT_OWN : ATT_SHORT);
+}
 bool attn_wide(size_t len) { return len >= ATT_WIDE_FROM; }
 
 // Between ATT_SHORT and ATT_MID rows under grouped query heads: one workgroup per (query head, split of at least ATT_MID_KEYS
@@ -1535,7 +1542,7 @@ int attn_mid_splits(size_t len, int n_head) {
 // Splits of the key range beyond ATT_SHORT: about two workgroups per CU over all KV heads, at least 64 keys each (two rounds of the
 // workgroup's 16 streams x 2 keys), at most 256 (the combine kernel's LDS tables).
 int attn_splits(size_t len, int n_kv) {
-    if (n_kv <= 0 || attn_per_query_head(len)) return 1;
+    if (n_kv <= 0) return 1;
     constexpr int keys = 64;
     int want = (2 * device_cus() + n_kv - 1) / n_kv;
     size_t by_keys = (len + (size_t)keys - 1) / (size_t)keys;
@@ -1544,7 +1551,8 @@ int attn_splits(size_t len, int n_kv) {
 }
 
 // the most splits any launch shape takes for this cache length: what the workspace has to hold
-int attn_ws_splits(size_t len, int n_head, int n_kv) {
+int attn_ws_splits(size_t len, int n_head, int n_kv, int hd) {
+    if (attn_per_query_head(len, n_head, n_kv, hd)) return 1;
     const int a = attn_splits(len, n_kv);
     const int b = attn_per_head_splits(len, n_head, n_kv) ? attn_mid_splits(len, n_head) : 1;
     return a > b ? a : b;
@@ -1561,7 +1569,7 @@ int launch_decode_attention(const float* q, const float* K, const float* V, int 
     const float scale = 1.0f / sqrtf((float)hd);
     const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;   // a window that large is no window
     if (g > 8) return set_error(FHIP_ERR_SHAPE, "decode_attention: %d query heads per KV head (1..=8 supported)", g);
-    if (attn_per_query_head(len)) {
+    if (attn_per_query_head(len, n_head, n_kv, hd, ws != nullptr)) {
         int rc = launch_attn_g<1>(hd, dim3((unsigned)n_head, 1), s, q, K, V, n_kv, (uint32_t)len, d_len, scale, 1, win, softcap, ws, out, g, attn_wide(len));
         return rc ? rc : check_hip(hipGetLastError(), "decode_attention launch");
     }
@@ -1603,7 +1611,7 @@ static int launch_attention_over_kvq(const char* who, int fmt, const float* q, c
     if (hd != 64 && hd != 128) return set_error(FHIP_ERR_SHAPE, "%s: head_dim must be 64 or 128", who);
     if (len > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "%s: cache length exceeds 2^31", who);
     const int g = n_head / n_kv;
-    const bool per_head = g >= 1 && g <= 8 && attn_per_query_head(len);   // as the f32 cache's launch: the same sums, the same bits
+    const bool per_head = g >= 1 && g <= 8 && attn_per_query_head(len, n_head, n_kv, hd, ws != nullptr);   // as the f32 cache's launch: the same sums, the same bits
     const bool mid = g >= 1 && g <= 8 && attn_per_head_splits(len, n_head, n_kv);
     const int splits = per_head ? 1 : mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "%s: this cache length needs the workspace", who);
@@ -1671,14 +1679,15 @@ int launch_qkv_post_attention(const float* qkv, const float* bias, const float* 
     if (len > 0x7FFFFFFFull || len > cap) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention: length outside the cache");
     const int g = n_head / n_kv;
     const bool mid = g <= 8 && attn_per_head_splits(len, n_head, n_kv);
-    const int splits = attn_per_query_head(len) ? 1 : (mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv));
+    const bool per_head = attn_per_query_head(len, n_head, n_kv, hd, ws != nullptr);
+    const int splits = per_head ? 1 : (mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv));
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "qkv_post_attention: this cache length needs the workspace");
     QkvPostParams fp = one_token_post(qkv, bias, q_norm, k_norm, d_pos, freq_scale, n_head, n_kv, hd, n_rot, interleaved, eps, base, cap);
     fp.k_cache = k_cache; fp.v_cache = v_cache;
     const float scale = 1.0f / sqrtf((float)hd);
     const uint32_t win = window > 0x7FFFFFFFull ? 0u : (uint32_t)window;
     if (g > 8) return set_error(FHIP_ERR_SHAPE, "qkv_post_attention: %d query heads per KV head (1..=8 supported)", g);
-    if (attn_per_query_head(len)) {
+    if (per_head) {
         // every workgroup of a KV head forms the new token's K and V rows and stores them (the same bits from each) before
         // it reads them back with the other keys
         int rc = launch_attn_fused_g<1>(hd, dim3((unsigned)n_head, 1), s, fp, n_kv, (uint32_t)len, d_pos, scale, 1, win, softcap, ws, out, g, attn_wide(len));
