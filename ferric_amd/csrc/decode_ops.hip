@@ -1344,10 +1344,11 @@ int launch_attn_kvq(int g, int hd, dim3 grid, const KvqLaunch& a, int gq, bool w
     }
 }
 
-// Which launches take it: its cost does not depend on the number of query heads a KV head, the kernel above costs less for one and two. us, this | that
-// without the combine launch, 8 KV heads, head size 128, 32768 Q8_0 keys: 2 query heads each 26.4 | 23.1, 3: 26.7 | 27.6, 4: 26.8 | 32.2, 5: 27.0 | 38.3;
-// Q4_0, 3: 26.3 | 30.1, 5: 25.7 | 38.8; 8000 keys Q8_0, 3: 11.4 | 12.0, 4: 11.3 | 13.6; head size 64, 32768 keys, 3: 16.8 | 19.5, 4: 17.2 | 23.0; 8000 keys,
-// 3: 8.8 | 9.2; 4 KV heads of 128, 9000 keys, 3: 10.6 | 9.8, 5: 10.9 | 13.5.
+// Which launches take it: its cost does not depend on the number of query heads a KV head, the kernel above costs less for one and two. us, this | that, both
+// with the combine launch, on rows no cache holds. Three query heads a KV head, post-processed in the launch: heads of 128, Q8_0, 8 KV heads 5200 / 9000 / 32768 keys 13.8 | 14.4,
+// 16.5 | 17.5, 30.2 | 31.6; 4 KV heads 13.3 | 13.1, 14.3 | 14.9, 20.2 | 22.2; 1 KV head 10.8 | 11.2, 11.7 | 12.7, 14.5 | 16.3; Q4_0 4 KV heads 14.2 | 13.3, 14.7 | 14.8, 20.5 | 23.0;
+// heads of 64, 4 KV heads Q8_0 10.7 | 10.5, 11.1 | 11.6, 14.8 | 17.0. Post-processed before: Q8_0 8 KV heads 12.8 | 13.4, 15.8 | 15.7, 29.6 | 29.0; 16 KV heads 17.5 | 16.4, 20.9 | 20.3,
+// 48.8 | 46.5 (in the launch 18.4 | 18.4, 21.4 | 22.7, 49.6 | 49.2). Four: 8 KV heads of 128, Q8_0 14.0 | 16.0, 16.6 | 19.1, 30.3 | 36.0; five 14.5 | 18.8, 17.2 | 21.3, 31.4 | 40.7.
 // Key codes are read eight bytes at a time; a lane's offset inside a round's rows is kept in 32 bits (n_kv).
 bool attn_long_takes(int fmt, int g, int n_kv, const uint32_t* k_codes) {
     if (fmt == FHIP_KVQ_Q4_1 || g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
