@@ -103,16 +103,16 @@ int device_cus() { return g_cus; }
 size_t device_lds_bytes() { return g_lds; }
 
 // The streaming mat-vec exists in two copies, one per activation precision; these forward to the one the weight names.
-// From three rows on, Q4_K, Q5_K, Q6_K and Q8_0 batches go four rows at a time through the kernel that multiplies on the 4 x 4 x 4 int8
+// From three rows on (Q8_0: four), Q4_K, Q5_K, Q6_K and Q8_0 batches go four rows at a time through the kernel that multiplies on the 4 x 4 x 4 int8
 // matrix instruction (gemv_quad.hip: the same arithmetic and the same bits per row, one pass over the weight for four rows);
 // what is left of a batch, one or two rows, takes the dot-product kernel.
 // Batches of the 32-value formats from here on go up to sixteen rows at a time through the kernel that multiplies on the 16 x 16 x 32
-// int8 matrix instruction (gemv_wide.hip: the same bits per row). Its cost is the quantiser's, per activation row and workgroup,
+// int8 matrix instruction (gemv_wide.hip: the same bits per row); what is left of a batch goes on as a batch of its own. Its cost is the quantiser's, per activation row and workgroup,
 // plus the weight once; the dot-product kernel's is a launch and the weight per four rows. us, cold, dot-product | wide, three rows:
 // IQ4_NL 1024 x 5120 7.8 | 10.1, 4096 x 4096 9.6 | 10.1, 9728 x 2560 11.7 | 10.8, 34816 x 5120 43 | 30.5; four: Q4_0 1024 x 5120 9.4 | 10.3,
 // 1946 x 1504 6.8 | 7.7, 4096 x 4096 12.8 | 9.8, 34816 x 5120 43 | 29.7; five: 1024 x 1024 9.7 | 8.0, 1024 x 5120 13.8 | 11.8, 34816 x 5120
-// 60 | 38; sixteen: 1467 x 1760 38.8 | 15.8, 4096 x 4096 50 | 23, 34816 x 5120 171 | 61. Q8_0 has the four-row kernel (gemv_quad.hip) at three
-// and four rows of up to 5120 columns (4096 x 4096 9.5 | 11.5).
+// 60 | 38; sixteen: 1467 x 1760 38.8 | 15.8, 4096 x 4096 50 | 23, 34816 x 5120 171 | 61. Q8_0 has the others at three
+// and four rows of up to 5120 columns (three, 4096 x 4096 9.6 | 11.5).
 bool takes_wide(const fhip_weight* w, size_t t) {
     const size_t weights = w->rows * w->cols;
     if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
@@ -120,37 +120,36 @@ bool takes_wide(const fhip_weight* w, size_t t) {
     return w->planes == 3 ? gemv_wide_supports_p3(w, t < 16 ? t : 16) : gemv_wide_supports_p2(w, t < 16 ? t : 16);
 }
 bool g_quad_matvec = true, g_generic_forced = false;
+// What the first rows of a mat-vec batch of `left` rows take: the kernel and how many rows. Three rows of Q8_0 are one pass of the dot-product kernel
+// and four one pass of the four-row one, us, dot-product | four-row, three rows: 1024 x 1024 4.8 | 5.7, 1024 x 5120 7.7 | 9.6, 2048 x 2048 6.1 | 7.3, 4096 x 4096
+// 9.6 | 12.1, 12288 x 4096 16.7 | 22.0, 34816 x 5120 45.8 | 48.6; four: 1024 x 5120 9.1 | 9.9, 2048 x 2048 9.7 | 7.5, 4096 x 4096 14.3 | 12.4, 34816 x 5120 54.8 | 48.3.
+struct MatvecPass { int kernel; size_t rows; };
+MatvecPass matvec_pass(const fhip_weight* w, size_t left, size_t n_ff) {
+    if (left >= 3 && g_quad_matvec && !g_generic_forced) {
+        if (!n_ff && takes_wide(w, left)) return {FHIP_ROUTE_WIDE, left < 16 ? left : 16};
+        if (w->type == FHIP_Q8_0 && left == 3) return {FHIP_ROUTE_DOT, left};
+        if (w->planes == 3 ? gemv_quad_supports_p3(w, 4, n_ff) : gemv_quad_supports_p2(w, 4, n_ff)) return {FHIP_ROUTE_QUAD, left < 4 ? left : 4};
+    }
+    return {FHIP_ROUTE_DOT, left};
+}
 int launch_gemv(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, size_t n_ff, hipStream_t s) {
     const bool p3 = w->planes == 3;
-    if (!n_ff && g_quad_matvec && !g_generic_forced && d_x && d_y && takes_wide(w, rows_x)) {
-        for (size_t m0 = 0; m0 < rows_x;) {
-            const size_t t = rows_x - m0 < 16 ? rows_x - m0 : 16;
-            const float* x = d_x + m0 * w->cols;
-            float* y = d_y + m0 * w->rows;
-            int rc;
-            if (takes_wide(w, t)) rc = p3 ? launch_gemv_wide_p3(w, x, t, y, s) : launch_gemv_wide_p2(w, x, t, y, s);
-            else rc = p3 ? launch_gemv_p3(w, x, t, y, 0, s) : launch_gemv_p2(w, x, t, y, 0, s);
-            if (rc) return rc;
-            m0 += t;
+    if (rows_x < 3 || !d_x || !d_y) return p3 ? launch_gemv_p3(w, d_x, rows_x, d_y, n_ff, s) : launch_gemv_p2(w, d_x, rows_x, d_y, n_ff, s);
+    const size_t out_rows = n_ff ? n_ff : w->rows;
+    for (size_t m0 = 0; m0 < rows_x;) {
+        const MatvecPass pass = matvec_pass(w, rows_x - m0, n_ff);
+        const float* x = d_x + m0 * w->cols;
+        float* y = d_y + m0 * out_rows;
+        int rc;
+        switch (pass.kernel) {
+            case FHIP_ROUTE_WIDE: rc = p3 ? launch_gemv_wide_p3(w, x, pass.rows, y, s) : launch_gemv_wide_p2(w, x, pass.rows, y, s); break;
+            case FHIP_ROUTE_QUAD: rc = p3 ? launch_gemv_quad_p3(w, x, pass.rows, y, n_ff, s) : launch_gemv_quad_p2(w, x, pass.rows, y, n_ff, s); break;
+            default: rc = p3 ? launch_gemv_p3(w, x, pass.rows, y, n_ff, s) : launch_gemv_p2(w, x, pass.rows, y, n_ff, s);
         }
-        return FHIP_OK;
+        if (rc) return rc;
+        m0 += pass.rows;
     }
-    if (rows_x >= 3 && g_quad_matvec && !g_generic_forced && d_x && d_y &&
-        (p3 ? gemv_quad_supports_p3(w, 4, n_ff) : gemv_quad_supports_p2(w, 4, n_ff))) {
-        const size_t out_rows = n_ff ? n_ff : w->rows;
-        for (size_t m0 = 0; m0 < rows_x;) {
-            const size_t t = rows_x - m0 < 4 ? rows_x - m0 : 4;
-            const float* x = d_x + m0 * w->cols;
-            float* y = d_y + m0 * out_rows;
-            int rc;
-            if (t >= 3) rc = p3 ? launch_gemv_quad_p3(w, x, t, y, n_ff, s) : launch_gemv_quad_p2(w, x, t, y, n_ff, s);
-            else rc = p3 ? launch_gemv_p3(w, x, t, y, n_ff, s) : launch_gemv_p2(w, x, t, y, n_ff, s);
-            if (rc) return rc;
-            m0 += t;
-        }
-        return FHIP_OK;
-    }
-    return p3 ? launch_gemv_p3(w, d_x, rows_x, d_y, n_ff, s) : launch_gemv_p2(w, d_x, rows_x, d_y, n_ff, s);
+    return FHIP_OK;
 }
 bool gemv_quad_matvec(bool on) {
     const bool before = g_quad_matvec;
@@ -285,18 +284,25 @@ int zero_outputs(size_t t, size_t rows, float* d_y, hipStream_t s) {
 size_t f16x2_matmul_ws(const fhip_weight* w, size_t t) {
     return align256(fhip::gemm_f16x2_xp_bytes(w, t)) + (w->batch_policy == FHIP_BATCH_ORDERED ? align256(fhip::gemm_f16x2_part_bytes_upto(w, t)) : 0);
 }
+// What such a product takes: the held kernel, or the streaming ones with operand rows of their own or prepared ones (own: the rows come as they are)
+int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, const float* d_y) {
+    if (own && fhip::gemm_f16x2_held(w, d_x, t, d_y)) return FHIP_ROUTE_HELD;
+    const bool cut = fhip::gemm_f16x2_adds_into_y(w, t);   // along K
+    return (own && !(cut && w->batch_policy != FHIP_BATCH_ORDERED) && fhip::gemm_f16x2_own_x(w, d_x, t) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (cut ? FHIP_ROUTE_CUT : 0);
+}
 // deferred: the ordered sum of K-split groups is left to the reader of y, which gets *deferred as its `src`
 int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
                  fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
-    if (!swiglu_in && !src && fhip::gemm_f16x2_held(w, d_x, t, d_y)) {
+    const int route = f16x2_route(w, d_x, t, !swiglu_in && !src, d_y);
+    if (route == FHIP_ROUTE_HELD) {
         if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0, 0, 128};
         return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
     }
     uint16_t* xp = (uint16_t*)d_ws;
-    const bool ordered = w->batch_policy == FHIP_BATCH_ORDERED;
-    float* part = ordered && fhip::gemm_f16x2_part_bytes(w, t) ? (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))) : nullptr;
-    const bool clr = !part && fhip::gemm_f16x2_adds_into_y(w, t);   // then the split clears y on the side
-    if (!swiglu_in && !src && !clr && fhip::gemm_f16x2_own_x(w, d_x, t)) return fhip::launch_gemm_f16x2(w, nullptr, t, d_y, s, false, part, deferred, d_x);
+    const bool cut = (route & FHIP_ROUTE_CUT) != 0, ordered = w->batch_policy == FHIP_BATCH_ORDERED;
+    float* part = cut && ordered ? (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))) : nullptr;
+    const bool clr = cut && !ordered;   // then the split clears y on the side
+    if ((route & ~FHIP_ROUTE_CUT) == FHIP_ROUTE_OWN_ROWS) return fhip::launch_gemm_f16x2(w, nullptr, t, d_y, s, false, part, deferred, d_x);
     int rc = fhip::launch_xsplit_f16(w, d_x, t, swiglu_in, xp, s, clr ? d_y : nullptr, clr ? t * w->rows : 0, src);
     if (rc) return rc;
     return fhip::launch_gemm_f16x2(w, xp, t, d_y, s, clr, part, deferred);
@@ -1130,6 +1136,25 @@ int fhip_debug_generic_matvec(int on) {
 int fhip_debug_gemm_tile(int tile) { return fhip::gemm_bf16_force_tile(tile); }
 
 int fhip_debug_quad_matvec(int on) { return fhip::gemv_quad_matvec(on != 0) ? 1 : 0; }
+
+int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_x, const float* d_y, int* kernels, size_t* rows, size_t cap, size_t* n) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (!w || !d_x || !d_y || !kernels || !rows || !n) return set_error(FHIP_ERR_ARG, "fhip_debug_matmul_route: NULL pointer");
+    *n = 0;
+    auto add = [&](int kernel, size_t r) { if (*n < cap) { kernels[*n] = kernel; rows[*n] = r; } ++*n; };
+    const size_t grp = takes_f16x2(w, rows_x) ? f16x2_group(w) : rows_x;
+    for (size_t m0 = 0; m0 < rows_x && w->rows; m0 += grp) {
+        const size_t t = rows_x - m0 < grp ? rows_x - m0 : grp;
+        if (takes_f16x2(w, t)) { add(f16x2_route(w, d_x + m0 * w->cols, t, true, d_y + m0 * w->rows), t); continue; }
+        for (size_t r = 0; r < t;) {
+            const fhip::MatvecPass pass = fhip::matvec_pass(w, t - r, 0);
+            add(pass.kernel, pass.rows);
+            r += pass.rows;
+        }
+    }
+    return FHIP_OK;
+}
 
 int fhip_debug_read_probe(const void* d_src, size_t nbytes, uint32_t* d_sink, void* stream) {
     int rc = need_init();

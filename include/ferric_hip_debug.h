@@ -19,11 +19,22 @@ int fhip_debug_generic_matvec(int on);
  * launches; fhip_workspace_bytes_coop follows it. No counterpart in the reference. */
 int fhip_debug_gemm_tile(int tile);
 
-/* Debugging and tests: on == 0 keeps Q4_K / Q5_K / Q6_K / Q8_0 batches of three and more rows off the kernel that multiplies on the
- * 4 x 4 x 4 int8 matrix instruction, so that the mat-vec entry points run them on the dot-product kernel two rows at a time
- * (the two give the same bits; the tests compare them this way). Returns the setting before the call (1 = on, the default).
+/* Debugging and tests: on == 0 keeps batches of three and more rows off the kernels that multiply on the 4 x 4 x 4 (Q4_K / Q5_K / Q6_K /
+ * Q8_0) and 16 x 16 x 32 (the 32-value formats) int8 matrix instructions, so that the mat-vec entry points run them on the dot-product kernel
+ * a few rows at a time (they give the same bits; the tests compare them this way). Returns the setting before the call (1 = on, the default).
  * Process-wide, not thread-safe against concurrent launches. No counterpart in the reference. */
 int fhip_debug_quad_matvec(int on);
+
+/* Tests: the launches fhip_matmul_q makes of a call with these arguments, one after the other: kernels[i] multiplies rows[i] activation
+ * rows. *n: how many there are (the first `cap` are stored). Nothing is launched and no operand is read. No counterpart in the reference. */
+#define FHIP_ROUTE_DOT 0         /* the dot-product mat-vec, up to four rows a pass over the weight */
+#define FHIP_ROUTE_QUAD 1        /* four rows a pass, 4 x 4 x 4 int8 matrix instruction */
+#define FHIP_ROUTE_WIDE 2        /* up to sixteen, 16 x 16 x 32 int8 matrix instruction */
+#define FHIP_ROUTE_HELD 3        /* f16 hi / lo: a weight row's whole K inside one workgroup */
+#define FHIP_ROUTE_OWN_ROWS 4    /* f16 hi / lo: operand rows made by the workgroups that multiply them */
+#define FHIP_ROUTE_PREPARED 5    /* f16 hi / lo: operand rows made by a launch in front */
+#define FHIP_ROUTE_CUT 8         /* with the last two: weight rows are cut along K between workgroups */
+int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_x, const float* d_y, int* kernels, size_t* rows, size_t cap, size_t* n);
 
 /* Measurement aid: one launch that reads nbytes at d_src (16-byte loads over the whole chip) and does nothing else; d_sink is
  * one device word that is practically never written. Timed beside a mat-vec of the same size it gives the time a perfect reader

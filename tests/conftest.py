@@ -39,6 +39,20 @@ def bits(a):
     return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
 
 
+# ---- which launches a product takes (fhip_debug_matmul_route), for tests that name the kernel they are about
+ROUTES = {"DOT": 0, "QUAD": 1, "WIDE": 2, "HELD": 3, "OWN_ROWS": 4, "PREPARED": 5, "CUT": 8}
+
+
+def route(F, w, x, t):
+    """[(kernel, activation rows)] of fhip_matmul_q on the first t rows of x and an output of its own."""
+    import ctypes as C
+    lib = F._lib.load()
+    y = F.Tensor.empty((t, lib.fhip_weight_rows(w.handle)))
+    kernels, rows, n = (C.c_int * 64)(), (C.c_size_t * 64)(), C.c_size_t()
+    F._lib.check(lib.fhip_debug_matmul_route(w.handle, x.buf.ptr, t, y.buf.ptr, kernels, rows, 64, C.byref(n)))
+    return list(zip(kernels[:n.value], rows[:n.value]))
+
+
 # ---- precision of the streaming mat-vec's activations (a property of the weight handle; fhip_matvec_precision sets what new
 # handles start with): the tests of the mat-vec entry points run once per setting, making their weights under it. At 24
 # bits (what a handle has unless told otherwise) the dot products are held to the bar the reference's examples use for its

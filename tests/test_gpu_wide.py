@@ -4,7 +4,7 @@ against single rows on the dot-product mat-vec it restates: the same bits for ev
 import numpy as np
 import pytest
 
-from conftest import bits
+from conftest import ROUTES, bits, route
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("precision")]
 Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, IQ4_NL, IQ4_XS, MXFP4 = 2, 3, 6, 7, 8, 20, 23, 39
@@ -49,6 +49,18 @@ def test_three_and_four_rows_of_large_weights(F, ty, rows, cols, m):
     qm.batch_policy(F.BATCH_F32_MATVEC)
     x = np.random.default_rng(4).standard_normal((m, cols)).astype(np.float32)
     assert same(F.Tensor.from_vec(x, x.shape).matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
+
+
+@pytest.mark.parametrize("ty,rows,cols,m,last", [(Q8_0, 130, 4096, 19, "DOT"), (Q8_0, 130, 4096, 20, "QUAD"), (Q8_0, 96, 5120, 36, "QUAD"), (Q8_0, 40, 5152, 20, "DOT"), (Q8_0, 1700, 5152, 20, "WIDE"), (Q4_0, 70, 1024, 19, "DOT"),
+                                                  (IQ4_NL, 64, 512, 21, "WIDE"), (Q5_0, 33, 96, 18, "DOT")])
+def test_the_rows_behind_the_last_sixteen_go_where_a_batch_of_them_would(F, ty, rows, cols, m, last):
+    from ferric_amd.synth import synth_weights
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 5), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(6).standard_normal((m, cols)).astype(np.float32)
+    xt = F.Tensor.from_vec(x, x.shape)
+    assert route(F, qm, xt, m) == [(ROUTES["WIDE"], 16)] * (m // 16) + [(ROUTES[last], m % 16)]
+    assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
 
 
 def test_mxfp4_blocks_that_may_overflow(F):
