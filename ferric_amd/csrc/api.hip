@@ -285,15 +285,15 @@ size_t f16x2_matmul_ws(const fhip_weight* w, size_t t) {
     return align256(fhip::gemm_f16x2_xp_bytes(w, t)) + (w->batch_policy == FHIP_BATCH_ORDERED ? align256(fhip::gemm_f16x2_part_bytes_upto(w, t)) : 0);
 }
 // What such a product takes: the held kernel, or the streaming ones with operand rows of their own or prepared ones (own: the rows come as they are)
-int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, const float* d_y) {
-    if (own && fhip::gemm_f16x2_held(w, d_x, t, d_y)) return FHIP_ROUTE_HELD;
+int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, const float* d_y, bool deferred) {
+    if (own && fhip::gemm_f16x2_held(w, d_x, t, d_y, deferred && w->batch_policy == FHIP_BATCH_ORDERED)) return FHIP_ROUTE_HELD;
     const bool cut = fhip::gemm_f16x2_adds_into_y(w, t);   // along K
     return (own && !(cut && w->batch_policy != FHIP_BATCH_ORDERED) && fhip::gemm_f16x2_own_x(w, d_x, t) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (cut ? FHIP_ROUTE_CUT : 0);
 }
 // deferred: the ordered sum of K-split groups is left to the reader of y, which gets *deferred as its `src`
 int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
                  fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
-    const int route = f16x2_route(w, d_x, t, !swiglu_in && !src, d_y);
+    const int route = f16x2_route(w, d_x, t, !swiglu_in && !src, d_y, deferred != nullptr);
     if (route == FHIP_ROUTE_HELD) {
         if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0, 0, 128};
         return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
@@ -1146,7 +1146,7 @@ int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_
     const size_t grp = takes_f16x2(w, rows_x) ? f16x2_group(w) : rows_x;
     for (size_t m0 = 0; m0 < rows_x && w->rows; m0 += grp) {
         const size_t t = rows_x - m0 < grp ? rows_x - m0 : grp;
-        if (takes_f16x2(w, t)) { add(f16x2_route(w, d_x + m0 * w->cols, t, true, d_y + m0 * w->rows), t); continue; }
+        if (takes_f16x2(w, t)) { add(f16x2_route(w, d_x + m0 * w->cols, t, true, d_y + m0 * w->rows, false), t); continue; }
         for (size_t r = 0; r < t;) {
             const fhip::MatvecPass pass = fhip::matvec_pass(w, t - r, 0);
             add(pass.kernel, pass.rows);

@@ -156,8 +156,9 @@ int launch_gemm_f16x2(const fhip_weight* w, const uint16_t* d_xp, size_t t, floa
                       float* d_part = nullptr, F16Parts* deferred = nullptr, const float* d_x = nullptr);
 // true: launch_gemm_f16x2 given d_x (the f32 rows) makes its operand rows itself, without launch_xsplit_f16 in front of it (d_xp is not read)
 bool gemm_f16x2_own_x(const fhip_weight* w, const float* d_x, size_t t);
-// true: launch_gemm_f16x2_held does the whole product, y = x W^T, in one launch without a workspace
-bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y);
+// true: launch_gemm_f16x2_held does the whole product, y = x W^T, in one launch without a workspace. summed_later: launch_gemm_f16x2's partial
+// sums would be left to the launch that reads y
+bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y, bool summed_later);
 int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s);
 size_t gemm_f16x2_part_bytes(const fhip_weight* w, size_t t);
 size_t gemm_f16x2_part_bytes_upto(const fhip_weight* w, size_t t);   // the largest over batches of 1..t rows

@@ -1260,6 +1260,7 @@ __global__ void zero_f32_kernel(float* __restrict__ out, size_t n) {
 struct Plan {
     int nt, nchunks;
     long long units, groups;
+    long long wgs;        // workgroups that are resident together
     unsigned grid;
     bool split;
     int kmax;             // most workgroups that hold part of one group's K
@@ -1284,7 +1285,7 @@ Plan make_plan(const fhip_weight* w, size_t t) {
     }
     const long long groups = ((long long)w->rows + q.group - 1) / q.group;
     q.units = groups * q.nchunks;
-    const long long wgs = q.group == 256 ? cus : cus * (w->type == FHIP_Q6_K ? slots<Q6K>(q.nt) : w->type == FHIP_Q8_0 ? slots<Q80>(q.nt) :
+    const long long wgs = q.wgs = q.group == 256 ? cus : cus * (w->type == FHIP_Q6_K ? slots<Q6K>(q.nt) : w->type == FHIP_Q8_0 ? slots<Q80>(q.nt) :
                                  w->type == FHIP_Q5_K ? slots<Q5K>(q.nt) : slots<Q4K>(q.nt));
     // one workgroup per resident slot, each with the same share of the units (a grid of 2.66 workgroups per CU leaves
     // two thirds of the CUs with half as much again to do as the rest); shares of three quarters of a group's chunks or
@@ -1370,18 +1371,20 @@ int launch_held_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y
     p.row_bytes = w->row_bytes;
     const int cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     // Both sets of 9..16 rows in one workgroup where the tiles alone fill the chip several times over: 16 rows, us, apart | together:
-    // 34000 x 4096 Q4_K 40.7 | 36.4, Q8_0 64.0 | 50.5, but 12000 x 3072 Q4_K 14.6 | 19.2, 2000 x 4096 Q8_0 9.0 | 14.9
+    // 34000 x 4096 Q4_K 36.7 | 32.2, Q8_0 62.7 | 47.7, 12000 x 3072 Q6_K 18.1 | 18.3, Q4_K 15.3 | 18.0, 2000 x 4096 Q8_0 9.2 | 14.8
     const bool two = t > 8 && t <= 16 && p.nchunks <= 16 && p.tiles > 4 * cus;
     const int sets = two ? 1 : (int)((t + 7) / 8);
-    // waves: one a chunk up to 16 (4096 x 4096 Q8_0 at 8 rows 10.2 us, 11.9 with eight of two chunks each); beyond, 12 with two chunks each while
-    // every workgroup has a CU to itself (2000 x 5120 Q6_K 11.8 us against 12.9), eight with three chunks and no spill where
-    // they go through several tiles (12000 x 6144 Q8_0 25.9 us against 28.0)
-    const int most = two || p.nchunks <= 8 ? 8 : p.nchunks <= 16 ? 16 : p.tiles * sets <= cus ? 12 : 8;
+    // waves: one a chunk up to 16 (4096 x 4096 Q8_0 at 8 rows 9.1 us, 13.7 with eight of two chunks each); beyond, 12 with two chunks each, or eight with three
+    // and no spill. Eight where workgroups go through several tiles of a format with minima (12 | 8 waves, 12000 x 5120 Q4_K 20.9 | 18.6, 2000 x 5120 11.9 | 12.2) and of rows
+    // that leave the twelve no wave idle (12000 x 6144 Q8_0 27.2 | 26.1, 3000 x 5120 at 32 rows Q6_K 1.06 of the time with eight)
+    const bool mins = w->type == FHIP_Q4_K || w->type == FHIP_Q5_K, several = p.tiles * sets > cus;
+    const int most = two || p.nchunks <= 8 ? 8 : p.nchunks <= 16 ? 16 : several && (mins || p.nchunks > 22) ? 8 : 12;
     const int held = (p.nchunks + most - 1) / most;
     p.nw = (p.nchunks + held - 1) / held;
     p.like_rows = t <= 8;
-    // one workgroup a CU; two of eight waves where there are many tiles (34000 x 2048 Q6_K 19.3 us against 21.6, but 5120 x 2048 9.9 against 8.7)
-    int slots = cus * (!two && held == 1 && most == 8 && p.tiles * sets > 4 * cus ? 2 : 1) / sets;
+    // one workgroup a CU; two of eight waves where there are many tiles for their chunks. Q4_K, 8 rows, one | two: 34000 x 512 10.3 | 9.0, 12000 x 512 5.7 | 5.5, 34000 x 2048
+    // 15.9 | 15.8, 5120 x 2048 7.2 | 8.6; 32 rows: 5120 x 2048 1.18 of the time with two, 20000 x 2048 0.91, 5120 x 1024 1.04, 8000 x 1024 0.89
+    int slots = cus * (!two && held == 1 && most == 8 && 2 * p.tiles * sets > 3 * p.nchunks * cus ? 2 : 1) / sets;
     if (slots < 1) slots = 1;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles < slots ? p.tiles : slots), (unsigned)sets), dim3(64 * p.nw), 0, s, p); };
     if (two) {
@@ -1398,29 +1401,57 @@ int launch_held_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y
 
 namespace fhip {
 
-// Where the held kernel is the faster one, us, the other kernels | it:
-// - up to 16 chunks (4096 columns) nearly always (the figures at the kernel). Not with one chunk and more than two tiles a CU, where the streaming
-//   kernel is one launch as well (8 rows, 12000 x 256 Q4_K 5.3 | 6.3; 8000 x 256 5.3 | 5.2), and at more than 8 rows of a tall weight not
-//   where the other kernels cut nothing along K (34000 x 512 Q4_K at 24 rows 16.8 | 18.3, Q5_K at 16 13.7 | 16.6).
-// - 17 to 24 chunks, two or three of them one after the other in a wave: 8 rows from half a tile a CU on (600 x 5120 Q4_K 9.4 | 11.3, 2000 x 5120
-//   11.9 | 11.8, 4096 x 5120 14.4 | 12.4) but for the first quarter of a second pass (4600 x 5120 14.7 | 15.6, 5120 x 5120 16.4 | 15.4); 9..16
-//   rows from a quarter of a tile a CU (2000 x 5120 16.0 | 12.4) to four (34000 x 5120 54.8 | 56.5); more rows of a format with minima, whose other
-//   kernel is the slower one, to two (600 x 5120 Q4_K at 32 17.8 | 11.8, 8000 41.6 | 30.8, 34000 83.7 | 97.9), of Q6_K while the sets
-//   of all tiles are two and a half a CU (3000 x 5120 at 24 23.5 | 19.4, 4096 22.0 | 22.8).
-bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+// Where the held kernel is the faster one: the other kernels' time over its own (above 1: faster), cold weights, sums in order. Tiles (of 16 weight rows) are counted in
+// the chip's CUs.
+// - One chunk (256 columns): up to three and a half tiles a CU: Q4_K at 8 rows 3.4 tiles 1.13, 4.4 1.01, 6.6 0.91, at 16 3.4 1.24, 5.9 0.81; Q8_0 at 8 to twelve (8.5 1.19, 17 1.02).
+// - 2 to 16 chunks, up to eight rows: always (Q4_K 2048 columns 0.1 tiles 1.59, 1.0 1.68, 37 1.22), but for two or three of a K-quant with more than 24 tiles (Q4_K 512
+//   columns 24 tiles 1.06, 37 0.90). Nine to sixteen: with long rows always (Q4_K 4096 columns 8.5 tiles 1.55, 37 1.35), with few chunks until the others cut
+//   nothing along K (Q5_K 1024 columns 5.9 tiles 1.83, 11.7 0.93); Q6_K from four chunks to 24 tiles (17 tiles 1.22; 37 of 5 chunks 0.87), Q8_0 from two always (17 1.25). More: four tiles, to nine
+//   where the others cut (Q4_K at 32 rows, 1024 columns 6.6 tiles 2.06, 8.5, not cut, 0.97).
+// - 17 to 24 chunks, two or three of them one after the other in a wave. Up to eight rows: Q4_K and Q5_K from half a tile on (5120 columns 0.2 tiles 0.90, 0.5 1.01,
+//   0.7 1.05), Q6_K and Q8_0 from where the others' units (128 rows x a chunk) are more than the CUs (0.2 0.89, 0.5 1.08). With minima, not in a second pass of tiles while
+//   the others have three units a CU at most, which run side by side (Q5_K 1.06 tiles of 20 chunks 0.93, 1.25 1.07). More rows: up to HELD_TILES, 20 chunks, last
+//   inside | first outside: Q4_K at 16 rows 11.7 tiles 1.05 | 24 0.96, at 24 8.5 1.04 | 17 0.87, at 32 4.4 1.13 | 6.6 0.99; Q5_K 3.4 1.05 | 5.9 0.96, 6.6 1.08 |
+//   8.5 0.98, 4.4 1.07 | 6.6 0.92; Q6_K 8.5 1.12 | 11.7 0.96, 2.9 1.22 | 6.6 1.02, 2.9 1.07 | 4.4 1.00; Q8_0 8.5 1.08 | 11.7 0.96.
+// - Beyond that, Q6_K and Q8_0 of 17 to 24 chunks at up to sixteen rows and any Q6_K at more, whose other kernel keeps two and one workgroup a CU: where its last round is
+//   mostly idle (16 rows 17 tiles, 547 workgroups of 1024, Q6_K 1.20 .. 1.36, Q8_0 1.25 .. 1.27, 11.7 tiles, 375 of 512, 0.94 .. 0.97; Q6_K at 24 rows 8.5 tiles, 272 of
+//   512, 1.20 .. 1.56, 5.9, 188 of 256, 0.91 .. 1.16, 6.6, 211 of 256, 0.88 .. 1.05; at 32 8.5 1.02 .. 1.27, 17, 547 of 768, 0.78 .. 0.97).
+// - summed_later: the next launch adds the others' partial sums as it reads them, and Q6_K at 17 rows and more then loses 1 - 13 % with more than 16 chunks or, at 32
+//   rows, two tiles a CU (feed-forward block 2560 x 9728 at 32 rows 63.3 us with the others, 69.6 with it; 2560 x 4096 at 32 46.3 | 46.3).
+// - Sums by atomics (FHIP_BATCH_AUTO) save the others a launch: of 13 to 16 chunks at up to eight rows from half a tile on (Q4_K 4096 columns 0.2 tiles 0.89, 0.7 1.09), of
+//   9 to 16 at more than 16 four tiles at most (Q4_K 3072 columns at 32 rows 4.4 tiles 1.01, 6.6 0.82), of more: up to eight rows from one and a half (Q8_0 5120 columns
+//   0.5 tiles 0.98, 2.0 1.31), with minima only over 20 chunks (Q4_K 20 chunks 2.2 tiles 0.89, 24 1.05), to sixteen a half to four (Q4_K 0.2 0.85, 0.5 1.03, 2.9 1.05, 6.6 0.89; not
+//   Q5_K, 2.2 0.87), to 24 three, to 32 two (Q4_K 2.9 1.04, 4.4 0.90; 2.0 1.04, 2.9 0.90), Q6_K while tiles times sets of eight rows are two and a half (24 rows 0.7 1.07, 1.0 0.88).
+constexpr int HELD_TILES[3][3] = {{12, 9, 6}, {4, 7, 5}, {9, 4, 3}};   // Q4_K; Q5_K; Q6_K and Q8_0: at up to 16, 24, 32 rows
+int places_taken(const Plan& q) { return (int)(100 * q.groups / ((q.groups + q.wgs - 1) / q.wgs * q.wgs)); }   // percent of its rounds' workgroups
+bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y, bool summed_later) {
     if (!gemm_f16x2_supports(w, t) || !d_x || ((uintptr_t)d_x & 15) != 0 || w->rows > 0x7FFFFF00ull) return false;
     // (all workgroups read the rows: none may have written over them)
     if ((uintptr_t)d_y < (uintptr_t)(d_x + t * w->cols) && (uintptr_t)d_x < (uintptr_t)(d_y + t * w->rows)) return false;
     const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16, sets = (t + 7) / 8;
     const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
-    if (chunks == 1) { if (tiles > 2 * cus) return false; }
-    else if (chunks > 24) return false;
-    else if (chunks > 16) {
-        if (t <= 8) return 2 * tiles >= cus && (tiles <= cus || 4 * tiles >= 5 * cus);
-        if (t <= 16) { if (4 * tiles < cus || tiles > 4 * cus) return false; }
-        else if (w->type == FHIP_Q6_K ? 2 * tiles * sets > 5 * cus : tiles > 2 * cus) return false;
+    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, atomics = w->batch_policy != FHIP_BATCH_ORDERED;
+    if (chunks > 24) return false;
+    if (chunks == 1) return 2 * tiles <= 7 * cus || (q8 && t <= 8 && tiles <= 12 * cus);
+    if (t <= 8) {
+        if (chunks <= 3) return q8 || tiles <= 24 * cus;
+        if (chunks <= 16) return !atomics || chunks <= 12 || 2 * tiles > cus;
+        if (atomics) return (q6 || q8 || chunks > 20) && 2 * tiles > 3 * cus;
+        if (q6 || q8) return (w->rows + 127) / 128 * chunks > cus;
+        return 2 * tiles >= cus && (tiles <= cus || tiles * chunks > 24 * cus);
     }
-    return t <= 8 || tiles <= 4 * cus || make_plan(w, t).split;
+    if (t <= 16) {
+        if (chunks <= 16) return tiles <= 4 * cus || q8 || chunks >= (q6 && tiles <= 24 * cus ? 4 : 8) || make_plan(w, t).split;
+        if ((q6 || q8) && tiles > 9 * cus) return places_taken(make_plan(w, t)) < 70;
+        if (atomics) return w->type != FHIP_Q5_K && 2 * tiles >= cus && tiles <= 4 * cus;
+        return tiles <= HELD_TILES[w->type == FHIP_Q4_K ? 0 : w->type == FHIP_Q5_K ? 1 : 2][0] * cus;
+    }
+    const Plan q = make_plan(w, t);
+    if (summed_later && q6 && q.split && (chunks > 16 || (t > 24 && tiles > 2 * cus))) return false;
+    if (q6 && (t <= 24 && !atomics ? tiles > 4 * cus : q.groups > q.wgs) && places_taken(q) < (t <= 24 ? 70 : 60)) return true;
+    if (chunks <= 16) return tiles <= 4 * cus || (tiles <= 9 * cus && q.split && !(atomics && chunks > 8));
+    if (atomics) return q6 ? 2 * tiles * sets <= 5 * cus : tiles <= (t <= 24 ? 3 : 2) * cus;
+    return tiles <= HELD_TILES[w->type == FHIP_Q4_K ? 0 : w->type == FHIP_Q5_K ? 1 : 2][sets - 2] * cus;
 }
 
 int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {

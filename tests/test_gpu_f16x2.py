@@ -376,11 +376,14 @@ def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows,
     (Q4_K, 1, 512, 8), (Q4_K, 17, 2048, 5), (Q5_K, 31, 2304, 7), (Q6_K, 4100, 1024, 8), (Q8_0, 15, 2080, 6), (Q8_0, 257, 4096, 8),      # 8 and 16 waves
     (Q4_K, 33, 4096, 9), (Q6_K, 100, 768, 16), (Q8_0, 4200, 288, 13), (Q5_K, 48, 2048, 17), (Q6_K, 130, 4096, 25), (Q4_K, 64, 512, 32),  # sets apart
     (Q4_K, 16400, 1024, 12), (Q6_K, 16390, 2304, 16), (Q8_0, 16385, 2080, 9), (Q8_0, 17000, 992, 8),                        # tall: sets together
-    (Q6_K, 2050, 4352, 8), (Q8_0, 2064, 6112, 5), (Q4_K, 5130, 6144, 7), (Q5_K, 1040, 5120, 16), (Q4_K, 700, 4608, 20), (Q6_K, 5130, 5120, 8)])  # 17 to 24 chunks
+    (Q6_K, 2050, 4352, 8), (Q8_0, 2064, 6112, 5), (Q4_K, 5130, 6144, 7), (Q5_K, 1040, 5120, 16), (Q4_K, 700, 4608, 20), (Q6_K, 5130, 5120, 8),  # 17 to 24 chunks
+    (Q4_K, 600, 5120, 12), (Q8_0, 4200, 5152, 16), (Q6_K, 1300, 4608, 32), (Q8_0, 2100, 4384, 5), (Q4_K, 4360, 6144, 8),   # twelve waves, one tile or several; eight
+    (Q4_K, 3110, 512, 30), (Q8_0, 14300, 256, 6)])  # two workgroups a CU; one chunk
 def test_whole_rows_inside_a_workgroup(F, O, ty, rows, cols, t):
     # The one-launch product at the edges of its tiles (16 weight rows), of its sets (8 activation rows) and of the chunks its waves hold (a last
     # wave without one, Q8_0's partial chunk), at the bar of the kernels it stands in for; a row of inf or NaN stays alone, and a second run
     # has the same bits.
+    from conftest import ROUTES, route
     from ferric_amd.synth import synth_weights
     w = synth_weights(ty, rows, cols, rows + t)
     x = np.random.default_rng(cols + t).standard_normal((t, cols)).astype(np.float32)
@@ -388,6 +391,8 @@ def test_whole_rows_inside_a_workgroup(F, O, ty, rows, cols, t):
     x[1], x[t - 1, -3] = 0.0, np.nan
     x[t - 2, 1] = -np.inf
     qm, xt = F.QMatrix.from_bytes(w, ty, rows, cols), F.Tensor.from_vec(x, x.shape)
+    qm.batch_policy(F.BATCH_ORDERED)
+    assert route(F, qm, xt, t) == [(ROUTES["HELD"], t)]
     good = np.arange(t - 2)
     y64, wn = O.matmul_f64(x[good], w, ty, rows, cols)
     bound = TIGHT * wn[None, :] * np.linalg.norm(x[good].astype(np.float64), axis=1)[:, None]
