@@ -328,8 +328,7 @@ def test_ordered_policy_gives_the_same_bits_on_every_run(F, O):
         y = xt.ffn(wgu, wdn).to_vec()
         for _ in range(3):
             assert np.array_equal(xt.ffn(wgu, wdn).to_vec(), y)
-        # the block leaves gate|up's partial sums to the launch that prepares the down projection's activations; the three
-        # calls it stands for add them in a launch of their own, in the same order: the same bits
+        # the three calls the block stands for: the same bits
         steps = xt.try_matmul_swiglu(wgu).matmul_q(wdn).to_vec()
         assert np.array_equal(steps, y)
         wgu.batch_policy(0), wdn.batch_policy(0)
@@ -345,21 +344,46 @@ def test_ordered_policy_gives_the_same_bits_on_every_run(F, O):
         lib.fhip_batch_policy(before)
 
 
-@pytest.mark.parametrize("ty,rows,cols", [(8, 130, 32), (8, 33, 288), (8, 600, 512), (12, 40, 256), (12, 1100, 512), (13, 300, 512), (14, 600, 256), (14, 129, 512)])
-def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows, cols):
-    """A small weight's ordered launch converts its chunks itself; fhip_matmul_q_f16x2 prepares them by a launch of its own. Up to two chunks
-    (sums of two terms, whose order does not matter) both have the same bits, for every number of rows the kernel takes, a last
+@pytest.mark.parametrize("ty,n_embd,n_ff,out,t,own", [(Q4_K, 7168, 256, 14400, 8, True), (Q6_K, 6400, 256, 14401, 5, True), (Q5_K, 7168, 256, 14400, 20, False),
+                                                       (Q6_K, 10240, 256, 14400, 12, True), (Q4_K, 5120, 17408, 515, 32, False)])
+def test_ffn_leaves_the_sums_of_a_cut_gate_up_to_the_next_launch(F, ty, n_embd, n_ff, out, t, own):
+    # gate|up whose rows are cut along K between workgroups: the block leaves its partial sums to the launch that prepares the down projection's
+    # activations; the three calls it stands for add them in a launch of their own, in the same order: the same bits
+    # (on down projections whose rows are prepared in three calls too)
+    from conftest import ROUTES, route
+    from ferric_amd.synth import synth_weights
+    wgu = F.QMatrix.from_bytes(synth_weights(ty, 2 * n_ff, n_embd, 36), ty, 2 * n_ff, n_embd)
+    wdn = F.QMatrix.from_bytes(synth_weights(Q6_K, out, n_ff, 37), Q6_K, out, n_ff)
+    wgu.batch_policy(F.BATCH_ORDERED), wdn.batch_policy(F.BATCH_ORDERED)
+    xt = F.Tensor.from_vec(np.random.default_rng(38).standard_normal((t, n_embd)).astype(np.float32), (t, n_embd))
+    assert route(F, wgu, xt, t) == [((ROUTES["OWN_ROWS"] if own else ROUTES["PREPARED"]) | ROUTES["CUT"], t)]
+    h = xt.try_matmul_swiglu(wgu)
+    assert route(F, wdn, h, t)[0][0] != ROUTES["HELD"]
+    y = xt.ffn(wgu, wdn).to_vec()
+    assert np.isfinite(y).all() and np.array_equal(h.matmul_q(wdn).to_vec(), y)
+
+
+@pytest.mark.parametrize("ty,rows,cols,kernel,ts", [
+    (8, 130, 32, "HELD", (5, 7, 8, 9, 13, 16)), (8, 33, 288, "HELD", (5, 7, 8, 9, 13, 16)), (8, 600, 512, "HELD", (5, 7, 8, 9, 13, 16)), (12, 40, 256, "HELD", (5, 7, 8, 9, 13, 16)),
+    (12, 1100, 512, "HELD", (5, 7, 8, 9, 13, 16)), (13, 300, 512, "HELD", (5, 7, 8, 9, 13, 16)), (14, 600, 256, "HELD", (5, 7, 8, 9, 13, 16)), (14, 129, 512, "HELD", (5, 7, 8, 9, 13, 16)),
+    (12, 600, 5120, "OWN_ROWS", (5, 7, 8)), (13, 301, 7168, "OWN_ROWS", (5, 8)), (14, 130, 4608, "OWN_ROWS", (5, 7, 8)), (14, 129, 6400, "OWN_ROWS", (5, 8, 9, 13, 16)),
+    (8, 257, 5152, "OWN_ROWS", (5, 7, 8)), (8, 131, 6432, "OWN_ROWS", (5, 8, 9, 13, 16))])
+def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows, cols, kernel, ts):
+    """A launch that makes its chunks' operand rows itself; fhip_matmul_q_f16x2 prepares them by a launch of its own. Where two chunks
+    at most are not zero (sums of two terms, whose order does not matter) both have the same bits, for every number of rows the kernel takes, a last
     chunk that is not full, an odd number of weight rows, rows of zeros, chunks of tiny, huge and non-finite values."""
-    from conftest import bits
+    from conftest import ROUTES, bits, route
     from ferric_amd.synth import synth_weights
     rng = np.random.default_rng(rows + cols)
     lib = F._lib.load()
     w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 1), ty, rows, cols)
     w.batch_policy(F.BATCH_ORDERED)
-    for t in (5, 7, 8, 9, 13, 16):
+    for t in ts:
         x = (rng.standard_normal((t, cols)) * np.exp2(rng.integers(-20, 20, (t, 1)))).astype(np.float32)
         x[0, :30], x[1], x[2, 7], x[3, -1], x[4, 20] = 1e-41, 0.0, 3e38, -np.inf, np.nan
+        x[:, 256:(cols - 1) // 256 * 256] = 0.0
         xt, ws, ys = F.Tensor.from_vec(x, x.shape), F.DeviceBuffer(lib.fhip_matmul_q_f16x2_ws_bytes(w.handle, t)), []
+        assert [(k & ~ROUTES["CUT"], n) for k, n in route(F, w, xt, t)] == [(ROUTES[kernel], t)]
         for prepared in (False, True):
             y = F.Tensor.empty((t, rows))
             if prepared:
