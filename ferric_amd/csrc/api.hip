@@ -291,9 +291,8 @@ int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, cons
     return (own && !(cut && w->batch_policy != FHIP_BATCH_ORDERED) && fhip::gemm_f16x2_own_x(w, d_x, t) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (cut ? FHIP_ROUTE_CUT : 0);
 }
 // deferred: the ordered sum of K-split groups is left to the reader of y, which gets *deferred as its `src`
-int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
-                 fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
-    const int route = f16x2_route(w, d_x, t, !swiglu_in && !src, d_y, deferred != nullptr);
+int f16x2_launch(int route, const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
+                 fhip::F16Parts* deferred, const fhip::F16Parts* src) {
     if (route == FHIP_ROUTE_HELD) {
         if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0, 0, 128};
         return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
@@ -306,6 +305,10 @@ int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_i
     int rc = fhip::launch_xsplit_f16(w, d_x, t, swiglu_in, xp, s, clr ? d_y : nullptr, clr ? t * w->rows : 0, src);
     if (rc) return rc;
     return fhip::launch_gemm_f16x2(w, xp, t, d_y, s, clr, part, deferred);
+}
+int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
+                 fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
+    return f16x2_launch(f16x2_route(w, d_x, t, !swiglu_in && !src, d_y, deferred != nullptr), w, d_x, t, swiglu_in, d_y, d_ws, s, deferred, src);
 }
 
 }  // namespace
@@ -623,7 +626,12 @@ int fhip_matmul_q(const fhip_weight* w, const float* d_x, size_t rows_x, float* 
     if (!takes_f16x2(w, rows_x)) return fhip::launch_gemv(w, d_x, rows_x, d_y, 0, s);
     const size_t grp = f16x2_group(w);
     void* ws = nullptr;
-    if ((rc = lib_workspace(s, f16x2_matmul_ws(w, rows_x < grp ? rows_x : grp), &ws, "fhip_matmul_q"))) return rc;
+    if (rows_x <= grp) {   // one group: the held kernel needs no workspace
+        const int route = f16x2_route(w, d_x, rows_x, true, d_y, false);
+        if (route != FHIP_ROUTE_HELD && (rc = lib_workspace(s, f16x2_matmul_ws(w, rows_x), &ws, "fhip_matmul_q"))) return rc;
+        return f16x2_launch(route, w, d_x, rows_x, false, d_y, ws, s, nullptr, nullptr);
+    }
+    if ((rc = lib_workspace(s, f16x2_matmul_ws(w, grp), &ws, "fhip_matmul_q"))) return rc;
     for (size_t m0 = 0; m0 < rows_x; m0 += grp) {
         const size_t t = rows_x - m0 < grp ? rows_x - m0 : grp;
         if (takes_f16x2(w, t)) rc = f16x2_matmul(w, d_x + m0 * w->cols, t, false, d_y + m0 * w->rows, ws, s);

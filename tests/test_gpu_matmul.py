@@ -479,3 +479,30 @@ def test_batched_calls_inside_a_graph_need_the_workspace_reserved(F, O):
     lib.fhip_workspace_release(stream.handle)                                         # and a released workspace comes back on demand
     check(lib.fhip_ffn(gu.handle, dn.handle, xt.buf.ptr, batch, y.buf.ptr, ws.buf.ptr, stream.handle))
     assert np.abs(y.to_vec(stream) - eager).max() <= 2e-6 * np.abs(eager).max()
+
+
+def test_a_product_in_one_launch_is_captured_without_a_workspace(F):
+    """fhip_matmul_q on a batch whose rows' whole K lies inside a workgroup needs nothing beside its operands: a capture on a stream that has no
+    workspace takes it, and one it cannot serve is refused with nothing recorded."""
+    from conftest import ROUTES, route
+    from ferric_amd.synth import synth_weights
+    lib, check = F._lib.load(), F._lib.check
+    stream = F.Stream()
+    for rows, cols, t, held in ((1024, 1024, 8, True), (300, 7168, 8, False), (1024, 1024, 40, False)):
+        w = F.QMatrix.from_bytes(synth_weights(Q4_K, rows, cols, 41), Q4_K, rows, cols)
+        w.batch_policy(F.BATCH_ORDERED)
+        x = np.random.default_rng(42).standard_normal((t, cols)).astype(np.float32)
+        xt, y = F.Tensor.from_vec(x, x.shape), F.Tensor.empty((t, rows))
+        assert (route(F, w, xt, t) == [(ROUTES["HELD"], t)]) == held
+        g = F.Graph.begin(stream)
+        rc = lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, stream.handle)
+        g.end()
+        if not held:
+            assert rc == F._lib.ERR_ARG and "fhip_workspace_reserve" in F._lib.last_error()
+            continue
+        check(rc)
+        want = xt.matmul_q(w).to_vec()
+        for _ in range(3):
+            check(lib.fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
+            g.launch()
+            assert np.array_equal(y.to_vec(stream), want)
