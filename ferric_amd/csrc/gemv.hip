@@ -42,6 +42,7 @@
 // crates/ferric-gguf/src/lib.rs:497 then a dense dot): NaN stays NaN, inf * w is +-inf, inf * 0 is NaN.
 #include "common.hpp"
 #include "deq_at.hpp"
+#include "fixed_point.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -51,9 +52,6 @@
 // This file is compiled twice, once per activation precision (FHIP_GEMV_PLANES = 2 and 3); the two copies export their
 // launchers under different names and the precision of the weight handle picks between them at every launch. The kernel
 // carries the suffix too, so that a profiler's trace says which copy ran.
-#ifndef FHIP_GEMV_PLANES
-#define FHIP_GEMV_PLANES 2
-#endif
 #if FHIP_GEMV_PLANES == 2
 #define GEMV_EXPORT(name) name##_p2
 #else
@@ -63,15 +61,6 @@
 
 namespace {
 
-constexpr int NP = FHIP_GEMV_PLANES;   // byte planes per activation run
-static_assert(NP == 2 || NP == 3, "two or three activation planes");
-// Largest quantised magnitude: every digit at 127; the run's largest activation maps onto it. With two planes the rounding
-// of the reciprocal and of the product moves that by at most 0.02, never to the next integer; with three (8.4e6 * 2^-22 = 2)
-// the quantiser clamps.
-constexpr float QMAX = NP == 2 ? 32639.0f : 8355711.0f;
-constexpr float TINY_RUN = 7.888609052210118e-31f;   // 2^-100: below this QMAX / amax leaves the f32 range's comfortable part
-constexpr float HUGE_RUN = 7.922816251426434e28f;    // 2^96
-
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 struct __attribute__((packed, aligned(2))) U4A2 { u32x4 v; };
@@ -80,7 +69,6 @@ struct __attribute__((packed, aligned(2))) U2A2 { u32x2 v; };
 __device__ __forceinline__ float f16_bits(uint32_t b) { return __half2float(__ushort_as_half((unsigned short)b)); }
 __device__ __forceinline__ float ub(uint32_t v, int k) { return (float)((v >> (8 * k)) & 0xFFu); }
 __device__ __forceinline__ float sb(uint32_t v, int k) { return (float)(int8_t)((v >> (8 * k)) & 0xFFu); }
-__device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) { return __builtin_amdgcn_sdot4((int)a, (int)b, c, false); }
 
 // Keeps a prefetched row as the packed dwords that were loaded (otherwise the optimizer unpacks
 // bytes as soon as a load returns and carries the unpacked values across the pipeline, which spills).
@@ -88,13 +76,7 @@ __device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(u32x2& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(u32x4& v) { asm volatile("" : "+v"(v)); }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;   // quad_perm [1,0,3,2], [2,3,0,1]; row_*
+constexpr int DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;   // row_*
 constexpr int DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;   // rotate within the 16-lane row: lane l reads lane l - 4 / l - 8, so l & 3 is kept
 // All-reduce over the 16 lanes of a DPP row.
 __device__ __forceinline__ float slot_sum(float v) {
@@ -141,12 +123,6 @@ __device__ __forceinline__ int slot_of(int l) {
     if constexpr (U == 1) return 0;
     if constexpr (U == 2) return (l >> 1) & 1;
     return ((l & 1) << 1) | ((l >> 1) & 1);
-}
-
-// exact integer plane sums -> f32 (one rounding, at most 2^-24 relative)
-__device__ __forceinline__ float planes_f32(const int (&a)[NP]) {
-    if constexpr (NP == 2) return (float)((a[0] << 8) + a[1]);
-    else return fmaf((float)a[0], 65536.0f, (float)((a[1] << 8) + a[NP - 1]));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -705,63 +681,6 @@ template <class F> int wave_limit(int M, size_t cols, size_t wbytes) {
 }
 
 __device__ __forceinline__ uint32_t div_magic(uint32_t n, uint32_t magic) { return magic ? __umulhi(n, magic) : n; }
-
-// Eight consecutive activations of one run -> NP plane dword pairs, the run's scale and the run's quantised sum.
-// The 2 (RUN 16) or 4 (RUN 32) lanes of a run sit in one quad and agree on amax, the scale and the sum afterwards.
-template <int RUN>
-__device__ __forceinline__ void quantize8(const float (&v)[8], uint32_t (&pl)[NP][2], float& scale_out, float& sum_out) {
-    float amax = fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
-                       fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7]))));
-    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));   // NaN / inf detector (fmaxf drops NaNs)
-    amax = fmaxf(amax, dpp_f<DPP_XOR1>(amax));
-    sum += dpp_f<DPP_XOR1>(sum);
-    if (RUN == 32) {
-        amax = fmaxf(amax, dpp_f<DPP_XOR2>(amax));
-        sum += dpp_f<DPP_XOR2>(sum);
-    }
-    // not representable in block fixed point: non-finite members (their sum is not finite either), a run so large that a
-    // format's offset term (up to 128 times the run's sum) could leave the f32 range where the element-wise products do not,
-    // or a run so small that QMAX / amax would overflow
-    const bool special = !(fabsf(sum) <= 3.4028234663852886e38f) || amax > HUGE_RUN || (amax < TINY_RUN && amax > 0.f);
-    const float inv = amax > 0.f ? QMAX * __builtin_amdgcn_rcpf(amax) : 0.f;
-    uint32_t t[8];
-    if constexpr (NP == 2) {
-        // round to nearest by adding 1.5 * 2^23; the 128 makes the low byte an offset-binary digit
-#pragma unroll
-        for (int i = 0; i < 8; i++) t[i] = __float_as_uint(fmaf(v[i], inv, 12582912.0f + 128.0f));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            int q = __float2int_rn(v[i] * inv);
-            q = q > (int)QMAX ? (int)QMAX : (q < -(int)QMAX ? -(int)QMAX : q);
-            t[i] = (uint32_t)(q + 0x8080);
-        }
-    }
-#pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-        const uint32_t t0 = t[4 * hh], t1 = t[4 * hh + 1], t2 = t[4 * hh + 2], t3 = t[4 * hh + 3];
-        const uint32_t p01 = __builtin_amdgcn_perm(t1, t0, 0x05010400u), p23 = __builtin_amdgcn_perm(t3, t2, 0x05010400u);
-        pl[NP - 1][hh] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;   // bytes 0, back to signed digits
-        if constexpr (NP == 2) {
-            pl[0][hh] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);                  // bytes 1: the signed top digit
-        } else {
-            pl[1][hh] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
-            const uint32_t u01 = __builtin_amdgcn_perm(t1, t0, 0x00000602u), u23 = __builtin_amdgcn_perm(t3, t2, 0x00000602u);
-            pl[0][hh] = __builtin_amdgcn_perm(u23, u01, 0x05040100u);                  // bytes 2
-        }
-    }
-    int qs[NP];
-#pragma unroll
-    for (int p = 0; p < NP; p++) qs[p] = dot4(pl[p][1], 0x01010101u, dot4(pl[p][0], 0x01010101u, 0));
-    int qsum = qs[0];
-#pragma unroll
-    for (int p = 1; p < NP; p++) qsum = (qsum << 8) + qs[p];
-    qsum += dpp_i<DPP_XOR1>(qsum);
-    if (RUN == 32) qsum += dpp_i<DPP_XOR2>(qsum);
-    const float scale = amax * (1.0f / QMAX);
-    scale_out = special ? __uint_as_float(0x7FC00000u) : scale;
-    sum_out = scale * (float)qsum;
-}
 
 template <class F, int M, int U, bool SWIGLU, bool NORM, bool LATE>
 __global__ void __launch_bounds__(max_threads<F>(M)) gemv_stream_kernel(GemvParams p) {

@@ -30,12 +30,10 @@
 // Built once per activation precision like gemv.hip (FHIP_GEMV_PLANES = 2 or 3).
 #include "common.hpp"
 #include "deq_at.hpp"
+#include "fixed_point.hpp"
 
 #include <hip/hip_fp16.h>
 
-#ifndef FHIP_GEMV_PLANES
-#define FHIP_GEMV_PLANES 2
-#endif
 #if FHIP_GEMV_PLANES == 2
 #define QUAD_EXPORT(name) name##_p2
 #else
@@ -44,13 +42,6 @@
 #define gemv_quad_kernel QUAD_EXPORT(gemv_quad_kernel)
 
 namespace {
-
-constexpr int NP = FHIP_GEMV_PLANES;
-static_assert(NP == 2 || NP == 3, "two or three activation planes");
-// the quantiser's constants: those of gemv.hip, or the two kernels' bits part
-constexpr float QMAX = NP == 2 ? 32639.0f : 8355711.0f;
-constexpr float TINY_RUN = 7.888609052210118e-31f;   // 2^-100
-constexpr float HUGE_RUN = 7.922816251426434e28f;    // 2^96
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -61,28 +52,14 @@ struct __attribute__((packed, aligned(2))) U2A2 { u32x2 v; };
 __device__ __forceinline__ float f16_bits(uint32_t b) { return __half2float(__ushort_as_half((unsigned short)b)); }
 __device__ __forceinline__ float ub(uint32_t v, int k) { return (float)((v >> (8 * k)) & 0xFFu); }
 __device__ __forceinline__ float sb(uint32_t v, int k) { return (float)(int8_t)((v >> (8 * k)) & 0xFFu); }
-__device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) { return __builtin_amdgcn_sdot4((int)a, (int)b, c, false); }
 __device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(u32x2& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(u32x4& v) { asm volatile("" : "+v"(v)); }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;   // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;   // lane l of a 16-lane row reads lane l - 4 / l - 8 of the row
 // the value lane `src` holds
 __device__ __forceinline__ float lane_read(float v, int src) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(v)));
-}
-
-// exact integer plane sums -> f32 (one rounding), as gemv.hip
-__device__ __forceinline__ float planes_f32(const int (&a)[NP]) {
-    if constexpr (NP == 2) return (float)((a[0] << 8) + a[1]);
-    else return fmaf((float)a[0], 65536.0f, (float)((a[1] << 8) + a[NP - 1]));
 }
 
 __device__ __forceinline__ i32x4 mma(uint32_t a, uint32_t b, i32x4 c) { return __builtin_amdgcn_mfma_i32_4x4x4i8((int)a, (int)b, c, 0, 0, 0); }
@@ -363,60 +340,6 @@ struct Q6K {
         }
     }
 };
-
-// Eight consecutive activations of one run -> NP plane dword pairs, the run's scale and the run's quantised sum: the
-// streaming mat-vec's quantiser (gemv.hip), operation for operation. The 2 (RUN 16) or 4 (RUN 32) lanes of a run sit in one
-// quad and agree on the maximum, the scale and the sum afterwards.
-template <int RUN>
-__device__ __forceinline__ void quantize8(const float (&v)[8], uint32_t (&pl)[NP][2], float& scale_out, float& sum_out) {
-    float amax = fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))),
-                       fmaxf(fmaxf(fabsf(v[4]), fabsf(v[5])), fmaxf(fabsf(v[6]), fabsf(v[7]))));
-    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));   // NaN / inf detector (fmaxf drops NaNs)
-    amax = fmaxf(amax, dpp_f<DPP_XOR1>(amax));
-    sum += dpp_f<DPP_XOR1>(sum);
-    if (RUN == 32) {
-        amax = fmaxf(amax, dpp_f<DPP_XOR2>(amax));
-        sum += dpp_f<DPP_XOR2>(sum);
-    }
-    const bool special = !(fabsf(sum) <= 3.4028234663852886e38f) || amax > HUGE_RUN || (amax < TINY_RUN && amax > 0.f);
-    const float inv = amax > 0.f ? QMAX * __builtin_amdgcn_rcpf(amax) : 0.f;
-    uint32_t t[8];
-    if constexpr (NP == 2) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) t[i] = __float_as_uint(fmaf(v[i], inv, 12582912.0f + 128.0f));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            int q = __float2int_rn(v[i] * inv);
-            q = q > (int)QMAX ? (int)QMAX : (q < -(int)QMAX ? -(int)QMAX : q);
-            t[i] = (uint32_t)(q + 0x8080);
-        }
-    }
-#pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-        const uint32_t t0 = t[4 * hh], t1 = t[4 * hh + 1], t2 = t[4 * hh + 2], t3 = t[4 * hh + 3];
-        const uint32_t p01 = __builtin_amdgcn_perm(t1, t0, 0x05010400u), p23 = __builtin_amdgcn_perm(t3, t2, 0x05010400u);
-        pl[NP - 1][hh] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
-        if constexpr (NP == 2) {
-            pl[0][hh] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
-        } else {
-            pl[1][hh] = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
-            const uint32_t u01 = __builtin_amdgcn_perm(t1, t0, 0x00000602u), u23 = __builtin_amdgcn_perm(t3, t2, 0x00000602u);
-            pl[0][hh] = __builtin_amdgcn_perm(u23, u01, 0x05040100u);
-        }
-    }
-    int qs[NP];
-#pragma unroll
-    for (int p = 0; p < NP; p++) qs[p] = dot4(pl[p][1], 0x01010101u, dot4(pl[p][0], 0x01010101u, 0));
-    int qsum = qs[0];
-#pragma unroll
-    for (int p = 1; p < NP; p++) qsum = (qsum << 8) + qs[p];
-    qsum += dpp_i<DPP_XOR1>(qsum);
-    if (RUN == 32) qsum += dpp_i<DPP_XOR2>(qsum);
-    const float scale = amax * (1.0f / QMAX);
-    scale_out = special ? __uint_as_float(0x7FC00000u) : scale;
-    sum_out = scale * (float)qsum;
-}
 
 // Q8_0: 34 B = [f16 d][32 int8] (crates/ferric-gguf/src/lib.rs:608-615). Unit = one block: the quants are the B operand as they
 // lie in memory.
