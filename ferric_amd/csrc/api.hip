@@ -109,10 +109,10 @@ size_t device_lds_bytes() { return g_lds; }
 // Batches of the 32-value formats from here on go up to sixteen rows at a time through the kernel that multiplies on the 16 x 16 x 32
 // int8 matrix instruction (gemv_wide.hip: the same bits per row); what is left of a batch goes on as a batch of its own. Its cost is the quantiser's, per activation row and workgroup,
 // plus the weight once; the dot-product kernel's is a launch and the weight per four rows. us, cold, dot-product | wide, three rows:
-// IQ4_NL 1024 x 5120 7.8 | 10.1, 4096 x 4096 9.6 | 10.1, 9728 x 2560 11.7 | 10.8, 34816 x 5120 43 | 30.5; four: Q4_0 1024 x 5120 9.4 | 10.3,
-// 1946 x 1504 6.8 | 7.7, 4096 x 4096 12.8 | 9.8, 34816 x 5120 43 | 29.7; five: 1024 x 1024 9.7 | 8.0, 1024 x 5120 13.8 | 11.8, 34816 x 5120
-// 60 | 38; sixteen: 1467 x 1760 38.8 | 15.8, 4096 x 4096 50 | 23, 34816 x 5120 171 | 61. Q8_0 has the others at three
-// and four rows of up to 5120 columns (three, 4096 x 4096 9.6 | 11.5).
+// IQ4_NL 1024 x 5120 7.9 | 9.7, 4096 x 4096 10.0 | 9.7, 9728 x 2560 12.5 | 11.1, 34816 x 5120 42.9 | 33.6, Q4_0 4096 x 4096 8.9 | 9.4; four: Q4_0 1024 x 5120 9.3 | 9.7,
+// 1946 x 1504 6.5 | 6.5, 4096 x 4096 13.1 | 9.6, 34816 x 5120 42.3 | 32.6; five: 1024 x 1024 8.8 | 5.7, 1024 x 5120 13.5 | 11.2, 34816 x 5120 62.9 | 38.9; sixteen: IQ4_NL
+// 1467 x 1760 37.1 | 12.1, Q4_0 4096 x 4096 50.9 | 20.9, 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up to 5120 columns: three, dot-product |
+// wide, 4096 x 4096 9.6 | 10.7; four, four-row | wide, 34816 x 5120 48.4 | 57.5, 5120 x 5120 15.1 | 17.5, 2048 x 4096 10.1 | 10.8 (but 4096 x 4096 12.5 | 11.0, 12288 x 4096 22.8 | 19.6).
 bool takes_wide(const fhip_weight* w, size_t t) {
     const size_t weights = w->rows * w->cols;
     if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
@@ -236,9 +236,9 @@ static int gemm_bf16_lib_ws(const fhip_weight* w, const uint16_t* d_x, size_t t,
 // ---- which kernel a batch takes ---------------------------------------------------------------------------------------------
 // One or two activation rows go through the streaming mat-vec (one pass over the weights serves two rows). From three rows on
 // (five for Q8_0) the f16 hi/lo matrix-core kernels read the weights once for up to 32 (Q8_0: 16) rows; longer batches are cut
-// into such groups. FHIP_BATCH_F32_MATVEC keeps every batch on the mat-vec's arithmetic (launch_gemv: four rows a pass on the
-// int8 matrix instruction for Q4_K / Q5_K / Q6_K, the dot-product kernel otherwise): a row then has the same bits whatever batch it
-// is part of.
+// into such groups. FHIP_BATCH_F32_MATVEC keeps every batch on the mat-vec's arithmetic (launch_gemv: four rows a pass for Q4_K /
+// Q5_K / Q6_K, up to sixteen for the 32-value formats, on the int8 matrix instructions, a few rows on the dot-product kernel): a row then has the same
+// bits whatever batch it is part of.
 
 size_t f16x2_group(const fhip_weight* w) { return w->type == FHIP_Q8_0 ? 16 : 32; }
 // Three and four rows of a Q4_K / Q5_K / Q6_K weight whose rows the four-row mat-vec (gemv_quad.hip) covers in one pass (up to 10240

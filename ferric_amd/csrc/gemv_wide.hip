@@ -23,9 +23,9 @@
 // What bounds it: instruction issue, twice. A block of a tile takes E matrix instructions (16 cycles each) and some 12 + 11 E
 // vector instructions (four cycles each) at E pairs a lane; the quantiser takes about 16 per activation value and is repeated by
 // every workgroup, 0.6 us an activation row of 4096 columns, which is what a batch of sixteen on a small weight spends its time on.
-// us, cold, dot-product kernel -> this one, 24 bits: Q4_0 34816 x 5120 at 4 / 8 / 16 rows 42.7 / 84.9 / 167.9 -> 28.4 / 37.1 / 58.8 (the
-// 100 MB of the weight: 18), 4096 x 4096 12.9 / 25.0 / 49.0 -> 9.3 / 12.0 / 21.7; MXFP4 9728 x 2560 14.3 / 27.9 / 55.4 -> 10.8 / 12.2 / 20.9;
-// IQ4_NL 1467 x 1760 at 16 rows 38.5 -> 12.3.
+// us, cold, dot-product kernel -> this one, 24 bits: Q4_0 34816 x 5120 at 4 / 8 / 16 rows 42.3 / 84.1 / 169 -> 32.6 / 41.0 / 64.0 (the
+// 100 MB of the weight: 18), 4096 x 4096 13.1 / 25.6 / 50.9 -> 9.6 / 12.3 / 20.9; MXFP4 9728 x 2560 15.1 / 28.3 / 55.9 -> 11.7 / 13.1 / 21.8;
+// IQ4_NL 1467 x 1760 at 16 rows 37.1 -> 12.1.
 //
 // Built once per activation precision like gemv.hip (FHIP_GEMV_PLANES = 2 or 3).
 #include "common.hpp"

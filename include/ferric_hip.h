@@ -184,10 +184,12 @@ int fhip_deq_raw(const uint8_t* h_raw, size_t nbytes, size_t n, uint32_t ggml_ty
  * :1172 matmul_q6_k): y[rows_x, rows] = x[rows_x, cols] * W^T, f32 in, f32 accumulate, f32 out.
  * rows_x = 1 is the decode GEMV; any rows_x >= 1 is accepted.
  * Which kernel a batch takes (fhip_batch_policy): one or two rows go through the streaming mat-vec; three and four rows of a
- * Q4_K / Q5_K / Q6_K weight with rows of up to 10240 columns (Q8_0: 5120) through its four-row form (the same arithmetic on the int8 matrix
- * instruction: every row has the bits it has in a batch of one; one launch, no workspace); otherwise, from three rows on (five
+ * Q4_K / Q5_K / Q6_K weight with rows of up to 10240 columns (Q8_0: four rows, 5120 columns) through its four-row form (the same arithmetic on the int8 matrix
+ * instruction: every row has the bits it has in a batch of one; one launch, no workspace), three rows and more of the other 32-value formats, up to sixteen a
+ * pass, through its wide form (the same, without a workspace too); otherwise, from three rows on (five
  * for Q8_0) Q4_K / Q5_K / Q6_K / Q8_0 weights are read once per group of up to 32 (Q8_0: 16) rows by the f16 hi/lo matrix-core
- * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. That path keeps its
+ * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Most products of up to 6144
+ * columns are one launch that needs nothing beside its operands. The others keep their
  * prepared activations in a workspace the library owns per stream (fhip_workspace_reserve); inside a graph capture the
  * workspace cannot grow, and the call then fails with FHIP_ERR_ARG and says how many bytes to reserve beforehand.
  * Non-finite activations: on the mat-vec kernel a NaN or infinite x gives what the f32 dot gives (NaN, +-inf by the weight's
@@ -212,7 +214,8 @@ int fhip_swiglu(const float* d_gu, size_t t, size_t d, float* d_out, void* strea
  * d_ws is caller-provided scratch of at least rows_x * n_ff f32 (n_ff = gate_up rows / 2). Batches of three rows and more
  * run as fhip_ffn_f16x2 does (one pass over each weight per group of up to 32 rows) out of the library's workspace; in a
  * group of three or four rows gate|up + SwiGLU is the call fhip_matmul_q_swiglu makes for such a batch, and the block gives
- * the bits of that call followed by fhip_matmul_q on the down projection. */
+ * the bits of that call followed by fhip_matmul_q on the down projection. Of more rows its value to f32 rounding: the block prepares the down
+ * projection's rows with the SwiGLU, where the call by itself may be one launch that sums in another order. */
 int fhip_ffn(const fhip_weight* gate_up, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
              float* d_ws, void* stream);
 
@@ -429,7 +432,7 @@ int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_re
 /* fhip_ffn for callers that cannot allocate or bring a workspace (code under graph capture, tight serving loops, harnesses
  * that forbid hipMalloc): the [rows_x, n_ff] intermediate lives in a 512 KiB array built into the library's code object (one
  * copy per device, held until the process ends), so the call takes inputs and outputs only and calls no allocating routine.
- * Always the mat-vec kernels (two rows per pass over the weights), so its result has the bits of fhip_ffn under
+ * Always the mat-vec kernels (FHIP_BATCH_F32_MATVEC's), so its result has the bits of fhip_ffn under
  * FHIP_BATCH_F32_MATVEC. rows_x * n_ff > 131072 floats: FHIP_ERR_SHAPE. Every call on a device shares that device's array:
  * calls that overlap in time on one GPU (two streams, two threads) race on it. It has no counterpart in the reference. */
 int fhip_ffn_noalloc(const fhip_weight* gate_up, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y, void* stream);
@@ -444,9 +447,9 @@ int fhip_ffn_noalloc(const fhip_weight* gate_up, const fhip_weight* down, const 
  * last bits vary from run to run (within 2e-6 of the largest output).
  * FHIP_BATCH_F32_MATVEC: the streaming mat-vec's arithmetic for every row; an output row then has the same bits whatever
  * batch it was part of (the guarantee the reference's CPU path gives, crates/ferric-tensor/src/cpu_simd.rs:175-200), at the
- * price of one pass over the weights per four rows (Q4_K, Q5_K, Q6_K and short-row Q8_0: the products of four rows at a time go through the
- * 4 x 4 x 4 int8 matrix instruction, three quarters of the time of two dot-product passes; other formats: two to four rows
- * a pass on the dot-product kernel).
+ * price of one pass over the weights per four rows (Q4_K, Q5_K, Q6_K: the products of four rows at a time go through the 4 x 4 x 4 int8 matrix
+ * instruction, three quarters of the time of two dot-product passes) or sixteen (the 32-value formats, through the 16 x 16 x 32 one; three and
+ * four rows of a small weight on the dot-product kernel, four of Q8_0 of up to 5120 columns on the 4 x 4 x 4 one).
  * fhip_weight_batch_policy sets one handle's policy and returns the one before; any value that is no policy only queries. Set it
  * before sizing or reserving the workspace and not while another thread launches on the handle.
  * fhip_batch_policy sets what handles made AFTERWARDS start with (existing handles keep theirs) and returns the previous
