@@ -39,7 +39,7 @@ def kernel_source_sha():
     code than the one that runs can be told."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("gemv.hip", "common.hpp", "deq_at.hpp"):
+    for name in ("gemv.hip", "common.hpp", "deq_at.hpp", "fixed_point.hpp"):
         with open(os.path.join(ROOT, "ferric_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
