@@ -848,36 +848,40 @@ __global__ __launch_bounds__(64 * WV) void attn_split_fused_kvq_kernel(QkvPostPa
 
 // One workgroup per query head: weights exp(m_s - max m) of the splits once (each wave reduces them for itself; through LDS to
 // the threads that need one), then every output dim is a weighted sum of the splits' accumulators over the weighted sum of their
-// sums. splits <= 256. Thread (group, dim): group i of COMBINE_GROUPS takes splits i, i + COMBINE_GROUPS, ..., the groups meet in LDS.
+// sums. splits <= 256. Thread (group, dim): group i of GROUPS takes splits i, i + GROUPS, ..., EARLY of them at once, the groups meet in LDS.
 // Nothing but latency: with one thread a dim the splits came in six trips to memory one after the other, now in one (up to 64 splits;
-// 128 in two): 40 heads of 128, 64 splits 5.0 us, 20 heads, 128 splits 8.4.
-constexpr int COMBINE_GROUPS = 8;
-__global__ __launch_bounds__(128 * COMBINE_GROUPS) void attn_combine_kernel(const float* __restrict__ part, int hd, int splits, float* __restrict__ out) {
-    __shared__ float w[256];
-    __shared__ float red[COMBINE_GROUPS][128];
-    const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, grp = tid / hd, d = tid - grp * hd;   // (hd: 64 or 128)
+// 128 in two): 40 heads of 128, 64 splits 5.0 us, 20 heads, 128 splits 8.4. A workgroup of sixteen waves takes longer to start and to meet, though, than a
+// few splits take to add: one thread a dim | four | eight, us with the attention launch: 6 splits of 8 heads 6.3 | 6.6 | 7.2, 16 of 40 8.8 | 9.1 | 9.7, 24 of 8 without grouped
+// heads 8.2 | 7.9 | 8.4, 41 of 8 heads 8.5 | 8.0 | 8.6, 52 10.4 (four) | 10.6, 64 of 40 24.7 | 23.6 | 23.6.
+template <int GROUPS, int EARLY, int SPLITS>   // SPLITS: at most
+__global__ __launch_bounds__(128 * GROUPS) void attn_combine_kernel(const float* __restrict__ part, int hd, int splits, float* __restrict__ out) {
+    constexpr int NM = (SPLITS + 63) / 64;
+    __shared__ float w[64 * NM];
+    __shared__ float red[GROUPS][128];
+    const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, grp = GROUPS == 1 ? 0 : tid / hd, d = tid - grp * hd;   // (hd: 64 or 128)
     const float* pp = part + (size_t)head * splits * (hd + 2);
-    // the first eight of the thread's splits are requested together with the splits' maxima and sums
-    constexpr int EARLY = 8;
+    // the first EARLY of the thread's splits are requested together with the splits' maxima and sums
     float pv[EARLY];
 #pragma unroll
     for (int i = 0; i < EARLY; i++) {
-        const int s = grp + COMBINE_GROUPS * i;
+        const int s = grp + GROUPS * i;
         pv[i] = s < splits ? pp[(size_t)s * (hd + 2) + d] : 0.f;
     }
-    float mv[4], lv[4];
+    float mv[NM], lv[NM];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < NM; i++) {
         const int s = lane + 64 * i;
         mv[i] = -3.0e38f; lv[i] = 0.f;
         if (s < splits) { mv[i] = pp[(size_t)s * (hd + 2) + hd]; lv[i] = pp[(size_t)s * (hd + 2) + hd + 1]; }
     }
-    float M = fmaxf(fmaxf(mv[0], mv[1]), fmaxf(mv[2], mv[3]));
+    float M = mv[0];
+#pragma unroll
+    for (int i = 1; i < NM; i++) M = fmaxf(M, mv[i]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
     float L = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < NM; i++) {
         const int s = lane + 64 * i;
         const float f = s < splits ? __expf(mv[i] - M) : 0.f;
         L = fmaf(lv[i], f, L);
@@ -888,23 +892,32 @@ __global__ __launch_bounds__(128 * COMBINE_GROUPS) void attn_combine_kernel(cons
     __syncthreads();
     float A = 0.f;
 #pragma unroll
-    for (int i = 0; i < EARLY; i++) A = fmaf(pv[i], w[grp + COMBINE_GROUPS * i], A);   // (0 past the last split)
-    for (int s0 = grp + COMBINE_GROUPS * EARLY; s0 < splits; s0 += COMBINE_GROUPS * EARLY) {
-        float v[EARLY];
+    for (int i = 0; i < EARLY; i++) A = fmaf(pv[i], w[grp + GROUPS * i], A);   // (0 past the last split)
+    if constexpr (GROUPS * EARLY < SPLITS)
+        for (int s0 = grp + GROUPS * EARLY; s0 < splits; s0 += GROUPS * EARLY) {
+            float v[EARLY];
 #pragma unroll
-        for (int i = 0; i < EARLY; i++) {
-            const int s = s0 + COMBINE_GROUPS * i;
-            v[i] = s < splits ? pp[(size_t)s * (hd + 2) + d] : 0.f;
+            for (int i = 0; i < EARLY; i++) {
+                const int s = s0 + GROUPS * i;
+                v[i] = s < splits ? pp[(size_t)s * (hd + 2) + d] : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < EARLY; i++) A = fmaf(v[i], w[s0 + GROUPS * i], A);
         }
+    if constexpr (GROUPS > 1) {
+        red[grp][d] = A;
+        __syncthreads();
+        if (grp != 0) return;
 #pragma unroll
-        for (int i = 0; i < EARLY; i++) A = fmaf(v[i], w[s0 + COMBINE_GROUPS * i], A);
+        for (int i = 1; i < GROUPS; i++) A += red[i][d];
     }
-    red[grp][d] = A;
-    __syncthreads();
-    if (grp != 0) return;
-#pragma unroll
-    for (int i = 1; i < COMBINE_GROUPS; i++) A += red[i][d];
     out[(size_t)head * hd + d] = A / L;
+}
+void launch_attn_combine(const float* part, int n_head, int hd, int splits, float* out, hipStream_t s) {
+    const dim3 grid((unsigned)n_head);
+    if (splits <= 16) hipLaunchKernelGGL((attn_combine_kernel<1, 16, 16>), grid, dim3((unsigned)hd), 0, s, part, hd, splits, out);
+    else if (splits <= 64) hipLaunchKernelGGL((attn_combine_kernel<4, 8, 64>), grid, dim3((unsigned)(4 * hd)), 0, s, part, hd, splits, out);
+    else hipLaunchKernelGGL((attn_combine_kernel<8, 8, 256>), grid, dim3((unsigned)(8 * hd)), 0, s, part, hd, splits, out);
 }
 
 // ---------------------------------------------------------------- the same over a long block-quantized cache, on the matrix cores
@@ -1597,7 +1610,7 @@ int launch_decode_attention(const float* q, const float* K, const float* V, int 
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "decode_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
+        launch_attn_combine(ws, n_head, hd, splits, out, s);
         rc = check_hip(hipGetLastError(), "decode_attention combine launch");
     }
     return rc;
@@ -1636,7 +1649,7 @@ static int launch_attention_over_kvq(const char* who, int fmt, const float* q, c
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "decode_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
+        launch_attn_combine(ws, n_head, hd, splits, out, s);
         rc = check_hip(hipGetLastError(), "decode_attention combine launch");
     }
     return rc;
@@ -1714,7 +1727,7 @@ int launch_qkv_post_attention(const float* qkv, const float* bias, const float* 
     if (rc) return rc;
     if ((rc = check_hip(hipGetLastError(), "qkv_post_attention launch"))) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)n_head), dim3((unsigned)(hd * COMBINE_GROUPS)), 0, s, ws, hd, splits, out);
+        launch_attn_combine(ws, n_head, hd, splits, out, s);
         rc = check_hip(hipGetLastError(), "qkv_post_attention combine launch");
     }
     return rc;
