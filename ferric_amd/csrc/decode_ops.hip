@@ -1523,29 +1523,28 @@ int launch_kv_append(const float* k, const float* v, size_t t, size_t width, con
 // combine launch. The rows of a KV head are read by each of its query heads' workgroups (a few hundred KB out of the L2), which costs less
 // than the second launch and the trip of the partial results through memory. A step of a workgroup's streams is a trip to memory (0.9 us on rows no
 // cache holds), so from ATT_WIDE_FROM rows on it has sixteen waves, 128 keys a step, in place of four; fewer rows leave most of those without a key (48 rows
-// 4.6 -> 5.6 us). Four waves -> sixteen, f32 cache, us: 130 / 200 / 256 rows 6.2 / 6.9 / 7.1 -> 5.8 / 6.2 / 6.5. us a token through four layers (d 2048, 16 and 8 heads of 128), one
-// workgroup a head | per (head, split) and combined: f32 300 rows 153.6 | 159.4, 400 158.0 | 159.4, 490 162.1 | 160.4; Q8_0 300 154.4 | 159.7,
-// 490 160.9 | 159.6; d 5120, 40 heads, f32 300 320.3 | 323.6, 400 326.7 | 322.4, Q8_0 300 313.5 | 326.9, 490 318.3 | 324.2.
-// A head per KV head shares its rows with no other, and beyond ATT_SHORT_ROWS rows times heads of 128 dims on an f32 cache its workgroup waits for memory
-// where splits of 64 keys bring more workgroups; so there it ends at ATT_SHORT_OWN rows. us a launch on rows no cache holds, one workgroup a head | splits:
-// f32, 16 heads 304 / 352 rows 7.7 | 8.1, 8.6 | 8.5; 24 heads 320 / 352 rows 8.2 | 8.6, 11.6 | 9.4; 32 heads 256 / 288 / 352 rows 8.3 | 9.3, 9.9 | 9.2, 11.6 | 9.9;
-// 40 heads 256 / 352 rows 10.8 | 9.8, 13.1 | 10.4; 4 heads 352 rows 8.1 | 7.9; heads of 64, 64 of them, 352 rows 8.3 | 9.1. A quantized cache takes the f32 one's
-// way, whose bits it promises, though it reads a quarter: Q8_0, 32 heads 288 rows 7.9 | 8.9, 224 rows 7.3 | 8.8. Grouped heads in one workgroup each | per (head, split)
-// at 352 rows: f32 2 heads 8.0 | 8.2, 16 of 4 8.6 | 9.0, 40 of 8 8.9 | 9.3, 64 of 8 9.2 | 9.4, 32 of 8 of 64 dims 6.2 | 8.0; Q8_0 2 heads 7.6 | 8.7.
-constexpr size_t ATT_SHORT = 352, ATT_SHORT_OWN = 256, ATT_SHORT_ROWS = 8192, ATT_WIDE_FROM = 97;
+// 4.6 -> 5.6 us). Four waves -> sixteen, f32 cache, us: 130 / 200 / 256 rows 6.2 / 6.9 / 7.1 -> 5.8 / 6.2 / 6.5.
+// Where it ends: heads of 128 dims on an f32 cache wait for memory in their one workgroup, where splits bring more of them: there it ends at ATT_SHORT_128 rows,
+// and at ATT_SHORT_OWN for a head per KV head, whose rows no other workgroup reads. us with the post-processing, one workgroup a head | splits and combined, rows that
+// no cache holds (over 700 MB) and, in brackets, that the Infinity Cache does: f32, 40 heads of 8 at 208 / 256 / 288 / 352 rows 8.8 | 9.5, 9.5 | 9.7, 10.2 | 9.1, 11.3 | 9.8 (256 / 288 / 352
+// 7.8 | 8.3, 8.3 | 8.0, 9.2 | 8.5), 16 of 4 at 256 / 288 / 352 9.0 | 9.2, 9.9 | 9.0, 11.0 | 9.7, 2 of 1 at 288 / 352 7.3 | 6.9, 7.9 | 7.4; a KV head each, 8 heads at 128 / 192 / 256 / 352
+// 7.7 | 8.1, 8.4 | 7.8, 9.8 | 8.1, 11.9 | 8.2 (192 / 256 / 352 6.8 | 6.9, 7.2 | 7.1, 8.4 | 7.3), 32 heads 7.9 | 8.3, 8.9 | 8.4, 9.9 | 8.7, 12.1 | 9.0. Heads of 64: 32 of 8 at 352 / 448
+// 7.5 | 8.8, 8.4 | 8.8, a KV head each, 32 heads at 256 / 352 6.9 | 7.4, 8.0 | 7.5 (6.5 | 7.3). A quantized cache takes the f32 one's way, whose bits it promises, though it reads a
+// quarter: Q8_0, 40 heads of 8 at 256 / 288 / 352 rows 7.6 | 8.8, 7.8 | 8.5, 8.8 | 9.6; a KV head each, 8 heads at 192 / 256 / 352 6.8 | 7.6, 7.4 | 7.7, 8.5 | 8.1.
+constexpr size_t ATT_SHORT = 352, ATT_SHORT_128 = 256, ATT_SHORT_OWN = 192, ATT_WIDE_FROM = 97;
 bool attn_per_query_head(size_t len, int n_head, int n_kv, int hd, bool ws = true) {   // ws: splits have a workspace to go to
-    return len <= (ws && n_head == n_kv && hd == 128 && len * (size_t)n_kv > ATT_SHORT_ROWS ? ATT_SHORT_OWN : ATT_SHORT);
+    return len <= (!ws || hd != 128 ? ATT_SHORT : n_head == n_kv ? ATT_SHORT_OWN : ATT_SHORT_128);
 }
 bool attn_wide(size_t len) { return len >= ATT_WIDE_FROM; }
 
-// Between ATT_SHORT and ATT_MID rows under grouped query heads: one workgroup per (query head, split of at least ATT_MID_KEYS
+// Beyond that, up to ATT_MID rows under grouped query heads: one workgroup per (query head, split of at least ATT_MID_KEYS
 // keys). The kernel that takes all query heads of a KV head at once holds 180 registers a lane (two waves per SIMD) and its
 // waves spend their time in the dependent arithmetic of five softmax chains; with one head a workgroup (107 registers, four
 // waves per SIMD) the same arithmetic is spread over five times the waves, and the rows they share come out of one XCD's L2
 // (see the kernel's workgroup numbering). Chained 64-layer step, ms per token, this shape | all heads of a KV head per
 // workgroup: 500 keys 3.99 | 4.24, 1000: 4.06 | 4.28, 2048: 4.22 | 4.56, 4096: 4.63 | 4.77, 6000: 4.97 | 4.90, 8000: 5.41 | 5.08.
 constexpr size_t ATT_MID = 5120, ATT_MID_KEYS = 128;
-bool attn_per_head_splits(size_t len, int n_head, int n_kv) { return n_kv > 0 && n_head > n_kv && len > ATT_SHORT && len <= ATT_MID; }
+bool attn_per_head_splits(size_t len, int n_head, int n_kv) { return n_kv > 0 && n_head > n_kv && len <= ATT_MID; }   // (asked behind attn_per_query_head)
 // splits of at least ATT_MID_KEYS keys, at most about two and a half workgroups per CU over all query heads
 int attn_mid_splits(size_t len, int n_head) {
     const int by_keys = (int)((len + ATT_MID_KEYS - 1) / ATT_MID_KEYS), cap = 5 * device_cus() / 2 / (n_head > 0 ? n_head : 1);
@@ -1553,7 +1552,7 @@ int attn_mid_splits(size_t len, int n_head) {
     return s < 1 ? 1 : (s > 256 ? 256 : s);
 }
 
-// Splits of the key range beyond ATT_SHORT: about two workgroups per CU over all KV heads, at least 64 keys each (two rounds of the
+// Splits of the key range otherwise: about two workgroups per CU over all KV heads, at least 64 keys each (two rounds of the
 // workgroup's 16 streams x 2 keys), at most 256 (the combine kernel's LDS tables).
 int attn_splits(size_t len, int n_kv) {
     if (n_kv <= 0) return 1;

@@ -213,28 +213,29 @@ def test_attention_over_the_blocks_is_attention_over_the_dequantized_rows(F, Q, 
     assert b"head_dim must be 64 or 128" in lib.fhip_last_error()
 
 
-@pytest.mark.parametrize("nh,hd,rows", [(32, 128, 256), (32, 128, 257), (32, 128, 352), (32, 128, 353), (24, 128, 341), (24, 128, 342), (23, 128, 352), (40, 64, 352)])
-def test_a_head_per_kv_head_about_the_end_of_the_short_caches(F, Q, K, nh, hd, rows):
-    """One workgroup a head, or splits from rows x heads = 8192 on, f32 and Q8_0 caches at the 1e-5 of the attention tests, the same bits from both; a launch
-    without a workspace is taken up to 352 rows, as the one workgroup needs none."""
+@pytest.mark.parametrize("nh,nkv,hd,rows", [(32, 32, 128, 192), (32, 32, 128, 193), (8, 8, 128, 352), (32, 32, 128, 353), (2, 2, 128, 256), (40, 40, 64, 352), (40, 40, 64, 353),
+                                           (40, 8, 128, 256), (40, 8, 128, 257), (16, 2, 128, 352), (16, 2, 128, 353), (2, 1, 128, 300), (24, 8, 64, 352), (24, 8, 64, 353)])
+def test_about_the_end_of_the_short_caches(F, Q, K, nh, nkv, hd, rows):
+    """One workgroup a head, or splits: heads of 128 dims from 257 rows on, from 193 with a KV head each; f32 and Q8_0 caches at the 1e-5 of the attention tests,
+    the same bits from both; a launch without a workspace is taken up to 352 rows, as the one workgroup needs none."""
     from types import SimpleNamespace
     from ferric_amd import decode as X
     from oracle import decode_oracle as D
-    lib, rng, width = F._lib.load(), np.random.default_rng(rows + nh), nh * hd
+    lib, rng, width = F._lib.load(), np.random.default_rng(rows + nh), nkv * hd
     k, v = (rng.standard_normal((rows, width)).astype(np.float32) for _ in range(2))
-    q = rng.standard_normal((1, width)).astype(np.float32)
+    q = rng.standard_normal((1, nh * hd)).astype(np.float32)
     kq, vq = (Q.QKvCache.from_tensor(F.Tensor.from_vec(a, a.shape), Q.Q8_0) for a in (k, v))
     qt = F.Tensor.from_vec(q, q.shape)
     plain = SimpleNamespace(k=kq.dequantize(), v=vq.dequantize(), cap=rows, width=width, len=rows)
-    want = D.decode_attention(q[0], K.roundtrip(k, rows, width, Q.Q8_0), K.roundtrip(v, rows, width, Q.Q8_0), nh, nh).reshape(-1)
-    a, b = X.decode_attention_kvq(qt, kq, vq, nh, nh).to_vec(), X.decode_attention(qt, plain, nh, nh).to_vec()
+    want = D.decode_attention(q[0], K.roundtrip(k, rows, width, Q.Q8_0), K.roundtrip(v, rows, width, Q.Q8_0), nh, nkv)[0]
+    a, b = X.decode_attention_kvq(qt, kq, vq, nh, nkv).to_vec(), X.decode_attention(qt, plain, nh, nkv).to_vec()
     assert np.array_equal(bits(a), bits(b)) and np.abs(b - want).max() <= 1e-5 * np.abs(want).max()
-    out = F.Tensor.empty((1, width))
-    rc = lib.fhip_decode_attention_ex(qt.buf.ptr, plain.k.buf.ptr, plain.v.buf.ptr, nh, nh, hd, rows, None, 0, 0.0, None, out.buf.ptr, None)
+    out = F.Tensor.empty((1, nh * hd))
+    rc = lib.fhip_decode_attention_ex(qt.buf.ptr, plain.k.buf.ptr, plain.v.buf.ptr, nh, nkv, hd, rows, None, 0, 0.0, None, out.buf.ptr, None)
     assert (rc == 0) == (rows <= 352)
     if rc == 0:
         assert np.abs(out.to_vec() - want).max() <= 1e-5 * np.abs(want).max()
-    assert (lib.fhip_decode_attention_ws_bytes(nh, nh, hd, rows) > 0) == (rows > 352 or (hd == 128 and rows > 256 and rows * nh > 8192))
+    assert (lib.fhip_decode_attention_ws_bytes(nh, nkv, hd, rows) > 0) == (rows > (352 if hd == 64 else 192 if nh == nkv else 256))
 
 
 @pytest.mark.parametrize("fmt", [0, 1])
