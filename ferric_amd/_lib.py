@@ -58,6 +58,7 @@ SYMBOLS = {
     "fhip_swiglu": (C.c_int, [_vp, _sz, _sz, _vp, _vp]),
     "fhip_ffn": (C.c_int, [_vp, _vp, _vp, _sz, _vp, _vp, _vp]),
     "fhip_gemm_q_bf16": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
+    "fhip_gemm_q_bf16_run_sums": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
     "fhip_moe_topk": (C.c_int, [_vp, _vp, _sz, _sz, _sz, C.c_int, C.c_float, C.c_int, _vp, _vp]),
     "fhip_matmul_q_swiglu_id": (C.c_int, [_vp, _vp, _sz, _vp, _sz, _sz, _vp, _vp]),
     "fhip_matmul_q_relu2_id": (C.c_int, [_vp, _vp, _sz, _vp, _sz, _sz, _vp, _vp]),
@@ -94,6 +95,7 @@ SYMBOLS = {
     "fhip_add_rmsnorm_bf16": (C.c_int, [_vp, _vp, _vp, _sz, _sz, C.c_float, _vp, _vp, _vp]),
     "fhip_causal_attention_bf16": (C.c_int, [_vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, _sz, C.c_float, _vp, _vp]),
     "fhip_ffn_bf16": (C.c_int, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp]),
+    "fhip_ffn_bf16_run_sums": (C.c_int, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp]),
     "fhip_add": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
     "fhip_mul_sigmoid": (C.c_int, [_vp, _vp, _sz, _vp, _vp]),
     "fhip_kvq_sizes": (C.c_int, [C.c_int, _sz, _sz, C.POINTER(_sz), C.POINTER(_sz)]),

@@ -35,7 +35,10 @@ UNITS = {
     "gemv_wide.hip": ["-DFHIP_GEMV_PLANES=2"],
     "gemv_wide.hip@p3": ["-DFHIP_GEMV_PLANES=3"],
     "gemv_generic.hip": [],
-    "gemm_mfma.hip": [],
+    "gemm_mfma.hip": ["-DFHIP_GEMM_FORMAT=Q4K", "-Wno-unused-const-variable", "-DFHIP_GEMM_ENTRY"],   # one copy per weight format
+    "gemm_mfma.hip@q5k": ["-DFHIP_GEMM_FORMAT=Q5K", "-Wno-unused-const-variable"],
+    "gemm_mfma.hip@q6k": ["-DFHIP_GEMM_FORMAT=Q6K", "-Wno-unused-const-variable"],
+    "gemm_mfma.hip@q80": ["-DFHIP_GEMM_FORMAT=Q80", "-Wno-unused-const-variable"],
     "gemm_f16x2.hip": [],
     "moe.hip": [],
     "probe.hip": [],

@@ -223,14 +223,14 @@ void release_workspace(hipStream_t s) {
 
 // The matrix-core GEMM with its K-split scratch (partial tiles of the tiles that several workgroups share) taken from the
 // stream's library workspace.
-static int gemm_bf16_lib_ws(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, const char* who) {
-    const size_t need = fhip::gemm_bf16_ws_bytes(w, t);
+static int gemm_bf16_lib_ws(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, const char* who, bool run_sums = false) {
+    const size_t need = fhip::gemm_bf16_ws_bytes(w, t, run_sums);
     void* ws = nullptr;
     if (need) {
         int rc = lib_workspace(s, need, &ws, who);
         if (rc) return rc;
     }
-    return fhip::launch_gemm_bf16(w, d_x, t, d_y, s, (float*)ws, need);
+    return fhip::launch_gemm_bf16(w, d_x, t, d_y, s, (float*)ws, need, run_sums);
 }
 
 // ---- which kernel a batch takes ---------------------------------------------------------------------------------------------
@@ -797,9 +797,18 @@ size_t fhip_workspace_bytes(const fhip_weight* gu, const fhip_weight* down, size
 }
 
 size_t fhip_workspace_bytes_coop(const fhip_weight* w, const fhip_weight* down, size_t rows_x) {
-    const size_t a = fhip::gemm_bf16_ws_bytes(w, rows_x), b = fhip::gemm_bf16_ws_bytes(down, rows_x), c = fhip::gemm_bf16_swiglu_ws_bytes(w, rows_x);
-    const size_t ab = a > b ? a : b;
-    return ab > c ? ab : c;
+    // A smaller batch may need more than a larger one, whose tiles fill the chip whole: the most over the batches up to rows_x. A plan
+    // follows from the number of 64-row tiles (more than 32 rows) or from the staged rows (8 or 32).
+    size_t need = 0;
+    auto most = [&](size_t t) {
+        for (size_t n : {fhip::gemm_bf16_ws_bytes(w, t), fhip::gemm_bf16_ws_bytes(down, t), fhip::gemm_bf16_swiglu_ws_bytes(w, t), fhip::gemm_bf16_ws_bytes(w, t, true),
+                         fhip::gemm_bf16_ws_bytes(down, t, true)}) need = n > need ? n : need;
+    };
+    most(rows_x);
+    if (rows_x > 8) most(8);
+    if (rows_x > 32) most(32);
+    for (size_t t = 64; t < rows_x; t += 64) most(t);
+    return need;
 }
 
 void fhip_workspace_release(void* stream) {
@@ -807,14 +816,20 @@ void fhip_workspace_release(void* stream) {
     fhip::pool_trim();
 }
 
-int fhip_gemm_q_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, void* stream) {
+static int gemm_q_bf16(const char* who, const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, void* stream, bool run_sums) {
     int rc = need_init();
     if (rc) return rc;
-    if (!w) return set_error(FHIP_ERR_ARG, "fhip_gemm_q_bf16: NULL weight");
+    if (!w) return set_error(FHIP_ERR_ARG, "%s: NULL weight", who);
     if (t == 0 || w->rows == 0) return FHIP_OK;
-    if (!d_y || (!d_x && w->cols)) return set_error(FHIP_ERR_ARG, "fhip_gemm_q_bf16: NULL pointer");
+    if (!d_y || (!d_x && w->cols)) return set_error(FHIP_ERR_ARG, "%s: NULL pointer", who);
     if (w->cols == 0) return zero_outputs(t, w->rows, d_y, (hipStream_t)stream);   // empty inner dimension: every dot product is 0
-    return gemm_bf16_lib_ws(w, d_x, t, d_y, (hipStream_t)stream, "fhip_gemm_q_bf16");
+    return gemm_bf16_lib_ws(w, d_x, t, d_y, (hipStream_t)stream, who, run_sums);
+}
+int fhip_gemm_q_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, void* stream) {
+    return gemm_q_bf16("fhip_gemm_q_bf16", w, d_x, t, d_y, stream, false);
+}
+int fhip_gemm_q_bf16_run_sums(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, void* stream) {
+    return gemm_q_bf16("fhip_gemm_q_bf16_run_sums", w, d_x, t, d_y, stream, true);
 }
 
 // ---- mixture-of-experts entry points (crates/ferric-tensor/src/dtype.rs:1582-1780) ----------------------
@@ -1318,7 +1333,7 @@ size_t fhip_ffn_coop_ws_bytes(const fhip_weight* gu, const fhip_weight* down, si
 
 // d_x f32 (converted into the workspace first), or already bf16 in d_xb; d_gu: null, or where gate|up goes in f32 between two launches
 static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* down, const float* d_x, const uint16_t* d_xb, float* d_gu, size_t rows_x,
-                    float* d_y, void* d_ws, hipStream_t s) {
+                    float* d_y, void* d_ws, hipStream_t s, bool run_sums = false) {
     int rc = need_init();
     if (rc) return rc;
     if (!gu || !down) return set_error(FHIP_ERR_ARG, "%s: NULL weight", who);
@@ -1347,9 +1362,9 @@ static int ffn_coop(const char* who, const fhip_weight* gu, const fhip_weight* d
         if ((rc = fhip::launch_gemm_bf16_swiglu(gu, d_xb, rows_x, hb, s, (float*)split, need))) return rc;
         return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, who);
     }
-    if ((rc = gemm_bf16_lib_ws(gu, d_xb, rows_x, g, s, who))) return rc;
+    if ((rc = gemm_bf16_lib_ws(gu, d_xb, rows_x, g, s, who, run_sums))) return rc;
     if ((rc = fhip::launch_swiglu_bf16(g, rows_x, n_ff, hb, s))) return rc;
-    return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, who);
+    return gemm_bf16_lib_ws(down, hb, rows_x, d_y, s, who, run_sums);
 }
 
 int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d_x, size_t rows_x, float* d_y,
@@ -1360,6 +1375,11 @@ int fhip_ffn_coop(const fhip_weight* gu, const fhip_weight* down, const float* d
 int fhip_ffn_bf16(const fhip_weight* gu, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
                   void* stream) {
     return ffn_coop("fhip_ffn_bf16", gu, down, nullptr, d_x_bf16, d_gate_up, rows_x, d_y, d_ws, (hipStream_t)stream);
+}
+int fhip_ffn_bf16_run_sums(const fhip_weight* gu, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
+                           void* stream) {
+    if (!d_gate_up && need_init() == FHIP_OK && rows_x) return set_error(FHIP_ERR_ARG, "fhip_ffn_bf16_run_sums: NULL pointer");
+    return ffn_coop("fhip_ffn_bf16_run_sums", gu, down, nullptr, d_x_bf16, d_gate_up, rows_x, d_y, d_ws, (hipStream_t)stream, true);
 }
 
 size_t fhip_matmul_q_f16x2_ws_bytes(const fhip_weight* w, size_t rows_x) {

@@ -10,10 +10,11 @@
 // operations to turn into bf16, an MFMA retires 16K multiply-adds in 32 cycles. So
 //   * each lane dequantizes 8 consecutive quants of one weight row, which is exactly the B fragment a lane
 //     holds in a 32x32x16 MFMA: no transposition for the weights;
-//   * a dequantized fragment is published once in LDS and used by both waves of a T-pair for every 32-row
-//     slab they own, so unpack cost is amortised over the workgroup's 64*MI activation rows;
-//   * the fragments of step s+1 are produced while the MFMAs of step s run, one MFMA alternating with its
-//     share of the unpack arithmetic, with two waves per SIMD to fill each other's issue gaps;
+//   * a dequantized fragment is published once in LDS and used by every wave that multiplies those outputs, so unpack cost is amortised
+//     over the workgroup's 256 activation rows -- or, on the tiles for shorter prompts, one wave unpacks for its own 64 or 128 rows and
+//     LDS carries the activations alone;
+//   * the next fragments are produced while the current MFMAs run, one MFMA alternating with its share of the unpack arithmetic, with
+//     two waves per SIMD to fill each other's issue gaps;
 //   * the activation tile, which all 8 waves of a workgroup share, is staged through LDS (padded rows,
 //     16-byte reads);
 //   * the 16 k of one MFMA are chosen inside ONE scale sub-block (the k order inside an MFMA is free as
@@ -23,20 +24,35 @@
 // One k-step is 64 columns = 4 MFMA slices; a chunk is 4 steps = one K-quant super-block or 8 Q8_0 blocks.
 // Dequantized values are exactly the f32 the CPU dequantizer produces, rounded to bf16 (RNE) by
 // v_cvt_pk_bf16_f32.
-// Three kernels: the tiled one (64, 128 or 256 activation rows x 256 or 128 outputs per workgroup), its 160-column variant
-// (256 or 128 rows) for output widths that 160 deals to the chip's workgroups exactly, and one for up to 32 rows; the
-// launcher picks by a cost estimate. A launch that cuts output tiles along K sums the partial tiles in a fixed order: the same inputs give the
+// Four kernels: the tiled one (256 activation rows x 256 outputs per workgroup), its 160-column variant (256 or 128 rows) for output
+// widths that 160 deals to the chip's workgroups exactly, one of 64 or 128 rows x 64 ... 256 outputs whose waves unpack for themselves
+// (short prompts, small weights), and one for up to 32 rows; the launcher picks by a cost estimate. A launch that cuts output tiles along K sums the partial tiles in a fixed order: the same inputs give the
 // same bits on every run.
 #include "prompt.hpp"
 #include "loads.hpp"
 
 #include <hip/hip_fp16.h>
 
-#include <cstdlib>
+#include <numeric>
 #include <type_traits>
+
+// This file is compiled once per weight format (FHIP_GEMM_FORMAT: its struct below); the copy for Q4_K holds the entry points.
+#define FHIP_GEMM_PASTE2(a, b) a##b
+#define FHIP_GEMM_PASTE(a, b) FHIP_GEMM_PASTE2(a, b)
+#define FHIP_GEMM_NAME(what) FHIP_GEMM_PASTE(FHIP_GEMM_PASTE(gemm_, FHIP_GEMM_FORMAT), what)
+namespace fhip {
+constexpr int GEMM_TILES = 12;
+extern int g_gemm_tile;   // tests: 0 ... 11 pins a tile (BM_OF x BN_OF below), anything else: the estimate decides
+#define FHIP_GEMM_DECLARE(F) \
+    size_t gemm_##F##_ws_bytes(const fhip_weight* w, size_t columns, size_t t, bool run_sums); \
+    int gemm_##F##_launch(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums); \
+    int gemm_##F##_launch_swiglu(const fhip_weight* w, const uint16_t* d_x, size_t t, uint16_t* d_h, hipStream_t s, float* d_ws, size_t ws_bytes);
+FHIP_GEMM_DECLARE(Q4K) FHIP_GEMM_DECLARE(Q5K) FHIP_GEMM_DECLARE(Q6K) FHIP_GEMM_DECLARE(Q80)
+}  // namespace fhip
 
 namespace {
 
+constexpr int NTILES = fhip::GEMM_TILES;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -44,19 +60,27 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float f16_bits(uint32_t b) { return __half2float(__ushort_as_half((unsigned short)b)); }
 __device__ __forceinline__ float ub(uint32_t v, int k) { return (float)((v >> (8 * k)) & 0xFFu); }
 using fhip::pk_bf16;
-// 8 weights w_i = fma(s, q_i, o) from the bytes of two dwords -> one MFMA operand (8 bf16)
-__device__ __forceinline__ bf16x8 frag8(uint32_t q0, uint32_t q1, float s, float o) {
-    // Hide from the optimiser which bits of the bytes are known zero: with that knowledge it narrows every
-    // byte extraction to a bit-field extract and adds one instruction per weight in front of the byte-lane
-    // conversions v_cvt_f32_ubyte0..3, which take the byte lane as it is.
-    asm("" : "+v"(q0));
-    asm("" : "+v"(q1));
+// 8 weights w_i = fma(s, q_i, o) from the bytes of two dwords -> one MFMA operand (8 bf16). A byte in the low half of a 16-bit field is the
+// f16 denormal q * 2^-24, which v_fma_mix_f32 takes as it stands (exact, with 2^24 in the scale: `s` is 2^24 times the weight's scale): two
+// masks or byte shuffles a dword in place of four byte conversions.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+constexpr float Q_ULP = 16777216.f;   // 1 / the f16 denormal of the integer 1
+__device__ __forceinline__ bf16x8 frag8(uint32_t e0, uint32_t o0, uint32_t e1, uint32_t o1, float s, float o) {   // even and odd bytes of each dword
+    const f16x2 a = __builtin_bit_cast(f16x2, e0), b = __builtin_bit_cast(f16x2, o0), c = __builtin_bit_cast(f16x2, e1), d = __builtin_bit_cast(f16x2, o1);
     u32x4 r;
-    r[0] = pk_bf16(fmaf(s, ub(q0, 0), o), fmaf(s, ub(q0, 1), o));
-    r[1] = pk_bf16(fmaf(s, ub(q0, 2), o), fmaf(s, ub(q0, 3), o));
-    r[2] = pk_bf16(fmaf(s, ub(q1, 0), o), fmaf(s, ub(q1, 1), o));
-    r[3] = pk_bf16(fmaf(s, ub(q1, 2), o), fmaf(s, ub(q1, 3), o));
+    r[0] = pk_bf16(fmaf((float)a[0], s, o), fmaf((float)b[0], s, o));
+    r[1] = pk_bf16(fmaf((float)a[1], s, o), fmaf((float)b[1], s, o));
+    r[2] = pk_bf16(fmaf((float)c[0], s, o), fmaf((float)d[0], s, o));
+    r[3] = pk_bf16(fmaf((float)c[1], s, o), fmaf((float)d[1], s, o));
     return __builtin_bit_cast(bf16x8, r);
+}
+__device__ __forceinline__ bf16x8 frag8(uint32_t q0, uint32_t q1, float s, float o) {
+    constexpr uint32_t ODD = 0x0C030C01u;   // bytes 1 and 3, each above a zero byte
+    return frag8(q0 & 0x00FF00FFu, __builtin_amdgcn_perm(q0, q0, ODD), q1 & 0x00FF00FFu, __builtin_amdgcn_perm(q1, q1, ODD), s, o);
+}
+// the same from the nibbles of two dwords that `mask` (0x000F000F or 0x00F000F0) leaves
+__device__ __forceinline__ bf16x8 frag8_nibbles(uint32_t q0, uint32_t q1, uint32_t mask, float s, float o) {
+    return frag8(q0 & mask, (q0 >> 8) & mask, q1 & mask, (q1 >> 8) & mask, s, o);
 }
 
 constexpr int KSTEP = 64;            // columns per k-step: 4 MFMA slices of 16
@@ -66,6 +90,7 @@ constexpr int LDS_ROW = KSTEP + 8;   // bf16 per staged activation row (+16 B pa
 // Column of the 8 consecutive k that lane half h (= lane / 32) holds in slice t of a step, for both
 // operands and every format: sub-block (t >> 1) of the step, elements 16h + 8(t & 1) + [0, 8).
 __device__ __forceinline__ constexpr int kcol(int t, int h) { return 32 * (t >> 1) + 16 * h + 8 * (t & 1); }
+
 
 // ------------------------------------------------------------------------------------------------
 // Per-format weight streams. `Raw` is the per-lane register image of one chunk of one weight row (the
@@ -79,8 +104,9 @@ struct Q4K {
     using Eager = Q4K;
     static constexpr int BLOCK = 144;
     static constexpr float UNPACK_US = 1.4f;   // unpack of a 256 x 256 chunk by one workgroup
-    // one chunk of a workgroup tile of 64 x 256, 128 x 256, 256 x 256, 256 x 160, 128 x 128, 64 x 128, 128 x 160, in us (fitted, see plan_cost_us)
-    static constexpr float CHUNK_US[7] = {3.43f, 4.76f, 8.15f, 5.19f, 2.84f, 2.00f, 3.29f};
+    // one chunk of a workgroup tile, in us, in the order of BM_OF x BN_OF (fitted, see plan_cost_us)
+    static constexpr float CHUNK_US[NTILES] = {2.39f, 3.62f, 7.17f, 4.81f, 2.02f, 1.29f, 3.00f, 1.75f, 1.16f, 1.62f, 0.78f, 1.22f};
+    static constexpr float RUN_CHUNK_US[7] = {3.43f, 4.76f, 8.15f, 5.19f, 2.84f, 2.00f, 3.29f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
     struct Raw { u32x4 hd, hdn, q[4]; };
@@ -107,7 +133,7 @@ struct Q4K {
     template <int G>
     static __device__ __forceinline__ void begin(Raw& r, const uint8_t*, int, int, int, Ctx& x) {
         if (G == 0) r.hd = r.hdn;
-        const float d = f16_bits(r.hd[0] & 0xFFFFu), dmin = f16_bits(r.hd[0] >> 16);
+        const float d = f16_bits(r.hd[0] & 0xFFFFu) * Q_ULP, dmin = f16_bits(r.hd[0] >> 16);
         float s0, m0, s1, m1;
         sc_min(r.hd, 2 * G, s0, m0);
         sc_min(r.hd, 2 * G + 1, s1, m1);
@@ -118,8 +144,7 @@ struct Q4K {
     // slice T: sub-block 2G + (T >> 1) = low (T < 2) or high nibbles of bytes 32G + 16h + 8(T & 1) + [0, 8)
     template <int G, int T>
     static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
-        constexpr uint32_t M = T < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
-        return frag8(r.q[G][2 * (T & 1)] & M, r.q[G][2 * (T & 1) + 1] & M, T < 2 ? x.d0 : x.d1, T < 2 ? x.o0 : x.o1);
+        return frag8_nibbles(r.q[G][2 * (T & 1)], r.q[G][2 * (T & 1) + 1], T < 2 ? 0x000F000Fu : 0x00F000F0u, T < 2 ? x.d0 : x.d1, T < 2 ? x.o0 : x.o1);
     }
     template <int G>
     static __device__ __forceinline__ void refill(Raw& r, const uint8_t* row, int nc, int h, int) {
@@ -139,7 +164,8 @@ struct Q5K {
     using Eager = Q5K;
     static constexpr int BLOCK = 176;
     static constexpr float UNPACK_US = 1.8f;
-    static constexpr float CHUNK_US[7] = {3.83f, 5.16f, 9.41f, 6.12f, 3.17f, 2.26f, 3.78f};
+    static constexpr float CHUNK_US[NTILES] = {2.86f, 4.08f, 7.68f, 5.20f, 2.28f, 1.51f, 3.37f, 1.95f, 1.34f, 1.90f, 0.92f, 1.36f};
+    static constexpr float RUN_CHUNK_US[7] = {3.83f, 5.16f, 9.41f, 6.12f, 3.17f, 2.26f, 3.78f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
     struct Raw { u32x4 hd, hdn, qh, qhn, q[4]; };
@@ -156,7 +182,7 @@ struct Q5K {
     template <int G>
     static __device__ __forceinline__ void begin(Raw& r, const uint8_t*, int, int, int, Ctx& x) {
         if (G == 0) { r.hd = r.hdn; r.qh = r.qhn; }
-        const float d = f16_bits(r.hd[0] & 0xFFFFu), dmin = f16_bits(r.hd[0] >> 16);
+        const float d = f16_bits(r.hd[0] & 0xFFFFu) * Q_ULP, dmin = f16_bits(r.hd[0] >> 16);
         float s0, m0, s1, m1;
         Q4K::sc_min(r.hd, 2 * G, s0, m0);
         Q4K::sc_min(r.hd, 2 * G + 1, s1, m1);
@@ -190,7 +216,8 @@ struct Q6K {
     // whose scale is sc[8hf + 2g + h]  (crates/ferric-gguf/src/lib.rs:833-851).
     static constexpr int BLOCK = 210;
     static constexpr float UNPACK_US = 2.3f;
-    static constexpr float CHUNK_US[7] = {5.93f, 6.83f, 9.84f, 6.27f, 4.68f, 3.95f, 4.35f};
+    static constexpr float CHUNK_US[NTILES] = {4.70f, 5.89f, 8.29f, 5.71f, 2.78f, 2.21f, 4.16f, 2.27f, 1.73f, 2.72f, 1.73f, 2.04f};
+    static constexpr float RUN_CHUNK_US[7] = {5.93f, 6.83f, 9.84f, 6.27f, 4.68f, 3.95f, 4.35f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
     struct Raw { u32x4 ql[2][2], qh[2], sc, scn; uint32_t d, dn; };
@@ -232,7 +259,7 @@ struct Q6K {
         const uint32_t scw = r.sc[2 * hf + (g >> 1)];
         const float ds = x.d * (float)(int8_t)((scw >> (16 * (g & 1))) & 0xFFu);
         // (d*sc)*(q-32) = ds*q - 32*ds, every term exact in f32
-        return frag8(n0 | u0, n1 | u1, ds, -32.0f * ds);
+        return frag8(n0 | u0, n1 | u1, ds * Q_ULP, -32.0f * ds);
     }
     template <int G>
     static __device__ __forceinline__ void refill(Raw& r, const uint8_t* row, int nc, int h, int) {
@@ -266,7 +293,8 @@ struct Q80T {
     // read from the last valid block's address and given scale 0 (their activations are staged as 0 too).
     static constexpr int BLOCK = 34;
     static constexpr float UNPACK_US = 5.1f;
-    static constexpr float CHUNK_US[7] = {9.40f, 9.88f, 11.93f, 6.86f, 7.00f, 6.50f, 5.05f};
+    static constexpr float CHUNK_US[NTILES] = {6.25f, 7.76f, 10.02f, 5.99f, 3.94f, 3.29f, 4.15f, 4.13f, 3.11f, 3.91f, 1.70f, 2.08f};
+    static constexpr float RUN_CHUNK_US[7] = {9.40f, 9.88f, 11.93f, 6.86f, 7.00f, 6.50f, 5.05f};
     static constexpr bool PARTIAL = true;   // a row may end inside a chunk
     static __host__ __device__ int chunks(int K) { return (K + 255) / 256; }
     struct Raw { fhip::Un16 q[4][2]; uint32_t d[4][2]; };
@@ -300,7 +328,7 @@ struct Q80T {
     static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
         // q = (q ^ 0x80) - 128 with the biased byte unsigned: d*q = d*u - 128*d, every term exact in f32
         const float d = x.d[T >> 1];
-        return frag8(r.q[G][T >> 1].w[2 * (T & 1)] ^ 0x80808080u, r.q[G][T >> 1].w[2 * (T & 1) + 1] ^ 0x80808080u, d, -128.0f * d);
+        return frag8(r.q[G][T >> 1].w[2 * (T & 1)] ^ 0x80808080u, r.q[G][T >> 1].w[2 * (T & 1) + 1] ^ 0x80808080u, d * Q_ULP, -128.0f * d);
     }
     template <int G>
     static __device__ __forceinline__ void refill(Raw& r, const uint8_t* row, int nc, int h, int nblk) {
@@ -344,10 +372,11 @@ __device__ __forceinline__ int swiglu_row(int v, int ff) {
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 // the 32 x 32 accumulator of rows t0 .. and columns v0 ..: outputs 16 * (v0 / 32) + (c & 15)
+template <int R0 = 0, int NR = 16>
 __device__ __forceinline__ void store_swiglu(const GemmParams& p, const f32x16& acc, int t0, int v0, int h, int c) {
     const int n = 16 * (v0 >> 5) + (c & 15);
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) {
+    for (int r = R0; r < R0 + NR; r += 2) {
         const auto gu = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[r]), __float_as_uint(acc[r + 1]), false, false);
         const int t = t0 + 8 * (r >> 2) + 4 * h + (r & 3) + (c >> 4);
         if (t < p.T && n < p.ff)
@@ -363,7 +392,7 @@ __device__ __forceinline__ void static_for(Fn&& f) {
     }
 }
 
-// Workgroup = 8 waves, 2 along T x 4 along N; wave tile = (32*MI) x 64; workgroup tile = (64*MI) x 256.
+// Workgroup = 8 waves, 2 along T x 4 along N; wave tile = 128 x 64; workgroup tile = 256 x 256.
 // Two waves per SIMD: a wave issues one VALU instruction per ~6 cycles and one 16-byte LDS read per ~16, so
 // a single wave cannot feed its own MFMAs and unpack at the same time; two can.
 // The two waves of a T-pair need the same 64 weight rows. Each unpacks 32 of them (all four slices of a
@@ -379,14 +408,9 @@ __device__ __forceinline__ void static_for(Fn&& f) {
 // the runs that touch the tile, and sum_split_tiles_kernel adds a tile's slots in that order afterwards: the result does not
 // depend on which workgroup finishes first (f32 atomics into Y, which this replaced, gave run-to-run differences in the
 // last bits wherever a tile had three contributors or more).
-//
-// NI = 1 is the same layout at half the width, a workgroup tile of (64*MI) x 128 for short prompts: a T-pair then needs one
-// block of 32 weight rows, both waves carry its raw bytes and each unpacks two of a step's four slices, so that at 128
-// activation rows (MI = 2) every weight is unpacked once (the 64 x 256 tile unpacks it twice, once per tile row) with the
-// same partial-tile bytes per workgroup.
-template <class F, int MI, int NI, bool SWIGLU>
+template <class F, bool SWIGLU>
 __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
-    constexpr int BM = 64 * MI, BN = 128 * NI;
+    constexpr int MI = 4, NI = 2, BM = 64 * MI, BN = 128 * NI;
     constexpr int FRAG = 512;                                   // bf16 per published fragment (64 lanes x 8)
     __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LDS_ROW];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[2][16 * NI * FRAG];   // [n-block 0..4 NI - 1][slice 0..3]
@@ -416,17 +440,15 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
     const int n0 = tile_x * BN + wn * (32 * NI);
     const int c_last = c_end - 1;
 
-    // the weight row this lane unpacks: n-block 2*wn + wm of the workgroup tile (NI = 1: n-block wn, of which this wave
-    // unpacks slices 2*wm and 2*wm + 1); clamped: rows past N are computed but not stored
+    // the weight row this lane unpacks: n-block 2*wn + wm of the workgroup tile; clamped: rows past N are computed but not stored
     const uint8_t* wrow;
     {
-        int n = n0 + (NI == 2 ? 32 * wm : 0) + c;
+        int n = n0 + 32 * wm + c;
         n = n < p.N ? n : p.N - 1;
         wrow = p.W + (size_t)(SWIGLU ? swiglu_row(n, p.ff) : n) * p.row_bytes;
     }
-    const int b_wr = ((NI == 2 ? 2 * wn + wm : wn) * 4) * FRAG + lane * 8;    // + t * FRAG
+    const int b_wr = ((2 * wn + wm) * 4) * FRAG + lane * 8;                     // + t * FRAG
     const int b_rd = ((NI * wn) * 4) * FRAG + lane * 8;                        // + (4 * j + t) * FRAG
-    auto mine = [&](int t) { return NI == 2 || (t >> 1) == wm; };             // does this wave unpack slice t (wave-uniform)
 
     f32x16 acc[MI][NI];
 #pragma unroll
@@ -477,7 +499,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
         typename F::Ctx x;
         F::template begin<0>(raw, wrow, c_begin, h, p.nblk, x);
         static_for<0, 4>([&](auto T) {
-            if (mine(T.value)) *(bf16x8*)(&Bs[0][b_wr + T.value * FRAG]) = F::template frag<0, T.value>(raw, x);
+            *(bf16x8*)(&Bs[0][b_wr + T.value * FRAG]) = F::template frag<0, T.value>(raw, x);
         });
         F::template refill<0>(raw, wrow, nc, h, p.nblk);
     }
@@ -517,7 +539,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
 #pragma unroll
                 for (int j = 0; j < NI; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t & 1][i], b[t & 1][j], acc[i][j], 0, 0, 0);
-            if (mine(t)) *(bf16x8*)(&Bs[buf ^ 1][b_wr + t * FRAG]) = F::template frag<GN, t>(raw, ctx);
+            *(bf16x8*)(&Bs[buf ^ 1][b_wr + t * FRAG]) = F::template frag<GN, t>(raw, ctx);
             if constexpr (t < 3) __builtin_amdgcn_sched_group_barrier(0x100, MI + NI, 0);
 #pragma unroll
             for (int u = 0; u < MI * NI; u++) {
@@ -793,6 +815,392 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The kernel for short prompts and small weights: a wave unpacks its own weights. A low tile of the kind above is bound by what a step
+// moves through LDS (operands of both sides written once and read by every wave) and by its barrier every 64 columns: a 128 x 128 x 256
+// chunk of Q4_K took 2.84 us there, 1.1 of it matrix instructions at the clock the chip holds. It takes 1.97 here (1.45 with no loads,
+// 0.6 without the matrix instructions). Here a wave holds BM activation rows x 32 outputs, so a weight is
+// unpacked by the one wave that multiplies it, straight into its B operand, and LDS carries the activations alone: a whole chunk of them
+// at a time, double buffered, one barrier a chunk. The eight waves are NW along N x KW = 8 / NW along the chunk's four steps (a wave does
+// S = 4 / KW of them), and the KW partial sums of an output meet in LDS when a run ends, added in order of the steps. Work distribution
+// and slots of partial tiles are those of the tiled kernel. Measured with the tile the estimate picks, us: Q4_K 5120 x 5120 at 64 / 128 /
+// 512 rows 17.6 / 22.8 / 45.2 -> 14.5 / 19.0 / 38.2, 6112 x 2816 at 132 42.0 -> 16.6, 10176 x 2560 at 82 27.2 -> 15.8; Q6_K 5120 x 17408 at
+// 128 58.2 -> 48.0; Q8_0 12152 x 1536 at 107 26.0 -> 18.1. Loading a chunk's activations and storing them to LDS at its end, where all
+// waves wait, cost 2.45 us a chunk: a piece now goes to LDS behind each slice, a chunk after it was asked for.
+// Per format: `Raw` holds what a lane half unpacks of S steps of one weight row, as it was loaded (pieces at 2-byte alignment are shifted
+// into place by settle(), where they are first read); begin<I>() derives step I's scales, frag<I, T>() the operand of its slice T.
+// ------------------------------------------------------------------------------------------------
+template <int S>
+struct OwnQ4K {
+    struct Raw { u32x4 hd, q[S]; };
+    struct Ctx { float d0, o0, d1, o1; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
+        const uint8_t* blk = row + (size_t)c * 144;
+        r.hd = *(const u32x4*)blk;
+#pragma unroll
+        for (int i = 0; i < S; i++) r.q[i] = *(const u32x4*)(blk + 16 + 32 * (g0 + i) + 16 * h);
+    }
+    static __device__ __forceinline__ void settle(Raw&, const uint8_t*, int, int, int) {}
+    // the scales (or minima) of sub-blocks 2G and 2G + 1 in the two low bytes, G = g0 + I
+    static __device__ __forceinline__ uint32_t pair(uint32_t lo, uint32_t hi, uint32_t top, bool high, int sh) {
+        return (high ? hi | ((top >> 2) & 0x30303030u) : lo & 0x3F3F3F3Fu) >> sh;
+    }
+    template <int I>
+    static __device__ __forceinline__ void begin(const Raw& r, const uint8_t*, int, int g0, int, int, Ctx& x) {
+        const int G = g0 + I, sh = 16 * (G & 1);
+        const uint32_t a = r.hd[1], b = r.hd[2], cc = r.hd[3];
+        const uint32_t sc = pair(a, cc & 0x0F0F0F0Fu, a, G >= 2, sh), mn = pair(b, (cc >> 4) & 0x0F0F0F0Fu, b, G >= 2, sh);
+        const float d = f16_bits(r.hd[0] & 0xFFFFu) * Q_ULP, dmin = f16_bits(r.hd[0] >> 16);
+        x.d0 = d * ub(sc, 0); x.o0 = -(dmin * ub(mn, 0)); x.d1 = (d * ub(sc, 1)) * 0.0625f; x.o1 = -(dmin * ub(mn, 1));
+    }
+    template <int I, int T>
+    static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
+        return frag8_nibbles(r.q[I][2 * (T & 1)], r.q[I][2 * (T & 1) + 1], T < 2 ? 0x000F000Fu : 0x00F000F0u, T < 2 ? x.d0 : x.d1, T < 2 ? x.o0 : x.o1);
+    }
+};
+
+template <int S>
+struct OwnQ5K {
+    struct Raw { u32x4 hd, qh, q[S]; };
+    using Ctx = typename OwnQ4K<S>::Ctx;
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
+        const uint8_t* blk = row + (size_t)c * 176;
+        r.hd = *(const u32x4*)blk;
+        r.qh = *(const u32x4*)(blk + 16 + 16 * h);
+#pragma unroll
+        for (int i = 0; i < S; i++) r.q[i] = *(const u32x4*)(blk + 48 + 32 * (g0 + i) + 16 * h);
+    }
+    // bits 2 g0 ... of every qh byte to the bottom
+    static __device__ __forceinline__ void settle(Raw& r, const uint8_t*, int, int g0, int) {
+#pragma unroll
+        for (int w = 0; w < 4; w++) r.qh[w] >>= 2 * g0;
+    }
+    template <int I>
+    static __device__ __forceinline__ void begin(const Raw& r, const uint8_t*, int, int g0, int, int, Ctx& x) {
+        const int G = g0 + I, sh = 16 * (G & 1);
+        const uint32_t a = r.hd[1], b = r.hd[2], cc = r.hd[3];
+        const uint32_t sc = OwnQ4K<S>::pair(a, cc & 0x0F0F0F0Fu, a, G >= 2, sh), mn = OwnQ4K<S>::pair(b, (cc >> 4) & 0x0F0F0F0Fu, b, G >= 2, sh);
+        const float d = f16_bits(r.hd[0] & 0xFFFFu) * Q_ULP, dmin = f16_bits(r.hd[0] >> 16);
+        x.d0 = d * ub(sc, 0); x.o0 = -(dmin * ub(mn, 0)); x.d1 = d * ub(sc, 1); x.o1 = -(dmin * ub(mn, 1));
+    }
+    template <int I, int T>
+    static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
+        constexpr int w = 2 * (T & 1), s = 2 * I + (T >> 1);
+        uint32_t v[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t nib = T < 2 ? r.q[I][w + i] & 0x0F0F0F0Fu : (r.q[I][w + i] >> 4) & 0x0F0F0F0Fu;
+            const uint32_t bit = (s >= 4 ? r.qh[w + i] >> (s - 4) : r.qh[w + i] << (4 - s)) & 0x10101010u;
+            v[i] = nib | bit;
+        }
+        return frag8(v[0], v[1], T < 2 ? x.d0 : x.d1, T < 2 ? x.o0 : x.o1);
+    }
+};
+
+template <int S>
+struct OwnQ6K {
+    static constexpr int NH = S == 4 ? 2 : 1;                   // halves of the super-block the steps lie in
+    struct Raw { fhip::Un16 ql[NH][2], qh[NH]; uint32_t sc[NH][3], d; };
+    struct Ctx { float d; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
+        const uint8_t* blk = row + (size_t)c * 210;
+#pragma unroll
+        for (int i = 0; i < NH; i++) {
+            const int hf = (g0 >> 1) + i;
+            r.ql[i][0] = fhip::load16_un<true>(blk + 64 * hf + 16 * h);
+            r.ql[i][1] = fhip::load16_un<true>(blk + 64 * hf + 32 + 16 * h);
+            r.qh[i] = fhip::load16_un<true>(blk + 128 + 32 * hf + 16 * h);
+            const uint8_t* s = blk + 192 + 8 * hf;
+            const fhip::ld_u32x2 v = ((const fhip::LdU2A4*)(s - ((uint32_t)(uintptr_t)s & 2u)))->v;
+            r.sc[i][0] = v[0];
+            r.sc[i][1] = v[1];
+            r.sc[i][2] = *(const uint16_t*)(s + 6);
+        }
+        r.d = *(const uint16_t*)(blk + 208);
+    }
+    static __device__ __forceinline__ void settle(Raw& r, const uint8_t* row, int c, int g0, int h) {
+        const uint32_t m = ((uint32_t)(uintptr_t)row + 2u * (uint32_t)(c & 1)) & 2u;     // every piece starts at a multiple of 4 of its block
+#pragma unroll
+        for (int i = 0; i < NH; i++) {
+            fhip::shift_in_place(r.ql[i][0], m);
+            fhip::shift_in_place(r.ql[i][1], m);
+            fhip::shift_in_place(r.qh[i], m);
+            // byte h of every 16-bit pair is this lane half's scale
+            r.sc[i][0] = __builtin_amdgcn_alignbyte(r.sc[i][1], r.sc[i][0], m) >> (8 * h);
+            r.sc[i][1] = __builtin_amdgcn_alignbyte(r.sc[i][2], r.sc[i][1], m) >> (8 * h);
+        }
+        if constexpr (S == 1) {                                 // an odd step's nibbles, bit pairs and scales to an even step's places
+            const int sh = 4 * (g0 & 1);
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                r.ql[0][0].w[w] >>= sh;
+                r.ql[0][1].w[w] >>= sh;
+                r.qh[0].w[w] >>= sh;
+            }
+            r.sc[0][0] = g0 & 1 ? r.sc[0][1] : r.sc[0][0];
+        }
+    }
+    template <int I>
+    static __device__ __forceinline__ void begin(const Raw& r, const uint8_t*, int, int, int, int, Ctx& x) { x.d = f16_bits(r.d); }
+    template <int I, int T>
+    static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
+        constexpr int hf = I >> 1, odd = I & 1, g = 2 * odd + (T >> 1), par = T >> 1, w = 2 * (T & 1);
+        const uint32_t l0 = r.ql[hf][par].w[w], l1 = r.ql[hf][par].w[w + 1];
+        const uint32_t h0 = r.qh[hf].w[w], h1 = r.qh[hf].w[w + 1];
+        const uint32_t n0 = (odd ? l0 >> 4 : l0) & 0x0F0F0F0Fu, n1 = (odd ? l1 >> 4 : l1) & 0x0F0F0F0Fu;
+        const uint32_t u0 = (g < 2 ? h0 << (4 - 2 * (g & 1)) : h0 >> (2 * (g & 1))) & 0x30303030u;
+        const uint32_t u1 = (g < 2 ? h1 << (4 - 2 * (g & 1)) : h1 >> (2 * (g & 1))) & 0x30303030u;
+        const float ds = x.d * (float)(int8_t)((r.sc[hf][odd] >> (16 * (g & 1))) & 0xFFu);
+        return frag8(n0 | u0, n1 | u1, ds * Q_ULP, -32.0f * ds);
+    }
+};
+
+template <int S>
+struct OwnQ80 {
+    struct Raw { fhip::Un16 q[S][2]; uint32_t d[S][2]; };
+    struct Ctx { float d[2]; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int nblk) {
+#pragma unroll
+        for (int i = 0; i < S; i++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint8_t* p = Q80T<true>::blk(row, c, 2 * (g0 + i) + u, nblk);
+                r.d[i][u] = *(const uint16_t*)p;
+                r.q[i][u] = fhip::load16_un<true>(p + 2 + 16 * h);
+            }
+    }
+    static __device__ __forceinline__ void settle(Raw&, const uint8_t*, int, int, int) {}
+    template <int I>
+    static __device__ __forceinline__ void begin(Raw& r, const uint8_t* row, int c, int g0, int, int nblk, Ctx& x) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i = 8 * c + 2 * (g0 + I) + u, bi = i < nblk ? i : nblk - 1;
+            fhip::shift_in_place(r.q[I][u], ((uint32_t)(uintptr_t)row + 2u * (uint32_t)(bi & 1) + 2u) & 2u);
+            x.d[u] = i < nblk ? f16_bits(r.d[I][u]) : 0.0f;
+        }
+    }
+    template <int I, int T>
+    static __device__ __forceinline__ bf16x8 frag(const Raw& r, const Ctx& x) {
+        const float d = x.d[T >> 1];
+        return frag8(r.q[I][T >> 1].w[2 * (T & 1)] ^ 0x80808080u, r.q[I][T >> 1].w[2 * (T & 1) + 1] ^ 0x80808080u, d * Q_ULP, -128.0f * d);
+    }
+};
+
+template <class F, int S> struct Own;
+template <int S> struct Own<Q4K, S> { using type = OwnQ4K<S>; };
+template <int S> struct Own<Q5K, S> { using type = OwnQ5K<S>; };
+template <int S> struct Own<Q6K, S> { using type = OwnQ6K<S>; };
+template <int S> struct Own<Q80, S> { using type = OwnQ80<S>; };
+
+constexpr int XROW = CHUNK + 8;      // bf16 per staged activation row of a chunk (+16 B pad: conflict-free 16-byte reads)
+
+template <class FMT, int MI, int NW, int KW, bool SWIGLU>
+__global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParams p) {
+    constexpr int BM = 32 * MI, BN = 32 * NW, S = 4 / KW;
+    constexpr int KEEP = 16 / KW;                               // of a fragment's 16 accumulator registers, those a wave stores in the end
+    using F = typename Own<FMT, S>::type;
+    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * XROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave % NW, kg = wave / NW, g0 = S * kg;
+    const int h = lane >> 5, c = lane & 31;
+    const int nchunks = p.nchunks;
+    long long u = (long long)blockIdx.x * p.per;
+    const long long u_end = u + p.per < p.units ? u + p.per : p.units;
+  for (int round = 0;; round++) {
+    int tile, c_begin, c_end;
+    if (round < p.whole_rounds) {
+        tile = round * gridDim.x + blockIdx.x;
+        c_begin = 0;
+        c_end = nchunks;
+    } else {
+        if (u >= u_end) break;
+        const int rt = (int)(u / nchunks);
+        tile = p.whole_rounds * gridDim.x + rt;
+        c_begin = (int)(u - (long long)rt * nchunks);
+        c_end = (long long)(nchunks - c_begin) < u_end - u ? nchunks : c_begin + (int)(u_end - u);
+        u += c_end - c_begin;
+    }
+    const bool whole = c_begin == 0 && c_end == nchunks;
+    const int tile_y = tile / p.tiles_n, tile_x = tile - tile_y * p.tiles_n;
+    const int t0 = tile_y * BM, n0 = tile_x * BN + 32 * wn;
+    const int c_last = c_end - 1;
+    const uint8_t* wrow;                                        // rows past N are computed but not stored
+    {
+        int n = n0 + c;
+        n = n < p.N ? n : p.N - 1;
+        wrow = p.W + (size_t)(SWIGLU ? swiglu_row(n, p.ff) : n) * p.row_bytes;
+    }
+    f32x16 acc[MI];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
+
+    // Activation staging: thread `tid` moves the 16-byte piece (tid & 31) of rows (tid >> 5) + 16 q. Rows past T are read from row T-1,
+    // columns past K (a partial last chunk) are staged as zeros.
+    constexpr int RQ = 2 * NW * KW, NQ = (BM + RQ - 1) / RQ;    // rows a round of the threads moves, rounds
+    const int a_col = (tid & 31) * 8;
+    uint32_t a_src[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        int t = (tid >> 5) + RQ * q;
+        t = t0 + (t < BM ? t : BM - 1);
+        a_src[q] = (uint32_t)(t < p.T ? t : p.T - 1) * (uint32_t)p.K + a_col;
+    }
+    const int a_dst = (tid >> 5) * XROW + a_col;
+    // a last round of fewer rows: the threads past it write the tile's last row again, with what it holds
+    const int a_dst_last = ((tid >> 5) + RQ * (NQ - 1) < BM ? (tid >> 5) + RQ * (NQ - 1) : BM - 1) * XROW + a_col;
+    u32x4 stage[NQ];
+    auto load_a = [&](int ck, int q) {
+        const bool ok = !FMT::PARTIAL || ck * CHUNK + a_col < p.K;
+        stage[q] = *(const u32x4*)(p.X + (a_src[q] + (ok ? ck * CHUNK : 0)));
+        if (FMT::PARTIAL) {
+            const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
+            stage[q] = (u32x4){stage[q][0] & keep, stage[q][1] & keep, stage[q][2] & keep, stage[q][3] & keep};
+        }
+    };
+    auto store_a = [&](int buf, int q) { *(u32x4*)(&As[buf][q == NQ - 1 && BM % RQ != 0 ? a_dst_last : a_dst + RQ * q * XROW]) = stage[q]; };
+    const int a_rd = c * XROW + 16 * h + KSTEP * g0;            // + 32 i rows, + KSTEP I + kcol(t, 0)
+
+    // Chunk ck from activation buffer P and register set P. Slice by slice: the next slice's activations are read from LDS, then the
+    // matrix instructions alternate with the unpacking of the next slice; behind them a piece of chunk ck + 1's activations, requested a
+    // chunk ago, goes to the other buffer and its register asks for chunk ck + 2. The barrier stands in front of the last slice, whose
+    // matrix instructions cover the first reads and the first unpacking of the next chunk.
+    constexpr int NS = 4 * S, QS = (NQ + NS - 3) / (NS - 2);    // slices of a chunk; pieces moved behind each of the first NS - 2
+    typename F::Raw raw[2];
+    bf16x8 a[2][MI], b[2];
+    typename F::Ctx ctx;
+    auto read_a = [&](int buf, int s, bf16x8 (&d)[MI]) {
+#pragma unroll
+        for (int i = 0; i < MI; i++) d[i] = *(const bf16x8*)(&As[buf][a_rd + 32 * i * XROW + KSTEP * (s >> 2) + kcol(s & 3, 0)]);
+    };
+    auto chunk = [&](auto Pc, auto Lc, int ck) {
+        constexpr int P = decltype(Pc)::value;
+        constexpr bool LOADS = decltype(Lc)::value;
+        const int c2 = ck + 2 < c_last ? ck + 2 : c_last;
+        static_for<0, NS>([&](auto Sc) {
+            constexpr int s = decltype(Sc)::value, n = s + 1;
+            if constexpr (n < NS) read_a(P, n, a[n & 1]);
+            else read_a(P ^ 1, 0, a[0]);
+            if constexpr (n == NS) {
+                F::settle(raw[P ^ 1], wrow, ck + 1, g0, h);
+                F::template begin<0>(raw[P ^ 1], wrow, ck + 1, g0, h, p.nblk, ctx);
+            } else if constexpr ((n & 3) == 0) F::template begin<(n >> 2)>(raw[P], wrow, ck, g0, h, p.nblk, ctx);
+#pragma unroll
+            for (int i = 0; i < MI; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][i], b[s & 1], acc[i], 0, 0, 0);
+            if constexpr (n == NS) b[0] = F::template frag<0, 0>(raw[P ^ 1], ctx);
+            else b[n & 1] = F::template frag<(n >> 2), (n & 3)>(raw[P], ctx);
+            if constexpr (LOADS && s == NS - 2) F::load(raw[P], wrow, c2, g0, h, p.nblk);
+#pragma unroll
+            for (int q = QS * s; q < QS * (s + 1) && q < NQ; q++) {
+                store_a(P ^ 1, q);
+                if (LOADS) load_a(c2, q);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, MI, 0);
+            constexpr int VPM = (24 + MI - 1) / MI;
+#pragma unroll
+            for (int m = 0; m < MI; m++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+            }
+            if constexpr (s == NS - 2) __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    {
+        const int c1 = c_begin < c_last ? c_begin + 1 : c_last;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) load_a(c_begin, q);
+        F::load(raw[0], wrow, c_begin, g0, h, p.nblk);
+        if (round > 0) __syncthreads();                         // the last run's sums are read
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            store_a(0, q);
+            load_a(c1, q);
+        }
+        F::load(raw[1], wrow, c1, g0, h, p.nblk);
+        __syncthreads();
+        read_a(0, 0, a[0]);
+        F::settle(raw[0], wrow, c_begin, g0, h);
+        F::template begin<0>(raw[0], wrow, c_begin, g0, h, p.nblk, ctx);
+        b[0] = F::template frag<0, 0>(raw[0], ctx);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    using std::integral_constant;
+    int ck = c_begin;
+    for (; ck + 2 < c_end; ck += 2) {
+        chunk(integral_constant<int, 0>{}, std::true_type{}, ck);
+        chunk(integral_constant<int, 1>{}, std::true_type{}, ck + 1);
+    }
+    chunk(integral_constant<int, 0>{}, std::false_type{}, ck);
+    if (ck + 1 < c_end) chunk(integral_constant<int, 1>{}, std::false_type{}, ck + 1);
+
+    // the waves that share outputs meet: wave kg keeps registers [KEEP kg, KEEP kg + KEEP) of every fragment
+    if constexpr (KW > 1) {
+        float* sums = (float*)&As[0][0];
+        // [wave][other steps][MI x KEEP registers][lane]
+        auto slot = [&](int k_from, int k_to) { return ((k_from * NW + wn) * (KW - 1) + (k_to < k_from ? k_to : k_to - 1)) * (MI * KEEP * 64) + lane; };
+        static_for<0, KW>([&](auto To) {
+            constexpr int to = decltype(To)::value;
+            if (to != kg) {
+                float* q = sums + slot(kg, to);
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int r = 0; r < KEEP; r++) q[(i * KEEP + r) * 64] = acc[i][to * KEEP + r];
+            }
+        });
+        __syncthreads();
+        static_for<0, KW>([&](auto Kc) {
+            constexpr int k = decltype(Kc)::value;
+            if (k == kg) {
+#pragma unroll
+                for (int from = 0; from < KW; from++)
+                    if (from != k) {
+                        const float* q = sums + slot(from, k);
+#pragma unroll
+                        for (int i = 0; i < MI; i++)
+#pragma unroll
+                            for (int r = 0; r < KEEP; r++) acc[i][k * KEEP + r] += q[(i * KEEP + r) * 64];
+                    }
+            }
+        });
+    }
+    float* part = nullptr;
+    if (!whole) {
+        const int rt = tile - p.whole_rounds * (int)gridDim.x;
+        const int k = (int)blockIdx.x - (int)(((long long)rt * nchunks) / p.per);
+        part = p.ws + ((size_t)rt * p.kmax + k) * (size_t)(BM * BN);
+    }
+    static_for<0, KW>([&](auto Kc) {
+        constexpr int k = decltype(Kc)::value;
+        if (k != kg) return;
+        const int n = n0 + c;
+#pragma unroll
+        for (int i = 0; i < MI; i++) {
+            if (SWIGLU && whole) {
+                store_swiglu<k * KEEP, KEEP>(p, acc[i], t0 + 32 * i, n0, h, c);
+                continue;
+            }
+            if (!whole) {                                       // a slot holds the whole tile, rows past T and columns past N included
+#pragma unroll
+                for (int r = k * KEEP; r < (k + 1) * KEEP; r++)
+                    part[(32 * i + 8 * (r >> 2) + 4 * h + (r & 3)) * BN + 32 * wn + c] = acc[i][r];
+                continue;
+            }
+            if (n >= p.N) continue;
+            float* y = p.Y + (size_t)(t0 + 32 * i + 4 * h) * p.N + n;
+            const int left = p.T - t0 - 32 * i - 4 * h;
+#pragma unroll
+            for (int r = k * KEEP; r < (k + 1) * KEEP; r++) {
+                const int t = 8 * (r >> 2) + (r & 3);
+                if (t < left) y[(size_t)t * p.N] = acc[i][r];
+            }
+        }
+    });
+  }
+}
+
 // Left-over tile `blockIdx.x` (BM x BN outputs, BN a multiple of 4), if more than one run contributed to it: Y = slot 0 +
 // slot 1 + ... in that order. A thread owns four adjacent columns of one row (item blockIdx.y * 256 + threadIdx.x of the
 // tile's BM * BN / 4) and asks for up to eight slots at once: the launch is a few dependent trips to memory long, so it
@@ -897,8 +1305,6 @@ struct SkinnyParams {
     int kmax;          // contributor slots per group
 };
 
-constexpr int XROW = CHUNK + 8;   // bf16 per staged activation row of a chunk (+16 B pad)
-
 template <class F, int TP>
 __global__ void __launch_bounds__(256, TP == 8 ? 4 : 2) gemm_q_bf16_skinny_kernel(SkinnyParams p) {
     __shared__ __attribute__((aligned(16))) uint16_t Xs[2][TP * XROW];
@@ -938,7 +1344,6 @@ __global__ void __launch_bounds__(256, TP == 8 ? 4 : 2) gemm_q_bf16_skinny_kerne
         const int c_end = (long long)(nchunks - c_begin) < u_end - u ? nchunks : c_begin + (int)(u_end - u);
         u += c_end - c_begin;
         const bool whole = c_begin == 0 && c_end == nchunks;
-        const int c_last = c_end - 1;
         const int n = grp * 128 + wave * 32 + c;
         const uint8_t* wrow = p.W + (size_t)(n < p.N ? n : p.N - 1) * p.row_bytes;
 
@@ -1079,160 +1484,217 @@ int launch_skinny(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_
     return fhip::check_hip(hipGetLastError(), "gemm_q_bf16 launch");
 }
 
-// How a launch of the tiled kernel with tile height 64 * mi is dealt to the chip: `whole_rounds` whole tiles per workgroup,
-// then the left-over tiles cut along K into runs of `per` chunks.
+// The tiles: rows x outputs. 2, 3 and 6 share a weight's unpacking among the waves that multiply it, the others leave it to the one wave.
+// 12 and 13 are 4 and 5 with one wave along K (run sums, below).
+constexpr int BM_OF[NTILES + 2] = {64, 128, 256, 256, 128, 64, 128, 128, 64, 64, 64, 128, 128, 64}, BN_OF[NTILES + 2] = {256, 256, 256, 160, 128, 128, 160, 96, 96, 160, 64, 64, 128, 128};
+
+// How a launch is dealt to the chip: `whole_rounds` whole tiles per workgroup, then the left-over tiles cut along K into runs of `per` chunks.
 struct TilePlan {
-    int mi, bn;                         // tile of 64 * mi activation rows x bn outputs (256, 128, or 160 with mi = 4 or 2)
+    int tile, bm, bn, nchunks;
     int whole_rounds, per;
-    long long left, units, split_wgs;   // left-over tiles, their chunks, workgroups whose run ends in partial tiles
+    long long left, units, runs;        // left-over tiles, their chunks, the runs they are cut into
+    bool split;                         // a run ends inside a tile
     int kmax;                           // most runs that touch one left-over tile
-    long long slots;                    // partial tiles the launch writes: over the left-over tiles cut along K, the runs that touch each
-    float extra_starts;                 // tiles a run touches beyond its first, on average (a run that ends in the next tile starts twice)
     unsigned grid;
 };
 
-static TilePlan plan_tiles(long long tiles_n, int nchunks, size_t t, int mi, long long cus, int bn = 256) {
+static TilePlan plan_tiles(size_t columns, int nchunks, size_t t, int tile, long long cus) {
     TilePlan q;
-    q.mi = mi; q.bn = bn;
-    const long long tiles = tiles_n * (long long)((t + 64 * mi - 1) / (64 * mi));
+    q.tile = tile; q.bm = BM_OF[tile]; q.bn = BN_OF[tile]; q.nchunks = nchunks;
+    const long long tiles = (long long)((columns + q.bn - 1) / q.bn) * (long long)((t + q.bm - 1) / q.bm);
     q.whole_rounds = (int)(tiles / cus);
     q.left = tiles - q.whole_rounds * cus;
     q.units = q.left * nchunks;
-    long long per = (q.units + cus - 1) / cus;
+    int per = (int)((q.units + cus - 1) / cus);
     // a run shorter than a tile's K that is close to it is rounded up to whole tiles: no partial tiles, no summing launch
-    if (per * 4 >= (long long)nchunks * 3) per = nchunks;
+    if (per * 4 >= nchunks * 3) per = nchunks;
     if (per < 1) per = 1;
-    q.per = (int)per;
-    const long long runs = (q.units + per - 1) / per;
-    q.grid = q.whole_rounds > 0 ? (unsigned)cus : (unsigned)runs;
-    q.split_wgs = (q.left > 0 && per % nchunks != 0) ? runs : 0;
+    q.per = per;
+    q.runs = (q.units + per - 1) / per;
+    q.grid = q.whole_rounds > 0 ? (unsigned)cus : (unsigned)q.runs;
+    q.split = q.left > 0 && per < nchunks;
     q.kmax = 1;
-    q.slots = 0;
-    long long segs = 0;
-    for (long long rt = 0; rt < q.left && q.split_wgs > 0; rt++) {
-        const long long u0 = rt * nchunks;
-        const int k = (int)((u0 + nchunks - 1) / per - u0 / per) + 1;
+    // tile rt starts at unit rt * nchunks, `start` units into a run: the latest start meets the most runs
+    for (long long rt = 0, start = 0; rt < q.left && q.split; rt++) {
+        const int k = (int)(start + nchunks - 1) / per + 1;
         if (k > q.kmax) q.kmax = k;
-        if (k > 1) q.slots += k;
-        segs += k;
+        start = (start + nchunks) % per;
+        if (start == 0) break;
     }
-    q.extra_starts = q.split_wgs > 0 ? (float)segs / (float)runs - 1.f : 0.f;
     return q;
 }
 
-// Estimated duration of a plan in us: 4.3 for the launch, 1.5 per tile or run a workgroup starts (4.0 more per further tile a
-// run reaches into), chunks per workgroup x the cost of a chunk of that tile and format (F::CHUNK_US), and, when tiles are cut
-// along K, the partial tiles and the launch that sums them: 7.8 per 256 partial tiles of 64 x 256 written and read back, plus a
-// constant per tile shape. A linear model fitted (relative least squares, 7 % rms) to 620 forced-tile launches: ten weights of
-// the four formats (5120 x 5120, 34816 x 5120, 7168 x 5120, 10240 x 5120, 4096 x 4096 Q4_K; 5120 x 17408, 5120 x 5120 Q6_K;
-// 4096 x 4096, 12288 x 4096 Q8_0; 5120 x 5120 Q5_K) at 48 ... 2048 rows, every tile. On those the tile it picks is 1.0 % slower
-// than the measured best on average (worst: 17 %, Q6_K 5120 x 5120 at 256 rows).
-constexpr float FIXUP_US[7] = {0.9f, -2.3f, -13.2f, -5.2f, -1.0f, 1.5f, 0.4f};
-static int tile_index(const TilePlan& q) { return q.bn == 256 ? (q.mi == 1 ? 0 : q.mi == 2 ? 1 : 2) : q.bn == 160 ? (q.mi == 4 ? 3 : 6) : (q.mi == 2 ? 4 : 5); }
+// the partial tiles of a plan that cuts: runs meet one more tile for every tile boundary inside one
+static long long plan_segments(const TilePlan& q) { return q.runs + (q.left - 1) - (q.left - 1) / (q.per / std::gcd(q.per, q.nchunks)); }
+
+// Estimated duration of a plan in us: a start per tile or run a workgroup begins, chunks per workgroup x the cost of a chunk of that tile and format
+// (F::CHUNK_US), and, where tiles are cut along K, 0.1 a chunk, the summing launch and the partial tiles, 4.2 per 256 of 128 x 128 written and read back.
+// A linear model fitted (non-negative least squares on relative errors, 7 % rms) to 3700 launches: 357 weights of the four formats, 1024 ... 34816 rows
+// of 1024 ... 17408 columns, 33 ... 2048 activation rows, every tile. On those the tile it picks is 1.4 % slower than the measured best on average
+// (worst 25 %); the model it replaced, fitted to ten large weights, and the seven tiles it had were 20 % slower on average and up to 2.7 times
+// (6112 x 2816 Q4_K at 132 rows 42.0 -> 16.6 us). Left out, a tile costs 0.1 % (64 x 256, 64 x 160) to 2.5 % (64 x 64) of the mean.
+constexpr float START_US[NTILES] = {3.77f, 3.88f, 4.04f, 4.53f, 3.92f, 3.12f, 4.91f, 3.57f, 2.73f, 4.01f, 2.31f, 3.95f}, FIX_US = 3.29f, SLOT_US = 4.18f, CUT_US = 0.1f;
 template <class F>
-static float plan_cost_us(const TilePlan& q, int nchunks, long long cus) {
-    const int ti = tile_index(q);
-    const float chunks = (float)q.whole_rounds * (float)nchunks + (q.left > 0 ? (float)q.per : 0.f);
+static float plan_cost_us(const TilePlan& q, long long cus) {
+    const float chunks = (float)q.whole_rounds * (float)q.nchunks + (q.left > 0 ? (float)q.per : 0.f);
     const float starts = (float)q.whole_rounds + (q.left > 0 ? 1.f : 0.f);
-    float fix = 0.f;
-    if (q.split_wgs > 0) {
-        fix = FIXUP_US[ti] + 7.77f * (float)q.mi * ((float)q.bn / 256.f) * (float)q.slots / (float)cus;
-        fix = fix > 0.f ? fix : 0.f;
+    float fix = 0.f, again = 0.f;
+    if (q.split) {
+        const long long segs = plan_segments(q);
+        fix = FIX_US + CUT_US * (float)q.per + SLOT_US * (float)(q.bm * q.bn) / 16384.f * (float)segs / (float)cus;
+        again = (float)segs / (float)q.runs - 1.f;
     }
-    return 4.29f + 1.5f * starts + 3.96f * q.extra_starts + chunks * F::CHUNK_US[ti] + fix;
+    return START_US[q.tile] * (starts + again) + chunks * F::CHUNK_US[q.tile] + fix;
 }
 
 static size_t plan_ws_bytes(const TilePlan& q) {
-    return q.split_wgs > 0 ? (size_t)q.left * q.kmax * (size_t)(64 * q.mi * q.bn) * sizeof(float) : 0;
+    return q.split ? (size_t)q.left * q.kmax * (size_t)(q.bm * q.bn) * sizeof(float) : 0;
 }
 
 // columns of a SwiGLU launch (see swiglu_row)
 static size_t swiglu_columns(size_t ff) { return (ff + 15) / 16 * 32; }
 
-template <class F, int MI, int BN, bool SWIGLU>
-int launch_cfg(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out, hipStream_t s, const TilePlan& q, long long cus, float* d_ws,
-               size_t ws_bytes) {
-    GemmParams p;
-    const size_t columns = SWIGLU ? swiglu_columns(w->rows / 2) : w->rows;
-    p.W = w->d_raw; p.X = d_x; p.Y = SWIGLU ? nullptr : (float*)d_out; p.H = SWIGLU ? (uint16_t*)d_out : nullptr; p.ff = (int)(w->rows / 2);
+static int fill_params(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out, bool swiglu, int block, const TilePlan& q, float* d_ws, size_t ws_bytes,
+                       GemmParams& p) {
+    const size_t columns = swiglu ? swiglu_columns(w->rows / 2) : w->rows;
+    p.W = w->d_raw; p.X = d_x; p.Y = swiglu ? nullptr : (float*)d_out; p.H = swiglu ? (uint16_t*)d_out : nullptr; p.ff = (int)(w->rows / 2);
     p.T = (int)t; p.N = (int)columns; p.K = (int)w->cols; p.row_bytes = w->row_bytes;
-    p.nblk = (int)(w->row_bytes / F::BLOCK);
-    p.nchunks = F::chunks(p.K);
-    p.tiles_n = (int)((columns + BN - 1) / BN);
+    p.nblk = (int)(w->row_bytes / block);
+    p.nchunks = q.nchunks;
+    p.tiles_n = (int)((columns + q.bn - 1) / q.bn);
     // one workgroup per CU (its LDS tiles take most of a CU's 160 KB)
     p.whole_rounds = q.whole_rounds;
     p.units = q.units;
     p.per = q.per;
     p.ws = d_ws; p.kmax = q.kmax;
-    if (q.split_wgs > 0 && (!d_ws || ws_bytes < plan_ws_bytes(q)))
+    if (q.split && (!d_ws || ws_bytes < plan_ws_bytes(q)))
         return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: the launch cuts tiles along K and needs %zu bytes of workspace", plan_ws_bytes(q));
-    using W = std::conditional_t<MI == 4, typename F::Eager, F>;
-    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<W, MI, 2, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
-    else if constexpr (BN == 128) hipLaunchKernelGGL((gemm_q_bf16_kernel<W, MI, 1, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<W, MI, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
-    if (q.split_wgs > 0 && SWIGLU)
-        hipLaunchKernelGGL(sum_split_swiglu_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 8 + 255) / 256)), dim3(256), 0, s, p.H, (const float*)d_ws, p.T, p.ff, 64 * MI,
-                           BN, p.tiles_n, p.nchunks, p.per, p.kmax, (int)(p.whole_rounds * cus));
-    else if (q.split_wgs > 0)
-        hipLaunchKernelGGL(sum_split_tiles_kernel, dim3((unsigned)q.left, (unsigned)((64 * MI * BN / 4 + 255) / 256)), dim3(256), 0, s, p.Y, (const float*)d_ws, p.T, p.N, 64 * MI,
-                           BN, p.tiles_n, p.nchunks, p.per, p.kmax, (int)(p.whole_rounds * cus));
+    return FHIP_OK;
+}
+static int launch_sums(const GemmParams& p, const TilePlan& q, bool swiglu, hipStream_t s) {
+    const unsigned per_tile = (unsigned)(q.bm * q.bn / (swiglu ? 8 : 4) + 255) / 256;
+    const int first = q.whole_rounds * (int)q.grid;
+    if (q.split && swiglu)
+        hipLaunchKernelGGL(sum_split_swiglu_kernel, dim3((unsigned)q.left, per_tile), dim3(256), 0, s, p.H, (const float*)p.ws, p.T, p.ff, q.bm, q.bn, p.tiles_n, p.nchunks, p.per,
+                           p.kmax, first);
+    else if (q.split)
+        hipLaunchKernelGGL(sum_split_tiles_kernel, dim3((unsigned)q.left, per_tile), dim3(256), 0, s, p.Y, (const float*)p.ws, p.T, p.N, q.bm, q.bn, p.tiles_n, p.nchunks, p.per, p.kmax,
+                           first);
     return fhip::check_hip(hipGetLastError(), "gemm_q_bf16 launch");
 }
+template <class F, int MI, int BN, bool SWIGLU>
+int launch_shared(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out, hipStream_t s, const TilePlan& q, float* d_ws, size_t ws_bytes) {
+    GemmParams p;
+    if (int rc = fill_params(w, d_x, t, d_out, SWIGLU, F::BLOCK, q, d_ws, ws_bytes, p)) return rc;
+    using W = std::conditional_t<MI == 4, typename F::Eager, F>;
+    if constexpr (BN == 256) hipLaunchKernelGGL((gemm_q_bf16_kernel<W, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((gemm_q_bf16_n160_kernel<W, MI, SWIGLU>), dim3(q.grid), dim3(512), 0, s, p);
+    return launch_sums(p, q, SWIGLU, s);
+}
+template <class F, int MI, int NW, int KW, bool SWIGLU>
+int launch_own(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out, hipStream_t s, const TilePlan& q, float* d_ws, size_t ws_bytes) {
+    GemmParams p;
+    if (int rc = fill_params(w, d_x, t, d_out, SWIGLU, F::BLOCK, q, d_ws, ws_bytes, p)) return rc;
+    hipLaunchKernelGGL((gemm_q_bf16_own_kernel<F, MI, NW, KW, SWIGLU>), dim3(q.grid), dim3(64 * NW * KW), 0, s, p);
+    return launch_sums(p, q, SWIGLU, s);
+}
 
-int g_force_tile = -1;   // tests: 0..3 = 64, 128, 256 rows x 256 columns, 256 x 160; 4, 5 = 128, 64 rows x 128 columns; 6 = 128 x 160; anything else: the estimate decides
 
-// the tile the estimate picks for this launch (one of the seven the loop lists) with its plan
+// A launch of run sums: one wave adds all products of a run for an output, and the runs are those of seven tiles and this estimate, which
+// therefore stand as they are. For rows whose every last bit is stored further on, as the codes of a block-quantized cache: in four layers of a
+// prompt block on one, sums in another order make 38 % of the codes others (none is nearer f64), and a cache that was stored before would not
+// be met again. The tiles of short prompts run on the kernel whose waves unpack for themselves, one along K, which adds in the same order.
+constexpr int RUN_TILE_OF[7] = {0, 1, 2, 3, 12, 13, 6};
+constexpr float RUN_FIXUP_US[7] = {0.9f, -2.3f, -13.2f, -5.2f, -1.0f, 1.5f, 0.4f};
 template <class F>
-static void choose_plan(const fhip_weight* w, size_t columns, size_t t, TilePlan& out) {
+static float run_sums_cost_us(const TilePlan& q, int i, long long cus) {
+    const float chunks = (float)q.whole_rounds * (float)q.nchunks + (q.left > 0 ? (float)q.per : 0.f);
+    const float starts = (float)q.whole_rounds + (q.left > 0 ? 1.f : 0.f);
+    float fix = 0.f, extra_starts = 0.f;
+    if (q.split) {
+        const long long segs = plan_segments(q);
+        fix = RUN_FIXUP_US[i] + 7.77f * (float)(q.bm / 64) * ((float)q.bn / 256.f) * (float)segs / (float)cus;
+        fix = fix > 0.f ? fix : 0.f;
+        extra_starts = (float)segs / (float)q.runs - 1.f;
+    }
+    return 4.29f + 1.5f * starts + 3.96f * extra_starts + chunks * F::RUN_CHUNK_US[i] + fix;
+}
+
+// the tile the estimate picks for this launch
+template <class F>
+static void choose_plan(const fhip_weight* w, size_t columns, size_t t, bool run_sums, TilePlan& out) {
     const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     const int nchunks = F::chunks((int)w->cols);
     float best_cost = 0.f;
-    for (int i = 0; i < 7; i++) {                 // 64, 128, 256 rows x 256 columns, 256 x 160, 128 and 64 rows x 128 columns, 128 x 160
-        constexpr int MI_OF[7] = {1, 2, 4, 4, 2, 1, 2}, BN_OF[7] = {256, 256, 256, 160, 128, 128, 160};
-        const int mi = MI_OF[i], bn = BN_OF[i];
-        if (g_force_tile >= 0 && g_force_tile <= 6 && i != g_force_tile) continue;
-        const TilePlan q = plan_tiles((long long)((columns + bn - 1) / bn), nchunks, t, mi, cus, bn);
-        const float c = plan_cost_us<F>(q, nchunks, cus);
-        if (best_cost == 0.f || c < 0.98f * best_cost) { best_cost = c; out = q; }
+    if (run_sums) {
+        for (int i = 0; i < 7; i++) {
+            const TilePlan q = plan_tiles(columns, nchunks, t, RUN_TILE_OF[i], cus);
+            const float c = run_sums_cost_us<F>(q, i, cus);
+            if (best_cost == 0.f || c < 0.98f * best_cost) { best_cost = c; out = q; }
+        }
+        return;
+    }
+    for (int i = 0; i < NTILES; i++) {
+        if (fhip::g_gemm_tile >= 0 && fhip::g_gemm_tile < NTILES && i != fhip::g_gemm_tile) continue;
+        const TilePlan q = plan_tiles(columns, nchunks, t, i, cus);
+        const float c = plan_cost_us<F>(q, cus);
+        if (best_cost == 0.f || c < best_cost) { best_cost = c; out = q; }
     }
 }
 
 template <class F>
-static size_t ws_bytes_fmt(const fhip_weight* w, size_t columns, size_t t) {
+static size_t ws_bytes_fmt(const fhip_weight* w, size_t columns, size_t t, bool run_sums) {
     if (t <= 32) return skinny_ws_bytes(plan_skinny(w->rows, F::chunks((int)w->cols), t, fhip::device_cus() > 0 ? fhip::device_cus() : 256));
     TilePlan q;
-    choose_plan<F>(w, columns, t, q);
+    choose_plan<F>(w, columns, t, run_sums, q);
     return plan_ws_bytes(q);
 }
 
 template <class F, bool SWIGLU>
-int launch_tiled(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
-    // Which tile. The 256 x 256 tile unpacks each weight once per 256 activation rows, but when there is no whole round of
-    // such tiles for the chip every tile is cut along K, each workgroup writes a whole partial tile for a few chunks of
-    // work, and a lower tile (twice the tiles, half the fix-up, longer runs), the 256 x 160 tile (whose count divides the
-    // chip for output widths like 5120 and 4096) or, for short prompts, a 128-column tile (half the partial-tile bytes a
-    // workgroup writes, every weight unpacked once at 128 rows) can win: the estimate decides. Measured, us at 64 / 128 / 256
-    // rows x 256, 256 x 160, 128 / 64 rows x 128: Q4_K 5120 x 5120 T = 64 21 / 25 / 32 / 34 / 21 / 18, T = 128 25 / 27 / 35 / 36 /
-    // 22 / 27, T = 512 67 / 56 / 53 / 47 / 54 / 62; Q4_K 34816 x 5120 T = 64 57 / 68 / 102 / 96 / 68 / 55, T = 256 157 / 113 / 119 /
-    // 100 / 132 / 187; Q6_K 5120 x 17408 T = 128 80 / 62 / 77 / 73 / 67 / 103, T = 512 254 / 157 / 133 / 116 / 209 / 327; Q8_0
-    // 4096 x 4096 T = 128 35 / 33 / 37 / 32 / 31 / 40.
-    const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+int launch_tiled(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums = false) {
     TilePlan q;
-    choose_plan<F>(w, SWIGLU ? swiglu_columns(w->rows / 2) : w->rows, t, q);
-    if (q.bn == 160) return q.mi == 4 ? launch_cfg<F, 4, 160, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
-                                      : launch_cfg<F, 2, 160, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.bn == 128) return q.mi == 2 ? launch_cfg<F, 2, 128, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes)
-                                      : launch_cfg<F, 1, 128, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.mi == 4) return launch_cfg<F, 4, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    if (q.mi == 2) return launch_cfg<F, 2, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
-    return launch_cfg<F, 1, 256, SWIGLU>(w, d_x, t, d_y, s, q, cus, d_ws, ws_bytes);
+    choose_plan<F>(w, SWIGLU ? swiglu_columns(w->rows / 2) : w->rows, t, run_sums, q);
+    switch (q.tile) {
+        case 0: return launch_own<F, 2, 8, 1, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 1: return launch_own<F, 4, 8, 1, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 2: return launch_shared<F, 4, 256, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 3: return launch_shared<F, 4, 160, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 4: return launch_own<F, 4, 4, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 5: return launch_own<F, 2, 4, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 6: return launch_shared<F, 2, 160, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 7: return launch_own<F, 4, 3, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 8: return launch_own<F, 2, 3, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 9: return launch_own<F, 2, 5, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 10: return launch_own<F, 2, 2, 4, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 11: return launch_own<F, 4, 2, 4, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+    }
+    if constexpr (!SWIGLU) {
+        if (q.tile == 12) return launch_own<F, 4, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        if (q.tile == 13) return launch_own<F, 2, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+    }
+    return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: no tile %d", q.tile);
 }
 
 template <class F>
-int launch_fmt(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
+int launch_fmt(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums) {
     if (t <= 32) return launch_skinny<F>(w, d_x, t, d_y, s, d_ws, ws_bytes);
-    return launch_tiled<F, false>(w, d_x, t, d_y, s, d_ws, ws_bytes);
+    return launch_tiled<F, false>(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
 }
+
+}  // namespace
+
+namespace fhip {
+size_t FHIP_GEMM_NAME(_ws_bytes)(const fhip_weight* w, size_t columns, size_t t, bool run_sums) { return ws_bytes_fmt<FHIP_GEMM_FORMAT>(w, columns, t, run_sums); }
+int FHIP_GEMM_NAME(_launch)(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums) {
+    return launch_fmt<FHIP_GEMM_FORMAT>(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
+}
+int FHIP_GEMM_NAME(_launch_swiglu)(const fhip_weight* w, const uint16_t* d_x, size_t t, uint16_t* d_h, hipStream_t s, float* d_ws, size_t ws_bytes) {
+    return launch_tiled<FHIP_GEMM_FORMAT, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
+}
+}  // namespace fhip
+
+#ifdef FHIP_GEMM_ENTRY
+namespace {
 
 // f32 -> bf16 (round to nearest even), 8 values per thread, the tail one by one
 __global__ void __launch_bounds__(256) cvt_f32_bf16_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, size_t n) {
@@ -1275,35 +1737,41 @@ int launch_cvt_bf16(const float* d_x, size_t n, uint16_t* d_out, hipStream_t s) 
     return check_hip(hipGetLastError(), "cvt_f32_bf16 launch");
 }
 
+int g_gemm_tile = -1;
 int gemm_bf16_force_tile(int tile) {
-    const int before = g_force_tile;
-    g_force_tile = tile;
+    const int before = g_gemm_tile;
+    g_gemm_tile = tile;
     return before;
 }
 
-size_t gemm_bf16_ws_bytes(const fhip_weight* w, size_t t) {
+size_t gemm_bf16_ws_bytes(const fhip_weight* w, size_t t, bool run_sums) {
     if (!w || t == 0 || w->rows == 0) return 0;
     switch (w->type) {
-        case FHIP_Q4_K: return ws_bytes_fmt<Q4K>(w, w->rows, t);
-        case FHIP_Q6_K: return ws_bytes_fmt<Q6K>(w, w->rows, t);
-        case FHIP_Q8_0: return ws_bytes_fmt<Q80>(w, w->rows, t);
-        case FHIP_Q5_K: return ws_bytes_fmt<Q5K>(w, w->rows, t);
+        case FHIP_Q4_K: return gemm_Q4K_ws_bytes(w, w->rows, t, run_sums);
+        case FHIP_Q6_K: return gemm_Q6K_ws_bytes(w, w->rows, t, run_sums);
+        case FHIP_Q8_0: return gemm_Q80_ws_bytes(w, w->rows, t, run_sums);
+        case FHIP_Q5_K: return gemm_Q5K_ws_bytes(w, w->rows, t, run_sums);
         default: return 0;
     }
 }
 
-int launch_gemm_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
+int launch_gemm_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums) {
     if (t == 0 || w->rows == 0) return FHIP_OK;
     if (((uintptr_t)d_x & 15) != 0) return set_error(FHIP_ERR_ARG, "gemm_q_bf16: x must be 16-byte aligned");
     if ((unsigned long long)t * w->cols >= (1ull << 31))
         return set_error(FHIP_ERR_SHAPE, "gemm_q_bf16: t * cols must be below 2^31 (got %zu x %zu)", t, w->cols);
     switch (w->type) {
-        case FHIP_Q4_K: return launch_fmt<Q4K>(w, d_x, t, d_y, s, d_ws, ws_bytes);
-        case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_x, t, d_y, s, d_ws, ws_bytes);
-        case FHIP_Q8_0: return launch_fmt<Q80>(w, d_x, t, d_y, s, d_ws, ws_bytes);
-        case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_x, t, d_y, s, d_ws, ws_bytes);
+        case FHIP_Q4_K: return gemm_Q4K_launch(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
+        case FHIP_Q6_K: return gemm_Q6K_launch(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
+        case FHIP_Q8_0: return gemm_Q80_launch(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
+        case FHIP_Q5_K: return gemm_Q5K_launch(w, d_x, t, d_y, s, d_ws, ws_bytes, run_sums);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "QMatrix: no native matmul for ggml type %u", w->type);
     }
+}
+
+size_t gemm_bf16_ws_bytes(const fhip_weight* w, size_t t) { return gemm_bf16_ws_bytes(w, t, false); }
+int launch_gemm_bf16(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes) {
+    return launch_gemm_bf16(w, d_x, t, d_y, s, d_ws, ws_bytes, false);
 }
 
 // H [t, rows / 2] = bf16(silu(gate) * up) of the stacked [gate | up] weight, for more than 32 rows (fewer: launch_gemm_bf16 and
@@ -1312,10 +1780,10 @@ size_t gemm_bf16_swiglu_ws_bytes(const fhip_weight* w, size_t t) {
     if (!w || t <= 32 || w->rows == 0 || w->rows % 2 != 0) return 0;
     const size_t columns = swiglu_columns(w->rows / 2);
     switch (w->type) {
-        case FHIP_Q4_K: return ws_bytes_fmt<Q4K>(w, columns, t);
-        case FHIP_Q6_K: return ws_bytes_fmt<Q6K>(w, columns, t);
-        case FHIP_Q8_0: return ws_bytes_fmt<Q80>(w, columns, t);
-        case FHIP_Q5_K: return ws_bytes_fmt<Q5K>(w, columns, t);
+        case FHIP_Q4_K: return gemm_Q4K_ws_bytes(w, columns, t, false);
+        case FHIP_Q6_K: return gemm_Q6K_ws_bytes(w, columns, t, false);
+        case FHIP_Q8_0: return gemm_Q80_ws_bytes(w, columns, t, false);
+        case FHIP_Q5_K: return gemm_Q5K_ws_bytes(w, columns, t, false);
         default: return 0;
     }
 }
@@ -1325,12 +1793,13 @@ int launch_gemm_bf16_swiglu(const fhip_weight* w, const uint16_t* d_x, size_t t,
     if ((unsigned long long)t * w->cols >= (1ull << 31))
         return set_error(FHIP_ERR_SHAPE, "gemm_q_bf16: t * cols must be below 2^31 (got %zu x %zu)", t, w->cols);
     switch (w->type) {
-        case FHIP_Q4_K: return launch_tiled<Q4K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
-        case FHIP_Q6_K: return launch_tiled<Q6K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
-        case FHIP_Q8_0: return launch_tiled<Q80, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
-        case FHIP_Q5_K: return launch_tiled<Q5K, true>(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q4_K: return gemm_Q4K_launch_swiglu(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q6_K: return gemm_Q6K_launch_swiglu(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q8_0: return gemm_Q80_launch_swiglu(w, d_x, t, d_h, s, d_ws, ws_bytes);
+        case FHIP_Q5_K: return gemm_Q5K_launch_swiglu(w, d_x, t, d_h, s, d_ws, ws_bytes);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "QMatrix: no native matmul for ggml type %u", w->type);
     }
 }
 
 }  // namespace fhip
+#endif

@@ -372,8 +372,8 @@ class Qwen3Decoder:
         att = E((t, self.q_out), np.float32 if self.gate is not None else rows)
         o, x1, y = E((t, c.d_model)), E((t, c.d_model)), E((t, c.d_model))
         normed = E((t, c.d_model)) if self.on is not None else None                   # a post-normed branch output
-        # On a quantized cache gate|up is formed apart from SwiGLU: a code follows every rounding in front of it, and a sum that the fused launch
-        # cuts elsewhere along K would move a tenth of the codes that later layers store. An f32 cache has no codes: there the fused launch
+        # On a quantized cache the products are added in an order that stays (fhip_gemm_q_bf16_run_sums) and gate|up is formed apart from SwiGLU: a
+        # code follows every rounding in front of it, and a sum cut elsewhere along K would move a tenth to two fifths of the codes that later layers store. An f32 cache has no codes: there the fused launch
         # takes part, as exact against f64 as the two launches and up to 1.7e-3 of the norm away from them after four layers.
         f, gu = E((t, c.n_ff)), (E((t, 2 * c.n_ff)) if c.geglu or (self.kv_fmt is not None and not precise) else None)
         gate = E((t, self.q_out)) if self.gate is not None else None
@@ -387,6 +387,10 @@ class Qwen3Decoder:
         def matmul(w, a, out):
             if precise:
                 _check(lib.fhip_matmul_q(w.handle, a.buf.ptr, t, out.buf.ptr, s))
+            elif self.kv_fmt is not None:
+                if a.dtype != np.uint16:
+                    _check(lib.fhip_cvt_f32_bf16(a.buf.ptr, t * w.cols(), ws16.ptr, s))
+                _check(lib.fhip_gemm_q_bf16_run_sums(w.handle, a.buf.ptr if a.dtype == np.uint16 else ws16.ptr, t, out.buf.ptr, s))
             elif a.dtype == np.uint16:
                 _check(lib.fhip_gemm_q_bf16(w.handle, a.buf.ptr, t, out.buf.ptr, s))
             else:
@@ -412,8 +416,8 @@ class Qwen3Decoder:
                 need = lib.fhip_ffn_coop_ws_bytes(l.ffn_gate_up.handle, l.ffn_down.handle, t)
                 if wsf[0] is None or wsf[0].nbytes < need:
                     wsf[0] = DeviceBuffer(max(need, 256))
-                _check(lib.fhip_ffn_bf16(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, gu.buf.ptr if gu is not None else None, t, out.buf.ptr,
-                                         wsf[0].ptr, s))
+                block = lib.fhip_ffn_bf16 if gu is None else lib.fhip_ffn_bf16_run_sums
+                _check(block(l.ffn_gate_up.handle, l.ffn_down.handle, a.buf.ptr, gu.buf.ptr if gu is not None else None, t, out.buf.ptr, wsf[0].ptr, s))
 
         pending = None                                   # the previous layer's FFN branch: joins the residual in the next norm's launch
         for l, kv in zip(self.layers, self.caches):

@@ -225,6 +225,9 @@ int fhip_ffn(const fhip_weight* gate_up, const fhip_weight* down, const float* d
  * output tiles along K keeps their partial tiles in the library's workspace of the stream (fhip_workspace_bytes_coop)
  * and adds them in a fixed order: the same inputs give the same bits on every run. */
 int fhip_gemm_q_bf16(const fhip_weight* w, const uint16_t* d_x_bf16, size_t t, float* d_y, void* stream);
+/* The same with every output's products added in an order that stays from version to version: for rows whose last bits are stored further on, as
+ * the codes of a block-quantized cache. Up to 32 rows the same bits; above, last bits may differ from fhip_gemm_q_bf16's, which adds in the order that is fastest. */
+int fhip_gemm_q_bf16_run_sums(const fhip_weight* w, const uint16_t* d_x_bf16, size_t t, float* d_y, void* stream);
 
 /* ---- mixture-of-experts decode: the "_id" variants that sit behind the same matmul entry points ---------- */
 
@@ -468,7 +471,8 @@ int fhip_batch_policy(int policy);
  * e.g. before a graph capture, during which it cannot grow. A buffer that was outgrown stays allocated until the release,
  * because a graph captured earlier may still name it. No counterpart in the reference (wgpu allocates per dispatch).
  * fhip_workspace_bytes_coop: the same for the matrix-core entry points fhip_gemm_q_bf16, fhip_matmul_q_coop (down NULL) and
- * fhip_ffn_coop, which keep there the partial tiles of a launch that cuts output tiles along K (0 when no tile is cut). */
+ * fhip_ffn_coop, which keep there the partial tiles of a launch that cuts output tiles along K: what calls of up to rows_x rows need at most
+ * (fewer rows may need more; 0 when no such call cuts a tile). */
 size_t fhip_workspace_bytes(const fhip_weight* w, const fhip_weight* down, size_t rows_x);
 size_t fhip_workspace_bytes_coop(const fhip_weight* w, const fhip_weight* down, size_t rows_x);
 int fhip_workspace_reserve(void* stream, size_t nbytes);
@@ -517,6 +521,9 @@ int fhip_ffn_coop(const fhip_weight* gate_up, const fhip_weight* down, const flo
  * the rounding to bf16. */
 int fhip_ffn_bf16(const fhip_weight* gate_up, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
                   void* stream);
+/* With gate|up in memory (d_gate_up is not NULL) and both products as fhip_gemm_q_bf16_run_sums makes them. */
+int fhip_ffn_bf16_run_sums(const fhip_weight* gate_up, const fhip_weight* down, const uint16_t* d_x_bf16, float* d_gate_up, size_t rows_x, float* d_y, void* d_ws,
+                           void* stream);
 
 /* crates/ferric-tensor/src/dtype.rs:935-944 Tensor::matmul_q for 1..32 activation rows in ONE pass over the weights
  * with f32-grade results (the reference's kernels, :2995-3051 and :3423-3469, walk the weight row once per activation

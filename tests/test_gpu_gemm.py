@@ -77,6 +77,43 @@ def test_every_tile_on_ragged_shapes(F, O, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
+@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11])
+def test_tiles_whose_waves_unpack_for_themselves(F, O, tile):
+    # 64 / 128 rows x 64 ... 256 outputs: one, two and three chunks of K a run (the pipeline is two deep), an odd chunk count, a run that
+    # starts in one tile and ends in the next, rows and outputs that end inside a tile, a Q8_0 row that ends inside a chunk, every format,
+    # and SwiGLU in the launch; the same bits again on a second run.
+    lib = F._lib.load()
+    before = lib.fhip_debug_gemm_tile(tile)
+    try:
+        shapes = [(Q4_K, 33, 65, 256), (Q5_K, 129, 193, 512), (Q6_K, 64, 321, 768), (Q8_0, 127, 100, 1312), (Q6_K, 200, 5000, 1280), (Q4_K, 321, 4100, 1792), (Q5_K, 65, 9000, 2304),
+                  (Q8_0, 130, 2049, 2080)]
+        for i, (ty, t, n, k) in enumerate(shapes):
+            y = run_case(F, O, ty, t, n, k, 500 + 10 * tile + i)
+            assert np.array_equal(y.view(np.uint32), run_case(F, O, ty, t, n, k, 500 + 10 * tile + i).view(np.uint32)), (tile, ty)
+    finally:
+        lib.fhip_debug_gemm_tile(before)
+
+
+@pytest.mark.parametrize("ty", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_run_sums_add_in_the_order_of_one_accumulator(F, ty):
+    # fhip_gemm_q_bf16_run_sums: the tiles whose waves unpack for themselves, one wave along K, have the bits of the tiles that share the
+    # unpacking, one matrix instruction's sum after the other. One chunk of K, which no tile cuts: 256 x 256 pinned against the tile of 64 or
+    # 128 rows that run sums take. Up to 32 rows both entry points are one launch.
+    from ferric_amd.synth import synth_weights
+    lib, k = F._lib.load(), 256
+    for t, n in ((60, 3000), (60, 20000), (120, 3000), (250, 30000), (20, 700)):
+        qm = F.QMatrix.from_bytes(synth_weights(ty, n, k, 77), ty, n, k)
+        xb, _ = bf16_round(np.random.default_rng(78).standard_normal((t, k)).astype(np.float32))
+        x, y = F.Tensor.from_bf16_bits(xb, (t, k)), F.Tensor.empty((t, n))
+        F._lib.check(lib.fhip_gemm_q_bf16_run_sums(qm.handle, x.buf.ptr, t, y.buf.ptr, None))
+        before = lib.fhip_debug_gemm_tile(2)
+        try:
+            want = x.gemm_q_bf16(qm).to_vec()
+        finally:
+            lib.fhip_debug_gemm_tile(before)
+        assert np.array_equal(y.to_vec().view(np.uint32), want.view(np.uint32)), (ty, t)
+
+
 def test_reference_coop_example_shapes(F, O):
     # crates/ferric-tensor/examples/coop_q4_k.rs: reference-generator weights, M a multiple of 8 and not
     run_case(F, O, Q4_K, 16, 64, 512, 3, gen=O.gen_kquant_matrix)
