@@ -1042,7 +1042,7 @@ int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, 
     if (rc) return rc;
     if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
     if ((rc = check_causal("fhip_causal_attention", d_q, d_k, d_v, d_out, n_head, n_kv))) return rc;
-    return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, d_out, (hipStream_t)stream);
+    return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, d_out, nullptr, 0, (hipStream_t)stream);
 }
 
 int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
@@ -1051,7 +1051,7 @@ int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* 
     if (rc) return rc;
     if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
     if ((rc = check_causal("fhip_causal_attention_bf16", d_q, d_k, d_v, d_out_bf16, n_head, n_kv))) return rc;
-    return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, d_out_bf16, (hipStream_t)stream);
+    return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, d_out_bf16, nullptr, 0, (hipStream_t)stream);
 }
 
 int fhip_causal_attention_f32_products(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
@@ -1061,8 +1061,26 @@ int fhip_causal_attention_f32_products(const float* d_q, const float* d_k, const
     if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
     if ((rc = check_causal("fhip_causal_attention_f32_products", d_q, d_k, d_v, d_out, n_head, n_kv))) return rc;
     if (out_bf16)
-        return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, false, (uint16_t*)d_out, (hipStream_t)stream);
-    return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, false, (float*)d_out, (hipStream_t)stream);
+        return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, false, (uint16_t*)d_out, nullptr, 0,
+                                                  (hipStream_t)stream);
+    return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, false, (float*)d_out, nullptr, 0, (hipStream_t)stream);
+}
+
+size_t fhip_causal_attention_ws_bytes(size_t t, size_t s, size_t n_head, size_t head_dim, size_t window) {
+    return g_device < 0 || (head_dim != 64 && head_dim != 128) ? 0 : fhip::causal_attention_ws_bytes(t, s, n_head, head_dim, window);
+}
+
+int fhip_causal_attention_split(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
+                                size_t window, float softcap, int out_bf16, void* d_out, float* d_ws, size_t ws_bytes, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (t == 0 || n_head == 0 || head_dim == 0) return FHIP_OK;
+    if ((rc = check_causal("fhip_causal_attention_split", d_q, d_k, d_v, d_out, n_head, n_kv))) return rc;
+    if (((uintptr_t)d_ws & 15) != 0) return set_error(FHIP_ERR_ARG, "fhip_causal_attention_split: pointers must be 16-byte aligned");
+    if (out_bf16)
+        return fhip::launch_causal_attention_bf16(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, (uint16_t*)d_out, d_ws, ws_bytes,
+                                                  (hipStream_t)stream);
+    return fhip::launch_causal_attention(d_q, d_k, d_v, t, s, (int)n_head, (int)n_kv, (int)head_dim, window, softcap, true, (float*)d_out, d_ws, ws_bytes, (hipStream_t)stream);
 }
 
 size_t fhip_decode_attention_ws_bytes(size_t n_head, size_t n_kv, size_t head_dim, size_t len) {

@@ -181,7 +181,8 @@ int launch_qkv_post_attention_kvq(int fmt, const float* qkv, const float* bias, 
 int launch_kvq_dequantize(int fmt, const uint32_t* codes, const uint16_t* scales, size_t row0, size_t rows, size_t width, const uint32_t* d_last_pos,
                           float* out, hipStream_t s);
 int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                            float softcap, bool cuts, float* out, hipStream_t st);
+                            float softcap, bool cuts, float* out, float* ws, size_t ws_bytes, hipStream_t st);
+size_t causal_attention_ws_bytes(size_t t, size_t s, size_t n_head, size_t hd, size_t window);   // 0: these keys are not split
 int launch_mul_sigmoid(const float* a, const float* g, size_t n, float* out, hipStream_t s);   // out = a * sigmoid(g); out may be a
 int launch_geglu(const float* gu, size_t t, size_t d, float* out, hipStream_t s);              // rows [gate | up] -> gelu_tanh(gate) * up
 int launch_rope(const float* x, size_t src_row_stride, size_t t, int heads, int hd, int n_rot, float base, const uint32_t* d_pos, uint32_t pos_off,

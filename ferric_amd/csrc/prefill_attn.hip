@@ -14,7 +14,9 @@
 // 274, 512 x 8192 1163 -> 789; few workgroups: 39 x 929, 8 heads 85.7 -> 70.3; heads of 64: 512 x 512, 32 heads 31.7 -> 27.7, 49 x 49 7.0 ->
 // 6.8. Relative error against f64, same shapes: 5.6e-7 -> 4.5e-7, 4.5e-7 -> 3.7e-7, 1.65e-6 -> 1.41e-6, 6.8e-7 -> 5.6e-7, 2.7e-7 -> 2.0e-7,
 // 1.7e-7 -> 1.2e-7. What bounds the cut kernel: the chain of a tile (cut and store 32 keys, products, statistics, products: 2.2 us a wave
-// alone on its SIMD, of which 0.65 are MFMA) at one or two waves a SIMD.
+// alone on its SIMD, of which 0.65 are MFMA) at one or two waves a SIMD, one tile after the other. So where the query blocks leave CUs idle, or one
+// with two blocks working last, their keys are split between workgroups, whose sums a second launch joins (fhip_causal_attention_split): 509 x 809 rows 71.9 -> 56.8, 95 x 722, 8
+// heads 54.4 -> 14.2 (causal_split). Error against f64 with ranges: no larger, sums are shorter.
 //
 // Why f32 matrix instructions (the second kernel, and the first one's tiling). v_mfma_f32_16x16x4_f32 multiplies f32 operands exactly and accumulates in f32: results have the
 // grade of the reference's f32 arithmetic (the tests hold them to 1e-5 of the largest output against an f64 evaluation), where
@@ -42,6 +44,7 @@
 #include "common.hpp"
 #include "prompt.hpp"
 
+#include <limits.h>
 #include <math.h>
 
 namespace {
@@ -274,10 +277,40 @@ __device__ __forceinline__ void mfma_cuts(const bf16x8 (&a)[N][3], const bf16x8 
 
 constexpr float V_UP = 0x1p40f;
 
-template <int HD, int NW, typename Out>
+// the largest magnitude of a lane's sums and of `top`; a NaN stays
+template <int ND>
+__device__ __forceinline__ float largest(float top, const f32x4 (&acc)[ND]) {
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) top = __builtin_elementwise_maximum(top, fabsf(acc[d][r]));
+    return top;
+}
+
+// The key tiles kt_lo .. kt_hi that the query rows wg_first .. wg_last see, in n ranges of per (the last one's may be fewer; none is empty, since (n - 1) per <=
+// (n - 1) * most < the count).
+struct KeyRanges { int kt_lo, kt_hi, n, per; };
+__host__ __device__ inline KeyRanges key_ranges(int off, int wg_first, int wg_last, int window, int most) {
+    KeyRanges k;
+    k.kt_hi = (off + wg_last) / 32;
+    const int first = off + wg_first - window + 1;
+    k.kt_lo = window > 0 && first > 0 ? first / 32 : 0;
+    const int count = k.kt_hi - k.kt_lo + 1;
+    k.n = (count + most - 1) / most;
+    k.per = (count + k.n - 1) / k.n;
+    return k;
+}
+// What a wave hands over of its 16 rows and one range of keys: [HD / 16][64] accumulators as its lanes hold them, [16] largest scores (NaN: these rows are
+// the f32 body's), [16] sums of weights.
+constexpr int part_floats(int hd) { return 16 * hd + 32; }
+constexpr int CUT_WAVES = 4;                // of a workgroup whose keys are split
+
+// SPLIT: blockIdx.z is a range of keys of at most `most` tiles, and the workgroup leaves what it has of them in `part`, [head][16 rows][ranges] slots, for
+// causal_attn_join_kernel.
+template <int HD, int NW, bool SPLIT, typename Out>
 __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
                                                                      int S, int n_head, int n_kv, float scale, int window, float softcap,
-                                                                     Out* __restrict__ out) {
+                                                                     Out* __restrict__ out, float* __restrict__ part, int most) {
     constexpr int KROW = HD + 8;            // bf16 per K row and plane
     constexpr int VROW = 32 + 8;            // bf16 per V dim and plane
     constexpr int KP = 32 * KROW, VP = HD * VROW;   // bf16 per plane
@@ -297,8 +330,10 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
     const bool wave_live = i0 < T;
     const int i_last = min(i0 + 15, T - 1);
     const int i = min(i0 + c, T - 1), qpos = off + i;
-    const int kt_hi = (off + wg_last) / 32;
-    const int kt_lo = window > 0 ? max(0, off + wg_first - window + 1) / 32 : 0;
+    const KeyRanges kr = key_ranges(off, wg_first, wg_last, window, SPLIT ? most : INT_MAX);
+    if (SPLIT && (int)blockIdx.z >= kr.n) return;
+    const int kt_lo = SPLIT ? kr.kt_lo + (int)blockIdx.z * kr.per : kr.kt_lo;
+    const int kt_hi = SPLIT ? min(kr.kt_hi, kt_lo + kr.per - 1) : kr.kt_hi;
     const int my_hi = wave_live ? (off + i_last) / 32 : -1;
     const int my_lo = window > 0 ? max(0, off + i0 - window + 1) / 32 : 0;
 
@@ -434,11 +469,17 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     if (!wave_live) return;
-    float top = l > 0.f ? l : INFINITY;
+    if constexpr (SPLIT) {
+        if (my_hi < kt_lo || my_lo > kt_hi) return;             // the join does not ask for it
+        const bool bad = !(largest<ND>(l, oacc) < INFINITY);    // rows that see none of these keys have l = 0 and a weight of 0 below
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) m = NAN;
+        float* slot = part + (((size_t)head * ((T + 15) / 16) + i0 / 16) * gridDim.z + blockIdx.z) * part_floats(HD);
 #pragma unroll
-    for (int d = 0; d < ND; d++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) top = __builtin_elementwise_maximum(top, fabsf(oacc[d][r]));    // a NaN stays
+        for (int d = 0; d < ND; d++) *(f32x4*)(slot + (64 * d + lane) * 4) = oacc[d];
+        if (ks == 0) { slot[16 * HD + c] = m; slot[16 * HD + 16 + c] = l; }
+        return;
+    }
+    const float top = largest<ND>(l > 0.f ? l : INFINITY, oacc);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(top < INFINITY)) != 0, 0)) {
         f32_body<HD, NW, false>(nullptr, nullptr, q, K, V, T, S, n_head, n_kv, scale, window, softcap, out);
         return;
@@ -450,45 +491,169 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
     for (int d = 0; d < ND; d++) store_out(op + 16 * d, float4{oacc[d][0] * inv, oacc[d][1] * inv, oacc[d][2] * inv, oacc[d][3] * inv});
 }
 
+// The ranges of keys of 16 rows of a head, a wave: sum_j exp(m_j - max m) (acc_j, l_j) in the ranges' order. A wave that finds what the cuts do not carry, in a
+// range or in the sum over them, does its rows on the f32 body, as it would have done without ranges.
+template <int HD, typename Out>
+__global__ __launch_bounds__(64) void causal_attn_join_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T, int S,
+                                                              int n_head, int n_kv, float scale, int window, float softcap, Out* __restrict__ out,
+                                                              const float* __restrict__ part, int most, int slots) {
+    constexpr int ND = HD / 16;
+    const int lane = threadIdx.x, c = lane & 15, ks = lane >> 4;
+    const int head = blockIdx.x, tile = (int)gridDim.y - 1 - (int)blockIdx.y, i0 = 16 * tile, off = S - T;   // the f32 body numbers its rows the same way
+    const int wg_first = i0 / (16 * CUT_WAVES) * (16 * CUT_WAVES), wg_last = min(T - 1, wg_first + 16 * CUT_WAVES - 1);
+    const KeyRanges kr = key_ranges(off, wg_first, wg_last, window, most);
+    const int my_hi = (off + min(i0 + 15, T - 1)) / 32, my_lo = window > 0 ? max(0, off + i0 - window + 1) / 32 : 0;
+    const int j_lo = (my_lo - kr.kt_lo) / kr.per, j_hi = (my_hi - kr.kt_lo) / kr.per;
+    const float* slot = part + ((size_t)head * gridDim.y + tile) * slots * part_floats(HD);
+    float m = -3.0e38f;
+    bool bad = false;
+#pragma unroll 4
+    for (int j = j_lo; j <= j_hi; j++) {
+        const float mj = slot[(size_t)j * part_floats(HD) + 16 * HD + c];
+        bad |= mj != mj;
+        m = fmaxf(m, mj);
+    }
+    f32x4 acc[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll 2
+    for (int j = j_lo; j <= j_hi; j++) {
+        const float* p = slot + (size_t)j * part_floats(HD);
+        const float w = __expf(p[16 * HD + c] - m);
+        l = fmaf(w, p[16 * HD + 16 + c], l);
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            const f32x4 o = *(const f32x4*)(p + (64 * d + lane) * 4);
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[d][r] = fmaf(w, o[r], acc[d][r]);
+        }
+    }
+    const float top = largest<ND>(l > 0.f ? l : INFINITY, acc);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad || !(top < INFINITY)) != 0, 0)) {
+        f32_body<HD, 1, false>(nullptr, nullptr, q, K, V, T, S, n_head, n_kv, scale, window, softcap, out);
+        return;
+    }
+    if (i0 + c >= T) return;
+    const float inv = 1.0f / l * (1.0f / V_UP);
+    Out* op = out + ((size_t)(i0 + c) * n_head + head) * HD + 4 * ks;
+#pragma unroll
+    for (int d = 0; d < ND; d++) store_out(op + 16 * d, float4{acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv});
+}
+
 }  // namespace
 
 namespace fhip {
 
+static int waves_of(size_t t, size_t n_head) {
+    // waves (16 query rows each) per workgroup: 8, or 4 while that leaves the chip fewer than two workgroups per CU
+    const size_t cus = device_cus() > 0 ? device_cus() : 256;
+    return ((t + 127) / 128) * n_head < 2 * cus ? 4 : 8;
+}
+
+// Ranges of at most `most` key tiles, at most `slots` of them a query block; most = 0: the keys stay in one piece.
+// A workgroup takes 2.15 us a tile of 64 rows at head size 128 and 1.3 at 64, and a CU's workgroups together 1.95 and 1.0, so a launch of one workgroup a CU or fewer
+// lasts as long as the block with the most tiles, one of up to two a CU as long as that block and the shortest that lies beside it. Ranges cost 4 us (the
+// join's launch) and a seventh (their starts, the partial results' way through memory) and level the CUs' shares. The best size is 0.6 of a CU's share, two at least; it is flat around
+// that and from 14 on, where the share, not the last workgroup, counts. us, one piece | ranges of 2, 3, 4, 6, 8, 14, 18 tiles (rows x keys, heads, KV heads, head size):
+//   95 x 722, 8, 8, 128     54.4 | 14.2  15.4  16.8  20.7  25.3  32.2        377 x 954, 8, 4, 64     46.0 | 16.3  15.1  16.0  15.5  17.7  26.0  27.5
+//   33 x 1057, 4, 4, 128    78.1 | 16.5  16.7  17.9  21.3  23.2  33.5  44.0  152 x 940, 8, 8, 64     44.9 | 13.5  12.4  12.9  14.7  17.5  25.8  27.0
+//   234 x 355, 32, 4, 128   31.4 | 24.6  21.0  21.9  22.1  26.3              65 x 600, 64, 8, 64     31.5 | 19.6  18.4  17.9  17.2  18.5  20.6  20.7
+//   1024 x 1024, 8, 4, 128  77.4 | 40.6  36.5  35.4  30.1  35.1  41.9  48.4  700 x 1200, 24, 8, 64   59.4 | 52.7  43.7  41.6  39.0  38.9  39.3  44.2
+//   509 x 809, 40, 8, 128   71.9 | 82.3  68.8  63.5  63.0  58.8  59.8  56.8  1024 x 2048, 16, 4, 64  94.5 | 80.2  67.1  62.1  59.4  58.2  55.7  59.0
+// and not split: 77 x 77, 40 heads of 128 7.2 | 8.9  9.5, 205 x 205, 64 of 64 12.6 | 13.6  13.6  13.3  15.3, 1024 x 1024, 40 of 128 (640 workgroups) 85.6 | 139  119  110  101  97.8  95.6  97.6.
+struct CausalSplit { int most = 0, slots = 0; };
+static CausalSplit causal_split(size_t t, size_t s, size_t n_head, size_t hd, int win) {
+    constexpr size_t ROWS = 16 * CUT_WAVES;
+    constexpr int FEWEST = 5, RANGES = 32;       // tiles that are worth a join; what the join adds one after the other
+    if (t == 0 || n_head == 0 || n_head > 65535 || s < t || s > 0x3FFFFFFFull || waves_of(t, n_head) != CUT_WAVES) return {};
+    const size_t cus = device_cus() > 0 ? device_cus() : 256, blocks = (t + ROWS - 1) / ROWS, groups = blocks * n_head;
+    if (groups > 2 * cus) return {};
+    const int off = (int)(s - t);
+    auto tiles = [&](size_t b) {
+        const KeyRanges k = key_ranges(off, (int)(b * ROWS), (int)((b + 1) * ROWS < t ? (b + 1) * ROWS : t) - 1, win, INT_MAX);
+        return k.kt_hi - k.kt_lo + 1;
+    };
+    size_t total = 0;
+    int longest = 0;
+    for (size_t b = 0; b < blocks; b++) {
+        const int n = tiles(b);
+        total += n * n_head;
+        longest = n > longest ? n : longest;
+    }
+    if (longest < FEWEST) return {};
+    const float one = hd == 128 ? 2.15f : 1.3f, both = hd == 128 ? 1.95f : 1.0f, share = (float)total / cus;
+    int most = share <= 24.f ? (int)ceilf(0.6f * share) : (int)fmaxf(14.f, share / 4);
+    most = most < 2 ? 2 : most;
+    most = most * RANGES < longest ? (longest + RANGES - 1) / RANGES : most;
+    for (int m = most; m <= most + most / 4; m++) {      // a little longer where all of them then start at once (509 x 809: 15 tiles 62.5, 18 57)
+        size_t units = 0;
+        for (size_t b = 0; b < blocks; b++) units += (tiles(b) + m - 1) / m * n_head;
+        if (units <= 2 * cus) { most = m; break; }
+    }
+    const float whole = groups <= cus ? one * longest : both * (longest + tiles(blocks - 1 - cus / n_head));   // blocks go out last first, all heads of each
+    if (whole <= 4.f + fmaxf(one * (most < longest ? most : longest), 1.15f * both * share)) return {};
+    return {most, (longest + most - 1) / most};
+}
+
+static int causal_window(size_t window, size_t s) { return window == 0 || window >= s ? 0 : (int)window; }   // a window that covers the cache is no window
+
+static size_t split_bytes(const CausalSplit& sp, size_t t, size_t n_head, size_t hd) {
+    return n_head * ((t + 15) / 16) * sp.slots * part_floats((int)hd) * sizeof(float);
+}
+
+size_t causal_attention_ws_bytes(size_t t, size_t s, size_t n_head, size_t hd, size_t window) {
+    return split_bytes(causal_split(t, s, n_head, hd, causal_window(window, s)), t, n_head, hd);
+}
+
 template <typename Out>
 static int launch_causal_out(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                             float softcap, bool cuts, Out* out, hipStream_t st) {
+                             float softcap, bool cuts, Out* out, float* ws, size_t ws_bytes, hipStream_t st) {
     if (t == 0 || n_head == 0 || hd == 0) return FHIP_OK;
     if (s < t) return set_error(FHIP_ERR_SHAPE, "cache (%zu) cannot be shorter than the query block (%zu)", s, t);   // nn.rs:73, :249
     if (n_kv <= 0 || n_head % n_kv != 0) return set_error(FHIP_ERR_SHAPE, "causal_attention: n_heads must be a multiple of n_kv_heads");
     if (hd != 64 && hd != 128) return set_error(FHIP_ERR_SHAPE, "causal_attention: head_dim must be 64 or 128");
     if (s > 0x3FFFFFFFull || n_head > 65535) return set_error(FHIP_ERR_SHAPE, "causal_attention: too large for one launch");
-    // waves (16 query rows each) per workgroup: 8, or 4 while that leaves the chip fewer than two workgroups per CU
-    const int cus = device_cus() > 0 ? device_cus() : 256;
-    int nw = 8;
-    if (((t + 127) / 128) * (size_t)n_head < 2 * (size_t)cus) nw = 4;
+    const int nw = waves_of(t, n_head);
     const size_t qblocks = (t + (size_t)nw * 16 - 1) / ((size_t)nw * 16);
     if (qblocks > 65535) return set_error(FHIP_ERR_SHAPE, "causal_attention: too many query rows for one launch");
-    const dim3 grid((unsigned)n_head, (unsigned)qblocks), wg(64 * nw);
+    dim3 grid((unsigned)n_head, (unsigned)qblocks);
+    const dim3 wg(64 * nw);
     const float scale = 1.0f / sqrtf((float)hd);
-    const int win = window == 0 || window >= s ? 0 : (int)window;     // a window that covers the cache is no window
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out); };
-    if (cuts) {
-        if (hd == 128) nw == 8 ? go(causal_attn_cut_kernel<128, 8, Out>) : go(causal_attn_cut_kernel<128, 4, Out>);
-        else nw == 8 ? go(causal_attn_cut_kernel<64, 8, Out>) : go(causal_attn_cut_kernel<64, 4, Out>);
-    } else {
-        if (hd == 128) nw == 8 ? go(causal_attn_kernel<128, 8, Out>) : go(causal_attn_kernel<128, 4, Out>);
-        else nw == 8 ? go(causal_attn_kernel<64, 8, Out>) : go(causal_attn_kernel<64, 4, Out>);
+    const int win = causal_window(window, s);
+    auto cut = [&](auto kernel, auto to, int most) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, to, ws, most); };
+    auto f32 = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out); };
+    if (!cuts) {
+        if (hd == 128) nw == 8 ? f32(causal_attn_kernel<128, 8, Out>) : f32(causal_attn_kernel<128, 4, Out>);
+        else nw == 8 ? f32(causal_attn_kernel<64, 8, Out>) : f32(causal_attn_kernel<64, 4, Out>);
+        return check_hip(hipGetLastError(), "causal_attention launch");
     }
+    const CausalSplit sp = ws ? causal_split(t, s, n_head, hd, win) : CausalSplit{};
+    if (sp.most) {
+        const size_t need = split_bytes(sp, t, n_head, hd);
+        if (ws_bytes < need) return set_error(FHIP_ERR_ARG, "causal_attention: %zu bytes of workspace, %zu needed", ws_bytes, need);
+        grid.z = (unsigned)sp.slots;
+        hd == 128 ? cut(causal_attn_cut_kernel<128, CUT_WAVES, true, float>, ws, sp.most) : cut(causal_attn_cut_kernel<64, CUT_WAVES, true, float>, ws, sp.most);
+        if (const int rc = check_hip(hipGetLastError(), "causal_attention launch")) return rc;
+        auto join = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)n_head, (unsigned)((t + 15) / 16)), dim3(64), 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out,
+                               (const float*)ws, sp.most, sp.slots);
+        };
+        hd == 128 ? join(causal_attn_join_kernel<128, Out>) : join(causal_attn_join_kernel<64, Out>);
+        return check_hip(hipGetLastError(), "causal_attention join launch");
+    }
+    if (hd == 128) nw == 8 ? cut(causal_attn_cut_kernel<128, 8, false, Out>, out, 0) : cut(causal_attn_cut_kernel<128, 4, false, Out>, out, 0);
+    else nw == 8 ? cut(causal_attn_cut_kernel<64, 8, false, Out>, out, 0) : cut(causal_attn_cut_kernel<64, 4, false, Out>, out, 0);
     return check_hip(hipGetLastError(), "causal_attention launch");
 }
 
 int launch_causal_attention(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                            float softcap, bool cuts, float* out, hipStream_t st) {
-    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, st);
+                            float softcap, bool cuts, float* out, float* ws, size_t ws_bytes, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, ws, ws_bytes, st);
 }
 int launch_causal_attention_bf16(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                                 float softcap, bool cuts, uint16_t* out, hipStream_t st) {
-    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, st);
+                                 float softcap, bool cuts, uint16_t* out, float* ws, size_t ws_bytes, hipStream_t st) {
+    return launch_causal_out(q, K, V, t, s, n_head, n_kv, hd, window, softcap, cuts, out, ws, ws_bytes, st);
 }
 
 }  // namespace fhip

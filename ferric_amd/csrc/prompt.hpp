@@ -20,6 +20,6 @@ size_t gemm_bf16_ws_bytes(const fhip_weight* w, size_t t, bool run_sums);
 int launch_rmsnorm_bf16(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, uint16_t* norm_out,
                         hipStream_t s);
 int launch_causal_attention_bf16(const float* q, const float* K, const float* V, size_t t, size_t s, int n_head, int n_kv, int hd, size_t window,
-                                 float softcap, bool cuts, uint16_t* out, hipStream_t st);
+                                 float softcap, bool cuts, uint16_t* out, float* ws, size_t ws_bytes, hipStream_t st);
 
 }  // namespace fhip

@@ -383,6 +383,7 @@ class Qwen3Decoder:
             k1, v1 = E((t, self.kv_out)), E((t, self.kv_out))
             kd, vd = E((pos0 + t, self.kv_out)), E((pos0 + t, self.kv_out))          # what the stored blocks dequantize to
         wsf = [None]
+        wsa = f.buf                                      # attention split along the keys: scratch that is not in use yet, or larger
 
         def matmul(w, a, out):
             if precise:
@@ -449,8 +450,14 @@ class Qwen3Decoder:
                 # of f64 rows (22.2 % and 22.3 %, hidden rows 5.42e-3 and 5.43e-3 off). A stored cache keeps its bytes at 30 us a layer (509 x 809 rows).
                 _check(lib.fhip_causal_attention_f32_products(*shape, int(att.dtype != np.float32), att.buf.ptr, s))
             else:
-                attend = lib.fhip_causal_attention if att.dtype == np.float32 else lib.fhip_causal_attention_bf16
-                _check(attend(*shape, att.buf.ptr, s))
+                need = lib.fhip_causal_attention_ws_bytes(t, pos0 + t, c.n_head, c.head_dim, l.window)
+                if wsa.nbytes < need:
+                    wsa = DeviceBuffer(need)
+                if need:
+                    _check(lib.fhip_causal_attention_split(*shape, int(att.dtype != np.float32), att.buf.ptr, wsa.ptr, wsa.nbytes, s))
+                else:
+                    attend = lib.fhip_causal_attention if att.dtype == np.float32 else lib.fhip_causal_attention_bf16
+                    _check(attend(*shape, att.buf.ptr, s))
             if l.attn_gate is not None:
                 matmul(l.attn_gate, h, gate)
                 _check(lib.fhip_mul_sigmoid(att.buf.ptr, gate.buf.ptr, t * self.q_out, att.buf.ptr, s))

@@ -370,6 +370,12 @@ int fhip_causal_attention(const float* d_q, const float* d_k, const float* d_v, 
 /* The same with the output rows as bf16, each value the one fhip_cvt_f32_bf16 makes of the f32 result. */
 int fhip_causal_attention_bf16(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv,
                                size_t head_dim, size_t window, float softcap, uint16_t* d_out_bf16, void* stream);
+/* Both with the keys of a query block split between workgroups where the blocks alone would leave the chip idle (few rows or heads behind many keys), and
+ * joined by a second launch: the same grade, other last bits. d_ws: fhip_causal_attention_ws_bytes(...) bytes of scratch that the call may write until the
+ * stream has passed it. 0 bytes: this shape is not split, d_ws may be null, and the result is the unsplit call's; so it is with a null d_ws. */
+size_t fhip_causal_attention_ws_bytes(size_t t, size_t s, size_t n_head, size_t head_dim, size_t window);
+int fhip_causal_attention_split(const float* d_q, const float* d_k, const float* d_v, size_t t, size_t s, size_t n_head, size_t n_kv, size_t head_dim,
+                                size_t window, float softcap, int out_bf16, void* d_out, float* d_ws, size_t ws_bytes, void* stream);
 /* The same result from the f32 matrix instructions (d_out f32, or bf16 with out_bf16): slower, its error against f64 a fifth larger, other last
  * bits. For stacks on a block-quantized cache, where behind bf16 roundings a last bit decides code bytes of the layers after it: the kernel above
  * would store other codes (13 .. 16 % of them in a fourth layer), which are no nearer to those of f64 rows. */

@@ -199,3 +199,77 @@ def test_small_and_large_values_keep_their_bits(F, X, D, shape, scale):
     for r in (0, t // 2, t - 1):
         want = D.decode_attention(q[r], k[:s - t + r + 1], v[:s - t + r + 1], nh, nkv)[0]
         assert np.abs(cut[r] - want).max() <= 4e-6 * np.abs(want).max() + 2.0 ** -149, (r, np.abs(cut[r] - want).max() / np.abs(want).max())
+
+
+def split(F, q, k, v, nh, nkv, w=0, cap=0.0):
+    """[t, nh * hd] of fhip_causal_attention_split; its bf16 form has to be the rounding of it."""
+    lib, T, t, s, hd = F._lib.load(), (lambda a: F.Tensor.from_vec(a, a.shape)), q.shape[0], k.shape[0], q.shape[1] // nh
+    need = lib.fhip_causal_attention_ws_bytes(t, s, nh, hd, w)
+    assert need, (t, s, nh, hd, w)
+    tq, tk, tv, out, half, ws = T(q), T(k), T(v), T(np.zeros(q.shape, np.float32)), T(np.zeros(q.shape, np.float32)), F.DeviceBuffer(need)
+    args = (tq.buf.ptr, tk.buf.ptr, tv.buf.ptr, t, s, nh, nkv, hd, w, cap)
+    assert lib.fhip_causal_attention_split(*args, 0, out.buf.ptr, ws.ptr, need, None) == 0
+    assert lib.fhip_causal_attention_split(*args, 1, half.buf.ptr, ws.ptr, need, None) == 0
+    got = out.to_vec().reshape(q.shape)
+    b = got.view(np.uint32).astype(np.uint64)
+    rounded = ((b + 0x7FFF + ((b >> 16) & 1)) >> 16).astype(np.uint16)
+    bf16 = half.to_vec().view(np.uint16).reshape(-1)[:got.size].reshape(got.shape)
+    assert np.array_equal(bf16[~np.isnan(got)], rounded[~np.isnan(got)]) and ((bf16[np.isnan(got)] & 0x7FFF) > 0x7F80).all()
+    assert lib.fhip_causal_attention_split(*args, 0, out.buf.ptr, ws.ptr, need - 1, None) != 0        # too little scratch
+    assert lib.fhip_causal_attention_split(*args, 0, out.buf.ptr, None, 0, None) == 0                 # none: the keys in one piece
+    whole = out.to_vec().reshape(q.shape)
+    assert lib.fhip_causal_attention(*args, out.buf.ptr, None) == 0
+    assert np.array_equal(bits(whole), bits(out.to_vec().reshape(q.shape)))
+    return got, whole
+
+
+# one row, ragged rows and tiles, the last range a single tile, 32 ranges, more workgroups than CUs, ranges that the first waves of a block do not see, a window that leaves
+# a block's first keys out, the softcap
+@pytest.mark.parametrize("t,s,nh,nkv,hd,w,cap", [(1, 193, 2, 1, 64, 0, 0.0), (95, 722, 8, 8, 128, 0, 0.0), (33, 1057, 4, 4, 64, 0, 30.0), (17, 2100, 1, 1, 128, 0, 0.0),
+                                                 (509, 809, 40, 8, 128, 0, 0.0), (129, 500, 10, 2, 64, 0, 0.0), (200, 640, 6, 3, 128, 333, 0.0), (160, 160, 8, 1, 128, 0, 50.0)])
+def test_keys_split_between_workgroups(F, X, D, t, s, nh, nkv, hd, w, cap):
+    rng = np.random.default_rng(t + s)
+    q = rng.standard_normal((t, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((s, nkv * hd)).astype(np.float32)
+    v = rng.standard_t(3, (s, nkv * hd)).astype(np.float32)
+    got, whole = split(F, q, k, v, nh, nkv, w, cap)
+    assert np.abs(got - whole).max() <= 4e-6 * np.abs(whole).max()                                    # two f32 sums of up to 2100 terms (2e-6 each at the most)
+    off = s - t
+    for r in sorted({0, min(15, t - 1), min(16, t - 1), t // 2, t - 1}):
+        lo = max(0, off + r + 1 - w) if w else 0
+        want = D.decode_attention(q[r], k[lo:off + r + 1], v[lo:off + r + 1], nh, nkv, 0, cap)[0]
+        assert np.abs(got[r] - want).max() <= 1e-5 * np.abs(want).max(), r
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("kind", ["key nan", "value inf", "sum past the largest", "key -inf"])
+def test_split_keys_that_three_cuts_do_not_carry(F, X, hd, kind):
+    """Rows that meet such a member, in a range or only in the sum over ranges, are the f32 kernel's, bit for bit; other rows keep theirs."""
+    t, s, nh, nkv = 70, 500, 4, 2
+    rng = np.random.default_rng(hd)
+    q, k, v = (rng.standard_normal((n, h * hd)).astype(np.float32) for n, h in ((t, nh), (s, nkv), (s, nkv)))
+    clean, _ = split(F, q, k, v, nh, nkv)
+    j, first = s - 20, t - 20
+    if kind == "key nan":
+        k[j, ::hd] = np.nan
+    elif kind == "value inf":
+        v[j, 5::hd] = -np.inf
+    elif kind == "key -inf":                                          # a row's only infinite score: weight 0
+        q[:, ::hd] = -np.abs(q[:, ::hd]) - 0.1
+        k[j, ::hd] = np.inf
+    else:
+        q[:] = 0                                                      # equal weights: sums of s values of 2^88 * 2^40 pass f32's largest in every range
+        v[:] = np.float32(2.0 ** 88)
+        first = 0
+    got, _ = split(F, q, k, v, nh, nkv)
+    lib, T = F._lib.load(), (lambda a: F.Tensor.from_vec(a, a.shape))
+    tq, tk, tv, out = T(q), T(k), T(v), T(np.zeros(q.shape, np.float32))
+    assert lib.fhip_causal_attention_f32_products(tq.buf.ptr, tk.buf.ptr, tv.buf.ptr, t, s, nh, nkv, hd, 0, 0.0, 0, out.buf.ptr, None) == 0
+    f32 = out.to_vec().reshape(q.shape)
+    same = (bits(got) == bits(f32)) | (np.isnan(got) & np.isnan(f32))
+    assert same[first:].all(), np.argwhere(~same[first:])[:4]
+    if kind in ("key nan", "value inf"):
+        before = first // 16 * 16
+        while before > 0 and (s - t + before - 1) // 32 >= j // 32:
+            before -= 16
+        assert np.array_equal(bits(got[:before]), bits(clean[:before]))
