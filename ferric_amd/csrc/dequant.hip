@@ -9,11 +9,15 @@
 //
 // These kernels are write-bound (4 B out per 0.53-1.06 B in): one lane produces 4 consecutive
 // outputs and stores them as one 16-byte vector, so a wave writes 1 KiB contiguous per store.
-#include "common.hpp"
+#include "hostmem.hpp"
+#include "through.hpp"
 
 #include <hip/hip_fp16.h>
 
 namespace {
+
+using fhip::store_through;
+using fhip::u32x4;
 
 __device__ __forceinline__ float f16_bits(uint32_t b) {
     // v_cvt_f32_f16: exact for every finite / subnormal / infinite pattern.
@@ -38,12 +42,7 @@ __global__ void bf16_to_f32_kernel(const uint16_t* __restrict__ in, size_t n, fl
 }
 
 // ---- Q8_0: 34 B = [f16 d][i8 q[32]] ------------------------------------------------------------
-__global__ void deq_q8_0_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one lane = 4 values
-    if (t >= nquads) return;
-    size_t blk = t >> 3;
-    int j = (int)(t & 7) * 4;
-    const uint8_t* b = raw + blk * 34;
+__device__ __forceinline__ float4 deq_q8_0(const uint8_t* b, int j) {
     float d = f16_bits(*(const uint16_t*)b);
     uint32_t q = ld4_a2(b + 2 + j);
     float4 o;
@@ -51,7 +50,7 @@ __global__ void deq_q8_0_kernel(const uint8_t* __restrict__ raw, size_t nquads, 
     o.y = __fmul_rn((float)(int8_t)((q >> 8) & 0xFF), d);
     o.z = __fmul_rn((float)(int8_t)((q >> 16) & 0xFF), d);
     o.w = __fmul_rn((float)(int8_t)(q >> 24), d);
-    *(float4*)(out + t * 4) = o;
+    return o;
 }
 
 // ---- Q4_K: 144 B = [f16 d][f16 dmin][u8 s[12]][u8 qs[128]] --------------------------------------
@@ -66,13 +65,8 @@ __device__ __forceinline__ void q4k_sc_min(const uint8_t* s, int j, uint32_t& sc
     }
 }
 
-__global__ void deq_q4_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one lane = 4 values, 64 lanes = one block
-    if (t >= nquads) return;
-    size_t blk = t >> 6;
-    int v = (int)(t & 63) * 4;
+__device__ __forceinline__ float4 deq_q4_k(const uint8_t* b, int v) {   // b 16-byte aligned
     int sb = v >> 5, l = v & 31;
-    const uint8_t* b = raw + blk * 144;  // 16-byte aligned
     uint32_t hd = *(const uint32_t*)b;
     float d = f16_bits(hd & 0xFFFFu), dmin = f16_bits(hd >> 16);
     uint32_t sc, m;
@@ -86,17 +80,12 @@ __global__ void deq_q4_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, 
     o.y = __fsub_rn(__fmul_rn(d1, (float)((q >> 8) & 0xFF)), mm);
     o.z = __fsub_rn(__fmul_rn(d1, (float)((q >> 16) & 0xFF)), mm);
     o.w = __fsub_rn(__fmul_rn(d1, (float)(q >> 24)), mm);
-    *(float4*)(out + t * 4) = o;
+    return o;
 }
 
 // ---- Q6_K: 210 B = [u8 ql[128]][u8 qh[64]][i8 sc[16]][f16 d] ------------------------------------
-__global__ void deq_q6_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nquads) return;
-    size_t blk = t >> 6;
-    int v = (int)(t & 63) * 4;
+__device__ __forceinline__ float4 deq_q6_k(const uint8_t* b, int v) {   // b 2-byte aligned
     int hf = v >> 7, w = v & 127, g = w >> 5, l = w & 31, is = l >> 4;
-    const uint8_t* b = raw + blk * 210;  // 2-byte aligned
     float d = f16_bits(*(const uint16_t*)(b + 208));
     float sc = (float)(int8_t)b[192 + 8 * hf + is + 2 * g];
     uint32_t ql = ld4_a2(b + 64 * hf + 32 * (g & 1) + l);
@@ -109,20 +98,15 @@ __global__ void deq_q6_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, 
     o.y = __fmul_rn(ds, (float)((int)((q >> 8) & 0xFF) - 32));
     o.z = __fmul_rn(ds, (float)((int)((q >> 16) & 0xFF) - 32));
     o.w = __fmul_rn(ds, (float)((int)(q >> 24) - 32));
-    *(float4*)(out + t * 4) = o;
+    return o;
 }
 
 // ---- the 32-value formats: [f16 d][f16 m]?[u32 qh]?[u8 qs[16]], blocks 2-byte aligned ----------------------
 // value i < 16 is the low nibble of qs[i], value 16 + i the high one; the fifth bit of value v is bit v of qh.
 //   Q4_0 y = f32(n - 8) * d            lib.rs:618-629      Q4_1 y = f32(n) * d + m            lib.rs:633-645
 //   Q5_0 y = f32((n | b<<4) - 16) * d  lib.rs:650-665      Q5_1 y = f32(n | b<<4) * d + m     lib.rs:669-684
-template <int BYTES, bool HAS_M, bool HAS_QH, int OFF>
-__global__ void deq_legacy_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one lane = 4 values, 8 lanes = one block
-    if (t >= nquads) return;
-    size_t blk = t >> 3;
-    int v = (int)(t & 7) * 4;
-    const uint8_t* b = raw + blk * BYTES;
+template <bool HAS_M, bool HAS_QH, int OFF>
+__device__ __forceinline__ float4 deq_legacy(const uint8_t* b, int v) {
     constexpr int QH = HAS_M ? 4 : 2, QS = QH + (HAS_QH ? 4 : 0);
     float d = f16_bits(*(const uint16_t*)b);
     float m = HAS_M ? f16_bits(*(const uint16_t*)(b + 2)) : 0.f;
@@ -139,17 +123,12 @@ __global__ void deq_legacy_kernel(const uint8_t* __restrict__ raw, size_t nquads
         float f = (float)((int)((q >> (8 * k)) & 0xFF) - OFF);
         o[k] = HAS_M ? __fadd_rn(__fmul_rn(f, d), m) : __fmul_rn(f, d);
     }
-    *(float4*)(out + t * 4) = make_float4(o[0], o[1], o[2], o[3]);
+    return make_float4(o[0], o[1], o[2], o[3]);
 }
 
 // ---- Q5_K: 176 B = [f16 d][f16 dmin][u8 s[12]][u8 qh[32]][u8 qs[128]]; y = (d*sc)*(n + 16*bit) - dmin*m, lib.rs:692-716
-__global__ void deq_q5_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nquads) return;
-    size_t blk = t >> 6;
-    int v = (int)(t & 63) * 4;
+__device__ __forceinline__ float4 deq_q5_k(const uint8_t* b, int v) {   // b 16-byte aligned
     int sb = v >> 5, l = v & 31;
-    const uint8_t* b = raw + blk * 176;  // 16-byte aligned
     uint32_t hd = *(const uint32_t*)b;
     float d = f16_bits(hd & 0xFFFFu), dmin = f16_bits(hd >> 16);
     uint32_t sc, m;
@@ -164,7 +143,7 @@ __global__ void deq_q5_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, 
     o.y = __fsub_rn(__fmul_rn(d1, (float)((q >> 8) & 0xFF)), mm);
     o.z = __fsub_rn(__fmul_rn(d1, (float)((q >> 16) & 0xFF)), mm);
     o.w = __fsub_rn(__fmul_rn(d1, (float)(q >> 24)), mm);
-    *(float4*)(out + t * 4) = o;
+    return o;
 }
 
 // ---- IQ4_NL / IQ4_XS: 4-bit indices into a 16-level non-linear codebook (lib.rs:751), value = scale * level.
@@ -175,25 +154,18 @@ __global__ void deq_q5_k_kernel(const uint8_t* __restrict__ raw, size_t nquads, 
 __device__ const float KV_IQ4NL[16] = {-127.f, -104.f, -83.f, -65.f, -49.f, -35.f, -22.f, -10.f, 1.f, 13.f, 25.f, 38.f, 53.f, 69.f, 89.f, 113.f};
 
 template <bool XS>
-__global__ void deq_iq4_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one lane = 4 values
-    if (t >= nquads) return;
+__device__ __forceinline__ float4 deq_iq4(const uint8_t* b, int v) {
     uint32_t q;
     float dl;
     bool high;
     if (XS) {
-        size_t blk = t >> 6;
-        int v = (int)(t & 63) * 4, ib = v >> 5, l = v & 31;
-        const uint8_t* b = raw + blk * 136;  // 8-byte aligned
+        int ib = v >> 5, l = v & 31;             // b 8-byte aligned
         uint32_t hd = *(const uint32_t*)b, sl = *(const uint32_t*)(b + 4);
         int ls = (int)(((sl >> (4 * ib)) & 0xFu) | ((((hd >> 16) >> (2 * ib)) & 3u) << 4));
         dl = __fmul_rn(f16_bits(hd & 0xFFFFu), (float)(ls - 32));
         q = *(const uint32_t*)(b + 8 + 16 * ib + (l & 15));
         high = l >= 16;
     } else {
-        size_t blk = t >> 3;
-        int v = (int)(t & 7) * 4;
-        const uint8_t* b = raw + blk * 18;
         dl = f16_bits(*(const uint16_t*)b);
         q = ld4_a2(b + 2 + (v & 15));
         high = v >= 16;
@@ -202,7 +174,7 @@ __global__ void deq_iq4_kernel(const uint8_t* __restrict__ raw, size_t nquads, f
     float o[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) o[k] = __fmul_rn(dl, KV_IQ4NL[(q >> (8 * k)) & 0xFu]);
-    *(float4*)(out + t * 4) = make_float4(o[0], o[1], o[2], o[3]);
+    return make_float4(o[0], o[1], o[2], o[3]);
 }
 
 // ---- MXFP4: 17 B = [u8 e][qs[16]]; y = (2 * E2M1[code]) * 2^(e - 128), lib.rs:857-908. The doubled table with the halved
@@ -210,12 +182,7 @@ __global__ void deq_iq4_kernel(const uint8_t* __restrict__ raw, size_t nquads, f
 // One IEEE multiply per value: it rounds only where the result is subnormal or overflows, exactly as the reference's does.
 __device__ const float KV_MXFP4_2X[16] = {0.f, 1.f, 2.f, 3.f, 4.f, 6.f, 8.f, 12.f, 0.f, -1.f, -2.f, -3.f, -4.f, -6.f, -8.f, -12.f};
 
-__global__ void deq_mxfp4_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nquads) return;
-    size_t blk = t >> 3;
-    int v = (int)(t & 7) * 4;
-    const uint8_t* b = raw + blk * 17;  // no alignment at all: byte loads
+__device__ __forceinline__ float4 deq_mxfp4(const uint8_t* b, int v) {   // b has no alignment at all: byte loads
     uint32_t e = b[0];
     float d = __uint_as_float(e == 0 ? (1u << 21) : e == 1 ? (1u << 22) : (e - 1u) << 23);
     const uint8_t* qs = b + 1 + (v & 15);
@@ -223,8 +190,88 @@ __global__ void deq_mxfp4_kernel(const uint8_t* __restrict__ raw, size_t nquads,
     float o[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) o[k] = __fmul_rn(KV_MXFP4_2X[(qs[k] >> sh) & 0xFu], d);
-    *(float4*)(out + t * 4) = make_float4(o[0], o[1], o[2], o[3]);
+    return make_float4(o[0], o[1], o[2], o[3]);
 }
+
+// values v .. v + 3 of the block at b
+template <uint32_t TYPE>
+__device__ __forceinline__ float4 deq4(const uint8_t* b, int v) {
+    if constexpr (TYPE == FHIP_Q8_0) return deq_q8_0(b, v);
+    else if constexpr (TYPE == FHIP_Q4_K) return deq_q4_k(b, v);
+    else if constexpr (TYPE == FHIP_Q5_K) return deq_q5_k(b, v);
+    else if constexpr (TYPE == FHIP_Q6_K) return deq_q6_k(b, v);
+    else if constexpr (TYPE == FHIP_Q4_0) return deq_legacy<false, false, 8>(b, v);
+    else if constexpr (TYPE == FHIP_Q4_1) return deq_legacy<true, false, 0>(b, v);
+    else if constexpr (TYPE == FHIP_Q5_0) return deq_legacy<false, true, 16>(b, v);
+    else if constexpr (TYPE == FHIP_Q5_1) return deq_legacy<true, true, 0>(b, v);
+    else if constexpr (TYPE == FHIP_IQ4_NL) return deq_iq4<false>(b, v);
+    else if constexpr (TYPE == FHIP_IQ4_XS) return deq_iq4<true>(b, v);
+    else return deq_mxfp4(b, v);
+}
+
+template <uint32_t TYPE, int VALS, int BYTES>
+__global__ void deq_kernel(const uint8_t* __restrict__ raw, size_t nquads, float* __restrict__ out) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one lane = 4 values
+    if (t >= nquads) return;
+    *(float4*)(out + t * 4) = deq4<TYPE>(raw + t / (VALS / 4) * BYTES, (int)(t % (VALS / 4)) * 4);
+}
+
+// Blocks in pinned host memory to floats in pinned host memory, a workgroup DEQ_TILE values: its bytes come over the bus in 16-byte pieces, all at
+// once, and are unpacked out of LDS (a load of a narrower piece is a request on the bus of its own); the floats go back as the copy kernels' do, and
+// so does the confirmation. The trip over the bus bounds it: one launch in the place of a copy up, an unpacking and a copy down, of which each
+// waited for the one before. us a call, three launches -> one: 8928 values Q5_0 21.2 -> 15.3, 17056 Q4_0 23.1 -> 16.0, 96192 Q5_1 39.3 -> 30.3; in
+// chunks 1352704 Q5_K 205 -> 187, 4283648 IQ4_XS 472 -> 418, 20971520 Q6_K 2463 -> 2348.
+constexpr int DEQ_TILE = 4096, DEQ_THREADS = 512;
+
+template <uint32_t TYPE, int VALS, int BYTES>
+__global__ __launch_bounds__(DEQ_THREADS) void deq_through_kernel(const uint8_t* __restrict__ raw, uint32_t nblocks, float* __restrict__ out, uint32_t* __restrict__ done, uint32_t seq) {
+    constexpr uint32_t TILE_BLOCKS = DEQ_TILE / VALS, PIECES = TILE_BLOCKS * BYTES / 16;
+    static_assert(TILE_BLOCKS * BYTES % 16 == 0, "a tile's bytes start on a piece");
+    __shared__ u32x4 lds[PIECES];
+    const uint32_t first = blockIdx.x * TILE_BLOCKS, blocks = min(TILE_BLOCKS, nblocks - first);
+    const u32x4* src = (const u32x4*)(raw + (size_t)first * BYTES);
+    for (uint32_t i = threadIdx.x; i < (blocks * BYTES + 15) / 16; i += DEQ_THREADS) lds[i] = src[i];
+    __syncthreads();
+    u32x4* dst = (u32x4*)(out + (size_t)first * VALS);
+    for (uint32_t i = threadIdx.x; i < blocks * (VALS / 4); i += DEQ_THREADS)
+        store_through(dst + i, __builtin_bit_cast(u32x4, deq4<TYPE>((const uint8_t*)lds + i / (VALS / 4) * BYTES, (int)(i % (VALS / 4)) * 4)));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) store_through(done + blockIdx.x, seq);
+}
+
+// go(kernel of the type)
+template <class Go>
+int of_type(uint32_t type, Go go) {
+    switch (type) {
+        case FHIP_Q8_0: go.template operator()<FHIP_Q8_0, 32, 34>(); break;
+        case FHIP_Q4_K: go.template operator()<FHIP_Q4_K, 256, 144>(); break;
+        case FHIP_Q6_K: go.template operator()<FHIP_Q6_K, 256, 210>(); break;
+        case FHIP_Q5_K: go.template operator()<FHIP_Q5_K, 256, 176>(); break;
+        case FHIP_Q4_0: go.template operator()<FHIP_Q4_0, 32, 18>(); break;
+        case FHIP_Q4_1: go.template operator()<FHIP_Q4_1, 32, 20>(); break;
+        case FHIP_Q5_0: go.template operator()<FHIP_Q5_0, 32, 22>(); break;
+        case FHIP_Q5_1: go.template operator()<FHIP_Q5_1, 32, 24>(); break;
+        case FHIP_IQ4_NL: go.template operator()<FHIP_IQ4_NL, 32, 18>(); break;
+        case FHIP_IQ4_XS: go.template operator()<FHIP_IQ4_XS, 256, 136>(); break;
+        case FHIP_MXFP4: go.template operator()<FHIP_MXFP4, 32, 17>(); break;
+        default: return fhip::set_error(FHIP_ERR_UNSUPPORTED_TYPE, "unsupported ggml type %u", type);
+    }
+    return fhip::check_hip(hipGetLastError(), "dequant launch");
+}
+struct ToDevice {
+    const uint8_t* raw; size_t nquads; float* out; hipStream_t s;
+    template <uint32_t TYPE, int VALS, int BYTES> void operator()() const {
+        hipLaunchKernelGGL((deq_kernel<TYPE, VALS, BYTES>), dim3((unsigned)((nquads + 255) / 256)), dim3(256), 0, s, raw, nquads, out);
+    }
+};
+struct ToHost {
+    const uint8_t* raw; uint32_t nblocks; float* out; uint32_t *done, seq; hipStream_t s; int* wgs;
+    template <uint32_t TYPE, int VALS, int BYTES> void operator()() const {
+        *wgs = (int)((nblocks + DEQ_TILE / VALS - 1) / (DEQ_TILE / VALS));
+        hipLaunchKernelGGL((deq_through_kernel<TYPE, VALS, BYTES>), dim3((unsigned)*wgs), dim3(DEQ_THREADS), 0, s, raw, nblocks, out, done, seq);
+    }
+};
 
 }  // namespace
 
@@ -250,21 +297,11 @@ int launch_dequant(uint32_t type, const uint8_t* d_raw, size_t nblocks, float* d
     size_t nquads = nblocks * vals / 4;
     size_t grid = (nquads + 255) / 256;
     if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_ARG, "dequant: %zu blocks exceed one launch", nblocks);
-    switch (type) {
-        case FHIP_Q8_0: hipLaunchKernelGGL(deq_q8_0_kernel, dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q4_K: hipLaunchKernelGGL(deq_q4_k_kernel, dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q6_K: hipLaunchKernelGGL(deq_q6_k_kernel, dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q5_K: hipLaunchKernelGGL(deq_q5_k_kernel, dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q4_0: hipLaunchKernelGGL((deq_legacy_kernel<18, false, false, 8>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q4_1: hipLaunchKernelGGL((deq_legacy_kernel<20, true, false, 0>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q5_0: hipLaunchKernelGGL((deq_legacy_kernel<22, false, true, 16>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_Q5_1: hipLaunchKernelGGL((deq_legacy_kernel<24, true, true, 0>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_IQ4_NL: hipLaunchKernelGGL((deq_iq4_kernel<false>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_IQ4_XS: hipLaunchKernelGGL((deq_iq4_kernel<true>), dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        case FHIP_MXFP4: hipLaunchKernelGGL(deq_mxfp4_kernel, dim3((unsigned)grid), dim3(256), 0, s, d_raw, nquads, d_out); break;
-        default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "unsupported ggml type %u", type);
-    }
-    return check_hip(hipGetLastError(), "dequant launch");
+    return of_type(type, ToDevice{d_raw, nquads, d_out, s});
+}
+
+int launch_dequant_through(uint32_t type, const uint8_t* pinned_raw, size_t nblocks, float* pinned_out, uint32_t* done, uint32_t seq, hipStream_t s, int* wgs) {
+    return of_type(type, ToHost{pinned_raw, (uint32_t)nblocks, pinned_out, done, seq, s, wgs});
 }
 
 }  // namespace fhip

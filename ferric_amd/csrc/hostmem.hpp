@@ -27,4 +27,8 @@ int upload(void* d, const void* h, size_t n, hipStream_t s);     // copy_h2d tha
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s);   // synchronises; refused in a capture
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nblocks, size_t block_values, size_t block_bytes, float* h_out);   // synchronises
 
+// dequant.hip: nblocks blocks of pinned host memory, which is read up to the next 16 bytes, to floats of pinned host memory; workgroup w < *wgs stores seq in done[w] when what it
+// writes has arrived. Both 16-byte aligned, at most 4096 values a word of `done`.
+int launch_dequant_through(uint32_t type, const uint8_t* pinned_raw, size_t nblocks, float* pinned_out, uint32_t* done, uint32_t seq, hipStream_t s, int* wgs);
+
 }  // namespace fhip

@@ -15,6 +15,7 @@
 // Nobody waits for another stream's work: a long copy takes the workers, which serve one at a time, once its own stream has got there, and who finds no slot
 // goes through the runtime.
 #include "hostmem.hpp"
+#include "through.hpp"
 
 #include <string.h>
 
@@ -28,7 +29,8 @@
 
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+using fhip::store_through;
+using fhip::u32x4;
 
 constexpr size_t OUT_BYTES = (size_t)1 << 20;    // a slot's part for data on its way to the host ...
 constexpr size_t IN_BYTES = fhip::H2D_STAGED;    // ... and to the device (a chunk of floats is at most 278 528 block bytes, Q8_0)
@@ -45,10 +47,6 @@ constexpr int MAX_DEVICES = 64;
 // in done[w] once everything it reads has been read and everything it writes has arrived.
 // A confirmation is one store behind a wait, not a release: a release at system scope writes back the whole L2 (5 us of a 4 KB copy).
 // The stores it stands for go through to memory themselves (sc0 sc1), and s_waitcnt holds the wave until they have arrived.
-template <class U>
-__device__ __forceinline__ void store_through(U* p, U v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
-template <>
-__device__ __forceinline__ void store_through(u32x4* p, u32x4 v) { asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory"); }
 
 // The copy in up to N parts one after the other, each confirmed by itself: part p ends at byte end[p] (a multiple of 16 but for the last one's).
 // A copy in one part is a kernel of its own: with eight parts' arguments and their loop it takes 0.3 us more (4096 values dequantized for the host
@@ -106,7 +104,6 @@ int launch_copy(const void* src, void* dst, size_t n, int max_wg, uint32_t* done
 
 struct Slot {
     uint8_t* host = nullptr;     // SLOT_BYTES pinned: [OUT_BYTES][IN_BYTES]
-    uint8_t* dev = nullptr;      // as much device memory (dequantization only)
     uint32_t* done = nullptr;    // MAX_WG pinned words, of a copy in parts the last part's ...
     uint32_t* early = nullptr;   // ... and (PARTS - 1) * MAX_WG for the parts before it
     uint32_t seq = 0;
@@ -507,10 +504,9 @@ static int dequant_plain(Ring* r, uint32_t type, const uint8_t* h_raw, size_t nb
     return rc;
 }
 
-// nb blocks (bytes each, vals values) of host memory to nb * vals floats of host memory: chunk by chunk the bytes go up, are unpacked
-// on the device, go down into the slot and out of it by a worker. Two streams, so that the way up of one chunk and its unpacking run
-// beside the way down of the one before it. (The unpacker wrote into the slot itself once; the way over device memory costs a chunk
-// 5 of its 40 us, beside the bus, and lets the copy kernel confirm the chunk instead of an event that the workers had to query.)
+// nb blocks (bytes each, vals values) of host memory to nb * vals floats of host memory: chunk by chunk a worker copies the bytes into a slot, one kernel takes
+// them out of it and leaves the floats there, and a worker copies those out. Two streams, so that one chunk's bytes come up while the floats of the one
+// before go down.
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, size_t bytes, float* h_out) {
     int rc;
     if ((rc = may_wait(nullptr, "fhip_deq_raw"))) return rc;
@@ -524,13 +520,9 @@ int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nb, size_t vals, si
     const size_t per = CHUNK / sizeof(float) / vals, out_chunk = per * vals * sizeof(float);   // blocks of a chunk, and their floats
     const size_t n = nb * vals * sizeof(float);
     if (!plain_host(h_raw) || !plain_host(h_out)) return dequant_plain(r, type, h_raw, nb, per, vals, bytes, h_out);
+    static_assert(CHUNK / sizeof(float) <= (size_t)4096 * MAX_WG, "a chunk's workgroups have a word each");
     auto launch = [&](size_t c, Slot* q, hipStream_t s, int* wgs) {
-        const size_t blocks = nb - c * per < per ? nb - c * per : per;
-        int err;
-        if (!q->dev && (err = device_malloc((void**)&q->dev, SLOT_BYTES, "hipMalloc"))) { q->dev = nullptr; return err; }
-        if ((err = launch_copy(q->host + OUT_BYTES, q->dev + OUT_BYTES, blocks * bytes, MAX_WG, nullptr, 0, s, wgs))) return err;
-        if ((err = launch_dequant(type, q->dev + OUT_BYTES, blocks, (float*)q->dev, s))) return err;
-        return launch_copy(q->dev, q->host, blocks * vals * sizeof(float), MAX_WG, q->done, q->seq + 1, s, wgs);
+        return launch_dequant_through(type, q->host + OUT_BYTES, nb - c * per < per ? nb - c * per : per, (float*)q->host, q->done, q->seq + 1, s, wgs);
     };
     if (nb > per) {
         Job j{};

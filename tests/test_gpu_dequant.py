@@ -134,3 +134,16 @@ def test_full_size_matrices_bit_exact(F, O):
         got = F.deq_raw(w, rows * cols, ty)
         want = O.deq_raw(w, rows * cols, ty)
         assert np.array_equal(bits(got), bits(want)), (ty, rows, cols)
+
+
+@pytest.mark.parametrize("ty,vals,size", [(2, 32, 18), (3, 32, 20), (6, 32, 22), (7, 32, 24), (8, 32, 34), (12, 256, 144), (13, 256, 176), (14, 256, 210), (20, 32, 18),
+                                          (23, 256, 136), (39, 32, 17)])
+def test_host_bytes_around_a_workgroups_and_a_chunks_values(F, O, ty, vals, size):
+    # a workgroup unpacks 4096 values out of LDS, a chunk of a longer call is 262144: one block, one less, one more, and bytes that end inside a 16-byte piece
+    rng = np.random.default_rng(ty)
+    for values in (vals, 4096 - vals, 4096, 4096 + vals, 8192 + vals, 262144 - vals, 262144, 262144 + vals, 2 * 262144 + 4096 + vals):
+        raw = rng.integers(0, 256, (values // vals, size), dtype=np.uint8)
+        for off in {39: (), 14: (208,), 3: (0, 2), 7: (0, 2), 12: (0, 2), 13: (0, 2)}.get(ty, (0,)):
+            raw[:, off + 1] &= 0xBB                               # f16 scales: finite (a NaN's payload is not part of the contract)
+        raw = np.concatenate([np.zeros(3, np.uint8), raw.reshape(-1)])[3:]      # an odd host address
+        assert_bits_equal(F.deq_raw(raw, values, ty), O.deq_raw(raw, values, ty), f"ty {ty} {values}")
