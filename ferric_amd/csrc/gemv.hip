@@ -43,6 +43,7 @@
 #include "common.hpp"
 #include "deq_at.hpp"
 #include "fixed_point.hpp"
+#include "lut16.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -464,13 +465,6 @@ typedef LegS<FHIP_Q5_1, 24, true, true, 0> Q51;
 // IQ4_NL (18 B = [f16 d][qs 16 B]) and IQ4_XS (136 B = [f16 d][u16 scales_h][scales_l 4 B][qs 128 B]): 4-bit indices into the
 // 16-level codebook {-127 .. 113} (crates/ferric-gguf/src/lib.rs:751-791), looked up four at a time by byte permute into int8
 // levels. Unit = one 32-value (sub-)block.
-__device__ __forceinline__ uint32_t lut16x4(uint32_t idx, uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
-    uint32_t sel = idx & 0x07070707u;
-    uint32_t lo = __builtin_amdgcn_perm(t1, t0, sel);   // selector 0..3: bytes of t0, 4..7: bytes of t1
-    uint32_t hi = __builtin_amdgcn_perm(t3, t2, sel);
-    uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu;
-    return (hi & m) | (lo & ~m);
-}
 struct __attribute__((packed, aligned(8))) U4A8 { u32x4 v; };
 
 template <bool XS>
@@ -506,7 +500,7 @@ struct IQ4S {
     static __device__ __forceinline__ void dot(const Data& D, const Lane& L, const uint32_t (&xp)[M][NRUN][NP][RUN / 4],
                                                const float (&xs)[M][NRUN], const float (&)[M][NRUN], float (&out)[M]) {
         // the codebook as int8 bytes, four levels per word
-        constexpr uint32_t T0 = 0xBFAD9881u, T1 = 0xF6EADDCFu, T2 = 0x26190D01u, T3 = 0x71594535u;
+        constexpr fhip::Lut16 LUT = fhip::lut16(0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u);
         int acc[M][NP];
 #pragma unroll
         for (int m = 0; m < M; m++)
@@ -514,7 +508,7 @@ struct IQ4S {
             for (int p = 0; p < NP; p++) acc[m][p] = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            uint32_t lo = lut16x4(D.q[j] & 0x0F0F0F0Fu, T0, T1, T2, T3), hi = lut16x4((D.q[j] >> 4) & 0x0F0F0F0Fu, T0, T1, T2, T3);
+            uint32_t lo = fhip::lut16x4(D.q[j] & 0x0F0F0F0Fu, LUT), hi = fhip::lut16x4((D.q[j] >> 4) & 0x0F0F0F0Fu, LUT);
 #pragma unroll
             for (int m = 0; m < M; m++)
 #pragma unroll
@@ -564,13 +558,13 @@ struct MXF4S {
     template <int M>
     static __device__ __forceinline__ void dot(const Data& D, const Lane&, const uint32_t (&xp)[M][NRUN][NP][RUN / 4],
                                                const float (&xs)[M][NRUN], const float (&)[M][NRUN], float (&out)[M]) {
-        constexpr uint32_t T0 = 0x03020100u, T1 = 0x0C080604u, T2 = 0xFDFEFF00u, T3 = 0xF4F8FAFCu;
+        constexpr fhip::Lut16 LUT = fhip::lut16(0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu);
         const float d = __uint_as_float(D.e == 0 ? (1u << 21) : D.e == 1 ? (1u << 22) : (D.e - 1u) << 23);
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            lo[j] = lut16x4(D.q[j] & 0x0F0F0F0Fu, T0, T1, T2, T3);
-            hi[j] = lut16x4((D.q[j] >> 4) & 0x0F0F0F0Fu, T0, T1, T2, T3);
+            lo[j] = fhip::lut16x4(D.q[j] & 0x0F0F0F0Fu, LUT);
+            hi[j] = fhip::lut16x4((D.q[j] >> 4) & 0x0F0F0F0Fu, LUT);
         }
         if (D.e >= 252u) {   // a weight of this block may be +-inf: the reference's per-element products
             // (indexed by unrolled loops only: a run-time index would keep the planes of every block in scratch memory)

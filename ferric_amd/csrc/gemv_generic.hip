@@ -23,6 +23,7 @@
 //     in LDS; after one barrier the S partials of each row are added in a fixed order, so the result
 //     does not depend on scheduling.
 #include "common.hpp"
+#include "lut16.hpp"
 
 #include <hip/hip_fp16.h>
 #include <stdlib.h>
@@ -335,14 +336,6 @@ struct Q5K {
     }
 };
 
-// Four 4-bit indices (one per byte of idx, the upper nibbles clear) looked up in a 16-entry byte table held in t0..t3.
-__device__ __forceinline__ uint32_t lut16x4(uint32_t idx, uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
-    uint32_t sel = idx & 0x07070707u;
-    uint32_t lo = __builtin_amdgcn_perm(t1, t0, sel);   // selector 0..3: bytes of t0, 4..7: bytes of t1
-    uint32_t hi = __builtin_amdgcn_perm(t3, t2, sel);
-    uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu;
-    return (hi & m) | (lo & ~m);
-}
 struct __attribute__((packed, aligned(8))) U4A8 { u32x4 v; };
 struct __attribute__((packed, aligned(1))) U4A1 { u32x4 v; };
 
@@ -375,13 +368,14 @@ struct IQ4 {
     template <int M>
     static __device__ __forceinline__ void dot(const Data& D, const Lane& L, const float (&x)[M][32], const float (&sx)[M][4],
                                                float (&out)[M]) {
+        constexpr fhip::Lut16 LUT = fhip::lut16(0x3F2D1801u, 0x766A5D4Fu, 0xA6998D81u, 0xF1D9C5B5u);
         float acc[M];
 #pragma unroll
         for (int m = 0; m < M; m++) acc[m] = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            uint32_t lo = lut16x4(D.q[i] & 0x0F0F0F0Fu, 0x3F2D1801u, 0x766A5D4Fu, 0xA6998D81u, 0xF1D9C5B5u);
-            uint32_t hi = lut16x4((D.q[i] >> 4) & 0x0F0F0F0Fu, 0x3F2D1801u, 0x766A5D4Fu, 0xA6998D81u, 0xF1D9C5B5u);
+            uint32_t lo = fhip::lut16x4(D.q[i] & 0x0F0F0F0Fu, LUT);
+            uint32_t hi = fhip::lut16x4((D.q[i] >> 4) & 0x0F0F0F0Fu, LUT);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 float fl = ub(lo, k), fh = ub(hi, k);

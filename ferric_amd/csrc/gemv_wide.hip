@@ -31,6 +31,7 @@
 #include "common.hpp"
 #include "deq_at.hpp"
 #include "fixed_point.hpp"
+#include "lut16.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -121,13 +122,6 @@ typedef Leg<FHIP_Q4_1, 20, true, false, 0> Q41;
 typedef Leg<FHIP_Q5_0, 22, false, true, 16> Q50;
 typedef Leg<FHIP_Q5_1, 24, true, true, 0> Q51;
 
-__device__ __forceinline__ uint32_t lut16x4(uint32_t idx, uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
-    const uint32_t sel = idx & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(t1, t0, sel);   // selector 0..3: bytes of t0, 4..7: bytes of t1
-    const uint32_t hi = __builtin_amdgcn_perm(t3, t2, sel);
-    const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu;
-    return (hi & m) | (lo & ~m);
-}
 
 template <bool XS>
 struct Iq4 {
@@ -165,8 +159,8 @@ struct Iq4 {
     }
     static __device__ __forceinline__ u32x2 operand(const Four& f, int j, int) {
         // the codebook as int8 bytes, four levels per word (crates/ferric-gguf/src/lib.rs:751-791)
-        constexpr uint32_t T0 = 0xBFAD9881u, T1 = 0xF6EADDCFu, T2 = 0x26190D01u, T3 = 0x71594535u;
-        return (u32x2){lut16x4(f.q[j] & 0x0F0F0F0Fu, T0, T1, T2, T3), lut16x4((f.q[j] >> 4) & 0x0F0F0F0Fu, T0, T1, T2, T3)};
+        constexpr fhip::Lut16 LUT = fhip::lut16(0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u);
+        return (u32x2){fhip::lut16x4(f.q[j] & 0x0F0F0F0Fu, LUT), fhip::lut16x4((f.q[j] >> 4) & 0x0F0F0F0Fu, LUT)};
     }
     static __device__ __forceinline__ float value(const Four& f, int j, float pf, float xs, float) { return (xs * pf) * __uint_as_float(f.d[j]); }
     static __device__ __forceinline__ bool big(const Four&, int) { return false; }
@@ -177,7 +171,7 @@ struct Iq4 {
 struct Mxf4 {
     static constexpr uint32_t TYPE = FHIP_MXFP4;
     static constexpr bool HAS_XQ = false, BIG = true;
-    static constexpr uint32_t T0 = 0x03020100u, T1 = 0x0C080604u, T2 = 0xFDFEFF00u, T3 = 0xF4F8FAFCu;
+    static constexpr fhip::Lut16 LUT = fhip::lut16(0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu);
     struct Data { u32x4 q; uint32_t e; };
     struct Four { u32x4 q, d; };
     static __device__ __forceinline__ Data load(const uint8_t* row, int u) {
@@ -197,7 +191,7 @@ struct Mxf4 {
         return Four{dwords4(wl + c * ROW + 4 * g4), ((const u32x4*)(wl + 16 * ROW))[c]};
     }
     static __device__ __forceinline__ u32x2 operand(const Four& f, int j, int) {
-        return (u32x2){lut16x4(f.q[j] & 0x0F0F0F0Fu, T0, T1, T2, T3), lut16x4((f.q[j] >> 4) & 0x0F0F0F0Fu, T0, T1, T2, T3)};
+        return (u32x2){fhip::lut16x4(f.q[j] & 0x0F0F0F0Fu, LUT), fhip::lut16x4((f.q[j] >> 4) & 0x0F0F0F0Fu, LUT)};
     }
     static __device__ __forceinline__ float value(const Four& f, int j, float pf, float xs, float) { return (xs * pf) * __uint_as_float(f.d[j]); }
     static constexpr uint32_t BIG_BITS = 251u << 23;     // the scale of e = 252
@@ -446,7 +440,7 @@ __global__ void __launch_bounds__((64 * max_waves<F, E>())) gemv_wide_kernel(Wid
 #pragma unroll 1
                                 for (int n = 0; n < 32; n++) {
                                     const uint32_t nib = n < 16 ? (uint32_t)qsb[n & 15] & 15u : (uint32_t)qsb[n & 15] >> 4;
-                                    const uint32_t k = lut16x4(nib, Mxf4::T0, Mxf4::T1, Mxf4::T2, Mxf4::T3);
+                                    const uint32_t k = fhip::lut16x4(nib, Mxf4::LUT);
                                     int xv = 0;
 #pragma unroll
                                     for (int pp = 0; pp < NP; pp++)
