@@ -101,6 +101,7 @@ __device__ __forceinline__ constexpr int kcol(int t, int h) { return 32 * (t >> 
 // ------------------------------------------------------------------------------------------------
 
 struct Q4K {
+    static constexpr bool OWN_TURNS = false;
     using Eager = Q4K;
     static constexpr int BLOCK = 144;
     static constexpr float UNPACK_US = 1.4f;   // unpack of a 256 x 256 chunk by one workgroup
@@ -161,6 +162,7 @@ struct Q4K {
 // step G takes bit 2G + (T >> 1) of them. The high nibbles are shifted down (with the fifth bit on top they do not fit a
 // byte in place), so both sub-block scales are plain d * sc.
 struct Q5K {
+    static constexpr bool OWN_TURNS = false;
     using Eager = Q5K;
     static constexpr int BLOCK = 176;
     static constexpr float UNPACK_US = 1.8f;
@@ -210,13 +212,14 @@ struct Q5K {
 };
 
 struct Q6K {
+    static constexpr bool OWN_TURNS = true;
     using Eager = Q6K;
     // Step G covers half hf = G >> 1 of the super-block and its groups g0 = 2(G & 1), g0 + 1 (low nibbles of
     // ql for G even, high nibbles for G odd); slice T is group g = g0 + (T >> 1), l = 16h + 8(T & 1) + [0, 8),
     // whose scale is sc[8hf + 2g + h]  (crates/ferric-gguf/src/lib.rs:833-851).
     static constexpr int BLOCK = 210;
     static constexpr float UNPACK_US = 2.3f;
-    static constexpr float CHUNK_US[NTILES] = {4.70f, 5.89f, 8.29f, 5.71f, 2.78f, 2.21f, 4.16f, 2.27f, 1.73f, 2.72f, 1.73f, 2.04f};
+    static constexpr float CHUNK_US[NTILES] = {4.15f, 5.47f, 8.75f, 5.95f, 2.78f, 2.03f, 4.40f, 2.43f, 1.76f, 2.52f, 1.37f, 1.75f};
     static constexpr float RUN_CHUNK_US[7] = {5.93f, 6.83f, 9.84f, 6.27f, 4.68f, 3.95f, 4.35f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
@@ -288,12 +291,13 @@ struct Q6K {
 template <bool LATE>
 struct Q80T {
     using Eager = Q80T<false>;
+    static constexpr bool OWN_TURNS = true;
     // A chunk is 8 blocks of 34 bytes; step G covers blocks 2G, 2G+1; slice T is block 2G + (T >> 1),
     // elements 16h + 8(T & 1) + [0, 8). A trailing partial chunk is allowed: blocks past the row's end are
     // read from the last valid block's address and given scale 0 (their activations are staged as 0 too).
     static constexpr int BLOCK = 34;
     static constexpr float UNPACK_US = 5.1f;
-    static constexpr float CHUNK_US[NTILES] = {6.25f, 7.76f, 10.02f, 5.99f, 3.94f, 3.29f, 4.15f, 4.13f, 3.11f, 3.91f, 1.70f, 2.08f};
+    static constexpr float CHUNK_US[NTILES] = {4.66f, 5.96f, 11.44f, 6.65f, 3.15f, 2.23f, 4.62f, 2.91f, 1.98f, 2.76f, 1.22f, 1.76f};
     static constexpr float RUN_CHUNK_US[7] = {9.40f, 9.88f, 11.93f, 6.86f, 7.00f, 6.50f, 5.05f};
     static constexpr bool PARTIAL = true;   // a row may end inside a chunk
     static __host__ __device__ int chunks(int K) { return (K + 255) / 256; }
@@ -832,6 +836,8 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 // ------------------------------------------------------------------------------------------------
 template <int S>
 struct OwnQ4K {
+    static constexpr bool TURNS = false;
+    static constexpr int SEGS = 2;
     struct Raw { u32x4 hd, q[S]; };
     struct Ctx { float d0, o0, d1, o1; };
     static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
@@ -861,6 +867,8 @@ struct OwnQ4K {
 
 template <int S>
 struct OwnQ5K {
+    static constexpr bool TURNS = false;
+    static constexpr int SEGS = 2;
     struct Raw { u32x4 hd, qh, q[S]; };
     using Ctx = typename OwnQ4K<S>::Ctx;
     static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
@@ -897,27 +905,45 @@ struct OwnQ5K {
     }
 };
 
+// Formats whose blocks are not whole 16-byte pieces (TURNS): their rows come in consecutive pieces and are turned through LDS (fetch, turn in the kernel). A segment is
+// five pieces of each of the wave's 32 rows, the first from the dword at or below its first byte; piece_off() says where a piece lies in the row's chunk, take() reads
+// segment G's part of a lane's Raw from its row's 80 bytes. 80 bytes apart, sixteen rows' 16-byte reads meet every bank once.
+// Why: a load whose lanes each read a row of their own takes the address unit a cycle a lane, 0.2 us for the eight waves of a workgroup, and Q6_K needed 17
+// such loads a chunk, Q8_0 24; of these, ten touch some twenty cache lines each. A chunk of 64 x 256 outputs: Q6_K 4.70 -> 4.15 us, Q8_0 6.25 -> 4.66, of 64 x 128 2.21 -> 2.03,
+// 3.29 -> 2.23 (what is left over Q4_K's 2.39 and 1.29 is their unpacking, 541 and 461 vector instructions to 342, and the way through LDS). With the estimate fitted again, us: Q8_0
+// 3160 x 3328 at 196 rows 26.0 -> 18.5, 2120 x 5632 at 206 28.9 -> 26.7; Q6_K 25736 x 11776 at 44 105 -> 90, 1712 x 13312 at 184 33.7 -> 29.8; FFN blocks of both, 1024 x 7680 at
+// 271 53.8 -> 46.5. Q4_K's five loads a chunk turned the same way: 3 - 6 % slower.
+constexpr int SEG_ROW = 80, SEG_BYTES = 32 * SEG_ROW;
+__device__ __forceinline__ fhip::Un16 un16(const uint8_t* p) { return fhip::Un16{((const fhip::LdU4A4*)p)->v, *(const uint16_t*)(p + 16)}; }
+
 template <int S>
 struct OwnQ6K {
+    static constexpr bool TURNS = true;
+    static constexpr int SEGS = S == 4 ? 4 : 2, CHUNK_BYTES = 210;    // of each half: the nibbles; the bit pairs (three pieces), scales and d (two)
+    static __device__ __forceinline__ int piece_off(int seg, int j, int g0) {
+        const int hf = (g0 >> 1) + (seg >> 1);
+        return (seg & 1) == 0 ? 64 * hf + 16 * j : j < 3 ? 128 + 32 * hf + 16 * j : 192 + 16 * (j - 3);
+    }
     static constexpr int NH = S == 4 ? 2 : 1;                   // halves of the super-block the steps lie in
     struct Raw { fhip::Un16 ql[NH][2], qh[NH]; uint32_t sc[NH][3], d; };
     struct Ctx { float d; };
-    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int) {
-        const uint8_t* blk = row + (size_t)c * 210;
-#pragma unroll
-        for (int i = 0; i < NH; i++) {
-            const int hf = (g0 >> 1) + i;
-            r.ql[i][0] = fhip::load16_un<true>(blk + 64 * hf + 16 * h);
-            r.ql[i][1] = fhip::load16_un<true>(blk + 64 * hf + 32 + 16 * h);
-            r.qh[i] = fhip::load16_un<true>(blk + 128 + 32 * hf + 16 * h);
-            const uint8_t* s = blk + 192 + 8 * hf;
-            const fhip::ld_u32x2 v = ((const fhip::LdU2A4*)(s - ((uint32_t)(uintptr_t)s & 2u)))->v;
-            r.sc[i][0] = v[0];
-            r.sc[i][1] = v[1];
-            r.sc[i][2] = *(const uint16_t*)(s + 6);
+    // m: the block's address modulo 4
+    template <int G>
+    static __device__ __forceinline__ void take(Raw& r, const uint8_t* row, int g0, int h, uint32_t m) {
+        constexpr int i = G >> 1;
+        if constexpr ((G & 1) == 0) {
+            r.ql[i][0] = un16(row + 16 * h);
+            r.ql[i][1] = un16(row + 32 + 16 * h);
+        } else {
+            r.qh[i] = un16(row + 16 * h);
+            const uint8_t* sc = row + 48 + 8 * ((g0 >> 1) + i);
+            r.sc[i][0] = *(const uint32_t*)sc;
+            r.sc[i][1] = *(const uint32_t*)(sc + 4);
+            r.sc[i][2] = *(const uint16_t*)(sc + 8);
+            if (G == SEGS - 1) r.d = *(const uint16_t*)(row + 64 + m);   // (the block before has taken its own from there)
         }
-        r.d = *(const uint16_t*)(blk + 208);
     }
+    static __device__ __forceinline__ uint32_t parity(const uint8_t* row, int c) { return ((uint32_t)(uintptr_t)row + 2u * (uint32_t)(c & 1)) & 2u; }
     static __device__ __forceinline__ void settle(Raw& r, const uint8_t* row, int c, int g0, int h) {
         const uint32_t m = ((uint32_t)(uintptr_t)row + 2u * (uint32_t)(c & 1)) & 2u;     // every piece starts at a multiple of 4 of its block
 #pragma unroll
@@ -957,18 +983,19 @@ struct OwnQ6K {
 
 template <int S>
 struct OwnQ80 {
+    static constexpr bool TURNS = true;
+    static constexpr int SEGS = S, CHUNK_BYTES = 272;                 // a step's two blocks; what lies behind a row's end has the scale 0
+    static __device__ __forceinline__ int piece_off(int seg, int j, int g0) { return 68 * (g0 + seg) + 16 * j; }
     struct Raw { fhip::Un16 q[S][2]; uint32_t d[S][2]; };
     struct Ctx { float d[2]; };
-    static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int c, int g0, int h, int nblk) {
-#pragma unroll
-        for (int i = 0; i < S; i++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const uint8_t* p = Q80T<true>::blk(row, c, 2 * (g0 + i) + u, nblk);
-                r.d[i][u] = *(const uint16_t*)p;
-                r.q[i][u] = fhip::load16_un<true>(p + 2 + 16 * h);
-            }
+    template <int G>
+    static __device__ __forceinline__ void take(Raw& r, const uint8_t* row, int, int h, uint32_t m) {
+        r.d[G][0] = *(const uint16_t*)(row + m);
+        r.d[G][1] = *(const uint16_t*)(row + 34 + m);
+        r.q[G][0] = un16(row + 16 * h + 2 * m);
+        r.q[G][1] = un16(row + 36 + 16 * h);
     }
+    static __device__ __forceinline__ uint32_t parity(const uint8_t* row, int) { return (uint32_t)(uintptr_t)row & 2u; }
     static __device__ __forceinline__ void settle(Raw&, const uint8_t*, int, int, int) {}
     template <int I>
     static __device__ __forceinline__ void begin(Raw& r, const uint8_t* row, int c, int g0, int, int nblk, Ctx& x) {
@@ -1000,6 +1027,7 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
     constexpr int KEEP = 16 / KW;                               // of a fragment's 16 accumulator registers, those a wave stores in the end
     using F = typename Own<FMT, S>::type;
     __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * XROW];
+    __shared__ __attribute__((aligned(16))) uint8_t Seg[F::TURNS ? NW * KW * SEG_BYTES : 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % NW, kg = wave / NW, g0 = S * kg;
     const int h = lane >> 5, c = lane & 31;
@@ -1030,6 +1058,59 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
         n = n < p.N ? n : p.N - 1;
         wrow = p.W + (size_t)(SWIGLU ? swiglu_row(n, p.ff) : n) * p.row_bytes;
     }
+    // Weights of a TURNS format. Of every two segments load k of five brings pieces 64 k + lane of their 2 x 160: row (64 k + lane) / 5 of the first, from
+    // 160 on of the second.
+    constexpr int PAIRS = (F::SEGS + 1) / 2, LOADS_A_PAIR = F::SEGS == 1 ? 3 : 5;
+    u32x4 G[F::TURNS ? LOADS_A_PAIR : 1];
+    uint32_t g_off[LOADS_A_PAIR];                               // from the wave's first row on (weights of 4 GB and more take other tiles: choose_plan)
+    const int rows = SWIGLU ? p.ff : p.N, n_first = SWIGLU ? n0 / 2 : n0, first_row = n_first < rows ? n_first : rows - 1;
+    uint8_t* const seg = Seg + (F::TURNS ? wave * SEG_BYTES : 0);
+    auto piece = [&](int k) { const int q = 64 * k + lane; return q < 160 ? q : F::SEGS == 1 ? 159 : q - 160; };   // (past an only segment: its last again)
+    auto second = [&](int k) { return F::SEGS > 1 && 64 * k + lane >= 160 ? 1 : 0; };
+    if constexpr (F::TURNS) {
+#pragma unroll
+        for (int k = 0; k < LOADS_A_PAIR; k++) {
+            const int q = piece(k), v = q / 5, r = SWIGLU ? v & 15 : v;
+            g_off[k] = (uint32_t)((first_row + r < rows ? r : rows - 1 - first_row) + (SWIGLU && v > 15 ? p.ff : 0)) * (uint32_t)p.row_bytes + (uint32_t)F::piece_off(second(k), q % 5, g0);
+        }
+    }
+    // the loads of segments 2 g and 2 g + 1 of chunk ck
+    auto fetch = [&](auto Gc, u32x4 (&G)[F::TURNS ? LOADS_A_PAIR : 1], int ck) {
+      if constexpr (F::TURNS) {
+        constexpr int g = decltype(Gc)::value;
+        const uint8_t* const from = p.W + ((size_t)first_row * p.row_bytes + (size_t)ck * F::CHUNK_BYTES);
+        const uint32_t odd = (uint32_t)(uintptr_t)from & 3u;
+#pragma unroll
+        for (int k = 0; k < LOADS_A_PAIR; k++) {
+            uint32_t off = g_off[k] + odd;
+            if (g) off += F::piece_off(2 + second(k), piece(k) % 5, g0) - F::piece_off(second(k), piece(k) % 5, g0);
+            G[k] = ((const fhip::LdU4A4*)(from - odd + (off & ~3u)))->v;
+        }
+      }
+    };
+    // ... to LDS and back, a row a lane. (One wave's LDS operations keep their order; the fence keeps the compiler's.)
+    auto turn = [&](auto Gc, const u32x4 (&G)[F::TURNS ? LOADS_A_PAIR : 1], typename F::Raw& r, int ck) {
+      if constexpr (F::TURNS) {
+        constexpr int g = decltype(Gc)::value;
+        const uint32_t m = F::parity(wrow, ck);
+        auto fence = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+        fence();
+        *(u32x4*)(seg + 16 * lane) = G[0];
+        *(u32x4*)(seg + 1024 + 16 * lane) = G[1];
+        if (lane < 32) *(u32x4*)(seg + 2048 + 16 * lane) = G[2];
+        fence();
+        F::template take<2 * g>(r, seg + c * SEG_ROW, g0, h, m);
+        fence();
+        if constexpr (F::SEGS > 1) {
+            if (lane >= 32) *(u32x4*)(seg + 16 * (lane - 32)) = G[2];
+            *(u32x4*)(seg + 512 + 16 * lane) = G[3];
+            *(u32x4*)(seg + 1536 + 16 * lane) = G[4];
+            fence();
+            F::template take<2 * g + 1>(r, seg + c * SEG_ROW, g0, h, m);
+            fence();
+        }
+      }
+    };
     f32x16 acc[MI];
 #pragma unroll
     for (int i = 0; i < MI; i++)
@@ -1067,7 +1148,7 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
     // chunk ago, goes to the other buffer and its register asks for chunk ck + 2. The barrier stands in front of the last slice, whose
     // matrix instructions cover the first reads and the first unpacking of the next chunk.
     constexpr int NS = 4 * S, QS = (NQ + NS - 3) / (NS - 2);    // slices of a chunk; pieces moved behind each of the first NS - 2
-    typename F::Raw raw[2];
+    typename F::Raw raw[F::TURNS ? 1 : 2];                      // (a turned chunk lies in G until its predecessor has been unpacked)
     bf16x8 a[2][MI], b[2];
     typename F::Ctx ctx;
     auto read_a = [&](int buf, int s, bf16x8 (&d)[MI]) {
@@ -1075,7 +1156,7 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
         for (int i = 0; i < MI; i++) d[i] = *(const bf16x8*)(&As[buf][a_rd + 32 * i * XROW + KSTEP * (s >> 2) + kcol(s & 3, 0)]);
     };
     auto chunk = [&](auto Pc, auto Lc, int ck) {
-        constexpr int P = decltype(Pc)::value;
+        constexpr int P = decltype(Pc)::value, R = F::TURNS ? 0 : P, RN = F::TURNS ? 0 : P ^ 1;   // Raw of this chunk and of the next
         constexpr bool LOADS = decltype(Lc)::value;
         const int c2 = ck + 2 < c_last ? ck + 2 : c_last;
         static_for<0, NS>([&](auto Sc) {
@@ -1083,14 +1164,22 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
             if constexpr (n < NS) read_a(P, n, a[n & 1]);
             else read_a(P ^ 1, 0, a[0]);
             if constexpr (n == NS) {
-                F::settle(raw[P ^ 1], wrow, ck + 1, g0, h);
-                F::template begin<0>(raw[P ^ 1], wrow, ck + 1, g0, h, p.nblk, ctx);
-            } else if constexpr ((n & 3) == 0) F::template begin<(n >> 2)>(raw[P], wrow, ck, g0, h, p.nblk, ctx);
+                F::settle(raw[RN], wrow, ck + 1, g0, h);
+                F::template begin<0>(raw[RN], wrow, ck + 1, g0, h, p.nblk, ctx);
+            } else if constexpr ((n & 3) == 0) F::template begin<(n >> 2)>(raw[R], wrow, ck, g0, h, p.nblk, ctx);
 #pragma unroll
             for (int i = 0; i < MI; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][i], b[s & 1], acc[i], 0, 0, 0);
-            if constexpr (n == NS) b[0] = F::template frag<0, 0>(raw[P ^ 1], ctx);
-            else b[n & 1] = F::template frag<(n >> 2), (n & 3)>(raw[P], ctx);
-            if constexpr (LOADS && s == NS - 2) F::load(raw[P], wrow, c2, g0, h, p.nblk);
+            if constexpr (n == NS) b[0] = F::template frag<0, 0>(raw[RN], ctx);
+            else b[n & 1] = F::template frag<(n >> 2), (n & 3)>(raw[R], ctx);
+            if constexpr (!F::TURNS) {
+                if constexpr (LOADS && s == NS - 2) F::load(raw[R], wrow, c2, g0, h, p.nblk);
+            } else if constexpr (s % (NS / PAIRS) == NS / PAIRS - 2) {   // behind the last frag() of a pair's registers: the next chunk's pair, then the loads of the pair behind it
+                using std::integral_constant;
+                constexpr int g = s / (NS / PAIRS);
+                turn(integral_constant<int, g>{}, G, raw[0], ck + 1);
+                if constexpr (g + 1 < PAIRS) fetch(integral_constant<int, g + 1>{}, G, ck + 1 < c_last ? ck + 1 : c_last);
+                else if (LOADS) fetch(integral_constant<int, 0>{}, G, c2);
+            }
 #pragma unroll
             for (int q = QS * s; q < QS * (s + 1) && q < NQ; q++) {
                 store_a(P ^ 1, q);
@@ -1111,14 +1200,23 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
         const int c1 = c_begin < c_last ? c_begin + 1 : c_last;
 #pragma unroll
         for (int q = 0; q < NQ; q++) load_a(c_begin, q);
-        F::load(raw[0], wrow, c_begin, g0, h, p.nblk);
+        u32x4 G1[F::TURNS ? LOADS_A_PAIR : 1];                  // the first chunk's second pair
+        using std::integral_constant;
+        if constexpr (F::TURNS) {
+            fetch(integral_constant<int, 0>{}, G, c_begin);
+            if constexpr (PAIRS > 1) fetch(integral_constant<int, 1>{}, G1, c_begin);
+        } else F::load(raw[0], wrow, c_begin, g0, h, p.nblk);
         if (round > 0) __syncthreads();                         // the last run's sums are read
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
             store_a(0, q);
             load_a(c1, q);
         }
-        F::load(raw[1], wrow, c1, g0, h, p.nblk);
+        if constexpr (F::TURNS) {
+            turn(integral_constant<int, 0>{}, G, raw[0], c_begin);
+            fetch(integral_constant<int, 0>{}, G, c1);
+            if constexpr (PAIRS > 1) turn(integral_constant<int, 1>{}, G1, raw[0], c_begin);
+        } else F::load(raw[1], wrow, c1, g0, h, p.nblk);
         __syncthreads();
         read_a(0, 0, a[0]);
         F::settle(raw[0], wrow, c_begin, g0, h);
@@ -1532,7 +1630,8 @@ static long long plan_segments(const TilePlan& q) { return q.runs + (q.left - 1)
 // A linear model fitted (non-negative least squares on relative errors, 7 % rms) to 3700 launches: 357 weights of the four formats, 1024 ... 34816 rows
 // of 1024 ... 17408 columns, 33 ... 2048 activation rows, every tile. On those the tile it picks is 1.4 % slower than the measured best on average
 // (worst 25 %); the model it replaced, fitted to ten large weights, and the seven tiles it had were 20 % slower on average and up to 2.7 times
-// (6112 x 2816 Q4_K at 132 rows 42.0 -> 16.6 us). Left out, a tile costs 0.1 % (64 x 256, 64 x 160) to 2.5 % (64 x 64) of the mean.
+// (6112 x 2816 Q4_K at 132 rows 42.0 -> 16.6 us). Q6_K's and Q8_0's chunks were fitted again when their rows came to be turned: 136 launches a tile, the pick 1.6 and
+// 2.2 % slower than the best on average (4.1 and 8.7 with the figures before). Left out, a tile costs 0.1 % (64 x 256, 64 x 160) to 2.5 % (64 x 64) of the mean.
 constexpr float START_US[NTILES] = {3.77f, 3.88f, 4.04f, 4.53f, 3.92f, 3.12f, 4.91f, 3.57f, 2.73f, 4.01f, 2.31f, 3.95f}, FIX_US = 3.29f, SLOT_US = 4.18f, CUT_US = 0.1f;
 template <class F>
 static float plan_cost_us(const TilePlan& q, long long cus) {
@@ -1636,10 +1735,12 @@ static void choose_plan(const fhip_weight* w, size_t columns, size_t t, bool run
     }
     for (int i = 0; i < NTILES; i++) {
         if (fhip::g_gemm_tile >= 0 && fhip::g_gemm_tile < NTILES && i != fhip::g_gemm_tile) continue;
+        if (F::OWN_TURNS && i != 2 && i != 3 && i != 6 && w->nbytes > 0xFFF00000u) continue;   // offsets of 32 bits within the weight
         const TilePlan q = plan_tiles(columns, nchunks, t, i, cus);
         const float c = plan_cost_us<F>(q, cus);
         if (best_cost == 0.f || c < best_cost) { best_cost = c; out = q; }
     }
+    if (best_cost == 0.f) out = plan_tiles(columns, nchunks, t, 3, cus);     // (a pinned tile that the weight is too large for)
 }
 
 template <class F>

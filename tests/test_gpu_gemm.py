@@ -280,6 +280,28 @@ def test_swiglu_inside_the_tiled_gemm(F, tile):
 
 
 # 272 tiles of 64 x 128, 312 of 64 x 256 and of 128 x 256, and the launcher's choice: 256 workgroups take a whole one each and the rest is cut along K
+@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11])
+def test_swiglu_of_rows_turned_through_lds(F, tile):
+    # Q6_K and Q8_0 gate|up on the tiles whose waves unpack for themselves: a wave's gate and up rows lie in two places. Rows of an odd number of blocks, whose
+    # addresses alternate modulo 4, widths that end inside a tile, one chunk and an odd number of them, a Q8_0 row that ends inside a chunk; against the
+    # 256 x 160 tile, whose waves share what they unpack. The f32 sums differ in their last bits, so a value of h may round to the other bf16 neighbour, 2^-8 of it.
+    from ferric_amd.synth import synth_weights
+    lib = F._lib.load()
+    before = lib.fhip_debug_gemm_tile(tile)
+    try:
+        for i, (ty, t, d, n_ff) in enumerate([(Q6_K, 33, 256, 32), (Q6_K, 70, 768, 160), (Q8_0, 65, 288, 96), (Q8_0, 129, 1312, 1312)]):
+            gu = F.QMatrix.from_bytes(synth_weights(ty, 2 * n_ff, d, 700 + i), ty, 2 * n_ff, d)
+            dn = F.QMatrix.from_bytes(synth_weights(Q8_0, 64, n_ff, 720 + i), Q8_0, 64, n_ff)
+            x = F.Tensor.from_vec(np.random.default_rng(i).standard_normal(t * d).astype(np.float32), (t, d))
+            lib.fhip_debug_gemm_tile(3)
+            want = x.ffn_coop(gu, dn).to_vec()
+            lib.fhip_debug_gemm_tile(tile)
+            got = x.ffn_coop(gu, dn).to_vec()
+            assert np.linalg.norm(got - want) <= 2.0 ** -8 * np.linalg.norm(want), (tile, ty, t, d, n_ff)
+    finally:
+        lib.fhip_debug_gemm_tile(before)
+
+
 @pytest.mark.parametrize("tile,t,d,n_ff", [(5, 40, 512, 17408), (0, 130, 512, 13312), (1, 270, 768, 13312), (-1, 520, 512, 17408)])
 def test_swiglu_beside_whole_and_cut_tiles(F, O, tile, t, d, n_ff):
     # The fused launch deals columns of gate and up in turn to a tile and so cuts other outputs than a launch over the stacked rows does:
