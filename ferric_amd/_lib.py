@@ -210,6 +210,7 @@ try:
     from ferric_amd import _host        # the device memory object, an extension module built with the library
     _host.setup(_host_first_use, check)
     DeviceBuffer, matmul_q = _host.DeviceBuffer, _host.matmul_q
+    moe_topk, swiglu_id, id_wsum = _host.moe_topk, _host.swiglu_id, _host.id_wsum
 except (ImportError, AttributeError) as _e:      # not built, or built from older source
     _why = str(_e)
 

@@ -4,7 +4,8 @@
 // class around ctypes (c_void_p, byref, __init__, __del__) it took 3.4 us of a 7.1 us Q4_K 1024 x 5120 mat-vec, whose kernel takes
 // 4.4 us. A C type over the library's fhip_malloc / fhip_free does the same in a few hundred nanoseconds. A launch itself costs
 // the host 3 us on this runtime (0.9 us without arguments: the argument block is written to device memory and read back), which is
-// most of what is left of such a call, so matmul_q does all of its conversions here instead of in ctypes.
+// most of what is left of such a call, so matmul_q does all of its conversions here instead of in ctypes, and the three calls of routed experts do: through ctypes
+// they took the host 21.5 us where their kernels take 11 - 14, now 16 (1024 x 2048, 2 of 128 experts, one token 22.0 -> 15.8).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
@@ -16,6 +17,9 @@ namespace {
 int (*p_malloc)(void**, size_t) = nullptr;
 int (*p_free)(void*) = nullptr;
 int (*p_matmul_q)(const void*, const void*, size_t, void*, void*) = nullptr;
+int (*p_moe_topk)(const void*, const void*, size_t, size_t, size_t, int, float, int, void*, void*) = nullptr;
+int (*p_swiglu_id)(const void*, const void*, size_t, const void*, size_t, size_t, void*, void*) = nullptr;
+int (*p_id_wsum)(const void*, const void*, size_t, const void*, size_t, size_t, void*, void*, void*) = nullptr;
 PyTypeObject* g_buffer_type = nullptr;
 PyObject* g_value = nullptr;         // "value"
 PyObject* g_c_void_p = nullptr;      // ctypes.c_void_p
@@ -143,6 +147,21 @@ PyType_Slot buffer_slots[] = {
 };
 PyType_Spec buffer_spec = {"ferric_amd._host.DeviceBuffer", sizeof(Buffer), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC, buffer_slots};
 
+// what a ctypes pointer, an address or None stands for
+bool address(PyObject* h, void** out) {
+    *out = nullptr;
+    if (h == Py_None) return true;
+    if (PyLong_Check(h)) {
+        *out = PyLong_AsVoidPtr(h);
+        return !PyErr_Occurred();
+    }
+    PyObject* v = PyObject_GetAttr(h, g_value);
+    if (!v) return false;
+    if (v != Py_None) *out = PyLong_AsVoidPtr(v);
+    Py_DECREF(v);
+    return !PyErr_Occurred();
+}
+
 // matmul_q(x buffer, weight handle, rows, output columns, stream) -> buffer of rows x columns f32: fhip_malloc and fhip_matmul_q.
 // The handle and the stream are ctypes pointers or addresses; the stream may be None. NotImplemented for a buffer of another type: the caller goes through
 // ctypes, which takes whatever `ptr` such an object has.
@@ -151,21 +170,8 @@ PyObject* matmul_q(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!PyObject_TypeCheck(a[0], g_buffer_type)) Py_RETURN_NOTIMPLEMENTED;
     const size_t rows = PyLong_AsSize_t(a[2]), cols = PyLong_AsSize_t(a[3]);
     if (PyErr_Occurred()) return nullptr;
-    void* handle[2] = {nullptr, nullptr};
-    for (int i = 0; i < 2; i++) {
-        PyObject* h = a[i ? 4 : 1];
-        if (h == Py_None) continue;
-        if (PyLong_Check(h)) {
-            handle[i] = PyLong_AsVoidPtr(h);
-            if (PyErr_Occurred()) return nullptr;
-            continue;
-        }
-        PyObject* v = PyObject_GetAttr(h, g_value);
-        if (!v) return nullptr;
-        if (v != Py_None) handle[i] = PyLong_AsVoidPtr(v);
-        Py_DECREF(v);
-        if (PyErr_Occurred()) return nullptr;
-    }
+    void *handle[2];
+    if (!address(a[1], &handle[0]) || !address(a[4], &handle[1])) return nullptr;
     PyObject* nbytes = PyLong_FromSize_t(rows * cols * sizeof(float));
     if (!nbytes) return nullptr;
     Buffer* out = ready() ? nullptr : (Buffer*)g_buffer_type->tp_alloc(g_buffer_type, 0);
@@ -180,6 +186,71 @@ PyObject* matmul_q(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_DECREF(nbytes);
     if (rc) { raise_rc(rc); Py_DECREF(out); return nullptr; }
     return (PyObject*)out;
+}
+
+bool sizes(PyObject* const* a, int n, size_t* out) {
+    for (int i = 0; i < n; i++) {
+        PyObject* whole = PyNumber_Index(a[i]);
+        if (!whole) return false;
+        out[i] = PyLong_AsSize_t(whole);
+        Py_DECREF(whole);
+        if (out[i] == (size_t)-1 && PyErr_Occurred()) return false;
+    }
+    return true;
+}
+// a DeviceBuffer of `floats` that launch(its memory, `scratch` floats more or null) has been enqueued into
+template <class Launch>
+PyObject* result(size_t floats, size_t scratch, Launch launch) {
+    PyObject* nbytes = PyLong_FromSize_t(floats * sizeof(float));
+    if (!nbytes) return nullptr;
+    Buffer* out = ready() ? nullptr : (Buffer*)g_buffer_type->tp_alloc(g_buffer_type, 0);
+    if (!out) { Py_DECREF(nbytes); return nullptr; }
+    void *y = nullptr, *ws = nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = p_malloc(&y, floats * sizeof(float));
+    if (!rc && scratch) rc = p_malloc(&ws, scratch * sizeof(float));
+    if (!rc) rc = launch(y, ws);
+    if (ws) (void)p_free(ws);        // (not handed out again before the device has been idle)
+    Py_END_ALLOW_THREADS
+    if (y) buffer_holds(out, y, nbytes);
+    Py_DECREF(nbytes);
+    if (rc) { raise_rc(rc); Py_DECREF(out); return nullptr; }
+    return (PyObject*)out;
+}
+bool is_buffer(PyObject* o) { return PyObject_TypeCheck(o, g_buffer_type); }
+
+// moe_topk(logits buffer, bias buffer or None, tokens, experts, k, sigmoid, scale, norm, stream) -> buffer of tokens x 2 k; NotImplemented as matmul_q
+PyObject* moe_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 9) { PyErr_SetString(PyExc_TypeError, "moe_topk(logits, bias, tokens, experts, k, sigmoid, scale, norm, stream)"); return nullptr; }
+    if (!is_buffer(a[0]) || (a[1] != Py_None && !is_buffer(a[1]))) Py_RETURN_NOTIMPLEMENTED;
+    size_t d[3];
+    void* stream;
+    const int sigmoid = PyObject_IsTrue(a[5]), norm = PyObject_IsTrue(a[7]);
+    const float scale = (float)PyFloat_AsDouble(a[6]);
+    if (PyErr_Occurred() || !sizes(a + 2, 3, d) || !address(a[8], &stream)) return nullptr;
+    const void *x = ((Buffer*)a[0])->mem, *bias = a[1] == Py_None ? nullptr : ((Buffer*)a[1])->mem;
+    return result(d[0] * 2 * d[2], 0, [&](void* y, void*) { return p_moe_topk(x, bias, d[0], d[1], d[2], sigmoid, scale, norm, y, stream); });
+}
+// swiglu_id(x buffer, weight handle, tokens, selection buffer, k, outputs, stream) -> buffer of tokens x k x outputs
+PyObject* swiglu_id(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 7) { PyErr_SetString(PyExc_TypeError, "swiglu_id(x, handle, tokens, selection, k, outputs, stream)"); return nullptr; }
+    if (!is_buffer(a[0]) || !is_buffer(a[3])) Py_RETURN_NOTIMPLEMENTED;
+    size_t t, d[2];
+    void *w, *stream;
+    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream)) return nullptr;
+    const void *x = ((Buffer*)a[0])->mem, *sel = ((Buffer*)a[3])->mem;
+    return result(t * d[0] * d[1], 0, [&](void* y, void*) { return p_swiglu_id(w, x, t, sel, d[0], d[1], y, stream); });
+}
+// id_wsum(x buffer, weight handle, tokens, selection buffer, k, outputs, stream) -> buffer of tokens x outputs
+PyObject* id_wsum(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 7) { PyErr_SetString(PyExc_TypeError, "id_wsum(x, handle, tokens, selection, k, outputs, stream)"); return nullptr; }
+    if (!is_buffer(a[0]) || !is_buffer(a[3])) Py_RETURN_NOTIMPLEMENTED;
+    size_t t, d[2];
+    void *w, *stream;
+    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream)) return nullptr;
+    const void *x = ((Buffer*)a[0])->mem, *sel = ((Buffer*)a[3])->mem;
+    return result(t * d[1], t * d[0] * d[1], [&](void* y, void* ws) { return p_id_wsum(w, x, t, sel, d[0], d[1], y, ws, stream); });
 }
 
 PyObject* setup(PyObject*, PyObject* args) {
@@ -199,13 +270,19 @@ PyObject* bind(PyObject*, PyObject* args) {
     if (!lib) { PyErr_Format(PyExc_ImportError, "%s", dlerror()); return nullptr; }
     p_free = (int (*)(void*))dlsym(lib, "fhip_free");
     p_matmul_q = (int (*)(const void*, const void*, size_t, void*, void*))dlsym(lib, "fhip_matmul_q");
+    p_moe_topk = (decltype(p_moe_topk))dlsym(lib, "fhip_moe_topk");
+    p_swiglu_id = (decltype(p_swiglu_id))dlsym(lib, "fhip_matmul_q_swiglu_id");
+    p_id_wsum = (decltype(p_id_wsum))dlsym(lib, "fhip_matmul_q_id_wsum");
     p_malloc = (int (*)(void**, size_t))dlsym(lib, "fhip_malloc");
-    if (!p_malloc || !p_free || !p_matmul_q) { p_malloc = nullptr; PyErr_Format(PyExc_ImportError, "%s does not export what it should", path); return nullptr; }
+    if (!p_malloc || !p_free || !p_matmul_q || !p_moe_topk || !p_swiglu_id || !p_id_wsum) { p_malloc = nullptr; PyErr_Format(PyExc_ImportError, "%s does not export what it should", path); return nullptr; }
     Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {{"setup", setup, METH_VARARGS, "setup(first_use, check)"},
                          {"matmul_q", (PyCFunction)(void*)matmul_q, METH_FASTCALL, "matmul_q(x buffer, weight handle, rows, columns, stream)"},
+                         {"moe_topk", (PyCFunction)(void*)moe_topk, METH_FASTCALL, "moe_topk(logits, bias, tokens, experts, k, sigmoid, scale, norm, stream)"},
+                         {"swiglu_id", (PyCFunction)(void*)swiglu_id, METH_FASTCALL, "swiglu_id(x, handle, tokens, selection, k, outputs, stream)"},
+                         {"id_wsum", (PyCFunction)(void*)id_wsum, METH_FASTCALL, "id_wsum(x, handle, tokens, selection, k, outputs, stream)"},
                          {"bind", bind, METH_VARARGS, "bind(library path)"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Device memory objects of ferric_amd.", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -101,6 +101,13 @@ def _upload(buf, a, stream=None):
     _lib.check(_lib.load().fhip_upload(buf.ptr, a.ctypes.data, a.nbytes, _stream_handle(stream)))
 
 
+def _result(buf, shape):
+    """The f32 tensor over a buffer the library has allocated."""
+    t = _new(Tensor)
+    t.shape, t.dtype, t.buf = tuple(map(int, shape)), _F32, buf
+    return t
+
+
 class Tensor:
     """A contiguous row-major device tensor (f32 unless made with from_bf16_bits)."""
 
@@ -271,7 +278,10 @@ class Tensor:
         t, ne = (self.shape[0], self.shape[1]) if len(self.shape) == 2 else (1, self.numel())
         assert 1 <= k <= 8, "k must be 1..=8"
         assert ne <= 1024, "moe_topk: n_expert <= 1024 (single-thread scan)"
-        out = Tensor.empty((t, 2 * k))
+        buf = _lib.moe_topk(self.buf, bias.buf if bias is not None else None, t, ne, k, sigmoid, scale, norm, None if stream is None else stream.handle)
+        if buf is not NotImplemented:
+            return _result(buf, (t, 2 * k))
+        out = Tensor.empty((t, 2 * k))   # tensors over other objects with a `ptr`
         _lib.check(_lib.load().fhip_moe_topk(self.buf.ptr, bias.buf.ptr if bias is not None else None, t, ne, k, int(bool(sigmoid)),
                                              float(scale), int(bool(norm)), out.buf.ptr, _stream_handle(stream)))
         return out
@@ -281,6 +291,9 @@ class Tensor:
         t, inn = self._rows_inner()
         assert inn == w.cols(), f"inner dim mismatch: x[..,{inn}] vs W[..,{w.cols()}]"
         assert 1 <= k <= 8, "k must be 1..=8"
+        buf = _lib.swiglu_id(self.buf, w.handle, t, selw.buf, k, eff, None if stream is None else stream.handle)
+        if buf is not NotImplemented:
+            return _result(buf, (t, k, eff))
         out = Tensor.empty((t, k, eff))
         _lib.check(_lib.load().fhip_matmul_q_swiglu_id(w.handle, self.buf.ptr, t, selw.buf.ptr, k, eff, out.buf.ptr, _stream_handle(stream)))
         return out
@@ -324,6 +337,9 @@ class Tensor:
         t, k, inn = self.shape if len(self.shape) == 3 else (1, self.shape[0], self.shape[1])
         assert 1 <= k <= 8, "k must be 1..=8"
         assert inn == w.cols(), f"inner dim mismatch: x[..,{inn}] vs W[..,{w.cols()}]"
+        buf = _lib.id_wsum(self.buf, w.handle, t, selw.buf, k, out_pe, None if stream is None else stream.handle)
+        if buf is not NotImplemented:
+            return _result(buf, (t, out_pe))
         out = Tensor.empty((t, out_pe))
         ws = Tensor.empty((t * k, out_pe))
         _lib.check(_lib.load().fhip_matmul_q_id_wsum(w.handle, self.buf.ptr, t, selw.buf.ptr, k, out_pe, out.buf.ptr, ws.buf.ptr,

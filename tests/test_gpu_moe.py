@@ -193,3 +193,35 @@ def test_indices_outside_the_slab_are_clamped_and_shapes_are_checked(F, O):
         xt.matmul_q4_k_id_wsum(w, st, 36)
     with pytest.raises(AssertionError, match="k must be"):
         F.Tensor.from_vec(np.zeros(9 * cols, np.float32), (9, cols)).matmul_q4_k_id_wsum(w, st, out_pe)
+
+
+def test_the_calls_convert_what_they_are_given(F):
+    """The three calls of routed experts take their arguments in C: NumPy integers, a stream, tensors over an object that is no DeviceBuffer (through ctypes, the same
+    bits), and the library's refusals as its exceptions."""
+    from ferric_amd.synth import synth_weights
+    rng = np.random.default_rng(3)
+    d, eff, ne, t, k = 512, 256, 4, 3, 2
+    gu = F.QMatrix.from_bytes(synth_weights(12, ne * 2 * eff, d, 1), 12, ne * 2 * eff, d)
+    dn = F.QMatrix.from_bytes(synth_weights(14, ne * d, eff, 2), 14, ne * d, eff)
+    x, logits, bias = (F.Tensor.from_vec(rng.standard_normal(s).astype(np.float32), s) for s in ((t, d), (t, ne), (ne,)))
+
+    class Other:
+        def __init__(self, buf):
+            self.keep, self.ptr, self.nbytes = buf, buf.ptr, buf.nbytes
+    other = lambda a: F.Tensor(Other(a.buf), a.shape)
+    stream = F.Stream()
+    runs = []
+    for wrap, n, s in ((lambda a: a, int, None), (lambda a: a, np.int64, stream), (other, int, None)):
+        sel = wrap(logits).moe_topk(wrap(bias), n(k), True, np.float32(1.5), s)
+        h = wrap(x).matmul_q_swiglu_id(gu, wrap(sel), n(k), n(eff), s)
+        y = wrap(h).matmul_q_id_wsum(dn, wrap(sel), n(d), s)
+        assert sel.shape == (t, 2 * k) and h.shape == (t, k, eff) and y.shape == (t, d) and all(type(v) is int for v in sel.shape + h.shape + y.shape)
+        if s is not None:
+            s.sync() if hasattr(s, "sync") else F._lib.check(F._lib.load().fhip_stream_sync(s.handle))
+        runs.append([a.to_vec().view(np.uint32) for a in (sel, h, y)])
+    for r in runs[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(runs[0], r))
+    with pytest.raises(AssertionError, match="whole number of experts"):
+        x.matmul_q_swiglu_id(gu, sel, k, 250)
+    with pytest.raises(AssertionError):
+        logits.moe_topk(None, 9, False, 1.0)
