@@ -198,18 +198,25 @@ bool sizes(PyObject* const* a, int n, size_t* out) {
     }
     return true;
 }
-// a DeviceBuffer of `floats` that launch(its memory, `scratch` floats more or null) has been enqueued into
+// bytes of a x b x c floats; a size that wraps is refused as the allocation of a Python int that large is
+bool float_bytes(size_t a, size_t b, size_t c, size_t* out) {
+    size_t n;
+    if (!__builtin_mul_overflow(a, b, &n) && !__builtin_mul_overflow(n, c, &n) && !__builtin_mul_overflow(n, sizeof(float), out)) return true;
+    PyErr_SetString(PyExc_OverflowError, "the result's size does not fit a size_t");
+    return false;
+}
+// a DeviceBuffer of `bytes` that launch(its memory, `scratch` bytes more or null) has been enqueued into
 template <class Launch>
-PyObject* result(size_t floats, size_t scratch, Launch launch) {
-    PyObject* nbytes = PyLong_FromSize_t(floats * sizeof(float));
+PyObject* result(size_t bytes, size_t scratch, Launch launch) {
+    PyObject* nbytes = PyLong_FromSize_t(bytes);
     if (!nbytes) return nullptr;
     Buffer* out = ready() ? nullptr : (Buffer*)g_buffer_type->tp_alloc(g_buffer_type, 0);
     if (!out) { Py_DECREF(nbytes); return nullptr; }
     void *y = nullptr, *ws = nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = p_malloc(&y, floats * sizeof(float));
-    if (!rc && scratch) rc = p_malloc(&ws, scratch * sizeof(float));
+    rc = p_malloc(&y, bytes);
+    if (!rc && scratch) rc = p_malloc(&ws, scratch);
     if (!rc) rc = launch(y, ws);
     if (ws) (void)p_free(ws);        // (not handed out again before the device has been idle)
     Py_END_ALLOW_THREADS
@@ -224,33 +231,33 @@ bool is_buffer(PyObject* o) { return PyObject_TypeCheck(o, g_buffer_type); }
 PyObject* moe_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 9) { PyErr_SetString(PyExc_TypeError, "moe_topk(logits, bias, tokens, experts, k, sigmoid, scale, norm, stream)"); return nullptr; }
     if (!is_buffer(a[0]) || (a[1] != Py_None && !is_buffer(a[1]))) Py_RETURN_NOTIMPLEMENTED;
-    size_t d[3];
+    size_t d[3], bytes;
     void* stream;
     const int sigmoid = PyObject_IsTrue(a[5]), norm = PyObject_IsTrue(a[7]);
     const float scale = (float)PyFloat_AsDouble(a[6]);
-    if (PyErr_Occurred() || !sizes(a + 2, 3, d) || !address(a[8], &stream)) return nullptr;
+    if (PyErr_Occurred() || !sizes(a + 2, 3, d) || !address(a[8], &stream) || !float_bytes(d[0], 2, d[2], &bytes)) return nullptr;
     const void *x = ((Buffer*)a[0])->mem, *bias = a[1] == Py_None ? nullptr : ((Buffer*)a[1])->mem;
-    return result(d[0] * 2 * d[2], 0, [&](void* y, void*) { return p_moe_topk(x, bias, d[0], d[1], d[2], sigmoid, scale, norm, y, stream); });
+    return result(bytes, 0, [&](void* y, void*) { return p_moe_topk(x, bias, d[0], d[1], d[2], sigmoid, scale, norm, y, stream); });
 }
 // swiglu_id(x buffer, weight handle, tokens, selection buffer, k, outputs, stream) -> buffer of tokens x k x outputs
 PyObject* swiglu_id(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 7) { PyErr_SetString(PyExc_TypeError, "swiglu_id(x, handle, tokens, selection, k, outputs, stream)"); return nullptr; }
     if (!is_buffer(a[0]) || !is_buffer(a[3])) Py_RETURN_NOTIMPLEMENTED;
-    size_t t, d[2];
+    size_t t, d[2], bytes;
     void *w, *stream;
-    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream)) return nullptr;
+    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream) || !float_bytes(t, d[0], d[1], &bytes)) return nullptr;
     const void *x = ((Buffer*)a[0])->mem, *sel = ((Buffer*)a[3])->mem;
-    return result(t * d[0] * d[1], 0, [&](void* y, void*) { return p_swiglu_id(w, x, t, sel, d[0], d[1], y, stream); });
+    return result(bytes, 0, [&](void* y, void*) { return p_swiglu_id(w, x, t, sel, d[0], d[1], y, stream); });
 }
 // id_wsum(x buffer, weight handle, tokens, selection buffer, k, outputs, stream) -> buffer of tokens x outputs
 PyObject* id_wsum(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 7) { PyErr_SetString(PyExc_TypeError, "id_wsum(x, handle, tokens, selection, k, outputs, stream)"); return nullptr; }
     if (!is_buffer(a[0]) || !is_buffer(a[3])) Py_RETURN_NOTIMPLEMENTED;
-    size_t t, d[2];
+    size_t t, d[2], bytes, scratch;
     void *w, *stream;
-    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream)) return nullptr;
+    if (!sizes(a + 2, 1, &t) || !sizes(a + 4, 2, d) || !address(a[1], &w) || !address(a[6], &stream) || !float_bytes(t, 1, d[1], &bytes) || !float_bytes(t, d[0], d[1], &scratch)) return nullptr;
     const void *x = ((Buffer*)a[0])->mem, *sel = ((Buffer*)a[3])->mem;
-    return result(t * d[1], t * d[0] * d[1], [&](void* y, void* ws) { return p_id_wsum(w, x, t, sel, d[0], d[1], y, ws, stream); });
+    return result(bytes, scratch, [&](void* y, void* ws) { return p_id_wsum(w, x, t, sel, d[0], d[1], y, ws, stream); });
 }
 
 PyObject* setup(PyObject*, PyObject* args) {

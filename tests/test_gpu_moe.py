@@ -225,3 +225,7 @@ def test_the_calls_convert_what_they_are_given(F):
         x.matmul_q_swiglu_id(gu, sel, k, 250)
     with pytest.raises(AssertionError):
         logits.moe_topk(None, 9, False, 1.0)
+    with pytest.raises(OverflowError):       # twice this many rows, and the bytes of this many outputs, wrap to sizes that exist
+        x.matmul_q_swiglu_id(gu, sel, k, 2 ** 63 + eff)
+    with pytest.raises(OverflowError):
+        h.matmul_q_id_wsum(dn, sel, 2 ** 62 + d)
