@@ -91,6 +91,12 @@ constexpr int LDS_ROW = KSTEP + 8;   // bf16 per staged activation row (+16 B pa
 // operands and every format: sub-block (t >> 1) of the step, elements 16h + 8(t & 1) + [0, 8).
 __device__ __forceinline__ constexpr int kcol(int t, int h) { return 32 * (t >> 1) + 16 * h + 8 * (t & 1); }
 
+// The elements of X (the launcher checks that T * K fits 31 bits) a thread stages: x_piece(t, T, K, col) + x_step(first, col, K) on, for columns first + col ... + 7 of
+// row t. A row past T is row T - 1 (its outputs are not stored); columns past K (of a partial last chunk, staged as zeros) are read from earlier ones of the
+// same row, whose end may be the end of mapped memory: nothing behind X is read.
+__host__ __device__ constexpr uint32_t x_piece(int t, int T, int K, int col) { return (uint32_t)(t < T ? t : T - 1) * (uint32_t)K + (uint32_t)(col < K ? col : K - 8); }
+__host__ __device__ constexpr int x_step(int first, int col, int K) { return first + col < K ? first : 0; }
+
 
 // ------------------------------------------------------------------------------------------------
 // Per-format weight streams. `Raw` is the per-lane register image of one chunk of one weight row (the
@@ -466,18 +472,18 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_kernel(GemmParams p) {
     // (tid >> 3) + 64q, q < MI. Rows past T are read from row T-1 (their outputs are never stored); columns
     // past K (a partial last chunk) are staged as zeros.
     const int a_col = (tid & 7) * 8;
-    uint32_t a_src[MI];   // element offsets into X (the launcher checks T*K fits 31 bits)
+    uint32_t a_src[MI];
 #pragma unroll
     for (int q = 0; q < MI; q++) {
         int t = tile_y * BM + (tid >> 3) + 64 * q;
-        a_src[q] = (uint32_t)(t < p.T ? t : p.T - 1) * (uint32_t)p.K + a_col;
+        a_src[q] = x_piece(t, p.T, p.K, a_col);
     }
     const int a_dst = (tid >> 3) * LDS_ROW + a_col;
     u32x4 stage[MI];
     auto load_a = [&](int s) {   // s = absolute step index (64 columns each)
         if constexpr (F::PARTIAL) {
             const bool ok = s * KSTEP + a_col < p.K;
-            const int off = ok ? s * KSTEP : 0;
+            const int off = x_step(s * KSTEP, a_col, p.K);
             const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
 #pragma unroll
             for (int q = 0; q < MI; q++) {
@@ -688,14 +694,14 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
             const int t = tile_y * BM + (sl >> 3) + RSTEP * q;
-            a_src[q] = (uint32_t)(t < p.T ? t : p.T - 1) * (uint32_t)p.K + a_col;
+            a_src[q] = x_piece(t, p.T, p.K, a_col);
         }
     }
     const int a_dst = (sl >> 3) * LDS_ROW + a_col;              // + RSTEP q LDS_ROW
     auto load_a = [&](int s) {
         if constexpr (F::PARTIAL) {
             const bool ok = s * KSTEP + a_col < p.K;
-            const int off = ok ? s * KSTEP : 0;
+            const int off = x_step(s * KSTEP, a_col, p.K);
             const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
 #pragma unroll
             for (int q = 0; q < NQ; q++)
@@ -1126,7 +1132,7 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
     for (int q = 0; q < NQ; q++) {
         int t = (tid >> 5) + RQ * q;
         t = t0 + (t < BM ? t : BM - 1);
-        a_src[q] = (uint32_t)(t < p.T ? t : p.T - 1) * (uint32_t)p.K + a_col;
+        a_src[q] = x_piece(t, p.T, p.K, a_col);
     }
     const int a_dst = (tid >> 5) * XROW + a_col;
     // a last round of fewer rows: the threads past it write the tile's last row again, with what it holds
@@ -1134,7 +1140,7 @@ __global__ void __launch_bounds__(64 * NW * KW) gemm_q_bf16_own_kernel(GemmParam
     u32x4 stage[NQ];
     auto load_a = [&](int ck, int q) {
         const bool ok = !FMT::PARTIAL || ck * CHUNK + a_col < p.K;
-        stage[q] = *(const u32x4*)(p.X + (a_src[q] + (ok ? ck * CHUNK : 0)));
+        stage[q] = *(const u32x4*)(p.X + (a_src[q] + (FMT::PARTIAL ? x_step(ck * CHUNK, a_col, p.K) : ck * CHUNK)));
         if (FMT::PARTIAL) {
             const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
             stage[q] = (u32x4){stage[q][0] & keep, stage[q][1] & keep, stage[q][2] & keep, stage[q][3] & keep};

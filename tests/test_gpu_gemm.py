@@ -94,6 +94,23 @@ def test_tiles_whose_waves_unpack_for_themselves(F, O, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
+@pytest.mark.parametrize("tile", range(-1, 12))
+def test_rows_shorter_than_a_chunk(F, O, tile):
+    # Q8_0 rows of one to seven blocks, one short of a chunk of 256 columns: what lies behind a row is staged as zeros, behind the last one too.
+    lib = F._lib.load()
+    before = lib.fhip_debug_gemm_tile(tile)
+    try:
+        for i, (t, n, k) in enumerate([(33, 65, 32), (64, 320, 64), (65, 130, 96), (128, 257, 160), (300, 100, 224)]):
+            from ferric_amd.synth import synth_weights
+            w = synth_weights(Q8_0, n, k, 900 + i)
+            xb, xv = bf16_round(np.random.default_rng(i).standard_normal((t, k)).astype(np.float32))
+            y = F.Tensor.from_bf16_bits(xb, (t, k)).gemm_q_bf16(F.QMatrix.from_bytes(w, Q8_0, n, k)).to_vec().reshape(t, n)
+            want = xv.astype(np.float64) @ bf16_round(O.deq_raw(w, n * k, Q8_0).reshape(n, k))[1].astype(np.float64).T
+            assert np.abs(y - want).max() < 2e-5 * np.abs(want).max(), (t, n, k)      # f32 sums of bf16 products
+    finally:
+        lib.fhip_debug_gemm_tile(before)
+
+
 @pytest.mark.parametrize("ty", [Q4_K, Q5_K, Q6_K, Q8_0])
 def test_run_sums_add_in_the_order_of_one_accumulator(F, ty):
     # fhip_gemm_q_bf16_run_sums: the tiles whose waves unpack for themselves, one wave along K, have the bits of the tiles that share the
