@@ -44,7 +44,6 @@
 #include "common.hpp"
 #include "prompt.hpp"
 
-#include <limits.h>
 #include <math.h>
 
 namespace {
@@ -287,18 +286,20 @@ __device__ __forceinline__ float largest(float top, const f32x4 (&acc)[ND]) {
     return top;
 }
 
-// The key tiles kt_lo .. kt_hi that the query rows wg_first .. wg_last see, in n ranges of per (the last one's may be fewer; none is empty, since (n - 1) per <=
-// (n - 1) * most < the count).
-struct KeyRanges { int kt_lo, kt_hi, n, per; };
-__host__ __device__ inline KeyRanges key_ranges(int off, int wg_first, int wg_last, int window, int most) {
-    KeyRanges k;
-    k.kt_hi = (off + wg_last) / 32;
+// The key tiles that the query rows wg_first .. wg_last see, at least one.
+struct KeyTiles {
+    int lo, hi;
+    __host__ __device__ int count() const { return hi - lo + 1; }
+};
+__host__ __device__ inline KeyTiles key_tiles(int off, int wg_first, int wg_last, int window) {
     const int first = off + wg_first - window + 1;
-    k.kt_lo = window > 0 && first > 0 ? first / 32 : 0;
-    const int count = k.kt_hi - k.kt_lo + 1;
-    k.n = (count + most - 1) / most;
-    k.per = (count + k.n - 1) / k.n;
-    return k;
+    return {window > 0 && first > 0 ? first / 32 : 0, (off + wg_last) / 32};
+}
+// Of `count` tiles, n ranges of per (the last one's may be fewer; none is empty, since (n - 1) per <= (n - 1) * most < the count).
+struct KeyRanges { int n, per; };
+__host__ __device__ inline KeyRanges key_ranges(int count, int most) {
+    const int n = (count - 1) / most + 1;
+    return {n, (count - 1) / n + 1};
 }
 // What a wave hands over of its 16 rows and one range of keys: [HD / 16][64] accumulators as its lanes hold them, [16] largest scores (NaN: these rows are
 // the f32 body's), [16] sums of weights.
@@ -330,10 +331,14 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attn_cut_kernel(const float
     const bool wave_live = i0 < T;
     const int i_last = min(i0 + 15, T - 1);
     const int i = min(i0 + c, T - 1), qpos = off + i;
-    const KeyRanges kr = key_ranges(off, wg_first, wg_last, window, SPLIT ? most : INT_MAX);
-    if (SPLIT && (int)blockIdx.z >= kr.n) return;
-    const int kt_lo = SPLIT ? kr.kt_lo + (int)blockIdx.z * kr.per : kr.kt_lo;
-    const int kt_hi = SPLIT ? min(kr.kt_hi, kt_lo + kr.per - 1) : kr.kt_hi;
+    const KeyTiles seen = key_tiles(off, wg_first, wg_last, window);
+    int kt_lo = seen.lo, kt_hi = seen.hi;
+    if constexpr (SPLIT) {
+        const KeyRanges kr = key_ranges(seen.count(), most);
+        if ((int)blockIdx.z >= kr.n) return;
+        kt_lo += (int)blockIdx.z * kr.per;
+        kt_hi = min(kt_hi, kt_lo + kr.per - 1);
+    }
     const int my_hi = wave_live ? (off + i_last) / 32 : -1;
     const int my_lo = window > 0 ? max(0, off + i0 - window + 1) / 32 : 0;
 
@@ -501,9 +506,10 @@ __global__ __launch_bounds__(64) void causal_attn_join_kernel(const float* __res
     const int lane = threadIdx.x, c = lane & 15, ks = lane >> 4;
     const int head = blockIdx.x, tile = (int)gridDim.y - 1 - (int)blockIdx.y, i0 = 16 * tile, off = S - T;   // the f32 body numbers its rows the same way
     const int wg_first = i0 / (16 * CUT_WAVES) * (16 * CUT_WAVES), wg_last = min(T - 1, wg_first + 16 * CUT_WAVES - 1);
-    const KeyRanges kr = key_ranges(off, wg_first, wg_last, window, most);
+    const KeyTiles seen = key_tiles(off, wg_first, wg_last, window);
+    const KeyRanges kr = key_ranges(seen.count(), most);
     const int my_hi = (off + min(i0 + 15, T - 1)) / 32, my_lo = window > 0 ? max(0, off + i0 - window + 1) / 32 : 0;
-    const int j_lo = (my_lo - kr.kt_lo) / kr.per, j_hi = (my_hi - kr.kt_lo) / kr.per;
+    const int j_lo = (my_lo - seen.lo) / kr.per, j_hi = (my_hi - seen.lo) / kr.per;
     const float* slot = part + ((size_t)head * gridDim.y + tile) * slots * part_floats(HD);
     float m = -3.0e38f;
     bool bad = false;
@@ -570,10 +576,7 @@ static CausalSplit causal_split(size_t t, size_t s, size_t n_head, size_t hd, in
     const size_t cus = device_cus() > 0 ? device_cus() : 256, blocks = (t + ROWS - 1) / ROWS, groups = blocks * n_head;
     if (groups > 2 * cus) return {};
     const int off = (int)(s - t);
-    auto tiles = [&](size_t b) {
-        const KeyRanges k = key_ranges(off, (int)(b * ROWS), (int)((b + 1) * ROWS < t ? (b + 1) * ROWS : t) - 1, win, INT_MAX);
-        return k.kt_hi - k.kt_lo + 1;
-    };
+    auto tiles = [&](size_t b) { return key_tiles(off, (int)(b * ROWS), (int)((b + 1) * ROWS < t ? (b + 1) * ROWS : t) - 1, win).count(); };
     size_t total = 0;
     int longest = 0;
     for (size_t b = 0; b < blocks; b++) {

@@ -8,18 +8,30 @@ import pytest
 from conftest import ROOT
 
 
-def build(d, harness, *flags):
-    """tests/<harness> as a shared object."""
-    obj, so = str(d / (harness + ".o")), str(d / (harness + ".so"))
+def build(d, harness, flags, link):
+    """tests/<harness> as a program or a shared object."""
+    obj, out = str(d / (harness + ".o")), str(d / (harness + ".so"))
     subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "--offload-arch=gfx950", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-fuse-cuid=none",
                     *flags, "-c", os.path.join(ROOT, "tests", harness), "-o", obj], check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
-    subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", so, obj], check=True)
-    return C.CDLL(so)
+    subprocess.run(["g++", *link, "-o", out, obj], check=True)
+    return out
 
 
 @pytest.fixture(scope="module")
 def gemm(tmp_path_factory):
-    return build(tmp_path_factory.mktemp("gemm"), "gemm_rules_harness.cpp", "-DFHIP_GEMM_FORMAT=Q80")
+    return C.CDLL(build(tmp_path_factory.mktemp("gemm"), "gemm_rules_harness.cpp", ["-DFHIP_GEMM_FORMAT=Q80"], ["-shared", "-Wl,-Bsymbolic"]))
+
+
+@pytest.fixture(scope="module")
+def attention(tmp_path_factory):
+    """[(rows, keys, heads, head size, window)] -> [(most key tiles of a range, ranges)]"""
+    program = build(tmp_path_factory.mktemp("attn"), "attn_rules_harness.cpp", ["-Xarch_host", "-fsanitize=undefined", "-Xarch_host", "-fsanitize-trap=undefined"], [])
+
+    def ask(shapes):
+        r = subprocess.run([program], input="".join("%d %d %d %d %d\n" % x for x in shapes), capture_output=True, text=True)
+        assert r.returncode == 0, (r.returncode, shapes[len(r.stdout.splitlines())])
+        return [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
+    return ask
 
 
 @pytest.mark.parametrize("width", [64, 256])      # columns of a step (unpacked weights shared) and of a chunk (waves that unpack for themselves)
@@ -34,3 +46,12 @@ def test_no_activation_is_read_from_behind_the_last(gemm, width):
                         at = gemm.h_x_at(t, T, K, first, col)
                         assert at % 8 == 0 and at + 8 <= T * K, (K, T, t, first, col)
                         assert at // K == min(t, T - 1) and (first + col >= K or at % K == first + col), (K, T, t, first, col)
+
+
+def test_key_ranges_of_a_query_block(attention):
+    """Causal attention, one piece or split: ragged rows, keys and windows, the smallest and the largest; the program checks every block's ranges."""
+    rows, behind, windows = (1, 15, 16, 17, 63, 64, 65, 95, 509, 1000), (0, 1, 31, 32, 64, 300, 8191, 1 << 20), (0, 1, 31, 32, 33, 64, 500)
+    shapes = [(t, t + b, heads, hd, w) for t in rows for b in behind for w in windows for heads, hd in ((1, 64), (8, 128), (40, 128))]
+    shapes += [(33, 0x3FFFFFFF, 1, 64, 0), (33, 0x3FFFFFFF, 1, 64, 4096), (0x3FFFFF, 0x3FFFFF, 1, 128, 0)]
+    got = attention(shapes)
+    assert len(got) == len(shapes) and all(most == 0 or 2 <= most and ranges <= 32 for most, ranges in got)
