@@ -560,14 +560,18 @@ static int waves_of(size_t t, size_t n_head) {
 // Ranges of at most `most` key tiles, at most `slots` of them a query block; most = 0: the keys stay in one piece.
 // A workgroup takes 2.15 us a tile of 64 rows at head size 128 and 1.3 at 64, and a CU's workgroups together 1.95 and 1.0, so a launch of one workgroup a CU or fewer
 // lasts as long as the block with the most tiles, one of up to two a CU as long as that block and the shortest that lies beside it. Ranges cost 4 us (the
-// join's launch) and a seventh (their starts, the partial results' way through memory) and level the CUs' shares. The best size is 0.6 of a CU's share, two at least; it is flat around
+// join's launch) and a seventh, three tenths at head size 128 (their starts, the partial results' way through memory), and level the CUs' shares; where they are more
+// than two a CU, a quarter of a range more, for the CUs that are left with one. The best size is 0.6 of a CU's share, two at least; it is flat around
 // that and from 14 on, where the share, not the last workgroup, counts. us, one piece | ranges of 2, 3, 4, 6, 8, 14, 18 tiles (rows x keys, heads, KV heads, head size):
 //   95 x 722, 8, 8, 128     54.4 | 14.2  15.4  16.8  20.7  25.3  32.2        377 x 954, 8, 4, 64     46.0 | 16.3  15.1  16.0  15.5  17.7  26.0  27.5
 //   33 x 1057, 4, 4, 128    78.1 | 16.5  16.7  17.9  21.3  23.2  33.5  44.0  152 x 940, 8, 8, 64     44.9 | 13.5  12.4  12.9  14.7  17.5  25.8  27.0
 //   234 x 355, 32, 4, 128   31.4 | 24.6  21.0  21.9  22.1  26.3              65 x 600, 64, 8, 64     31.5 | 19.6  18.4  17.9  17.2  18.5  20.6  20.7
 //   1024 x 1024, 8, 4, 128  77.4 | 40.6  36.5  35.4  30.1  35.1  41.9  48.4  700 x 1200, 24, 8, 64   59.4 | 52.7  43.7  41.6  39.0  38.9  39.3  44.2
 //   509 x 809, 40, 8, 128   71.9 | 82.3  68.8  63.5  63.0  58.8  59.8  56.8  1024 x 2048, 16, 4, 64  94.5 | 80.2  67.1  62.1  59.4  58.2  55.7  59.0
-// and not split: 77 x 77, 40 heads of 128 7.2 | 8.9  9.5, 205 x 205, 64 of 64 12.6 | 13.6  13.6  13.3  15.3, 1024 x 1024, 40 of 128 (640 workgroups) 85.6 | 139  119  110  101  97.8  95.6  97.6.
+// Over 520 shapes (33 ... 1024 rows behind 0 ... 1024 keys, 4 ... 64 heads, with and without a window) 306 are split, to 0.63 of the time on average and at
+// most to 1.00 (of 500 others 320, to 0.58, none slower); before the ranges' share at head size 128, the late ranges and blocks no longer than one range were counted, 319 were, up to 1.27 of the time:
+// 390 x 451, 64 heads of 128 42.0 | 53.4; 655 x 655, 40 of 128 53.7 | 57.5; 834 x 870, 32 of 128, window 433 52.9 | 59.5. Not split before
+// either: 77 x 77, 40 heads of 128 7.2 | 8.9  9.5, 205 x 205, 64 of 64 12.6 | 13.6  13.6  13.3  15.3, 1024 x 1024, 40 of 128 (640 workgroups) 85.6 | 139  119  110  101  97.8  95.6  97.6.
 struct CausalSplit { int most = 0, slots = 0; };
 static CausalSplit causal_split(size_t t, size_t s, size_t n_head, size_t hd, int win) {
     constexpr size_t ROWS = 16 * CUT_WAVES;
@@ -589,13 +593,17 @@ static CausalSplit causal_split(size_t t, size_t s, size_t n_head, size_t hd, in
     int most = share <= 24.f ? (int)ceilf(0.6f * share) : (int)fmaxf(14.f, share / 4);
     most = most < 2 ? 2 : most;
     most = most * RANGES < longest ? (longest + RANGES - 1) / RANGES : most;
-    for (int m = most; m <= most + most / 4; m++) {      // a little longer where all of them then start at once (509 x 809: 15 tiles 62.5, 18 57)
-        size_t units = 0;
-        for (size_t b = 0; b < blocks; b++) units += (tiles(b) + m - 1) / m * n_head;
-        if (units <= 2 * cus) { most = m; break; }
-    }
+    auto units = [&](int m) {
+        size_t n = 0;
+        for (size_t b = 0; b < blocks; b++) n += (tiles(b) + m - 1) / m * n_head;
+        return n;
+    };
+    for (int m = most; m <= most + most / 4; m++)        // a little longer where all of them then start at once (509 x 809: 15 tiles 62.5, 18 57)
+        if (units(m) <= 2 * cus) { most = m; break; }
+    if (most >= longest) return {};
     const float whole = groups <= cus ? one * longest : both * (longest + tiles(blocks - 1 - cus / n_head));   // blocks go out last first, all heads of each
-    if (whole <= 4.f + fmaxf(one * (most < longest ? most : longest), 1.15f * both * share)) return {};
+    const float late = units(most) > 2 * cus ? 0.25f * one * most : 0.f;
+    if (whole <= 4.f + fmaxf(one * most, (hd == 128 ? 1.3f : 1.15f) * both * share) + late) return {};
     return {most, (longest + most - 1) / most};
 }
 

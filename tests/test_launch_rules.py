@@ -55,3 +55,13 @@ def test_key_ranges_of_a_query_block(attention):
     shapes += [(33, 0x3FFFFFFF, 1, 64, 0), (33, 0x3FFFFFFF, 1, 64, 4096), (0x3FFFFF, 0x3FFFFF, 1, 128, 0)]
     got = attention(shapes)
     assert len(got) == len(shapes) and all(most == 0 or 2 <= most and ranges <= 32 for most, ranges in got)
+
+
+def test_keys_are_split_where_that_is_faster(attention):
+    """Both sides timed on 256 CUs: us in one piece, us split."""
+    timed = {(390, 451, 64, 128, 0): (42.0, 53.4), (834, 870, 32, 128, 433): (52.9, 59.5), (750, 978, 32, 64, 337): (32.4, 36.3), (655, 655, 40, 128, 0): (53.7, 57.5),
+             (628, 735, 40, 128, 0): (60.7, 64.3), (341, 341, 64, 128, 0): (31.9, 32.9), (719, 1125, 40, 64, 0): (59.4, 60.1), (205, 205, 64, 64, 0): (12.6, 13.3),
+             (95, 722, 8, 128, 0): (54.4, 14.2), (509, 809, 40, 128, 0): (71.9, 56.8), (751, 751, 32, 128, 0): (60.6, 50.4), (923, 1395, 20, 64, 0): (66.6, 47.0),
+             (130, 176, 40, 128, 0): (18.3, 15.6), (767, 767, 16, 64, 261): (20.4, 17.7), (589, 1561, 40, 64, 0): (80.0, 69.1), (406, 406, 40, 128, 0): (34.3, 32.8)}
+    for (shape, (whole, split)), (most, _) in zip(timed.items(), attention(list(timed))):
+        assert (most > 0) == (split < whole), shape
