@@ -225,7 +225,7 @@ struct Q6K {
     // whose scale is sc[8hf + 2g + h]  (crates/ferric-gguf/src/lib.rs:833-851).
     static constexpr int BLOCK = 210;
     static constexpr float UNPACK_US = 2.3f;
-    static constexpr float CHUNK_US[NTILES] = {4.15f, 5.47f, 8.75f, 5.95f, 2.78f, 2.03f, 4.40f, 2.43f, 1.76f, 2.52f, 1.37f, 1.75f};
+    static constexpr float CHUNK_US[NTILES] = {3.67f, 5.11f, 8.61f, 5.92f, 2.70f, 1.89f, 4.48f, 2.80f, 1.70f, 2.39f, 1.32f, 1.70f};
     static constexpr float RUN_CHUNK_US[7] = {5.93f, 6.83f, 9.84f, 6.27f, 4.68f, 3.95f, 4.35f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
@@ -1636,8 +1636,10 @@ static long long plan_segments(const TilePlan& q) { return q.runs + (q.left - 1)
 // A linear model fitted (non-negative least squares on relative errors, 7 % rms) to 3700 launches: 357 weights of the four formats, 1024 ... 34816 rows
 // of 1024 ... 17408 columns, 33 ... 2048 activation rows, every tile. On those the tile it picks is 1.4 % slower than the measured best on average
 // (worst 25 %); the model it replaced, fitted to ten large weights, and the seven tiles it had were 20 % slower on average and up to 2.7 times
-// (6112 x 2816 Q4_K at 132 rows 42.0 -> 16.6 us). Q6_K's and Q8_0's chunks were fitted again when their rows came to be turned: 136 launches a tile, the pick 1.6 and
-// 2.2 % slower than the best on average (4.1 and 8.7 with the figures before). Left out, a tile costs 0.1 % (64 x 256, 64 x 160) to 2.5 % (64 x 64) of the mean.
+// (6112 x 2816 Q4_K at 132 rows 42.0 -> 16.6 us). Q6_K's and Q8_0's chunks were fitted again when their rows came to be turned, Q8_0's to 136
+// launches a tile, Q6_K's to 350: fitted to 136 they priced 128 x 96 too low, and of 350 weights the pick was 3.0 % slower than the best on average and up to 1.30 times
+// as slow as the model before (2480 x 9984 at 215 rows 34.8 -> 45.2 us); 1.8 % and 1.11 times now, where Q4_K, Q5_K and Q8_0 have 1.4, 1.8 and 1.3 % and at most 1.08 times. On
+// those 1400 launches 64 x 256 is the pick of 3 %, which take 7 % longer without it, 64 x 160 of 4 % and 5 %, 64 x 64 of 22 % and 14 %; 128 x 96 of 3 %, to no gain.
 constexpr float START_US[NTILES] = {3.77f, 3.88f, 4.04f, 4.53f, 3.92f, 3.12f, 4.91f, 3.57f, 2.73f, 4.01f, 2.31f, 3.95f}, FIX_US = 3.29f, SLOT_US = 4.18f, CUT_US = 0.1f;
 template <class F>
 static float plan_cost_us(const TilePlan& q, long long cus) {
