@@ -804,10 +804,12 @@ size_t fhip_workspace_bytes_coop(const fhip_weight* w, const fhip_weight* down, 
         for (size_t n : {fhip::gemm_bf16_ws_bytes(w, t), fhip::gemm_bf16_ws_bytes(down, t), fhip::gemm_bf16_swiglu_ws_bytes(w, t), fhip::gemm_bf16_ws_bytes(w, t, true),
                          fhip::gemm_bf16_ws_bytes(down, t, true)}) need = n > need ? n : need;
     };
-    most(rows_x);
-    if (rows_x > 8) most(8);
-    if (rows_x > 32) most(32);
-    for (size_t t = 64; t < rows_x; t += 64) most(t);
+    auto rows_of = [](const fhip_weight* q) { return q && q->cols ? (((size_t)1 << 31) - 1) / q->cols : (size_t)0; };   // launch_gemm_bf16 refuses more
+    const size_t a = rows_of(w), b = rows_of(down), accepted = a > b ? a : b, last = rows_x < accepted ? rows_x : accepted;
+    most(last);
+    if (last > 8) most(8);
+    if (last > 32) most(32);
+    for (size_t t = 64; t < last; t += 64) most(t);
     return need;
 }
 

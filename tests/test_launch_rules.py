@@ -93,3 +93,21 @@ def test_the_tile_of_a_prompt_product(gemm):
         (Q8_0, 2384, 2816, 239): (25.2, 23.6, 32.8, 26.6, 25.0, 21.3, 29.8, 23.8, 20.6, 22.5, 19.0, 21.4)}
     for shape, us in timed.items():
         assert us[plan(gemm, *shape)[0]] <= 1.25 * min(us), shape
+
+
+class Weight(C.Structure):
+    """struct fhip_weight (ferric_amd/csrc/common.hpp), for a query that reads its type and shape."""
+    _fields_ = [("type", C.c_uint32), ("rows", C.c_size_t), ("cols", C.c_size_t), ("row_bytes", C.c_size_t), ("nbytes", C.c_size_t), ("d_raw", C.c_void_p), ("owns", C.c_bool),
+                ("planes", C.c_int), ("batch_policy", C.c_int)]
+
+
+@pytest.mark.parametrize("ty,rows,cols", [(Q4_K, 5120, 5120), (Q6_K, 5120, 17408), (Q8_0, 1283, 4064)])
+def test_workspace_of_every_batch_a_launch_accepts(ty, rows, cols):
+    """What batches of up to that many rows need at most: never less for more rows, and no more behind the largest batch that a launch accepts."""
+    from ferric_amd import _lib
+    lib, w = _lib.load(), Weight(ty, rows, cols)
+    ask = lambda t: lib.fhip_workspace_bytes_coop(C.addressof(w), None, t)
+    sizes = [ask(t) for t in (0, 1, 8, 9, 32, 33, 64, 65, 100, 509, 512, 1000, 2048, 4096)]
+    assert sizes[0] == 0 and sizes == sorted(sizes) and sizes[-1] > 0
+    accepted = (2 ** 31 - 1) // cols
+    assert ask(accepted) == ask(accepted + 1) == ask(2 ** 64 - 64) == ask(2 ** 64 - 1) >= sizes[-1]
