@@ -225,7 +225,7 @@ int fhip_ffn(const fhip_weight* gate_up, const fhip_weight* down, const float* d
  * output tiles along K keeps their partial tiles in the library's workspace of the stream (fhip_workspace_bytes_coop)
  * and adds them in a fixed order: the same inputs give the same bits on every run. */
 int fhip_gemm_q_bf16(const fhip_weight* w, const uint16_t* d_x_bf16, size_t t, float* d_y, void* stream);
-/* The same with every output's products added in an order that stays from version to version: for rows whose last bits are stored further on, as
+/* The same with every output's products added in an order that stays from version to version (and follows the number of CUs): for rows whose last bits are stored further on, as
  * the codes of a block-quantized cache. Up to 32 rows the same bits; above, last bits may differ from fhip_gemm_q_bf16's, which adds in the order that is fastest. */
 int fhip_gemm_q_bf16_run_sums(const fhip_weight* w, const uint16_t* d_x_bf16, size_t t, float* d_y, void* stream);
 

@@ -131,6 +131,54 @@ def test_run_sums_add_in_the_order_of_one_accumulator(F, ty):
         assert np.array_equal(y.to_vec().view(np.uint32), want.view(np.uint32)), (ty, t)
 
 
+# format, rows, outputs, columns and the CRC-32 of what the launches before waves unpacked for themselves made of these weights and activations: every tile of
+# run sums, whole and cut along K, runs of one to seven chunks, a run that ends in the next tile, whole tiles in front of cut ones, Q8_0 rows that end inside a chunk, up to 32 rows
+RUN_SUMS = [(Q6_K, 33, 2049, 5120, 0x91abb157), (Q6_K, 65, 9000, 1280, 0x4638172c), (Q5_K, 520, 4100, 2304, 0xc744183b),
+            (Q4_K, 129, 4100, 1280, 0x9ad97f0c), (Q8_0, 128, 9000, 736, 0x3eee9c02), (Q8_0, 40, 5120, 512, 0x8a60427a),
+            (Q4_K, 300, 7000, 256, 0x728fff2a), (Q5_K, 300, 7000, 1280, 0x20469f5f), (Q4_K, 300, 1283, 512, 0xbb42321c),
+            (Q6_K, 300, 2049, 5120, 0xea8fa64e), (Q6_K, 65, 700, 1792, 0x617b63db), (Q8_0, 64, 2049, 2080, 0x51921f06),
+            (Q8_0, 257, 9000, 512, 0xebb4198c), (Q5_K, 40, 9000, 512, 0xe2e70568), (Q4_K, 33, 7000, 2304, 0xcf249f68),
+            (Q5_K, 257, 7000, 1792, 0x0a1e6c7c), (Q4_K, 100, 7000, 256, 0x1a419dc0), (Q8_0, 33, 1283, 4064, 0x08c261e7),
+            (Q8_0, 64, 5120, 1312, 0x6aa96d04), (Q6_K, 64, 7000, 3328, 0xc9da5679), (Q6_K, 300, 5120, 1280, 0xf4d32ad6),
+            (Q4_K, 20, 700, 768, 0xeb2b6df8)]
+# formats of gate|up and down, rows, width, inner width, CRC-32 of gate|up and of the result
+FFN_RUN_SUMS = [(Q4_K, Q6_K, 65, 512, 768, 0x0b67cb61, 0x0b3ad60d),
+                (Q6_K, Q8_0, 200, 1280, 1312, 0x3b0411ae, 0x4f7554bb),
+                (Q5_K, Q4_K, 520, 768, 2304, 0x7c3c39a0, 0x61ed940b),
+                (Q4_K, Q8_0, 20, 512, 416, 0xe0c0b31a, 0x9d893b69)]
+
+
+@pytest.mark.parametrize("i", range(len(RUN_SUMS)))
+def test_run_sums_keep_their_bits(F, O, i):
+    import zlib
+    from ferric_amd.synth import synth_weights
+    ty, t, n, k, crc = RUN_SUMS[i]
+    w = synth_weights(ty, n, k, 20 + i)
+    xb, xv = bf16_round(np.random.default_rng(40 + i).standard_normal((t, k)))
+    qm, x, y = F.QMatrix.from_bytes(w, ty, n, k), F.Tensor.from_bf16_bits(xb, (t, k)), F.Tensor.empty((t, n))
+    F._lib.check(F._lib.load().fhip_gemm_q_bf16_run_sums(qm.handle, x.buf.ptr, t, y.buf.ptr, None))
+    got = y.to_vec().reshape(t, n)
+    want = xv.astype(np.float64) @ bf16_round(O.deq_raw(w, n * k, ty).reshape(n, k))[1].astype(np.float64).T
+    assert np.abs(got - want).max() < 2e-5 * np.abs(want).max()       # f32 sums of bf16 products
+    assert zlib.crc32(got.tobytes()) == crc
+
+
+@pytest.mark.parametrize("i", range(len(FFN_RUN_SUMS)))
+def test_ffn_run_sums_keep_their_bits(F, i):
+    import zlib
+    from ferric_amd.synth import synth_weights
+    lib, (tg, td, t, d, ff, crc_gate_up, crc) = F._lib.load(), FFN_RUN_SUMS[i]
+    gu = F.QMatrix.from_bytes(synth_weights(tg, 2 * ff, d, 60 + i), tg, 2 * ff, d)
+    dn = F.QMatrix.from_bytes(synth_weights(td, d, ff, 70 + i), td, d, ff)
+    xb, _ = bf16_round(np.random.default_rng(80 + i).standard_normal((t, d)))
+    x, g, y = F.Tensor.from_bf16_bits(xb, (t, d)), F.Tensor.empty((t, 2 * ff)), F.Tensor.empty((t, d))
+    ws = F.DeviceBuffer(lib.fhip_ffn_coop_ws_bytes(gu.handle, dn.handle, t))
+    args = (gu.handle, dn.handle, x.buf.ptr)
+    assert lib.fhip_ffn_bf16_run_sums(*args, None, t, y.buf.ptr, ws.ptr, None) != 0                   # gate|up has to be in memory
+    F._lib.check(lib.fhip_ffn_bf16_run_sums(*args, g.buf.ptr, t, y.buf.ptr, ws.ptr, None))
+    assert (zlib.crc32(g.to_vec().tobytes()), zlib.crc32(y.to_vec().tobytes())) == (crc_gate_up, crc)
+
+
 def test_reference_coop_example_shapes(F, O):
     # crates/ferric-tensor/examples/coop_q4_k.rs: reference-generator weights, M a multiple of 8 and not
     run_case(F, O, Q4_K, 16, 64, 512, 3, gen=O.gen_kquant_matrix)

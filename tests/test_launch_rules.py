@@ -95,6 +95,25 @@ def test_the_tile_of_a_prompt_product(gemm):
         assert us[plan(gemm, *shape)[0]] <= 1.25 * min(us), shape
 
 
+def test_where_the_runs_of_run_sums_end(gemm):
+    """fhip_gemm_q_bf16_run_sums promises the order of its sums from version to version: a tile's rows and outputs, the whole tiles of a workgroup and the chunks of a run are
+    that order, on 256 CUs, and stand as they are here whatever the launches without that promise come to prefer."""
+    order = {
+        (Q6_K, 2049, 5120, 33): (64, 256, 0, 1), (Q6_K, 9000, 1280, 65): (128, 256, 0, 1), (Q5_K, 4100, 2304, 520): (128, 256, 0, 3),
+        (Q4_K, 4100, 1280, 129): (256, 256, 0, 1), (Q8_0, 9000, 736, 128): (256, 256, 0, 1), (Q8_0, 5120, 512, 40): (256, 160, 0, 1),
+        (Q4_K, 7000, 256, 300): (128, 128, 0, 1), (Q5_K, 7000, 1280, 300): (128, 128, 0, 5), (Q4_K, 1283, 512, 300): (128, 128, 0, 1),
+        (Q6_K, 2049, 5120, 300): (128, 128, 0, 4), (Q6_K, 700, 1792, 65): (128, 128, 0, 1), (Q8_0, 2049, 2080, 64): (128, 160, 0, 1),
+        (Q8_0, 9000, 512, 257): (128, 160, 0, 2), (Q5_K, 9000, 512, 40): (64, 128, 0, 1), (Q4_K, 7000, 2304, 33): (64, 128, 0, 2),
+        (Q5_K, 7000, 1792, 257): (64, 128, 1, 1), (Q4_K, 7000, 256, 100): (64, 128, 0, 1), (Q8_0, 1283, 4064, 33): (64, 128, 0, 1),
+        (Q8_0, 5120, 1312, 64): (64, 128, 0, 1), (Q6_K, 7000, 3328, 64): (64, 128, 0, 3), (Q6_K, 5120, 1280, 300): (64, 128, 0, 5),
+        (Q4_K, 7168, 5120, 509): (256, 256, 0, 5), (Q4_K, 5120, 5120, 509): (256, 160, 0, 5), (Q4_K, 34816, 5120, 509): (256, 256, 1, 2),
+        (Q6_K, 5120, 17408, 509): (256, 160, 0, 17), (Q4_K, 34816, 5120, 2048): (256, 256, 4, 5), (Q6_K, 5120, 17408, 2048): (256, 160, 1, 1),
+        (Q4_K, 7168, 5120, 64): (64, 128, 0, 5), (Q5_K, 3072, 2048, 700): (256, 256, 0, 2), (Q8_0, 12288, 4096, 128): (128, 160, 0, 5),
+        (Q6_K, 4096, 8960, 882): (256, 256, 0, 9)}
+    for shape, runs in order.items():
+        assert plan(gemm, *shape, run_sums=True)[1:5] == runs, shape
+
+
 class Weight(C.Structure):
     """struct fhip_weight (ferric_amd/csrc/common.hpp), for a query that reads its type and shape."""
     _fields_ = [("type", C.c_uint32), ("rows", C.c_size_t), ("cols", C.c_size_t), ("row_bytes", C.c_size_t), ("nbytes", C.c_size_t), ("d_raw", C.c_void_p), ("owns", C.c_bool),
