@@ -29,7 +29,6 @@ constexpr Lut16 lut16(uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
         const int i = order[k];
         p[i] = t[i] ^ sign(n[2 * i + 1]);
         n[i] = t[8 + i] ^ sign(p[2 * i + 1]);
-        if (i == 0) p[0] = t[0] ^ sign(n[1]);
     }
     Lut16 r = {};
     for (int i = 0; i < 8; i++) {
