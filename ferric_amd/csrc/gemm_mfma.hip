@@ -287,13 +287,11 @@ struct Q6K {
 };
 
 // LATE: a piece stays as it was loaded until the step that reads it shifts it into place (loads.hpp). Shifted beside its load it is
-// waited for right there. At 64 and 128 rows a step is too short to hide that behind the other wave of a SIMD; at 256 rows it is not, and
-// the registers of the unshifted pieces cost more (Eager). Measured, us, shifted at once -> late: 128 x 160 tiles of 5120 x 13824 at 64 /
-// 128 / 256 rows 53.8 / 57.8 / 91.9 -> 47.4 / 50.7 / 80.2, of 4096 x 4096 29.4 -> 27.7 at 128; 64 x 256 78.8 -> 75.9, 64 x 128 109.8 ->
-// 105.3, 128 x 128 63.1 -> 61.6 at 128 rows; 256 x 256 at 2048 rows 379 -> 383, 256 x 160 on 17408 x 4096 387 -> 393. Q6_K, whose pieces
-// are shifted once for four steps but unpacked by more arithmetic, lost 2 ... 7 % in every tile and shifts at once. With CHUNK_US for what
-// a chunk takes now, 14 % of shapes change their tile, to 128 x 160: 1280 x 8704 at 378 rows 44.5 -> 36.8, 1616 x 2304 at 874 40.1 -> 27.9,
-// 9392 x 11776 at 40 69.7 -> 58.5, 9328 x 2304 at 267 50.3 -> 41.4 (worst of fourteen: 4424 x 5120 at 35 rows 28.0 -> 29.3).
+// waited for right there. In the 128 x 160 tile and the kernel of up to 32 rows a step is too short to hide that behind the other wave of a
+// SIMD; at 256 rows it is not, and the registers of the unshifted pieces cost more (Eager). Measured, us, shifted at once -> late: 128 x 160 tiles of
+// 5120 x 13824 at 64 / 128 / 256 rows 53.8 / 57.8 / 91.9 -> 47.4 / 50.7 / 80.2, of 4096 x 4096 at 128 29.4 -> 27.7; 256 x 256 at 2048 rows 379 -> 383,
+// 256 x 160 on 17408 x 4096 387 -> 393. Q6_K, whose pieces are shifted once for four steps but unpacked by more arithmetic, lost 2 ... 7 % in every
+// tile and shifts at once.
 template <bool LATE>
 struct Q80T {
     using Eager = Q80T<false>;
@@ -833,9 +831,9 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 // unpacked by the one wave that multiplies it, straight into its B operand, and LDS carries the activations alone: a whole chunk of them
 // at a time, double buffered, one barrier a chunk. The eight waves are NW along N x KW = 8 / NW along the chunk's four steps (a wave does
 // S = 4 / KW of them), and the KW partial sums of an output meet in LDS when a run ends, added in order of the steps. Work distribution
-// and slots of partial tiles are those of the tiled kernel. Measured with the tile the estimate picks, us: Q4_K 5120 x 5120 at 64 / 128 /
-// 512 rows 17.6 / 22.8 / 45.2 -> 14.5 / 19.0 / 38.2, 6112 x 2816 at 132 42.0 -> 16.6, 10176 x 2560 at 82 27.2 -> 15.8; Q6_K 5120 x 17408 at
-// 128 58.2 -> 48.0; Q8_0 12152 x 1536 at 107 26.0 -> 18.1. Loading a chunk's activations and storing them to LDS at its end, where all
+// and slots of partial tiles are those of the tiled kernel. Measured with the tile the estimate picks, us, the tiled kernel alone before:
+// Q4_K 5120 x 5120 at 64 / 128 / 512 rows 17.2 / 20.8 / 43.8 -> 14.3 / 20.4 / 37.6, 6112 x 2816 at 132 39.9 -> 15.9, 10176 x 2560 at 82 23.4 -> 15.2; Q6_K
+// 5120 x 17408 at 128 57.0 -> 45.3; Q8_0 12152 x 1536 at 107 24.0 -> 14.9. Loading a chunk's activations and storing them to LDS at its end, where all
 // waves wait, cost 2.45 us a chunk: a piece now goes to LDS behind each slice, a chunk after it was asked for.
 // Per format: `Raw` holds what a lane half unpacks of S steps of one weight row, as it was loaded (pieces at 2-byte alignment are shifted
 // into place by settle(), where they are first read); begin<I>() derives step I's scales, frag<I, T>() the operand of its slice T.

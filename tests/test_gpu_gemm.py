@@ -63,7 +63,7 @@ def test_seeded_random_shapes(F, O):
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6])
 def test_every_tile_on_ragged_shapes(F, O, tile):
-    # The launcher picks one of seven workgroup tiles by estimate; here each is pinned in turn (64 / 128 / 256 rows x 256
+    # The launcher picks one of twelve workgroup tiles by estimate; here the first seven are pinned in turn (64 / 128 / 256 rows x 256
     # outputs, 256 x 160, 128 / 64 rows x 128, 128 x 160) and run on shapes that fill no tile: rows and outputs that end inside a tile, outputs that are no
     # multiple of 4, launches with whole rounds of tiles and a cut remainder, launches where every tile is cut along K.
     lib = F._lib.load()
@@ -344,7 +344,6 @@ def test_swiglu_inside_the_tiled_gemm(F, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
-# 272 tiles of 64 x 128, 312 of 64 x 256 and of 128 x 256, and the launcher's choice: 256 workgroups take a whole one each and the rest is cut along K
 @pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11])
 def test_swiglu_of_rows_turned_through_lds(F, tile):
     # Q6_K and Q8_0 gate|up on the tiles whose waves unpack for themselves: a wave's gate and up rows lie in two places. Rows of an odd number of blocks, whose
@@ -367,6 +366,7 @@ def test_swiglu_of_rows_turned_through_lds(F, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
+# 272 tiles of 64 x 128, 312 of 64 x 256 and of 128 x 256, and the launcher's choice: 256 workgroups take a whole one each and the rest is cut along K
 @pytest.mark.parametrize("tile,t,d,n_ff", [(5, 40, 512, 17408), (0, 130, 512, 13312), (1, 270, 768, 13312), (-1, 520, 512, 17408)])
 def test_swiglu_beside_whole_and_cut_tiles(F, O, tile, t, d, n_ff):
     # The fused launch deals columns of gate and up in turn to a tile and so cuts other outputs than a launch over the stacked rows does:
