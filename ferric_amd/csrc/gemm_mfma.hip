@@ -826,8 +826,8 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 // ------------------------------------------------------------------------------------------------
 // The kernel for short prompts and small weights: a wave unpacks its own weights. A low tile of the kind above is bound by what a step
 // moves through LDS (operands of both sides written once and read by every wave) and by its barrier every 64 columns: a 128 x 128 x 256
-// chunk of Q4_K took 2.84 us there, 1.1 of it matrix instructions at the clock the chip holds. It takes 1.97 here (1.45 with no loads,
-// 0.6 without the matrix instructions). Here a wave holds BM activation rows x 32 outputs, so a weight is
+// chunk of Q4_K took 2.84 us there, 1.1 of it matrix instructions at the clock the chip holds. It takes 1.97 here (timing-only variants:
+// 1.45 with no loads, 0.6 without the matrix instructions). Here a wave holds BM activation rows x 32 outputs, so a weight is
 // unpacked by the one wave that multiplies it, straight into its B operand, and LDS carries the activations alone: a whole chunk of them
 // at a time, double buffered, one barrier a chunk. The eight waves are NW along N x KW = 8 / NW along the chunk's four steps (a wave does
 // S = 4 / KW of them), and the KW partial sums of an output meet in LDS when a run ends, added in order of the steps. Work distribution
@@ -914,8 +914,9 @@ struct OwnQ5K {
 // segment G's part of a lane's Raw from its row's 80 bytes. 80 bytes apart, sixteen rows' 16-byte reads meet every bank once.
 // Why: a load whose lanes each read a row of their own takes the address unit a cycle a lane, 0.2 us for the eight waves of a workgroup, and Q6_K needed 17
 // such loads a chunk, Q8_0 24; of these, ten touch some twenty cache lines each. A chunk of 64 x 256 outputs: Q6_K 4.70 -> 4.15 us, Q8_0 6.25 -> 4.66, of 64 x 128 2.21 -> 2.03,
-// 3.29 -> 2.23 (what is left over Q4_K's 2.39 and 1.29 is their unpacking, 541 and 461 vector instructions to 342, and the way through LDS). With the estimate fitted again, us: Q8_0
-// 3160 x 3328 at 196 rows 26.0 -> 18.5, 2120 x 5632 at 206 28.9 -> 26.7; Q6_K 25736 x 11776 at 44 105 -> 90, 1712 x 13312 at 184 33.7 -> 29.8; FFN blocks of both, 1024 x 7680 at
+// 3.29 -> 2.23 (what is left over Q4_K's 2.39 and 1.29 is their unpacking, 307 and 294 vector
+// instructions a wave for half a chunk of 32 outputs and 128 rows to Q4_K's 219, and the way through LDS, 0.6 and 2.3 cycles of bank conflicts an LDS
+// instruction: the scales are read two bytes a lane). With the estimate fitted again, us: Q8_0 3160 x 3328 at 196 rows 26.0 -> 18.5, 2120 x 5632 at 206 28.9 -> 26.7; Q6_K 25736 x 11776 at 44 105 -> 90, 1712 x 13312 at 184 33.7 -> 29.8; FFN blocks of both, 1024 x 7680 at
 // 271 53.8 -> 46.5. Q4_K's five loads a chunk turned the same way: 3 - 6 % slower.
 constexpr int SEG_ROW = 80, SEG_BYTES = 32 * SEG_ROW;
 __device__ __forceinline__ fhip::Un16 un16(const uint8_t* p) { return fhip::Un16{((const fhip::LdU4A4*)p)->v, *(const uint16_t*)(p + 16)}; }
