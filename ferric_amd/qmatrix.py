@@ -278,7 +278,7 @@ class Tensor:
         t, ne = (self.shape[0], self.shape[1]) if len(self.shape) == 2 else (1, self.numel())
         assert 1 <= k <= 8, "k must be 1..=8"
         assert ne <= 1024, "moe_topk: n_expert <= 1024 (single-thread scan)"
-        buf = _lib.moe_topk(self.buf, bias.buf if bias is not None else None, t, ne, k, sigmoid, scale, norm, None if stream is None else stream.handle)
+        buf = _lib.moe_topk(self.buf, bias.buf if bias is not None else None, t, ne, k, sigmoid, float(scale), norm, None if stream is None else stream.handle)
         if buf is not NotImplemented:
             return _result(buf, (t, 2 * k))
         out = Tensor.empty((t, 2 * k))   # tensors over other objects with a `ptr`

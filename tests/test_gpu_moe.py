@@ -229,3 +229,12 @@ def test_the_calls_convert_what_they_are_given(F):
         x.matmul_q_swiglu_id(gu, sel, k, 2 ** 63 + eff)
     with pytest.raises(OverflowError):
         h.matmul_q_id_wsum(dn, sel, 2 ** 62 + d)
+
+
+def test_the_scale_of_a_selection_is_whatever_float_takes(F):
+    logits = F.Tensor.from_vec(np.random.default_rng(4).standard_normal((2, 16)).astype(np.float32), (2, 16))
+    want = logits.moe_topk(None, 4, True, 1.5).to_vec()
+    for scale in ("1.5", np.float16(1.5), np.array(1.5), b"1.5"):
+        assert np.array_equal(logits.moe_topk(None, 4, True, scale).to_vec().view(np.uint32), want.view(np.uint32)), scale
+    with pytest.raises(ValueError):
+        logits.moe_topk(None, 4, True, "a")
