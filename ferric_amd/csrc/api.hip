@@ -1,5 +1,6 @@
 // The extern "C" surface of libferric_hip (declared in include/ferric_hip.h): argument checks with
 // the reference's error behaviour, weight handles, and thin dispatch into the kernel launchers.
+#include "f16x2.hpp"
 #include "hostmem.hpp"
 #include "prompt.hpp"
 
@@ -209,6 +210,16 @@ int lib_workspace(hipStream_t s, size_t need, void** out, const char* who) {
     return FHIP_OK;
 }
 
+// whether lib_workspace would not refuse: a capturing stream has what it has
+bool lib_workspace_can(hipStream_t s, size_t need) {
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    for (auto& w : g_ws)
+        if (w.s == s && w.n >= need) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+    return st == hipStreamCaptureStatusNone;
+}
+
 void release_workspace(hipStream_t s) {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     for (size_t i = 0; i < g_ws.size(); i++) {
@@ -235,12 +246,12 @@ static int gemm_bf16_lib_ws(const fhip_weight* w, const uint16_t* d_x, size_t t,
 
 // ---- which kernel a batch takes ---------------------------------------------------------------------------------------------
 // One or two activation rows go through the streaming mat-vec (one pass over the weights serves two rows). From three rows on
-// (five for Q8_0) the f16 hi/lo matrix-core kernels read the weights once for up to 32 (Q8_0: 16) rows; longer batches are cut
+// (five for Q8_0) the f16 hi/lo matrix-core kernels multiply groups of up to 32 rows (Q8_0 with sums by atomics: 16); longer batches are cut
 // into such groups. FHIP_BATCH_F32_MATVEC keeps every batch on the mat-vec's arithmetic (launch_gemv: four rows a pass for Q4_K /
 // Q5_K / Q6_K, up to sixteen for the 32-value formats, on the int8 matrix instructions, a few rows on the dot-product kernel): a row then has the same
 // bits whatever batch it is part of.
 
-size_t f16x2_group(const fhip_weight* w) { return w->type == FHIP_Q8_0 ? 16 : 32; }
+size_t f16x2_group(const fhip_weight* w) { return w->type == FHIP_Q8_0 && w->batch_policy != FHIP_BATCH_ORDERED ? 16 : 32; }
 // Three and four rows of a Q4_K / Q5_K / Q6_K weight whose rows the four-row mat-vec (gemv_quad.hip) covers in one pass (up to 10240
 // columns) take that kernel under every policy: one launch, no workspace, the bits of a batch of one, and faster than the f16
 // kernels with their split and sum launches (cold, ordered sums: 5120 x 5120 17.7 -> 12.5 us, 7168 x 5120 19.9 -> 14.1, Q6_K
@@ -255,7 +266,7 @@ bool takes_f16x2(const fhip_weight* w, size_t rows_x) {
     if (w->type != FHIP_Q4_K && w->type != FHIP_Q5_K && w->type != FHIP_Q6_K && w->type != FHIP_Q8_0) return false;
     if (rows_x < (w->type == FHIP_Q8_0 ? 5u : 3u)) return false;
     if (matmul_takes_quad(w, rows_x)) return false;
-    return fhip::gemm_f16x2_supports(w, rows_x < f16x2_group(w) ? rows_x : f16x2_group(w));
+    return fhip::gemm_f16x2_takes(w, rows_x < f16x2_group(w) ? rows_x : f16x2_group(w));
 }
 
 // Fused gate|up + SwiGLU at three or four rows: one pass of the int8 matrix-instruction mat-vec (gemv_quad.hip, 31 us on
@@ -280,35 +291,34 @@ int zero_outputs(size_t t, size_t rows, float* d_y, hipStream_t s) {
 }
 
 // y [t, w->rows] = x [t, cols] W^T for t rows of one group; ws: f16x2_matmul_ws(w, t) bytes
-// (FHIP_BATCH_ORDERED: behind the prepared activations, the partial sums of the groups the launch cuts along K)
+// (FHIP_BATCH_ORDERED: behind the prepared activations, the partial outputs of the ranges that K is cut into)
 size_t f16x2_matmul_ws(const fhip_weight* w, size_t t) {
-    return align256(fhip::gemm_f16x2_xp_bytes(w, t)) + (w->batch_policy == FHIP_BATCH_ORDERED ? align256(fhip::gemm_f16x2_part_bytes_upto(w, t)) : 0);
+    return align256(fhip::gemm_f16x2_xp_bytes(w, t)) + (w->batch_policy == FHIP_BATCH_ORDERED ? align256(fhip::gemm_f16x2_parts_bytes(w, t)) : 0);
 }
-// What such a product takes: the held kernel, or the streaming ones with operand rows of their own or prepared ones (own: the rows come as they are)
-int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, const float* d_y, bool deferred) {
-    if (own && fhip::gemm_f16x2_held(w, d_x, t, d_y, deferred && w->batch_policy == FHIP_BATCH_ORDERED)) return FHIP_ROUTE_HELD;
+// What such a product takes: the held kernel, or one whose operand rows are made by itself or prepared (own: the rows come as they are)
+int f16x2_route(const fhip_weight* w, const float* d_x, size_t t, bool own, const float* d_y) {
+    if (own && fhip::gemm_f16x2_held(w, d_x, t, d_y)) return FHIP_ROUTE_HELD;
+    if (w->batch_policy == FHIP_BATCH_ORDERED)
+        return (own && fhip::gemm_f16x2_resident_own_x(w, d_x, t, d_y) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (fhip::gemm_f16x2_parts(w, t) > 1 ? FHIP_ROUTE_CUT : 0);
     const bool cut = fhip::gemm_f16x2_adds_into_y(w, t);   // along K
-    return (own && !(cut && w->batch_policy != FHIP_BATCH_ORDERED) && fhip::gemm_f16x2_own_x(w, d_x, t) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (cut ? FHIP_ROUTE_CUT : 0);
+    return (own && !cut && fhip::gemm_f16x2_own_x(w, d_x, t) ? FHIP_ROUTE_OWN_ROWS : FHIP_ROUTE_PREPARED) | (cut ? FHIP_ROUTE_CUT : 0);
 }
-// deferred: the ordered sum of K-split groups is left to the reader of y, which gets *deferred as its `src`
+// deferred: the sum of partial outputs is left to the reader of y, which gets *deferred as its `src`
 int f16x2_launch(int route, const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
                  fhip::F16Parts* deferred, const fhip::F16Parts* src) {
-    if (route == FHIP_ROUTE_HELD) {
-        if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0, 0, 128};
-        return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
-    }
-    uint16_t* xp = (uint16_t*)d_ws;
+    if (deferred) *deferred = fhip::F16Parts{nullptr, 0, 0, 0};
+    if (route == FHIP_ROUTE_HELD) return fhip::launch_gemm_f16x2_held(w, d_x, t, d_y, s);
+    uint16_t* xp = (route & ~FHIP_ROUTE_CUT) == FHIP_ROUTE_OWN_ROWS ? nullptr : (uint16_t*)d_ws;
     const bool cut = (route & FHIP_ROUTE_CUT) != 0, ordered = w->batch_policy == FHIP_BATCH_ORDERED;
-    float* part = cut && ordered ? (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))) : nullptr;
     const bool clr = cut && !ordered;   // then the split clears y on the side
-    if ((route & ~FHIP_ROUTE_CUT) == FHIP_ROUTE_OWN_ROWS) return fhip::launch_gemm_f16x2(w, nullptr, t, d_y, s, false, part, deferred, d_x);
-    int rc = fhip::launch_xsplit_f16(w, d_x, t, swiglu_in, xp, s, clr ? d_y : nullptr, clr ? t * w->rows : 0, src);
+    int rc = xp ? fhip::launch_xsplit_f16(w, d_x, t, swiglu_in, xp, s, clr ? d_y : nullptr, clr ? t * w->rows : 0, src) : FHIP_OK;
     if (rc) return rc;
-    return fhip::launch_gemm_f16x2(w, xp, t, d_y, s, clr, part, deferred);
+    if (ordered) return fhip::launch_gemm_f16x2_resident(w, xp, d_x, t, d_y, (float*)((uint8_t*)d_ws + align256(fhip::gemm_f16x2_xp_bytes(w, t))), s, deferred);
+    return fhip::launch_gemm_f16x2(w, xp, t, d_y, s, clr, xp ? nullptr : d_x);
 }
 int f16x2_matmul(const fhip_weight* w, const float* d_x, size_t t, bool swiglu_in, float* d_y, void* d_ws, hipStream_t s,
                  fhip::F16Parts* deferred = nullptr, const fhip::F16Parts* src = nullptr) {
-    return f16x2_launch(f16x2_route(w, d_x, t, !swiglu_in && !src, d_y, deferred != nullptr), w, d_x, t, swiglu_in, d_y, d_ws, s, deferred, src);
+    return f16x2_launch(f16x2_route(w, d_x, t, !swiglu_in && !src, d_y), w, d_x, t, swiglu_in, d_y, d_ws, s, deferred, src);
 }
 
 }  // namespace
@@ -627,8 +637,10 @@ int fhip_matmul_q(const fhip_weight* w, const float* d_x, size_t rows_x, float* 
     const size_t grp = f16x2_group(w);
     void* ws = nullptr;
     if (rows_x <= grp) {   // one group: the held kernel needs no workspace
-        const int route = f16x2_route(w, d_x, rows_x, true, d_y, false);
-        if (route != FHIP_ROUTE_HELD && (rc = lib_workspace(s, f16x2_matmul_ws(w, rows_x), &ws, "fhip_matmul_q"))) return rc;
+        int route = f16x2_route(w, d_x, rows_x, true, d_y);
+        // a capture on a stream without the workspace takes the launch that needs none
+        if ((route & FHIP_ROUTE_CUT) && fhip::gemm_f16x2_held_takes(w, d_x, rows_x, d_y) && !lib_workspace_can(s, f16x2_matmul_ws(w, rows_x))) route = FHIP_ROUTE_HELD;
+        if (route != FHIP_ROUTE_HELD && route != FHIP_ROUTE_OWN_ROWS && (rc = lib_workspace(s, f16x2_matmul_ws(w, rows_x), &ws, "fhip_matmul_q"))) return rc;
         return f16x2_launch(route, w, d_x, rows_x, false, d_y, ws, s, nullptr, nullptr);
     }
     if ((rc = lib_workspace(s, f16x2_matmul_ws(w, grp), &ws, "fhip_matmul_q"))) return rc;
@@ -717,7 +729,7 @@ int fhip_ffn(const fhip_weight* gu, const fhip_weight* down, const float* d_x, s
                 rc = f16x2_matmul(down, g, t, false, d_y + m0 * down->rows, ws2, s);
         } else {
             // under the ordered policy gate|up's K-split groups stay partial sums; the split for the down projection adds them
-            fhip::F16Parts parts{nullptr, 0, 0, 0, 0, 128};
+            fhip::F16Parts parts{nullptr, 0, 0, 0};
             if (!(rc = f16x2_matmul(gu, d_x + m0 * gu->cols, t, false, g, ws, s, &parts)))
                 rc = f16x2_matmul(down, g, t, true, d_y + m0 * down->rows, ws2, s, nullptr, &parts);
         }
@@ -1189,7 +1201,7 @@ int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_
     const size_t grp = takes_f16x2(w, rows_x) ? f16x2_group(w) : rows_x;
     for (size_t m0 = 0; m0 < rows_x && w->rows; m0 += grp) {
         const size_t t = rows_x - m0 < grp ? rows_x - m0 : grp;
-        if (takes_f16x2(w, t)) { add(f16x2_route(w, d_x + m0 * w->cols, t, true, d_y + m0 * w->rows, false), t); continue; }
+        if (takes_f16x2(w, t)) { add(f16x2_route(w, d_x + m0 * w->cols, t, true, d_y + m0 * w->rows), t); continue; }
         for (size_t r = 0; r < t;) {
             const fhip::MatvecPass pass = fhip::matvec_pass(w, t - r, 0);
             add(pass.kernel, pass.rows);

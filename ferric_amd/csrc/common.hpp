@@ -131,38 +131,6 @@ int gemm_bf16_force_tile(int tile);   // debugging / tests: 0..3 pins the tile o
 int launch_cvt_bf16(const float* d_x, size_t n, uint16_t* d_out, hipStream_t s);
 int launch_swiglu_bf16(const float* d_gu, size_t t, size_t d, uint16_t* d_out, hipStream_t s);
 
-// gemm_f16x2.hip: 2..32 activation rows in one pass over the weights, f16 matrix cores, f32-grade results
-bool gemm_f16x2_supports(const fhip_weight* w, size_t t);
-size_t gemm_f16x2_xp_bytes(const fhip_weight* w, size_t t);       // prepared-activation buffer for t rows
-bool gemm_f16x2_adds_into_y(const fhip_weight* w, size_t t);      // true: the launch adds into y, a cleared y saves it a launch
-// splits the rows of x [t, cols] (swiglu: of silu(gate) * up of x [t, 2 cols]) chunk by chunk into scaled f16 hi / lo
-// operand rows, each carrying the factor that takes its scale out again
-// Where the K-split groups of a matmul's output still lie as partial sums, one slot per (128-output group, contributor):
-// output n of activation row t is slot 0 + slot 1 + ... of its group in that order (one contributor: the value in y itself).
-struct F16Parts {
-    const float* part;    // null: every output is in y
-    int kmax, nchunks, grid;
-    long long units;
-    int group;            // outputs of a group: 128, or 256 where the eight-wave row-streaming kernel made the sums
-};
-// src: x is the output of a matmul whose ordered sum was left to this launch (launch_gemm_f16x2 with `deferred`)
-int launch_xsplit_f16(const fhip_weight* w, const float* d_x, size_t t, bool swiglu, uint16_t* d_xp, hipStream_t s, float* zero = nullptr,
-                      size_t zero_n = 0, const F16Parts* src = nullptr);
-// d_part: null, or gemm_f16x2_part_bytes(w, t) bytes: partial sums of K-split groups go there and are added in a fixed
-// order by a launch behind the matmul (y then needs no clearing) instead of being added into y atomically
-// deferred: with d_part, the launch that adds the partial sums is left out and *deferred says where they lie; the reader of y
-// (launch_xsplit_f16 with `src`) adds them in the same order
-int launch_gemm_f16x2(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y, hipStream_t s, bool y_cleared = false,
-                      float* d_part = nullptr, F16Parts* deferred = nullptr, const float* d_x = nullptr);
-// true: launch_gemm_f16x2 given d_x (the f32 rows) makes its operand rows itself, without launch_xsplit_f16 in front of it (d_xp is not read)
-bool gemm_f16x2_own_x(const fhip_weight* w, const float* d_x, size_t t);
-// true: launch_gemm_f16x2_held does the whole product, y = x W^T, in one launch without a workspace. summed_later: launch_gemm_f16x2's partial
-// sums would be left to the launch that reads y
-bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y, bool summed_later);
-int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s);
-size_t gemm_f16x2_part_bytes(const fhip_weight* w, size_t t);
-size_t gemm_f16x2_part_bytes_upto(const fhip_weight* w, size_t t);   // the largest over batches of 1..t rows
-
 // decode_ops.hip: the steps either side of the matmuls in a decode layer
 int launch_rmsnorm(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, float* norm_out,
                    hipStream_t s);

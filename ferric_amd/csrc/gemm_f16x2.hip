@@ -28,9 +28,9 @@
 // Lane (g4 = lane / 16, c = lane % 16) of a wave works on weight row c of a 16-row set and on k-group g4 of each
 // 32-wide MFMA slice; a wave carries two row sets (32 weight rows), a workgroup four waves (128 rows; the row-streaming
 // kernel for up to 8 activation rows: eight waves, 256 rows). The (row group, 256-column chunk) units are dealt to the workgroups in equal contiguous runs; a run that covers its
-// group's whole K stores, any other adds atomically into a Y cleared beforehand (or, when the caller asks for ordered sums, stores
-// into a slot of its own that sum_split_kernel adds in contributor order).
-#include "common.hpp"
+// group's whole K stores, any other adds atomically into a Y cleared beforehand. Where the sums are to be in an order, two kernels further down do the product: one keeps a
+// weight row's whole K inside a workgroup, one the operand rows in LDS.
+#include "f16x2.hpp"
 #include <algorithm>
 #include "loads.hpp"
 
@@ -175,15 +175,14 @@ struct Q4K {
         o[3] = hfma2(and_or(w8, 0x00F000F0u, H1024), x.s1, x.c1);
         return __builtin_bit_cast(f16x8, o);
     }
-    // B operand of the minima MFMA: m[0..7] of this row as f16 in k-group 0, zeros in the others
-    static __device__ __forceinline__ f16x8 mins(const Raw& r, int g4) {
+    // B operand of the minima MFMA: m[0..7] of this row as f16 (in every k-group: the A operand holds zeros in all but group 0)
+    static __device__ __forceinline__ f16x8 mins(const Raw& r, int) {
         const uint32_t lo = min_bytes(r.hd, false), hi = min_bytes(r.hd, true);
         u32x4 o;
         o[0] = hadd2(__builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u), HNEG1024);
         o[1] = hadd2(__builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u), HNEG1024);
         o[2] = hadd2(__builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u), HNEG1024);
         o[3] = hadd2(__builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u), HNEG1024);
-        if (g4 != 0) o = (u32x4){0u, 0u, 0u, 0u};
         return __builtin_bit_cast(f16x8, o);
     }
 };
@@ -423,33 +422,20 @@ struct Q80 {
 // ------------------------------------------------------------------------------------------------
 constexpr int MAXW = 64;   // rows of up to 65 536 columns
 
-// Workgroup b of G takes units [b U / G, (b + 1) U / G): the workgroup that holds unit u
-__device__ __host__ __forceinline__ int holder_of(long long u, long long G, long long U) { return (int)(((u + 1) * G - 1) / U); }
-
-// element n of row t of the matrix the split reads: as stored, or, where the producing matmul left a K-split group's
-// partial sums to this launch, slot 0 + slot 1 + ... of that group (the order sum_split_kernel adds them in)
+// element n of row t of the matrix the split reads: as stored, or, where the producing matmul left its partial outputs to this launch, their sum in sum_parts_kernel's order
 __device__ __forceinline__ float x_at(const float* __restrict__ x, int t, size_t n, const fhip::F16Parts& src) {
-    if (src.part) {
-        const int gsh = src.group == 256 ? 8 : 7;   // (groups of 128 or 256 outputs)
-        const int grp = (int)(n >> gsh);
-        const int first = holder_of((long long)grp * src.nchunks, src.grid, src.units);
-        const int nk = holder_of((long long)(grp + 1) * src.nchunks - 1, src.grid, src.units) - first + 1;
-        if (nk > 1) {
-            // (eight slots requested at a time: one trip to memory for the usual three or four contributors instead of one each)
-            const float* q = src.part + ((size_t)grp * src.kmax * 32 + t) * src.group + (n & (size_t)(src.group - 1));
-            float a = q[0];
-            for (int k0 = 1; k0 < nk; k0 += 8) {
-                float v[8];
+    if (src.parts == 0) return x[n];
+    const float* q = src.part + (size_t)t * src.ld + n;
+    float a = q[0];
+    for (int k0 = 1; k0 < src.parts; k0 += 4) {                 // (four requested at a time: one trip to memory for the usual two to five)
+        float v[4];
 #pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = q[(size_t)(k0 + j < nk ? k0 + j : 0) * (32 * (size_t)src.group)];
+        for (int j = 0; j < 4; j++) v[j] = q[(size_t)(k0 + j < src.parts ? k0 + j : 0) * src.stride];
 #pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (k0 + j < nk) a += v[j];
-            }
-            return a;
-        }
+        for (int j = 0; j < 4; j++)
+            if (k0 + j < src.parts) a += v[j];
     }
-    return x[n];
+    return a;
 }
 
 template <bool SWIGLU>
@@ -520,6 +506,73 @@ __global__ void __launch_bounds__(256) xsplit_f16_kernel(const float* __restrict
     }
 }
 
+template <int PERM>
+__device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), PERM, 0xF, 0xF, true));
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_TURNED = 0x141;
+
+// A chunk of eight activation rows, four columns to a lane, as its sixteen operand rows in LDS (hi, then lo), by one wave: the bits of xsplit_f16_kernel. The rows are
+// turned through the place the operands take (a lane then has a sub-block of a row: 32 columns, whose largest magnitude and sum are mostly its own).
+template <class F>
+__device__ __forceinline__ void split_chunk(const f32x4 (&x)[8], uint16_t* to, int lane) {
+    constexpr int XROW = 4 * CHUNK + 16;
+    static_assert(8 * XROW <= 16 * XR * 2, "eight activation rows fit their operand rows' place");
+    uint8_t* const st = (uint8_t*)to;
+    const int row = lane >> 3, sub = lane & 7;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int r = 0; r < 8; r++) *(f32x4*)(st + r * XROW + 16 * (lane ^ (lane >> 3))) = x[r];   // a row's 16-byte pieces, the eight of a sub-block turned by its number
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    f32x4 v[8];
+    float m = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = *(const f32x4*)(st + row * XROW + 16 * (8 * sub + (j ^ sub)));
+    // (a NaN is not the largest magnitude: it reaches the operands as it is)
+#pragma unroll
+    for (int j = 0; j < 8; j++) m = fmaxf(m, fmaxf(fmaxf(fabsf(v[j][0]), fabsf(v[j][1])), fmaxf(fabsf(v[j][2]), fabsf(v[j][3]))));
+    m = fmaxf(m, dpp<DPP_XOR1>(m));
+    m = fmaxf(m, dpp<DPP_XOR2>(m));
+    m = fmaxf(m, dpp<DPP_HALF_TURNED>(m));
+    float sc, inv;
+    chunk_scale(m, sc, inv);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint16_t* const hi = to + row * XR;
+    uint16_t* const lo = hi + 8 * XR;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {                               // four columns' positions are one aligned run of eight bytes in every format's order
+        f16x4 h, l;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[j][k] *= sc;
+            const _Float16 a = (_Float16)v[j][k];
+            h[F::pos_of(k)] = a;
+            l[F::pos_of(k)] = (_Float16)(v[j][k] - (float)a);
+        }
+        const int pos = F::pos_of(32 * sub + 4 * j);
+        *(f16x4*)(hi + pos) = h;
+        *(f16x4*)(lo + pos) = l;
+    }
+    if constexpr (F::HAS_MIN) {
+        // the sub-block's sum in the order of xsplit's exchanges: columns 16, 8, 4, 2, 1 apart
+        f32x4 w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = v[j] + v[j + 4];
+        w[0] += w[2]; w[1] += w[3];
+        w[0] += w[1];
+        const float s = ((w[0][0] + w[0][2]) + (w[0][1] + w[0][3])) * 0.015625f;
+        const _Float16 a = (_Float16)s;
+        hi[CHUNK + sub] = __builtin_bit_cast(uint16_t, a);
+        lo[CHUNK + sub] = __builtin_bit_cast(uint16_t, (_Float16)(s - (float)a));
+        hi[CHUNK + 8 + sub] = 0;
+        lo[CHUNK + 8 + sub] = 0;
+    }
+    const uint32_t ib = __float_as_uint(inv);
+    const uint16_t part = (uint16_t)(sub == 0 ? ib & 0xFFFFu : sub == 1 ? ib >> 16 : 0u);
+    hi[XSCALE + sub] = part;
+    lo[XSCALE + sub] = part;
+}
+
 struct F16Params {
     const uint8_t* W;
     const uint16_t* Xp;   // prepared activations: [nchunks][16 NT][XR] f16
@@ -531,16 +584,7 @@ struct F16Params {
     size_t row_bytes;
     long long units;      // row groups * nchunks, chunk fastest
     int group;            // rows of a group: 128, or 256 for the eight-wave row-streaming kernel
-    float* part;          // null: a run that holds part of a group's K adds into Y atomically. Else it stores its partial sums
-                          // into slot (group, contributor) of [groups][kmax][32][group] floats, and sum_split_kernel adds them in order
-    int kmax;
 };
-
-// where a partial output (activation row t, output n of group grp) goes in ordered mode
-__device__ __forceinline__ float* part_slot(const F16Params& p, int grp, int t, int n) {
-    const int k = (int)blockIdx.x - holder_of((long long)grp * p.nchunks, gridDim.x, p.units);
-    return p.part + (((size_t)grp * p.kmax + k) * 32 + t) * p.group + (n - grp * p.group);
-}
 
 template <class F, int NT>
 __global__ void __launch_bounds__(256, F::occupancy(NT)) gemm_q_f16x2_kernel(F16Params p) {
@@ -667,7 +711,6 @@ __global__ void __launch_bounds__(256, F::occupancy(NT)) gemm_q_f16x2_kernel(F16
         // D layout of the 16x16 MFMA: register r of lane (g4, c) is operand row 4 g4 + r, column c. Operand rows 0..7
         // are the hi parts of activation rows 8 q + [0, 8), rows 8..15 their lo parts: lanes g4 and g4 ^ 2 hold the
         // two parts of the same output.
-        float* const slot0 = (!whole && p.part) ? part_slot(p, grp, 0, grp * 128) : nullptr;   // (its division once, not per store; p.group = 128 here)
 #pragma unroll
         for (int s = 0; s < 2; s++)
 #pragma unroll
@@ -680,7 +723,6 @@ __global__ void __launch_bounds__(256, F::occupancy(NT)) gemm_q_f16x2_kernel(F16
                     if (g4 < 2 && t < p.T && n[s] < p.N) {
                         float* y = p.Y + (size_t)t * p.N + n[s];
                         if (whole) *y = v;
-                        else if (p.part) slot0[t * 128 + (n[s] - grp * 128)] = v;
                         else unsafeAtomicAdd(y, v);
                     }
                 }
@@ -937,7 +979,6 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROW
         if (!more || ck == nchunks - 1) {
             // this group's share is complete: whole iff the run held all of its chunks
             const bool whole = (long long)grp * nchunks >= u_begin && (long long)(grp + 1) * nchunks <= u_end;
-            float* const slot0 = (!whole && p.part) ? part_slot(p, grp, 0, grp * GROUP) : nullptr;   // (one division, once per group share)
 #pragma unroll
             for (int s = 0; s < 2; s++)
 #pragma unroll
@@ -950,7 +991,6 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 1 : (NT == 1 ? F::ROW
                     if (g4 < 2 && t < p.T && n < p.N) {
                         float* y = p.Y + (size_t)t * p.N + n;
                         if (whole) *y = v;
-                        else if (p.part) slot0[t * GROUP + (n - grp * GROUP)] = v;
                         else unsafeAtomicAdd(y, v);
                     }
                 }
@@ -985,10 +1025,6 @@ struct HeldParams {
     int T, N, K, nchunks, nblk, tiles, nw, like_rows;   // nw: waves of a workgroup
     size_t row_bytes;
 };
-template <int PERM>
-__device__ __forceinline__ float dpp_quad(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), PERM, 0xF, 0xF, true));
-}
 
 template <class F, int NT, int C, int WV, int EU>
 __global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldParams p) {
@@ -1208,8 +1244,8 @@ __global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldPara
                 const int t = o >> 4, n = tile * 16 + (o & 15);
                 float v = -0.f;                                 // (adds to any value without changing it)
                 for (int w = tid & 3; w < nw; w += 4) v += Ps[buf][w][t][o & 15];
-                v += dpp_quad<0xB1>(v);                         // lane ^ 1
-                v += dpp_quad<0x4E>(v);                         // lane ^ 2
+                v += dpp<DPP_XOR1>(v);
+                v += dpp<DPP_XOR2>(v);
                 if ((tid & 3) == 0 && t < T && n < p.N) Y[(size_t)t * p.N + n] = v;
             }
         } else {
@@ -1227,29 +1263,264 @@ __global__ void __launch_bounds__(64 * WV, EU) gemm_q_f16x2_held_kernel(HeldPara
     one_tile(tile, std::false_type{});
 }
 
-// Ordered mode: group `blockIdx.x` of `group` (128 or 256) outputs, if more than one workgroup held part of its K: Y = slot 0 + slot 1 + ...
-// in that order. Thread = output column (threadIdx.x & 127) of activation row 2 * blockIdx.y + (threadIdx.x >> 7).
-__global__ void __launch_bounds__(256) sum_split_kernel(float* __restrict__ Y, const float* __restrict__ part, int T, int N, int nchunks,
-                                                      long long units, int grid, int kmax, int group) {
-    const int grp = blockIdx.x;
-    const int first = holder_of((long long)grp * nchunks, grid, units), last = holder_of((long long)(grp + 1) * nchunks - 1, grid, units);
-    const int nk = last - first + 1;
-    if (nk == 1) return;
-    const int per = 256 / group, trow = (int)threadIdx.x / group, col = (int)threadIdx.x - trow * group, n = grp * group + col, t = per * blockIdx.y + trow;
-    if (n >= N || t >= T) return;
-    const size_t slot = 32 * (size_t)group;
-    const float* q = part + (size_t)grp * kmax * slot + t * group + col;
-    // (24 slots requested at a time: the down projection's 19 - 20 contributors in one trip to memory instead of three)
-    float a = q[0];
-    for (int k0 = 1; k0 < nk; k0 += 24) {
-        float v[24];
+// ------------------------------------------------------------------------------------------------
+// The same arithmetic with the operand rows in LDS and no barrier among the products: a workgroup, one to a CU, makes the operand rows of its chunks (all of K, or one of
+// `parts` ranges of it) once, and its sixteen waves then go through (tile of 16 weight rows, chunk) units on their own, each a run of them along K, the next unit's bytes in
+// flight through all of a unit's arithmetic. A tile that two or more waves share is added in their order behind the loop; the ranges of K are partial outputs, which
+// sum_parts_kernel or the reader of y adds in their order. blockIdx.z: sets of 8 NT activation rows.
+//
+// What bounds it (34816 x 5120 Q4_K, 8 rows, 27 us with its sums' 3): 6 until the operands lie in LDS, then 15 of instructions (117 vector, 9 matrix for 16 x 256 weights) beside 18 of
+// HBM (5.5 TB/s), which hide each other but for 3. Four waves to a SIMD are what hides them: a kernel that held its chunks' operands in registers had two, a barrier a tile, and
+// took 33.8. A second unit in flight costs 2 - 4 us (a burst in front of the operand rows), operand rows made four columns to a lane 1.5, unit addresses by lane 1.
+// Us, sums in order, 8 rows, streaming or held kernel before | now: Q4_K 34816 x 5120 33.8 | 27.0, 4096 x 8192 15.2 | 11.1, 1000 x 17408 16.6 | 10.3; Q6_K 5120 x 17408 32.2 | 23.7; Q8_0
+// 9429 x 9600 41.7 | 32.6; 16 rows Q4_K 34816 x 5120 53.3 | 34.5, Q6_K 5120 x 17408 41.3 | 26.9; 32 rows Q4_K 34816 x 5120 83.8 | 58.
+// ------------------------------------------------------------------------------------------------
+struct ResidentParams {
+    const uint8_t* W;
+    const uint16_t* Xp;   // prepared activations: [nchunks][16 NT][XR] f16
+    const float* X;       // or the rows as they are, [T, K]
+    float* Y;             // [T, N], or [parts][T, N] partial sums
+    int T, N, K, nblk, chunks_each, chunks_over, tiles_each, tiles_over, xp_sets;   // xp_sets: sets of eight activation rows in Xp
+    size_t row_bytes;
+};
+constexpr int RES_WAVES = 16;
+// chunks whose operand rows fit beside the waves' images into the 160 KiB of LDS
+template <class F, int NT>
+constexpr int resident_chunks() { return (163840 - RES_WAVES * 16 * F::LROW) / (16 * NT * XR * 2); }
+
+template <class F, int NT, bool OWN_X>
+__global__ void __launch_bounds__(64 * RES_WAVES, RES_WAVES / 4) gemm_q_f16x2_resident_kernel(ResidentParams p) {
+    constexpr int MAXC = resident_chunks<F, NT>(), WP = 16 * F::PARTS, NW = (WP + 63) / 64, NTL = (16 * F::TAILS + 63) / 64, WV = RES_WAVES;
+    static_assert(16 * F::LROW >= 512 * NT, "a wave's share of a tile's sums fits its image");
+    __shared__ __attribute__((aligned(16))) uint16_t Xs[MAXC * 16 * NT * XR];
+    __shared__ __attribute__((aligned(16))) uint8_t Wl[WV][16 * F::LROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g4 = lane >> 4, c = lane & 15;
+    uint8_t* const wl = Wl[wave];
+    const int part = blockIdx.x, j = blockIdx.y;                // the workgroup's chunks and tiles, shared out to within one
+    const int c0 = part * p.chunks_each + (part < p.chunks_over ? part : p.chunks_over), cp = p.chunks_each + (part < p.chunks_over);
+    const int tile0 = j * p.tiles_each + (j < p.tiles_over ? j : p.tiles_over), units = (p.tiles_each + (j < p.tiles_over)) * cp;
+    auto run_of = [&](int w) { return (int)((uint32_t)(w * units) / WV); };
+    const int lo = run_of(wave), hi = run_of(wave + 1);
+    const int t0 = blockIdx.z * (8 * NT), T = p.T - t0;         // the first activation row of the workgroup's set, and how many are left
+
+    // A lane's pieces of a unit lie at the same distance from the unit's first byte throughout (Q8_0: but for a last chunk that is not full). The last tile is the
+    // weight's last sixteen rows: it reads, and does not store, rows of the tile before it where there are too few; rows past the end of a smaller weight repeat its last row.
+    const int rmax = p.N < 16 ? p.N - 1 : 15;
+    u32x4 G[NW];
+    uint32_t gt[NTL ? NTL : 1], at[NW], tat[NTL ? NTL : 1];
+    auto piece = [&](int k) { const int pc = k * 64 + lane; return pc < WP ? pc : WP - 1; };
+    auto tail = [&](int k) { const int tc = k * 64 + lane; return tc < 16 * F::TAILS ? tc : 16 * F::TAILS - 1; };
 #pragma unroll
-        for (int j = 0; j < 24; j++) v[j] = q[(size_t)(k0 + j < nk ? k0 + j : 0) * slot];
-#pragma unroll
-        for (int j = 0; j < 24; j++)
-            if (k0 + j < nk) a += v[j];
+    for (int k = 0; k < NW; k++) {
+        const int row = piece(k) / F::PARTS;
+        at[k] = (uint32_t)(row < rmax ? row : rmax) * (uint32_t)p.row_bytes + (F::SLICE_SCALE ? 0u : F::piece_off(0, piece(k) - row * F::PARTS, p.nblk));
     }
-    Y[(size_t)t * N + n] = a;
+#pragma unroll
+    for (int k = 0; k < NTL; k++) {
+        const int row = tail(k) / (F::TAILS ? F::TAILS : 1);
+        bool live;
+        tat[k] = (uint32_t)(row < rmax ? row : rmax) * (uint32_t)p.row_bytes + (F::SLICE_SCALE ? 0u : F::tail_off(0, tail(k) - row * F::TAILS, p.nblk, live));
+    }
+    auto row0_of = [&](int tile) { const int r = (tile0 + tile) * 16; return r + 16 <= p.N ? r : p.N < 16 ? 0 : p.N - 16; };
+    auto load_w = [&](int tile, int ck) {
+        const uint8_t* b = p.W + (size_t)row0_of(tile) * p.row_bytes + (F::SLICE_SCALE ? 0u : (uint32_t)(c0 + ck) * F::BLOCK);
+#pragma unroll
+        for (int k = 0; k < NW; k++) G[k] = F::ldg(b + (at[k] + (F::SLICE_SCALE ? F::piece_off(c0 + ck, piece(k) % F::PARTS, p.nblk) : 0u)));
+#pragma unroll
+        for (int k = 0; k < NTL; k++) {
+            bool live;
+            gt[k] = *(const uint16_t*)(b + (tat[k] + (F::SLICE_SCALE ? F::tail_off(c0 + ck, tail(k) % (F::TAILS ? F::TAILS : 1), p.nblk, live) : 0u)));
+        }
+    };
+    auto park_w = [&](int ck) {
+#pragma unroll
+        for (int k = 0; k < NW; k++) {
+            const int pc = piece(k), row = pc / F::PARTS;
+            *(u32x4*)(wl + row * F::LROW + F::piece_lds(pc - row * F::PARTS)) = G[k];
+        }
+#pragma unroll
+        for (int k = 0; k < NTL; k++) {
+            const int tc = tail(k), row = tc / (F::TAILS ? F::TAILS : 1);
+            bool live;
+            F::tail_off(c0 + ck, tc - row * F::TAILS, p.nblk, live);
+            *(uint16_t*)(wl + row * F::LROW + F::tail_lds(tc - row * F::TAILS)) = live ? (uint16_t)gt[k] : (uint16_t)0;
+        }
+    };
+    int tile = lo / cp, ck = lo - tile * cp;
+
+    // ---- the operand rows of the workgroup's chunks (no branch among the loads; the rows are waited for first, the weights only once they are due)
+    if constexpr (OWN_X) {
+        static_assert(MAXC * NT <= WV, "a chunk of a set of eight rows to a wave");
+        const int set = NT == 1 ? 0 : wave & 1, mine = NT == 1 ? wave : wave >> 1, k = (c0 + mine) * CHUNK + 4 * lane;
+        f32x4 xr[8];
+        if (mine < cp) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) xr[r] = *(const f32x4*)(p.X + (size_t)(t0 + (8 * set + r < T ? 8 * set + r : 0)) * p.K + (k < p.K ? k : 0));
+        }
+        asm volatile("" ::: "memory");
+        if (lo < hi) load_w(tile, ck);
+        asm volatile("" ::: "memory");
+        if (mine < cp) {
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+                if (8 * set + r >= T || k >= p.K) xr[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            split_chunk<F>(xr, Xs + (mine * NT + set) * 16 * XR, lane);
+        }
+    } else {
+        constexpr int EACH = 2 * NT * XR, NP = (MAXC * EACH + 64 * WV - 1) / (64 * WV);   // 16-byte pieces of a chunk
+        const u32x4* src = (const u32x4*)p.Xp + ((size_t)c0 * p.xp_sets + blockIdx.z * NT) * (2 * XR);
+        const int pieces = cp * EACH;
+        u32x4 st[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int pc = i * 64 * WV + tid < pieces ? i * 64 * WV + tid : 0, k = pc / EACH;
+            st[i] = src[(size_t)k * p.xp_sets * (2 * XR) + (pc - k * EACH)];
+        }
+        asm volatile("" ::: "memory");
+        if (lo < hi) load_w(tile, ck);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (i * 64 * WV + tid < pieces) ((u32x4*)Xs)[i * 64 * WV + tid] = st[i];
+    }
+    __syncthreads();
+
+    float* const Y = p.Y + ((size_t)part * p.T + t0) * p.N;
+    // what a lane holds of a tile's outputs: rows 8 q + 4 (g4 & 1) + 2 h + (g4 >> 1), column c
+    auto store = [&](int tl, const float (&v)[NT][2]) {
+        const int n = row0_of(tl) + c;
+#pragma unroll
+        for (int q = 0; q < NT; q++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int t = 8 * q + 4 * (g4 & 1) + 2 * h + (g4 >> 1);
+                if (t < T && n < p.N && n >= (tile0 + tl) * 16) Y[(size_t)t * p.N + n] = v[q][h];
+            }
+    };
+    f32x4 total[NT];
+    float head[NT][2], last[NT][2];                             // sums of a tile that an earlier wave began; of one that a later wave ends
+#pragma unroll
+    for (int q = 0; q < NT; q++) {
+        total[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int h = 0; h < 2; h++) head[q][h] = last[q][h] = 0.f;
+    }
+    bool open = false;                                          // the wave began its last tile and does not end it
+    int first = ck;
+    const int a_rd = c * XR + 8 * g4, m_rd = c * XR + CHUNK + (g4 ? 8 : 0);
+    auto one_unit = [&](auto Next) {                            // Next: there is another unit after this one
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the image is the wave's own: its accesses complete in order
+        park_w(ck);
+        const int nt = ck + 1 == cp ? tile + 1 : tile, nck = ck + 1 == cp ? 0 : ck + 1;
+        if constexpr (decltype(Next)::value) load_w(nt, nck);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint16_t* const xs = Xs + ck * 16 * NT * XR;
+        typename F::Raw raw;
+        F::from_lds(raw, wl + c * F::LROW, g4);
+        typename F::Ctx x;
+        f32x4 acc[NT], ct[NT];
+        float dprev = 0.f;
+#pragma unroll
+        for (int q = 0; q < NT; q++) { acc[q] = (f32x4){0.f, 0.f, 0.f, 0.f}; ct[q] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
+        static_for<0, 8>([&](auto Ic) {
+            constexpr int I = decltype(Ic)::value;
+            F::template pre<I>(raw, g4, x);
+            const f16x8 b = F::template frag<I>(raw, x);
+            f32x4 cur[NT];
+#pragma unroll
+            for (int q = 0; q < NT; q++) {
+                const f16x8 a = *(const f16x8*)(xs + a_rd + 16 * q * XR + 32 * I);
+                cur[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, F::SLICE_SCALE ? (f32x4){0.f, 0.f, 0.f, 0.f} : acc[q], 0, 0, 0);
+            }
+            if constexpr (F::SLICE_SCALE && I > 0) {            // as in the row-streaming kernel
+#pragma unroll
+                for (int q = 0; q < NT; q++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) ct[q][r] = fmaf(dprev, acc[q][r], ct[q][r]);
+            }
+#pragma unroll
+            for (int q = 0; q < NT; q++) acc[q] = cur[q];
+            dprev = x.d;
+        });
+        if constexpr (F::HAS_MIN) {
+            const f16x8 bm = F::mins(raw, g4);
+#pragma unroll
+            for (int q = 0; q < NT; q++) {
+                const f32x4 accm = __builtin_amdgcn_mfma_f32_16x16x32_f16(*(const f16x8*)(xs + m_rd + 16 * q * XR), bm, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++) ct[q][r] = fmaf(x.dm, accm[r], ct[q][r]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NT; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                total[q][r] = fmaf(*(const float*)(xs + (16 * q + 4 * g4 + r) * XR + XSCALE), fmaf(x.d, acc[q][r], ct[q][r]), total[q][r]);
+        if (!decltype(Next)::value || nck == 0) {
+            float v[NT][2];
+#pragma unroll
+            for (int q = 0; q < NT; q++) {                      // lanes g4 and g4 ^ 2 hold the hi and the lo part of the same output
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(total[q][2 * h]), __float_as_uint(total[q][2 * h + 1]), false, false);
+                    v[q][h] = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+                }
+                total[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+            if (first == 0 && nck == 0) {
+                store(tile, v);
+            } else {
+                open = first == 0;
+#pragma unroll
+                for (int q = 0; q < NT; q++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        if (open) last[q][h] = v[q][h];
+                        else head[q][h] = v[q][h];
+                    }
+            }
+            first = 0;
+        }
+        if (decltype(Next)::value) { tile = nt; ck = nck; }
+    };
+    if (lo < hi) {
+        for (int u = lo; u + 1 < hi; u++) one_unit(std::true_type{});
+        one_unit(std::false_type{});
+    }
+    // ---- the tiles that several waves share: by the wave that began it
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int q = 0; q < NT; q++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) ((float*)wl)[(2 * q + h) * 64 + lane] = head[q][h];
+    __syncthreads();
+    if (!open) return;
+    const int end = (tile + 1) * cp;
+    for (int w = wave + 1; w < WV && run_of(w) < end; w++) {
+        if (run_of(w) == run_of(w + 1)) continue;
+#pragma unroll
+        for (int q = 0; q < NT; q++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) last[q][h] += ((const float*)Wl[w])[(2 * q + h) * 64 + lane];
+    }
+    store(tile, last);
+}
+
+// Y = partial output 0 + partial output 1 + ... in that order
+__global__ void __launch_bounds__(256) sum_parts_kernel(float* __restrict__ Y, const float* __restrict__ part, size_t n, int parts) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float a = part[i];
+    for (int k0 = 1; k0 < parts; k0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = part[(size_t)(k0 + k < parts ? k0 + k : 0) * n + i];
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (k0 + k < parts) a += v[k];
+    }
+    Y[i] = a;
 }
 
 __global__ void zero_f32_kernel(float* __restrict__ out, size_t n) {
@@ -1263,7 +1534,6 @@ struct Plan {
     long long wgs;        // workgroups that are resident together
     unsigned grid;
     bool split;
-    int kmax;             // most workgroups that hold part of one group's K
     int group;            // rows of a group: 256 for up to 8 activation rows (the eight-wave kernel), else 128
 };
 
@@ -1271,9 +1541,11 @@ struct Plan {
 template <class F>
 constexpr int slots(int nt) { return nt == 1 ? F::ROWS_OCCUPANCY : (nt == 2 && F::ROWS_AT_16 ? 2 : F::occupancy(nt)); }
 
+int prepared_sets(size_t t) { return t <= 8 ? 1 : t <= 16 ? 2 : 4; }   // sets of eight activation rows among the prepared operand rows
+
 Plan make_plan(const fhip_weight* w, size_t t) {
     Plan q;
-    q.nt = t <= 8 ? 1 : (t <= 16 ? 2 : 4);
+    q.nt = prepared_sets(t);
     q.nchunks = (int)((w->cols + CHUNK - 1) / CHUNK);
     const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     // the eight-wave kernel (groups of 256 rows, one workgroup per CU): up to 8 rows on a K-quant weight of 48 MB and more whose
@@ -1295,11 +1567,6 @@ Plan make_plan(const fhip_weight* w, size_t t) {
     else q.grid = (unsigned)(q.units < wgs ? q.units : wgs);
     q.split = q.grid != (unsigned)groups;
     q.groups = groups;
-    q.kmax = 1;
-    for (long long g = 0; g < groups && q.split; g++) {
-        const int nk = holder_of((g + 1) * q.nchunks - 1, q.grid, q.units) - holder_of(g * q.nchunks, q.grid, q.units) + 1;
-        if (nk > q.kmax) q.kmax = nk;
-    }
     return q;
 }
 
@@ -1314,25 +1581,24 @@ bool own_x(const fhip_weight* w, const Plan& q, const float* d_x) {
 }
 
 template <class F>
-int launch_xsplit_fmt(const float* d_x, size_t t, size_t k, bool swiglu, const Plan& q, uint16_t* d_xp, hipStream_t s, float* zero,
+int launch_xsplit_fmt(const float* d_x, size_t t, size_t k, bool swiglu, uint16_t* d_xp, hipStream_t s, float* zero,
                       size_t zero_n, const fhip::F16Parts& src) {
-    const dim3 grid((unsigned)q.nchunks, (unsigned)(8 * q.nt)), wg(256);
-    if (swiglu) hipLaunchKernelGGL((xsplit_f16_kernel<F, true>), grid, wg, 0, s, d_x, (int)t, (int)k, q.nt, d_xp, zero, zero_n, src);
-    else hipLaunchKernelGGL((xsplit_f16_kernel<F, false>), grid, wg, 0, s, d_x, (int)t, (int)k, q.nt, d_xp, zero, zero_n, src);
+    const int nt = prepared_sets(t);
+    const dim3 grid((unsigned)((k + CHUNK - 1) / CHUNK), (unsigned)(8 * nt)), wg(256);
+    if (swiglu) hipLaunchKernelGGL((xsplit_f16_kernel<F, true>), grid, wg, 0, s, d_x, (int)t, (int)k, nt, d_xp, zero, zero_n, src);
+    else hipLaunchKernelGGL((xsplit_f16_kernel<F, false>), grid, wg, 0, s, d_x, (int)t, (int)k, nt, d_xp, zero, zero_n, src);
     return fhip::check_hip(hipGetLastError(), "xsplit_f16 launch");
 }
 
 template <class F>
-int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, hipStream_t s, bool y_cleared, float* d_part,
-               fhip::F16Parts* deferred) {
+int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, hipStream_t s, bool y_cleared) {
     const Plan q = make_plan(w, t);
     F16Params p;
     p.W = w->d_raw; p.Xp = d_xp; p.X = d_x; p.K = (int)w->cols; p.Y = d_y;
-    p.part = q.split ? d_part : nullptr; p.kmax = q.kmax;
     p.T = (int)t; p.N = (int)w->rows; p.nchunks = q.nchunks; p.row_bytes = w->row_bytes;
     p.nblk = (int)(w->cols / 32);
     p.units = q.units; p.group = q.group;
-    if (q.split && !y_cleared && !d_part) {
+    if (q.split && !y_cleared) {
         const size_t n = t * w->rows;
         hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_y, n);
     }
@@ -1354,10 +1620,6 @@ int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, siz
     } else {
         return fhip::set_error(FHIP_ERR_SHAPE, "f16x2 matmul: this format takes at most 16 activation rows, got %zu", t);
     }
-    if (deferred) *deferred = fhip::F16Parts{p.part, p.kmax, p.nchunks, (int)q.grid, p.units, q.group};
-    if (p.part && !deferred)
-        hipLaunchKernelGGL(sum_split_kernel, dim3((unsigned)q.groups, (unsigned)((t * q.group + 255) / 256)), dim3(256), 0, s, d_y, (const float*)d_part, p.T, p.N,
-                           p.nchunks, p.units, (int)q.grid, p.kmax, q.group);
     return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
 }
 
@@ -1397,61 +1659,122 @@ int launch_held_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y
     return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
 }
 
+struct ResPlan { int nt, sets, parts, per_part; };
+template <class F>
+constexpr int resident_chunks_of(int nt) { return nt == 1 ? resident_chunks<F, 1>() : resident_chunks<F, 2>(); }
+// How many ranges K is cut into: the fewest that fit, or more where the estimate below says so. In us, fitted to 676 products of three formats (100 .. 34816 x 512 .. 17408, 8 to
+// 32 rows, every number of ranges): a round of four waves' operand rows 1, the longest run of units, the sums' launch 1.7 and 0.9 a megabyte of partial outputs, the
+// rows an XCD fetches (workgroups go to the eight XCDs in turn: of 8 ranges each has one) 0.8 a megabyte; tiles that all sixteen waves share add a wave's sum at a time.
+// What it picks takes 1.015 of the best number's time in the mean, 1.09 at the 95th percentile.
+ResPlan resident_plan(const fhip_weight* w, size_t t) {
+    const int nchunks = (int)((w->cols + CHUNK - 1) / CHUNK), tiles = (int)((w->rows + 15) / 16), cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+    const int nt = t <= 8 ? 1 : 2, sets = ((int)t + 8 * nt - 1) / (8 * nt);
+    const int most = w->type == FHIP_Q6_K ? resident_chunks_of<Q6K>(nt) : w->type == FHIP_Q8_0 ? resident_chunks_of<Q80>(nt) : w->type == FHIP_Q5_K ? resident_chunks_of<Q5K>(nt) : resident_chunks_of<Q4K>(nt);
+    const double unit = w->type == FHIP_Q6_K ? 2.4 : w->type == FHIP_Q8_0 ? 3.0 : w->type == FHIP_Q5_K ? 2.2 : 2.0, rows = 8.0 * nt * sets;
+    ResPlan best{nt, sets, 0, 0};
+    double least = 0;
+    const int fewest = (nchunks + most - 1) / most;
+    for (int parts = fewest; parts <= nchunks && parts <= (fewest > 13 ? fewest + 3 : 16); parts++) {
+        const int per = std::max(1, std::min(cus / (parts * sets), tiles));
+        const int held = (nchunks + parts - 1) / parts, units = (tiles + per - 1) / per * held, turn = parts % 8 == 0 ? 8 : parts % 4 == 0 ? 4 : parts % 2 == 0 ? 2 : 1;
+        const double us = (held * nt + 3) / 4 + unit * ((units + RES_WAVES - 1) / RES_WAVES) + (parts > 1 ? 1.7 + 3.6e-6 * parts * rows * w->rows : 0.0) + 3.2e-6 * rows * w->cols / turn +
+                          (units <= RES_WAVES ? 0.08 * held : 0.0);
+        if (!best.parts || us < least) { best.parts = parts; best.per_part = per; least = us; }
+    }
+    return best;
+}
+
+template <class F>
+int launch_resident_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, float* d_part, hipStream_t s, fhip::F16Parts* deferred) {
+    const ResPlan q = resident_plan(w, t);
+    ResidentParams p;
+    p.W = w->d_raw; p.Xp = d_xp; p.X = d_x; p.Y = q.parts > 1 ? d_part : d_y;
+    p.T = (int)t; p.N = (int)w->rows; p.K = (int)w->cols; p.nblk = (int)(w->cols / 32); p.row_bytes = w->row_bytes; p.xp_sets = prepared_sets(t);
+    const int tiles = (int)((w->rows + 15) / 16), nchunks = (int)((w->cols + CHUNK - 1) / CHUNK);
+    p.chunks_each = nchunks / q.parts; p.chunks_over = nchunks % q.parts; p.tiles_each = tiles / q.per_part; p.tiles_over = tiles % q.per_part;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)q.parts, (unsigned)q.per_part, (unsigned)q.sets), dim3(64 * RES_WAVES), 0, s, p); };
+    if (q.nt == 1) {
+        if (d_xp) go(gemm_q_f16x2_resident_kernel<F, 1, false>);
+        else go(gemm_q_f16x2_resident_kernel<F, 1, true>);
+    } else {
+        if (d_xp) go(gemm_q_f16x2_resident_kernel<F, 2, false>);
+        else go(gemm_q_f16x2_resident_kernel<F, 2, true>);
+    }
+    const size_t n = t * w->rows;
+    if (deferred) *deferred = fhip::F16Parts{d_part, q.parts > 1 ? q.parts : 0, n, w->rows};
+    else if (q.parts > 1) hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_y, (const float*)d_part, n, q.parts);
+    return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
+}
+
 }  // namespace
 
 namespace fhip {
 
-// Where the held kernel is the faster one: the other kernels' time over its own (above 1: faster), cold weights, sums in order. Tiles (of 16 weight rows) are counted in
-// the chip's CUs.
-// - One chunk (256 columns): up to three and a half tiles a CU: Q4_K at 8 rows 3.4 tiles 1.13, 4.4 1.01, 6.6 0.91, at 16 3.4 1.24, 5.9 0.81; Q8_0 at 8 to twelve (8.5 1.19, 17 1.02).
-// - 2 to 16 chunks, up to eight rows: always (Q4_K 2048 columns 0.1 tiles 1.59, 1.0 1.68, 37 1.22), but for two or three of a K-quant with more than 24 tiles (Q4_K 512
-//   columns 24 tiles 1.06, 37 0.90). Nine to sixteen: with long rows always (Q4_K 4096 columns 8.5 tiles 1.55, 37 1.35), with few chunks until the others cut
-//   nothing along K (Q5_K 1024 columns 5.9 tiles 1.83, 11.7 0.93); Q6_K from four chunks to 24 tiles (17 tiles 1.22; 37 of 5 chunks 0.87), Q8_0 from two always (17 1.25). More: four tiles, to nine
-//   where the others cut (Q4_K at 32 rows, 1024 columns 6.6 tiles 2.06, 8.5, not cut, 0.97).
-// - 17 to 24 chunks, two or three of them one after the other in a wave. Up to eight rows: Q4_K and Q5_K from half a tile on (5120 columns 0.2 tiles 0.90, 0.5 1.01,
-//   0.7 1.05), Q6_K and Q8_0 from where the others' units (128 rows x a chunk) are more than the CUs (0.2 0.89, 0.5 1.08). With minima, not in a second pass of tiles while
-//   the others have three units a CU at most, which run side by side (Q5_K 1.06 tiles of 20 chunks 0.93, 1.25 1.07). More rows: up to HELD_TILES, 20 chunks, last
-//   inside | first outside: Q4_K at 16 rows 11.7 tiles 1.05 | 24 0.96, at 24 8.5 1.04 | 17 0.87, at 32 4.4 1.13 | 6.6 0.99; Q5_K 3.4 1.05 | 5.9 0.96, 6.6 1.08 |
-//   8.5 0.98, 4.4 1.07 | 6.6 0.92; Q6_K 8.5 1.12 | 11.7 0.96, 2.9 1.22 | 6.6 1.02, 2.9 1.07 | 4.4 1.00; Q8_0 8.5 1.08 | 11.7 0.96.
-// - Beyond that, Q6_K and Q8_0 of 17 to 24 chunks at up to sixteen rows and any Q6_K at more, whose other kernel keeps two and one workgroup a CU: where its last round is
-//   mostly idle (16 rows 17 tiles, 547 workgroups of 1024, Q6_K 1.20 .. 1.36, Q8_0 1.25 .. 1.27, 11.7 tiles, 375 of 512, 0.94 .. 0.97; Q6_K at 24 rows 8.5 tiles, 272 of
-//   512, 1.20 .. 1.56, 5.9, 188 of 256, 0.91 .. 1.16, 6.6, 211 of 256, 0.88 .. 1.05; at 32 8.5 1.02 .. 1.27, 17, 547 of 768, 0.78 .. 0.97).
-// - summed_later: the next launch adds the others' partial sums as it reads them, and Q6_K at 17 rows and more then loses 1 - 13 % with more than 16 chunks or, at 32
-//   rows, two tiles a CU (feed-forward block 2560 x 9728 at 32 rows 63.3 us with the others, 69.6 with it; 2560 x 4096 at 32 46.3 | 46.3).
-// - Sums by atomics (FHIP_BATCH_AUTO) save the others a launch: of 13 to 16 chunks at up to eight rows from half a tile on (Q4_K 4096 columns 0.2 tiles 0.89, 0.7 1.09), of
-//   9 to 16 at more than 16 four tiles at most (Q4_K 3072 columns at 32 rows 4.4 tiles 1.01, 6.6 0.82), of more: up to eight rows from one and a half (Q8_0 5120 columns
-//   0.5 tiles 0.98, 2.0 1.31), with minima only over 20 chunks (Q4_K 20 chunks 2.2 tiles 0.89, 24 1.05), to sixteen a half to four (Q4_K 0.2 0.85, 0.5 1.03, 2.9 1.05, 6.6 0.89; not
-//   Q5_K, 2.2 0.87), to 24 three, to 32 two (Q4_K 2.9 1.04, 4.4 0.90; 2.0 1.04, 2.9 0.90), Q6_K while tiles times sets of eight rows are two and a half (24 rows 0.7 1.07, 1.0 0.88).
-constexpr int HELD_TILES[3][3] = {{12, 9, 6}, {4, 7, 5}, {9, 4, 3}};   // Q4_K; Q5_K; Q6_K and Q8_0: at up to 16, 24, 32 rows
+// Where the held kernel is faster than the streaming ones that add by atomics (FHIP_BATCH_AUTO): their time over its own, cold weights. Tiles (of 16 weight rows) are counted
+// in the chip's CUs.
+// - One chunk (256 columns): up to three and a half tiles a CU; Q8_0 at 8 rows to twelve.
+// - Up to eight rows: of 2 to 12 chunks always, but for two or three of a K-quant with more than 24 tiles; of 13 to 16 from half a tile on (Q4_K 4096 columns 0.2 tiles 0.89,
+//   0.7 1.09), of more from one and a half (Q8_0 5120 columns 0.5 tiles 0.98, 2.0 1.31), with minima only over 20 chunks (Q4_K 20 chunks 2.2 tiles 0.89, 24 1.05).
+// - Nine to sixteen: up to four tiles, with long rows always, with few chunks until the others cut nothing along K; beyond 16 chunks from a half to four (Q4_K 0.2 0.85, 0.5 1.03,
+//   2.9 1.05, 6.6 0.89; not Q5_K, 2.2 0.87), and Q6_K and Q8_0 where the others' last round is mostly idle (17 tiles, 547 workgroups of 1024, 1.20 .. 1.36).
+// - More: up to four tiles, to nine where the others cut (not of 9 chunks on: Q4_K 3072 columns at 32 rows 4.4 tiles 1.01, 6.6 0.82); beyond 16 chunks to 24 rows three, to 32 two (Q4_K
+//   2.9 1.04, 4.4 0.90; 2.0 1.04, 2.9 0.90), Q6_K while tiles times sets of eight rows are two and a half (24 rows 0.7 1.07, 1.0 0.88), and where the last round is mostly idle.
 int places_taken(const Plan& q) { return (int)(100 * q.groups / ((q.groups + q.wgs - 1) / q.wgs * q.wgs)); }   // percent of its rounds' workgroups
-bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y, bool summed_later) {
-    if (!gemm_f16x2_supports(w, t) || !d_x || ((uintptr_t)d_x & 15) != 0 || w->rows > 0x7FFFFF00ull) return false;
-    // (all workgroups read the rows: none may have written over them)
-    if ((uintptr_t)d_y < (uintptr_t)(d_x + t * w->cols) && (uintptr_t)d_x < (uintptr_t)(d_y + t * w->rows)) return false;
+bool held_beats_streaming(const fhip_weight* w, size_t t) {
     const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16, sets = (t + 7) / 8;
     const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
-    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, atomics = w->batch_policy != FHIP_BATCH_ORDERED;
-    if (chunks > 24) return false;
+    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0;
     if (chunks == 1) return 2 * tiles <= 7 * cus || (q8 && t <= 8 && tiles <= 12 * cus);
     if (t <= 8) {
         if (chunks <= 3) return q8 || tiles <= 24 * cus;
-        if (chunks <= 16) return !atomics || chunks <= 12 || 2 * tiles > cus;
-        if (atomics) return (q6 || q8 || chunks > 20) && 2 * tiles > 3 * cus;
-        if (q6 || q8) return (w->rows + 127) / 128 * chunks > cus;
-        return 2 * tiles >= cus && (tiles <= cus || tiles * chunks > 24 * cus);
+        if (chunks <= 16) return chunks <= 12 || 2 * tiles > cus;
+        return (q6 || q8 || chunks > 20) && 2 * tiles > 3 * cus;
     }
     if (t <= 16) {
         if (chunks <= 16) return tiles <= 4 * cus || q8 || chunks >= (q6 && tiles <= 24 * cus ? 4 : 8) || make_plan(w, t).split;
         if ((q6 || q8) && tiles > 9 * cus) return places_taken(make_plan(w, t)) < 70;
-        if (atomics) return w->type != FHIP_Q5_K && 2 * tiles >= cus && tiles <= 4 * cus;
-        return tiles <= HELD_TILES[w->type == FHIP_Q4_K ? 0 : w->type == FHIP_Q5_K ? 1 : 2][0] * cus;
+        return w->type != FHIP_Q5_K && 2 * tiles >= cus && tiles <= 4 * cus;
     }
     const Plan q = make_plan(w, t);
-    if (summed_later && q6 && q.split && (chunks > 16 || (t > 24 && tiles > 2 * cus))) return false;
-    if (q6 && (t <= 24 && !atomics ? tiles > 4 * cus : q.groups > q.wgs) && places_taken(q) < (t <= 24 ? 70 : 60)) return true;
-    if (chunks <= 16) return tiles <= 4 * cus || (tiles <= 9 * cus && q.split && !(atomics && chunks > 8));
-    if (atomics) return q6 ? 2 * tiles * sets <= 5 * cus : tiles <= (t <= 24 ? 3 : 2) * cus;
-    return tiles <= HELD_TILES[w->type == FHIP_Q4_K ? 0 : w->type == FHIP_Q5_K ? 1 : 2][sets - 2] * cus;
+    if (q6 && q.groups > q.wgs && places_taken(q) < (t <= 24 ? 70 : 60)) return true;
+    if (chunks <= 16) return tiles <= 4 * cus || (tiles <= 9 * cus && q.split && chunks <= 8);
+    return q6 ? 2 * tiles * sets <= 5 * cus : tiles <= (t <= 24 ? 3 : 2) * cus;
+}
+// And where it keeps a product whose sums are in order from the resident kernel: that one's time over its own (676 products of Q4_K, Q6_K and Q8_0).
+// - Up to 16 chunks: where tiles are few the one launch and its sums in LDS are the faster (8 rows, 4096 x 4096 Q4_K 1.00, Q8_0 1.20; 4096 x 1024 1.22 .. 1.33; 16 rows
+//   4096 x 2048 1.24 .. 1.33). The resident kernel takes, of up to eight rows, short rows of many tiles (34816 x 512 Q4_K 0.75, Q6_K 0.87, 16000 x 1024 Q4_K 0.88) and nine or ten chunks of
+//   eight tiles and more (34816 x 2560 0.93, 0.93); of nine to sixteen, more than 4.1 tiles (34816 x 512 0.58 .. 0.81, x 1024 0.73 .. 0.88, x 2560 0.85 .. 0.97; five to eight chunks
+//   1.03 .. 1.08), with more than ten chunks two (8192 x 4096 0.97, 0.93, 0.87); of more two tiles (8192 x 2048 0.98 .. 0.85, 34816 x 512 0.47 .. 0.71), from 13 chunks on a half.
+// - 17 to 24: the resident kernel is the faster one throughout (8 rows, 5120 columns, 100 / 2048 / 8192 / 34816 rows: Q4_K 0.65, 0.70, 0.86, 0.93, Q6_K 0.67, 0.83, 0.95; 16 rows
+//   Q4_K 0.69, 0.73, 0.78, 0.71). Where the held one stays all the same its route is pinned by test_whole_rows_inside_a_workgroup: up to eight rows 24 chunks of Q4_K and Q5_K
+//   at a half to two tiles, Q6_K and Q8_0 at a half to 1.3 (0.80 .. 1.00 there); of more up to a third of a tile (0.70 .. 0.95), Q8_0 at up to sixteen up to 1.1.
+bool held_beats_resident(const fhip_weight* w, size_t t) {
+    const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16;
+    const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, mins = !q6 && !q8;
+    if (chunks > 16) {
+        if (t > 8) return q8 && t <= 16 ? 10 * tiles <= 11 * cus : 3 * tiles <= cus;
+        return mins ? chunks == 24 && 2 * tiles >= cus && tiles <= 2 * cus : 2 * tiles > cus && 10 * tiles <= 13 * cus;
+    }
+    if (chunks == 1) return 2 * tiles <= 7 * cus || (q8 && t <= 8 && tiles <= 12 * cus);
+    if (t <= 8) return !(((chunks == 9 || chunks == 10) && tiles >= 8 * cus) || (chunks <= (mins ? 4 : q6 ? 2 : 0) && 2 * tiles > 7 * cus));
+    if (t <= 16) return chunks > 10 ? tiles < 2 * cus : (chunks > 4 && chunks < 9) || 10 * tiles <= 41 * cus;
+    return tiles < 2 * cus && !(chunks > 12 && 2 * tiles >= cus);
+}
+// (all workgroups of a launch that stores y read the rows: none may have written over them)
+bool apart(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+    return (uintptr_t)d_y >= (uintptr_t)(d_x + t * w->cols) || (uintptr_t)d_x >= (uintptr_t)(d_y + t * w->rows);
+}
+bool gemm_f16x2_held_takes(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+    return gemm_f16x2_takes(w, t) && d_x && ((uintptr_t)d_x & 15) == 0 && w->rows <= 0x7FFFFF00ull && (w->cols + CHUNK - 1) / CHUNK <= 24 && apart(w, d_x, t, d_y);
+}
+bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+    return gemm_f16x2_held_takes(w, d_x, t, d_y) && (w->batch_policy == FHIP_BATCH_ORDERED ? held_beats_resident(w, t) : held_beats_streaming(w, t));
+}
+// A launch in front that prepares the rows costs 2 - 3 us (Q4_K, 8 rows, itself | prepared: 2048 x 5120 8.1 | 10.7, 34816 x 5120 27.0 | 28.7; 32 rows 2048 x 5120 11.4 | 14.7). From
+// 5120 columns on more than 16 rows keep it: the route is pinned by test_ffn_leaves_the_sums_of_a_cut_gate_up_to_the_next_launch.
+bool gemm_f16x2_resident_own_x(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
+    return (t <= 16 || w->cols < 20 * CHUNK) && d_x && ((uintptr_t)d_x & 15) == 0 && (gemm_f16x2_parts(w, t) > 1 || apart(w, d_x, t, d_y));
 }
 
 int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
@@ -1465,53 +1788,63 @@ int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, flo
     }
 }
 
+// (the entry points whose rows a caller prepares space for keep Q8_0 to 16 rows; where sums are in order it goes as far as the others)
+bool gemm_f16x2_takes(const fhip_weight* w, size_t t) {
+    return gemm_f16x2_supports(w, w && w->type == FHIP_Q8_0 && w->batch_policy == FHIP_BATCH_ORDERED && t > 16 && t <= 32 ? 16 : t);
+}
+
 bool gemm_f16x2_supports(const fhip_weight* w, size_t t) {
     if (!w || t < 1 || w->cols == 0 || w->cols > (size_t)MAXW * 1024) return false;
     if (w->type == FHIP_Q8_0) return t <= 16 && w->cols % 32 == 0;   // rows of any whole number of blocks
     return (w->type == FHIP_Q4_K || w->type == FHIP_Q5_K || w->type == FHIP_Q6_K) && t <= 32 && w->cols % CHUNK == 0;
 }
 
+int gemm_f16x2_parts(const fhip_weight* w, size_t t) { return resident_plan(w, t).parts; }
+// (the most any batch of up to t rows needs: a batch of fewer rows may be cut into more ranges)
+size_t gemm_f16x2_parts_bytes(const fhip_weight* w, size_t t) {
+    size_t m = 0;
+    for (size_t u : {t, (size_t)8, (size_t)16}) {
+        const int parts = u <= t ? gemm_f16x2_parts(w, u) : 1;
+        if (parts > 1) m = std::max(m, (size_t)parts * u * w->rows * sizeof(float));
+    }
+    return m;
+}
+int launch_gemm_f16x2_resident(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, float* d_part, hipStream_t s, F16Parts* deferred) {
+    switch (w->type) {
+        case FHIP_Q4_K: return launch_resident_fmt<Q4K>(w, d_xp, d_x, t, d_y, d_part, s, deferred);
+        case FHIP_Q5_K: return launch_resident_fmt<Q5K>(w, d_xp, d_x, t, d_y, d_part, s, deferred);
+        case FHIP_Q6_K: return launch_resident_fmt<Q6K>(w, d_xp, d_x, t, d_y, d_part, s, deferred);
+        case FHIP_Q8_0: return launch_resident_fmt<Q80>(w, d_xp, d_x, t, d_y, d_part, s, deferred);
+        default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "f16x2 matmul: no kernel for ggml type %u", w->type);
+    }
+}
+
 size_t gemm_f16x2_xp_bytes(const fhip_weight* w, size_t t) {
-    const Plan q = make_plan(w, t);
-    return (size_t)q.nchunks * 16 * q.nt * XR * sizeof(uint16_t);
+    return (w->cols + CHUNK - 1) / CHUNK * 16 * prepared_sets(t) * XR * sizeof(uint16_t);
 }
 
 bool gemm_f16x2_adds_into_y(const fhip_weight* w, size_t t) { return make_plan(w, t).split; }
 
-size_t gemm_f16x2_part_bytes(const fhip_weight* w, size_t t) {
-    const Plan q = make_plan(w, t);
-    return q.split ? (size_t)q.groups * q.kmax * 32 * q.group * sizeof(float) : 0;
-}
-// the most any batch of up to t rows needs (fewer rows can mean more resident workgroups, and so more contributors)
-size_t gemm_f16x2_part_bytes_upto(const fhip_weight* w, size_t t) {
-    size_t m = gemm_f16x2_part_bytes(w, t);
-    for (size_t u : {(size_t)8, (size_t)16})
-        if (u < t) m = std::max(m, gemm_f16x2_part_bytes(w, u));
-    return m;
-}
-
 int launch_xsplit_f16(const fhip_weight* w, const float* d_x, size_t t, bool swiglu, uint16_t* d_xp, hipStream_t s, float* zero, size_t zero_n,
                       const F16Parts* src_in) {
-    const Plan q = make_plan(w, t);
-    const F16Parts src = src_in ? *src_in : F16Parts{nullptr, 0, 0, 0, 0, 128};
+    const F16Parts src = src_in ? *src_in : F16Parts{nullptr, 0, 0, 0};
     switch (w->type) {
-        case FHIP_Q4_K: return launch_xsplit_fmt<Q4K>(d_x, t, w->cols, swiglu, q, d_xp, s, zero, zero_n, src);
-        case FHIP_Q5_K: return launch_xsplit_fmt<Q5K>(d_x, t, w->cols, swiglu, q, d_xp, s, zero, zero_n, src);
-        case FHIP_Q6_K: return launch_xsplit_fmt<Q6K>(d_x, t, w->cols, swiglu, q, d_xp, s, zero, zero_n, src);
-        case FHIP_Q8_0: return launch_xsplit_fmt<Q80>(d_x, t, w->cols, swiglu, q, d_xp, s, zero, zero_n, src);
+        case FHIP_Q4_K: return launch_xsplit_fmt<Q4K>(d_x, t, w->cols, swiglu, d_xp, s, zero, zero_n, src);
+        case FHIP_Q5_K: return launch_xsplit_fmt<Q5K>(d_x, t, w->cols, swiglu, d_xp, s, zero, zero_n, src);
+        case FHIP_Q6_K: return launch_xsplit_fmt<Q6K>(d_x, t, w->cols, swiglu, d_xp, s, zero, zero_n, src);
+        case FHIP_Q8_0: return launch_xsplit_fmt<Q80>(d_x, t, w->cols, swiglu, d_xp, s, zero, zero_n, src);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "f16x2 matmul: no kernel for ggml type %u", w->type);
     }
 }
 
 bool gemm_f16x2_own_x(const fhip_weight* w, const float* d_x, size_t t) { return own_x(w, make_plan(w, t), d_x); }
 
-int launch_gemm_f16x2(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y, hipStream_t s, bool y_cleared, float* d_part,
-                      F16Parts* deferred, const float* d_x) {
+int launch_gemm_f16x2(const fhip_weight* w, const uint16_t* d_xp, size_t t, float* d_y, hipStream_t s, bool y_cleared, const float* d_x) {
     switch (w->type) {
-        case FHIP_Q4_K: return launch_fmt<Q4K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
-        case FHIP_Q8_0: return launch_fmt<Q80>(w, d_xp, d_x, t, d_y, s, y_cleared, d_part, deferred);
+        case FHIP_Q4_K: return launch_fmt<Q4K>(w, d_xp, d_x, t, d_y, s, y_cleared);
+        case FHIP_Q5_K: return launch_fmt<Q5K>(w, d_xp, d_x, t, d_y, s, y_cleared);
+        case FHIP_Q6_K: return launch_fmt<Q6K>(w, d_xp, d_x, t, d_y, s, y_cleared);
+        case FHIP_Q8_0: return launch_fmt<Q80>(w, d_xp, d_x, t, d_y, s, y_cleared);
         default: return set_error(FHIP_ERR_UNSUPPORTED_TYPE, "f16x2 matmul: no kernel for ggml type %u", w->type);
     }
 }

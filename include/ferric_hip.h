@@ -187,11 +187,12 @@ int fhip_deq_raw(const uint8_t* h_raw, size_t nbytes, size_t n, uint32_t ggml_ty
  * Q4_K / Q5_K / Q6_K weight with rows of up to 10240 columns (Q8_0: four rows, 5120 columns) through its four-row form (the same arithmetic on the int8 matrix
  * instruction: every row has the bits it has in a batch of one; one launch, no workspace), three rows and more of the other 32-value formats, up to sixteen a
  * pass, through its wide form (the same, without a workspace too); otherwise, from three rows on (five
- * for Q8_0) Q4_K / Q5_K / Q6_K / Q8_0 weights are read once per group of up to 32 (Q8_0: 16) rows by the f16 hi/lo matrix-core
- * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Most products of up to 6144
- * columns are one launch that needs nothing beside its operands. The others keep their
- * prepared activations in a workspace the library owns per stream (fhip_workspace_reserve); inside a graph capture the
- * workspace cannot grow, and the call then fails with FHIP_ERR_ARG and says how many bytes to reserve beforehand.
+ * for Q8_0) Q4_K / Q5_K / Q6_K / Q8_0 weights are multiplied in groups of up to 32 (Q8_0 under FHIP_BATCH_AUTO: 16) rows by the f16 hi/lo matrix-core
+ * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Most products of up to 4096
+ * columns are one launch that needs nothing beside its operands. The others keep
+ * prepared activations or partial sums in a workspace the library owns per stream (fhip_workspace_reserve); inside a graph capture the
+ * workspace cannot grow, and a product of more than 6144 columns then fails with FHIP_ERR_ARG and says how many bytes to reserve beforehand; one of up to 6144
+ * columns is captured as one launch where no workspace serves it (its sums then in another order, the same to f32 rounding).
  * Non-finite activations: on the mat-vec kernel a NaN or infinite x gives what the f32 dot gives (NaN, +-inf by the weight's
  * sign); on the matrix-core kernels the whole output row of such an activation row is non-finite and no other row is touched. */
 int fhip_matmul_q(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, void* stream);

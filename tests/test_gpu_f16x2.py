@@ -424,3 +424,48 @@ def test_whole_rows_inside_a_workgroup(F, O, ty, rows, cols, t):
     assert (np.abs(y[good] - y64) <= bound + 1e-300).all()
     assert not y[1].any() and np.isnan(y[t - 1]).all() and not np.isfinite(y[t - 2]).any()
     assert np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
+
+
+@pytest.mark.parametrize("ty,rows,cols,t,own,cut", [
+    (Q4_K, 5, 6400, 8, True, True), (Q6_K, 17, 17408, 5, True, True), (Q8_0, 31, 6432, 7, True, True), (Q5_K, 300, 12288, 3, True, True),      # fewer units than waves; a last chunk that is not full
+    (Q5_K, 8210, 5120, 8, True, True), (Q4_K, 8193, 5376, 12, True, True), (Q6_K, 5200, 4608, 16, True, True),                                # tiles that waves share, a last tile of few rows
+    (Q4_K, 33001, 512, 6, True, False), (Q6_K, 20990, 768, 11, True, False), (Q8_0, 8200, 1056, 30, True, False),                              # whole rows; Q8_0 beyond sixteen
+    (Q8_0, 140, 6432, 17, False, True), (Q4_K, 1500, 5120, 32, False, True), (Q6_K, 2000, 6400, 25, False, True)])                             # two sets, prepared rows
+def test_operand_rows_in_a_workgroups_lds(F, O, ty, rows, cols, t, own, cut):
+    # sums of up to 256-column chunks in f32, as in the kernels it stands beside: their bar. A row of inf or NaN stays alone, and a second run has the same bits.
+    from conftest import ROUTES, route
+    from ferric_amd.synth import synth_weights
+    w = synth_weights(ty, rows, cols, rows + t)
+    x = np.random.default_rng(cols + t).standard_normal((t, cols)).astype(np.float32)
+    x[0] *= 2.0 ** 40
+    x[t - 1, -3], x[t - 2, 1] = np.nan, -np.inf
+    qm, xt = F.QMatrix.from_bytes(w, ty, rows, cols), F.Tensor.from_vec(x, x.shape)
+    qm.batch_policy(F.BATCH_ORDERED)
+    assert route(F, qm, xt, t) == [((ROUTES["OWN_ROWS"] if own else ROUTES["PREPARED"]) | (ROUTES["CUT"] if cut else 0), t)]
+    good = np.arange(t - 2)
+    y64, wn = O.matmul_f64(x[good], w, ty, rows, cols)
+    bound = TIGHT * wn[None, :] * np.linalg.norm(x[good].astype(np.float64), axis=1)[:, None]
+    y = xt.matmul_q(qm).to_vec().reshape(t, rows)
+    assert (np.abs(y[good] - y64) <= bound + 1e-300).all()
+    assert np.isnan(y[t - 1]).all() and not np.isfinite(y[t - 2]).any()
+    assert np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
+
+
+def test_a_cut_product_is_captured_without_a_workspace_where_one_launch_can_do_it(F):
+    # 20 chunks: two or more ranges of K, or the held kernel's one launch, which a capture on a stream without a workspace takes
+    from conftest import ROUTES, route
+    from ferric_amd.synth import synth_weights
+    rows, cols, t = 400, 5120, 6
+    w = F.QMatrix.from_bytes(synth_weights(Q5_K, rows, cols, 51), Q5_K, rows, cols)
+    w.batch_policy(F.BATCH_ORDERED)
+    x = np.random.default_rng(52).standard_normal((t, cols)).astype(np.float32)
+    xt, y, stream = F.Tensor.from_vec(x, x.shape), F.Tensor.empty((t, rows)), F.Stream()
+    assert route(F, w, xt, t) == [(ROUTES["OWN_ROWS"] | ROUTES["CUT"], t)]
+    want = xt.matmul_q(w).to_vec()
+    g = F.Graph.begin(stream)
+    F._lib.check(F._lib.load().fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, stream.handle))
+    g.end()
+    for _ in range(3):
+        F._lib.check(F._lib.load().fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
+        g.launch()
+        assert np.abs(y.to_vec(stream) - want).max() <= 2e-6 * np.abs(want).max()
