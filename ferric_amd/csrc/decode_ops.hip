@@ -932,17 +932,26 @@ void launch_attn_combine(const float* part, int n_head, int hd, int splits, floa
 //   accumulators, the running maximum's correction is skipped where no maximum moved.
 // Up to five query heads a KV head (SPL): the 16 columns hold every query three times and column n takes cut n / gq of its query's products
 // (the three sums meet at the end), a third of the values' instructions. Six to eight: a column a query, three instructions.
-// Scales come one row a lane and go round through LDS (the wave's own part of it), the cut queries are shared there. At head size 64 the next
-// round's key codes are requested when the scores are done; at 128 they would not fit the 128 registers that let four waves share a
-// SIMD, and the other waves' arithmetic runs under the request. The waves of a workgroup meet in LDS as above.
-// What bounds it: instruction issue. A wave's round is some 700 vector instructions (a fifth each: codes to bf16, probabilities times scales
-// and their cuts) and 32 matrix instructions of 16 cycles (SPL; 48 otherwise); the rows' bytes (71 MB at 8 KV heads of 128, 32768 Q8_0 keys) would take 13 us.
-// At that shape, us, before (values on f32 matrix instructions for six query heads and more, the dot-product kernel for fewer) -> now: 5 query
-// heads a KV head 38.3 -> 27.0, 8: 33.9 -> 26.4; head size 64, 4: 23.0 -> 17.2. Error against f64 (2-norm, relative, eighteen shapes) no larger in any:
-// 2.2e-7 .. 2.5e-7 before, 1.4e-7 .. 1.8e-7 with the combine launch's present order. Tried: the codes requested as consecutive
-// 16-byte pieces and turned through LDS (31 us at head size 128, level at 64: what the address unit saves goes into LDS reads and spills).
+// Scales and key codes are requested as they lie, a row's bytes by neighbouring lanes, and go round through LDS (the wave's own part of it): a lane's own
+// eight bytes of its key (row n) asked for directly cost the address unit a cycle a lane, 4 of the 7 thousand cycles of a round. Value codes come two blocks of a
+// row by 16 lanes and are exchanged between halves of them (pair_up). A round's keys are requested when the round before has its own in LDS, its
+// values when that round's are multiplied, the first round's keys in front of the post-processing; the raw heads before anything else, since loads return in
+// order. Every wave cuts up its own head, so one barrier stands in front of the keys, and the three cuts of a sum meet in LDS.
+// A workgroup a CU of eight waves, two a SIMD: 147 registers hold a round in flight, and the launch's fixed part (post-processing 4.5 us, the waves' sums 2)
+// is paid once a CU. Workgroup L is split L % splits of KV head L / splits: with splits a multiple of eight an XCD's workgroups share the lines that hold all heads' scales
+// of a row (KV head first, each of the eight XCDs fetched every one of them: 25.6 | 24.7 us).
+// What bounds it: the rows' bytes (71 MB at 8 KV heads of 128, 32768 Q8_0 keys, at 5.5 - 6 TB/s behind the first request: 12 - 13 us of 23), close behind
+// them instruction issue (640 vector instructions a round, a fifth each codes to bf16 and probabilities' cuts; 32 matrix instructions of 16 cycles, SPL).
+// At that shape, kernel trace, 5 query heads a KV head: two workgroups a CU, keys by row, values a half word a load, none of it ahead of its round 28.1 us; now 23.2.
+// With the combine launch, this kernel in that form -> now, us: head size 64, 8 KV heads, Q8_0 5200 / 16384 / 32768 keys 10.6 / 15.0 / 21.7 -> 8.8 / 11.0 / 14.8; 128, Q4_0,
+// 4 KV heads of 8, 32768 keys 19.9 -> 16.3; 98 shapes 0.81 of the time (geometric mean). Two rounds ahead: 28.1 (the waves that post-process wait to issue).
+// Before that, at that shape, us, values on f32 matrix instructions for six query heads and more, the dot-product kernel for fewer: 5 query
+// heads a KV head 38.3, 8: 33.9; head size 64, 4: 23.0. Error against f64 (2-norm, relative, eighteen shapes) no larger in any:
+// 2.2e-7 .. 2.5e-7 before, 1.4e-7 .. 1.8e-7 with the combine launch's present order.
 // Q4_1 is left to the kernel above: the minimum as a product of its own cost 2 % more error.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(8))) U4A8 { u32x4 v; };
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 union Frag { uint32_t w[4]; bf16x8 v; };
 // the upper halves of two f32: two bf16 (exact where the lower halves are zero)
@@ -976,17 +985,21 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                                                float scale, int splits, uint32_t window, float softcap, float* __restrict__ part, int gq,   // gq: query heads per KV head, at most 8 (SPL: 5)
                                                const QkvPostParams& fp, const KvqStore& st) {
     constexpr int NB = HD / 32, NT = LONG_KEYS / 16;                    // blocks of a row, tiles of 16 keys
-    constexpr bool Q8 = FMT == FHIP_KVQ_Q8_0, PRE = HD == 64;             // PRE: keys requested a round ahead
+    constexpr bool Q8 = FMT == FHIP_KVQ_Q8_0;
     constexpr int CW = Q8 ? 8 : 4;                                      // code words of a block
+    constexpr int LR = NB * CW / 4, KL = LONG_KEYS * LR / 64;           // lanes that request a row's key codes, 16 bytes each; requests of a round
+    constexpr int KROW = 16 * LR + 16;                                  // bytes of a row in LDS: sixteen rows' same 8 bytes lie in different banks
     static_assert(FMT == FHIP_KVQ_Q8_0 || FMT == FHIP_KVQ_Q4_0, "");
     __shared__ float sm_m[LONG_WAVES][8], sm_l[LONG_WAVES][8];
-    __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][8][HD + 4];    // rows four banks apart
+    constexpr int COLS = SPL ? 16 : 8;
+    __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][COLS][HD + 4];    // rows four banks apart
     __shared__ __attribute__((aligned(16))) float sm_d[LONG_WAVES][NB][64];   // rows 0 .. 31 the keys' scales, 32 .. 63 the values'
+    __shared__ __attribute__((aligned(16))) uint8_t sm_k[LONG_WAVES][LONG_KEYS * KROW];   // a round's key codes, row by row
     __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of column n's query at lane n + 16 g, three bf16 each
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
-    const int cut = SPL ? n / gq : 0, qn = SPL ? n - cut * gq : n;     // the column's query and, SPL, its cut (3: a column without one)
-    const int kvh = blockIdx.x, split = blockIdx.y, head0 = kvh * gq;
+    const int cut = SPL ? n / gq : 0;                                   // the cut column n takes of its query (3: a column without one)
+    const int kvh = blockIdx.y, split = blockIdx.x, head0 = kvh * gq;
     uint32_t len = len_dev ? *len_dev + 1u : len_host;
     if (len > len_host) len = len_host;
     const uint32_t first = (window > 0 && window < len) ? len - window : 0u;
@@ -994,45 +1007,90 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     const uint32_t k0 = first + (uint32_t)split * per, k1 = min(len, k0 + per);
     const int nblk = n_kv * NB;
 
-    uint32_t kw[NT][NB][2], sc[NB / 2];
-    auto request_k = [&](uint32_t kt) {
+    // What a round of 32 keys reads: key codes, scales (lanes 0 .. 31 the keys', 32 .. 63 the values'), and the value codes of block pair i at
+    // key 16 t + 4 g + r: two units a lane (a unit is what a lane's A row of one block takes at a key: a half word, Q8_0, or a byte), units 2 n and 2 n + 1
+    // of the pair's 32, so that lanes 0 .. 7 have the pair's first block and the others its second (pair_up).
+    struct Round { u32x4 k[KL]; uint32_t sc[NB / 2], v[NB / 2][NT][4]; } ra;
+    constexpr uint32_t STEP = LONG_KEYS * LONG_WAVES;
+    auto request_k = [&](Round& R, uint32_t kt) {
+        kt = min(kt, k1 - 1u);
         const uint32_t last = k1 - 1u - kt;                             // rows past the split re-read its last row and count nothing
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const size_t b = (size_t)(kt + min((uint32_t)(16 * t + n), last)) * nblk + (size_t)kvh * NB;
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const uint2 v = *(const uint2*)(qc.k_codes + (b + j) * CW + 2 * (g & (CW / 2 - 1)));
-                kw[t][j][0] = v.x; kw[t][j][1] = v.y;
-            }
-        }
+        for (int i = 0; i < KL; i++)
+            R.k[i] = ((const U4A8*)(qc.k_codes + ((size_t)(kt + min((uint32_t)(i * (64 / LR) + lane / LR), last)) * nblk + (size_t)kvh * NB) * CW + 4 * (lane % LR)))->v;
         const size_t b = ((size_t)(kt + min((uint32_t)(lane & 31), last)) * nblk + (size_t)kvh * NB);
         const uint32_t* sp = (const uint32_t*)((lane < 32 ? qc.k_scales : qc.v_scales) + b);
 #pragma unroll
-        for (int i = 0; i < NB / 2; i++) sc[i] = sp[i];
+        for (int i = 0; i < NB / 2; i++) R.sc[i] = sp[i];
+    };
+    const uint32_t row_b = (uint32_t)nblk * (CW * 4);                   // bytes from a row's codes to the next row's
+    auto load_units = [&](const char* p) -> uint32_t { return Q8 ? *(const uint32_t*)p : (uint32_t)*(const uint16_t*)p; };
+    auto request_v = [&](Round& R, uint32_t kt) {
+        kt = min(kt, k1 - 1u);
+        const uint32_t last = k1 - 1u - kt;
+        const char* vc = (const char*)(qc.v_codes + ((size_t)kt * nblk + (size_t)kvh * NB) * CW);
+        const uint32_t at = (uint32_t)(Q8 ? 4 * n : 2 * n);
+        if (last >= LONG_KEYS - 1u) {
+            // a lane's own part of the address is the same for every row (and fits 32 bits); the rest is the wave's
+            const uint32_t mine = (uint32_t)(4 * g) * row_b + at;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int i = 0; i < NB / 2; i++) R.v[i][t][r] = load_units(vc + (size_t)(16 * t + r) * row_b + i * (2 * CW * 4) + mine);
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    uint32_t mine = (uint32_t)(4 * g);
+                    asm volatile("" : "+v"(mine));                      // worked out here: kept from round to round these are eight more registers
+                    const char* p = vc + (size_t)min(mine + (uint32_t)(16 * t + r), last) * row_b + at;
+#pragma unroll
+                    for (int i = 0; i < NB / 2; i++) R.v[i][t][r] = load_units(p + i * (2 * CW * 4));
+                }
+        }
     };
     uint32_t kt = k0 + (uint32_t)(LONG_KEYS * wave);
     // the heads' rows, the token's rows and the waves' scratch rows lie where the sums of the waves will
     float* const sq = FUSED ? &sm_acc[0][0][0] : nullptr;               // [8][HD] | [2][HD] | [LONG_WAVES][HD]
     static_assert(18 * HD <= LONG_WAVES * 8 * (HD + 4), "");
     bool owner = false;
-    if constexpr (FUSED) {
-        const uint32_t pos = *len_dev;
-        owner = pos < fp.cap && (pos < len ? (pos >= k0 && pos < k1) : split == splits - 1);
-    }
-    if (PRE && kt < k1 && !owner) request_k(kt);
-    if constexpr (FUSED) {
-        const int njobs = gq + (owner ? 2 : 0);
-        const uint32_t pos = *len_dev;
-        PostHead<HD> raw[2];                                            // up to ten jobs for eight waves
+    PostHead<HD> raw[2];                                                // up to ten jobs for eight waves: the query heads, the key head, the value head
+    if constexpr (FUSED) {                                              // the first loads of all: behind the rows they would wait for them
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             const int j = wave + LONG_WAVES * r;
-            if (j < njobs)
+            if (j < gq + 2)
                 raw[r] = post_request<HD>(fp, j < gq ? head0 + j : (j == gq ? fp.n_head + kvh : fp.n_head + n_kv + kvh), j < gq ? fp.q_norm : (j == gq ? fp.k_norm : nullptr), lane);
         }
+        const uint32_t pos = *len_dev;
+        owner = pos < fp.cap && (pos < len ? (pos >= k0 && pos < k1) : split == splits - 1);
+    }
+    if (!owner) request_k(ra, kt);                                      // their trip runs under the post-processing
+    // A wave cuts its own query head up for all: lane 16 c + 4 j + g has dims 32 j + 8 g .. + 7 for the column of cut c (SPL; one column otherwise)
+    auto cut_up = [&](int h, const float* row) {
+        if (lane >= (SPL ? 48 : 16)) return;
+        const int j = (lane >> 2) & 3, gg = lane & 3, col = SPL ? h + (lane >> 4) * gq : h;
+        if (j >= NB) return;
+        float x[8];
+        load_dims<8>(row + 32 * j + 8 * gg, x);
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            sm_q[j][t][col + 16 * gg] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);   // exact
+        }
+    };
+    if (wave < NB && n >= (SPL ? 3 * gq : gq))                          // columns without a query
+#pragma unroll
+        for (int t = 0; t < 3; t++) sm_q[wave][t][lane] = make_uint4(0u, 0u, 0u, 0u);
+    if constexpr (FUSED) {
+        const int njobs = gq + (owner ? 2 : 0);
+        const uint32_t pos = *len_dev;
         float sn = 0.f, cs = 1.f;
-        if (lane < fp.n_rot / 2) sincosf((float)pos * rope_inv_freq(lane, fp.rate, fp.freq_scale), &sn, &cs);
+        if (wave < njobs && lane < fp.n_rot / 2) sincosf((float)pos * rope_inv_freq(lane, fp.rate, fp.freq_scale), &sn, &cs);
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             const int j = wave + LONG_WAVES * r;
@@ -1043,7 +1101,8 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
                 for (int i = 0; i < HD / 64; i++) dst[lane + 64 * i] = raw[r].x[i];
             }
-            if (j >= gq) {
+            if (j < gq) cut_up(j, dst);
+            else {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 const size_t b0 = ((size_t)pos * n_kv + kvh) * NB;
 #pragma unroll
@@ -1051,32 +1110,18 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                     quantize_lanes<FMT>(dst[e + lane], lane & 31, true, j == gq ? st.k_codes : st.v_codes, j == gq ? st.k_scales : st.v_scales, b0 + (size_t)((e + lane) >> 5));
             }
         }
-        __syncthreads();
-        if (PRE && kt < k1 && owner) request_k(kt);
-    }
-
-    if (wave < NB) {                                                    // wave j cuts the queries' block j up for all
-        float x[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) x[i] = 0.f;
-        if (qn < gq) {
-            if constexpr (FUSED) load_dims<8>(sq + qn * HD + 32 * wave + 8 * g, x);
-            else load_dims<8>(q + ((size_t)head0 + qn) * HD + 32 * wave + 8 * g, x);
-        }
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            sm_q[wave][t][lane] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
-#pragma unroll
-            for (int i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);   // exact
-        }
-    }
+    } else if (wave < gq) cut_up(wave, q + ((size_t)head0 + wave) * HD);
+    if (!owner) request_v(ra, kt);
     __syncthreads();
+    if (owner) { request_k(ra, kt); request_v(ra, kt); }
 
-    // The lane's A row of a block's two tiles: dims 2 n and 2 n + 1 (Q8_0, the two bytes of a half word), n and 16 + n (4-bit formats, the two
-    // nibbles of a byte).
-    const uint32_t row_b = (uint32_t)nblk * (CW * 4);                   // bytes from a row's codes to the next row's
-    const uint32_t vco = (uint32_t)(4 * g) * row_b + (uint32_t)(Q8 ? 2 * n : n);
-    auto load_code = [&](const char* p) -> uint32_t { return Q8 ? (uint32_t)*(const uint16_t*)p : (uint32_t)*(const uint8_t*)p; };
+    // Two keys' units of a block pair -> the lane's A rows of the first and of the second block, the later key's in the upper half: lanes 0 .. 7 of a row of 16
+    // give their second units away for the first units of lanes 8 .. 15.
+    auto pair_up = [&](uint32_t w0, uint32_t w1, uint32_t& first, uint32_t& second) {
+        const uint32_t u0 = __builtin_amdgcn_perm(w1, w0, Q8 ? 0x05040100u : 0x0C040C00u), u1 = __builtin_amdgcn_perm(w1, w0, Q8 ? 0x07060302u : 0x0C050C01u);
+        first = (uint32_t)__builtin_amdgcn_update_dpp((int)u0, (int)u1, 0x128, 0xF, 0xC, false);    // row_ror:8 into lanes 8 .. 15
+        second = (uint32_t)__builtin_amdgcn_update_dpp((int)u1, (int)u0, 0x128, 0xF, 0x3, false);   // ... and 0 .. 7
+    };
     const uint32_t cut1 = cut >= 1 ? 0xFFFF0000u : 0u, cut2 = cut >= 2 ? 0xFFFF0000u : 0u;
 
     f32x4 run[NB][2];                       // [block][tile]: A rows 4 g + r of column n
@@ -1086,42 +1131,19 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
         for (int i = 0; i < 2; i++) run[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (; kt < k1; kt += LONG_KEYS * LONG_WAVES) {
+    // a round; more: its registers then take the round after the next one
+    auto round = [&](Round& R, uint32_t kt, auto more) {
         const uint32_t last = k1 - 1u - kt;
-        if (!PRE) request_k(kt);
-        uint32_t vw[NB][NT][2];                 // [block][tile of keys]: the codes of keys 16 t + 4 g + (0, 1) and + (2, 3), a half word each
-        const char* vc = (const char*)(qc.v_codes + ((size_t)kt * nblk + (size_t)kvh * NB) * CW);
-        if (last >= LONG_KEYS - 1u) {
-            // a lane's own part of the address is the same for every row (and fits 32 bits); the rest is the wave's
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r += 2)
-#pragma unroll
-                    for (int j = 0; j < NB; j++) {
-                        const char* p = vc + (size_t)(16 * t + r) * row_b + j * (CW * 4);
-                        vw[j][t][r >> 1] = load_code(p + vco) | load_code(p + row_b + vco) << 16;
-                    }
-        } else {
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r += 2) {
-                    uint32_t mine = (uint32_t)(4 * g);
-                    asm volatile("" : "+v"(mine));                      // worked out here: kept from round to round these are eight more registers
-                    const char* p0 = vc + (size_t)min(mine + (uint32_t)(16 * t + r), last) * row_b + (Q8 ? 2 * n : n);
-                    const char* p1 = vc + (size_t)min(mine + (uint32_t)(16 * t + r + 1), last) * row_b + (Q8 ? 2 * n : n);
-#pragma unroll
-                    for (int j = 0; j < NB; j++) vw[j][t][r >> 1] = load_code(p0 + j * (CW * 4)) | load_code(p1 + j * (CW * 4)) << 16;
-                }
-        }
 #pragma unroll
         for (int i = 0; i < NB / 2; i++) {
-            const float lo = __half2float(__ushort_as_half((uint16_t)sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(sc[i] >> 16)));
+            const float lo = __half2float(__ushort_as_half((uint16_t)R.sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(R.sc[i] >> 16)));
             sm_d[wave][2 * i][lane] = lo;
             sm_d[wave][2 * i + 1][lane] = hi;
         }
+#pragma unroll
+        for (int i = 0; i < KL; i++) *(u32x4*)&sm_k[wave][(i * (64 / LR) + lane / LR) * KROW + 16 * (lane % LR)] = R.k[i];
         asm volatile("" ::: "memory");          // a wave's LDS accesses complete in order; this keeps the compiler's in order too
+        if constexpr (decltype(more)::value) request_k(R, kt + STEP);
 
         float p[NT][4];                         // [tile][r]: key 16 t + 4 g + r of column n's query
 #pragma unroll
@@ -1135,7 +1157,9 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             for (int i = 0; i < 3; i++) { const uint4 w = sm_q[j][i][lane]; qf[i].w[0] = w.x; qf[i].w[1] = w.y; qf[i].w[2] = w.z; qf[i].w[3] = w.w; }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const bf16x8 c = codes_bf16<FMT>(kw[t][j], 4 * (g >> 1));
+                const uint2 w = *(const uint2*)&sm_k[wave][(16 * t + n) * KROW + 4 * CW * j + 8 * (g & (CW / 2 - 1))];
+                const uint32_t kw[2] = {w.x, w.y};
+                const bf16x8 c = codes_bf16<FMT>(kw, 4 * (g >> 1));
                 f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int i = 2; i >= 0; i--) a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, qf[i].v, a, 0, 0, 0);
@@ -1146,7 +1170,6 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             asm volatile("" ::: "memory");      // a block at a time: the operands of all of them do not fit the registers
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (PRE && kt + LONG_KEYS * LONG_WAVES < k1) request_k(kt + LONG_KEYS * LONG_WAVES);
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -1158,24 +1181,36 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                 for (int r = 0; r < 4; r++) p[t][r] = softcap * tanhf(p[t][r] / softcap);
         }
         const int lim = (int)min(last, (uint32_t)LONG_KEYS);
+        const bool full = lim >= LONG_KEYS - 1;
+        if (!full) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (4 * g > lim - (16 * t + r)) p[t][r] = -3.0e38f;
+        }
         float top = -3.0e38f;
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                if (4 * g > lim - (16 * t + r)) p[t][r] = -3.0e38f;
-                top = fmaxf(top, p[t][r]);
-            }
+            for (int r = 0; r < 4; r++) top = fmaxf(top, p[t][r]);
         top = fmaxf(top, __shfl_xor(top, 16));
         top = fmaxf(top, __shfl_xor(top, 32));
         const float m_new = fmaxf(m, top), corr = __expf(m - m_new);
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[t][r] = __expf(p[t][r] - m_new);
+        if (!full) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (4 * g > lim - (16 * t + r)) p[t][r] = 0.f;
+        }
         float ps[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) p[t][r] = 4 * g > lim - (16 * t + r) ? 0.f : __expf(p[t][r] - m_new);
-            ps[t] = (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
-        }
+        for (int t = 0; t < NT; t++) ps[t] = (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
         l = fmaf(l, corr, ps[0] + ps[1]);
         if (__builtin_amdgcn_ballot_w64(m_new != m) != 0) {
 #pragma unroll
@@ -1184,6 +1219,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                 for (int i = 0; i < 2; i++) run[j][i] *= corr;
         }
         m = m_new;
+        uint32_t vw[2][4];                      // [block of the pair]: the codes of keys 16 (e / 2) + 4 g + 2 (e % 2) and the next, a half word each
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             float x[2 * 4];                     // probability times the block's scale, key 16 t + 4 g + r at 4 t + r
@@ -1193,12 +1229,15 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
                 for (int r = 0; r < 4; r++) x[4 * t + r] = p[t][r] * d[r];
             }
+            if (j % 2 == 0)
+#pragma unroll
+                for (int e = 0; e < 4; e++) pair_up(R.v[j / 2][e >> 1][2 * (e & 1)], R.v[j / 2][e >> 1][2 * (e & 1) + 1], vw[0][e], vw[1][e]);
             Frag a[2];                          // the codes of the block's two tiles of dims
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const uint32_t w = vw[j][e >> 1][e & 1];
+                    const uint32_t w = vw[j & 1][e];
                     float lo, hi;
                     if constexpr (Q8) { lo = (float)(int8_t)(w >> (8 * i)); hi = (float)(int8_t)(w >> (16 + 8 * i)); }
                     else { lo = (float)((w >> (4 * i)) & 15u) - 8.0f; hi = (float)((w >> (16 + 4 * i)) & 15u) - 8.0f; }
@@ -1233,58 +1272,56 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             asm volatile("" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
+        if constexpr (decltype(more)::value) request_v(R, kt + STEP);
+    };
+    for (; kt + STEP < k1; kt += STEP) round(ra, kt, std::true_type{});
+    if (kt < k1) round(ra, kt, std::false_type{});
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    if constexpr (SPL) {                        // column n < gq takes its other two cuts
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float v = run[j][i][r];
-                    run[j][i][r] = v + (__shfl(v, (lane & 48) | ((n + gq) & 15)) + __shfl(v, (lane & 48) | ((n + 2 * gq) & 15)));
-                }
-    }
     if (lane < gq) { sm_m[wave][lane] = m; sm_l[wave][lane] = l; }
-    if (n < gq) {
+    if (n < (SPL ? 3 * gq : gq)) {
 #pragma unroll
         for (int j = 0; j < NB; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int mrow = 4 * g + r;     // A row: dims 2 mrow, 2 mrow + 1 (Q8_0), mrow, 16 + mrow
-                sm_acc[wave][n][32 * j + (Q8 ? 2 * mrow : mrow)] = run[j][0][r];
-                sm_acc[wave][n][32 * j + (Q8 ? 2 * mrow + 1 : 16 + mrow)] = run[j][1][r];
+                const int mrow = 4 * g + r, unit = 2 * (mrow & 7) + (mrow >> 3);   // the A row's unit of the block: dims 2 u, 2 u + 1 (Q8_0), u, 16 + u
+                sm_acc[wave][n][32 * j + (Q8 ? 2 * unit : unit)] = run[j][0][r];
+                sm_acc[wave][n][32 * j + (Q8 ? 2 * unit + 1 : 16 + unit)] = run[j][1][r];
             }
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < gq * HD; idx += 64 * LONG_WAVES) {
-        const int h = idx / HD, d = idx % HD;
+    // four dims a thread; a query's three cuts meet here
+    for (int idx = threadIdx.x; idx < gq * (HD / 4); idx += 64 * LONG_WAVES) {
+        const int h = idx / (HD / 4), d = 4 * (idx % (HD / 4));
         float M = sm_m[0][h];
 #pragma unroll
         for (int w = 1; w < LONG_WAVES; w++) M = fmaxf(M, sm_m[w][h]);
-        float L = 0.f, A = 0.f;
+        float L = 0.f;
+        f32x4 A = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < LONG_WAVES; w++) {
             const float f = __expf(sm_m[w][h] - M);
             L = fmaf(sm_l[w][h], f, L);
-            A = fmaf(sm_acc[w][h][d], f, A);
+            f32x4 v = *(const f32x4*)&sm_acc[w][h][d];
+            if constexpr (SPL) v += *(const f32x4*)&sm_acc[w][h + gq][d] + *(const f32x4*)&sm_acc[w][h + 2 * gq][d];
+#pragma unroll
+            for (int i = 0; i < 4; i++) A[i] = fmaf(v[i], f, A[i]);
         }
         float* pp = part + ((size_t)(head0 + h) * splits + split) * (HD + 2);
-        pp[d] = A;
+#pragma unroll
+        for (int i = 0; i < 4; i++) pp[d + i] = A[i];
         if (d == 0) { pp[HD] = M; pp[HD + 1] = L; }
     }
 }
 
 template <int HD, int FMT, bool SPL>
-__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
+__global__ __launch_bounds__(64 * LONG_WAVES, 2) void attn_long_kvq_kernel(const float* __restrict__ q, QCache qc, int n_kv, uint32_t len_host,
                                                                            const uint32_t* __restrict__ len_dev, float scale, int splits,
                                                                            uint32_t window, float softcap, float* __restrict__ part, int gq) {
     attn_long_body<HD, FMT, SPL, false>(q, qc, n_kv, len_host, len_dev, scale, splits, window, softcap, part, gq, QkvPostParams{}, KvqStore{});
 }
 template <int HD, int FMT, bool SPL>
-__global__ __launch_bounds__(64 * LONG_WAVES, 4) void attn_long_fused_kvq_kernel(QkvPostParams fp, KvqStore st, int n_kv, uint32_t len_host,
+__global__ __launch_bounds__(64 * LONG_WAVES, 2) void attn_long_fused_kvq_kernel(QkvPostParams fp, KvqStore st, int n_kv, uint32_t len_host,
                                                                                  const uint32_t* __restrict__ len_dev, float scale, int splits,
                                                                                  uint32_t window, float softcap, float* __restrict__ part, int gq) {
     attn_long_body<HD, FMT, SPL, true>(nullptr, QCache{st.k_codes, st.k_scales, st.v_codes, st.v_scales}, n_kv, len_host, len_dev, scale, splits, window, softcap, part, gq,
@@ -1367,11 +1404,14 @@ bool attn_long_takes(int fmt, int g, int n_kv, const uint32_t* k_codes) {
     if (fmt == FHIP_KVQ_Q4_1 || g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
     return g >= 3;
 }
+// Half the splits of the kernels above, about one workgroup a CU, and never the one that needs no combine launch. 98 shapes of one to sixteen KV heads, 5200 .. 32768 keys: as many
+// splits as above take 1.18 times as long (the fixed part twice a CU).
+int attn_long_splits(int splits) { return splits <= 3 ? 2 : (splits + 1) / 2; }
 template <int FMT>
 void launch_attn_long_kvq(int g, int hd, dim3 grid, const KvqLaunch& a) {
     auto go = [&](auto kernel, auto fused) {
-        if (a.fp) hipLaunchKernelGGL(fused, grid, dim3(64 * LONG_WAVES), 0, a.s, *a.fp, a.cache, a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
-        else hipLaunchKernelGGL(kernel, grid, dim3(64 * LONG_WAVES), 0, a.s, a.q, a.qc(), a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
+        if (a.fp) hipLaunchKernelGGL(fused, dim3(grid.y, grid.x), dim3(64 * LONG_WAVES), 0, a.s, *a.fp, a.cache, a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
+        else hipLaunchKernelGGL(kernel, dim3(grid.y, grid.x), dim3(64 * LONG_WAVES), 0, a.s, a.q, a.qc(), a.n_kv, a.len, a.d_len, a.scale, a.splits, a.window, a.softcap, a.part, g);
     };
     if (hd == 64) {
         if (g <= 5) go(attn_long_kvq_kernel<64, FMT, true>, attn_long_fused_kvq_kernel<64, FMT, true>);
@@ -1626,12 +1666,14 @@ static int launch_attention_over_kvq(const char* who, int fmt, const float* q, c
     const int g = n_head / n_kv;
     const bool per_head = g >= 1 && g <= 8 && attn_per_query_head(len, n_head, n_kv, hd, ws != nullptr);   // as the f32 cache's launch: the same sums, the same bits
     const bool mid = g >= 1 && g <= 8 && attn_per_head_splits(len, n_head, n_kv);
-    const int splits = per_head ? 1 : mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
+    int splits = per_head ? 1 : mid ? attn_mid_splits(len, n_head) : attn_splits(len, n_kv);
+    const bool lng = !per_head && !mid && splits > 1 && attn_long_takes(fmt, g, n_kv, cache.k_codes);
+    if (lng) splits = attn_long_splits(splits);
     if (splits > 1 && !ws) return set_error(FHIP_ERR_ARG, "%s: this cache length needs the workspace", who);
     const KvqLaunch a{s, q, fp, cache, n_kv, (uint32_t)len, d_len, 1.0f / sqrtf((float)hd), splits, window > 0x7FFFFFFFull ? 0u : (uint32_t)window, softcap, ws, out};
     const dim3 grid = per_head ? dim3((unsigned)n_head, 1) : mid ? dim3((unsigned)((n_kv * splits + 7) / 8 * 8 * g), 1) : dim3((unsigned)n_kv, (unsigned)splits);
     const int G = per_head || mid ? 1 : g, gq = per_head ? g : mid ? -g : g;
-    const bool wide = per_head && attn_wide(len), lng = !per_head && !mid && splits > 1 && attn_long_takes(fmt, g, n_kv, cache.k_codes);
+    const bool wide = per_head && attn_wide(len);
     int rc = FHIP_OK;
     switch (fmt) {
         case FHIP_KVQ_Q8_0:

@@ -275,6 +275,24 @@ def test_long_caches_by_cut_columns_and_by_query_columns(F, Q, K, fmt, nh, nkv, 
     test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, hd, rows, lengths)
 
 
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("nkv,g,n", [(171, 3, 700), (300, 3, 511), (511, 3, 290), (171, 6, 257), (171, 8, 31)])
+def test_long_caches_of_many_kv_heads_in_the_fewest_splits(F, Q, K, fmt, nkv, g, n):
+    """Two splits of a cache that other kernels would cut into two or three: a wave's first round only, a second one partly filled, waves without a key. Rows behind
+    the length on the device hold nothing. The bar is the one above."""
+    from ferric_amd import decode as X
+    from oracle import decode_oracle as D
+    rng, hd, cap = np.random.default_rng(n + fmt), 64, 5121
+    width = nkv * hd
+    k, v = (rng.standard_normal((n, width)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((1, nkv * g * hd)).astype(np.float32)
+    kq, vq = (Q.QKvCache(fmt, cap, width).append(F.Tensor.from_vec(x, x.shape)) for x in (k, v))
+    word = F.Tensor.from_vec(np.array([n - 1], np.uint32).view(np.float32), (1,))
+    got = X.decode_attention_kvq(F.Tensor.from_vec(q, q.shape), kq, vq, nkv * g, nkv, length=cap, last_pos=word).to_vec()
+    want = D.decode_attention(q[0], K.roundtrip(k, n, width, fmt), K.roundtrip(v, n, width, fmt), nkv * g, nkv, 0, 0.0).reshape(-1)
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
 def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
     rng = np.random.default_rng(80)
     t, width, cap = 5, 256, 16
