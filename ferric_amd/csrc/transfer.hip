@@ -7,7 +7,7 @@
 // their own, which a host thread polls without a call into the runtime.
 //   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time)
 //   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
-//                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation); more is cut into chunks, each
+//                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise; more is cut into chunks, each
 //                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
 //                   included, which is why there are several workers)
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms. A whole copy to the host reaches
@@ -40,6 +40,7 @@ constexpr int SLOTS = 16, JOB_SLOTS = 12;        // a chunked copy takes up to J
 constexpr int MAX_WG = 64, THREADS = 512;        // workgroups of a copy (each confirms its part in a word of its own)
 constexpr size_t IN_PARTS = (size_t)96 << 10;    // copies to the host from here on go in parts, the host copying one out while the next ones cross
 constexpr int PARTS = 8;                         // at most
+constexpr size_t D2H_ALONE = 3 * OUT_BYTES;      // longer copies to the host are the workers'
 constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
@@ -140,10 +141,10 @@ struct Ring {                    // one per device
 
     // The lowest slot that neither the host holds nor the GPU still reads: low slots stay warm in the CPU's caches. A slot's
     // pinned memory is made when it is first taken. null: all are taken.
-    Slot* take(int* rc) {
+    Slot* take(int* rc, int of = SLOTS) {
         std::lock_guard<std::mutex> lock(mu);
         *rc = FHIP_OK;
-        for (int i = 0; i < SLOTS; i++) {
+        for (int i = 0; i < of; i++) {
             Slot& q = slot[i];
             if (q.held || !q.read_by_gpu()) continue;
             if (!words) {
@@ -432,6 +433,61 @@ static int copy_d2h_plain(void* h, const void* d, size_t n, hipStream_t s) {
     return rc ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 
+// n bytes into the slot in parts, and out of it as they arrive.
+// The host copies out at 30 GB/s what crosses at 53, so the total is the first part's way over and the host's whole copy: parts of 60 KB, at least four. A
+// kernel of two thirds and one of the rest | four parts | eight, us on an idle device: 125 KB 15.4 | 13.3 | 16.6, 250 KB 19.3 | 16.5 | 17.7, 432 KB 25.0 |
+// 22.8 | 21.7, 593 KB 31.5 | 28.4 | 26.1, 976 KB 45.4 | 41.5 | 39.0.
+static int send_parts(Slot* q, const uint8_t* from, size_t n, hipStream_t s, Parts<PARTS>* out) {
+    const size_t by_size = n / ((size_t)60 << 10);
+    Parts<PARTS> parts{n < IN_PARTS ? 1 : by_size < 4 ? 4 : by_size < PARTS ? (int)by_size : PARTS, {}, {}};
+    for (int p = 0; p < parts.count; p++) {
+        const bool last = p == parts.count - 1;
+        parts.end[p] = last ? n : (n / parts.count * (p + 1) + 255) & ~(size_t)255;
+        parts.done[p] = last ? q->done : q->early + p * MAX_WG;
+    }
+    int wgs = 0;
+    const uint32_t seq = q->seq + 1;
+    const int rc = parts.count == 1 ? launch_copy(from, q->host, Parts<1>{1, {n}, {q->done}}, MAX_WG, 1, seq, s, &wgs) : launch_copy(from, q->host, parts, MAX_WG, 1, seq, s, &wgs);
+    if (!rc) { q->seq = seq; q->wgs = wgs; }
+    *out = parts;
+    return rc;
+}
+static int take_parts(Slot* q, uint8_t* h, const Parts<PARTS>& parts, hipStream_t s) {
+    int rc = FHIP_OK;
+    for (int p = 0; p < parts.count && !rc; p++) {
+        const size_t begin = p ? parts.end[p - 1] : 0;
+        if (!(rc = await_words(parts.done[p], q->seq, q->wgs, s))) memcpy(h + begin, q->host + begin, parts.end[p] - begin);
+    }
+    return rc;
+}
+// The same for two and three slots, all sent before the first is taken: up to D2H_ALONE the host by itself is done before the workers are awake (us, idle device,
+// the workers | the host: 1.06 MB 80 | 41, 1.5 83 | 53, 2.0 92 | 69, 2.36 100 | 77, 3.0 109 | 99; 4.0 would be 125 | 131). *took false: there were not enough slots at once, and
+// nothing was done.
+static int copy_d2h_alone(Ring* r, uint8_t* h, const uint8_t* from, size_t n, hipStream_t s, bool* took) {
+    constexpr size_t MOST = D2H_ALONE / OUT_BYTES;
+    const size_t count = (n + OUT_BYTES - 1) / OUT_BYTES, each = ((n + count - 1) / count + 255) & ~(size_t)255;
+    static_assert(D2H_ALONE % OUT_BYTES == 0 && MOST <= BEGUN, "as many slots as a chunked copy holds while its stream is behind other work");
+    Slot* q[MOST];
+    Parts<PARTS> parts[MOST];
+    size_t have = 0, sent = 0;
+    int rc = FHIP_OK;
+    while (have < count && !rc) {
+        Slot* next = r->take(&rc, JOB_SLOTS);
+        if (!next) break;
+        q[have++] = next;
+    }
+    *took = !rc && have == count;
+    while (*took && !rc && sent < count) {
+        const size_t at = sent * each;
+        rc = send_parts(q[sent], from + at, n - at < each ? n - at : each, s, &parts[sent]);
+        if (!rc) sent++;
+    }
+    for (size_t i = 0; i < sent && !rc; i++) rc = take_parts(q[i], h + i * each, parts[i], s);
+    if (rc && sent) (void)hipStreamSynchronize(s);      // an enqueued part may still use a slot
+    for (size_t i = 0; i < have; i++) r->release(q[i]);
+    return rc;
+}
+
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     int rc, wgs = 0;
     if ((rc = may_wait(s, "fhip_memcpy_d2h"))) return rc;
@@ -441,6 +497,10 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;
+    if (n > OUT_BYTES && n <= D2H_ALONE) {
+        bool took;
+        if ((rc = copy_d2h_alone(r, (uint8_t*)h, from, n, s, &took)) || took) return rc;
+    }
     if (n > OUT_BYTES) {
         Job j{};
         j.count = (n + CHUNK - 1) / CHUNK;
@@ -467,22 +527,8 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     }
     Slot* q = r->get(&rc);
     if (!q) return rc ? rc : copy_d2h_plain(h, d, n, s);
-    // The host copies out at 30 GB/s what crosses at 53, so the total is the first part's way over and the host's whole copy: parts of 60 KB, at least four. A
-    // kernel of two thirds and one of the rest | four parts | eight, us on an idle device: 125 KB 15.4 | 13.3 | 16.6, 250 KB 19.3 | 16.5 | 17.7, 432 KB 25.0 |
-    // 22.8 | 21.7, 593 KB 31.5 | 28.4 | 26.1, 976 KB 45.4 | 41.5 | 39.0.
-    const size_t by_size = n / ((size_t)60 << 10);
-    Parts<PARTS> parts{n < IN_PARTS ? 1 : by_size < 4 ? 4 : by_size < PARTS ? (int)by_size : PARTS, {}, {}};
-    for (int p = 0; p < parts.count; p++) {
-        const bool last = p == parts.count - 1;
-        parts.end[p] = last ? n : (n / parts.count * (p + 1) + 255) & ~(size_t)255;
-        parts.done[p] = last ? q->done : q->early + p * MAX_WG;
-    }
-    const uint32_t seq = q->seq + 1;
-    if (!(rc = parts.count == 1 ? launch_copy(from, q->host, Parts<1>{1, {n}, {q->done}}, MAX_WG, 1, seq, s, &wgs) : launch_copy(from, q->host, parts, MAX_WG, 1, seq, s, &wgs))) { q->seq = seq; q->wgs = wgs; }
-    for (int p = 0; p < parts.count && !rc; p++) {
-        const size_t begin = p ? parts.end[p - 1] : 0;
-        if (!(rc = await_words(parts.done[p], seq, wgs, s))) memcpy((uint8_t*)h + begin, q->host + begin, parts.end[p] - begin);
-    }
+    Parts<PARTS> parts;
+    if (!(rc = send_parts(q, from, n, s, &parts))) rc = take_parts(q, (uint8_t*)h, parts, s);
     r->release(q);
     return rc;
 }

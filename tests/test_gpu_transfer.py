@@ -32,6 +32,13 @@ def test_round_trip(F, n, offset):
     assert (out[:offset] == 0xA5).all() and (out[offset + n:] == 0xA5).all()
 
 
+# two and three slots that the host empties by itself, and one byte more (64 + offset bytes are added to n)
+@pytest.mark.parametrize("n", [MIB + 200, 2 * MIB - 64, 2 * MIB - 63, 3 * MIB - 65, 3 * MIB - 64, 3 * MIB - 63])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_copies_back_of_two_and_three_slots(F, n, offset):
+    test_round_trip(F, n, offset)
+
+
 @pytest.mark.parametrize("ty,block", [(8, 32), (12, 256), (14, 256), (7, 32), (39, 32)])
 @pytest.mark.parametrize("values", [32 * 8, MIB // 4 - 256, MIB // 4, MIB // 4 + 256, 2 * MIB // 4 + 256, 17 * MIB // 4 + 512])
 def test_host_dequantization_in_chunks(F, O, ty, block, values):
