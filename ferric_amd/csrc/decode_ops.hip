@@ -1131,7 +1131,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
         for (int i = 0; i < 2; i++) run[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // a round; more: its registers then take the round after the next one
+    // a round; more: its registers take the wave's next one as they come free
     auto round = [&](Round& R, uint32_t kt, auto more) {
         const uint32_t last = k1 - 1u - kt;
 #pragma unroll
