@@ -957,7 +957,9 @@ union Frag { uint32_t w[4]; bf16x8 v; };
 // the upper halves of two f32: two bf16 (exact where the lower halves are zero)
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
 
-// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16 (4-bit formats: less 8)
+// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16. 4-bit formats: less 8, and a sixteenth (v_cvt_off_f32_i4 makes that of a two's complement nibble in one
+// instruction, where the byte, its conversion and the 8 were three; the scales carry the 16, so every bit is the same). 128 x 8 KV heads of 5, 32768 keys, with the combine launch 23.1 -> 21.2 us,
+// 4 KV heads of 8 16.5 -> 15.6, heads of 64 16.4 -> 15.3: 804 -> 613 vector instructions a round beside its softmax.
 template <int FMT>
 __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) {
     Frag f;
@@ -968,9 +970,9 @@ __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) 
             v[0] = (float)(int8_t)(w[i] & 255u); v[1] = (float)(int8_t)((w[i] >> 8) & 255u);
             v[2] = (float)(int8_t)((w[i] >> 16) & 255u); v[3] = (float)(int8_t)(w[i] >> 24);
         } else {
-            const uint32_t x = (w[i] >> shift) & 0x0F0F0F0Fu;
+            const uint32_t x = (w[i] ^ 0x88888888u) >> shift;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = (float)((x >> (8 * j)) & 255u) - 8.0f;
+            for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_cvt_off_f32_i4((int)(j % 3 ? (x >> (8 * j)) & 255u : x >> (8 * j)));
         }
         f.w[2 * i] = upper_halves(v[0], v[1]);
         f.w[2 * i + 1] = upper_halves(v[2], v[3]);
@@ -1137,8 +1139,8 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
         for (int i = 0; i < NB / 2; i++) {
             const float lo = __half2float(__ushort_as_half((uint16_t)R.sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(R.sc[i] >> 16)));
-            sm_d[wave][2 * i][lane] = lo;
-            sm_d[wave][2 * i + 1][lane] = hi;
+            sm_d[wave][2 * i][lane] = Q8 ? lo : 16.0f * lo;             // (4-bit codes are sixteenths)
+            sm_d[wave][2 * i + 1][lane] = Q8 ? hi : 16.0f * hi;
         }
 #pragma unroll
         for (int i = 0; i < KL; i++) *(u32x4*)&sm_k[wave][(i * (64 / LR) + lane / LR) * KROW + 16 * (lane % LR)] = R.k[i];
@@ -1240,7 +1242,10 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                     const uint32_t w = vw[j & 1][e];
                     float lo, hi;
                     if constexpr (Q8) { lo = (float)(int8_t)(w >> (8 * i)); hi = (float)(int8_t)(w >> (16 + 8 * i)); }
-                    else { lo = (float)((w >> (4 * i)) & 15u) - 8.0f; hi = (float)((w >> (16 + 4 * i)) & 15u) - 8.0f; }
+                    else {
+                        const uint32_t x = (w ^ 0x88888888u) >> (4 * i);
+                        lo = __builtin_amdgcn_cvt_off_f32_i4((int)x); hi = __builtin_amdgcn_cvt_off_f32_i4((int)(x >> 16));
+                    }
                     a[i].w[e] = upper_halves(lo, hi);
                 }
             if constexpr (SPL) {
