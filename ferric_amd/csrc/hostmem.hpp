@@ -19,6 +19,7 @@ bool pool_range(const void* ptr, uintptr_t* base, uintptr_t* end);   // the bloc
 enum class Place { inside, outside, elsewhere };
 Place pool_place(const void* ptr, size_t n, int dev);
 int device_malloc(void** out, size_t n, const char* what);           // hipMalloc; with no memory left, once more after pool_trim
+void* device_malloc_beside_captures(size_t n);                       // hipMalloc also while threads have captures open, which it leaves as they are; null: no memory
 
 // transfer.hip: copies through pinned memory of the library's own; both directions and the host-to-host unpackers
 constexpr size_t H2D_STAGED = (size_t)640 << 10;   // up to here copy_h2d has read its source when it returns

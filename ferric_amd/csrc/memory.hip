@@ -201,6 +201,18 @@ int device_malloc(void** out, size_t n, const char* what) {
     return check_hip(e, what);
 }
 
+// A refused hipMalloc would invalidate the captures that refuse it; in this mode none does (the memory is no part of a graph).
+void* device_malloc_beside_captures(size_t n) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    void* p = nullptr;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipMalloc(&p, n);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 int pool_malloc(void** out, size_t nbytes) {
     *out = nullptr;
     if (thread_captures())

@@ -191,8 +191,9 @@ int fhip_deq_raw(const uint8_t* h_raw, size_t nbytes, size_t n, uint32_t ggml_ty
  * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Most products of up to 4096
  * columns are one launch that needs nothing beside its operands. The others keep
  * prepared activations or partial sums in a workspace the library owns per stream (fhip_workspace_reserve); inside a graph capture the
- * workspace cannot grow, and a product of more than 6144 columns then fails with FHIP_ERR_ARG and says how many bytes to reserve beforehand; one of up to 6144
- * columns is captured as one launch where no workspace serves it (its sums then in another order, the same to f32 rounding).
+ * workspace cannot grow, and a product of more than 6144 columns, or of more than one group of rows, then fails with FHIP_ERR_ARG and says how many bytes to reserve
+ * beforehand. One group of up to 6144 columns (x and y apart) is captured all the same: under FHIP_BATCH_ORDERED as a launch for each range of its columns, with the
+ * bits it has with the workspace and two to five times its time; under FHIP_BATCH_AUTO as one launch. So it is where there is no memory for the workspace.
  * Non-finite activations: on the mat-vec kernel a NaN or infinite x gives what the f32 dot gives (NaN, +-inf by the weight's
  * sign); on the matrix-core kernels the whole output row of such an activation row is non-finite and no other row is touched. */
 int fhip_matmul_q(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, void* stream);

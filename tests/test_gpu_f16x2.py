@@ -451,21 +451,37 @@ def test_operand_rows_in_a_workgroups_lds(F, O, ty, rows, cols, t, own, cut):
     assert np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
 
 
-def test_a_cut_product_is_captured_without_a_workspace_where_one_launch_can_do_it(F):
-    # 20 chunks: two or more ranges of K, or the held kernel's one launch, which a capture on a stream without a workspace takes
-    from conftest import ROUTES, route
+@pytest.mark.parametrize("ty,rows,cols,t", [(Q5_K, 400, 5120, 6), (Q4_K, 2050, 5632, 13), (Q6_K, 1605, 6144, 30), (Q8_0, 301, 5152, 8), (Q8_0, 4200, 4384, 25)])
+def test_a_cut_product_has_the_same_bits_with_and_without_a_workspace(F, ty, rows, cols, t):
+    """K in two or more ranges, whose partial outputs meet in the stream's workspace; where a capture on the stream, or one that the thread has open on another stream, keeps
+    the library from making that workspace, the product goes on without it. It has the bits it has with it, replay after replay, and another product's workspace changes none."""
+    from conftest import ROUTES, bits, route
     from ferric_amd.synth import synth_weights
-    rows, cols, t = 400, 5120, 6
-    w = F.QMatrix.from_bytes(synth_weights(Q5_K, rows, cols, 51), Q5_K, rows, cols)
+    lib, check = F._lib.load(), F._lib.check
+    w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 51), ty, rows, cols)
     w.batch_policy(F.BATCH_ORDERED)
     x = np.random.default_rng(52).standard_normal((t, cols)).astype(np.float32)
-    xt, y, stream = F.Tensor.from_vec(x, x.shape), F.Tensor.empty((t, rows)), F.Stream()
-    assert route(F, w, xt, t) == [(ROUTES["OWN_ROWS"] | ROUTES["CUT"], t)]
-    want = xt.matmul_q(w).to_vec()
-    g = F.Graph.begin(stream)
-    F._lib.check(F._lib.load().fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, stream.handle))
-    g.end()
-    for _ in range(3):
-        F._lib.check(F._lib.load().fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
+    xt, y, y2 = F.Tensor.from_vec(x, x.shape), F.Tensor.empty((t, rows)), F.Tensor.empty((t, rows))
+    (kernel, _), = route(F, w, xt, t)
+    assert kernel & ROUTES["CUT"]
+    want = bits(xt.matmul_q(w).to_vec())
+
+    def capture(stream, other=None):
+        g = F.Graph.begin(stream)
+        rc = [lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, stream.handle)]
+        if other is not None:
+            rc.append(lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y2.buf.ptr, other.handle))
+        g.end()
+        for r in rc:
+            check(r)
+        return g
+
+    stream, other = F.Stream(), F.Stream()
+    graphs = [capture(stream, other)]                   # neither stream has a workspace
+    assert np.array_equal(bits(y2.to_vec(other)), want)
+    check(lib.fhip_workspace_reserve(stream.handle, lib.fhip_workspace_bytes(w.handle, None, t)))
+    graphs.append(capture(stream))
+    for g in graphs * 3:
+        check(lib.fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
         g.launch()
-        assert np.abs(y.to_vec(stream) - want).max() <= 2e-6 * np.abs(want).max()
+        assert np.array_equal(bits(y.to_vec(stream)), want)
