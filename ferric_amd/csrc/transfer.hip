@@ -7,7 +7,7 @@
 // their own, which a host thread polls without a call into the runtime.
 //   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time)
 //   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
-//                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise; more is cut into chunks, each
+//                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise (one and a half into fresh memory); more is cut into chunks, each
 //                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
 //                   included, which is why there are several workers)
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms. A whole copy to the host reaches
@@ -18,6 +18,8 @@
 #include "through.hpp"
 
 #include <string.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <atomic>
 #include <chrono>
@@ -40,7 +42,8 @@ constexpr int SLOTS = 16, JOB_SLOTS = 12;        // a chunked copy takes up to J
 constexpr int MAX_WG = 64, THREADS = 512;        // workgroups of a copy (each confirms its part in a word of its own)
 constexpr size_t IN_PARTS = (size_t)96 << 10;    // copies to the host from here on go in parts, the host copying one out while the next ones cross
 constexpr int PARTS = 8;                         // at most
-constexpr size_t D2H_ALONE = 3 * OUT_BYTES;      // longer copies to the host are the workers'
+constexpr size_t D2H_ALONE = 3 * OUT_BYTES;      // longer copies to the host are the workers' ...
+constexpr size_t D2H_ALONE_NEW = D2H_ALONE / 2;  // ... and those from here on whose destination has pages that nobody has touched
 constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
@@ -374,6 +377,17 @@ bool plain_host(const void* h) {
     return true;
 }
 
+// whether every page of the range is in memory: a fresh allocation's are made by whoever writes to them first
+bool in_memory(const void* h, size_t n) {
+    static const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
+    const uintptr_t begin = (uintptr_t)h / page * page, pages = ((uintptr_t)h + n - begin + page - 1) / page;
+    unsigned char there[D2H_ALONE / 4096 + 2];
+    if (page < 4096 || mincore((void*)begin, pages * page, there) != 0) return false;
+    unsigned char all = 1;
+    for (uintptr_t i = 0; i < pages; i++) all &= there[i];
+    return all & 1;
+}
+
 // Whether the copy kernels, which look nothing up, may take this copy (*yes): the device side inside one block of the library's on the current device,
 // the host side no device memory. Other memory is the runtime's, to copy or to refuse; what leaves one of the library's blocks is refused
 // here, since the runtime knows the block of the pool and not what was asked for. (0.15 us)
@@ -460,8 +474,9 @@ static int take_parts(Slot* q, uint8_t* h, const Parts<PARTS>& parts, hipStream_
     }
     return rc;
 }
-// The same for two and three slots, all sent before the first is taken: up to D2H_ALONE the host by itself is done before the workers are awake (us, idle device,
-// the workers | the host: 1.06 MB 80 | 41, 1.5 83 | 53, 2.0 92 | 69, 2.36 100 | 77, 3.0 109 | 99; 4.0 would be 125 | 131). *took false: there were not enough slots at once, and
+// The same for two and three slots, all sent before the first is taken: up to D2H_ALONE the host by itself is done before the workers are awake. us, idle device, the workers | the
+// host, a destination in memory: 1.04 MB 98 | 46, 1.5 99 | 60, 2.0 106 | 72, 2.36 105 | 80, 3.0 113 | 97 (4.0 125 | 131), 2 of them the question. Into fresh memory, whose pages are made on the way, one thread
+// takes 0.16 us a KB more and ten share it: 1.04 MB 312 | 205, 1.5 326 | 290, 2.0 350 | 382, 2.36 365 | 450, 3.0 372 | 575. *took false: there were not enough slots at once, and
 // nothing was done.
 static int copy_d2h_alone(Ring* r, uint8_t* h, const uint8_t* from, size_t n, hipStream_t s, bool* took) {
     constexpr size_t MOST = D2H_ALONE / OUT_BYTES;
@@ -497,7 +512,7 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;
-    if (n > OUT_BYTES && n <= D2H_ALONE) {
+    if (n > OUT_BYTES && n <= D2H_ALONE && (n <= D2H_ALONE_NEW || in_memory(h, n))) {
         bool took;
         if ((rc = copy_d2h_alone(r, (uint8_t*)h, from, n, s, &took)) || took) return rc;
     }

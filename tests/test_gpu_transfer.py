@@ -39,6 +39,22 @@ def test_copies_back_of_two_and_three_slots(F, n, offset):
     test_round_trip(F, n, offset)
 
 
+# who empties the slots goes by whether the destination's pages are there: none of them, all, all but the first or the last
+@pytest.mark.parametrize("n", [3 * MIB // 2, 3 * MIB // 2 + 1, 2 * MIB + 4097, 3 * MIB])
+@pytest.mark.parametrize("touched", ["none", "all", "not the first", "not the last"])
+def test_copies_back_into_fresh_memory(F, n, touched):
+    import mmap
+    a = np.random.default_rng(n).integers(0, 256, n, np.uint8)
+    buf = F.DeviceBuffer(n)
+    F._lib.check(F._lib.load().fhip_upload(buf.ptr, a.ctypes.data, n, None))
+    for offset in (0, 4000):                      # (a range that does not begin with a page)
+        out = np.frombuffer(mmap.mmap(-1, n + 8192), np.uint8)[offset:offset + n]
+        if touched != "none":
+            out[8192 if touched == "not the first" else 0:-8192 if touched == "not the last" else None] = 1
+        F._lib.check(F._lib.load().fhip_memcpy_d2h(out.ctypes.data, buf.ptr, n, None))
+        assert np.array_equal(out, a)
+
+
 @pytest.mark.parametrize("ty,block", [(8, 32), (12, 256), (14, 256), (7, 32), (39, 32)])
 @pytest.mark.parametrize("values", [32 * 8, MIB // 4 - 256, MIB // 4, MIB // 4 + 256, 2 * MIB // 4 + 256, 17 * MIB // 4 + 512])
 def test_host_dequantization_in_chunks(F, O, ty, block, values):
