@@ -136,6 +136,7 @@ SYMBOLS = {
     "fhip_workspace_reserve": (C.c_int, [_vp, C.c_size_t]),
     "fhip_workspace_release": (None, [_vp]),
     "fhip_debug_matmul_route": (C.c_int, [_vp, _vp, _sz, _vp, C.POINTER(C.c_int), C.POINTER(_sz), _sz, C.POINTER(_sz)]),
+    "fhip_debug_matmul_by": (C.c_int, [_vp, C.c_int, _vp, _sz, _vp, _vp]),
     "fhip_debug_read_probe": (C.c_int, [_vp, _sz, _vp, _vp]),
     "fhip_debug_mfma_probe": (C.c_int, [C.c_int, _vp, C.POINTER(C.c_double), _vp]),
     "fhip_debug_matmul_q_loop": (C.c_int, [_vp, _sz, _sz, _vp, C.c_int, _vp, _vp]),

@@ -1211,6 +1211,20 @@ int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_
     return FHIP_OK;
 }
 
+int fhip_debug_matmul_by(const fhip_weight* w, int kernel, const float* d_x, size_t rows_x, float* d_y, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (!w || !d_x || !d_y) return set_error(FHIP_ERR_ARG, "fhip_debug_matmul_by: NULL pointer");
+    if (rows_x == 0 || rows_x > f16x2_group(w) || w->rows == 0 || !fhip::gemm_f16x2_takes(w, rows_x)) return set_error(FHIP_ERR_ARG, "fhip_debug_matmul_by: not a group of the f16 kernels");
+    const bool ordered = w->batch_policy == FHIP_BATCH_ORDERED, cut = ordered ? fhip::gemm_f16x2_parts(w, rows_x) > 1 : fhip::gemm_f16x2_adds_into_y(w, rows_x);
+    const bool can = kernel == FHIP_ROUTE_PREPARED || (kernel == FHIP_ROUTE_HELD && fhip::gemm_f16x2_held_takes(w, d_x, rows_x, d_y)) ||
+                     (kernel == FHIP_ROUTE_OWN_ROWS && (ordered ? fhip::gemm_f16x2_resident_own_x(w, d_x, rows_x, d_y) : !cut && fhip::gemm_f16x2_own_x(w, d_x, rows_x)));
+    if (!can) return set_error(FHIP_ERR_ARG, "fhip_debug_matmul_by: kernel %d cannot do this product", kernel);
+    void* ws = nullptr;
+    if (kernel != FHIP_ROUTE_HELD && (rc = lib_workspace((hipStream_t)stream, f16x2_matmul_ws(w, rows_x), &ws, "fhip_debug_matmul_by"))) return rc;
+    return f16x2_launch(kernel == FHIP_ROUTE_HELD ? kernel : kernel | (cut ? FHIP_ROUTE_CUT : 0), w, d_x, rows_x, false, d_y, ws, (hipStream_t)stream, nullptr, nullptr);
+}
+
 int fhip_debug_read_probe(const void* d_src, size_t nbytes, uint32_t* d_sink, void* stream) {
     int rc = need_init();
     if (rc) return rc;

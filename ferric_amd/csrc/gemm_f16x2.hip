@@ -1750,26 +1750,29 @@ bool held_beats_streaming(const fhip_weight* w, size_t t) {
     if (chunks <= 16) return tiles <= 4 * cus || (tiles <= 9 * cus && q.split && chunks <= 8);
     return q6 ? 2 * tiles * sets <= 5 * cus : tiles <= (t <= 24 ? 3 : 2) * cus;
 }
-// And where it keeps a product whose sums are in order from the resident kernel: that one's time over its own (676 products of Q4_K, Q6_K and Q8_0).
-// - Up to 16 chunks: where tiles are few the one launch and its sums in LDS are the faster (8 rows, 4096 x 4096 Q4_K 1.00, Q8_0 1.20; 4096 x 1024 1.22 .. 1.33; 16 rows
-//   4096 x 2048 1.24 .. 1.33). The resident kernel takes, of up to eight rows, short rows of many tiles (34816 x 512 Q4_K 0.75, Q6_K 0.87, 16000 x 1024 Q4_K 0.88) and nine or ten chunks of
-//   eight tiles and more (34816 x 2560 0.93, 0.93); of nine to sixteen, more than 4.1 tiles (34816 x 512 0.58 .. 0.81, x 1024 0.73 .. 0.88, x 2560 0.85 .. 0.97; five to eight chunks
-//   1.03 .. 1.08), with more than ten chunks two (8192 x 4096 0.97, 0.93, 0.87); of more two tiles (8192 x 2048 0.98 .. 0.85, 34816 x 512 0.47 .. 0.71), from 13 chunks on a half.
-// - 17 to 24: the resident kernel is the faster one throughout (8 rows, 5120 columns, 100 / 2048 / 8192 / 34816 rows: Q4_K 0.65, 0.70, 0.86, 0.93, Q6_K 0.67, 0.83, 0.95; 16 rows
-//   Q4_K 0.69, 0.73, 0.78, 0.71). Where the held one stays all the same its route is pinned by test_whole_rows_inside_a_workgroup: up to eight rows 24 chunks of Q4_K and Q5_K
-//   at a half to two tiles, Q6_K and Q8_0 at a half to 1.3 (0.80 .. 1.00 there); of more up to a third of a tile (0.70 .. 0.95), Q8_0 at up to sixteen up to 1.1.
+// And where it keeps a product whose sums are in order from the resident kernel: where tiles are few its one launch, with its sums in LDS, is the faster, and the longer so the fewer
+// unpacking passes its sets of eight rows make (us, held | resident, cold weights, sums in order).
+// - One chunk: only where the resident kernel's sixteen rows at a time are half empty (Q4_K 1300 x 256 at 8 rows 3.7 | 3.5, 16 3.7 | 3.9, 32 4.6 | 4.0; 34816 x 256 at 8 7.3 | 5.1).
+// - Up to eight rows: a tile and a half a CU of the formats with minima, three of 8 to 12 chunks (Q4_K 4090 x 1280 5.5 | 5.6, 8200 x 1280 7.6 | 6.2, 12000 x 2304 9.7 | 9.3, 16400 12.1 |
+//   11.3); Q6_K five (16400 x 3072 16.6 | 18.3, 34816 29.3 | 29.0), Q8_0 nine (34816 x 4064 45.9 | 47.6).
+// - Nine to sixteen: a tile and a half (Q4_K 4090 x 1024 5.4 | 7.0, 8200 x 1024 7.7 | 7.3, 34816 x 1280 22.8 | 13.4), three of eight chunks (12000 x 2048 11.4 | 12.7), five where there
+//   are no minima either (Q6_K 20000 x 2048 16.6 | 18.4, Q8_0 20000 x 1760 17.4 | 19.6); two beyond (8200 x 2560 11.9 | 12.1).
+// - More: eight tenths (Q4_K 3070 x 1024 at 24 rows 6.2 | 6.7, 4090 x 1024 7.0 | 6.7, 34816 x 1024 at 32 25.9 | 16.1), with 8 to 12 chunks a tile and a half to 24 rows (Q8_0 6100 x 2272 15.3 |
+//   14.5, 8200 19.7 | 18.2), then one (4090 x 2272 at 32 12.7 | 14.0, 6100 17.2 | 14.9); with more chunks half of one (Q5_K 2050 x 3584 at 32 12.1 | 10.3).
+// - Beyond 16 chunks: nowhere. 572 products (17, 20 and 24 chunks, 100 .. 8200 rows, 5 .. 32 activation rows) 0.61 .. 1.00 of its time, geometric mean 0.75.
+// 2816 products of the four formats (1 .. 16 chunks, 515 .. 34816 rows, 8, 16, 24 and 32 activation rows): what this picks takes 1.006 of the faster one's time (geometric mean), 1.054 at the
+// 95th percentile, 1.20 at most.
 bool held_beats_resident(const fhip_weight* w, size_t t) {
     const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16;
     const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
-    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, mins = !q6 && !q8;
-    if (chunks > 16) {
-        if (t > 8) return q8 && t <= 16 ? 10 * tiles <= 11 * cus : 3 * tiles <= cus;
-        return mins ? chunks == 24 && 2 * tiles >= cus && tiles <= 2 * cus : 2 * tiles > cus && 10 * tiles <= 13 * cus;
-    }
-    if (chunks == 1) return 2 * tiles <= 7 * cus || (q8 && t <= 8 && tiles <= 12 * cus);
-    if (t <= 8) return !(((chunks == 9 || chunks == 10) && tiles >= 8 * cus) || (chunks <= (mins ? 4 : q6 ? 2 : 0) && 2 * tiles > 7 * cus));
-    if (t <= 16) return chunks > 10 ? tiles < 2 * cus : (chunks > 4 && chunks < 9) || 10 * tiles <= 41 * cus;
-    return tiles < 2 * cus && !(chunks > 12 && 2 * tiles >= cus);
+    const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, mins = !q6 && !q8, middle = chunks >= (q8 ? 6 : 8) && chunks <= 12;
+    auto halves = [&](size_t most) { return 2 * tiles <= most * cus; };   // half tiles a CU
+    if (chunks > 16) return false;
+    if (chunks == 1) return t > 8 && t <= 24 && halves(1);
+    if (t <= 8) return halves(mins ? (middle ? 6 : 3) : q6 ? 10 : 18);
+    if (chunks > 12) return halves(t <= 16 ? 4 : 1);
+    if (t <= 16) return halves(!middle ? 3 : chunks > 8 ? 4 : mins ? 6 : 10);
+    return middle ? halves(t <= 24 ? 3 : 2) : 5 * tiles <= 4 * cus;
 }
 // (all workgroups of a launch that stores y read the rows: none may have written over them)
 bool apart(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
@@ -1781,10 +1784,11 @@ bool gemm_f16x2_held_takes(const fhip_weight* w, const float* d_x, size_t t, con
 bool gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
     return gemm_f16x2_held_takes(w, d_x, t, d_y) && (w->batch_policy == FHIP_BATCH_ORDERED ? held_beats_resident(w, t) : held_beats_streaming(w, t));
 }
-// A launch in front that prepares the rows costs 2 - 3 us (Q4_K, 8 rows, itself | prepared: 2048 x 5120 8.1 | 10.7, 34816 x 5120 27.0 | 28.7; 32 rows 2048 x 5120 11.4 | 14.7). From
-// 5120 columns on more than 16 rows keep it: the route is pinned by test_ffn_leaves_the_sums_of_a_cut_gate_up_to_the_next_launch.
+// The resident kernel makes its operand rows itself wherever it can: a launch in front that prepares them costs 2 - 10 us more, or as much where it is hidden (us, itself | prepared, Q4_K, 8 rows
+// 2048 x 5120 8.1 | 10.7, 34816 x 5120 27.0 | 28.7; 32 rows 2048 x 5120 11.7 | 15.2, 34816 x 5120 61.2 | 64.1, 300 x 65536 17.8 | 27.5; 132 products of the four formats at 17, 24 and 32 rows
+// 0.61 .. 1.02 of the time).
 bool gemm_f16x2_resident_own_x(const fhip_weight* w, const float* d_x, size_t t, const float* d_y) {
-    return (t <= 16 || w->cols < 20 * CHUNK) && d_x && ((uintptr_t)d_x & 15) == 0 && (gemm_f16x2_parts(w, t) > 1 || apart(w, d_x, t, d_y));
+    return d_x && ((uintptr_t)d_x & 15) == 0 && (gemm_f16x2_parts(w, t) > 1 || apart(w, d_x, t, d_y));
 }
 
 int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {

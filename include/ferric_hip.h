@@ -188,7 +188,7 @@ int fhip_deq_raw(const uint8_t* h_raw, size_t nbytes, size_t n, uint32_t ggml_ty
  * instruction: every row has the bits it has in a batch of one; one launch, no workspace), three rows and more of the other 32-value formats, up to sixteen a
  * pass, through its wide form (the same, without a workspace too); otherwise, from three rows on (five
  * for Q8_0) Q4_K / Q5_K / Q6_K / Q8_0 weights are multiplied in groups of up to 32 (Q8_0 under FHIP_BATCH_AUTO: 16) rows by the f16 hi/lo matrix-core
- * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Most products of up to 4096
+ * kernels (see fhip_matmul_q_f16x2: f32-grade, 22-bit activations), longer batches group by group. Many products of up to 4096
  * columns are one launch that needs nothing beside its operands. The others keep
  * prepared activations or partial sums in a workspace the library owns per stream (fhip_workspace_reserve); inside a graph capture the
  * workspace cannot grow, and a product of more than 6144 columns, or of more than one group of rows, then fails with FHIP_ERR_ARG and says how many bytes to reserve

@@ -36,6 +36,10 @@ int fhip_debug_quad_matvec(int on);
 #define FHIP_ROUTE_CUT 8         /* with the last two: weight rows are cut along K between workgroups */
 int fhip_debug_matmul_route(const fhip_weight* w, const float* d_x, size_t rows_x, const float* d_y, int* kernels, size_t* rows, size_t cap, size_t* n);
 
+/* Tests: fhip_matmul_q of one group of rows by the f16 hi / lo kernel named (FHIP_ROUTE_HELD, _OWN_ROWS or _PREPARED), whichever fhip_matmul_q itself would pick; the
+ * weight's batch policy says how the sums are made. FHIP_ERR_ARG where that kernel cannot do it. No counterpart in the reference. */
+int fhip_debug_matmul_by(const fhip_weight* w, int kernel, const float* d_x, size_t rows_x, float* d_y, void* stream);
+
 /* Measurement aid: one launch that reads nbytes at d_src (16-byte loads over the whole chip) and does nothing else; d_sink is
  * one device word that is practically never written. Timed beside a mat-vec of the same size it gives the time a perfect reader
  * needs for those bytes on this device. No counterpart in the reference (its matvec_roofline example prints bytes / time of the

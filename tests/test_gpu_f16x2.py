@@ -344,8 +344,8 @@ def test_ordered_policy_gives_the_same_bits_on_every_run(F, O):
         lib.fhip_batch_policy(before)
 
 
-@pytest.mark.parametrize("ty,n_embd,n_ff,out,t,own", [(Q4_K, 7168, 256, 14400, 8, True), (Q6_K, 6400, 256, 14401, 5, True), (Q5_K, 7168, 256, 14400, 20, False),
-                                                       (Q6_K, 10240, 256, 14400, 12, True), (Q4_K, 5120, 17408, 515, 32, False)])
+@pytest.mark.parametrize("ty,n_embd,n_ff,out,t,own", [(Q4_K, 7168, 256, 14400, 8, True), (Q6_K, 6400, 256, 14401, 5, True), (Q5_K, 7168, 256, 14400, 20, True),
+                                                       (Q6_K, 10240, 256, 14400, 12, True), (Q4_K, 5120, 17408, 515, 32, True)])
 def test_ffn_leaves_the_sums_of_a_cut_gate_up_to_the_next_launch(F, ty, n_embd, n_ff, out, t, own):
     # gate|up whose rows are cut along K between workgroups: the block leaves its partial sums to the launch that prepares the down projection's
     # activations; the three calls it stands for add them in a launch of their own, in the same order: the same bits
@@ -363,16 +363,23 @@ def test_ffn_leaves_the_sums_of_a_cut_gate_up_to_the_next_launch(F, ty, n_embd, 
     assert np.isfinite(y).all() and np.array_equal(h.matmul_q(wdn).to_vec(), y)
 
 
+def by(F, w, kernel, xt, t):
+    """fhip_matmul_q of the first t rows by the kernel named"""
+    y = F.Tensor.empty((t, F._lib.load().fhip_weight_rows(w.handle)))
+    F._lib.check(F._lib.load().fhip_debug_matmul_by(w.handle, kernel, xt.buf.ptr, t, y.buf.ptr, None))
+    return y.to_vec().reshape(y.shape)
+
+
 @pytest.mark.parametrize("ty,rows,cols,kernel,ts", [
     (8, 130, 32, "HELD", (5, 7, 8, 9, 13, 16)), (8, 33, 288, "HELD", (5, 7, 8, 9, 13, 16)), (8, 600, 512, "HELD", (5, 7, 8, 9, 13, 16)), (12, 40, 256, "HELD", (5, 7, 8, 9, 13, 16)),
     (12, 1100, 512, "HELD", (5, 7, 8, 9, 13, 16)), (13, 300, 512, "HELD", (5, 7, 8, 9, 13, 16)), (14, 600, 256, "HELD", (5, 7, 8, 9, 13, 16)), (14, 129, 512, "HELD", (5, 7, 8, 9, 13, 16)),
     (12, 600, 5120, "OWN_ROWS", (5, 7, 8)), (13, 301, 7168, "OWN_ROWS", (5, 8)), (14, 130, 4608, "OWN_ROWS", (5, 7, 8)), (14, 129, 6400, "OWN_ROWS", (5, 8, 9, 13, 16)),
     (8, 257, 5152, "OWN_ROWS", (5, 7, 8)), (8, 131, 6432, "OWN_ROWS", (5, 8, 9, 13, 16))])
 def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows, cols, kernel, ts):
-    """A launch that makes its chunks' operand rows itself; fhip_matmul_q_f16x2 prepares them by a launch of its own. Where two chunks
+    """A launch that makes its chunks' operand rows itself (the kernel named, whichever fhip_matmul_q picks); fhip_matmul_q_f16x2 prepares them by a launch of its own. Where two chunks
     at most are not zero (sums of two terms, whose order does not matter) both have the same bits, for every number of rows the kernel takes, a last
     chunk that is not full, an odd number of weight rows, rows of zeros, chunks of tiny, huge and non-finite values."""
-    from conftest import ROUTES, bits, route
+    from conftest import ROUTES, bits
     from ferric_amd.synth import synth_weights
     rng = np.random.default_rng(rows + cols)
     lib = F._lib.load()
@@ -382,15 +389,9 @@ def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows,
         x = (rng.standard_normal((t, cols)) * np.exp2(rng.integers(-20, 20, (t, 1)))).astype(np.float32)
         x[0, :30], x[1], x[2, 7], x[3, -1], x[4, 20] = 1e-41, 0.0, 3e38, -np.inf, np.nan
         x[:, 256:(cols - 1) // 256 * 256] = 0.0
-        xt, ws, ys = F.Tensor.from_vec(x, x.shape), F.DeviceBuffer(lib.fhip_matmul_q_f16x2_ws_bytes(w.handle, t)), []
-        assert [(k & ~ROUTES["CUT"], n) for k, n in route(F, w, xt, t)] == [(ROUTES[kernel], t)]
-        for prepared in (False, True):
-            y = F.Tensor.empty((t, rows))
-            if prepared:
-                F._lib.check(lib.fhip_matmul_q_f16x2(w.handle, xt.buf.ptr, t, y.buf.ptr, ws.ptr, None))
-            else:
-                F._lib.check(lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, None))
-            ys.append(y.to_vec())
+        xt, ws, y = F.Tensor.from_vec(x, x.shape), F.DeviceBuffer(lib.fhip_matmul_q_f16x2_ws_bytes(w.handle, t)), F.Tensor.empty((t, rows))
+        F._lib.check(lib.fhip_matmul_q_f16x2(w.handle, xt.buf.ptr, t, y.buf.ptr, ws.ptr, None))
+        ys = [by(F, w, ROUTES[kernel], xt, t).reshape(-1), y.to_vec()]
         nan = np.isnan(ys[0])
         assert np.array_equal(nan, np.isnan(ys[1])) and nan.any(), t
         assert np.array_equal(bits(ys[0])[~nan], bits(ys[1])[~nan]), t
@@ -404,7 +405,7 @@ def test_operand_rows_made_by_the_workgroups_have_the_prepared_bits(F, ty, rows,
     (Q4_K, 600, 5120, 12), (Q8_0, 4200, 5152, 16), (Q6_K, 1300, 4608, 32), (Q8_0, 2100, 4384, 5), (Q4_K, 4360, 6144, 8),   # twelve waves, one tile or several; eight
     (Q4_K, 3110, 512, 30), (Q8_0, 14300, 256, 6)])  # two workgroups a CU; one chunk
 def test_whole_rows_inside_a_workgroup(F, O, ty, rows, cols, t):
-    # The one-launch product at the edges of its tiles (16 weight rows), of its sets (8 activation rows) and of the chunks its waves hold (a last
+    # The one-launch product (by its name, whether or not fhip_matmul_q takes it there) at the edges of its tiles (16 weight rows), of its sets (8 activation rows) and of the chunks its waves hold (a last
     # wave without one, Q8_0's partial chunk), at the bar of the kernels it stands in for; a row of inf or NaN stays alone, and a second run
     # has the same bits.
     from conftest import ROUTES, route
@@ -416,23 +417,26 @@ def test_whole_rows_inside_a_workgroup(F, O, ty, rows, cols, t):
     x[t - 2, 1] = -np.inf
     qm, xt = F.QMatrix.from_bytes(w, ty, rows, cols), F.Tensor.from_vec(x, x.shape)
     qm.batch_policy(F.BATCH_ORDERED)
-    assert route(F, qm, xt, t) == [(ROUTES["HELD"], t)]
+    routed = route(F, qm, xt, t) == [(ROUTES["HELD"], t)]
+    product = lambda: by(F, qm, ROUTES["HELD"], xt, t)
     good = np.arange(t - 2)
     y64, wn = O.matmul_f64(x[good], w, ty, rows, cols)
     bound = TIGHT * wn[None, :] * np.linalg.norm(x[good].astype(np.float64), axis=1)[:, None]
-    y = xt.matmul_q(qm).to_vec().reshape(t, rows)
+    y = product()
     assert (np.abs(y[good] - y64) <= bound + 1e-300).all()
     assert not y[1].any() and np.isnan(y[t - 1]).all() and not np.isfinite(y[t - 2]).any()
-    assert np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
+    assert np.array_equal(product(), y, equal_nan=True)
+    assert not routed or np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
 
 
 @pytest.mark.parametrize("ty,rows,cols,t,own,cut", [
     (Q4_K, 5, 6400, 8, True, True), (Q6_K, 17, 17408, 5, True, True), (Q8_0, 31, 6432, 7, True, True), (Q5_K, 300, 12288, 3, True, True),      # fewer units than waves; a last chunk that is not full
     (Q5_K, 8210, 5120, 8, True, True), (Q4_K, 8193, 5376, 12, True, True), (Q6_K, 5200, 4608, 16, True, True),                                # tiles that waves share, a last tile of few rows
     (Q4_K, 33001, 512, 6, True, False), (Q6_K, 20990, 768, 11, True, False), (Q8_0, 8200, 1056, 30, True, False),                              # whole rows; Q8_0 beyond sixteen
-    (Q8_0, 140, 6432, 17, False, True), (Q4_K, 1500, 5120, 32, False, True), (Q6_K, 2000, 6400, 25, False, True)])                             # two sets, prepared rows
+    (Q8_0, 140, 6432, 17, True, True), (Q4_K, 1500, 5120, 32, True, True), (Q6_K, 2000, 6400, 25, True, True)])                                # two sets
 def test_operand_rows_in_a_workgroups_lds(F, O, ty, rows, cols, t, own, cut):
-    # sums of up to 256-column chunks in f32, as in the kernels it stands beside: their bar. A row of inf or NaN stays alone, and a second run has the same bits.
+    # sums of up to 256-column chunks in f32, as in the kernels it stands beside: their bar. A row of inf or NaN stays alone, and a second run has the same bits, as has
+    # one from rows that a launch in front prepares.
     from conftest import ROUTES, route
     from ferric_amd.synth import synth_weights
     w = synth_weights(ty, rows, cols, rows + t)
@@ -449,9 +453,10 @@ def test_operand_rows_in_a_workgroups_lds(F, O, ty, rows, cols, t, own, cut):
     assert (np.abs(y[good] - y64) <= bound + 1e-300).all()
     assert np.isnan(y[t - 1]).all() and not np.isfinite(y[t - 2]).any()
     assert np.array_equal(xt.matmul_q(qm).to_vec().reshape(t, rows), y, equal_nan=True)
+    assert np.array_equal(by(F, qm, ROUTES["PREPARED"], xt, t), y, equal_nan=True)
 
 
-@pytest.mark.parametrize("ty,rows,cols,t", [(Q5_K, 400, 5120, 6), (Q4_K, 2050, 5632, 13), (Q6_K, 1605, 6144, 30), (Q8_0, 301, 5152, 8), (Q8_0, 4200, 4384, 25)])
+@pytest.mark.parametrize("ty,rows,cols,t", [(Q5_K, 400, 5120, 6), (Q4_K, 2050, 5632, 13), (Q6_K, 515, 6144, 30), (Q8_0, 301, 5152, 8), (Q8_0, 4200, 4384, 25)])
 def test_a_cut_product_has_the_same_bits_with_and_without_a_workspace(F, ty, rows, cols, t):
     """K in two or more ranges, whose partial outputs meet in the stream's workspace; where a capture on the stream, or one that the thread has open on another stream, keeps
     the library from making that workspace, the product goes on without it. It has the bits it has with it, replay after replay, and another product's workspace changes none."""

@@ -114,6 +114,41 @@ def test_where_the_runs_of_run_sums_end(gemm):
         assert plan(gemm, *shape, run_sums=True)[1:5] == runs, shape
 
 
+@pytest.fixture(scope="module")
+def f16x2(tmp_path_factory):
+    lib = C.CDLL(build(tmp_path_factory.mktemp("f16x2"), "f16x2_rules_harness.cpp", [], ["-shared", "-Wl,-Bsymbolic"]))
+    lib.h_held.argtypes = [C.c_uint32, C.c_size_t, C.c_size_t, C.c_size_t]
+    lib.h_resident.argtypes = lib.h_held.argtypes + [C.POINTER(C.c_int64)]
+    return lib
+
+
+def test_the_kernel_of_a_small_batch(f16x2):
+    """Sums in order, both kernels timed, us: the held one, the one whose operand rows lie in LDS (cold weights, 256 CUs). The rule may be off by a tenth, as near its lines, and no more."""
+    timed = {
+        (Q4_K, 515, 512, 8): (3.8, 4.2), (Q4_K, 34816, 256, 8): (7.3, 5.1), (Q4_K, 8200, 256, 16): (5.4, 4.4), (Q4_K, 4090, 1280, 8): (5.5, 5.6), (Q4_K, 8200, 1280, 8): (7.6, 6.2),
+        (Q4_K, 34816, 1280, 8): (13.0, 10.9), (Q6_K, 16400, 3072, 8): (16.6, 18.3), (Q8_0, 20000, 2784, 8): (20.8, 23.3), (Q4_K, 4090, 1024, 16): (5.4, 7.0), (Q4_K, 34816, 1280, 16): (22.8, 13.4),
+        (Q4_K, 12000, 2048, 16): (11.4, 12.7), (Q6_K, 20000, 2048, 16): (16.6, 18.4), (Q4_K, 8200, 3584, 16): (14.8, 13.1), (Q8_0, 4090, 2272, 32): (12.7, 14.0), (Q8_0, 6100, 2272, 32): (17.2, 14.9),
+        (Q4_K, 34816, 1024, 32): (25.9, 16.1), (Q5_K, 2050, 3584, 32): (12.1, 10.3), (Q4_K, 5130, 6144, 8): (15.7, 11.1), (Q6_K, 515, 6144, 32): (11.4, 9.4), (Q4_K, 100, 4352, 16): (10.2, 7.4)}
+    for shape, (held, resident) in timed.items():
+        assert (held, resident)[f16x2.h_held(*shape) == 0] <= 1.1 * min(held, resident), shape
+
+
+@pytest.mark.parametrize("ty,block", [(Q4_K, 256), (Q5_K, 256), (Q6_K, 256), (Q8_0, 32)])
+def test_ranges_of_k_of_a_small_batch(f16x2, ty, block):
+    """A range's operand rows fit the LDS, no range is empty, the workgroups are no more than the CUs unless K alone asks for them, and the partial outputs fit the space asked for; from one
+    chunk to the longest rows."""
+    out, cus = (C.c_int64 * 6)(), 256
+    for cols in sorted({block, 256, 288 // block * block, *range(256, 65537, 1280 if block == 256 else 1248), 16640, 16896 if block == 256 else 16672, 65536}):
+        for rows in (1, 17, 700, 5120, 151936):
+            for t in (3, 8, 9, 16, 17, 24, 32):
+                f16x2.h_resident(ty, rows, cols, t, out)
+                nt, sets, parts, per_part, most, ws = out
+                chunks = (cols + 255) // 256
+                assert 8 * nt * sets >= t and 1 <= parts <= chunks and (chunks + parts - 1) // parts <= most, (rows, cols, t)
+                assert 1 <= per_part <= (rows + 15) // 16 and (per_part == 1 or parts * sets * per_part <= cus), (rows, cols, t)
+                assert ws >= (parts * t * rows * 4 if parts > 1 else 0), (rows, cols, t)
+
+
 class Weight(C.Structure):
     """struct fhip_weight (ferric_amd/csrc/common.hpp), for a query that reads its type and shape."""
     _fields_ = [("type", C.c_uint32), ("rows", C.c_size_t), ("cols", C.c_size_t), ("row_bytes", C.c_size_t), ("nbytes", C.c_size_t), ("d_raw", C.c_void_p), ("owns", C.c_bool),
