@@ -80,6 +80,7 @@ int make_weight(uint32_t ty, size_t nbytes, size_t rows, size_t cols, fhip_weigh
     if (rows > 0x7FFFFFFFull || cols > 0x7FFFFFFFull) return fhip::set_error(FHIP_ERR_SHAPE, "weight dimensions exceed 2^31");
     w.type = ty; w.rows = rows; w.cols = cols; w.row_bytes = row_bytes; w.nbytes = nbytes; w.d_raw = nullptr; w.owns = false;
     w.planes = g_default_planes; w.batch_policy = g_default_batch_policy;
+    fhip::gemm_f16x2_lay_out(&w);
     return FHIP_OK;
 }
 

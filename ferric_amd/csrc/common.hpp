@@ -8,6 +8,11 @@
 #include "../../include/ferric_hip.h"
 #include "../../include/ferric_hip_debug.h"
 
+namespace fhip {
+// Launch of the small-batch kernel whose operand rows lie in LDS (gemm_f16x2.hip): sets of eight activation rows of a workgroup and workgroups' sets, ranges of K, workgroups of a range
+struct F16Plan { int nt, sets, parts, per_part; };
+}  // namespace fhip
+
 struct fhip_weight {
     uint32_t type;      // ggml id: 2 / 3 / 6 / 7 / 8 / 12 / 13 / 14 / 20 / 23 / 39
     size_t rows, cols;  // [out, in]
@@ -19,6 +24,7 @@ struct fhip_weight {
     // changed only through the handle's own setters: launches on other handles never see it.
     int planes;         // activation planes of its streaming mat-vec: 3 = 24-bit (the f32 significand), 2 = 16-bit
     int batch_policy;   // FHIP_BATCH_*: which kernels its batches of three rows and more take
+    fhip::F16Plan f16[3];   // up to 8, 16 and 32 activation rows (gemm_f16x2_lay_out); they follow from the shape, and working one out takes 0.2 us
 };
 
 namespace fhip {

@@ -33,6 +33,7 @@ int launch_gemm_f16x2_held(const fhip_weight* w, const float* d_x, size_t t, flo
 // the product from prepared rows (d_xp) or, where gemm_f16x2_resident_own_x says so, from the rows as they are (d_xp null): one launch and, where it cuts K into more than
 // one part, one that adds the partial outputs (d_part: gemm_f16x2_parts_bytes) or leaves them to the reader of y (deferred). d_part null: a launch a part, each adding to y,
 // which has the same bits (the rows as they are, apart from y, and not deferred)
+void gemm_f16x2_lay_out(fhip_weight* w);     // a new handle's plans, which the others read
 int gemm_f16x2_parts(const fhip_weight* w, size_t t);
 size_t gemm_f16x2_parts_bytes(const fhip_weight* w, size_t t);
 bool gemm_f16x2_resident_own_x(const fhip_weight* w, const float* d_x, size_t t, const float* d_y);

@@ -1663,7 +1663,7 @@ int launch_held_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y
     return fhip::check_hip(hipGetLastError(), "gemm_q_f16x2 launch");
 }
 
-struct ResPlan { int nt, sets, parts, per_part; };
+using ResPlan = fhip::F16Plan;
 template <class F>
 constexpr int resident_chunks_of(int nt) { return nt == 1 ? resident_chunks<F, 1>() : resident_chunks<F, 2>(); }
 // How many ranges K is cut into: the fewest that fit, or more where the estimate below says so. In us, fitted to 676 products of three formats (100 .. 34816 x 512 .. 17408, 8 to
@@ -1688,9 +1688,11 @@ ResPlan resident_plan(const fhip_weight* w, size_t t) {
     return best;
 }
 
+const ResPlan& plan_of(const fhip_weight* w, size_t t) { return w->f16[t <= 8 ? 0 : t <= 16 ? 1 : 2]; }
+
 template <class F>
 int launch_resident_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, size_t t, float* d_y, float* d_part, hipStream_t s, fhip::F16Parts* deferred) {
-    const ResPlan q = resident_plan(w, t);
+    const ResPlan q = plan_of(w, t);
     ResidentParams p;
     p.W = w->d_raw; p.Xp = d_xp; p.X = d_x; p.Y = q.parts > 1 ? d_part : d_y;
     p.T = (int)t; p.N = (int)w->rows; p.K = (int)w->cols; p.nblk = (int)(w->cols / 32); p.row_bytes = w->row_bytes; p.xp_sets = prepared_sets(t);
@@ -1813,7 +1815,10 @@ bool gemm_f16x2_supports(const fhip_weight* w, size_t t) {
     return (w->type == FHIP_Q4_K || w->type == FHIP_Q5_K || w->type == FHIP_Q6_K) && t <= 32 && w->cols % CHUNK == 0;
 }
 
-int gemm_f16x2_parts(const fhip_weight* w, size_t t) { return resident_plan(w, t).parts; }
+void gemm_f16x2_lay_out(fhip_weight* w) {
+    for (size_t t : {(size_t)8, (size_t)16, (size_t)32}) w->f16[t / 16] = gemm_f16x2_supports(w, 8) ? resident_plan(w, t) : ResPlan{1, 1, 1, 1};
+}
+int gemm_f16x2_parts(const fhip_weight* w, size_t t) { return plan_of(w, t).parts; }
 // (the most any batch of up to t rows needs: a batch of fewer rows may be cut into more ranges)
 size_t gemm_f16x2_parts_bytes(const fhip_weight* w, size_t t) {
     size_t m = 0;
