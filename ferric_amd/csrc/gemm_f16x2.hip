@@ -1756,22 +1756,27 @@ bool held_beats_streaming(const fhip_weight* w, size_t t) {
 // unpacking passes its sets of eight rows make (us, held | resident, cold weights, sums in order).
 // - One chunk: only where the resident kernel's sixteen rows at a time are half empty (Q4_K 1300 x 256 at 8 rows 3.7 | 3.5, 16 3.7 | 3.9, 32 4.6 | 4.0; 34816 x 256 at 8 7.3 | 5.1).
 // - Up to eight rows: a tile and a half a CU of the formats with minima, three of 8 to 12 chunks (Q4_K 4090 x 1280 5.5 | 5.6, 8200 x 1280 7.6 | 6.2, 12000 x 2304 9.7 | 9.3, 16400 12.1 |
-//   11.3); Q6_K five (16400 x 3072 16.6 | 18.3, 34816 29.3 | 29.0), Q8_0 nine (34816 x 4064 45.9 | 47.6).
+//   11.3); Q6_K five, Q8_0 nine, and both whatever the tiles from 12 chunks on (Q6_K 16400 x 3072 16.6 | 18.3, 151936 x 4096 118.0 | 134.0, 128256 x 2560
+//   76.0 | 68.9; Q8_0 34816 x 4064 45.9 | 47.6, 151936 x 3584 144.5 | 159.7).
 // - Nine to sixteen: a tile and a half (Q4_K 4090 x 1024 5.4 | 7.0, 8200 x 1024 7.7 | 7.3, 34816 x 1280 22.8 | 13.4), three of eight chunks (12000 x 2048 11.4 | 12.7), five where there
-//   are no minima either (Q6_K 20000 x 2048 16.6 | 18.4, Q8_0 20000 x 1760 17.4 | 19.6); two beyond (8200 x 2560 11.9 | 12.1).
+//   are no minima either (Q6_K 20000 x 2048 16.6 | 18.4, Q8_0 20000 x 1760 17.4 | 19.6); two beyond (8200 x 2560 11.9 | 12.1). Vocabularies without minima are the held
+//   one's again, from 12 chunks and 11 tiles on (Q6_K 41500 x 4096 at 16 42.6 | 44.9, 151936 x 3584 at 16 110.8 | 136.7, Q8_0 153.5 | 174.0).
 // - More: eight tenths (Q4_K 3070 x 1024 at 24 rows 6.2 | 6.7, 4090 x 1024 7.0 | 6.7, 34816 x 1024 at 32 25.9 | 16.1), with 8 to 12 chunks a tile and a half to 24 rows (Q8_0 6100 x 2272 15.3 |
 //   14.5, 8200 19.7 | 18.2), then one (4090 x 2272 at 32 12.7 | 14.0, 6100 17.2 | 14.9); with more chunks half of one (Q5_K 2050 x 3584 at 32 12.1 | 10.3).
-// - Beyond 16 chunks: nowhere. 572 products (17, 20 and 24 chunks, 100 .. 8200 rows, 5 .. 32 activation rows) 0.61 .. 1.00 of its time, geometric mean 0.75.
+// - Beyond 16 chunks: up to eight rows of a vocabulary without minima, Q6_K from ten tiles a CU on, Q8_0 from six (Q6_K 34816 x 5120 40.6 | 40.3, 60000 65.1 | 68.1, 151936 148.9 | 164.4; Q8_0
+//   24600 x 5120 39.8 | 39.7, 60000 87.3 | 92.8, 151936 206.6 | 221.5; Q4_K 151936 x 5120 108.4 | 109.0). Elsewhere nowhere: 572 products (17, 20 and 24 chunks, 100 .. 8200 rows, 5 .. 32
+//   activation rows) 0.61 .. 1.00 of its time, geometric mean 0.75.
 // 2816 products of the four formats (1 .. 16 chunks, 515 .. 34816 rows, 8, 16, 24 and 32 activation rows): what this picks takes 1.006 of the faster one's time (geometric mean), 1.054 at the
-// 95th percentile, 1.20 at most.
+// 95th percentile, 1.20 at most; of 2424 more (4 .. 24 chunks, 8200 .. 151936 rows, 5 .. 32 activation rows) 1.004, 1.036 and 1.20, 1.013 without the lines of vocabularies.
 bool held_beats_resident(const fhip_weight* w, size_t t) {
     const size_t chunks = (w->cols + CHUNK - 1) / CHUNK, tiles = (w->rows + 15) / 16;
     const size_t cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     const bool q6 = w->type == FHIP_Q6_K, q8 = w->type == FHIP_Q8_0, mins = !q6 && !q8, middle = chunks >= (q8 ? 6 : 8) && chunks <= 12;
     auto halves = [&](size_t most) { return 2 * tiles <= most * cus; };   // half tiles a CU
-    if (chunks > 16) return false;
+    if (chunks > 16) return t <= 8 && !mins && tiles > (q6 ? 10 : 6) * cus;
     if (chunks == 1) return t > 8 && t <= 24 && halves(1);
-    if (t <= 8) return halves(mins ? (middle ? 6 : 3) : q6 ? 10 : 18);
+    if (t <= 8) return halves(mins ? (middle ? 6 : 3) : q6 ? 10 : 18) || (!mins && chunks >= 12);
+    if (t <= 16 && !mins && chunks >= 12 && tiles > 11 * cus) return true;
     if (chunks > 12) return halves(t <= 16 ? 4 : 1);
     if (t <= 16) return halves(!middle ? 3 : chunks > 8 ? 4 : mins ? 6 : 10);
     return middle ? halves(t <= 24 ? 3 : 2) : 5 * tiles <= 4 * cus;

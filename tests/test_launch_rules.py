@@ -128,7 +128,9 @@ def test_the_kernel_of_a_small_batch(f16x2):
         (Q4_K, 515, 512, 8): (3.8, 4.2), (Q4_K, 34816, 256, 8): (7.3, 5.1), (Q4_K, 8200, 256, 16): (5.4, 4.4), (Q4_K, 4090, 1280, 8): (5.5, 5.6), (Q4_K, 8200, 1280, 8): (7.6, 6.2),
         (Q4_K, 34816, 1280, 8): (13.0, 10.9), (Q6_K, 16400, 3072, 8): (16.6, 18.3), (Q8_0, 20000, 2784, 8): (20.8, 23.3), (Q4_K, 4090, 1024, 16): (5.4, 7.0), (Q4_K, 34816, 1280, 16): (22.8, 13.4),
         (Q4_K, 12000, 2048, 16): (11.4, 12.7), (Q6_K, 20000, 2048, 16): (16.6, 18.4), (Q4_K, 8200, 3584, 16): (14.8, 13.1), (Q8_0, 4090, 2272, 32): (12.7, 14.0), (Q8_0, 6100, 2272, 32): (17.2, 14.9),
-        (Q4_K, 34816, 1024, 32): (25.9, 16.1), (Q5_K, 2050, 3584, 32): (12.1, 10.3), (Q4_K, 5130, 6144, 8): (15.7, 11.1), (Q6_K, 515, 6144, 32): (11.4, 9.4), (Q4_K, 100, 4352, 16): (10.2, 7.4)}
+        (Q4_K, 34816, 1024, 32): (25.9, 16.1), (Q5_K, 2050, 3584, 32): (12.1, 10.3), (Q4_K, 5130, 6144, 8): (15.7, 11.1), (Q6_K, 515, 6144, 32): (11.4, 9.4), (Q4_K, 100, 4352, 16): (10.2, 7.4),
+        (Q6_K, 151936, 5120, 8): (148.9, 164.4), (Q6_K, 8200, 5120, 8): (18.0, 16.2), (Q8_0, 80000, 5632, 8): (115.3, 137.6), (Q6_K, 151936, 3584, 16): (110.8, 136.7),
+        (Q8_0, 151936, 3584, 16): (153.5, 174.0), (Q4_K, 151936, 5120, 16): (192.5, 131.7), (Q6_K, 128256, 2560, 8): (76.0, 68.9), (Q8_0, 100000, 5120, 12): (212.3, 153.5)}
     for shape, (held, resident) in timed.items():
         assert (held, resident)[f16x2.h_held(*shape) == 0] <= 1.1 * min(held, resident), shape
 
