@@ -583,7 +583,6 @@ struct F16Params {
     int nblk;             // Q8_0: blocks in a weight row (the last chunk may hold fewer than 8)
     size_t row_bytes;
     long long units;      // row groups * nchunks, chunk fastest
-    int group;            // rows of a group: 128, or 256 for the eight-wave row-streaming kernel
 };
 
 template <class F, int NT>
@@ -1574,14 +1573,13 @@ Plan make_plan(const fhip_weight* w, size_t t) {
     return q;
 }
 
-// Whether the launch makes its operand rows itself: the same bits, a launch and a trip of the rows through memory less, but every
-// workgroup that holds a chunk converts it (two rows of 256 values a wave, between a chunk's products and the next barrier). Ordered
-// sums, 8 rows, us, itself | prepared: one unit a workgroup Q8_0 4096 x 4096 12.4 | 14.2, Q4_K 1024 x 5120 9.3 | 11.4, Q6_K 2048 x 9728 14.2 | 16.3;
-// two, 12288 x 4096 Q8_0 22.0 | 22.8, Q4_K 16.5 | 16.9, Q6_K 20.4 | 20.4; more, 5120 x 17408 Q8_0 34.5 | 35.5, Q4_K 25.8 | 24.2, 34816 x 5120 Q4_K
-// 38.9 | 34.2. At 16 rows: 4096 x 4096 Q8_0 15.3 | 16.4, Q6_K 14.1 | 15.2, 12288 x 4096 (three) Q6_K 26.2 | 25.7.
+// Whether a launch that adds by atomics makes its operand rows itself: the same bits, a launch and a trip of the rows through memory less, but every workgroup that holds a chunk converts
+// it (two rows of 256 values a wave, between a chunk's products and the next barrier). Rows of one chunk that the held kernel leaves (held_beats_streaming) only: us, itself | prepared, 8 rows,
+// 20000 x 256 Q4_K 5.7 | 7.0, Q6_K 5.8 | 7.6, 60000 x 256 7.7 | 8.8, 8.3 | 9.8, Q8_0 9.8 | 11.2, 151936 x 256 14.1 | 12.8, 14.4 | 16.2, 18.5 | 19.0; 16 rows Q6_K 60000 x 256 10.8 | 11.5, 151936
+// 23.1 | 21.7. Of two chunks 100000 x 512 Q4_K 18.3 | 15.8, Q6_K 21.5 | 20.9, 151936 x 512 22.3 | 20.2, 26.4 | 25.4. Of more, products that are not cut have too many.
 bool own_x(const fhip_weight* w, const Plan& q, const float* d_x) {
     const bool rows_kernel = (q.nt == 1 && q.group == 128) || (q.nt == 2 && (w->type == FHIP_Q8_0 || w->type == FHIP_Q6_K));
-    return rows_kernel && d_x && ((uintptr_t)d_x & 15) == 0 && q.units <= 2 * (long long)q.grid;
+    return rows_kernel && d_x && ((uintptr_t)d_x & 15) == 0 && q.nchunks == 1;
 }
 
 template <class F>
@@ -1601,7 +1599,7 @@ int launch_fmt(const fhip_weight* w, const uint16_t* d_xp, const float* d_x, siz
     p.W = w->d_raw; p.Xp = d_xp; p.X = d_x; p.K = (int)w->cols; p.Y = d_y;
     p.T = (int)t; p.N = (int)w->rows; p.nchunks = q.nchunks; p.row_bytes = w->row_bytes;
     p.nblk = (int)(w->cols / 32);
-    p.units = q.units; p.group = q.group;
+    p.units = q.units;
     if (q.split && !y_cleared) {
         const size_t n = t * w->rows;
         hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_y, n);

@@ -490,3 +490,40 @@ def test_a_cut_product_has_the_same_bits_with_and_without_a_workspace(F, ty, row
         check(lib.fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
         g.launch()
         assert np.array_equal(bits(y.to_vec(stream)), want)
+
+
+@pytest.mark.parametrize("ty,rows,cols,t", [(Q4_K, 300, 256, 7), (Q5_K, 129, 256, 5), (Q6_K, 600, 256, 13), (Q6_K, 257, 256, 16), (Q8_0, 130, 32, 5), (Q8_0, 301, 224, 16), (Q8_0, 257, 256, 8)])
+def test_rows_of_one_chunk_under_atomic_sums(F, ty, rows, cols, t):
+    """The row-streaming kernel that makes its operand rows itself: the bits it has from rows that a launch in front prepares. Nothing is cut, so nothing is added by atomics."""
+    from conftest import ROUTES, bits
+    from ferric_amd.synth import synth_weights
+    w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
+    w.batch_policy(F.BATCH_AUTO)
+    x = np.random.default_rng(rows).standard_normal((t, cols)).astype(np.float32)
+    x[0, :30], x[1], x[2, 7], x[3, -1], x[4, 20] = 1e-41, 0.0, 3e38, -np.inf, np.nan
+    xt = F.Tensor.from_vec(x, x.shape)
+    own, prepared = by(F, w, ROUTES["OWN_ROWS"], xt, t), by(F, w, ROUTES["PREPARED"], xt, t)
+    nan = np.isnan(own)
+    assert np.array_equal(nan, np.isnan(prepared)) and nan[4].all() and np.isfinite(own[:2]).all()   # (3e38 times a weight overflows)
+    assert np.array_equal(bits(own)[~nan], bits(prepared)[~nan])
+
+
+@pytest.mark.parametrize("ty,rows,cols,t,kernel", [(Q4_K, 14500, 256, 12, "PREPARED"), (Q6_K, 98400, 512, 8, "PREPARED"), (Q4_K, 14500, 256, 7, "OWN_ROWS")])
+def test_atomic_sums_without_a_cut_are_captured_without_a_workspace(F, ty, rows, cols, t, kernel):
+    # whole rows a workgroup whose operand rows are prepared, in the stream's workspace: a capture on a stream that has none takes the held kernel's one launch
+    from conftest import ROUTES, route
+    from ferric_amd.synth import synth_weights
+    lib, check = F._lib.load(), F._lib.check
+    w = F.QMatrix.from_bytes(np.tile(synth_weights(ty, 100, cols, 5), rows // 100), ty, rows, cols)
+    w.batch_policy(F.BATCH_AUTO)
+    x = np.random.default_rng(6).standard_normal((t, cols)).astype(np.float32)
+    xt, y, stream = F.Tensor.from_vec(x, x.shape), F.Tensor.empty((t, rows)), F.Stream()
+    assert route(F, w, xt, t) == [(ROUTES[kernel], t)]
+    want = xt.matmul_q(w).to_vec()
+    g = F.Graph.begin(stream)
+    check(lib.fhip_matmul_q(w.handle, xt.buf.ptr, t, y.buf.ptr, stream.handle))
+    g.end()
+    for _ in range(3):
+        check(lib.fhip_memset(y.buf.ptr, 0xFF, t * rows * 4, stream.handle))
+        g.launch()
+        assert np.abs(y.to_vec(stream) - want).max() <= 2e-6 * np.abs(want).max()
