@@ -456,6 +456,34 @@ def test_operand_rows_in_a_workgroups_lds(F, O, ty, rows, cols, t, own, cut):
     assert np.array_equal(by(F, qm, ROUTES["PREPARED"], xt, t), y, equal_nan=True)
 
 
+@pytest.mark.parametrize("ty,rows,cols,t", [(Q8_0, 70, 16960, 17), (Q4_K, 40, 23552, 24), (Q5_K, 33, 40960, 9), (Q6_K, 33, 65536, 32), (Q6_K, 20, 30720, 16), (Q8_0, 301, 1056, 5), (Q4_K, 17, 65536, 8)])
+def test_rows_of_every_magnitude_and_every_length_in_a_workgroups_lds(F, O, ty, rows, cols, t):
+    # the kernel above (by its name, so that short rows are its own too) over long rows in many ranges, one and two sets of eight or sixteen activation rows, whose chunks are tiny,
+    # huge and zero side by side; Q6_K's weights at the ends of their range, products beyond f16's exact integers: 2.5e-4 for those, as above
+    from conftest import ROUTES
+    from ferric_amd.synth import synth_weights
+    rng = np.random.default_rng(cols)
+    w, tol = synth_weights(ty, rows, cols, rows), TIGHT
+    x = rng.standard_normal((t, cols)).astype(np.float32)
+    x[0] *= np.float32(1e-30)
+    x[1] *= np.float32(1e30)
+    x[2] = 0.0
+    x[3, 17] = np.float32(3e6)
+    x[4] *= np.exp2(rng.integers(-60, 60, (cols + 255) // 256)).repeat(256)[:cols].astype(np.float32)
+    x[t - 1] *= np.float32(2.0 ** -118)
+    if ty == Q6_K:
+        w, tol = w.reshape(rows, cols // 256, 210).copy(), 2.5e-4
+        w[:, :, 192:208] = rng.choice(np.array([127, 125, -127, -128], np.int8).view(np.uint8), size=(rows, cols // 256, 16))
+        w = w.reshape(-1)
+    qm, xt = F.QMatrix.from_bytes(w, ty, rows, cols), F.Tensor.from_vec(x, x.shape)
+    qm.batch_policy(F.BATCH_ORDERED)
+    y64, wn = O.matmul_f64(x, w, ty, rows, cols)
+    bound = tol * wn[None, :] * np.linalg.norm(x.astype(np.float64), axis=1)[:, None]
+    own, prepared = by(F, qm, ROUTES["OWN_ROWS"], xt, t), by(F, qm, ROUTES["PREPARED"], xt, t)
+    assert (np.abs(own - y64) <= bound + 1e-300).all() and not own[2].any()
+    assert np.array_equal(own, prepared)
+
+
 @pytest.mark.parametrize("ty,rows,cols,t", [(Q5_K, 400, 5120, 6), (Q4_K, 2050, 5632, 13), (Q6_K, 515, 6144, 30), (Q8_0, 301, 5152, 8), (Q8_0, 4200, 4384, 25)])
 def test_a_cut_product_has_the_same_bits_with_and_without_a_workspace(F, ty, rows, cols, t):
     """K in two or more ranges, whose partial outputs meet in the stream's workspace; where a capture on the stream, or one that the thread has open on another stream, keeps
