@@ -1667,7 +1667,8 @@ constexpr int resident_chunks_of(int nt) { return nt == 1 ? resident_chunks<F, 1
 // How many ranges K is cut into: the fewest that fit, or more where the estimate below says so. In us, fitted to 676 products of three formats (100 .. 34816 x 512 .. 17408, 8 to
 // 32 rows, every number of ranges): a round of four waves' operand rows 1, the longest run of units, the sums' launch 1.7 and 0.9 a megabyte of partial outputs, the
 // rows an XCD fetches (workgroups go to the eight XCDs in turn: of 8 ranges each has one) 0.8 a megabyte; tiles that all sixteen waves share add a wave's sum at a time.
-// What it picks takes 1.015 of the best number's time in the mean, 1.09 at the 95th percentile.
+// What it picks takes 1.015 of the best number's time in the mean, 1.09 at the 95th percentile. Q5_K's unit stands between its neighbours': 96 products of it (300 .. 34816 x 2560 .. 17408) 1.029,
+// Q4_K's of the same shapes 1.027, at most 1.12 (300 rows, either format).
 ResPlan resident_plan(const fhip_weight* w, size_t t) {
     const int nchunks = (int)((w->cols + CHUNK - 1) / CHUNK), tiles = (int)((w->rows + 15) / 16), cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
     const int nt = t <= 8 ? 1 : 2, sets = ((int)t + 8 * nt - 1) / (8 * nt);

@@ -244,7 +244,7 @@ def test_about_the_end_of_the_short_caches(F, Q, K, nh, nkv, hd, rows):
     (16, 2, 64, 6150, (6150, 5000)), (10, 2, 64, 5200, (5200,)), (6, 1, 128, 5121, (5121, 33)), (8, 1, 128, 7000, (7000, 6999)),
     (7, 1, 128, 16384, (16384, 9001))])
 def test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, hd, rows, lengths):
-    """Group sizes and lengths at the edges of the long-cache kernel's rounds (32 keys a wave, six waves, 64 or 256 splits), with the
+    """Group sizes and lengths at the edges of the long-cache kernel's rounds (32 keys a wave, eight waves, 41 to 128 splits), with the
     length on the device, a window and a softcap, against the oracle over the oracle's dequantized rows: the f32 attention's 1e-5
     of the largest output. Large scores (a query of magnitude 4) sharpen the softmax, where an error in a score would show."""
     from ferric_amd import decode as X
@@ -291,6 +291,38 @@ def test_long_caches_of_many_kv_heads_in_the_fewest_splits(F, Q, K, fmt, nkv, g,
     got = X.decode_attention_kvq(F.Tensor.from_vec(q, q.shape), kq, vq, nkv * g, nkv, length=cap, last_pos=word).to_vec()
     want = D.decode_attention(q[0], K.roundtrip(k, n, width, fmt), K.roundtrip(v, n, width, fmt), nkv * g, nkv, 0, 0.0).reshape(-1)
     assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("nkv,g,hd,n", [(8, 5, 128, 33), (8, 3, 64, 1), (5, 8, 128, 8340), (171, 3, 64, 514), (171, 5, 128, 514), (171, 8, 128, 258), (300, 6, 128, 31)])
+def test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, fmt, nkv, g, hd, n):
+    """The token's row is the first of a wave's round, its first round or a later one, or the only row of its split; splits behind it are empty; two splits at both head sizes.
+    With the post-processing inside the launch and in front of it: the same bits and the same row in the cache, the outputs at the bar above."""
+    from ferric_amd import decode as X
+    from oracle import decode_oracle as D
+    rng, lib, cap, nh, width = np.random.default_rng(n + fmt), F._lib.load(), max(n, 5121), nkv * g, nkv * hd
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    rows = [rng.standard_normal((n, width)).astype(np.float32) for _ in range(2)]
+    raw = rng.standard_normal((1, (nh + 2 * nkv) * hd)).astype(np.float32)
+    qkv, p, ws = T(raw), X._u32_tensor([n - 1]), F.DeviceBuffer(lib.fhip_decode_attention_ws_bytes(nh, nkv, hd, cap))
+    got = []
+    for one in (False, True):
+        kc, vc = (Q.QKvCache(fmt, cap, width).append(T(r)) for r in rows)
+        out, q = T(np.zeros((1, nh * hd), np.float32)), T(np.zeros((1, nh * hd), np.float32))
+        where = (kc.codes.ptr, kc.scales.ptr, vc.codes.ptr, vc.scales.ptr)
+        if one:
+            F._lib.check(lib.fhip_qkv_post_attention_kvq(fmt, qkv.buf.ptr, None, None, None, p.buf.ptr, None, nh, nkv, hd, 0, 0, 1e-6, 1e6, *where, cap, cap, 0, 0.0, ws.ptr,
+                                                         out.buf.ptr, None))
+        else:
+            F._lib.check(lib.fhip_qkv_post_kvq(fmt, qkv.buf.ptr, None, None, None, p.buf.ptr, None, 1, nh, nkv, hd, 0, 0, 1e-6, 1e6, q.buf.ptr, *where, cap, None))
+            F._lib.check(lib.fhip_decode_attention_kvq(fmt, q.buf.ptr, *where, nh, nkv, hd, cap, p.buf.ptr, 0, 0.0, ws.ptr, out.buf.ptr, None))
+        got.append([out.to_vec()] + [c.dequantize().to_vec() for c in (kc, vc)])
+    for a, b in zip(*got):
+        assert np.array_equal(bits(a), bits(b))
+    for r, own in zip(rows, (raw[0, nh * hd:nh * hd + width], raw[0, nh * hd + width:])):
+        r[n - 1] = own
+    want = D.decode_attention(raw[0, :nh * hd], *(K.roundtrip(r, n, width, fmt) for r in rows), nh, nkv, 0, 0.0).reshape(-1)
+    assert np.abs(got[1][0] - want).max() <= 1e-5 * np.abs(want).max()
 
 
 def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
