@@ -1279,7 +1279,7 @@ struct ResidentParams {
     const uint16_t* Xp;   // prepared activations: [nchunks][16 NT][XR] f16
     const float* X;       // or the rows as they are, [T, K]
     float* Y;             // [T, N], or [parts][T, N] partial sums
-    int part0, add;       // the range of K that blockIdx.x == 0 does; add: to what is in Y
+    int part0;            // ADD: the range of K
     int T, N, K, nblk, chunks_each, chunks_over, tiles_each, tiles_over, xp_sets;   // xp_sets: sets of eight activation rows in Xp
     size_t row_bytes;
 };
@@ -1288,7 +1288,8 @@ constexpr int RES_WAVES = 16;
 template <class F, int NT>
 constexpr int resident_chunks() { return (163840 - RES_WAVES * 16 * F::LROW) / (16 * NT * XR * 2); }
 
-template <class F, int NT, bool OWN_X>
+// ADD: one range of K, added to what is in Y (asked in the store of every launch, 12288 x 4608 Q4_K at 24 rows took 26.3 us in place of 25.5)
+template <class F, int NT, bool OWN_X, bool ADD = false>
 __global__ void __launch_bounds__(64 * RES_WAVES, RES_WAVES / 4) gemm_q_f16x2_resident_kernel(ResidentParams p) {
     constexpr int MAXC = resident_chunks<F, NT>(), WP = 16 * F::PARTS, NW = (WP + 63) / 64, NTL = (16 * F::TAILS + 63) / 64, WV = RES_WAVES;
     static_assert(16 * F::LROW >= 512 * NT, "a wave's share of a tile's sums fits its image");
@@ -1297,7 +1298,7 @@ __global__ void __launch_bounds__(64 * RES_WAVES, RES_WAVES / 4) gemm_q_f16x2_re
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g4 = lane >> 4, c = lane & 15;
     uint8_t* const wl = Wl[wave];
-    const int part = p.part0 + blockIdx.x, j = blockIdx.y;      // the workgroup's chunks and tiles, shared out to within one
+    const int part = ADD ? p.part0 : blockIdx.x, j = blockIdx.y;   // the workgroup's chunks and tiles, shared out to within one
     const int c0 = part * p.chunks_each + (part < p.chunks_over ? part : p.chunks_over), cp = p.chunks_each + (part < p.chunks_over);
     const int tile0 = j * p.tiles_each + (j < p.tiles_over ? j : p.tiles_over), units = (p.tiles_each + (j < p.tiles_over)) * cp;
     auto run_of = [&](int w) { return (int)((uint32_t)(w * units) / WV); };
@@ -1386,7 +1387,7 @@ __global__ void __launch_bounds__(64 * RES_WAVES, RES_WAVES / 4) gemm_q_f16x2_re
     }
     __syncthreads();
 
-    float* const Y = p.Y + ((size_t)blockIdx.x * p.T + t0) * p.N;
+    float* const Y = p.Y + ((size_t)(ADD ? 0 : part) * p.T + t0) * p.N;
     // what a lane holds of a tile's outputs: rows 8 q + 4 (g4 & 1) + 2 h + (g4 >> 1), column c
     auto store = [&](int tl, const float (&v)[NT][2]) {
         const int n = row0_of(tl) + c;
@@ -1397,7 +1398,7 @@ __global__ void __launch_bounds__(64 * RES_WAVES, RES_WAVES / 4) gemm_q_f16x2_re
                 const int t = 8 * q + 4 * (g4 & 1) + 2 * h + (g4 >> 1);
                 if (t < T && n < p.N && n >= (tile0 + tl) * 16) {
                     float* const y = Y + (size_t)t * p.N + n;
-                    *y = p.add ? *y + v[q][h] : v[q][h];
+                    *y = ADD ? *y + v[q][h] : v[q][h];
                 }
             }
     };
@@ -1698,18 +1699,19 @@ int launch_resident_fmt(const fhip_weight* w, const uint16_t* d_xp, const float*
     const int tiles = (int)((w->rows + 15) / 16), nchunks = (int)((w->cols + CHUNK - 1) / CHUNK);
     p.chunks_each = nchunks / q.parts; p.chunks_over = nchunks % q.parts; p.tiles_each = tiles / q.per_part; p.tiles_over = tiles % q.per_part;
     const bool in_turn = q.parts > 1 && !d_part;     // the ranges one after the other, each added to y: the order and the bits of the sum of partial outputs
-    p.part0 = p.add = 0;
+    p.part0 = 0;
     if (in_turn) p.Y = d_y;
-    auto go = [&](auto kernel) {
-        for (; p.part0 < (in_turn ? q.parts : 1); p.add = ++p.part0)
-            hipLaunchKernelGGL(kernel, dim3(in_turn ? 1u : (unsigned)q.parts, (unsigned)q.per_part, (unsigned)q.sets), dim3(64 * RES_WAVES), 0, s, p);
-    };
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(in_turn ? 1u : (unsigned)q.parts, (unsigned)q.per_part, (unsigned)q.sets), dim3(64 * RES_WAVES), 0, s, p); };
     if (q.nt == 1) {
         if (d_xp) go(gemm_q_f16x2_resident_kernel<F, 1, false>);
         else go(gemm_q_f16x2_resident_kernel<F, 1, true>);
     } else {
         if (d_xp) go(gemm_q_f16x2_resident_kernel<F, 2, false>);
         else go(gemm_q_f16x2_resident_kernel<F, 2, true>);
+    }
+    for (p.part0 = 1; in_turn && p.part0 < q.parts; p.part0++) {
+        if (q.nt == 1) go(gemm_q_f16x2_resident_kernel<F, 1, true, true>);
+        else go(gemm_q_f16x2_resident_kernel<F, 2, true, true>);
     }
     const size_t n = t * w->rows;
     if (deferred) *deferred = fhip::F16Parts{d_part, q.parts > 1 ? q.parts : 0, n, w->rows};
