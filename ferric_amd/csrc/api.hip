@@ -248,10 +248,9 @@ static int gemm_bf16_lib_ws(const fhip_weight* w, const uint16_t* d_x, size_t t,
 
 size_t f16x2_group(const fhip_weight* w) { return w->type == FHIP_Q8_0 && w->batch_policy != FHIP_BATCH_ORDERED ? 16 : 32; }
 // Three and four rows of a Q4_K / Q5_K / Q6_K weight whose rows the four-row mat-vec (gemv_quad.hip) covers in one pass (up to 10240
-// columns) take that kernel under every policy: one launch, no workspace, the bits of a batch of one, and faster than the f16
-// kernels with their split and sum launches (cold, ordered sums: 5120 x 5120 17.7 -> 12.5 us, 7168 x 5120 19.9 -> 14.1, Q6_K
-// 151936 x 5120 178 -> 164; with atomic sums 12.6 / 14.5 / 178). Longer rows take two passes and lose (5120 x 17408: 36.6 against
-// 43.8), so they stay on the f16 kernels.
+// columns) take that kernel under every policy: one launch, no workspace, and the bits of a batch of one, which callers are promised. The f16 kernels are the faster
+// ones where sums are in order (4 rows, us, this kernel | held or resident: 1024 x 5120 Q4_K 10.9 | 7.1, 5120 x 5120 12.3 | 10.3, 34816 x 5120 29.5 | 26.2, Q6_K 151936 x 5120
+// 162 | 136); with atomic sums they were level (12.5 | 12.6, 7168 x 5120 14.1 | 14.5, the last 164 | 178). Longer rows take two passes (5120 x 17408 43.8 | 18.4) and stay on the f16 kernels.
 bool matmul_takes_quad(const fhip_weight* w, size_t t) {
     if (t < 3 || t > 4 || w->cols > 10240) return false;      // (Q8_0: 5120, gemv_quad_supports)
     return w->planes == 3 ? fhip::gemv_quad_supports_p3(w, t, 0) : fhip::gemv_quad_supports_p2(w, t, 0);
@@ -264,9 +263,9 @@ bool takes_f16x2(const fhip_weight* w, size_t rows_x) {
     return fhip::gemm_f16x2_takes(w, rows_x < f16x2_group(w) ? rows_x : f16x2_group(w));
 }
 
-// Fused gate|up + SwiGLU at three or four rows: one pass of the int8 matrix-instruction mat-vec (gemv_quad.hip, 31 us on
-// 34816 x 5120) is faster than the one-pass f16 kernel plus the SwiGLU launch behind it (34 + 4), and its rows carry the bits
-// they have in a batch of one. The plain matmuls of such batches stay on the f16 kernels (down 5120 x 17408: 27 us against 42).
+// Fused gate|up + SwiGLU at three or four rows: one pass of the int8 matrix-instruction mat-vec (gemv_quad.hip, 32 us on
+// 34816 x 5120), whose rows carry the bits they have in a batch of one; the f16 kernel and the SwiGLU launch behind it take 24 + 4
+// with sums in order, 31 + 5 by atomics. The down projection of such batches stays on the f16 kernels (5120 x 17408: 21 us against 43).
 bool swiglu_takes_quad(const fhip_weight* gu, size_t t) {
     if (t < 3 || t > 4 || gu->rows % 2 != 0 || gu->cols > 10240) return false;   // (one pass of the kernel, as matmul_takes_quad)
     return gu->planes == 3 ? fhip::gemv_quad_supports_p3(gu, t, gu->rows / 2) : fhip::gemv_quad_supports_p2(gu, t, gu->rows / 2);

@@ -454,8 +454,8 @@ int fhip_ffn_noalloc(const fhip_weight* gate_up, const fhip_weight* down, const 
  * FHIP_BATCH_ORDERED (what a new handle starts with): the one-pass matrix-core kernels described at fhip_matmul_q; where a
  * launch cuts a weight row's columns between workgroups the pieces go to the library workspace (fhip_workspace_bytes counts
  * them) and one more launch adds them in a fixed order, so the same call on the same inputs returns the same bits on every run.
- * FHIP_BATCH_AUTO: the same kernels with the pieces added by f32 atomics instead: a few microseconds per matmul faster, the
- * last bits vary from run to run (within 2e-6 of the largest output).
+ * FHIP_BATCH_AUTO: kernels that add the pieces by f32 atomics instead: less workspace, slower from five rows on (the feed-forward block of
+ * 5120 x 17408 at 8 rows 61.5 us against 51.9), and the last bits vary from run to run (within 2e-6 of the largest output).
  * FHIP_BATCH_F32_MATVEC: the streaming mat-vec's arithmetic for every row; an output row then has the same bits whatever
  * batch it was part of (the guarantee the reference's CPU path gives, crates/ferric-tensor/src/cpu_simd.rs:175-200), at the
  * price of one pass over the weights per four rows (Q4_K, Q5_K, Q6_K: the products of four rows at a time go through the 4 x 4 x 4 int8 matrix
