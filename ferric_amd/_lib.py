@@ -109,6 +109,8 @@ SYMBOLS = {
     "fhip_qkv_post_packed": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, C.c_int, C.c_float, C.c_float, _vp, _vp, _vp, _vp]),
     "fhip_qkv_post_kvq": (C.c_int, [C.c_int, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, C.c_int, C.c_float, C.c_float, _vp, _vp, _vp, _vp, _vp,
                                     _sz, _vp]),
+    "fhip_qkv_post_kvq_rows": (C.c_int, [C.c_int, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, C.c_int, C.c_float, C.c_float, _vp, _vp, _vp, _vp, _vp,
+                                         _sz, _vp, _vp, _sz, _sz, _vp]),
     "fhip_kvq_dequantize_rows": (C.c_int, [C.c_int, _vp, _vp, _sz, _sz, _sz, _vp, _vp, _vp]),
     "fhip_geglu": (C.c_int, [_vp, _sz, _sz, _vp, _vp]),
     "fhip_rope": (C.c_int, [_vp, _sz, _sz, _sz, _sz, _sz, C.c_float, _vp, _u32, _vp, C.c_int, _vp, _vp]),

@@ -1011,21 +1011,37 @@ int fhip_kvq_append2(int fmt, const float* d_k, const float* d_v, size_t src_row
                                    (hipStream_t)stream, d_v, d_v_codes, (uint16_t*)d_v_scales);
 }
 
+static int qkv_post_kvq(const char* who, int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
+                        const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps, float base, float* d_q_out,
+                        uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap, float* d_k_rows, float* d_v_rows, size_t n_rows,
+                        size_t past, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if ((rc = kvq_checks(who, fmt, n_kv * head_dim)) || (rc = rope_checks(who, n_head + 2 * n_kv, head_dim, n_rot))) return rc;
+    if (t == 0 || head_dim == 0 || n_head + n_kv == 0) return FHIP_OK;
+    if (!fhip::qkv_post_kvq_takes((int)head_dim)) return set_error(FHIP_ERR_SHAPE, "%s: head_dim must be a multiple of 32 up to 256, got %zu", who, head_dim);
+    if (!d_qkv || !d_positions || !d_q_out || !d_k_codes || !d_k_scales || !d_v_codes || !d_v_scales) return set_error(FHIP_ERR_ARG, "%s: NULL pointer", who);
+    if (cap > 0xFFFFFFFFull) return set_error(FHIP_ERR_SHAPE, "%s: too large for one launch", who);
+    return fhip::launch_qkv_post_kvq(fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_positions, d_freq_scale, t, (int)n_head, (int)n_kv, (int)head_dim, (int)n_rot,
+                                     interleaved != 0, eps, base, d_q_out, d_k_codes, (uint16_t*)d_k_scales, d_v_codes, (uint16_t*)d_v_scales, cap,
+                                     (hipStream_t)stream, d_k_rows, d_v_rows, n_rows, past);
+}
 int fhip_qkv_post_kvq(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
                       const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
                       float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
                       void* stream) {
-    int rc = need_init();
-    if (rc) return rc;
-    if ((rc = kvq_checks("fhip_qkv_post_kvq", fmt, n_kv * head_dim)) || (rc = rope_checks("fhip_qkv_post_kvq", n_head + 2 * n_kv, head_dim, n_rot))) return rc;
-    if (t == 0 || head_dim == 0 || n_head + n_kv == 0) return FHIP_OK;
-    if (!fhip::qkv_post_kvq_takes((int)head_dim)) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_kvq: head_dim must be a multiple of 32 up to 256, got %zu", head_dim);
-    if (!d_qkv || !d_positions || !d_q_out || !d_k_codes || !d_k_scales || !d_v_codes || !d_v_scales)
-        return set_error(FHIP_ERR_ARG, "fhip_qkv_post_kvq: NULL pointer");
-    if (cap > 0xFFFFFFFFull) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_kvq: too large for one launch");
-    return fhip::launch_qkv_post_kvq(fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_positions, d_freq_scale, t, (int)n_head, (int)n_kv, (int)head_dim, (int)n_rot,
-                                     interleaved != 0, eps, base, d_q_out, d_k_codes, (uint16_t*)d_k_scales, d_v_codes, (uint16_t*)d_v_scales, cap,
-                                     (hipStream_t)stream);
+    return qkv_post_kvq("fhip_qkv_post_kvq", fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_positions, d_freq_scale, t, n_head, n_kv, head_dim, n_rot, interleaved, eps, base, d_q_out,
+                        d_k_codes, d_k_scales, d_v_codes, d_v_scales, cap, nullptr, nullptr, 0, 0, stream);
+}
+int fhip_qkv_post_kvq_rows(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
+                           const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                           float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
+                           float* d_k_rows, float* d_v_rows, size_t n_rows, size_t past, void* stream) {
+    if (!d_k_rows || !d_v_rows || (((uintptr_t)d_k_rows | (uintptr_t)d_v_rows) & 15) != 0)
+        return set_error(FHIP_ERR_ARG, "fhip_qkv_post_kvq_rows: the rows' outputs must be there and 16-byte aligned");
+    if (past > n_rows || n_rows > cap) return set_error(FHIP_ERR_SHAPE, "fhip_qkv_post_kvq_rows: %zu earlier rows of %zu, a cache of %zu", past, n_rows, cap);
+    return qkv_post_kvq("fhip_qkv_post_kvq_rows", fmt, d_qkv, d_bias, d_q_norm, d_k_norm, d_positions, d_freq_scale, t, n_head, n_kv, head_dim, n_rot, interleaved, eps, base,
+                        d_q_out, d_k_codes, d_k_scales, d_v_codes, d_v_scales, cap, d_k_rows, d_v_rows, n_rows, past, stream);
 }
 
 int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_codes, const uint32_t* d_k_scales, const uint32_t* d_v_codes,

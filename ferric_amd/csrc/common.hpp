@@ -167,7 +167,8 @@ int launch_qkv_post(const float* qkv, const float* bias, const float* q_norm, co
 bool qkv_post_kvq_takes(int hd);
 int launch_qkv_post_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos,
                         const float* freq_scale, size_t t, int n_head, int n_kv, int hd, int n_rot, int interleaved, float eps, float base, float* q_out,
-                        uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes, uint16_t* v_scales, size_t cap, hipStream_t s);
+                        uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes, uint16_t* v_scales, size_t cap, hipStream_t s, float* k_rows = nullptr,
+                        float* v_rows = nullptr, size_t n_rows = 0, size_t past = 0);   // with k_rows, v_rows [n_rows, n_kv * hd]: what the blocks of these tokens and of rows 0 .. past - 1 stand for
 int launch_kv_append(const float* k, const float* v, size_t t, size_t width, const uint32_t* d_pos, uint32_t pos_off, size_t cap, float* kc,
                      float* vc, hipStream_t s);
 int attn_ws_splits(size_t len, int n_head, int n_kv, int hd);

@@ -12,6 +12,7 @@
 #include "common.hpp"
 
 #include <type_traits>
+#include "kvblock.hpp"
 #include "prompt.hpp"
 
 #include <hip/hip_fp16.h>
@@ -327,9 +328,9 @@ __device__ __forceinline__ uint16_t kv_f16_bits(float x) {   // a NaN keeps its 
     return __half_as_ushort(__float2half_rn(x));
 }
 __device__ __forceinline__ int kv_code(float r, float lo, float hi) { return r != r ? 0 : (int)fminf(fmaxf(r, lo), hi); }
-// lane j of a half wave holds value j of block b (live: the same for the whole half)
+// lane j of a half wave holds value j of block b (live: the same for the whole half); what its code stands for
 template <int FMT>
-__device__ __forceinline__ void quantize_lanes(float v, int j, bool live, uint32_t* __restrict__ codes, uint16_t* __restrict__ scales, size_t b) {
+__device__ __forceinline__ float quantize_lanes(float v, int j, bool live, uint32_t* __restrict__ codes, uint16_t* __restrict__ scales, size_t b) {
 #pragma clang fp contract(off)
     if constexpr (FMT == FHIP_KVQ_Q8_0) {
         const float amax = half32_max(fmaxf(0.f, fabsf(v)));
@@ -337,10 +338,13 @@ __device__ __forceinline__ void quantize_lanes(float v, int j, bool live, uint32
         const float inv = d > 0.f ? 1.0f / d : 0.f;
         const float t = v * inv;
         const float r = copysignf(floorf(fabsf(t) + 0.5f), t);
+        const int c = kv_code(r, -127.0f, 127.0f);
+        const uint16_t dbits = kv_f16_bits(d);
         if (live) {
-            ((uint8_t*)codes)[b * 32 + j] = (uint8_t)kv_code(r, -127.0f, 127.0f);
-            if (j == 0) scales[b] = kv_f16_bits(d);
+            ((uint8_t*)codes)[b * 32 + j] = (uint8_t)c;
+            if (j == 0) scales[b] = dbits;
         }
+        return fhip::kvq_value<FMT>(c, fhip::kvq_scale(dbits), 0.f);
     } else {
         float d, q;
         uint16_t mbits = 0;
@@ -365,21 +369,44 @@ __device__ __forceinline__ void quantize_lanes(float v, int j, bool live, uint32
             mbits = kv_f16_bits(mn);
         }
         const int c = kv_code(q, 0.f, 15.f), c2 = __shfl_xor(c, 16);
+        const uint16_t dbits = kv_f16_bits(d);
         if (live) {
             if (j < 16) ((uint8_t*)codes)[b * 16 + j] = (uint8_t)(c | (c2 << 4));
             if (j == 0) {
-                if constexpr (FMT == FHIP_KVQ_Q4_0) scales[b] = kv_f16_bits(d);
-                else { scales[2 * b] = kv_f16_bits(d); scales[2 * b + 1] = mbits; }
+                if constexpr (FMT == FHIP_KVQ_Q4_0) scales[b] = dbits;
+                else { scales[2 * b] = dbits; scales[2 * b + 1] = mbits; }
             }
         }
+        return fhip::kvq_value<FMT>(c, fhip::kvq_scale(dbits), fhip::kvq_scale(mbits));
     }
 }
 struct KvqStore {
     uint32_t* k_codes; uint16_t* k_scales;
     uint32_t* v_codes; uint16_t* v_scales;
 };
+// The f32 rows that the stored blocks stand for, for an attention that reads those: a token's at its position, and rows 0 .. past - 1 of the caches, which
+// `past_wgs` workgroups behind the others bring.
+struct KvqRows {
+    float *k, *v;            // [n, n_kv * hd]: a token whose position is n or more leaves no row
+    uint32_t n, past;
+    unsigned post_wgs;       // workgroups in front of those
+};
 template <int FMT>
-__global__ __launch_bounds__(256) void qkv_post_kvq_kernel(QkvPostParams p, KvqStore st) {
+__device__ __forceinline__ void past_rows(const KvqStore& st, const KvqRows& rows, int width) {
+    const size_t w4 = width / 4, all = rows.past * w4;
+    size_t id = (size_t)(blockIdx.x - rows.post_wgs) * 256 + threadIdx.x;
+    const bool value = id >= all;
+    id -= value ? all : 0;
+    if (id >= all) return;
+    const size_t i = id / w4;
+    const int col = (int)(id - i * w4) * 4;
+    const size_t b = i * (size_t)(width / 32) + col / 32;
+    const float4 o = value ? fhip::kvq_values4<FMT>(st.v_codes, st.v_scales, b, col % 32) : fhip::kvq_values4<FMT>(st.k_codes, st.k_scales, b, col % 32);
+    *(float4*)((value ? rows.v : rows.k) + 4 * id) = o;
+}
+template <int FMT, bool ROWS>
+__global__ __launch_bounds__(256) void qkv_post_kvq_kernel(QkvPostParams p, KvqStore st, KvqRows out) {
+    if (ROWS && blockIdx.x >= out.post_wgs) { past_rows<FMT>(st, out, p.n_kv * p.hd); return; }
     constexpr int EPL = POST_KVQ_HD / 64;
     __shared__ float rows[4][2][POST_KVQ_HD];                    // a wave's head: normed, then rotated
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -440,7 +467,82 @@ __global__ __launch_bounds__(256) void qkv_post_kvq_kernel(QkvPostParams p, KvqS
     for (int e = 0; e < p.hd; e += 64) {                         // uniform: both halves of the wave take part in the exchanges
         const int j = e + lane;
         const bool live = j < p.hd;
-        quantize_lanes<FMT>(live ? src[j] : 0.f, lane & 31, live, is_k ? st.k_codes : st.v_codes, is_k ? st.k_scales : st.v_scales, b0 + (size_t)(j >> 5));
+        const float stored = quantize_lanes<FMT>(live ? src[j] : 0.f, lane & 31, live, is_k ? st.k_codes : st.v_codes, is_k ? st.k_scales : st.v_scales, b0 + (size_t)(j >> 5));
+        if (ROWS && live && pos < out.n) (is_k ? out.k : out.v)[((size_t)pos * p.n_kv + head) * p.hd + j] = stored;
+    }
+}
+
+// The same with the rows for heads of 64 or 128 dims rotated whole in the split-half layout, in registers: HD = 128 as qkv_post128_kernel holds a head (a lane's two
+// values are a pair), HD = 64 a value a lane, its pair's other one 32 lanes away. A wave takes HPW consecutive heads of a token. A prompt's layer on a quantized
+// cache was four launches here (post-processing, stores, both caches' rows), 3 - 4 us each; stacks of 42 ... 191 rows, us: 42 x 3584, one layer behind 581 rows 209 -> 195,
+// 86 x 3072 298 -> 281, 93 x 1280, four layers 460 -> 424, 139 x 2560, three 565 -> 543; 937 x 4608, four layers, 3081 -> 3071.
+template <int FMT, int HD, int HPW>
+__global__ __launch_bounds__(256) void qkv_post_rows_kernel(QkvPostParams p, KvqStore st, KvqRows out) {
+    constexpr int E = HD / 64;
+    if (blockIdx.x >= out.post_wgs) { past_rows<FMT>(st, out, p.n_kv * HD); return; }
+    const int lane = threadIdx.x & 63;
+    const int per_tok = p.n_head + 2 * p.n_kv, waves_per_tok = (per_tok + HPW - 1) / HPW;
+    const size_t wid = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wid >= (size_t)p.t * waves_per_tok) return;
+    const int i = (int)(wid / waves_per_tok), h0 = (int)(wid % waves_per_tok) * HPW;
+    const float* x = p.qkv + ((size_t)i * per_tok + h0) * HD + lane;
+    float a[HPW][E];
+#pragma unroll
+    for (int j = 0; j < HPW; j++)
+#pragma unroll
+        for (int e = 0; e < E; e++) a[j][e] = x[(h0 + j < per_tok ? HD * j : 0) + 64 * e];
+    const uint32_t pos = p.pos[i];
+    float wq[E], wk[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        wq[e] = p.q_norm ? p.q_norm[lane + 64 * e] : 1.f;
+        wk[e] = p.k_norm ? p.k_norm[lane + 64 * e] : 1.f;
+    }
+    if (p.bias) {
+        const float* bias = p.bias + (size_t)h0 * HD + lane;
+#pragma unroll
+        for (int j = 0; j < HPW; j++)
+#pragma unroll
+            for (int e = 0; e < E; e++) a[j][e] += bias[(h0 + j < per_tok ? HD * j : 0) + 64 * e];
+    }
+    float sn = 0.f, cs = 1.f;
+    if (h0 < p.n_head + p.n_kv) sincosf((float)pos * rope_inv_freq(lane & (HD / 2 - 1), p.rate, p.freq_scale), &sn, &cs);
+    const bool stored = pos < p.cap;                             // a position past the cache is dropped, never written out of bounds
+#pragma unroll
+    for (int j = 0; j < HPW; j++) {
+        const int h = h0 + j;
+        if (h >= per_tok || (h >= p.n_head && !stored)) return;  // (uniform: a wave has one token)
+        const bool value = h >= p.n_head + p.n_kv, key = !value && h >= p.n_head;
+        float v[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = a[j][e];
+        if (!value) {
+            if (key ? p.k_norm : p.q_norm) {
+                const float sq = fmaf(v[E - 1], v[E - 1], E == 2 ? v[0] * v[0] : 0.f);   // (a plain product would be fused with the sum's first addition)
+                const float inv = 1.0f / sqrtf(wave_sum(sq) / (float)HD + p.eps);
+#pragma unroll
+                for (int e = 0; e < E; e++) v[e] = v[e] * inv * (key ? wk[e] : wq[e]);
+            }
+            if constexpr (E == 2) {
+                const float y1 = rot_lo(v[0], v[1], cs, sn), y2 = rot_hi(v[0], v[1], cs, sn);
+                v[0] = y1;
+                v[1] = y2;
+            } else {
+                const float other = __shfl_xor(v[0], 32);
+                v[0] = lane < 32 ? rot_lo(v[0], other, cs, sn) : rot_hi(other, v[0], cs, sn);
+            }
+        }
+        if (h < p.n_head) {
+#pragma unroll
+            for (int e = 0; e < E; e++) p.q_out[((size_t)i * p.n_head + h) * HD + lane + 64 * e] = v[e];
+            continue;
+        }
+        const size_t at = (size_t)pos * p.n_kv + (h - p.n_head - (value ? p.n_kv : 0));
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const float row = quantize_lanes<FMT>(v[e], lane & 31, true, value ? st.v_codes : st.k_codes, value ? st.v_scales : st.k_scales, at * (HD / 32) + 2 * e + (lane >> 5));
+            if (pos < out.n) (value ? out.v : out.k)[at * HD + lane + 64 * e] = row;
+        }
     }
 }
 
@@ -1534,25 +1636,40 @@ int launch_qkv_post(const float* qkv, const float* bias, const float* q_norm, co
 }
 
 bool qkv_post_kvq_takes(int hd) { return hd > 0 && hd % 32 == 0 && hd <= POST_KVQ_HD; }
+template <int FMT>
+static int post_kvq(const QkvPostParams& p, const KvqStore& st, KvqRows rows, hipStream_t s) {
+    const size_t t = p.t, per_tok = (size_t)(p.n_head + 2 * p.n_kv), past = rows.past * ((size_t)p.n_kv * p.hd / 4) * 2, past_wgs = (past + 255) / 256;
+    const bool whole = rows.k && (p.hd == 64 || p.hd == 128) && p.n_rot == p.hd && !p.interleaved;
+    // heads a wave: as in launch_qkv_post
+    const size_t hpw = whole && t * ((per_tok + 7) / 8) >= 4 * (size_t)device_cus() ? 8 : 1, grid = (t * ((per_tok + hpw - 1) / hpw) + 3) / 4;
+    if (t * per_tok > 0x7FFFFFFFull || grid + past_wgs > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post_kvq: too many rows for one launch");
+    rows.post_wgs = (unsigned)grid;
+    const dim3 g((unsigned)(grid + past_wgs)), wg(256);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, wg, 0, s, p, st, rows); };
+    if (!rows.k) go(qkv_post_kvq_kernel<FMT, false>);
+    else if (!whole) go(qkv_post_kvq_kernel<FMT, true>);
+    else if (p.hd == 128) hpw == 8 ? go(qkv_post_rows_kernel<FMT, 128, 8>) : go(qkv_post_rows_kernel<FMT, 128, 1>);
+    else hpw == 8 ? go(qkv_post_rows_kernel<FMT, 64, 8>) : go(qkv_post_rows_kernel<FMT, 64, 1>);
+    return check_hip(hipGetLastError(), "qkv_post_kvq launch");
+}
 int launch_qkv_post_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos,
                         const float* freq_scale, size_t t, int n_head, int n_kv, int hd, int n_rot, int interleaved, float eps, float base, float* q_out,
-                        uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes, uint16_t* v_scales, size_t cap, hipStream_t s) {
+                        uint32_t* k_codes, uint16_t* k_scales, uint32_t* v_codes, uint16_t* v_scales, size_t cap, hipStream_t s, float* k_rows, float* v_rows, size_t n_rows, size_t past) {
     if (t == 0) return FHIP_OK;
-    const size_t per_tok = (size_t)(n_head + 2 * n_kv), grid = (t * per_tok + 3) / 4;
-    if (t > 0x7FFFFFFFull || grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post_kvq: too many rows for one launch");
+    if (t > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post_kvq: too many rows for one launch");
     QkvPostParams p;
     p.qkv = qkv; p.bias = bias; p.q_norm = q_norm; p.k_norm = k_norm; p.pos = d_pos; p.freq_scale = freq_scale;
     p.q_out = q_out; p.k_cache = nullptr; p.v_cache = nullptr;
     p.t = (int)t; p.n_head = n_head; p.n_kv = n_kv; p.hd = hd; p.n_rot = n_rot; p.interleaved = interleaved;
     p.cap = (uint32_t)cap; p.eps = eps; p.rate = rope_rate(n_rot, base); p.kv_packed = 0;
     const KvqStore st{k_codes, k_scales, v_codes, v_scales};
+    const KvqRows rows{k_rows, v_rows, (uint32_t)n_rows, (uint32_t)past, 0u};
     switch (fmt) {
-        case FHIP_KVQ_Q8_0: hipLaunchKernelGGL(qkv_post_kvq_kernel<FHIP_KVQ_Q8_0>, dim3((unsigned)grid), dim3(256), 0, s, p, st); break;
-        case FHIP_KVQ_Q4_0: hipLaunchKernelGGL(qkv_post_kvq_kernel<FHIP_KVQ_Q4_0>, dim3((unsigned)grid), dim3(256), 0, s, p, st); break;
-        case FHIP_KVQ_Q4_1: hipLaunchKernelGGL(qkv_post_kvq_kernel<FHIP_KVQ_Q4_1>, dim3((unsigned)grid), dim3(256), 0, s, p, st); break;
+        case FHIP_KVQ_Q8_0: return post_kvq<FHIP_KVQ_Q8_0>(p, st, rows, s);
+        case FHIP_KVQ_Q4_0: return post_kvq<FHIP_KVQ_Q4_0>(p, st, rows, s);
+        case FHIP_KVQ_Q4_1: return post_kvq<FHIP_KVQ_Q4_1>(p, st, rows, s);
         default: return set_error(FHIP_ERR_ARG, "qkv_post_kvq: unknown format %d", fmt);
     }
-    return check_hip(hipGetLastError(), "qkv_post_kvq launch");
 }
 
 int launch_kv_append(const float* k, const float* v, size_t t, size_t width, const uint32_t* d_pos, uint32_t pos_off, size_t cap, float* kc,

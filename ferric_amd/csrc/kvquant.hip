@@ -13,6 +13,7 @@
 // Every f32 operation is the reference's, one rounding each: this file is compiled with -ffp-contract=off (no fused
 // multiply-add where the reference multiplies and then adds), and divisions are IEEE divisions.
 #include "common.hpp"
+#include "kvblock.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -28,7 +29,6 @@ __device__ __forceinline__ uint16_t f16_bits(float x) {
         return (uint16_t)(((b >> 16) & 0x8000u) | 0x7C00u | 0x0200u | ((b & 0x007FFFFFu) >> 13));
     return __half_as_ushort(__float2half_rn(x));
 }
-__device__ __forceinline__ float f16_val(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 
 // Rust's `x as i32` behind a clamp: NaN -> 0
 __device__ __forceinline__ int clamp_to_int(float r, float lo, float hi) { return r != r ? 0 : (int)fminf(fmaxf(r, lo), hi); }
@@ -143,27 +143,7 @@ __global__ __launch_bounds__(256) void kvq_dequant_kernel(const uint32_t* __rest
     const int col = (int)(id % w4) * 4;
     if (last_pos && row0 + i > (size_t)*last_pos) return;
     const size_t b = (row0 + i) * (size_t)(width / QK) + col / QK;
-    const int j = col % QK;
-    float4 o;
-    if constexpr (FMT == FHIP_KVQ_Q8_0) {
-        const float d = f16_val(scales[b]);
-        const uint32_t word = codes[b * 8 + j / 4];
-        o.x = (float)(int8_t)(word & 255u) * d;
-        o.y = (float)(int8_t)((word >> 8) & 255u) * d;
-        o.z = (float)(int8_t)((word >> 16) & 255u) * d;
-        o.w = (float)(int8_t)(word >> 24) * d;
-    } else {
-        const uint32_t word = codes[b * 4 + (j % 16) / 4] >> (j < 16 ? 0 : 4);
-        const float n0 = (float)(word & 15u), n1 = (float)((word >> 8) & 15u), n2 = (float)((word >> 16) & 15u), n3 = (float)((word >> 24) & 15u);
-        if constexpr (FMT == FHIP_KVQ_Q4_0) {
-            const float d = f16_val(scales[b]);
-            o.x = (n0 - 8.0f) * d; o.y = (n1 - 8.0f) * d; o.z = (n2 - 8.0f) * d; o.w = (n3 - 8.0f) * d;
-        } else {
-            const float d = f16_val(scales[2 * b]), m = f16_val(scales[2 * b + 1]);
-            o.x = n0 * d + m; o.y = n1 * d + m; o.z = n2 * d + m; o.w = n3 * d + m;
-        }
-    }
-    *(float4*)(out + i * (size_t)width + col) = o;
+    *(float4*)(out + i * (size_t)width + col) = fhip::kvq_values4<FMT>(codes, scales, b, col % QK);
 }
 
 }  // namespace

@@ -378,9 +378,8 @@ class Qwen3Decoder:
         f, gu = E((t, c.n_ff)), (E((t, 2 * c.n_ff)) if c.geglu or (self.kv_fmt is not None and not precise) else None)
         gate = E((t, self.q_out)) if self.gate is not None else None
         ws16 = DeviceBuffer(2 * t * max(c.d_model, self.q_out, c.n_ff) + 256)          # bf16 copies of the coop matmuls' inputs
-        k1 = v1 = kd = vd = None
+        kd = vd = None
         if self.kv_fmt is not None:
-            k1, v1 = E((t, self.kv_out)), E((t, self.kv_out))
             kd, vd = E((pos0 + t, self.kv_out)), E((pos0 + t, self.kv_out))          # what the stored blocks dequantize to
         wsf = [None]
         wsa = f.buf                                      # attention split along the keys: scratch that is not in use yet, or larger
@@ -435,13 +434,9 @@ class Qwen3Decoder:
                 kp, vp = kv.k.buf.ptr, kv.v.buf.ptr
             else:
                 kq, vq = kv
-                _check(lib.fhip_qkv_post_packed(qkv.buf.ptr, bias, qn, kn, positions.buf.ptr, None, t, c.n_head, c.n_head_kv, c.head_dim, n_rot,
-                                                int(c.rope_interleaved), c.eps, base, q.buf.ptr, k1.buf.ptr, v1.buf.ptr, s))
-                _check(lib.fhip_kvq_append2(self.kv_fmt, k1.buf.ptr, v1.buf.ptr, 0, t, self.kv_out, positions.buf.ptr, 0, kq.cap, kq.codes.ptr,
-                                            kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, s))
-                for cache, dst in ((kq, kd), (vq, vd)):
-                    _check(lib.fhip_kvq_dequantize_rows(self.kv_fmt, cache.codes.ptr, cache.scales.ptr, 0, pos0 + t, self.kv_out, None,
-                                                        dst.buf.ptr, s))
+                _check(lib.fhip_qkv_post_kvq_rows(self.kv_fmt, qkv.buf.ptr, bias, qn, kn, positions.buf.ptr, None, t, c.n_head, c.n_head_kv, c.head_dim, n_rot,
+                                                  int(c.rope_interleaved), c.eps, base, q.buf.ptr, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, kq.cap,
+                                                  kd.buf.ptr, vd.buf.ptr, pos0 + t, pos0, s))
                 kp, vp = kd.buf.ptr, vd.buf.ptr
             shape = (q.buf.ptr, kp, vp, t, pos0 + t, c.n_head, c.n_head_kv, c.head_dim, l.window, c.attn_softcap)
             if self.kv_fmt is not None:

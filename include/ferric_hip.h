@@ -395,6 +395,13 @@ int fhip_qkv_post_kvq(int fmt, const float* d_qkv, const float* d_bias, const fl
                       const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
                       float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
                       void* stream);
+/* The same, and what the blocks dequantize to for an attention over f32 rows (fhip_kvq_dequantize_rows' bits): d_k_rows, d_v_rows [n_rows, n_kv *
+ * head_dim], 16-byte aligned, n_rows <= cap, get row d_positions[i] of token i (a position of n_rows and more leaves none) and rows 0 .. past - 1 as the
+ * caches hold them, which no position may name. t = 0: nothing is done. */
+int fhip_qkv_post_kvq_rows(int fmt, const float* d_qkv, const float* d_bias, const float* d_q_norm, const float* d_k_norm, const uint32_t* d_positions,
+                           const float* d_freq_scale, size_t t, size_t n_head, size_t n_kv, size_t head_dim, size_t n_rot, int interleaved, float eps,
+                           float base, float* d_q_out, uint32_t* d_k_codes, uint32_t* d_k_scales, uint32_t* d_v_codes, uint32_t* d_v_scales, size_t cap,
+                           float* d_k_rows, float* d_v_rows, size_t n_rows, size_t past, void* stream);
 
 /* crates/ferric-tensor/src/nn.rs:140 decode_attention -> lib.rs:762 fused_decode_attention (kernels :2675, :2740 ff.):
  * one query row q [n_head * head_dim] against the cache rows [0, len) of K and V [., n_kv * head_dim];

@@ -397,6 +397,57 @@ def test_post_processing_and_quantized_stores_in_one_launch(F, Q, fmt, nh, nkv, 
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("nh,nkv,hd,n_rot,inter,norms,t,past", [
+    # heads rotated whole, one a wave and eight (the last wave of a token with six, four, all); other rotations and head sizes
+    (10, 2, 128, 128, 0, True, 5, 0), (5, 1, 64, 64, 0, True, 7, 33), (10, 2, 128, 128, 0, True, 600, 3), (8, 2, 64, 64, 0, False, 700, 130), (4, 2, 64, 64, 0, True, 1100, 0),
+    (4, 4, 64, 64, 1, True, 5, 9), (6, 3, 32, 16, 0, False, 41, 1), (2, 1, 96, 96, 0, True, 3, 3), (8, 2, 128, 0, 0, True, 4, 1)])
+def test_post_processing_stores_and_rows_in_one_launch(F, Q, fmt, nh, nkv, hd, n_rot, inter, norms, t, past):
+    """fhip_qkv_post_kvq_rows against fhip_qkv_post_packed, fhip_kvq_append2 and fhip_kvq_dequantize_rows of both caches: the same bits everywhere, over blocks of zeros
+    of both signs, equal magnitudes, NaN and infinities; a position past the rows' outputs is stored and leaves no row, one past the cache neither."""
+    rng = np.random.default_rng(nh * hd + fmt)
+    lib, width = F._lib.load(), nkv * hd
+    n, cap = past + t - 1, past + t + 2
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    qkv = (rng.standard_normal((t, (nh + 2 * nkv) * hd)) * 3).astype(np.float32)
+    v = qkv[:, (nh + nkv) * hd:]
+    v[0, :32] = np.where(np.arange(32) % 2, 0.0, -0.0)
+    v[1, :32] = np.where(np.arange(32) % 3, 2.5, -2.5)
+    v[2, 3], v[2, 20] = np.nan, np.inf
+    bias, qn, kn = (rng.standard_normal(m).astype(np.float32) for m in (qkv.shape[1], hd, hd))
+    bt, qnt, knt = (T(bias), T(qn), T(kn)) if norms else (None, None, None)
+    P = lambda x: x.buf.ptr if x is not None else None
+    where = past + rng.permutation(t).astype(np.uint32)
+    where[where == past + 1] = cap + 2
+    qt, pt = T(qkv), F.Tensor(F.DeviceBuffer(4 * t), (t,), np.uint32)
+    F._lib.check(lib.fhip_memcpy_h2d(pt.buf.ptr, where.ctypes.data, 4 * t, None))
+    old = [rng.standard_normal((cap, width)).astype(np.float32) for _ in range(2)]
+    got = []
+    for one in (True, False):
+        kq, vq = (Q.QKvCache.from_tensor(T(o), fmt) for o in old)
+        qo, rows = T(np.full((t, nh * hd), 7.0, np.float32)), [T(np.full((n, width), 7.0, np.float32)) for _ in range(2)]
+        if one:
+            F._lib.check(lib.fhip_qkv_post_kvq_rows(fmt, qt.buf.ptr, P(bt), P(qnt), P(knt), pt.buf.ptr, None, t, nh, nkv, hd, n_rot, inter, 1e-6, 1e6, qo.buf.ptr, kq.codes.ptr,
+                                                    kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, cap, rows[0].buf.ptr, rows[1].buf.ptr, n, past, None))
+        else:
+            k1, v1 = F.Tensor.empty((t, width)), F.Tensor.empty((t, width))
+            F._lib.check(lib.fhip_qkv_post_packed(qt.buf.ptr, P(bt), P(qnt), P(knt), pt.buf.ptr, None, t, nh, nkv, hd, n_rot, inter, 1e-6, 1e6, qo.buf.ptr, k1.buf.ptr,
+                                                  v1.buf.ptr, None))
+            F._lib.check(lib.fhip_kvq_append2(fmt, k1.buf.ptr, v1.buf.ptr, 0, t, width, pt.buf.ptr, 0, cap, kq.codes.ptr, kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, None))
+            for c, r in zip((kq, vq), rows):
+                F._lib.check(lib.fhip_kvq_dequantize_rows(fmt, c.codes.ptr, c.scales.ptr, 0, n, width, None, r.buf.ptr, None))
+        r = [bits(x.to_vec()).reshape(n, width) for x in rows]
+        if not one and past + 1 < n:
+            for x in r:
+                x[past + 1] = np.float32(7.0).view(np.uint32)    # the position that went past the cache
+        got.append([bits(qo.to_vec())] + [x.view(np.uint8) for c in (kq, vq) for x in c.to_host()] + r)
+    for name, a, b in zip(("q", "k codes", "k scales", "v codes", "v scales", "k rows", "v rows"), *got):
+        assert np.array_equal(a, b), (name, np.flatnonzero(a.reshape(-1) != b.reshape(-1))[:8])
+    call = lambda rows, n_rows, first: lib.fhip_qkv_post_kvq_rows(fmt, qt.buf.ptr, None, None, None, pt.buf.ptr, None, 1, nh, nkv, hd, n_rot, inter, 1e-6, 1e6, qo.buf.ptr, kq.codes.ptr,
+                                                                  kq.scales.ptr, vq.codes.ptr, vq.scales.ptr, cap, rows, rows, n_rows, first, None)
+    assert call(None, 1, 0) != 0 and call(rows[0].buf.ptr, cap + 1, 0) != 0 and call(rows[0].buf.ptr, 1, 2) != 0
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
 @pytest.mark.parametrize("nh,nkv,hd,cap,pos,norm,bias,inter,n_rot,window,cap_soft", [
     # one workgroup a query head: four waves, the first of sixteen, full, the last; a head of its own per KV head
     (10, 2, 128, 1, 0, True, False, False, 128, 0, 0.0), (8, 4, 64, 96, 95, True, True, False, 64, 0, 0.0), (8, 4, 64, 97, 64, False, False, True, 64, 0, 30.0),
