@@ -5,11 +5,13 @@
 // to fresh host memory 12.5 ms (a single thread taking page faults one by one). Here a copy goes through slots of pinned memory
 // that a small kernel on the caller's own stream reads or writes directly; the kernel's workgroups confirm in pinned words of
 // their own, which a host thread polls without a call into the runtime.
-//   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time)
+//   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time); an upload of 1.25 to 12 MB goes
+//                   through several, one filled while the one before crosses the bus
 //   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
 //                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise (one and a half into fresh memory); more is cut into chunks, each
 //                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
-//                   included, which is why there are several workers)
+//                   included, which is why there are several workers). While the stream has other work in front of the copy, the waiting thread makes the
+//                   destination's pages: into fresh memory behind 350 us of work, us, 608 KB 477 -> 379, 2 MB 810 -> 417, 10.4 MB 2420 -> 1800
 // The kernel's rate is the bus's: 84 MB in 1.6 ms (53 GB/s) from 64 workgroups on, where the DMA engines took 1.6 - 3.0 ms. A whole copy to the host reaches
 // 40 - 42 GB/s (16 MB in 396 us), the host's side included.
 // Nobody waits for another stream's work: a long copy takes the workers, which serve one at a time, once its own stream has got there, and who finds no slot
@@ -38,12 +40,14 @@ constexpr size_t OUT_BYTES = (size_t)1 << 20;    // a slot's part for data on it
 constexpr size_t IN_BYTES = fhip::H2D_STAGED;    // ... and to the device (a chunk of floats is at most 278 528 block bytes, Q8_0)
 constexpr size_t CHUNK = OUT_BYTES;              // of a long copy
 constexpr size_t SLOT_BYTES = OUT_BYTES + IN_BYTES;
-constexpr int SLOTS = 16, JOB_SLOTS = 12;        // a chunked copy takes up to JOB_SLOTS and leaves the others to small copies
+constexpr int SLOTS = 28, JOB_SLOTS = 12;        // a chunked copy takes up to JOB_SLOTS of the first SMALL_SLOTS and leaves the others to small copies; ...
+constexpr int SMALL_SLOTS = 16;                  // ... those behind are the chunked uploads', which hold them until their stream has got there
 constexpr int MAX_WG = 64, THREADS = 512;        // workgroups of a copy (each confirms its part in a word of its own)
 constexpr size_t IN_PARTS = (size_t)96 << 10;    // copies to the host from here on go in parts, the host copying one out while the next ones cross
 constexpr int PARTS = 8;                         // at most
 constexpr size_t D2H_ALONE = 3 * OUT_BYTES;      // longer copies to the host are the workers' ...
 constexpr size_t D2H_ALONE_NEW = D2H_ALONE / 2;  // ... and those from here on whose destination has pages that nobody has touched
+constexpr size_t IN_CHUNKS_FROM = (size_t)1280 << 10, IN_CHUNKS_TO = (SLOTS - SMALL_SLOTS) * OUT_BYTES;   // uploads that the calling thread takes in chunks
 constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
@@ -121,10 +125,35 @@ struct Slot {
     }
 };
 
-// Until the first n of the words hold `want`: polled for two milliseconds (a decode step), then left to the runtime.
-int await_words(const uint32_t* words, uint32_t want, int n, hipStream_t s) {
+// The pages of a destination, which a fresh allocation does not have until somebody writes to it, made a few at a time: by a thread that waits for the device
+// anyway, in place of the copy behind the wait (0.16 us a KB). step() is false when all are there, or the kernel has no such call (Linux before 5.14).
+class Pages {
+    uintptr_t at, end;
+    bool refused = false;
+
+public:
+    Pages(const void* h, size_t n) {
+        static const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
+        at = (uintptr_t)h / page * page;
+        end = ((uintptr_t)h + n + page - 1) / page * page;
+    }
+    bool step() {
+        constexpr int POPULATE_WRITE = 23;           // MADV_POPULATE_WRITE
+        constexpr uintptr_t STEP = (uintptr_t)64 << 10;
+        if (at >= end) return false;
+        const uintptr_t n = end - at < STEP ? end - at : STEP;
+        refused = madvise((void*)at, n, POPULATE_WRITE) != 0;
+        at = refused ? end : at + n;
+        return !refused;
+    }
+    bool made() const { return at >= end && !refused; }
+};
+
+// Until the first n of the words hold `want`: polled for two milliseconds (a decode step), then left to the runtime. `pages` are made meanwhile.
+int await_words(const uint32_t* words, uint32_t want, int n, hipStream_t s, Pages* pages = nullptr) {
     const auto start = std::chrono::steady_clock::now();
     for (unsigned i = 0; !Slot::confirmed(words, want, n); i++) {
+        if (pages && pages->step()) continue;
 #if defined(__x86_64__)
         __builtin_ia32_pause();
 #endif
@@ -144,10 +173,10 @@ struct Ring {                    // one per device
 
     // The lowest slot that neither the host holds nor the GPU still reads: low slots stay warm in the CPU's caches. A slot's
     // pinned memory is made when it is first taken. null: all are taken.
-    Slot* take(int* rc, int of = SLOTS) {
+    Slot* take(int* rc, int to = SMALL_SLOTS, int from = 0) {
         std::lock_guard<std::mutex> lock(mu);
         *rc = FHIP_OK;
-        for (int i = 0; i < of; i++) {
+        for (int i = from; i < to; i++) {
             Slot& q = slot[i];
             if (q.held || !q.read_by_gpu()) continue;
             if (!words) {
@@ -412,6 +441,32 @@ int may_wait(hipStream_t s, const char* who) {
 
 namespace fhip {
 
+// A source longer than a slot's IN_BYTES in chunks, by the calling thread, one crossing the bus while the next goes into its slot: the source has been read when this returns, while the
+// last chunks still cross. *took false: there were not enough slots at once, and nothing was done.
+// us on an idle device, the runtime's copy, which is waited for | this: returned 1.5 MB 66 | 29, 2.4 92 | 45, 3.3 118 | 62, 5.0 152 | 90, 10.4 350 | 285; arrived, with the wait's own
+// 10, 1.5 MB 71 | 65, 2.4 97 | 85, 3.3 123 | 107, 5.0 157 | 153, 10.4 355 | 320. Shorter ones arrive later this way (0.7 MB 37 | 42, 1.0 47 | 55) and stay with the runtime. Chunks of
+// 448 KB cost their launches: 3.3 MB returned 89, arrived 127.
+static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStream_t s, bool* took) {
+    const size_t count = (n + OUT_BYTES - 1) / OUT_BYTES, each = ((n + count - 1) / count + 255) & ~(size_t)255;
+    Slot* q[SLOTS - SMALL_SLOTS];
+    size_t have = 0;
+    int rc = FHIP_OK;
+    while (have < count && !rc) {
+        Slot* next = r->take(&rc, SLOTS, SMALL_SLOTS);
+        if (!next) break;
+        q[have++] = next;
+    }
+    *took = !rc && have == count;
+    for (size_t c = 0; c < count && *took && !rc; c++) {
+        int wgs = 0;
+        const size_t bytes = part(n, each, c);
+        memcpy(q[c]->host, h + c * each, bytes);
+        if (!(rc = launch_copy(q[c]->host, d + c * each, bytes, 4, q[c]->done, q[c]->seq + 1, s, &wgs))) { q[c]->seq++; q[c]->wgs = wgs; }
+    }
+    for (size_t i = 0; i < have; i++) r->release(q[i]);
+    return rc;
+}
+
 // Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime (10 MB in 285 us;
 // chunks of it copied into slots by workers and pulled over the bus by kernels took 300 - 360), and it returns when the source has
 // been read or is known to be pinned. A copy in a stream capture stays a copy node; on another stream than the captured one it goes
@@ -438,8 +493,15 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
 }
 
 int upload(void* d, const void* h, size_t n, hipStream_t s) {
-    if (int rc = may_wait(s, "fhip_upload")) return rc;
-    const int rc = copy_h2d(d, h, n, s);
+    int rc = may_wait(s, "fhip_upload");
+    if (rc) return rc;
+    if (n > IN_CHUNKS_FROM && n <= IN_CHUNKS_TO) {
+        bool kernels, took = false;
+        if ((rc = for_kernels(d, n, h, "fhip_upload", &kernels))) return rc;
+        Ring* r = kernels ? ring(&rc) : nullptr;
+        if (rc || (r && ((rc = upload_chunks(r, (uint8_t*)d, (const uint8_t*)h, n, s, &took)) || took))) return rc;
+    }
+    rc = copy_h2d(d, h, n, s);
     return rc || n <= IN_BYTES ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 
@@ -468,11 +530,11 @@ static int send_parts(Slot* q, const uint8_t* from, size_t n, hipStream_t s, Par
     *out = parts;
     return rc;
 }
-static int take_parts(Slot* q, uint8_t* h, const Parts<PARTS>& parts, hipStream_t s) {
+static int take_parts(Slot* q, uint8_t* h, const Parts<PARTS>& parts, hipStream_t s, Pages* pages = nullptr) {
     int rc = FHIP_OK;
     for (int p = 0; p < parts.count && !rc; p++) {
         const size_t begin = p ? parts.end[p - 1] : 0;
-        if (!(rc = await_words(parts.done[p], q->seq, q->wgs, s))) memcpy(h + begin, q->host + begin, parts.end[p] - begin);
+        if (!(rc = await_words(parts.done[p], q->seq, q->wgs, s, p ? nullptr : pages))) memcpy(h + begin, q->host + begin, parts.end[p] - begin);
     }
     return rc;
 }
@@ -480,7 +542,8 @@ static int take_parts(Slot* q, uint8_t* h, const Parts<PARTS>& parts, hipStream_
 // host, a destination in memory: 1.04 MB 98 | 46, 1.5 99 | 60, 2.0 106 | 72, 2.36 105 | 80, 3.0 113 | 97 (4.0 125 | 131), 2 of them the question. Into fresh memory, whose pages are made on the way, one thread
 // takes 0.16 us a KB more and ten share it: 1.04 MB 312 | 205, 1.5 326 | 290, 2.0 350 | 382, 2.36 365 | 450, 3.0 372 | 575. *took false: there were not enough slots at once, and
 // nothing was done.
-static int copy_d2h_alone(Ring* r, uint8_t* h, const uint8_t* from, size_t n, hipStream_t s, bool* took) {
+// A destination that is not in memory: its pages are made while the stream gets there; if they are not all there when the first part is, the workers take the slots.
+static int copy_d2h_alone(Ring* r, uint8_t* h, const uint8_t* from, size_t n, bool there, hipStream_t s, bool* took) {
     constexpr size_t MOST = D2H_ALONE / OUT_BYTES;
     const size_t count = (n + OUT_BYTES - 1) / OUT_BYTES, each = ((n + count - 1) / count + 255) & ~(size_t)255;
     static_assert(D2H_ALONE % OUT_BYTES == 0 && MOST <= BEGUN, "as many slots as a chunked copy holds while its stream is behind other work");
@@ -499,7 +562,16 @@ static int copy_d2h_alone(Ring* r, uint8_t* h, const uint8_t* from, size_t n, hi
         rc = send_parts(q[sent], from + at, n - at < each ? n - at : each, s, &parts[sent]);
         if (!rc) sent++;
     }
-    for (size_t i = 0; i < sent && !rc; i++) rc = take_parts(q[i], h + i * each, parts[i], s);
+    Pages pages(h, n);
+    if (*took && !rc && !there) {
+        if (!(rc = await_words(parts[0].done[0], q[0]->seq, q[0]->wgs, s, &pages)) && !pages.made()) {
+            Job j{};
+            j.count = count;
+            j.down = h; j.down_bytes = n; j.down_chunk = each;
+            return run_chunks(r, j, &s, 1, q, count, [](size_t, Slot*, hipStream_t, int*) { return (int)FHIP_OK; });   // (everything has been launched)
+        }
+    }
+    for (size_t i = 0; i < sent && !rc; i++) rc = take_parts(q[i], h + i * each, parts[i], s, i ? nullptr : &pages);
     if (rc && sent) (void)hipStreamSynchronize(s);      // an enqueued part may still use a slot
     for (size_t i = 0; i < have; i++) r->release(q[i]);
     return rc;
@@ -514,9 +586,9 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     Ring* r = ring(&rc);
     if (!r) return rc;
     const uint8_t* from = (const uint8_t*)d;
-    if (n > OUT_BYTES && n <= D2H_ALONE && (n <= D2H_ALONE_NEW || in_memory(h, n))) {
+    if (n > OUT_BYTES && n <= D2H_ALONE) {
         bool took;
-        if ((rc = copy_d2h_alone(r, (uint8_t*)h, from, n, s, &took)) || took) return rc;
+        if ((rc = copy_d2h_alone(r, (uint8_t*)h, from, n, n <= D2H_ALONE_NEW || in_memory(h, n), s, &took)) || took) return rc;
     }
     if (n > OUT_BYTES) {
         Job j{};
@@ -536,7 +608,8 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
             if (!(rc = launch(n_begun++, q, s, &wgs))) { q->seq++; q->wgs = wgs; }
         }
         if (!rc && !n_begun) return copy_d2h_plain(h, d, n, s);
-        if (!rc) rc = await_words(begun[0]->done, begun[0]->seq, begun[0]->wgs, s);
+        Pages pages(h, n);
+        if (!rc) rc = await_words(begun[0]->done, begun[0]->seq, begun[0]->wgs, s, &pages);
         if (!rc) return run_chunks(r, j, &s, 1, begun, n_begun, launch);
         (void)hipStreamSynchronize(s);              // an enqueued chunk may still use a slot
         for (size_t i = 0; i < n_begun; i++) r->release(begun[i]);
@@ -545,7 +618,8 @@ int copy_d2h(void* h, const void* d, size_t n, hipStream_t s) {
     Slot* q = r->get(&rc);
     if (!q) return rc ? rc : copy_d2h_plain(h, d, n, s);
     Parts<PARTS> parts;
-    if (!(rc = send_parts(q, from, n, s, &parts))) rc = take_parts(q, (uint8_t*)h, parts, s);
+    Pages pages(h, n);
+    if (!(rc = send_parts(q, from, n, s, &parts))) rc = take_parts(q, (uint8_t*)h, parts, s, &pages);
     r->release(q);
     return rc;
 }

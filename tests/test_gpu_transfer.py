@@ -39,6 +39,45 @@ def test_copies_back_of_two_and_three_slots(F, n, offset):
     test_round_trip(F, n, offset)
 
 
+# the runtime's, in two chunks, in as many as there are slots, the runtime's again; to an idle stream and behind other work
+@pytest.mark.parametrize("n", [1280 * KIB, 1280 * KIB + 1, 2 * MIB, 2 * MIB + 3, 7 * MIB + 260, 12 * MIB, 12 * MIB + 1])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_uploads_have_read_their_source(F, n, offset):
+    lib, check = F._lib.load(), F._lib.check
+    a = np.random.default_rng(n).integers(0, 256, n, np.uint8)
+    buf, other, s = F.DeviceBuffer(n + offset + 64), F.DeviceBuffer(64 * MIB), F.Stream()
+    for busy in (False, True):
+        check(lib.fhip_memset(buf.ptr, 0xA5, n + offset + 64, s.handle))
+        if busy:
+            for _ in range(4):
+                check(lib.fhip_memset(other.ptr, 1, 64 * MIB, s.handle))
+        else:
+            s.synchronize()
+        src = a.copy()
+        check(lib.fhip_upload(C.c_void_p(buf.ptr.value + offset), src.ctypes.data, n, s.handle))
+        src[:] = 0
+        out = np.empty(n + offset + 64, np.uint8)
+        check(lib.fhip_memcpy_d2h(out.ctypes.data, buf.ptr, out.size, s.handle))
+        assert np.array_equal(out[offset:offset + n], a) and (out[:offset] == 0xA5).all() and (out[offset + n:] == 0xA5).all(), busy
+
+
+# a destination whose pages are made while its stream is busy: in parts, two and three slots, the workers; nothing around it is written
+@pytest.mark.parametrize("n", [20 * KIB, 608 * KIB, MIB + 5, 2 * MIB + 4097, 3 * MIB, 5 * MIB + 3])
+@pytest.mark.parametrize("fills", [1, 40])
+def test_copies_back_into_fresh_memory_behind_other_work(F, n, fills):
+    import mmap
+    lib, check = F._lib.load(), F._lib.check
+    a = np.random.default_rng(n).integers(0, 256, n, np.uint8)
+    buf, other, s = F.DeviceBuffer(n), F.DeviceBuffer(64 * MIB), F.Stream()
+    check(lib.fhip_upload(buf.ptr, a.ctypes.data, n, s.handle))
+    for offset in (0, 4000):
+        whole = np.frombuffer(mmap.mmap(-1, n + 8192), np.uint8)
+        for k in range(fills):
+            check(lib.fhip_memset(other.ptr, k, 64 * MIB, s.handle))
+        check(lib.fhip_memcpy_d2h(whole[offset:].ctypes.data, buf.ptr, n, s.handle))
+        assert np.array_equal(whole[offset:offset + n], a) and not whole[:offset].any() and not whole[offset + n:].any()
+
+
 # who empties the slots goes by whether the destination's pages are there: none of them, all, all but the first or the last
 @pytest.mark.parametrize("n", [3 * MIB // 2, 3 * MIB // 2 + 1, 2 * MIB + 4097, 3 * MIB])
 @pytest.mark.parametrize("touched", ["none", "all", "not the first", "not the last"])
