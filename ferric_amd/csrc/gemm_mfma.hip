@@ -25,7 +25,7 @@
 // Dequantized values are exactly the f32 the CPU dequantizer produces, rounded to bf16 (RNE) by
 // v_cvt_pk_bf16_f32.
 // Four kernels: the tiled one (256 activation rows x 256 outputs per workgroup), its 160-column variant (256 or 128 rows) for output
-// widths that 160 deals to the chip's workgroups exactly, one of 64 or 128 rows x 64 ... 256 outputs whose waves unpack for themselves
+// widths that 160 deals to the chip's workgroups exactly, one of 64 or 128 rows x 32 ... 256 outputs whose waves unpack for themselves
 // (short prompts, small weights), and one for up to 32 rows; the launcher picks by a cost estimate. A launch that cuts output tiles along K sums the partial tiles in a fixed order: the same inputs give the
 // same bits on every run.
 #include "prompt.hpp"
@@ -41,8 +41,8 @@
 #define FHIP_GEMM_PASTE(a, b) FHIP_GEMM_PASTE2(a, b)
 #define FHIP_GEMM_NAME(what) FHIP_GEMM_PASTE(FHIP_GEMM_PASTE(gemm_, FHIP_GEMM_FORMAT), what)
 namespace fhip {
-constexpr int GEMM_TILES = 12;
-extern int g_gemm_tile;   // tests: 0 ... 11 pins a tile (BM_OF x BN_OF below), anything else: the estimate decides
+constexpr int GEMM_TILES = 13;
+extern int g_gemm_tile;   // tests: 0 ... 12 pins a tile (BM_OF x BN_OF below), anything else: the estimate decides
 #define FHIP_GEMM_DECLARE(F) \
     size_t gemm_##F##_ws_bytes(const fhip_weight* w, size_t columns, size_t t, bool run_sums); \
     int gemm_##F##_launch(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_y, hipStream_t s, float* d_ws, size_t ws_bytes, bool run_sums); \
@@ -112,7 +112,7 @@ struct Q4K {
     static constexpr int BLOCK = 144;
     static constexpr float UNPACK_US = 1.4f;   // unpack of a 256 x 256 chunk by one workgroup
     // one chunk of a workgroup tile, in us, in the order of BM_OF x BN_OF (fitted, see plan_cost_us)
-    static constexpr float CHUNK_US[NTILES] = {2.39f, 3.62f, 7.17f, 4.81f, 2.02f, 1.29f, 3.00f, 1.75f, 1.16f, 1.62f, 0.78f, 1.22f};
+    static constexpr float CHUNK_US[NTILES] = {2.39f, 3.62f, 7.17f, 4.81f, 2.02f, 1.29f, 3.00f, 1.75f, 1.16f, 1.62f, 0.78f, 1.22f, 0.61f};
     static constexpr float RUN_CHUNK_US[7] = {3.43f, 4.76f, 8.15f, 5.19f, 2.84f, 2.00f, 3.29f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
@@ -172,7 +172,7 @@ struct Q5K {
     using Eager = Q5K;
     static constexpr int BLOCK = 176;
     static constexpr float UNPACK_US = 1.8f;
-    static constexpr float CHUNK_US[NTILES] = {2.86f, 4.08f, 7.68f, 5.20f, 2.28f, 1.51f, 3.37f, 1.95f, 1.34f, 1.90f, 0.92f, 1.36f};
+    static constexpr float CHUNK_US[NTILES] = {2.86f, 4.08f, 7.68f, 5.20f, 2.28f, 1.51f, 3.37f, 1.95f, 1.34f, 1.90f, 0.92f, 1.36f, 0.72f};
     static constexpr float RUN_CHUNK_US[7] = {3.83f, 5.16f, 9.41f, 6.12f, 3.17f, 2.26f, 3.78f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
@@ -225,7 +225,7 @@ struct Q6K {
     // whose scale is sc[8hf + 2g + h]  (crates/ferric-gguf/src/lib.rs:833-851).
     static constexpr int BLOCK = 210;
     static constexpr float UNPACK_US = 2.3f;
-    static constexpr float CHUNK_US[NTILES] = {3.67f, 5.11f, 8.61f, 5.92f, 2.70f, 1.89f, 4.48f, 2.80f, 1.70f, 2.39f, 1.32f, 1.70f};
+    static constexpr float CHUNK_US[NTILES] = {3.67f, 5.11f, 8.61f, 5.92f, 2.70f, 1.89f, 4.48f, 2.80f, 1.70f, 2.39f, 1.32f, 1.70f, 0.92f};
     static constexpr float RUN_CHUNK_US[7] = {5.93f, 6.83f, 9.84f, 6.27f, 4.68f, 3.95f, 4.35f};
     static constexpr bool PARTIAL = false;
     static __host__ __device__ int chunks(int K) { return K / 256; }
@@ -301,7 +301,7 @@ struct Q80T {
     // read from the last valid block's address and given scale 0 (their activations are staged as 0 too).
     static constexpr int BLOCK = 34;
     static constexpr float UNPACK_US = 5.1f;
-    static constexpr float CHUNK_US[NTILES] = {4.66f, 5.96f, 11.44f, 6.65f, 3.15f, 2.23f, 4.62f, 2.91f, 1.98f, 2.76f, 1.22f, 1.76f};
+    static constexpr float CHUNK_US[NTILES] = {4.66f, 5.96f, 11.44f, 6.65f, 3.15f, 2.23f, 4.62f, 2.91f, 1.98f, 2.76f, 1.22f, 1.76f, 0.93f};
     static constexpr float RUN_CHUNK_US[7] = {9.40f, 9.88f, 11.93f, 6.86f, 7.00f, 6.50f, 5.05f};
     static constexpr bool PARTIAL = true;   // a row may end inside a chunk
     static __host__ __device__ int chunks(int K) { return (K + 255) / 256; }
@@ -829,7 +829,7 @@ __global__ void __launch_bounds__(512) gemm_q_bf16_n160_kernel(GemmParams p) {
 // chunk of Q4_K took 2.84 us there, 1.1 of it matrix instructions at the clock the chip holds. It takes 1.97 here (timing-only variants:
 // 1.45 with no loads, 0.6 without the matrix instructions). Here a wave holds BM activation rows x 32 outputs, so a weight is
 // unpacked by the one wave that multiplies it, straight into its B operand, and LDS carries the activations alone: a whole chunk of them
-// at a time, double buffered, one barrier a chunk. The eight waves are NW along N x KW = 8 / NW along the chunk's four steps (a wave does
+// at a time, double buffered, one barrier a chunk. The waves, mostly eight, are NW along N x KW along the chunk's four steps (a wave does
 // S = 4 / KW of them), and the KW partial sums of an output meet in LDS when a run ends, added in order of the steps. Work distribution
 // and slots of partial tiles are those of the tiled kernel. Measured with the tile the estimate picks, us, the tiled kernel alone before:
 // Q4_K 5120 x 5120 at 64 / 128 / 512 rows 17.2 / 20.8 / 43.8 -> 14.3 / 20.4 / 37.6, 6112 x 2816 at 132 39.9 -> 15.9, 10176 x 2560 at 82 23.4 -> 15.2; Q6_K
@@ -1588,8 +1588,8 @@ int launch_skinny(const fhip_weight* w, const uint16_t* d_x, size_t t, float* d_
 }
 
 // The tiles: rows x outputs. 2, 3 and 6 share a weight's unpacking among the waves that multiply it, the others leave it to the one wave.
-// 12 and 13 are 4 and 5 with one wave along K (run sums, below).
-constexpr int BM_OF[NTILES + 2] = {64, 128, 256, 256, 128, 64, 128, 128, 64, 64, 64, 128, 128, 64}, BN_OF[NTILES + 2] = {256, 256, 256, 160, 128, 128, 160, 96, 96, 160, 64, 64, 128, 128};
+// The two behind the last are 4 and 5 with one wave along K (run sums, below).
+constexpr int BM_OF[NTILES + 2] = {64, 128, 256, 256, 128, 64, 128, 128, 64, 64, 64, 128, 64, 128, 64}, BN_OF[NTILES + 2] = {256, 256, 256, 160, 128, 128, 160, 96, 96, 160, 64, 64, 32, 128, 128};
 
 // How a launch is dealt to the chip: `whole_rounds` whole tiles per workgroup, then the left-over tiles cut along K into runs of `per` chunks.
 struct TilePlan {
@@ -1639,7 +1639,10 @@ static long long plan_segments(const TilePlan& q) { return q.runs + (q.left - 1)
 // launches a tile, Q6_K's to 350: fitted to 136 they priced 128 x 96 too low, and of 350 weights the pick was 3.0 % slower than the best on average and up to 1.30 times
 // as slow as the model before (2480 x 9984 at 215 rows 34.8 -> 45.2 us); 1.8 % and 1.11 times now, where Q4_K, Q5_K and Q8_0 have 1.4, 1.8 and 1.3 % and at most 1.08 times. On
 // those 1400 launches 64 x 256 is the pick of 3 %, which take 7 % longer without it, 64 x 160 of 4 % and 5 %, 64 x 64 of 22 % and 14 %; 128 x 96 of 3 %, to no gain.
-constexpr float START_US[NTILES] = {3.77f, 3.88f, 4.04f, 4.53f, 3.92f, 3.12f, 4.91f, 3.57f, 2.73f, 4.01f, 2.31f, 3.95f}, FIX_US = 3.29f, SLOT_US = 4.18f, CUT_US = 0.1f;
+// 64 x 32, four waves, came later and was fitted by itself, to 560 of its launches, the near ones weighted: where 64 x 64 leaves half the chip idle and has to be cut along K, it
+// does not, and the summing launch is saved. It is the pick of 5 % of 480 drawn launches, to 0.77 of the time (at most 0.94): us, before -> now, Q4_K 6688 x 1024 at 54 rows 10.1 -> 7.2, Q5_K 7560 x 2560
+// at 63 14.3 -> 12.1, Q6_K 2168 x 1024 at 134 11.6 -> 9.2, Q8_0 1856 x 1280 at 146 14.4 -> 10.2.
+constexpr float START_US[NTILES] = {3.77f, 3.88f, 4.04f, 4.53f, 3.92f, 3.12f, 4.91f, 3.57f, 2.73f, 4.01f, 2.31f, 3.95f, 4.19f}, FIX_US = 3.29f, SLOT_US = 4.18f, CUT_US = 0.1f;
 template <class F>
 static float plan_cost_us(const TilePlan& q, long long cus) {
     const float chunks = (float)q.whole_rounds * (float)q.nchunks + (q.left > 0 ? (float)q.per : 0.f);
@@ -1711,7 +1714,7 @@ int launch_own(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_out,
 // prompt block on one, sums in another order make 38 % of the codes others (none is nearer f64), and a cache that was stored before would not
 // be met again. The tiles of short prompts run on the kernel whose waves unpack for themselves, one along K, which adds in the same order.
 // The figures below are no times of today's kernels, four of the seven tiles' kernels are gone: they say where runs end, on a chip of as many CUs, and are kept for that.
-constexpr int RUN_TILE_OF[7] = {0, 1, 2, 3, 12, 13, 6};
+constexpr int RUN_TILE_OF[7] = {0, 1, 2, 3, NTILES, NTILES + 1, 6};
 constexpr float RUN_FIXUP_US[7] = {0.9f, -2.3f, -13.2f, -5.2f, -1.0f, 1.5f, 0.4f};
 template <class F>
 static float run_sums_cost_us(const TilePlan& q, int i, long long cus) {
@@ -1776,10 +1779,11 @@ int launch_tiled(const fhip_weight* w, const uint16_t* d_x, size_t t, void* d_y,
         case 9: return launch_own<F, 2, 5, 2, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
         case 10: return launch_own<F, 2, 2, 4, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
         case 11: return launch_own<F, 4, 2, 4, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        case 12: return launch_own<F, 2, 1, 4, SWIGLU>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
     }
     if constexpr (!SWIGLU) {
-        if (q.tile == 12) return launch_own<F, 4, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
-        if (q.tile == 13) return launch_own<F, 2, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        if (q.tile == NTILES) return launch_own<F, 4, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
+        if (q.tile == NTILES + 1) return launch_own<F, 2, 4, 1, false>(w, d_x, t, d_y, s, q, d_ws, ws_bytes);
     }
     return fhip::set_error(FHIP_ERR_ARG, "gemm_q_bf16: no tile %d", q.tile);
 }

@@ -63,7 +63,7 @@ def test_seeded_random_shapes(F, O):
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6])
 def test_every_tile_on_ragged_shapes(F, O, tile):
-    # The launcher picks one of twelve workgroup tiles by estimate; here the first seven are pinned in turn (64 / 128 / 256 rows x 256
+    # The launcher picks one of thirteen workgroup tiles by estimate; here the first seven are pinned in turn (64 / 128 / 256 rows x 256
     # outputs, 256 x 160, 128 / 64 rows x 128, 128 x 160) and run on shapes that fill no tile: rows and outputs that end inside a tile, outputs that are no
     # multiple of 4, launches with whole rounds of tiles and a cut remainder, launches where every tile is cut along K.
     lib = F._lib.load()
@@ -77,9 +77,9 @@ def test_every_tile_on_ragged_shapes(F, O, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
-@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11])
+@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11, 12])
 def test_tiles_whose_waves_unpack_for_themselves(F, O, tile):
-    # 64 / 128 rows x 64 ... 256 outputs: one, two and three chunks of K a run (the pipeline is two deep), an odd chunk count, a run that
+    # 64 / 128 rows x 32 ... 256 outputs: one, two and three chunks of K a run (the pipeline is two deep), an odd chunk count, a run that
     # starts in one tile and ends in the next, rows and outputs that end inside a tile, a Q8_0 row that ends inside a chunk, every format,
     # and SwiGLU in the launch; the same bits again on a second run.
     lib = F._lib.load()
@@ -94,7 +94,7 @@ def test_tiles_whose_waves_unpack_for_themselves(F, O, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
-@pytest.mark.parametrize("tile", range(-1, 12))
+@pytest.mark.parametrize("tile", range(-1, 13))
 def test_rows_shorter_than_a_chunk(F, O, tile):
     # Q8_0 rows of one to seven blocks, one short of a chunk of 256 columns: what lies behind a row is staged as zeros, behind the last one too.
     lib = F._lib.load()
@@ -344,7 +344,7 @@ def test_swiglu_inside_the_tiled_gemm(F, tile):
         lib.fhip_debug_gemm_tile(before)
 
 
-@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11])
+@pytest.mark.parametrize("tile", [0, 1, 4, 5, 7, 8, 9, 10, 11, 12])
 def test_swiglu_of_rows_turned_through_lds(F, tile):
     # Q6_K and Q8_0 gate|up on the tiles whose waves unpack for themselves: a wave's gate and up rows lie in two places. Rows of an odd number of blocks, whose
     # addresses alternate modulo 4, widths that end inside a tile, one chunk and an odd number of them, a Q8_0 row that ends inside a chunk; against the
