@@ -124,6 +124,8 @@ SYMBOLS = {
     "fhip_qkv_post_attention": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _sz, C.c_int, C.c_float, C.c_float, _vp, _vp, _sz, _sz, _sz,
                                           C.c_float, _vp, _vp, _vp]),
     "fhip_decode_attention_ex": (C.c_int, [_vp, _vp, _vp, _sz, _sz, _sz, _sz, _vp, _sz, C.c_float, _vp, _vp, _vp]),
+    "fhip_add_count": (C.c_int, [_vp, _vp, _sz, _vp, _vp, _u32, _vp]),
+    "fhip_norm_matmul_q_count": (C.c_int, [_vp, _vp, _vp, _vp, C.c_float, _vp, _vp, C.c_int, _vp, _vp, _u32, _vp]),
     "fhip_norm_matmul_q": (C.c_int, [_vp, _vp, _vp, _vp, C.c_float, _vp, _vp, C.c_int, _vp, _vp]),
     "fhip_debug_generic_matvec": (C.c_int, [C.c_int]),
     "fhip_debug_quad_matvec": (C.c_int, [C.c_int]),

@@ -1171,8 +1171,8 @@ int fhip_qkv_post_attention_kvq(int fmt, const float* d_qkv, const float* d_bias
                                                (hipStream_t)stream);
 }
 
-int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
-                       float* d_h_scratch, int swiglu, float* d_y, void* stream) {
+static int norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
+                         float* d_h_scratch, int swiglu, float* d_y, uint32_t* d_count, uint32_t by, void* stream) {
     int rc = need_init();
     if (rc) return rc;
     if (!w || !d_x || !d_norm_w || !d_h_scratch || !d_y) return set_error(FHIP_ERR_ARG, "fhip_norm_matmul_q: NULL pointer");
@@ -1194,9 +1194,18 @@ int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_re
     const size_t n_ff = swiglu ? w->rows / 2 : 0;
     fhip::NormParams np{d_norm_w, d_resid, d_resid ? d_x_out : nullptr, eps};   // without a residual there is no sum to store
     rc = fhip::launch_gemv_norm(w, d_x, d_y, n_ff, np, (hipStream_t)stream);
-    if (rc != fhip::NORM_NOT_FUSED) return rc;
-    if ((rc = fhip::launch_rmsnorm(d_x, d_resid, d_norm_w, 1, w->cols, eps, d_resid ? d_x_out : nullptr, d_h_scratch, (hipStream_t)stream))) return rc;
+    if (rc != fhip::NORM_NOT_FUSED) return rc || !d_count ? rc : fhip::launch_u32_add(d_count, 1, by, (hipStream_t)stream);
+    if ((rc = fhip::launch_rmsnorm(d_x, d_resid, d_norm_w, 1, w->cols, eps, d_resid ? d_x_out : nullptr, d_h_scratch, (hipStream_t)stream, d_count, by))) return rc;
     return fhip::launch_gemv(w, d_h_scratch, 1, d_y, n_ff, (hipStream_t)stream);
+}
+int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
+                       float* d_h_scratch, int swiglu, float* d_y, void* stream) {
+    return norm_matmul_q(w, d_x, d_resid, d_norm_w, eps, d_x_out, d_h_scratch, swiglu, d_y, nullptr, 0, stream);
+}
+int fhip_norm_matmul_q_count(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
+                             float* d_h_scratch, int swiglu, float* d_y, uint32_t* d_count, uint32_t by, void* stream) {
+    if (!d_count) return set_error(FHIP_ERR_ARG, "fhip_norm_matmul_q_count: NULL pointer");
+    return norm_matmul_q(w, d_x, d_resid, d_norm_w, eps, d_x_out, d_h_scratch, swiglu, d_y, d_count, by, stream);
 }
 
 int fhip_debug_generic_matvec(int on) {
@@ -1275,6 +1284,13 @@ int fhip_matvec_precision(int bits) {
     if (bits != 16 && bits != 24) return set_error(FHIP_ERR_ARG, "fhip_matvec_precision: 16 or 24 bits (0 to query), not %d", bits);
     g_default_planes = bits == 24 ? 3 : 2;
     return before;
+}
+
+int fhip_add_count(const float* d_a, const float* d_b, size_t n, float* d_out, uint32_t* d_count, uint32_t by, void* stream) {
+    int rc = need_init();
+    if (rc) return rc;
+    if (!d_count || (n && (!d_a || !d_b || !d_out))) return set_error(FHIP_ERR_ARG, "fhip_add_count: NULL pointer");
+    return fhip::launch_add(d_a, d_b, n, d_out, (hipStream_t)stream, d_count, by);
 }
 
 int fhip_u32_add(uint32_t* d_words, size_t n, uint32_t delta, void* stream) {

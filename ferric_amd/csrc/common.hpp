@@ -139,8 +139,8 @@ int launch_swiglu_bf16(const float* d_gu, size_t t, size_t d, uint16_t* d_out, h
 
 // decode_ops.hip: the steps either side of the matmuls in a decode layer
 int launch_rmsnorm(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, float* norm_out,
-                   hipStream_t s);
-int launch_add(const float* a, const float* b, size_t n, float* out, hipStream_t s);
+                   hipStream_t s, uint32_t* count = nullptr, uint32_t by = 0);   // count: `by` more in it, by the same launch
+int launch_add(const float* a, const float* b, size_t n, float* out, hipStream_t s, uint32_t* count = nullptr, uint32_t by = 0);
 int launch_u32_add(uint32_t* w, size_t n, uint32_t delta, hipStream_t s);
 // block-quantized K / V cache (kvquant.hip); scales addressed as uint16 [block] (Q4_1: [block][2])
 int launch_kvq_append(int fmt, const float* src, size_t src_row_stride, size_t t, size_t width, const uint32_t* d_pos, uint32_t pos_off,

@@ -42,7 +42,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // out[r, j] = x[r, j] * (1 / sqrt(mean_j x^2 + eps)) * weight[j]   (lib.rs:2018-2033); with b: x = a + b, and the sum is
 // written too (lib.rs:2057-2074). TPR threads share a row (a fixed-shape tree sum, so results do not depend on scheduling).
 // Out = uint16_t: the normed rows as bf16, rounded as fhip_cvt_f32_bf16 rounds them -- what the matrix cores read, for a prompt: a
-// launch and a trip of the f32 rows through memory less per matmul.
+// launch and a trip of the f32 rows through memory less per matmul. count: a word that gets `by` more beside the rows, a decode step's position, whose own launch
+// cost 2.5 us a token (null: none): eight layers behind 128 rows 634.4 -> 630.1 us a token, with the weights' trip under the row's.
 using fhip::pk_bf16;
 __device__ __forceinline__ void store_norm(float* out, size_t j, float4 v) { ((float4*)out)[j] = v; }
 __device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float4 v) { ((uint2*)out)[j] = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
@@ -51,7 +52,8 @@ __device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float v) { o
 template <int TPR, typename Out>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const float* __restrict__ b,
                                                       const float* __restrict__ weight, size_t rows, int d, float eps,
-                                                      float* sum_out, Out* __restrict__ norm_out) {   // sum_out may be a
+                                                      float* sum_out, Out* __restrict__ norm_out, uint32_t* count, uint32_t by) {   // sum_out may be a
+    if (count && blockIdx.x == 0 && threadIdx.x == 0) *count += by;
     constexpr int RPW = 256 / TPR;   // rows per workgroup
     constexpr int NV = 8;            // float4 per thread held in registers: rows up to 4 * NV * TPR values
     __shared__ float red[4];
@@ -62,18 +64,20 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
     const bool vec = (d & 3) == 0 && d <= 4 * NV * TPR && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)weight | (uintptr_t)sum_out | (uintptr_t)norm_out) & 15) == 0;
     float ms = 0.f;
     if (vec) {
-        // every load of the row is issued before the first use, so the row costs one memory round trip, not one per element
+        // every load of the row is issued before the first use, so the row costs one memory round trip, not one per element (and the weights none behind the sum)
         const int nv = d >> 2;
-        float4 r[NV];
+        float4 r[NV], w[NV];
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const int j = t + i * TPR;
             r[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (j < nv) {
                 r[i] = ((const float4*)(a + base))[j];
+                w[i] = ((const float4*)weight)[j];
                 if (b) { const float4 y = ((const float4*)(b + base))[j]; r[i].x += y.x; r[i].y += y.y; r[i].z += y.z; r[i].w += y.w; }
             }
         }
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < NV; i++) ms = fmaf(r[i].x, r[i].x, fmaf(r[i].y, r[i].y, fmaf(r[i].z, r[i].z, fmaf(r[i].w, r[i].w, ms))));
         ms = wave_sum(ms);
@@ -88,9 +92,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
         for (int i = 0; i < NV; i++) {
             const int j = t + i * TPR;
             if (j < nv) {
-                const float4 w = ((const float4*)weight)[j];
                 if (sum_out) ((float4*)(sum_out + base))[j] = r[i];
-                store_norm(norm_out + base, (size_t)j, make_float4(r[i].x * inv * w.x, r[i].y * inv * w.y, r[i].z * inv * w.z, r[i].w * inv * w.w));
+                store_norm(norm_out + base, (size_t)j, make_float4(r[i].x * inv * w[i].x, r[i].y * inv * w[i].y, r[i].z * inv * w[i].z, r[i].w * inv * w[i].w));
             }
         }
         return;
@@ -121,7 +124,8 @@ __global__ void u32_add_kernel(uint32_t* w, size_t n, uint32_t delta) {
     if (i < n) w[i] += delta;
 }
 
-__global__ void add_kernel(const float* a, const float* __restrict__ b, size_t n, float* out) {   // out may be a
+__global__ void add_kernel(const float* a, const float* __restrict__ b, size_t n, float* out, uint32_t* count, uint32_t by) {   // out may be a
+    if (count && blockIdx.x == 0 && threadIdx.x == 0) *count += by;
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[i] = a[i] + b[i];
 }
@@ -1546,23 +1550,23 @@ namespace fhip {
 
 template <typename Out>
 static int launch_rmsnorm_out(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, Out* norm_out,
-                              hipStream_t s) {
-    if (rows == 0 || d == 0) return FHIP_OK;
+                              hipStream_t s, uint32_t* count = nullptr, uint32_t by = 0) {
+    if (rows == 0 || d == 0) return count ? launch_u32_add(count, 1, by, s) : FHIP_OK;
     if (d > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: row length exceeds 2^31");
     if (d <= 512) {
         size_t grid = (rows + 3) / 4;
         if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<64, Out>), dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
+        hipLaunchKernelGGL((rmsnorm_kernel<64, Out>), dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out, count, by);
     } else {
         if (rows > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<256, Out>), dim3((unsigned)rows), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out);
+        hipLaunchKernelGGL((rmsnorm_kernel<256, Out>), dim3((unsigned)rows), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out, count, by);
     }
     return check_hip(hipGetLastError(), "rmsnorm launch");
 }
 
 int launch_rmsnorm(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, float* norm_out,
-                   hipStream_t s) {
-    return launch_rmsnorm_out(a, b, weight, rows, d, eps, sum_out, norm_out, s);
+                   hipStream_t s, uint32_t* count, uint32_t by) {
+    return launch_rmsnorm_out(a, b, weight, rows, d, eps, sum_out, norm_out, s, count, by);
 }
 int launch_rmsnorm_bf16(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, uint16_t* norm_out,
                         hipStream_t s) {
@@ -1576,11 +1580,11 @@ int launch_u32_add(uint32_t* w, size_t n, uint32_t delta, hipStream_t s) {
     return check_hip(hipGetLastError(), "u32_add launch");
 }
 
-int launch_add(const float* a, const float* b, size_t n, float* out, hipStream_t s) {
-    if (n == 0) return FHIP_OK;
+int launch_add(const float* a, const float* b, size_t n, float* out, hipStream_t s, uint32_t* count, uint32_t by) {
+    if (n == 0) return count ? launch_u32_add(count, 1, by, s) : FHIP_OK;
     size_t grid = (n + 255) / 256;
     if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "add: too many elements for one launch");
-    hipLaunchKernelGGL(add_kernel, dim3((unsigned)grid), dim3(256), 0, s, a, b, n, out);
+    hipLaunchKernelGGL(add_kernel, dim3((unsigned)grid), dim3(256), 0, s, a, b, n, out, count, by);
     return check_hip(hipGetLastError(), "add launch");
 }
 

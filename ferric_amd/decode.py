@@ -243,10 +243,9 @@ class Qwen3Decoder:
         # a default-arm layer; short caches, whose attention splits nothing, need no combine launch behind it
         short = self.ws is None
         self.launches_per_layer = (7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) - (1 if short else 0)
-        # per token beside the layers: the position word's increment and the head (final norm inside the head's mat-vec; a head of
-        # 128 MB and more takes the norm as a launch of its own, which costs less than the wider workgroups the fused norm needs)
-        big_head = lm_head is not None and lm_head.nbytes() >= (128 << 20)
-        self.launches_per_token_extra = 1 + ((1 if self.fuse_norm and not big_head else 2) if lm_head is not None else 0)
+        # per token beside the layers: the head and the position word's increment, which the final norm's launch or the last residual add takes with it (the
+        # final norm is inside the head's mat-vec, but for a head of 128 MB and more: there a launch of its own costs less than the wider workgroups the fused norm needs)
+        self.launches_per_token_extra = (2 if self.fuse_norm else 3) if lm_head is not None else 1
         self._graph = None
 
     # -- state ------------------------------------------------------------------------------------
@@ -265,9 +264,13 @@ class Qwen3Decoder:
         _upload(self.xa.buf, a, self.stream)
 
     # -- one step ---------------------------------------------------------------------------------
-    def _norm_matmul(self, w, cur, alt, resid, norm_w, y, swiglu):
-        """y = [swiglu] rmsnorm(cur [+ resid]) W^T; returns the buffer that holds cur + resid afterwards."""
+    def _norm_matmul(self, w, cur, alt, resid, norm_w, y, swiglu, count=None):
+        """y = [swiglu] rmsnorm(cur [+ resid]) W^T; returns the buffer that holds cur + resid afterwards. count: a word that gets one more."""
         lib, c, s = _lib.load(), self.cfg, _stream_handle(self.stream)
+        if self.fuse_norm and count is not None:
+            _check(lib.fhip_norm_matmul_q_count(w.handle, cur.buf.ptr, resid.buf.ptr if resid is not None else None, norm_w.buf.ptr, c.eps,
+                                                alt.buf.ptr if resid is not None else None, self.h.buf.ptr, int(swiglu), y.buf.ptr, count.buf.ptr, 1, s))
+            return alt if resid is not None else cur
         if self.fuse_norm:
             _check(lib.fhip_norm_matmul_q(w.handle, cur.buf.ptr, resid.buf.ptr if resid is not None else None, norm_w.buf.ptr, c.eps,
                                           alt.buf.ptr if resid is not None else None, self.h.buf.ptr, int(swiglu), y.buf.ptr, s))
@@ -278,6 +281,8 @@ class Qwen3Decoder:
             _check(lib.fhip_add_rmsnorm(cur.buf.ptr, resid.buf.ptr, norm_w.buf.ptr, 1, c.d_model, c.eps, cur.buf.ptr, self.h.buf.ptr, s))
         fn = lib.fhip_matmul_q_swiglu if swiglu else lib.fhip_matmul_q
         _check(fn(w.handle, self.h.buf.ptr, 1, y.buf.ptr, s))
+        if count is not None:
+            _check(lib.fhip_u32_add(count.buf.ptr, 1, 1, s))
         return cur
 
     def _enqueue_step(self):
@@ -342,11 +347,10 @@ class Qwen3Decoder:
                 _check(lib.fhip_rmsnorm(self.y.buf.ptr, l.post_ffn_norm.buf.ptr, 1, c.d_model, c.post_norm_eps, self.yn.buf.ptr, s))
                 pending = self.yn
         if self.lm_head is not None:   # last residual add fused with the output norm, then the LM head
-            cur = self._norm_matmul(self.lm_head, cur, alt, pending, self.output_norm, self.logits, False)
+            cur = self._norm_matmul(self.lm_head, cur, alt, pending, self.output_norm, self.logits, False, count=self.pos)
         else:
-            _check(lib.fhip_add(cur.buf.ptr, pending.buf.ptr, c.d_model, cur.buf.ptr, s))
+            _check(lib.fhip_add_count(cur.buf.ptr, pending.buf.ptr, c.d_model, cur.buf.ptr, self.pos.buf.ptr, 1, s))
         self.x = cur
-        _check(lib.fhip_u32_add(self.pos.buf.ptr, 1, 1, s))
 
     # -- a block of prompt rows -------------------------------------------------------------------
     def prefill(self, x_host, precise=False):
@@ -468,8 +472,9 @@ class Qwen3Decoder:
                 _check(lib.fhip_rmsnorm(y.buf.ptr, l.post_ffn_norm.buf.ptr, t, c.d_model, c.post_norm_eps, normed.buf.ptr, s))
                 pending = normed
         if pending is not None:
-            _check(lib.fhip_add(x1.buf.ptr, pending.buf.ptr, t * c.d_model, X.buf.ptr, s))
-        _check(lib.fhip_u32_add(self.pos.buf.ptr, 1, t, s))
+            _check(lib.fhip_add_count(x1.buf.ptr, pending.buf.ptr, t * c.d_model, X.buf.ptr, self.pos.buf.ptr, t, s))
+        else:
+            _check(lib.fhip_u32_add(self.pos.buf.ptr, 1, t, s))
         out = X.to_vec(self.stream).reshape(t, c.d_model)      # synchronises: the temporaries may go
         for cache in self._all_caches():
             cache.len += t

@@ -284,6 +284,8 @@ int fhip_add_rmsnorm_bf16(const float* d_a, const float* d_b, const float* d_wei
 
 /* lib.rs:279 Tensor::add, same shapes: out = a + b, n elements. */
 int fhip_add(const float* d_a, const float* d_b, size_t n, float* d_out, void* stream);
+/* fhip_add and fhip_u32_add of the one word d_count in one launch. */
+int fhip_add_count(const float* d_a, const float* d_b, size_t n, float* d_out, uint32_t* d_count, uint32_t by, void* stream);
 /* out = a * sigmoid(g), n values; d_out may be d_a. The gate of a gated-attention layer on the attention output,
  * crates/ferric-llama/src/qwen3.rs:936-938 (`o.mul(&h.matmul_q(wg).sigmoid())`), sigmoid as lib.rs:299 / :1915. */
 int fhip_mul_sigmoid(const float* d_a, const float* d_g, size_t n, float* d_out, void* stream);
@@ -446,6 +448,10 @@ int fhip_qkv_post_attention_kvq(int fmt, const float* d_qkv, const float* d_bias
  * rounding (the sum of squares is added in a different order), not the same bits. No single counterpart in the reference. */
 int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
                        float* d_h_scratch, int swiglu, float* d_y, void* stream);
+/* The same, and *d_count += by (a decode step's position word) before the call's last launch ends: inside the norm's launch where that is one of its own, by one more
+ * otherwise. No other argument may share memory with d_count. */
+int fhip_norm_matmul_q_count(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
+                             float* d_h_scratch, int swiglu, float* d_y, uint32_t* d_count, uint32_t by, void* stream);
 
 /* fhip_ffn for callers that cannot allocate or bring a workspace (code under graph capture, tight serving loops, harnesses
  * that forbid hipMalloc): the [rows_x, n_ff] intermediate lives in a 512 KiB array built into the library's code object (one

@@ -334,6 +334,32 @@ def test_post_processing_inside_the_attention_launch(F, X, D):
                                                  vc2.buf.ptr, cap, cap, 0, 0.0, ws.ptr, got.buf.ptr, None))
 
 
+# the norm inside the mat-vec (Q4_K), in a launch of its own whose thread takes the word along (Q4_0; rows that are and are not whole 16-byte pieces)
+@pytest.mark.parametrize("ty,cols", [(12, 1024), (2, 1024), (2, 8224), (2, 9248)])
+@pytest.mark.parametrize("resid", [False, True])
+def test_the_position_word_goes_along(F, ty, cols, resid):
+    """fhip_norm_matmul_q_count and fhip_add_count: the bits of the calls without the word, and the word."""
+    from ferric_amd.synth import synth_weights
+    lib, rng = F._lib.load(), np.random.default_rng(cols)
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    x, r, nw = (T(rng.standard_normal(cols).astype(np.float32)) for _ in range(3))
+    w = F.QMatrix.from_bytes(synth_weights(ty, 70, cols, 3), ty, 70, cols)
+    word = F.Tensor(F.DeviceBuffer(8), (2,), np.uint32)
+    start = np.array([0xFFFFFFFE, 7], np.uint32)
+    F._lib.check(lib.fhip_memcpy_h2d(word.buf.ptr, start.ctypes.data, 8, None))
+    got = []
+    for count in (False, True):
+        y, xo, hs, total = (F.Tensor.empty((n,)) for n in (70, cols, cols, cols))
+        args = (w.handle, x.buf.ptr, r.buf.ptr if resid else None, nw.buf.ptr, 1e-6, xo.buf.ptr if resid else None, hs.buf.ptr, 0, y.buf.ptr)
+        F._lib.check(lib.fhip_norm_matmul_q_count(*args, word.buf.ptr, 1, None) if count else lib.fhip_norm_matmul_q(*args, None))
+        F._lib.check(lib.fhip_add_count(x.buf.ptr, r.buf.ptr, cols, total.buf.ptr, word.buf.ptr, 40, None) if count else lib.fhip_add(x.buf.ptr, r.buf.ptr, cols, total.buf.ptr, None))
+        got.append([t.to_vec().view(np.uint32) for t in ((y, total, xo) if resid else (y, total))])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    assert word.to_vec().tolist() == [(0xFFFFFFFE + 41) & 0xFFFFFFFF, 7]
+    assert lib.fhip_add_count(x.buf.ptr, r.buf.ptr, 4, total.buf.ptr, None, 1, None) != 0
+
+
 def test_norm_fused_into_the_matvec(F, X, D, O, precision):
     """fhip_norm_matmul_q against rmsnorm / add_rmsnorm followed by the mat-vec: the residual sum bit-exact, the product
     within the dot-product bound of the unfused pair (the sum of squares is added in another order: ~1e-7 on the scale),
