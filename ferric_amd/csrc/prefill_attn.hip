@@ -55,6 +55,45 @@ using fhip::pk_bf16;
 __device__ __forceinline__ void store_out(float* p, float4 v) { *(float4*)p = v; }
 __device__ __forceinline__ void store_out(uint16_t* p, float4 v) { *(uint2*)p = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
 
+// Scores of a lane's query, at position qpos, against its keys j .. j + 3
+__device__ __forceinline__ void scores(f32x4& s, int j, int qpos, bool whole, float scale, int window, float softcap) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) s[r] *= scale;
+    if (softcap > 0.f) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) s[r] = softcap * tanhf(s[r] / softcap);    // cap * tanh(x / cap), crates/ferric-tensor/src/lib.rs:308
+    }
+    if (!whole) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) s[r] = j + r <= qpos && (window == 0 || qpos - (j + r) < window) ? s[r] : -3.0e38f;   // nn.rs:128-133
+    }
+}
+// A tile's scores into weights under the running statistics; returns what the sums so far are multiplied by.
+__device__ __forceinline__ float weights(f32x4 (&s)[2], float& m, float& l) {
+    float mt = -3.0e38f;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) mt = fmaxf(mt, s[u][r]);
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+    mt = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+    const float m_new = fmaxf(m, fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1])));
+    const float corr = __expf(m - m_new);
+    float ps = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float p = s[u][r] > -2.9e38f ? __expf(s[u][r] - m_new) : 0.f;
+            s[u][r] = p;
+            ps += p;
+        }
+    l = fmaf(l, corr, ps);
+    m = m_new;
+    return corr;
+}
+
 // NW: waves (16 query rows each) per workgroup. STAGED: the workgroup's waves call it together and share the tiles in Ks [32][HD + 4] and Vs
 // [32][HD]. Otherwise a wave comes alone, waits for no other and takes its operands from memory: the same instructions on the same
 // values, the same bits, about three times the time.
@@ -152,38 +191,11 @@ __device__ __forceinline__ void f32_body(float* Ks, float* Vs, const float* __re
             sacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0.w, qf[t + 3], sacc[0], 0, 0, 0);
             sacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k1.w, qf[t + 3], sacc[1], 0, 0, 0);
         }
-        // scores of this lane's query against its 8 keys of the tile; a tile every query of the wave sees whole needs no mask
+        // a tile every query of the wave sees whole needs no mask
         const bool whole = kt * 32 + 31 <= off + i0 && (window == 0 || off + i_last - kt * 32 < window);
-        float mt = -3.0e38f;
 #pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                float s = sacc[u][r] * scale;
-                if (softcap > 0.f) s = softcap * tanhf(s / softcap);        // cap * tanh(x / cap), crates/ferric-tensor/src/lib.rs:308
-                if (!whole) {
-                    const int j = kt * 32 + 16 * u + 4 * ks + r;
-                    const bool ok = j <= qpos && (window == 0 || qpos - j < window);   // nn.rs:128-133
-                    s = ok ? s : -3.0e38f;
-                }
-                sacc[u][r] = s;
-                mt = fmaxf(mt, s);
-            }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float m_new = fmaxf(m, mt);
-        const float corr = __expf(m - m_new);
-        float ps = 0.f;
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float p = sacc[u][r] > -2.9e38f ? __expf(sacc[u][r] - m_new) : 0.f;
-                sacc[u][r] = p;
-                ps += p;
-            }
-        l = fmaf(l, corr, ps);
-        m = m_new;
+        for (int u = 0; u < 2; u++) scores(sacc[u], kt * 32 + 16 * u + 4 * ks, qpos, whole, scale, window, softcap);
+        const float corr = weights(sacc, m, l);
 #pragma unroll
         for (int d = 0; d < NDT; d++) oacc[d] *= corr;
 #pragma unroll
@@ -224,6 +236,186 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) void causal_attn_kernel(c
     __shared__ __attribute__((aligned(16))) float Ks[32 * (HD + 4)];    // floats per K row in LDS: four banks on from row to row
     __shared__ __attribute__((aligned(16))) float Vs[32 * HD];
     f32_body<HD, NW, true>(Ks, Vs, q, K, V, T, S, n_head, n_kv, scale, window, softcap, out);
+}
+
+// The key tiles that the query rows wg_first .. wg_last see, at least one.
+struct KeyTiles {
+    int lo, hi;
+    __host__ __device__ int count() const { return hi - lo + 1; }
+};
+__host__ __device__ inline KeyTiles key_tiles(int off, int wg_first, int wg_last, int window) {
+    const int first = off + wg_first - window + 1;
+    return {window > 0 && first > 0 ? first / 32 : 0, (off + wg_last) / 32};
+}
+
+// 16 query rows of a head by a workgroup of four waves, for launches whose rows would leave SIMDs idle at a wave each (team_pays). A step is two key tiles:
+// wave w takes the products of keys 16 w .. 16 w + 15 with the queries, the scores go to the others through LDS, every wave forms all weights and takes a
+// quarter of the outputs' dims over all of the step's keys. Each sum is over the same products in the same order as where a wave has its rows to itself: the
+// same bits. No two waves want the same K row or the same dims of V, so K goes through LDS only to be read coalesced, by the wave that multiplies it, and V not
+// at all; one barrier a step, for the scores. The next step's products (one chain of dh / 4 instructions) run beside this step's weights, the next loads
+// beside its outputs.
+//
+// What bounds it: 64 KB a step at head size 128 through one CU's L1, 28 bytes a ns, 1.9 us (1.2 us for 32 KB), of which the products are 0.9 at 2.4 GHz. Stages
+// one after the other took 2.4 (issue of the loads 0.6, products 0.5, scores and their way through LDS 0.3, weights 0.2, outputs 0.8); K and V staged in
+// LDS for all waves, three barriers, 2.6; eight waves and four tiles a step the same time a tile. us, a wave per 16 rows -> this (rows x keys, heads, KV
+// heads, head size): 33 x 1057, 4, 4, 128 91.9 -> 34.2; 95 x 722, 8, 8, 128 63.5 -> 25.4; 152 x 152, 8, 4, 128 16.3 -> 8.9; 234 x 355, 32, 4, 128 36.2 -> 21.3;
+// 509 x 809, 16, 8, 128 73.2 -> 40.5; 152 x 940, 8, 8, 64 48.3 -> 21.3; 512 x 512, 32, 8, 64 29.0 -> 21.9; 60 x 60, 16, 4, 64 6.0 -> 4.3.
+template <int HD, typename Out>
+__global__ __launch_bounds__(256, 2) void causal_attn_team_kernel(const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, int T,
+                                                                  int S, int n_head, int n_kv, float scale, int window, float softcap,
+                                                                  Out* __restrict__ out) {
+    constexpr int KEYS = 64, QD = HD / 4;
+    constexpr int NE = HD / 64;                 // output tiles of 16 dims a wave
+    constexpr int KS = HD + 4;                  // floats a K row in LDS
+    constexpr int NF = HD / 16;                 // 16-byte pieces of a wave's 16 K rows a lane
+    constexpr int RL = HD / 4;                  // lanes a K row
+    typedef float vec __attribute__((ext_vector_type(NE)));
+    __shared__ __attribute__((aligned(16))) float Ks[KEYS * KS];        // each wave its own rows
+    __shared__ __attribute__((aligned(16))) f32x4 Ss[2][256];           // scores [16 keys][lane], four keys of a query: a step's, the next one's
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, ks = lane >> 4;
+    const int head = blockIdx.x, kvh = head / (n_head / n_kv);
+    const int i0 = 16 * ((int)gridDim.y - 1 - (int)blockIdx.y);         // longest first
+    const int off = S - T, i_last = min(i0 + 15, T - 1);
+    const int i = min(i0 + c, T - 1), qpos = off + i;
+    const KeyTiles seen = key_tiles(off, i0, i_last, window);
+    const unsigned row_bytes = (unsigned)n_kv * HD * 4;                 // 64 rows of it stay under 2^32
+    const int last_step = seen.lo + (seen.hi - seen.lo) / 2 * 2;
+
+    float qf[QD];
+    {
+        const float* qp = q + ((size_t)i * n_head + head) * HD + ks * QD;
+#pragma unroll
+        for (int t = 0; t < QD; t += 4) {
+            const f32x4 v = *(const f32x4*)(qp + t);
+#pragma unroll
+            for (int e = 0; e < 4; e++) qf[t + e] = v[e];
+        }
+    }
+    f32x4 oacc[NE];
+#pragma unroll
+    for (int e = 0; e < NE; e++) oacc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -3.0e38f, l = 0.f;
+    float* kmine = Ks + 16 * wave * KS;
+    f32x4 kreg[NF], kf[NF];
+    vec v[2][2][4];
+    f32x4 sacc;
+    // rows past the cache repeat its last row (masked below), steps past the last one that one
+    const unsigned kcol = lane % RL * 16, vcol = (16 * wave + c) * NE * 4;
+    unsigned krow[NF], vrow[2][2][4];
+#pragma unroll
+    for (int n = 0; n < NF; n++) krow[n] = (16 * wave + n * (64 / RL) + lane / RL) * row_bytes + kcol;
+#pragma unroll
+    for (int x = 0; x < 16; x++) vrow[x >> 3][x >> 2 & 1][x & 3] = (16 * (x >> 2) + 4 * ks + (x & 3)) * row_bytes + vcol;
+    auto base = [&](const float* p, int kt) { return (const char*)(p + (size_t)kt * 32 * n_kv * HD + kvh * HD); };
+    auto end = [&](int kt) { return (unsigned)min(S - 1 - kt * 32, KEYS) * row_bytes; };
+    auto request_k = [&](int n, int kt) { kreg[n] = *(const f32x4*)(base(K, kt) + min(krow[n], end(kt) + kcol)); };
+    auto request_v = [&](int x, int u, int r, int kt) { v[x][u][r] = *(const vec*)(base(V, kt) + min(vrow[x][u][r], end(kt) + vcol)); };
+    auto store_k = [&](int n) { *(f32x4*)(kmine + (n * (64 / RL) + lane / RL) * KS + lane % RL * 4) = kreg[n]; };
+    auto fragments = [&]() {
+#pragma unroll
+        for (int t = 0; t < NF; t++) kf[t] = *(const f32x4*)(kmine + c * KS + ks * QD + 4 * t);
+    };
+    auto own_rows = [&]() {                     // a wave's rows, written and read by different lanes of it
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto products = [&]() {
+        sacc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < QD; t++) sacc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t / 4][t % 4], qf[t], sacc, 0, 0, 0);
+    };
+    auto hand_over = [&](int kt, int buf) {
+        const int my = kt + (wave >> 1);        // past the last tile: masked
+        const bool whole = my * 32 + 31 <= off + i0 && (window == 0 || off + i_last - my * 32 < window);
+        scores(sacc, kt * 32 + 16 * wave + 4 * ks, qpos, whole, scale, window, softcap);
+        Ss[buf][64 * wave + lane] = sacc;
+    };
+    f32x4 p[2][2];
+    float corr[2];
+    auto take = [&](int buf) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) p[x >> 1][x & 1] = Ss[buf][64 * x + lane];
+    };
+    auto step_weights = [&]() {
+#pragma unroll
+        for (int x = 0; x < 2; x++) corr[x] = weights(p[x], m, l);      // of a tile past the last: 1, and m and l stay
+    };
+    auto outputs = [&](int x, auto beside) {
+#pragma unroll
+        for (int e = 0; e < NE; e++) oacc[e] *= corr[x];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+#pragma unroll
+                for (int e = 0; e < NE; e++) oacc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x][u][r][e], p[x][u][r], oacc[e], 0, 0, 0);
+                beside(x, u, r);
+            }
+    };
+
+    auto at = [&](int kt) { return min(kt, last_step); };
+#pragma unroll
+    for (int n = 0; n < NF; n++) request_k(n, seen.lo);
+#pragma unroll
+    for (int n = 0; n < NF; n++) store_k(n);
+#pragma unroll
+    for (int n = 0; n < NF; n++) request_k(n, at(seen.lo + 2));
+#pragma unroll
+    for (int x = 0; x < 16; x++) request_v(x >> 3, x >> 2 & 1, x & 3, seen.lo);
+    own_rows();
+    fragments();
+    products();
+    own_rows();
+#pragma unroll
+    for (int n = 0; n < NF; n++) store_k(n);
+#pragma unroll
+    for (int n = 0; n < NF; n++) request_k(n, at(seen.lo + 4));
+    own_rows();
+    fragments();
+    hand_over(seen.lo, 0);
+    int buf = 0;
+    for (int kt = seen.lo; kt < last_step; kt += 2) {
+        __syncthreads();    // the only one: scores written next were read before it
+        take(buf);
+        buf ^= 1;
+        products();                             // of the next step
+        step_weights();
+#pragma unroll
+        for (int t = 0; t < QD; t++) {          // the weights beside the products: else these wait for each other first
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 128 / QD, 0);
+        }
+        own_rows();
+        const int then = kt + 2;
+        outputs(0, [&](int x, int u, int r) {
+            request_v(x, u, r, then);
+            if (4 * u + r < NF) store_k(4 * u + r);
+        });
+        outputs(1, [&](int x, int u, int r) {
+            request_v(x, u, r, then);
+            if (4 * u + r < NF) request_k(4 * u + r, at(kt + 6));
+        });
+        own_rows();
+        fragments();
+        hand_over(then, buf);
+    }
+    __syncthreads();
+    take(buf);
+    step_weights();
+    outputs(0, [](int, int, int) {});
+    if (last_step < seen.hi) outputs(1, [](int, int, int) {});
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (i0 + c >= T) return;
+    const float inv = 1.0f / l;
+    // register r of output tile e is row 4 ks + r of it, i.e. dim NE (16 wave + 4 ks + r) + e
+    Out* op = out + ((size_t)i * n_head + head) * HD + NE * (16 * wave + 4 * ks);
+#pragma unroll
+    for (int y = 0; y < NE; y++) {
+        auto value = [&](int n) { return oacc[n % NE][n / NE] * inv; };
+        store_out(op + 4 * y, float4{value(4 * y), value(4 * y + 1), value(4 * y + 2), value(4 * y + 3)});
+    }
 }
 
 // ------------------------------------------------------------------------------------------------------------------------------
@@ -286,15 +478,6 @@ __device__ __forceinline__ float largest(float top, const f32x4 (&acc)[ND]) {
     return top;
 }
 
-// The key tiles that the query rows wg_first .. wg_last see, at least one.
-struct KeyTiles {
-    int lo, hi;
-    __host__ __device__ int count() const { return hi - lo + 1; }
-};
-__host__ __device__ inline KeyTiles key_tiles(int off, int wg_first, int wg_last, int window) {
-    const int first = off + wg_first - window + 1;
-    return {window > 0 && first > 0 ? first / 32 : 0, (off + wg_last) / 32};
-}
 // Of `count` tiles, n ranges of per (the last one's may be fewer; none is empty, since (n - 1) per <= (n - 1) * most < the count).
 struct KeyRanges { int n, per; };
 __host__ __device__ inline KeyRanges key_ranges(int count, int most) {
@@ -557,6 +740,22 @@ static int waves_of(size_t t, size_t n_head) {
     return ((t + 127) / 128) * n_head < 2 * cus ? 4 : 8;
 }
 
+// Whether 16 rows of a head get four waves of the f32 kernel's work (causal_attn_team_kernel) or one. A wave to itself takes 2.7 us a key tile at head size
+// 128 and 1.55 at 64, and a launch that leaves CUs idle lasts as long as its longest row; four waves take 2.2 and 1.2 .. 1.45 us for two tiles, a CU's workgroups one after
+// the other (they share its L1's bytes). So they are taken where the steps of a CU's share are at most 5/4 of the longest row's tiles. Over 150
+// shapes (2 .. 1024 rows behind 0 .. 3000 keys, 4 .. 64 heads) 132 are: 0.41 .. 0.95 of the time and 4.0 | 4.1 at 3 x 4, 0.64 on average; the others would be 0.88 .. 1.31:
+// 632 x 632, 32 heads of 64 39.2 | 34.4; 364 x 570, 40 of 128 54.8 | 52.7; 542 x 542, 64 of 128 74.5 | 82.4; 804 x 902, 64 of 64 89.5 | 117.3.
+static bool team_pays(size_t t, size_t s, size_t n_head, int win) {
+    const size_t cus = device_cus() > 0 ? device_cus() : 256, blocks = (t + 15) / 16;
+    if (blocks > 65535) return false;
+    const int off = (int)(s - t);
+    auto tiles = [&](size_t b) { return (size_t)key_tiles(off, (int)(16 * b), (int)(16 * b + 16 < t ? 16 * b + 16 : t) - 1, win).count(); };
+    const size_t most = 5 * tiles(blocks - 1) * cus / 4;
+    size_t steps = 0;
+    for (size_t b = 0; b < blocks && steps <= most; b++) steps += (tiles(b) + 1) / 2 * n_head;
+    return steps <= most;
+}
+
 // Ranges of at most `most` key tiles, at most `slots` of them a query block; most = 0: the keys stay in one piece.
 // A workgroup takes 2.15 us a tile of 64 rows at head size 128 and 1.3 at 64, and a CU's workgroups together 1.95 and 1.0, so a launch of one workgroup a CU or fewer
 // lasts as long as the block with the most tiles, one of up to two a CU as long as that block and the shortest that lies beside it. Ranges cost 4 us (the
@@ -635,6 +834,12 @@ static int launch_causal_out(const float* q, const float* K, const float* V, siz
     auto cut = [&](auto kernel, auto to, int most) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, to, ws, most); };
     auto f32 = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out); };
     if (!cuts) {
+        if (team_pays(t, s, n_head, win)) {
+            grid.y = (unsigned)((t + 15) / 16);
+            auto team = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, q, K, V, (int)t, (int)s, n_head, n_kv, scale, win, softcap, out); };
+            hd == 128 ? team(causal_attn_team_kernel<128, Out>) : team(causal_attn_team_kernel<64, Out>);
+            return check_hip(hipGetLastError(), "causal_attention launch");
+        }
         if (hd == 128) nw == 8 ? f32(causal_attn_kernel<128, 8, Out>) : f32(causal_attn_kernel<128, 4, Out>);
         else nw == 8 ? f32(causal_attn_kernel<64, 8, Out>) : f32(causal_attn_kernel<64, 4, Out>);
         return check_hip(hipGetLastError(), "causal_attention launch");

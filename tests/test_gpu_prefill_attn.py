@@ -122,6 +122,31 @@ def test_f32_products_beside_the_cut_ones(F, X, D, t, s, nh, nkv, hd, w, cap, vs
     assert lib.fhip_causal_attention_f32_products(*args[:3], s + 1, s, *args[5:], 0, out.buf.ptr, None) != 0
 
 
+@pytest.mark.parametrize("t,nh,nkv,hd,w,cap", [(1100, 64, 8, 64, 0, 0.0), (800, 64, 8, 128, 0, 30.0), (1100, 64, 16, 64, 77, 0.0), (1100, 64, 4, 128, 300, 0.0)])
+def test_f32_products_by_four_waves(F, X, t, nh, nkv, hd, w, cap):
+    # all rows at once give a wave its 16 rows, few of them four waves of work: the same products in the same order, so the same bits.
+    # Blocks of 1, 15 .. 17, 33 and 70 rows whose keys end at, before and behind the ends of tiles and of steps of two tiles; values of
+    # both signs and of a wide range.
+    lib, T = F._lib.load(), (lambda a: F.Tensor.from_vec(a, a.shape))
+    rng = np.random.default_rng(t + hd + w)
+    q = rng.standard_normal((t, nh * hd)).astype(np.float32) * 2
+    k = rng.standard_normal((t, nkv * hd)).astype(np.float32)
+    v = (rng.standard_normal((t, nkv * hd)) * np.exp(3 * rng.standard_normal((t, 1)))).astype(np.float32)
+
+    def rows(first, end, half):
+        tq, tk, tv = T(np.ascontiguousarray(q[first:end])), T(np.ascontiguousarray(k[:end])), T(np.ascontiguousarray(v[:end]))
+        out = T(np.zeros((end - first, nh * hd), np.float32))
+        assert lib.fhip_causal_attention_f32_products(tq.buf.ptr, tk.buf.ptr, tv.buf.ptr, end - first, end, nh, nkv, hd, w, cap, int(half), out.buf.ptr, None) == 0
+        got = out.to_vec()
+        return got.view(np.uint16).reshape(-1)[:got.size].reshape(end - first, -1) if half else got.reshape(end - first, -1)
+
+    for half in (False, True):
+        all_rows = rows(0, t, half)
+        assert np.abs(all_rows.view(np.uint16 if half else np.uint32)).max() > 0
+        for first, end in ((0, 1), (0, 15), (0, 16), (1, 18), (31, 64), (30, 63), (33, 65), (64, 97), (200, 270), (400, 401), (479, 512), (703, 720), (t - 17, t)):
+            assert np.array_equal(rows(first, end, half), all_rows[first:end]), (half, first, end)
+
+
 def both_kernels(F, X, q, k, v, nh, nkv, cap=0.0):
     """[t, nh * hd] of fhip_causal_attention and of fhip_causal_attention_f32_products, f32; the bf16 form of the first has to be its rounding."""
     lib, T, t, s, hd = F._lib.load(), (lambda a: F.Tensor.from_vec(a, a.shape)), q.shape[0], k.shape[0], q.shape[1] // nh
