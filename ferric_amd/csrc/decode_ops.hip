@@ -18,7 +18,6 @@
 #include <hip/hip_fp16.h>
 
 #include <math.h>
-#include <stdlib.h>
 
 namespace {
 
@@ -250,40 +249,41 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvPostParams p) {
     for (int j = p.n_rot + lane; j < p.hd; j += 64) dst[j] = val(j);
 }
 
-// The same operations for heads of 128 dims rotated whole in the split-half layout, the common case: a lane's two values are a pair,
-// so a head is read once and nothing is read again. A wave takes HPW consecutive heads of a token, requests them all before the first
-// is worked on, and works the token's angles out once for them. The one-head form above paid, per head, three round trips in a row (the
-// squares, the pair again, the weights) and the f64 exponential: 509 rows of 40 + 8 + 8 heads (29 MB) 19.2 -> 10.2 us.
-template <int HPW>
-__global__ __launch_bounds__(256) void qkv_post128_kernel(QkvPostParams p) {
+// The same operations for heads of 64 or 128 dims rotated whole in the split-half layout, the common case. Of 128 a lane's two values are a pair, of 64 it has
+// one, whose pair is 32 lanes away, so a head is read once and nothing is read again. A wave takes HPW consecutive heads of a token, requests them all before the
+// first is worked on, and works the token's angles out once for them. The one-head form above paid, per head, three round trips in a row (the squares,
+// the pair again, the weights) and the f64 exponential: 509 rows of 40 + 8 + 8 heads of 128 (29 MB) 19.2 us, here 7.6; 435 rows of 64 + 8 + 8 of 64 12.9 -> 8.3,
+// 1016 of 8 + 8 + 8 8.9 -> 6.5.
+template <int HD, int HPW>
+__global__ __launch_bounds__(256) void qkv_post_heads_kernel(QkvPostParams p) {
+    constexpr int E = HD / 64;
     const int lane = threadIdx.x & 63;
     const int per_tok = p.n_head + 2 * p.n_kv, waves_per_tok = (per_tok + HPW - 1) / HPW;
     const size_t wid = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wid >= (size_t)p.t * waves_per_tok) return;
     const int i = (int)(wid / waves_per_tok), h0 = (int)(wid % waves_per_tok) * HPW;
-    const float* x = p.qkv + ((size_t)i * per_tok + h0) * 128 + lane;
-    float a[HPW], b[HPW];
+    const float* x = p.qkv + ((size_t)i * per_tok + h0) * HD + lane;
+    float a[HPW][E];
 #pragma unroll
-    for (int j = 0; j < HPW; j++) {
-        const int o = h0 + j < per_tok ? 128 * j : 0;
-        a[j] = x[o];
-        b[j] = x[o + 64];
-    }
+    for (int j = 0; j < HPW; j++)
+#pragma unroll
+        for (int e = 0; e < E; e++) a[j][e] = x[(h0 + j < per_tok ? HD * j : 0) + 64 * e];
     const uint32_t pos = p.pos[i];
-    float wq[2] = {1.f, 1.f}, wk[2] = {1.f, 1.f};
-    if (p.q_norm) { wq[0] = p.q_norm[lane]; wq[1] = p.q_norm[lane + 64]; }
-    if (p.k_norm) { wk[0] = p.k_norm[lane]; wk[1] = p.k_norm[lane + 64]; }
-    if (p.bias) {
-        const float* bias = p.bias + (size_t)h0 * 128 + lane;
+    float wq[E], wk[E];
 #pragma unroll
-        for (int j = 0; j < HPW; j++) {
-            const int o = h0 + j < per_tok ? 128 * j : 0;
-            a[j] += bias[o];
-            b[j] += bias[o + 64];
-        }
+    for (int e = 0; e < E; e++) {
+        wq[e] = p.q_norm ? p.q_norm[lane + 64 * e] : 1.f;
+        wk[e] = p.k_norm ? p.k_norm[lane + 64 * e] : 1.f;
+    }
+    if (p.bias) {
+        const float* bias = p.bias + (size_t)h0 * HD + lane;
+#pragma unroll
+        for (int j = 0; j < HPW; j++)
+#pragma unroll
+            for (int e = 0; e < E; e++) a[j][e] += bias[(h0 + j < per_tok ? HD * j : 0) + 64 * e];
     }
     float sn = 0.f, cs = 1.f;
-    if (h0 < p.n_head + p.n_kv) sincosf((float)pos * rope_inv_freq(lane, p.rate, p.freq_scale), &sn, &cs);
+    if (h0 < p.n_head + p.n_kv) sincosf((float)pos * rope_inv_freq(lane & (HD / 2 - 1), p.rate, p.freq_scale), &sn, &cs);
     const bool stored = p.kv_packed || pos < p.cap;              // a position past the cache is dropped, never written out of bounds
     const size_t kv_row = (p.kv_packed ? (size_t)i : (size_t)pos) * p.n_kv;
 #pragma unroll
@@ -291,21 +291,29 @@ __global__ __launch_bounds__(256) void qkv_post128_kernel(QkvPostParams p) {
         const int h = h0 + j;
         if (h >= per_tok || (h >= p.n_head && !stored)) return;
         const bool value = h >= p.n_head + p.n_kv, key = !value && h >= p.n_head;
-        float* dst = value ? p.v_cache + (kv_row + (h - p.n_head - p.n_kv)) * 128
-                           : key ? p.k_cache + (kv_row + (h - p.n_head)) * 128 : p.q_out + ((size_t)i * p.n_head + h) * 128;
-        float x1 = a[j], x2 = b[j];
+        float* dst = value ? p.v_cache + (kv_row + (h - p.n_head - p.n_kv)) * HD
+                           : key ? p.k_cache + (kv_row + (h - p.n_head)) * HD : p.q_out + ((size_t)i * p.n_head + h) * HD;
+        float v[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = a[j][e];
         if (!value) {
             if (key ? p.k_norm : p.q_norm) {
-                const float inv = 1.0f / sqrtf(wave_sum(fmaf(x2, x2, x1 * x1)) / 128.0f + p.eps);
-                x1 = x1 * inv * (key ? wk[0] : wq[0]);
-                x2 = x2 * inv * (key ? wk[1] : wq[1]);
+                const float sq = fmaf(v[E - 1], v[E - 1], E == 2 ? v[0] * v[0] : 0.f);
+                const float inv = 1.0f / sqrtf(wave_sum(sq) / (float)HD + p.eps);
+#pragma unroll
+                for (int e = 0; e < E; e++) v[e] = v[e] * inv * (key ? wk[e] : wq[e]);
             }
-            const float y1 = rot_lo(x1, x2, cs, sn), y2 = rot_hi(x1, x2, cs, sn);
-            x1 = y1;
-            x2 = y2;
+            if constexpr (E == 2) {
+                const float y1 = rot_lo(v[0], v[1], cs, sn), y2 = rot_hi(v[0], v[1], cs, sn);
+                v[0] = y1;
+                v[1] = y2;
+            } else {
+                const float other = __shfl_xor(v[0], 32);
+                v[0] = lane < 32 ? rot_lo(v[0], other, cs, sn) : rot_hi(other, v[0], cs, sn);
+            }
         }
-        dst[lane] = x1;
-        dst[lane + 64] = x2;
+#pragma unroll
+        for (int e = 0; e < E; e++) dst[lane + 64 * e] = v[e];
     }
 }
 
@@ -315,16 +323,19 @@ __global__ __launch_bounds__(256) void qkv_post128_kernel(QkvPostParams p) {
 // thread walks its block). Operation by operation the two launches' arithmetic, so the same bytes. A token of 40 + 8 + 8 heads of
 // 128, Q8_0: 5.0 us against 4.7 + 4.4.
 constexpr int POST_KVQ_HD = 256;   // head sizes it takes: multiples of 32 up to this
-__device__ __forceinline__ float half32_max(float v) {
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+// Over the 32 lanes of a block, all of them active: in the 16 lanes of a row by rotations, then with the other row (in any order the same value).
+template <typename Op>
+__device__ __forceinline__ float half32(float v, Op op) {
+    auto turned = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, false)); };
+    v = op(v, turned(std::integral_constant<int, 0x128>()));     // row_ror:8, 4, 2, 1
+    v = op(v, turned(std::integral_constant<int, 0x124>()));
+    v = op(v, turned(std::integral_constant<int, 0x122>()));
+    v = op(v, turned(std::integral_constant<int, 0x121>()));
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
 }
-__device__ __forceinline__ float half32_min(float v) {
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    return v;
-}
+__device__ __forceinline__ float half32_max(float v) { return half32(v, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float half32_min(float v) { return half32(v, [](float a, float b) { return fminf(a, b); }); }
 __device__ __forceinline__ uint16_t kv_f16_bits(float x) {   // a NaN keeps its sign and top payload bits and stays quiet, as kvquant.hip
     const uint32_t b = __float_as_uint(x);
     if ((b & 0x7F800000u) == 0x7F800000u && (b & 0x007FFFFFu) != 0)
@@ -353,15 +364,10 @@ __device__ __forceinline__ float quantize_lanes(float v, int j, bool live, uint3
         float d, q;
         uint16_t mbits = 0;
         if constexpr (FMT == FHIP_KVQ_Q4_0) {
-            float a = fabsf(v) > 0.f ? fabsf(v) : 0.f, mx = fabsf(v) > 0.f ? v : 0.f;   // the value of largest magnitude, the first of equals
-            int at = j;
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) {
-                const float a2 = __shfl_xor(a, o), mx2 = __shfl_xor(mx, o);
-                const int at2 = __shfl_xor(at, o);
-                const bool take = a2 > a || (a2 == a && at2 < at);
-                a = take ? a2 : a; mx = take ? mx2 : mx; at = take ? at2 : at;
-            }
+            const float a = fabsf(v) > 0.f ? fabsf(v) : 0.f, amax = half32_max(a);          // the value of largest magnitude, the first of equals
+            const int half = __lane_id() & 32;
+            const uint32_t at = (uint32_t)(__builtin_amdgcn_ballot_w64(a == amax) >> half), neg = (uint32_t)(__builtin_amdgcn_ballot_w64(v < 0.f) >> half);
+            const float mx = neg & (at & 0u - at) ? -amax : amax;
             d = mx / -8.0f;
             const float inv = d != 0.f ? 1.0f / d : 0.f;
             q = floorf(v * inv + 8.5f);
@@ -372,7 +378,7 @@ __device__ __forceinline__ float quantize_lanes(float v, int j, bool live, uint3
             q = floorf((v - mn) * inv + 0.5f);
             mbits = kv_f16_bits(mn);
         }
-        const int c = kv_code(q, 0.f, 15.f), c2 = __shfl_xor(c, 16);
+        const int c = kv_code(q, 0.f, 15.f), c2 = __builtin_amdgcn_permlane16_swap((uint32_t)c, (uint32_t)c, false, false)[1];   // in the lower row the upper one's
         const uint16_t dbits = kv_f16_bits(d);
         if (live) {
             if (j < 16) ((uint8_t*)codes)[b * 16 + j] = (uint8_t)(c | (c2 << 4));
@@ -476,7 +482,7 @@ __global__ __launch_bounds__(256) void qkv_post_kvq_kernel(QkvPostParams p, KvqS
     }
 }
 
-// The same with the rows for heads of 64 or 128 dims rotated whole in the split-half layout, in registers: HD = 128 as qkv_post128_kernel holds a head (a lane's two
+// The same with the rows for heads of 64 or 128 dims rotated whole in the split-half layout, in registers: HD = 128 as qkv_post_heads_kernel holds a head (a lane's two
 // values are a pair), HD = 64 a value a lane, its pair's other one 32 lanes away. A wave takes HPW consecutive heads of a token. A prompt's layer on a quantized
 // cache was four launches here (post-processing, stores, both caches' rows), 3 - 4 us each; stacks of 42 ... 191 rows, us: 42 x 3584, one layer behind 581 rows 209 -> 195,
 // 86 x 3072 298 -> 281, 93 x 1280, four layers 460 -> 424, 139 x 2560, three 565 -> 543; 937 x 4608, four layers, 3081 -> 3071.
@@ -1627,12 +1633,14 @@ int launch_qkv_post(const float* qkv, const float* bias, const float* q_norm, co
     p.cap = (uint32_t)cap; p.eps = eps; p.rate = rope_rate(n_rot, base); p.kv_packed = kv_packed ? 1 : 0;
     const size_t per_tok = (size_t)(n_head + 2 * n_kv);
     if (t > 0x7FFFFFFFull || (t * per_tok + 3) / 4 > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post: too many rows for one launch");
-    // eight heads a wave once that leaves the CUs some four waves each; a token or two needs all the waves it can have
-    const size_t hpw = t * ((per_tok + 7) / 8) >= 4 * (size_t)device_cus() ? 8 : 1;
-    if (hd == 128 && n_rot == 128 && !interleaved) {
+    // Four heads a wave once that leaves the CUs some four waves each; a token or two needs all the waves it can have. us, one | two | four | eight heads
+    // of 128: 139 rows of 40 4.6 | 4.7 | 4.1 | 5.0; 276 of 32 5.1 | 4.8 | 4.5 | 5.7; 509 of 56 9.8 | 8.2 | 7.6 | 8.4; 699 of 80 16.9 | 12.6 | 12.0 | 12.9
+    if ((hd == 64 || hd == 128) && n_rot == hd && !interleaved) {
+        const size_t hpw = t * ((per_tok + 3) / 4) >= 4 * (size_t)device_cus() ? 4 : 1;
         const dim3 grid((unsigned)((t * ((per_tok + hpw - 1) / hpw) + 3) / 4));
-        if (hpw == 8) hipLaunchKernelGGL(qkv_post128_kernel<8>, grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL(qkv_post128_kernel<1>, grid, dim3(256), 0, s, p);
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p); };
+        if (hd == 128) hpw == 4 ? go(qkv_post_heads_kernel<128, 4>) : go(qkv_post_heads_kernel<128, 1>);
+        else hpw == 4 ? go(qkv_post_heads_kernel<64, 4>) : go(qkv_post_heads_kernel<64, 1>);
     } else {
         hipLaunchKernelGGL(qkv_post_kernel, dim3((unsigned)((t * per_tok + 3) / 4)), dim3(256), 0, s, p);
     }
@@ -1644,16 +1652,16 @@ template <int FMT>
 static int post_kvq(const QkvPostParams& p, const KvqStore& st, KvqRows rows, hipStream_t s) {
     const size_t t = p.t, per_tok = (size_t)(p.n_head + 2 * p.n_kv), past = rows.past * ((size_t)p.n_kv * p.hd / 4) * 2, past_wgs = (past + 255) / 256;
     const bool whole = rows.k && (p.hd == 64 || p.hd == 128) && p.n_rot == p.hd && !p.interleaved;
-    // heads a wave: as in launch_qkv_post
-    const size_t hpw = whole && t * ((per_tok + 7) / 8) >= 4 * (size_t)device_cus() ? 8 : 1, grid = (t * ((per_tok + hpw - 1) / hpw) + 3) / 4;
+    // Two heads a wave: us, one | two | four | eight on Q8_0 (Q4_0 and Q4_1 alike): 42 rows of 32 + 8 + 8 heads of 64 5.1 | 4.9 | 5.0 | 8.3, 276 of 16 + 8 + 8 of 128
+    // 6.5 | 6.6 | 7.2 | 12.1, 509 of 40 + 8 + 8 of 128 11.8 | 10.8 | 11.1 | 16.1, 699 of 64 + 8 + 8 of 128 18.6 | 15.6 | 15.9 | 20.1 (a key or value head is a chain of a microsecond).
+    const size_t hpw = whole ? 2 : 1, grid = (t * ((per_tok + hpw - 1) / hpw) + 3) / 4;
     if (t * per_tok > 0x7FFFFFFFull || grid + past_wgs > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "qkv_post_kvq: too many rows for one launch");
     rows.post_wgs = (unsigned)grid;
     const dim3 g((unsigned)(grid + past_wgs)), wg(256);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, wg, 0, s, p, st, rows); };
     if (!rows.k) go(qkv_post_kvq_kernel<FMT, false>);
     else if (!whole) go(qkv_post_kvq_kernel<FMT, true>);
-    else if (p.hd == 128) hpw == 8 ? go(qkv_post_rows_kernel<FMT, 128, 8>) : go(qkv_post_rows_kernel<FMT, 128, 1>);
-    else hpw == 8 ? go(qkv_post_rows_kernel<FMT, 64, 8>) : go(qkv_post_rows_kernel<FMT, 64, 1>);
+    else p.hd == 128 ? go(qkv_post_rows_kernel<FMT, 128, 2>) : go(qkv_post_rows_kernel<FMT, 64, 2>);
     return check_hip(hipGetLastError(), "qkv_post_kvq launch");
 }
 int launch_qkv_post_kvq(int fmt, const float* qkv, const float* bias, const float* q_norm, const float* k_norm, const uint32_t* d_pos,
