@@ -16,7 +16,7 @@
 // row's blocks. (Loaded one row per lane of sixteen and exchanged with v_permlane32_swap and v_permlane16_swap instead,
 // neighbouring lanes ask for different cache lines: 34816 x 5120 Q4_0 at 4 rows 40.8 us against 36.8.)
 //
-// The activations of a pass of P groups (16 blocks, 512 columns each) are quantised once per workgroup into LDS, laid out as the A
+// A workgroup has R of the activation rows. Those of a pass of P groups (16 blocks, 512 columns each) are quantised once per workgroup into LDS, laid out as the A
 // operands; an item of work is (tile of 16 weight rows, group) and the waves share the pass's items evenly. The group sums go
 // to LDS and are added there in the row's group order, so neither the number of passes nor the dealing shows in the bits.
 //
@@ -231,6 +231,7 @@ struct WideParams {
     const float* x;        // [T, cols]
     float* y;              // [T, N]
     int T, N, cols;
+    int R;                 // activation rows per workgroup, blockIdx.y of them before its own
     size_t row_bytes;
     int units, NG;         // blocks of a row; 16-block groups of a row
     int P, passes;         // groups per pass
@@ -261,6 +262,12 @@ __global__ void __launch_bounds__((64 * max_waves<F, E>())) gemv_wide_kernel(Wid
     const int tid = threadIdx.x, lane = tid & 63, W = (int)(blockDim.x >> 6);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g4 = lane >> 4, c = lane & 15;
+    {                                                     // the workgroup's activation rows
+        const int first = (int)blockIdx.y * p.R;
+        p.T = p.T - first < p.R ? p.T - first : p.R;
+        p.x += (size_t)first * p.cols;
+        p.y += (size_t)first * p.N;
+    }
     const int row0 = (int)blockIdx.x * p.tiles * 16;
     if (row0 >= p.N) return;                              // (the launcher sends no such workgroup)
     int nrows = p.N - row0;
@@ -524,9 +531,8 @@ __global__ void __launch_bounds__((64 * max_waves<F, E>())) gemv_wide_kernel(Wid
     }
 }
 
-template <int E>
-size_t lds_of(int P, int tiles, int passes, int W, int image, WideParams* p) {
-    size_t o = (size_t)P * 16 * unit_stride<E>();
+size_t lds_of(int E, int P, int tiles, int passes, int W, int image, WideParams* p) {
+    size_t o = (size_t)P * 16 * (NP * 128 * E + 8);
     o = (o + 15) & ~(size_t)15;
     const size_t scales = o; o += (size_t)P * 16 * 4 * E * 4;
     const size_t sums = o; o += (size_t)P * 16 * 4 * E * 4;
@@ -541,43 +547,85 @@ size_t lds_of(int P, int tiles, int passes, int W, int image, WideParams* p) {
     return o;
 }
 
+// How a launch of t rows is laid out with R of them a workgroup.
+struct WidePlan { int R, E, tiles, P, passes, W; unsigned grid, row_groups; };
+constexpr int pairs_of(int R) { return R <= 4 ? 1 : R <= 8 ? 2 : 4; }
+WidePlan wide_plan(int rows, int NG, int t, int R, int image, bool big, int cus, size_t lds_max) {
+    WidePlan q;
+    q.R = R; q.E = pairs_of(R);
+    q.row_groups = (unsigned)((t + R - 1) / R);
+    // one workgroup per CU, those of a row group each with the same number of 16-row tiles, at most sixteen (their sums lie in LDS beside the planes)
+    const int share = cus > (int)q.row_groups ? cus / (int)q.row_groups : 1, all = (rows + 15) / 16, rounds = (all + share * 16 - 1) / (share * 16);
+    q.tiles = (all + share * rounds - 1) / (share * rounds);
+    q.grid = (unsigned)((all + q.tiles - 1) / q.tiles);
+    // as many groups a pass as fit, the passes of equal size; a wave for every item of a pass, eight at least (they all quantise)
+    const int most = q.E == 1 ? 16 : q.E == 4 && big ? 8 : 12;
+    auto waves = [&](int P) { const int n = q.tiles * P; return n < 8 ? 8 : (n > most ? most : n); };
+    q.passes = 0;
+    const size_t fixed = lds_of(q.E, 0, q.tiles, 2, most, image, nullptr), each = lds_of(q.E, 1, q.tiles, 2, most, image, nullptr) - fixed;
+    const int fit = lds_max > fixed ? (int)((unsigned)(lds_max - fixed) / (unsigned)each) : 0;       // of that many a pass all fit, and perhaps of some more
+    for (int n = fit > 0 ? (NG + fit) / (fit + 1) : 1; n <= NG && !q.passes; n++) {
+        q.P = (NG + n - 1) / n;
+        if (lds_of(q.E, q.P, q.tiles, n, waves(q.P), image, nullptr) <= lds_max) q.passes = n;
+    }
+    if (!q.passes) return q;
+    q.passes = (NG + q.P - 1) / q.P;
+    q.W = waves(q.P);
+    return q;
+}
+
+// us, on a weight of `mb` megabytes: a launch, per pass its barriers and first loads, the quantiser (rows x groups over the waves), the items (issue of the
+// waves that share a SIMD), and the weight once for every row group. The constants are the best fit over 400 products of 3 .. 16 rows, 512 .. 34816 x
+// 1024 .. 17408, seven formats, in every R: 11 % rms.
+float wide_us(const WidePlan& q, float mb, int cus) {
+    const float quantise = (NP == 3 ? 0.62f : 0.46f) * (q.R * q.P) / q.W, item = (NP == 3 ? 1.19f : 1.f) * (q.E == 1 ? 0.056f : q.E == 2 ? 0.107f : 0.19f) * q.W;
+    const unsigned rounds = (q.grid * q.row_groups + (unsigned)cus - 1) / (unsigned)cus;
+    return 3.1f + rounds * q.passes * (2.6f + quantise + (q.tiles * q.P + q.W - 1) / q.W * item) + 0.16f * mb * q.row_groups;
+}
+
 template <class F, int E>
-int launch_wide(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
+int launch_wide(const fhip_weight* w, const float* d_x, size_t t, const WidePlan& q, size_t lds_max, float* d_y, hipStream_t s) {
     WideParams p;
     p.W = w->d_raw; p.x = d_x; p.y = d_y;
-    p.T = (int)t; p.N = (int)w->rows; p.cols = (int)w->cols; p.row_bytes = w->row_bytes;
+    p.T = (int)t; p.R = q.R; p.N = (int)w->rows; p.cols = (int)w->cols; p.row_bytes = w->row_bytes;
     p.units = (int)(w->cols / 32);
     p.NG = (p.units + 15) / 16;
-    const long long cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
-    const size_t lds_max = fhip::device_lds_bytes() > 0 ? fhip::device_lds_bytes() : 65536;
-    // one workgroup per CU, each with the same number of 16-row tiles, at most sixteen (their sums lie in LDS beside the planes)
-    const long long all = ((long long)w->rows + 15) / 16, rounds = (all + cus * 16 - 1) / (cus * 16);
-    p.tiles = (int)((all + cus * rounds - 1) / (cus * rounds));
-    // as many groups a pass as fit, the passes of equal size; a wave for every item of a pass, eight at least (they all quantise)
-    auto waves = [&](int P) { const int n = p.tiles * P; return n < 8 ? 8 : (n > max_waves<F, E>() ? max_waves<F, E>() : n); };
-    p.passes = 0;
-    for (int n = 1; n <= p.NG && !p.passes; n++) {
-        p.P = (p.NG + n - 1) / n;
-        if (lds_of<E>(p.P, p.tiles, n, waves(p.P), F::IMAGE, nullptr) <= lds_max) p.passes = n;
-    }
-    if (!p.passes) return fhip::set_error(FHIP_ERR_SHAPE, "gemv_wide: a pass does not fit the workgroup's LDS");
-    p.passes = (p.NG + p.P - 1) / p.P;
-    const int W = waves(p.P);
-    const size_t lds = lds_of<E>(p.P, p.tiles, p.passes, W, F::IMAGE, &p);
+    p.tiles = q.tiles; p.P = q.P; p.passes = q.passes;
+    const size_t lds = lds_of(E, p.P, p.tiles, p.passes, q.W, F::IMAGE, &p);
     static bool lds_raised = false;
     if (!lds_raised) {  // workgroups may use more than the default 64 KiB of the CU's 160 KiB
         (void)hipFuncSetAttribute((const void*)gemv_wide_kernel<F, E>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max);
         (void)hipGetLastError();
         lds_raised = true;
     }
-    const unsigned grid = (unsigned)((all + p.tiles - 1) / p.tiles);
-    hipLaunchKernelGGL((gemv_wide_kernel<F, E>), dim3(grid), dim3(64 * W), lds, s, p);
+    hipLaunchKernelGGL((gemv_wide_kernel<F, E>), dim3(q.grid, q.row_groups), dim3(64 * q.W), lds, s, p);
     return fhip::check_hip(hipGetLastError(), "gemv_wide launch");
 }
 
+// The rows of a batch by one workgroup or by up to four, each with its share of them and of the CUs: each then quantises fewer rows and holds fewer pairs a lane, and
+// tiles too few for the CUs meet more of these, for the weight once more a group. Dealt out where the estimate is 5 % under that of one group. us, one | two | three |
+// four groups, 24 bits: IQ4_XS 1636 x 13824 at 16 rows 55.2 | 32.7 | 31.6 | 25.0, MXFP4 1145 x 8160 at 8 20.3 | 13.7 | 13.2 | 16.2, 5433 x 14048 at 16 78.8 | 54.5 | 57.4 | 60.0,
+// Q4_0 918 x 3680 at 5 9.6 | 8.2 | 7.7 | 7.7; not: Q4_1 29831 x 2688 at 16 41.0 | 45.6 | 60.7 | 56.2, MXFP4 22048 x 2592 at 7 (16 bits) 19.2 | 22.2 | 34.6 | 39.6. Over
+// 500 other products 0.86 of the time in the mean, six of them 3 .. 9 % slower; the best choice of the four would give 0.845.
 template <class F>
 int launch_wide_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
-    return t <= 4 ? launch_wide<F, 1>(w, d_x, t, d_y, s) : t <= 8 ? launch_wide<F, 2>(w, d_x, t, d_y, s) : launch_wide<F, 4>(w, d_x, t, d_y, s);
+    const int cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
+    const size_t lds_max = fhip::device_lds_bytes() > 0 ? fhip::device_lds_bytes() : 65536;
+    const int NG = ((int)(w->cols / 32) + 15) / 16;
+    const float mb = (float)w->rows * (float)w->row_bytes * 1e-6f;
+    WidePlan best = wide_plan((int)w->rows, NG, (int)t, (int)t, F::IMAGE, F::BIG, cus, lds_max);
+    if (!best.passes) return fhip::set_error(FHIP_ERR_SHAPE, "gemv_wide: a pass does not fit the workgroup's LDS");
+    float us = wide_us(best, mb, cus) / 1.05f;
+    for (int groups = 2; us > 7.f && groups <= 4 && groups <= (int)t; groups++) {   // (not the shortest, which the fit does not tell apart; 0.1 us of the host)
+        const WidePlan q = wide_plan((int)w->rows, NG, (int)t, ((int)t + groups - 1) / groups, F::IMAGE, F::BIG, cus, lds_max);
+        const float u = q.passes ? wide_us(q, mb, cus) : us;
+        if (u < us) { us = u; best = q; }
+    }
+    switch (best.E) {
+        case 1: return launch_wide<F, 1>(w, d_x, t, best, lds_max, d_y, s);
+        case 2: return launch_wide<F, 2>(w, d_x, t, best, lds_max, d_y, s);
+        default: return launch_wide<F, 4>(w, d_x, t, best, lds_max, d_y, s);
+    }
 }
 
 }  // namespace

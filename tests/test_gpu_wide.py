@@ -42,6 +42,19 @@ def test_same_bits_as_single_rows(F, ty, rows, cols):
         assert same(got, one[:m]), m
 
 
+@pytest.mark.parametrize("ty,rows,cols", [(Q4_1, 530, 8192), (MXFP4, 2100, 11040), (IQ4_NL, 5200, 8224), (IQ4_XS, 900, 4096)])
+def test_rows_dealt_out_to_several_workgroups(F, ty, rows, cols):
+    # few tiles or long rows: two to four groups of activation rows, the last one short (13 = 4 + 4 + 4 + 1, 5 = 3 + 2), one tile a workgroup and several
+    from ferric_amd.synth import synth_weights
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, cols), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(rows).standard_normal((16, cols)).astype(np.float32)
+    x[12, 64:96] = np.float32(1e30)
+    one = singles_of(F, qm, x)
+    for m in (5, 6, 7, 10, 13, 16):
+        assert same(F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows), one[:m]), m
+
+
 @pytest.mark.parametrize("ty,rows,cols,m", [(Q5_1, 12300, 2080, 3), (IQ4_NL, 12289, 2048, 4), (Q8_0, 1200, 7040, 4)])
 def test_three_and_four_rows_of_large_weights(F, ty, rows, cols, m):
     from ferric_amd.synth import synth_weights
