@@ -1060,7 +1060,10 @@ void launch_attn_combine(const float* part, int n_head, int hd, int splits, floa
 // Before that, at that shape, us, values on f32 matrix instructions for six query heads and more, the dot-product kernel for fewer: 5 query
 // heads a KV head 38.3, 8: 33.9; head size 64, 4: 23.0. Error against f64 (2-norm, relative, eighteen shapes) no larger in any:
 // 2.2e-7 .. 2.5e-7 before, 1.4e-7 .. 1.8e-7 with the combine launch's present order.
-// Q4_1 is left to the kernel above: the minimum as a product of its own cost 2 % more error.
+// Q4_1: codes less 7.5 (an addition each) and, in place of the minimum, what 7.5 stands for, which is next to nothing where a block's values lie evenly about
+// zero: then neither term takes bits from the other. A score begins with those times the sums of the query's dims, a value's sum ends with their weighted
+// sum. Against the dot-product kernel, 252 products, error against f64 (2-norm) 0.95 of that (codes less 8 0.97, and 1.04 on zero-mean rows; the minimum itself 1.02); us, that -> this, with the
+// combine launch: 8 query heads on each of 8 KV heads of 128, 14413 keys 35.7 -> 16.2, 5 on 8 at 32768 42.0 -> 24.4, 5 on 8 of 64 at 9000 15.8 -> 10.4, 3 on 4 of 64 at 5200 9.5 -> 8.4.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct __attribute__((packed, aligned(8))) U4A8 { u32x4 v; };
@@ -1069,7 +1072,7 @@ union Frag { uint32_t w[4]; bf16x8 v; };
 // the upper halves of two f32: two bf16 (exact where the lower halves are zero)
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
 
-// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16. 4-bit formats: less 8, and a sixteenth (v_cvt_off_f32_i4 makes that of a two's complement nibble in one
+// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16. 4-bit formats: less 8 (Q4_1: 7.5), and a sixteenth (v_cvt_off_f32_i4 makes that of a two's complement nibble in one
 // instruction, where the byte, its conversion and the 8 were three; the scales carry the 16, so every bit is the same). 128 x 8 KV heads of 5, 32768 keys, with the combine launch 23.1 -> 21.2 us,
 // 4 KV heads of 8 16.5 -> 15.6, heads of 64 16.4 -> 15.3: 804 -> 613 vector instructions a round beside its softmax.
 template <int FMT>
@@ -1084,7 +1087,7 @@ __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) 
         } else {
             const uint32_t x = (w[i] ^ 0x88888888u) >> shift;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_cvt_off_f32_i4((int)(j % 3 ? (x >> (8 * j)) & 255u : x >> (8 * j)));
+            for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_cvt_off_f32_i4((int)(j % 3 ? (x >> (8 * j)) & 255u : x >> (8 * j))) + (FMT == FHIP_KVQ_Q4_1 ? 0.03125f : 0.f);
         }
         f.w[2 * i] = upper_halves(v[0], v[1]);
         f.w[2 * i + 1] = upper_halves(v[2], v[3]);
@@ -1103,11 +1106,15 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     constexpr int CW = Q8 ? 8 : 4;                                      // code words of a block
     constexpr int LR = NB * CW / 4, KL = LONG_KEYS * LR / 64;           // lanes that request a row's key codes, 16 bytes each; requests of a round
     constexpr int KROW = 16 * LR + 16;                                  // bytes of a row in LDS: sixteen rows' same 8 bytes lie in different banks
-    static_assert(FMT == FHIP_KVQ_Q8_0 || FMT == FHIP_KVQ_Q4_0, "");
+    constexpr bool MIN = FMT == FHIP_KVQ_Q4_1;
+    constexpr float HALF = MIN ? 0.03125f : 0.f;                        // half a step, in sixteenths
+    constexpr int SW = MIN ? NB : NB / 2;                               // words of a row's scales (Q4_1: scale and minimum a word)
     __shared__ float sm_m[LONG_WAVES][8], sm_l[LONG_WAVES][8];
     constexpr int COLS = SPL ? 16 : 8;
     __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][COLS][HD + 4];    // rows four banks apart
     __shared__ __attribute__((aligned(16))) float sm_d[LONG_WAVES][NB][64];   // rows 0 .. 31 the keys' scales, 32 .. 63 the values'
+    __shared__ __attribute__((aligned(16))) float sm_min[MIN ? LONG_WAVES : 1][NB][64];   // MIN: what code 7.5 stands for, the minimum and as many steps
+    __shared__ float sm_qs[NB][16];                                     // MIN: the sum of block j's dims of column n's query
     __shared__ __attribute__((aligned(16))) uint8_t sm_k[LONG_WAVES][LONG_KEYS * KROW];   // a round's key codes, row by row
     __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of column n's query at lane n + 16 g, three bf16 each
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1124,7 +1131,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     // What a round of 32 keys reads: key codes, scales (lanes 0 .. 31 the keys', 32 .. 63 the values'), and the value codes of block pair i at
     // key 16 t + 4 g + r: two units a lane (a unit is what a lane's A row of one block takes at a key: a half word, Q8_0, or a byte), units 2 n and 2 n + 1
     // of the pair's 32, so that lanes 0 .. 7 have the pair's first block and the others its second (pair_up).
-    struct Round { u32x4 k[KL]; uint32_t sc[NB / 2], v[NB / 2][NT][4]; } ra;
+    struct Round { u32x4 k[KL]; uint32_t sc[SW], v[NB / 2][NT][4]; } ra;
     constexpr uint32_t STEP = LONG_KEYS * LONG_WAVES;
     auto request_k = [&](Round& R, uint32_t kt) {
         kt = min(kt, k1 - 1u);
@@ -1133,9 +1140,9 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
         for (int i = 0; i < KL; i++)
             R.k[i] = ((const U4A8*)(qc.k_codes + ((size_t)(kt + min((uint32_t)(i * (64 / LR) + lane / LR), last)) * nblk + (size_t)kvh * NB) * CW + 4 * (lane % LR)))->v;
         const size_t b = ((size_t)(kt + min((uint32_t)(lane & 31), last)) * nblk + (size_t)kvh * NB);
-        const uint32_t* sp = (const uint32_t*)((lane < 32 ? qc.k_scales : qc.v_scales) + b);
+        const uint32_t* sp = (const uint32_t*)((lane < 32 ? qc.k_scales : qc.v_scales) + (MIN ? 2 * b : b));
 #pragma unroll
-        for (int i = 0; i < NB / 2; i++) R.sc[i] = sp[i];
+        for (int i = 0; i < SW; i++) R.sc[i] = sp[i];
     };
     const uint32_t row_b = (uint32_t)nblk * (CW * 4);                   // bytes from a row's codes to the next row's
     auto load_units = [&](const char* p) -> uint32_t { return Q8 ? *(const uint32_t*)p : (uint32_t)*(const uint16_t*)p; };
@@ -1190,6 +1197,12 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
         if (j >= NB) return;
         float x[8];
         load_dims<8>(row + 32 * j + 8 * gg, x);
+        if constexpr (MIN) {
+            float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+            sum = dpp_add<0xB1, 0xF>(sum);      // over the quad, the block's four k-groups
+            sum = dpp_add<0x4E, 0xF>(sum);
+            if (gg == 0) sm_qs[j][col] = sum;
+        }
 #pragma unroll
         for (int t = 0; t < 3; t++) {
             sm_q[j][t][col + 16 * gg] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
@@ -1197,9 +1210,11 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             for (int i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);   // exact
         }
     };
-    if (wave < NB && n >= (SPL ? 3 * gq : gq))                          // columns without a query
+    if (wave < NB && n >= (SPL ? 3 * gq : gq)) {                        // columns without a query
 #pragma unroll
         for (int t = 0; t < 3; t++) sm_q[wave][t][lane] = make_uint4(0u, 0u, 0u, 0u);
+        if (MIN && g == 0) sm_qs[wave][n] = 0.f;
+    }
     if constexpr (FUSED) {
         const int njobs = gq + (owner ? 2 : 0);
         const uint32_t pos = *len_dev;
@@ -1244,15 +1259,23 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     for (int j = 0; j < NB; j++)
 #pragma unroll
         for (int i = 0; i < 2; i++) run[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float qs[NB], floors[NB];               // MIN: sums of the query's dims; weighted sums of the values' minima over the lane's keys
+#pragma unroll
+    for (int j = 0; j < NB; j++) { qs[j] = MIN ? sm_qs[j][n] : 0.f; floors[j] = 0.f; }
 
     // a round; more: its registers take the wave's next one as they come free
     auto round = [&](Round& R, uint32_t kt, auto more) {
         const uint32_t last = k1 - 1u - kt;
 #pragma unroll
-        for (int i = 0; i < NB / 2; i++) {
+        for (int i = 0; i < SW; i++) {
             const float lo = __half2float(__ushort_as_half((uint16_t)R.sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(R.sc[i] >> 16)));
-            sm_d[wave][2 * i][lane] = Q8 ? lo : 16.0f * lo;             // (4-bit codes are sixteenths)
-            sm_d[wave][2 * i + 1][lane] = Q8 ? hi : 16.0f * hi;
+            if constexpr (MIN) {
+                sm_d[wave][i][lane] = 16.0f * lo;
+                sm_min[wave][i][lane] = fmaf(7.5f, lo, hi);
+            } else {
+                sm_d[wave][2 * i][lane] = Q8 ? lo : 16.0f * lo;         // (4-bit codes are sixteenths)
+                sm_d[wave][2 * i + 1][lane] = Q8 ? hi : 16.0f * hi;
+            }
         }
 #pragma unroll
         for (int i = 0; i < KL; i++) *(u32x4*)&sm_k[wave][(i * (64 / LR) + lane / LR) * KROW + 16 * (lane % LR)] = R.k[i];
@@ -1264,6 +1287,16 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
         for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) p[t][r] = 0.f;
+        if constexpr (MIN) {                    // before the products: the smaller terms first
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const f32x4 least = *(const f32x4*)&sm_min[wave][j][16 * t + 4 * g];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) p[t][r] = fmaf(least[r], qs[j], p[t][r]);
+                }
+        }
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             Frag qf[3];
@@ -1331,6 +1364,10 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             for (int j = 0; j < NB; j++)
 #pragma unroll
                 for (int i = 0; i < 2; i++) run[j][i] *= corr;
+            if constexpr (MIN) {
+#pragma unroll
+                for (int j = 0; j < NB; j++) floors[j] *= corr;
+            }
         }
         m = m_new;
         uint32_t vw[2][4];                      // [block of the pair]: the codes of keys 16 (e / 2) + 4 g + 2 (e % 2) and the next, a half word each
@@ -1342,6 +1379,10 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                 const f32x4 d = *(const f32x4*)&sm_d[wave][j][32 + 16 * t + 4 * g];
 #pragma unroll
                 for (int r = 0; r < 4; r++) x[4 * t + r] = p[t][r] * d[r];
+                if constexpr (MIN) {
+                    const f32x4 least = *(const f32x4*)&sm_min[wave][j][32 + 16 * t + 4 * g];
+                    floors[j] += fmaf(p[t][0], least[0], p[t][1] * least[1]) + fmaf(p[t][2], least[2], p[t][3] * least[3]);
+                }
             }
             if (j % 2 == 0)
 #pragma unroll
@@ -1356,7 +1397,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                     if constexpr (Q8) { lo = (float)(int8_t)(w >> (8 * i)); hi = (float)(int8_t)(w >> (16 + 8 * i)); }
                     else {
                         const uint32_t x = (w ^ 0x88888888u) >> (4 * i);
-                        lo = __builtin_amdgcn_cvt_off_f32_i4((int)x); hi = __builtin_amdgcn_cvt_off_f32_i4((int)(x >> 16));
+                        lo = __builtin_amdgcn_cvt_off_f32_i4((int)x) + HALF; hi = __builtin_amdgcn_cvt_off_f32_i4((int)(x >> 16)) + HALF;
                     }
                     a[i].w[e] = upper_halves(lo, hi);
                 }
@@ -1396,6 +1437,15 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     if (lane < gq) { sm_m[wave][lane] = m; sm_l[wave][lane] = l; }
+    if constexpr (MIN) {                    // to one of the query's columns
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            floors[j] += __shfl_xor(floors[j], 16);
+            floors[j] += __shfl_xor(floors[j], 32);
+#pragma unroll
+            for (int i = 0; i < 2; i++) run[j][i] += n < gq ? floors[j] : 0.f;
+        }
+    }
     if (n < (SPL ? 3 * gq : gq)) {
 #pragma unroll
         for (int j = 0; j < NB; j++)
@@ -1518,7 +1568,7 @@ int launch_attn_kvq(int g, int hd, dim3 grid, const KvqLaunch& a, int gq, bool w
 // 48.8 | 46.5 (in the launch 18.4 | 18.4, 21.4 | 22.7, 49.6 | 49.2). Four: 8 KV heads of 128, Q8_0 14.0 | 16.0, 16.6 | 19.1, 30.3 | 36.0; five 14.5 | 18.8, 17.2 | 21.3, 31.4 | 40.7.
 // Key codes are read eight bytes at a time; a lane's offset inside a round's rows is kept in 32 bits (n_kv).
 bool attn_long_takes(int fmt, int g, int n_kv, const uint32_t* k_codes) {
-    if (fmt == FHIP_KVQ_Q4_1 || g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
+    if (g > 8 || n_kv > 65535 || ((uintptr_t)k_codes & 7) != 0) return false;
     return g >= 3;
 }
 // Half the splits of the kernels above, about one workgroup a CU, and never the one that needs no combine launch. 98 shapes of one to sixteen KV heads, 5200 .. 32768 keys: as many
@@ -1818,7 +1868,10 @@ static int launch_attention_over_kvq(const char* who, int fmt, const float* q, c
             if (lng) launch_attn_long_kvq<FHIP_KVQ_Q4_0>(g, hd, grid, a);
             else rc = launch_attn_kvq<FHIP_KVQ_Q4_0>(G, hd, grid, a, gq, wide);
             break;
-        case FHIP_KVQ_Q4_1: rc = launch_attn_kvq<FHIP_KVQ_Q4_1>(G, hd, grid, a, gq, wide); break;
+        case FHIP_KVQ_Q4_1:
+            if (lng) launch_attn_long_kvq<FHIP_KVQ_Q4_1>(g, hd, grid, a);
+            else rc = launch_attn_kvq<FHIP_KVQ_Q4_1>(G, hd, grid, a, gq, wide);
+            break;
         default: return set_error(FHIP_ERR_ARG, "%s: unknown KV format %d", who, fmt);
     }
     if (rc) return rc;

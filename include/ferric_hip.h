@@ -353,7 +353,7 @@ int fhip_kvq_append2(int fmt, const float* d_k, const float* d_v, size_t src_row
  * is loaded (the use the reference chose the block layout for and left unbuilt, kvquant.rs:30-37, qwen3.rs:897-905: it
  * materialises `dequantize()` of the whole history per layer and step and attends over that). The values that enter the
  * softmax are exactly fhip_kvq_dequantize_rows', so the result has the bits of fhip_decode_attention_ex over the dequantized
- * rows -- behind more than 5120 rows of a Q8_0 or Q4_0 cache with three or more query heads per KV head its value to f32
+ * rows -- behind more than 5120 rows of a cache with three or more query heads per KV head its value to f32
  * rounding, the sums being formed on the matrix cores in another order (there an infinite query value or block scale makes NaN of outputs
  * that are infinite or NaN elsewhere) -- at 8.5 / 4.5 / 5 bits per value of traffic instead of 32 + 32 written and read back. */
 int fhip_decode_attention_kvq(int fmt, const float* d_q, const uint32_t* d_k_codes, const uint32_t* d_k_scales, const uint32_t* d_v_codes,

@@ -275,6 +275,13 @@ def test_long_caches_by_cut_columns_and_by_query_columns(F, Q, K, fmt, nh, nkv, 
     test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, fmt, nh, nkv, hd, rows, lengths)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,rows,lengths", [
+    (5, 1, 64, 5121, (5121, 97, 1)), (16, 2, 64, 6150, (6150, 5000)), (8, 1, 128, 7000, (7000, 6999)), (10, 2, 128, 9001, (9001, 33)), (21, 3, 128, 5200, (5200,)), (3, 1, 64, 5121, (257,))])
+def test_long_caches_of_blocks_with_a_minimum(F, Q, K, nh, nkv, hd, rows, lengths):
+    """Q4_1 on the long-cache kernel, at the same edges and the same bar: rows off zero, where a block's minimum carries most of its values, and about it."""
+    test_attention_over_long_caches_on_the_matrix_cores(F, Q, K, 2, nh, nkv, hd, rows, lengths)
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("nkv,g,n", [(171, 3, 700), (300, 3, 511), (511, 3, 290), (171, 6, 257), (171, 8, 31)])
 def test_long_caches_of_many_kv_heads_in_the_fewest_splits(F, Q, K, fmt, nkv, g, n):
@@ -323,6 +330,12 @@ def test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, fmt, nkv, g, hd, n
         r[n - 1] = own
     want = D.decode_attention(raw[0, :nh * hd], *(K.roundtrip(r, n, width, fmt) for r in rows), nh, nkv, 0, 0.0).reshape(-1)
     assert np.abs(got[1][0] - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nkv,g,hd,n", [(8, 5, 128, 33), (8, 3, 64, 1), (5, 8, 128, 8340), (171, 8, 128, 258), (300, 6, 128, 31)])
+def test_the_token_s_row_of_blocks_with_a_minimum(F, Q, K, nkv, g, hd, n):
+    """The same on a Q4_1 cache, fused and not."""
+    test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, 2, nkv, g, hd, n)
 
 
 def test_k_and_v_rows_stored_by_one_launch(F, Q, K):
