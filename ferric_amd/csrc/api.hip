@@ -1192,9 +1192,9 @@ static int norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_
     if (((uintptr_t)d_x | (uintptr_t)d_resid | (uintptr_t)d_norm_w | (uintptr_t)d_x_out) & 15)
         return set_error(FHIP_ERR_ARG, "fhip_norm_matmul_q: x, resid, norm_w and x_out must be 16-byte aligned");
     const size_t n_ff = swiglu ? w->rows / 2 : 0;
-    fhip::NormParams np{d_norm_w, d_resid, d_resid ? d_x_out : nullptr, eps};   // without a residual there is no sum to store
+    fhip::NormParams np{d_norm_w, d_resid, d_resid ? d_x_out : nullptr, eps, d_count, by};   // without a residual there is no sum to store
     rc = fhip::launch_gemv_norm(w, d_x, d_y, n_ff, np, (hipStream_t)stream);
-    if (rc != fhip::NORM_NOT_FUSED) return rc || !d_count ? rc : fhip::launch_u32_add(d_count, 1, by, (hipStream_t)stream);
+    if (rc != fhip::NORM_NOT_FUSED) return rc;
     if ((rc = fhip::launch_rmsnorm(d_x, d_resid, d_norm_w, 1, w->cols, eps, d_resid ? d_x_out : nullptr, d_h_scratch, (hipStream_t)stream, d_count, by))) return rc;
     return fhip::launch_gemv(w, d_h_scratch, 1, d_y, n_ff, (hipStream_t)stream);
 }

@@ -69,6 +69,8 @@ struct NormParams {
     const float* resid;
     float* x_out;
     float eps;
+    uint32_t* count;       // += by, on the way (null: nothing)
+    uint32_t by;
 };
 constexpr int NORM_NOT_FUSED = -100;   // internal: launch_gemv_norm launched nothing, run the two steps apart
 

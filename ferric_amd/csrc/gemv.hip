@@ -643,7 +643,9 @@ struct GemvParams {
     float* x_out;
     float eps;
     uint32_t red_off;    // byte offset in LDS of 64 floats: four partial sums of squares per wave
-    int row_wgs;         // workgroups that own rows; the launch may hold one more, which only stores x + resid
+    int row_wgs;         // workgroups that own rows; the launch may hold one more, which only stores x + resid and counts
+    uint32_t* count;     // fused norm: += by, by that workgroup (null: nothing)
+    uint32_t by;
 };
 
 // Threads per workgroup allowed for M activation rows (register budget: 1024 -> 128 VGPRs, 640 -> 168, 512 -> 256).
@@ -731,6 +733,7 @@ __global__ void __launch_bounds__(max_threads<F>(M)) gemv_stream_kernel(GemvPara
             xb0.x += rsb.x; xb0.y += rsb.y; xb0.z += rsb.z; xb0.w += rsb.w;
             *(float4*)(p.x_out + e0) = xa0; *(float4*)(p.x_out + e0 + 4) = xb0;
         }
+        if (p.count && tid == 0) *p.count += p.by;
         return;
     }
     const int rg = (int)(ww & 15u);                       // row group within the workgroup
@@ -1376,9 +1379,9 @@ int launch_one_u(const fhip_weight* w, const float* d_x, float* d_y, size_t out_
     const size_t nrg = (out_rows + rpg - 1) / rpg;
     int G = nrg >= slots ? Gcap : (int)((nrg + cus - 1) / cus);
     // Large weights (16 rows per row group and more, one round): rows dealt round-robin in chunks of 4 over the row groups of
-    // all CUs (one CU is left to the workgroup that stores x + resid when the fused norm asks for that).
+    // all CUs (one CU is left to the workgroup that stores x + resid or counts when the fused norm asks for that).
     p.rr = 0; p.nrg = 0; p.kfull = 0; p.rem = 0;
-    const bool spare = norm && norm->x_out && cus > 1;
+    const bool spare = norm && (norm->x_out || norm->count) && cus > 1;
     if ((F::RR || (F::RR_ONE_ROW && U == 1)) && rpg >= 16 && rounds == 1 && p.sel.npairs <= 1) {
         const size_t nrg_all = (size_t)(cus - (spare ? 1 : 0)) * G, S = nrg_all * 4;
         const size_t kfull = out_rows / S, rem = out_rows % S;
@@ -1410,7 +1413,7 @@ int launch_one_u(const fhip_weight* w, const float* d_x, float* d_y, size_t out_
     const size_t per_wg = (size_t)G * rpg;
     const size_t grid = p.rr ? (size_t)p.nrg / G : (out_rows + per_wg - 1) / per_wg;
     size_t lds = lds_bytes<F, M, SWIGLU>(w->cols, p.NG, G, rpg);
-    p.norm_w = nullptr; p.resid = nullptr; p.x_out = nullptr; p.eps = 0.f; p.red_off = 0;
+    p.norm_w = nullptr; p.resid = nullptr; p.x_out = nullptr; p.eps = 0.f; p.red_off = 0; p.count = nullptr; p.by = 0;
     if (norm) {
         if (M != 1 || w->cols > (size_t)8 * 64 * WPR * G) return fhip::NORM_NOT_FUSED;   // nothing launched
         p.norm_w = norm->norm_w; p.resid = norm->resid; p.x_out = norm->x_out; p.eps = norm->eps;
@@ -1426,9 +1429,12 @@ int launch_one_u(const fhip_weight* w, const float* d_x, float* d_y, size_t out_
         S = S < 4 ? 4 : S;
         p.S = norm || S > nwaves ? nwaves : S;
     }
-    const size_t launch_wgs = grid + ((norm && norm->x_out && grid < (size_t)cus) ? 1 : 0);
-    hipLaunchKernelGGL(kernel, fhip::sel_grid((unsigned)launch_wgs, p.sel), dim3(64 * WPR * G), lds, s, p);
-    return fhip::check_hip(hipGetLastError(), "gemv launch");
+    // The word of fhip_norm_matmul_q_count goes with the workgroup beside them (a launch of its own is 3.8 us and the gap before it), where there is a CU for it.
+    const bool beside = norm && (norm->x_out || norm->count) && grid < (size_t)cus;
+    if (beside) { p.count = norm->count; p.by = norm->by; }
+    hipLaunchKernelGGL(kernel, fhip::sel_grid((unsigned)(grid + (beside ? 1 : 0)), p.sel), dim3(64 * WPR * G), lds, s, p);
+    const int rc = fhip::check_hip(hipGetLastError(), "gemv launch");
+    return rc || !norm || !norm->count || beside ? rc : fhip::launch_u32_add(norm->count, 1, norm->by, s);
 }
 
 template <class F, int M, bool SWIGLU>

@@ -243,8 +243,8 @@ class Qwen3Decoder:
         # a default-arm layer; short caches, whose attention splits nothing, need no combine launch behind it
         short = self.ws is None
         self.launches_per_layer = (7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) - (1 if short else 0)
-        # per token beside the layers: the head and the position word's increment, which the final norm's launch or the last residual add takes with it (the
-        # final norm is inside the head's mat-vec, but for a head of 128 MB and more: there a launch of its own costs less than the wider workgroups the fused norm needs)
+        # per token beside the layers, at most: the head and the final norm, which takes the position word's increment with it and is inside the head's mat-vec but for
+        # a head of 128 MB and more (there a launch of its own costs less than the wider workgroups the fused norm needs)
         self.launches_per_token_extra = (2 if self.fuse_norm else 3) if lm_head is not None else 1
         self._graph = None
 
