@@ -110,15 +110,20 @@ size_t device_lds_bytes() { return g_lds; }
 // what is left of a batch, one or two rows, takes the dot-product kernel.
 // Batches of the 32-value formats from here on go up to sixteen rows at a time through the kernel that multiplies on the 16 x 16 x 32
 // int8 matrix instruction (gemv_wide.hip: the same bits per row); what is left of a batch goes on as a batch of its own. Its cost is the quantiser's, per activation row and workgroup,
-// plus the weight once; the dot-product kernel's is a launch and the weight per four rows. us, cold, dot-product | wide, three rows:
-// IQ4_NL 1024 x 5120 7.9 | 9.7, 4096 x 4096 10.0 | 9.7, 9728 x 2560 12.5 | 11.1, 34816 x 5120 42.9 | 33.6, Q4_0 4096 x 4096 8.9 | 9.4; four: Q4_0 1024 x 5120 9.3 | 9.7,
-// 1946 x 1504 6.5 | 6.5, 4096 x 4096 13.1 | 9.6, 34816 x 5120 42.3 | 32.6; five: 1024 x 1024 8.8 | 5.7, 1024 x 5120 13.5 | 11.2, 34816 x 5120 62.9 | 38.9; sixteen: IQ4_NL
-// 1467 x 1760 37.1 | 12.1, Q4_0 4096 x 4096 50.9 | 20.9, 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up to 5120 columns: three, dot-product |
+// plus the weight once; the dot-product kernel's is a launch and the weight per pass, of one to four rows by how many of them its registers hold at that width. us, dot-product |
+// wide, each by itself and the weights in the Infinity Cache, three rows at 24 bits: IQ4_NL 1024 x 5120 7.4 | 9.0, 1024 x 16384 20.3 | 22.0, 2000 x 8192 16.6 | 12.2, 3000 x 5632
+// 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1); four: Q4_0 520 x 1600 9.2 | 5.8,
+// 700 x 2048 10.0 | 5.6, 1024 x 5120 8.8 | 7.8, 1024 x 7168 11.1 | 9.5, 2000 x 4000 11.6 | 7.9; at 16 bits 500 x 6144 10.9 | 8.4, 1500 x 5120 8.1 | 8.6, 1024 x 7168 9.2 | 10.3, 500 x 16000
+// 15.6 | 17.4. Cold: Q4_0 34816 x 5120 at four rows 42.3 | 32.6, at five 62.9 | 38.9; sixteen: IQ4_NL 1467 x 1760 37.1 | 12.1, Q4_0 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up
+// to 5120 columns: three, dot-product |
 // wide, 4096 x 4096 9.6 | 10.7; four, four-row | wide, 34816 x 5120 48.4 | 57.5, 5120 x 5120 15.1 | 17.5, 2048 x 4096 10.1 | 10.8 (but 4096 x 4096 12.5 | 11.0, 12288 x 4096 22.8 | 19.6).
 bool takes_wide(const fhip_weight* w, size_t t) {
     const size_t weights = w->rows * w->cols;
     if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
-    if (t < 3 || (t == 3 && weights < ((size_t)24 << 20)) || (t == 4 && weights < ((size_t)8 << 20))) return false;
+    if (t < 3) return false;
+    const bool q8 = w->type == FHIP_Q8_0, whole = w->planes == 3 && !q8;     // 24 bits
+    if (t == 3 && weights < ((size_t)(whole && w->cols <= 8192 ? 12 : 24) << 20)) return false;
+    if (t == 4 && !whole && (q8 || w->cols > 6144) && weights < ((size_t)8 << 20)) return false;
     return w->planes == 3 ? gemv_wide_supports_p3(w, t < 16 ? t : 16) : gemv_wide_supports_p2(w, t < 16 ? t : 16);
 }
 bool g_quad_matvec = true, g_generic_forced = false;

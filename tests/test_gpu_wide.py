@@ -76,6 +76,21 @@ def test_the_rows_behind_the_last_sixteen_go_where_a_batch_of_them_would(F, ty, 
     assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
 
 
+@pytest.mark.parametrize("ty,rows,cols,m,at24,at16", [(Q4_0, 520, 1600, 4, "WIDE", "WIDE"), (MXFP4, 20, 352, 4, "WIDE", "WIDE"), (MXFP4, 300, 7168, 4, "WIDE", "DOT"), (IQ4_NL, 1600, 8192, 3, "WIDE", "DOT"),
+                                                       (IQ4_NL, 1500, 8192, 3, "DOT", "DOT"), (Q5_1, 1400, 9216, 3, "DOT", "DOT")])
+def test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16):
+    from ferric_amd.synth import synth_weights
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(4).standard_normal((m, cols)).astype(np.float32)
+    kernel = at24 if qm.matvec_precision(0) == 24 else at16
+    if kernel == "WIDE":
+        x[2, 5] = np.float32(1e38)      # a run that block fixed point cannot hold, in one row
+    xt = F.Tensor.from_vec(x, x.shape)
+    assert route(F, qm, xt, m) == [(ROUTES[kernel], m)]
+    assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
+
+
 def test_mxfp4_blocks_that_may_overflow(F):
     """Scale bytes from 252 on: inf weights, and finite ones near the top of f32, beside ordinary blocks."""
     rng = np.random.default_rng(21)
