@@ -448,8 +448,8 @@ int fhip_qkv_post_attention_kvq(int fmt, const float* d_qkv, const float* d_bias
  * rounding (the sum of squares is added in a different order), not the same bits. No single counterpart in the reference. */
 int fhip_norm_matmul_q(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
                        float* d_h_scratch, int swiglu, float* d_y, void* stream);
-/* The same, and *d_count += by (a decode step's position word) before the call's last launch ends: inside the norm's launch where that is one of its own, by one more
- * otherwise. No other argument may share memory with d_count. */
+/* The same, and *d_count += by (a decode step's position word) before the call's last launch ends: inside the norm's launch where that is one of its own, beside the mat-vec's
+ * workgroups where the norm is inside it and a CU is free, by one more launch otherwise. No other argument may share memory with d_count. */
 int fhip_norm_matmul_q_count(const fhip_weight* w, const float* d_x, const float* d_resid, const float* d_norm_w, float eps, float* d_x_out,
                              float* d_h_scratch, int swiglu, float* d_y, uint32_t* d_count, uint32_t by, void* stream);
 
