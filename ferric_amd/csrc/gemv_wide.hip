@@ -33,6 +33,7 @@
 #include "fixed_point.hpp"
 #include "lut16.hpp"
 
+#include <algorithm>
 #include <hip/hip_fp16.h>
 
 #if FHIP_GEMV_PLANES == 2
@@ -571,14 +572,20 @@ WidePlan wide_plan(int rows, int NG, int t, int R, int image, bool big, int cus,
     if (!q.passes) return q;
     q.passes = (NG + q.P - 1) / q.P;
     q.W = waves(q.P);
+    // More waves than items, as many as there may be, where each has two pieces to quantise and their images fit: the quantiser is what a workgroup of few tiles
+    // does longest. us, a wave an item | all: Q5_1 993 x 4320 at 8 rows 13.6 | 12.1, Q4_0 1458 x 17248 at 7 41.8 | 37.2, 1312 x 13280 at 14 33.1 | 29.4. With
+    // fewer pieces the barriers of more waves cost as much (IQ4_XS 1029 x 1792 at 4 rows 5.5 | 6.1), and where the images take a pass's room it has more of
+    // them (Q5_1 949 x 2368 at 10 rows 12.6 | 15.7).
+    if (q.W < most && R * q.P >= 2 * q.W && lds_of(q.E, q.P, q.tiles, q.passes, most, image, nullptr) <= lds_max) q.W = most;
     return q;
 }
 
 // us, on a weight of `mb` megabytes: a launch, per pass its barriers and first loads, the quantiser (rows x groups over the waves), the items (issue of the
-// waves that share a SIMD), and the weight once for every row group. The constants are the best fit over 400 products of 3 .. 16 rows, 512 .. 34816 x
+// waves with items that share a SIMD), and the weight once for every row group. The constants are the best fit over 400 products of 3 .. 16 rows, 512 .. 34816 x
 // 1024 .. 17408, seven formats, in every R: 11 % rms.
 float wide_us(const WidePlan& q, float mb, int cus) {
-    const float quantise = (NP == 3 ? 0.62f : 0.46f) * (q.R * q.P) / q.W, item = (NP == 3 ? 1.19f : 1.f) * (q.E == 1 ? 0.056f : q.E == 2 ? 0.107f : 0.19f) * q.W;
+    const float quantise = (NP == 3 ? 0.62f : 0.46f) * (q.R * q.P) / q.W, working = std::max(8, std::min(q.W, q.tiles * q.P)),
+                item = (NP == 3 ? 1.19f : 1.f) * (q.E == 1 ? 0.056f : q.E == 2 ? 0.107f : 0.19f) * working;
     const unsigned rounds = (q.grid * q.row_groups + (unsigned)cus - 1) / (unsigned)cus;
     return 3.1f + rounds * q.passes * (2.6f + quantise + (q.tiles * q.P + q.W - 1) / q.W * item) + 0.16f * mb * q.row_groups;
 }
@@ -603,10 +610,12 @@ int launch_wide(const fhip_weight* w, const float* d_x, size_t t, const WidePlan
 }
 
 // The rows of a batch by one workgroup or by up to four, each with its share of them and of the CUs: each then quantises fewer rows and holds fewer pairs a lane, and
-// tiles too few for the CUs meet more of these, for the weight once more a group. Dealt out where the estimate is 5 % under that of one group. us, one | two | three |
+// tiles too few for the CUs meet more of these, for the weight once more a group. Dealt out where the estimate is 8 % under that of one group. us, one | two | three |
 // four groups, 24 bits: IQ4_XS 1636 x 13824 at 16 rows 55.2 | 32.7 | 31.6 | 25.0, MXFP4 1145 x 8160 at 8 20.3 | 13.7 | 13.2 | 16.2, 5433 x 14048 at 16 78.8 | 54.5 | 57.4 | 60.0,
 // Q4_0 918 x 3680 at 5 9.6 | 8.2 | 7.7 | 7.7; not: Q4_1 29831 x 2688 at 16 41.0 | 45.6 | 60.7 | 56.2, MXFP4 22048 x 2592 at 7 (16 bits) 19.2 | 22.2 | 34.6 | 39.6. Over
-// 500 other products 0.86 of the time in the mean, six of them 3 .. 9 % slower; the best choice of the four would give 0.845.
+// 1173 products of 3 .. 16 rows 0.83 of the time of one group with a wave an item (or of the dot-product kernel, where that had them), ten 3 .. 10 % slower; over 633 of them 0.80, and
+// the best of all layouts would give 0.78. (At 5 % and a wave an item these 633 take 0.80 too, but seventeen are 3 .. 15 % slower: Q4_0 2057 x 4096 at four rows 8.4 -> 9.9, whose 129
+// tiles are one more than half the CUs.)
 template <class F>
 int launch_wide_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {
     const int cus = fhip::device_cus() > 0 ? fhip::device_cus() : 256;
@@ -615,7 +624,7 @@ int launch_wide_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y
     const float mb = (float)w->rows * (float)w->row_bytes * 1e-6f;
     WidePlan best = wide_plan((int)w->rows, NG, (int)t, (int)t, F::IMAGE, F::BIG, cus, lds_max);
     if (!best.passes) return fhip::set_error(FHIP_ERR_SHAPE, "gemv_wide: a pass does not fit the workgroup's LDS");
-    float us = wide_us(best, mb, cus) / 1.05f;
+    float us = wide_us(best, mb, cus) / 1.08f;
     for (int groups = 2; us > 7.f && groups <= 4 && groups <= (int)t; groups++) {   // (not the shortest, which the fit does not tell apart; 0.1 us of the host)
         const WidePlan q = wide_plan((int)w->rows, NG, (int)t, ((int)t + groups - 1) / groups, F::IMAGE, F::BIG, cus, lds_max);
         const float u = q.passes ? wide_us(q, mb, cus) : us;

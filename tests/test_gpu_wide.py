@@ -55,6 +55,23 @@ def test_rows_dealt_out_to_several_workgroups(F, ty, rows, cols):
         assert same(F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows), one[:m]), m
 
 
+@pytest.mark.parametrize("ty,rows,cols", [(Q5_1, 993, 4320), (Q4_1, 40, 11040), (Q8_0, 257, 5152), (IQ4_NL, 17, 17408)])
+def test_more_waves_than_items(F, ty, rows, cols):
+    # one tile a workgroup and 9 to 16 groups of 512 columns, the last one short: waves that quantise and have no item, in one pass and in several
+    from ferric_amd.synth import synth_weights
+    qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 7), ty, rows, cols)
+    qm.batch_policy(F.BATCH_F32_MATVEC)
+    x = np.random.default_rng(cols).standard_normal((16, cols)).astype(np.float32)
+    x[3, -32:] = np.float32(1e30)
+    one = singles_of(F, qm, x)
+    xt = F.Tensor.from_vec(x, x.shape)
+    # (four rows of this few weights: at 24 bits, Q8_0 apart; else they are the dot-product kernel's, which promises no row's bits beside the run of 1e30)
+    four = qm.matvec_precision(0) == 24 and ty != Q8_0
+    for m in (4, 5, 8, 9, 14, 16) if four else (5, 8, 9, 14, 16):
+        assert route(F, qm, xt, m) == [(ROUTES["WIDE"], m)]
+        assert same(F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows), one[:m]), m
+
+
 @pytest.mark.parametrize("ty,rows,cols,m", [(Q5_1, 12300, 2080, 3), (IQ4_NL, 12289, 2048, 4), (Q8_0, 1200, 7040, 4)])
 def test_three_and_four_rows_of_large_weights(F, ty, rows, cols, m):
     from ferric_amd.synth import synth_weights
