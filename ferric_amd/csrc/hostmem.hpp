@@ -24,7 +24,7 @@ void* device_malloc_beside_captures(size_t n);                       // hipMallo
 // transfer.hip: copies through pinned memory of the library's own; both directions and the host-to-host unpackers
 constexpr size_t H2D_STAGED = (size_t)640 << 10;   // up to here copy_h2d has read its source when it returns
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s);
-int upload(void* d, const void* h, size_t n, hipStream_t s);     // copy_h2d that has read its source when it returns; refused in a capture
+int upload(void* d, const void* h, size_t n, hipStream_t s);     // copy_h2d that has read its source when it returns, and from H2D_STAGED on brought it over; refused in a capture
 int copy_d2h(void* h, const void* d, size_t n, hipStream_t s);   // synchronises; refused in a capture
 int dequant_host(uint32_t type, const uint8_t* h_raw, size_t nblocks, size_t block_values, size_t block_bytes, float* h_out);   // synchronises
 

@@ -6,7 +6,7 @@
 // that a small kernel on the caller's own stream reads or writes directly; the kernel's workgroups confirm in pinned words of
 // their own, which a host thread polls without a call into the runtime.
 //   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time); an upload of 1.25 to 12 MB goes
-//                   through several, one filled while the one before crosses the bus
+//                   through several, one filled while the one before crosses the bus, and has arrived when the call returns, as longer ones have
 //   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
 //                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise (one and a half into fresh memory); more is cut into chunks, each
 //                   copied out of its slot by a worker thread while the next ones cross (page faults of the destination
@@ -443,9 +443,9 @@ namespace fhip {
 
 // A source longer than a slot's IN_BYTES in chunks, by the calling thread, one crossing the bus while the next goes into its slot: the source has been read when this returns, while the
 // last chunks still cross. *took false: there were not enough slots at once, and nothing was done.
-// us on an idle device, the runtime's copy, which is waited for | this: returned 1.5 MB 66 | 29, 2.4 92 | 45, 3.3 118 | 62, 5.0 152 | 90, 10.4 350 | 285; arrived, with the wait's own
-// 10, 1.5 MB 71 | 65, 2.4 97 | 85, 3.3 123 | 107, 5.0 157 | 153, 10.4 355 | 320. Shorter ones arrive later this way (0.7 MB 37 | 42, 1.0 47 | 55) and stay with the runtime. Chunks of
-// 448 KB cost their launches: 3.3 MB returned 89, arrived 127.
+// us on an idle device until the bytes have arrived, the runtime's copy | this, of a source that was sent before: 1.3 MB 60 | 57, 1.5 61 | 65, 1.9 69 | 77, 2.2 92 | 84, 3.3 118 | 107, 5.0
+// 154 | 155, 10.4 291 | 270, 12.5 343 | 320; of one that was not: 1.5 MB 75 | 71, 1.9 87 | 86, 2.2 103 | 91, 3.3 160 | 130. The first of a process 1.5 MB 6960 | 830, 10.4 9700 | 5000, and
+// the runtime's staging memory is as slow until 16 MB have gone through it (1.5 MB 560 | 70, 10.4 2300 | 400). Chunks of 448 KB cost their launches: 3.3 MB 127.
 static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStream_t s, bool* took) {
     const size_t count = (n + OUT_BYTES - 1) / OUT_BYTES, each = ((n + count - 1) / count + 255) & ~(size_t)255;
     Slot* q[SLOTS - SMALL_SLOTS];
@@ -492,16 +492,18 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     return rc;
 }
 
+// A source of more than IN_BYTES has arrived when this returns, whichever way it went: other streams may use it.
 int upload(void* d, const void* h, size_t n, hipStream_t s) {
     int rc = may_wait(s, "fhip_upload");
     if (rc) return rc;
+    bool kernels = false, took = false;
     if (n > IN_CHUNKS_FROM && n <= IN_CHUNKS_TO) {
-        bool kernels, took = false;
         if ((rc = for_kernels(d, n, h, "fhip_upload", &kernels))) return rc;
         Ring* r = kernels ? ring(&rc) : nullptr;
-        if (rc || (r && ((rc = upload_chunks(r, (uint8_t*)d, (const uint8_t*)h, n, s, &took)) || took))) return rc;
+        if (r) rc = upload_chunks(r, (uint8_t*)d, (const uint8_t*)h, n, s, &took);
+        if (rc) return rc;
     }
-    rc = copy_h2d(d, h, n, s);
+    if (!took) rc = copy_h2d(d, h, n, s);
     return rc || n <= IN_BYTES ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 

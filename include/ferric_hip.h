@@ -97,8 +97,8 @@ int fhip_free(void* d_ptr);
  * async on stream; a source of up to 640 KiB has been read when the call returns, unless the thread captures a stream: on a captured
  * stream the copy is recorded, and every replay reads the source */
 int fhip_memcpy_h2d(void* d_dst, const void* h_src, size_t nbytes, void* stream);
-/* The same with a source that has been read when the call returns, whatever its size (the copy itself is in stream order). FHIP_ERR_HIP while the
- * stream, or any stream by the calling thread, is captured. */
+/* The same with a source that has been read when the call returns, whatever its size. The copy is in stream order: up to 640 KiB it may still be under way
+ * (other streams wait for this one first), a longer one has arrived. FHIP_ERR_HIP while the stream, or any stream by the calling thread, is captured. */
 int fhip_upload(void* d_dst, const void* h_src, size_t nbytes, void* stream);
 /* synchronises stream before returning; FHIP_ERR_HIP while the stream, or any stream by the calling thread, is captured */
 int fhip_memcpy_d2h(void* h_dst, const void* d_src, size_t nbytes, void* stream);
