@@ -109,7 +109,7 @@ int launch_copy(const void* src, void* dst, size_t n, int units_per_thread, uint
 }
 
 struct Slot {
-    uint8_t* host = nullptr;     // SLOT_BYTES pinned: [OUT_BYTES][IN_BYTES]
+    uint8_t* host = nullptr;     // SLOT_BYTES pinned: [OUT_BYTES][IN_BYTES]; of a chunked upload's slots OUT_BYTES
     uint32_t* done = nullptr;    // MAX_WG pinned words, of a copy in parts the last part's ...
     uint32_t* early = nullptr;   // ... and (PARTS - 1) * MAX_WG for the parts before it
     uint32_t seq = 0;
@@ -183,7 +183,7 @@ struct Ring {                    // one per device
                 if ((*rc = fhip::check_hip(hipHostMalloc((void**)&words, SLOTS * PARTS * MAX_WG * sizeof(uint32_t), hipHostMallocPortable), "hipHostMalloc"))) return nullptr;
                 memset(words, 0, SLOTS * PARTS * MAX_WG * sizeof(uint32_t));
             }
-            if (!q.host && (*rc = fhip::check_hip(hipHostMalloc((void**)&q.host, SLOT_BYTES, hipHostMallocPortable), "hipHostMalloc"))) { q.host = nullptr; return nullptr; }
+            if (!q.host && (*rc = fhip::check_hip(hipHostMalloc((void**)&q.host, i < SMALL_SLOTS ? SLOT_BYTES : OUT_BYTES, hipHostMallocPortable), "hipHostMalloc"))) { q.host = nullptr; return nullptr; }
             q.done = words + i * PARTS * MAX_WG;
             q.early = q.done + MAX_WG;
             q.held = true;
@@ -442,7 +442,7 @@ int may_wait(hipStream_t s, const char* who) {
 namespace fhip {
 
 // A source longer than a slot's IN_BYTES in chunks, by the calling thread, one crossing the bus while the next goes into its slot: the source has been read when this returns, while the
-// last chunks still cross. *took false: there were not enough slots at once, and nothing was done.
+// last chunks still cross. *took false: there were not enough slots at once, or no pinned memory for them, and nothing was done.
 // us on an idle device until the bytes have arrived, the runtime's copy | this, of a source that was sent before: 1.3 MB 60 | 57, 1.5 61 | 65, 1.9 69 | 77, 2.2 92 | 84, 3.3 118 | 107, 5.0
 // 154 | 155, 10.4 291 | 270, 12.5 343 | 320; of one that was not: 1.5 MB 75 | 71, 1.9 87 | 86, 2.2 103 | 91, 3.3 160 | 130. The first of a process 1.5 MB 6960 | 830, 10.4 9700 | 5000, and
 // the runtime's staging memory is as slow until 16 MB have gone through it (1.5 MB 560 | 70, 10.4 2300 | 400). Chunks of 448 KB cost their launches: 3.3 MB 127.
@@ -451,12 +451,16 @@ static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStr
     Slot* q[SLOTS - SMALL_SLOTS];
     size_t have = 0;
     int rc = FHIP_OK;
-    while (have < count && !rc) {
+    while (have < count) {
         Slot* next = r->take(&rc, SLOTS, SMALL_SLOTS);
         if (!next) break;
         q[have++] = next;
     }
-    *took = !rc && have == count;
+    *took = have == count;
+    if (rc) {                               // the runtime's copy needs no slot, nor may the next launch be blamed for it
+        (void)hipGetLastError();
+        rc = FHIP_OK;
+    }
     for (size_t c = 0; c < count && *took && !rc; c++) {
         int wgs = 0;
         const size_t bytes = part(n, each, c);

@@ -48,3 +48,31 @@ def test_a_long_upload_has_arrived_when_it_returns(bus, n):
 def test_a_short_upload_waits_for_nobody(bus):
     d, a = upload(bus, 640 * KIB)
     assert not d.any() and bus.h_waiting(16) == 1 and bus.h_runtime_copies() == 0
+
+
+@pytest.mark.parametrize("slots", [0, 3])
+def test_an_upload_needs_no_pinned_memory(bus, slots):
+    """None left, or none left half way: the runtime's copy does it, as it did before there were slots for these sizes, and nothing of the failure stays behind."""
+    upload(bus, 100)
+    bus.h_no_more_pinned(slots * MIB)
+    d, a = upload(bus, 7 * MIB)
+    assert np.array_equal(d, a) and bus.h_runtime_copies() == 1 and bus.h_stale_error() == 0
+    if slots:
+        d, a = upload(bus, 3 * MIB)               # in the slots there are
+        assert np.array_equal(d, a) and bus.h_runtime_copies() == 1
+
+
+def test_slots_for_uploads_are_as_large_as_what_goes_through_them(bus):
+    upload(bus, 100)
+    before = bus.h_pinned()
+    upload(bus, 12 * MIB)
+    assert bus.h_pinned() - before == 12 * MIB
+
+
+def test_an_upload_without_slots_is_the_runtime_s(bus):
+    """Others hold them: too few for seven chunks, enough for two."""
+    bus.h_hold_upload_slots(7)
+    d, a = upload(bus, 7 * MIB)
+    assert np.array_equal(d, a) and bus.h_runtime_copies() == 1
+    d, a = upload(bus, 2 * MIB)
+    assert np.array_equal(d, a) and bus.h_runtime_copies() == 1
