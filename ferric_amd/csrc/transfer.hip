@@ -5,7 +5,7 @@
 // to fresh host memory 12.5 ms (a single thread taking page faults one by one). Here a copy goes through slots of pinned memory
 // that a small kernel on the caller's own stream reads or writes directly; the kernel's workgroups confirm in pinned words of
 // their own, which a host thread polls without a call into the runtime.
-//   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time); an upload of 1.25 to 12 MB goes
+//   to the device   up to H2D_STAGED the source is in a slot when the call returns, so nobody waits (3 us of host time); an upload of up to 12 MiB goes
 //                   through several, one filled while the one before crosses the bus, and has arrived when the call returns, as longer ones have
 //   to the host     up to a slot in one kernel that confirms part after part, the host copying one out while the next ones cross the bus
 //                   (608 KB, idle device: 26 us; 37 with one part and a stream synchronisation), up to three slots likewise (one and a half into fresh memory); more is cut into chunks, each
@@ -47,7 +47,7 @@ constexpr size_t IN_PARTS = (size_t)96 << 10;    // copies to the host from here
 constexpr int PARTS = 8;                         // at most
 constexpr size_t D2H_ALONE = 3 * OUT_BYTES;      // longer copies to the host are the workers' ...
 constexpr size_t D2H_ALONE_NEW = D2H_ALONE / 2;  // ... and those from here on whose destination has pages that nobody has touched
-constexpr size_t IN_CHUNKS_FROM = (size_t)1280 << 10, IN_CHUNKS_TO = (SLOTS - SMALL_SLOTS) * OUT_BYTES;   // uploads that the calling thread takes in chunks
+constexpr size_t IN_CHUNKS_TO = (SLOTS - SMALL_SLOTS) * OUT_BYTES;   // uploads up to there, from IN_BYTES on, the calling thread takes in chunks
 constexpr int WORKERS = 10;
 constexpr int MAX_DEVICES = 64;
 
@@ -441,13 +441,15 @@ int may_wait(hipStream_t s, const char* who) {
 
 namespace fhip {
 
-// A source longer than a slot's IN_BYTES in chunks, by the calling thread, one crossing the bus while the next goes into its slot: the source has been read when this returns, while the
-// last chunks still cross. *took false: there were not enough slots at once, or no pinned memory for them, and nothing was done.
-// us on an idle device until the bytes have arrived, the runtime's copy | this, of a source that was sent before: 1.3 MB 60 | 57, 1.5 61 | 65, 1.9 69 | 77, 2.2 92 | 84, 3.3 118 | 107, 5.0
-// 154 | 155, 10.4 291 | 270, 12.5 343 | 320; of one that was not: 1.5 MB 75 | 71, 1.9 87 | 86, 2.2 103 | 91, 3.3 160 | 130. The first of a process 1.5 MB 6960 | 830, 10.4 9700 | 5000, and
-// the runtime's staging memory is as slow until 16 MB have gone through it (1.5 MB 560 | 70, 10.4 2300 | 400). Chunks of 448 KB cost their launches: 3.3 MB 127.
+// A source longer than a slot's IN_BYTES in chunks, by the calling thread, one crossing the bus while the next goes into its slot; the last one's words say that all
+// have arrived. *took false: there were not enough slots at once, or no pinned memory for them, and nothing was done.
+// us on an idle device, the runtime's copy and hipStreamSynchronize | this, of a source that was sent before: 0.66 MB 30 | 30, 1.04 43 | 43, 1.1 64 | 46, 1.5 59 | 54, 1.9 66 | 63, 2.2 91 | 71,
+// 3.3 119 | 96, 5.0 154 | 131, 10.4 289 | 253, 12.5 343 | 312; of one that was not: 0.66 34 | 34, 1.04 52 | 46, 1.5 76 | 62, 1.9 87 | 73, 3.3 156 | 118. The first of a process 0.7 MB 6500 | 600,
+// 10.4 9700 | 5000, and the runtime's staging memory is slow until 16 MB have gone through it, from whatever call (0.7 MB 290, 1.1 400, 10.4 2300), so that sizes left to it
+// are slower the fewer others are: 56 prompt rows of 3072, 600 us a pass, took 842 where only uploads of up to 1 MiB still went that way.
+// Two chunks at least: 0.66 MB in one 3 us more. A unit a thread: with four 1.9 MB 8 us more, 5.0 14. hipStreamSynchronize in place of the words 6.
 static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStream_t s, bool* took) {
-    const size_t count = (n + OUT_BYTES - 1) / OUT_BYTES, each = ((n + count - 1) / count + 255) & ~(size_t)255;
+    const size_t slots = (n + OUT_BYTES - 1) / OUT_BYTES, count = slots < 2 ? 2 : slots, each = ((n + count - 1) / count + 255) & ~(size_t)255;
     Slot* q[SLOTS - SMALL_SLOTS];
     size_t have = 0;
     int rc = FHIP_OK;
@@ -465,8 +467,9 @@ static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStr
         int wgs = 0;
         const size_t bytes = part(n, each, c);
         memcpy(q[c]->host, h + c * each, bytes);
-        if (!(rc = launch_copy(q[c]->host, d + c * each, bytes, 4, q[c]->done, q[c]->seq + 1, s, &wgs))) { q[c]->seq++; q[c]->wgs = wgs; }
+        if (!(rc = launch_copy(q[c]->host, d + c * each, bytes, 1, q[c]->done, q[c]->seq + 1, s, &wgs))) { q[c]->seq++; q[c]->wgs = wgs; }
     }
+    if (*took && !rc) rc = await_words(q[count - 1]->done, q[count - 1]->seq, q[count - 1]->wgs, s);
     for (size_t i = 0; i < have; i++) r->release(q[i]);
     return rc;
 }
@@ -500,14 +503,14 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
 int upload(void* d, const void* h, size_t n, hipStream_t s) {
     int rc = may_wait(s, "fhip_upload");
     if (rc) return rc;
-    bool kernels = false, took = false;
-    if (n > IN_CHUNKS_FROM && n <= IN_CHUNKS_TO) {
+    if (n > IN_BYTES && n <= IN_CHUNKS_TO) {
+        bool kernels, took = false;
         if ((rc = for_kernels(d, n, h, "fhip_upload", &kernels))) return rc;
         Ring* r = kernels ? ring(&rc) : nullptr;
         if (r) rc = upload_chunks(r, (uint8_t*)d, (const uint8_t*)h, n, s, &took);
-        if (rc) return rc;
+        if (rc || took) return rc;
     }
-    if (!took) rc = copy_h2d(d, h, n, s);
+    rc = copy_h2d(d, h, n, s);
     return rc || n <= IN_BYTES ? rc : check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 

@@ -92,13 +92,19 @@ def _stream_handle(stream):
     return stream.handle if stream is not None else None
 
 
-H2D_STAGED = 640 << 10      # fhip_memcpy_h2d: a source of up to this many bytes has been read when the call returns
+H2D_STAGED = 640 << 10      # fhip_memcpy_h2d: a source of up to this many bytes has been read when the call returns; fhip_upload: a longer one has arrived
 
 
 def _upload(buf, a, stream=None):
     """A contiguous host array into a DeviceBuffer, in stream order; the array may go away afterwards (not inside a capture, whose
     replays would read it again)."""
     _lib.check(_lib.load().fhip_upload(buf.ptr, a.ctypes.data, a.nbytes, _stream_handle(stream)))
+
+
+def _arrived(a, stream=None):
+    """Waits until an array that has just been given to _upload is there for all streams."""
+    if a.nbytes <= H2D_STAGED:
+        _lib.check(_lib.load().fhip_stream_sync(_stream_handle(stream)))
 
 
 def _result(buf, shape):
@@ -121,7 +127,7 @@ class Tensor:
         assert a.size == int(np.prod(shape)), "from_vec: data does not match shape"
         t = Tensor(DeviceBuffer(a.nbytes), shape)
         _upload(t.buf, a, stream)
-        _lib.check(_lib.load().fhip_stream_sync(_stream_handle(stream)))    # a new tensor may be used on any stream
+        _arrived(a, stream)                       # a new tensor may be used on any stream
         return t
 
     @staticmethod
@@ -130,7 +136,7 @@ class Tensor:
         assert a.size == int(np.prod(shape))
         t = Tensor(DeviceBuffer(a.nbytes), shape, np.uint16)
         _upload(t.buf, a)
-        _lib.check(_lib.load().fhip_stream_sync(None))
+        _arrived(a)
         return t
 
     @staticmethod

@@ -61,18 +61,20 @@ def test_uploads_have_read_their_source(F, n, offset):
         assert np.array_equal(out[offset:offset + n], a) and (out[:offset] == 0xA5).all() and (out[offset + n:] == 0xA5).all(), busy
 
 
-@pytest.mark.parametrize("n", [640 * KIB + 1, 1280 * KIB + 1, 7 * MIB + 260, 12 * MIB + 1])
+@pytest.mark.parametrize("n", [640 * KIB + 1, MIB, MIB + 1, 7 * MIB + 260, 12 * MIB, 12 * MIB + 1])
 def test_a_long_upload_may_be_used_on_another_stream(F, n):
-    """Behind other work of its own: it has arrived when the call returns."""
+    """From an idle stream and behind other work: it has arrived when the call returns, also where the other stream has read what was there before."""
     lib, check = F._lib.load(), F._lib.check
-    a = np.random.default_rng(n).integers(0, 256, n, np.uint8)
-    buf, other, s, s2 = F.DeviceBuffer(n), F.DeviceBuffer(64 * MIB), F.Stream(), F.Stream()
-    for _ in range(4):
-        check(lib.fhip_memset(other.ptr, 1, 64 * MIB, s.handle))
-    check(lib.fhip_upload(buf.ptr, a.ctypes.data, n, s.handle))
-    out = np.empty(n, np.uint8)
-    check(lib.fhip_memcpy_d2h(out.ctypes.data, buf.ptr, n, s2.handle))
-    assert np.array_equal(out, a)
+    buf, copy, other, s, s2 = F.DeviceBuffer(n), F.DeviceBuffer(n), F.DeviceBuffer(64 * MIB), F.Stream(), F.Stream()
+    for k in range(6):
+        a = np.random.default_rng(n + k).integers(0, 256, n, np.uint8)
+        for _ in range(2 * (k % 3)):
+            check(lib.fhip_memset(other.ptr, 1, 64 * MIB, s.handle))
+        check(lib.fhip_upload(buf.ptr, a.ctypes.data, n, s.handle))
+        check(lib.fhip_memcpy_d2d(copy.ptr, buf.ptr, n, s2.handle))
+        out = np.empty(n, np.uint8)
+        check(lib.fhip_memcpy_d2h(out.ctypes.data, (copy if k % 2 else buf).ptr, n, s2.handle))
+        assert np.array_equal(out, a), k
 
 
 # a destination whose pages are made while its stream is busy: in parts, two and three slots, the workers; nothing around it is written

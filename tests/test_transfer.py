@@ -76,3 +76,9 @@ def test_an_upload_without_slots_is_the_runtime_s(bus):
     assert np.array_equal(d, a) and bus.h_runtime_copies() == 1
     d, a = upload(bus, 2 * MIB)
     assert np.array_equal(d, a) and bus.h_runtime_copies() == 1
+
+
+@pytest.mark.parametrize("n,by_runtime", [(640 * KIB, 0), (640 * KIB + 1, 0), (MIB, 0), (MIB + 1, 0), (12 * MIB, 0), (12 * MIB + 1, 1)])
+def test_who_takes_an_upload(bus, n, by_runtime):
+    upload(bus, n)
+    assert bus.h_runtime_copies() == by_runtime
