@@ -43,12 +43,13 @@ __device__ __forceinline__ float wave_sum(float v) {
 // Out = uint16_t: the normed rows as bf16, rounded as fhip_cvt_f32_bf16 rounds them -- what the matrix cores read, for a prompt: a
 // launch and a trip of the f32 rows through memory less per matmul. count: a word that gets `by` more beside the rows, a decode step's position, whose own launch
 // cost 2.5 us a token (null: none): eight layers behind 128 rows 634.4 -> 630.1 us a token, with the weights' trip under the row's.
+// AHEAD: the weights are requested with the row and held, which takes their trip out of a workgroup's chain, and up to 32 registers (norm_ahead).
 using fhip::pk_bf16;
 __device__ __forceinline__ void store_norm(float* out, size_t j, float4 v) { ((float4*)out)[j] = v; }
 __device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float4 v) { ((uint2*)out)[j] = make_uint2(pk_bf16(v.x, v.y), pk_bf16(v.z, v.w)); }
 __device__ __forceinline__ void store_norm(float* out, size_t j, float v) { out[j] = v; }
 __device__ __forceinline__ void store_norm(uint16_t* out, size_t j, float v) { out[j] = (uint16_t)(pk_bf16(v, 0.f) & 0xFFFFu); }
-template <int TPR, typename Out>
+template <int TPR, typename Out, bool AHEAD>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const float* __restrict__ b,
                                                       const float* __restrict__ weight, size_t rows, int d, float eps,
                                                       float* sum_out, Out* __restrict__ norm_out, uint32_t* count, uint32_t by) {   // sum_out may be a
@@ -63,20 +64,20 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
     const bool vec = (d & 3) == 0 && d <= 4 * NV * TPR && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)weight | (uintptr_t)sum_out | (uintptr_t)norm_out) & 15) == 0;
     float ms = 0.f;
     if (vec) {
-        // every load of the row is issued before the first use, so the row costs one memory round trip, not one per element (and the weights none behind the sum)
+        // every load of the row is issued before the first use, so the row costs one memory round trip, not one per element (and, AHEAD, the weights none behind the sum)
         const int nv = d >> 2;
-        float4 r[NV], w[NV];
+        float4 r[NV], w[AHEAD ? NV : 1];
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const int j = t + i * TPR;
             r[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (j < nv) {
                 r[i] = ((const float4*)(a + base))[j];
-                w[i] = ((const float4*)weight)[j];
+                if constexpr (AHEAD) w[i] = ((const float4*)weight)[j];
                 if (b) { const float4 y = ((const float4*)(b + base))[j]; r[i].x += y.x; r[i].y += y.y; r[i].z += y.z; r[i].w += y.w; }
             }
         }
-        asm volatile("" ::: "memory");
+        if constexpr (AHEAD) asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < NV; i++) ms = fmaf(r[i].x, r[i].x, fmaf(r[i].y, r[i].y, fmaf(r[i].z, r[i].z, fmaf(r[i].w, r[i].w, ms))));
         ms = wave_sum(ms);
@@ -91,8 +92,9 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* a, const floa
         for (int i = 0; i < NV; i++) {
             const int j = t + i * TPR;
             if (j < nv) {
+                const float4 wi = AHEAD ? w[AHEAD ? i : 0] : ((const float4*)weight)[j];
                 if (sum_out) ((float4*)(sum_out + base))[j] = r[i];
-                store_norm(norm_out + base, (size_t)j, make_float4(r[i].x * inv * w[i].x, r[i].y * inv * w[i].y, r[i].z * inv * w[i].z, r[i].w * inv * w[i].w));
+                store_norm(norm_out + base, (size_t)j, make_float4(r[i].x * inv * wi.x, r[i].y * inv * wi.y, r[i].z * inv * wi.z, r[i].w * inv * wi.w));
             }
         }
         return;
@@ -1604,19 +1606,21 @@ int launch_attn_fused_g(int hd, dim3 grid, hipStream_t s, const QkvPostParams& f
 
 namespace fhip {
 
+// The weights with the row (AHEAD) while every CU has at most four workgroups; beyond, its registers leave fewer of them on a CU. us, behind the sum | with the row: rmsnorm, 64 rows
+// of 4096 4.0 | 3.6, 256 of 2560 4.0 | 3.7, 1024 of 8192 11.6 | 10.7, 1500 of 1536 4.5 | 4.8, 2048 of 5120 12.9 | 13.7, 16384 of 768 16.4 | 19.4; sum, norm and bf16 rows, 1200 rows of
+// 2560 7.3 | 7.3, 1500 of 1536 5.5 | 6.7, 2048 of 2048 9.5 | 11.0, 2048 of 5120 21.3 | 23.3, 65536 of 64 (four rows a workgroup) 17.6 | 20.6.
+static bool norm_ahead(size_t grid) { return grid <= 4 * (size_t)(device_cus() > 0 ? device_cus() : 256); }
 template <typename Out>
 static int launch_rmsnorm_out(const float* a, const float* b, const float* weight, size_t rows, size_t d, float eps, float* sum_out, Out* norm_out,
                               hipStream_t s, uint32_t* count = nullptr, uint32_t by = 0) {
     if (rows == 0 || d == 0) return count ? launch_u32_add(count, 1, by, s) : FHIP_OK;
     if (d > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: row length exceeds 2^31");
-    if (d <= 512) {
-        size_t grid = (rows + 3) / 4;
-        if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<64, Out>), dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out, count, by);
-    } else {
-        if (rows > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
-        hipLaunchKernelGGL((rmsnorm_kernel<256, Out>), dim3((unsigned)rows), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out, count, by);
-    }
+    const size_t grid = d <= 512 ? (rows + 3) / 4 : rows;
+    if (grid > 0x7FFFFFFFull) return set_error(FHIP_ERR_SHAPE, "rmsnorm: too many rows for one launch");
+    const bool ahead = norm_ahead(grid);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, s, a, b, weight, rows, (int)d, eps, sum_out, norm_out, count, by); };
+    if (d <= 512) ahead ? go(rmsnorm_kernel<64, Out, true>) : go(rmsnorm_kernel<64, Out, false>);
+    else ahead ? go(rmsnorm_kernel<256, Out, true>) : go(rmsnorm_kernel<256, Out, false>);
     return check_hip(hipGetLastError(), "rmsnorm launch");
 }
 

@@ -52,6 +52,25 @@ def test_rmsnorm_and_add_rmsnorm(F, X, D):
         X.add_rmsnorm(xt, F.Tensor.from_vec(np.zeros(4, np.float32), (1, 4)), wt, 1e-5)
 
 
+# rows below and beyond which a norm requests its weights with the row (1024 workgroups, of a row or of four), by registers' worth of a row and its remainders
+@pytest.mark.parametrize("rows,d", [(1024, 516), (1025, 516), (1025, 5120), (1025, 8192), (4096, 64), (4097, 64), (4099, 500), (1100, 8196), (1030, 517)])
+def test_a_norm_s_bits_do_not_depend_on_how_many_rows_there_are(F, rows, d):
+    lib, rng = F._lib.load(), np.random.default_rng(d)
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    x, y, w = T(rng.standard_normal((rows, d)).astype(np.float32)), T(rng.standard_normal((rows, d)).astype(np.float32)), T(rng.standard_normal(d).astype(np.float32))
+
+    def norms(first, n):
+        at = lambda t, size: t.buf.ptr.value + first * d * size
+        o, s, h = F.Tensor.empty((n, d)), F.Tensor.empty((n, d)), F.Tensor.empty((n, d), np.uint16)
+        F._lib.check(lib.fhip_rmsnorm(at(x, 4), w.buf.ptr, n, d, 1e-6, o.buf.ptr, None))
+        F._lib.check(lib.fhip_add_rmsnorm_bf16(at(x, 4), at(y, 4), w.buf.ptr, n, d, 1e-6, s.buf.ptr, h.buf.ptr, None))
+        return [t.to_vec().reshape(n, d).view(np.uint16 if t is h else np.uint32) for t in (o, s, h)]
+    whole = norms(0, rows)
+    for first, n in ((0, 1), (rows - 9, 9), (rows // 2 & ~3, 64)):
+        for a, b in zip(whole, norms(first, n)):
+            assert np.array_equal(a[first:first + n], b), (first, n)
+
+
 def test_rope_variants(F, X, D):
     rng = np.random.default_rng(1)
     for t, heads, hd, base, off in [(1, 40, 128, 1e6, 0), (1, 48, 128, 1e6, 4095), (5, 8, 64, 1e4, 129), (3, 2, 8, 1e4, 7), (2, 3, 256, 5e5, 31999)]:

@@ -43,6 +43,18 @@ def attention(tmp_path_factory):
     return ask
 
 
+@pytest.fixture(scope="module")
+def decode(tmp_path_factory):
+    return C.CDLL(build(tmp_path_factory.mktemp("decode"), "decode_rules_harness.cpp", [], ["-shared", "-Wl,-Bsymbolic"]))
+
+
+def test_when_a_norm_requests_its_weights_with_the_row(decode):
+    """Both sides timed on 256 CUs, us by workgroups: weights behind the sum, with the row."""
+    timed = {64: (4.0, 3.6), 256: (4.0, 3.7), 1024: (11.6, 10.7), 1500: (5.5, 6.7), 2048: (21.3, 23.3), 16384: (17.6, 20.6)}
+    for grid, (behind, with_row) in timed.items():
+        assert bool(decode.h_norm_ahead(C.c_size_t(grid))) == (with_row < behind), grid
+
+
 @pytest.mark.parametrize("width", [64, 256])      # columns of a step (unpacked weights shared) and of a chunk (waves that unpack for themselves)
 def test_no_activation_is_read_from_behind_the_last(gemm, width):
     """Threads stage 16-byte pieces of whole steps or chunks of columns: rows and columns that do not exist are read from x all the same, those that do from where they are."""
