@@ -112,18 +112,30 @@ size_t device_lds_bytes() { return g_lds; }
 // int8 matrix instruction (gemv_wide.hip: the same bits per row); what is left of a batch goes on as a batch of its own. Its cost is the quantiser's, per activation row and workgroup,
 // plus the weight once; the dot-product kernel's is a launch and the weight per pass, of one to four rows by how many of them its registers hold at that width. us, dot-product |
 // wide, each by itself and the weights in the Infinity Cache, three rows at 24 bits: IQ4_NL 1024 x 5120 7.4 | 9.0, 1024 x 16384 20.3 | 22.0, 2000 x 8192 16.6 | 12.2, 3000 x 5632
-// 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1); four: Q4_0 520 x 1600 9.2 | 5.8,
-// 700 x 2048 10.0 | 5.6, 1024 x 5120 8.8 | 7.8, 1024 x 7168 11.1 | 9.5, 2000 x 4000 11.6 | 7.9; at 16 bits 500 x 6144 10.9 | 8.4, 1500 x 5120 8.1 | 8.6, 1024 x 7168 9.2 | 10.3, 500 x 16000
-// 15.6 | 17.4. Cold: Q4_0 34816 x 5120 at four rows 42.3 | 32.6, at five 62.9 | 38.9; sixteen: IQ4_NL 1467 x 1760 37.1 | 12.1, Q4_0 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up
-// to 5120 columns: three, dot-product |
+// 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1). Four, of small weights: where the
+// dot-product kernel needs two passes for four rows this one is ahead, Q4_0 560 x 1792 9.2 | 6.4, Q5_0 260 x 3616 9.8 | 8.9, MXFP4 258 x 3520 10.7 | 7.8, at 16 bits IQ4_XS 1498 x 2048 8.6 | 5.6
+// (but Q5_0 412 x 14336 19.6 | 21.8); where it has them in one it is behind, Q5_0 793 x 928 5.3 | 6.2, 696 x 4896 8.9 | 10.7, Q5_1 898 x 512 4.9 | 5.1, IQ4_NL 410 x 4480 8.2 | 9.1, at 16 bits
+// MXFP4 399 x 4256 7.1 | 8.3, Q5_0 92 x 4416 6.9 | 9.4, but at 24 bits over 1024 .. 3072 columns, Q4_0 338 x 2336 7.3 | 6.7, Q4_1 1234 x 2208 7.5 | 6.9 (formats with a minimum a block from 1536 on:
+// Q4_1 798 x 1376 5.8 | 6.2), over 6656 .. 7168, Q4_0 1024 x 7168 11.1 | 9.5, and IQ4_XS, 114 x 4352 7.9 | 7.3. Over 2963 products of four rows and up to 8 M weights 0.86 of the
+// dot-product kernel's time, two of them longer by more than 3 % (4 and 6 %; with this kernel for nearly all of them 0.83, but 408 longer, up to 1.35 times). At 16 bits and more than 6144 columns two passes
+// are ahead too: 1024 x 7168 9.2 | 10.3, 500 x 16000 15.6 | 17.4. Cold: Q4_0 34816 x 5120 at four rows 42.3 | 32.6, at five 62.9 | 38.9; sixteen: IQ4_NL 1467 x 1760 37.1 | 12.1, Q4_0
+// 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up to 5120 columns: three, dot-product |
 // wide, 4096 x 4096 9.6 | 10.7; four, four-row | wide, 34816 x 5120 48.4 | 57.5, 5120 x 5120 15.1 | 17.5, 2048 x 4096 10.1 | 10.8 (but 4096 x 4096 12.5 | 11.0, 12288 x 4096 22.8 | 19.6).
+static bool wide_for_four(const fhip_weight* w, bool whole) {      // of up to 8 M weights
+    const bool one_pass = (w->planes == 3 ? gemv_pass_rows_p3(w, 4, 0) : gemv_pass_rows_p2(w, 4, 0)) == 4;
+    if (!whole) return w->cols <= 6144 && !one_pass;
+    if (!one_pass) return w->type != FHIP_Q5_0 || w->cols <= 12288;
+    if (w->type == FHIP_Q5_0 || w->cols <= 1024) return false;
+    if (w->type == FHIP_IQ4_XS || (w->cols > 6656 && w->cols <= 7168)) return true;
+    return w->cols <= 3072 && (w->cols > 1536 || (w->type != FHIP_Q4_1 && w->type != FHIP_Q5_1));
+}
 bool takes_wide(const fhip_weight* w, size_t t) {
     const size_t weights = w->rows * w->cols;
     if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
     if (t < 3) return false;
     const bool q8 = w->type == FHIP_Q8_0, whole = w->planes == 3 && !q8;     // 24 bits
     if (t == 3 && weights < ((size_t)(whole && w->cols <= 8192 ? 12 : 24) << 20)) return false;
-    if (t == 4 && !whole && (q8 || w->cols > 6144) && weights < ((size_t)8 << 20)) return false;
+    if (t == 4 && weights < ((size_t)8 << 20) && (q8 || !wide_for_four(w, whole))) return false;
     return w->planes == 3 ? gemv_wide_supports_p3(w, t < 16 ? t : 16) : gemv_wide_supports_p2(w, t < 16 ? t : 16);
 }
 bool g_quad_matvec = true, g_generic_forced = false;

@@ -100,6 +100,7 @@ int launch_gemv(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_
     bool launch_gemv_wsum##sfx(const fhip_weight* w, const float* d_x, float* d_y, size_t out_rows, const struct SelParams& sel,      \
                                hipStream_t s, int* rc);                                                                              \
     void gemv_force_generic##sfx(bool on);                                                                                         \
+    int gemv_pass_rows##sfx(const fhip_weight* w, size_t left, size_t n_ff);                                                        \
     bool gemv_streams##sfx(const fhip_weight* w, size_t n_ff);                                                                      \
     bool gemv_quad_supports##sfx(const fhip_weight* w, size_t rows_x, size_t n_ff);                                                 \
     int launch_gemv_quad##sfx(const fhip_weight* w, const float* d_x, size_t rows_x, float* d_y, size_t n_ff, hipStream_t s);       \

@@ -1526,25 +1526,27 @@ int GEMV_EXPORT(launch_gemv)(const fhip_weight* w, const float* d_x, size_t rows
     }
 }
 
-// Whether launch_gemv runs this weight on the streaming kernel (and not on the shape-complete f32 kernel, whose sums round
-// differently): the four-row and the sixteen-row mat-vec, which promise the streaming kernel's bits, take a weight only then.
-bool GEMV_EXPORT(gemv_streams)(const fhip_weight* w, size_t n_ff) {
-    if (w->type == FHIP_Q4_K) return (n_ff ? max_batch<Q4K, true>(w, 1) : max_batch<Q4K, false>(w, 1)) > 0;
-    if (w->type == FHIP_Q6_K) return (n_ff ? max_batch<Q6K, true>(w, 1) : max_batch<Q6K, false>(w, 1)) > 0;
-    if (w->type == FHIP_Q5_K) return (n_ff ? max_batch<Q5K, true>(w, 1) : max_batch<Q5K, false>(w, 1)) > 0;
-    if (n_ff) return false;
+// Activation rows of a batch of `left` that one pass of launch_gemv over this weight takes; 0: the shape-complete f32 kernel has it.
+int GEMV_EXPORT(gemv_pass_rows)(const fhip_weight* w, size_t left, size_t n_ff) {
+    if (w->type == FHIP_Q4_K) return n_ff ? max_batch<Q4K, true>(w, left) : max_batch<Q4K, false>(w, left);
+    if (w->type == FHIP_Q6_K) return n_ff ? max_batch<Q6K, true>(w, left) : max_batch<Q6K, false>(w, left);
+    if (w->type == FHIP_Q5_K) return n_ff ? max_batch<Q5K, true>(w, left) : max_batch<Q5K, false>(w, left);
+    if (n_ff) return 0;
     switch (w->type) {
-        case FHIP_Q8_0: return max_batch<Q80, false>(w, 1) > 0;
-        case FHIP_Q4_0: return max_batch<Q40, false>(w, 1) > 0;
-        case FHIP_Q4_1: return max_batch<Q41, false>(w, 1) > 0;
-        case FHIP_Q5_0: return max_batch<Q50, false>(w, 1) > 0;
-        case FHIP_Q5_1: return max_batch<Q51, false>(w, 1) > 0;
-        case FHIP_IQ4_NL: return max_batch<IQ4NL, false>(w, 1) > 0;
-        case FHIP_IQ4_XS: return max_batch<IQ4XS, false>(w, 1) > 0;
-        case FHIP_MXFP4: return max_batch<MXF4S, false>(w, 1) > 0;
-        default: return false;
+        case FHIP_Q8_0: return max_batch<Q80, false>(w, left);
+        case FHIP_Q4_0: return max_batch<Q40, false>(w, left);
+        case FHIP_Q4_1: return max_batch<Q41, false>(w, left);
+        case FHIP_Q5_0: return max_batch<Q50, false>(w, left);
+        case FHIP_Q5_1: return max_batch<Q51, false>(w, left);
+        case FHIP_IQ4_NL: return max_batch<IQ4NL, false>(w, left);
+        case FHIP_IQ4_XS: return max_batch<IQ4XS, false>(w, left);
+        case FHIP_MXFP4: return max_batch<MXF4S, false>(w, left);
+        default: return 0;
     }
 }
+// Whether launch_gemv runs this weight on the streaming kernel (and not on the shape-complete f32 kernel, whose sums round
+// differently): the four-row and the sixteen-row mat-vec, which promise the streaming kernel's bits, take a weight only then.
+bool GEMV_EXPORT(gemv_streams)(const fhip_weight* w, size_t n_ff) { return GEMV_EXPORT(gemv_pass_rows)(w, 1, n_ff) > 0; }
 
 // One activation row with the input norm fused into its staging; NORM_NOT_FUSED (nothing launched) when this weight's
 // shape goes to the generic kernel or its row is longer than one pass of the workgroup.
