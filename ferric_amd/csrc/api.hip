@@ -112,7 +112,8 @@ size_t device_lds_bytes() { return g_lds; }
 // int8 matrix instruction (gemv_wide.hip: the same bits per row); what is left of a batch goes on as a batch of its own. Its cost is the quantiser's, per activation row and workgroup,
 // plus the weight once; the dot-product kernel's is a launch and the weight per pass, of one to four rows by how many of them its registers hold at that width. us, dot-product |
 // wide, each by itself and the weights in the Infinity Cache, three rows at 24 bits: IQ4_NL 1024 x 5120 7.4 | 9.0, 1024 x 16384 20.3 | 22.0, 2000 x 8192 16.6 | 12.2, 3000 x 5632
-// 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1). Four, of small weights: where the
+// 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1; Q5_0
+// 4124 x 5024 11.1 | 14.4, 2579 x 7296 11.6 | 13.5, 12677 x 1920 10.1 | 10.9: the dot-product kernel's up to 24 M weights). Four, of small weights: where the
 // dot-product kernel needs two passes for four rows this one is ahead, Q4_0 560 x 1792 9.2 | 6.4, Q5_0 260 x 3616 9.8 | 8.9, MXFP4 258 x 3520 10.7 | 7.8, at 16 bits IQ4_XS 1498 x 2048 8.6 | 5.6
 // (but Q5_0 412 x 14336 19.6 | 21.8); where it has them in one it is behind, Q5_0 793 x 928 5.3 | 6.2, 696 x 4896 8.9 | 10.7, Q5_1 898 x 512 4.9 | 5.1, IQ4_NL 410 x 4480 8.2 | 9.1, at 16 bits
 // MXFP4 399 x 4256 7.1 | 8.3, Q5_0 92 x 4416 6.9 | 9.4, but at 24 bits over 1024 .. 3072 columns, Q4_0 338 x 2336 7.3 | 6.7, Q4_1 1234 x 2208 7.5 | 6.9 (formats with a minimum a block from 1536 on:
@@ -134,7 +135,7 @@ bool takes_wide(const fhip_weight* w, size_t t) {
     if (w->type == FHIP_Q8_0 && t < 5 && w->cols <= 5120) return false;
     if (t < 3) return false;
     const bool q8 = w->type == FHIP_Q8_0, whole = w->planes == 3 && !q8;     // 24 bits
-    if (t == 3 && weights < ((size_t)(whole && w->cols <= 8192 ? 12 : 24) << 20)) return false;
+    if (t == 3 && weights < ((size_t)(whole && w->cols <= 8192 && w->type != FHIP_Q5_0 ? 12 : 24) << 20)) return false;
     if (t == 4 && weights < ((size_t)8 << 20) && (q8 || !wide_for_four(w, whole))) return false;
     return w->planes == 3 ? gemv_wide_supports_p3(w, t < 16 ? t : 16) : gemv_wide_supports_p2(w, t < 16 ? t : 16);
 }

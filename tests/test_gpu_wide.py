@@ -100,7 +100,7 @@ def test_the_rows_behind_the_last_sixteen_go_where_a_batch_of_them_would(F, ty, 
     (Q4_1, 50, 2080, 4, "WIDE", "DOT"), (Q5_0, 50, 2080, 4, "DOT", "DOT"), (Q4_0, 40, 3072, 4, "WIDE", "DOT"), (Q5_1, 326, 4896, 4, "DOT", "DOT"), (MXFP4, 399, 4256, 4, "DOT", "DOT"),
     (MXFP4, 30, 6656, 4, "DOT", "DOT"), (MXFP4, 300, 7168, 4, "WIDE", "DOT"), (Q5_0, 30, 7168, 4, "DOT", "DOT"), (IQ4_XS, 30, 1024, 4, "DOT", "DOT"), (IQ4_XS, 30, 4608, 4, "WIDE", "DOT"),
     (Q5_0, 20, 12288, 4, "WIDE", "DOT"), (Q5_0, 20, 12320, 4, "DOT", "DOT"), (Q5_0, 1728, 4864, 4, "WIDE", "WIDE"),
-    (IQ4_NL, 1600, 8192, 3, "WIDE", "DOT"), (IQ4_NL, 1500, 8192, 3, "DOT", "DOT"), (Q5_1, 1400, 9216, 3, "DOT", "DOT")])
+    (IQ4_NL, 1600, 8192, 3, "WIDE", "DOT"), (Q5_0, 1600, 8192, 3, "DOT", "DOT"), (IQ4_NL, 1500, 8192, 3, "DOT", "DOT"), (Q5_1, 1400, 9216, 3, "DOT", "DOT")])
 def test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16):
     from ferric_amd.synth import synth_weights
     qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
