@@ -1062,10 +1062,12 @@ void launch_attn_combine(const float* part, int n_head, int hd, int splits, floa
 // Before that, at that shape, us, values on f32 matrix instructions for six query heads and more, the dot-product kernel for fewer: 5 query
 // heads a KV head 38.3, 8: 33.9; head size 64, 4: 23.0. Error against f64 (2-norm, relative, eighteen shapes) no larger in any:
 // 2.2e-7 .. 2.5e-7 before, 1.4e-7 .. 1.8e-7 with the combine launch's present order.
-// Q4_1: codes less 7.5 (an addition each) and, in place of the minimum, what 7.5 stands for, which is next to nothing where a block's values lie evenly about
-// zero: then neither term takes bits from the other. A score begins with those times the sums of the query's dims, a value's sum ends with their weighted
-// sum. Against the dot-product kernel, 252 products, error against f64 (2-norm) 0.95 of that (codes less 8 0.97, and 1.04 on zero-mean rows; the minimum itself 1.02); us, that -> this, with the
-// combine launch: 8 query heads on each of 8 KV heads of 128, 14413 keys 35.7 -> 16.2, 5 on 8 at 32768 42.0 -> 24.4, 5 on 8 of 64 at 9000 15.8 -> 10.4, 3 on 4 of 64 at 5200 9.5 -> 8.4.
+// Q4_1: codes less the block's own code next to zero (an addition each) and, in place of the minimum, what that code stands for: at most half a step where the block has
+// values on both sides of zero, and of the values' sign where it has not, so that neither term takes bits from the other. A score begins with those times the sums of the
+// query's dims, a value's sum ends with their weighted sum. Error against f64 (2-norm) in that of the dot-product kernel, 120 products a kind of rows, geometric mean: about zero 0.95,
+// every channel off zero by thrice the spread 0.98, one in sixteen by 12 times in keys 0.82, in values 1.01 (one code for all blocks, 7.5: 0.95, 0.99, 1.20 and 1.06; by 60 times 0.77 and
+// 1.01, 1.57 and 1.10). us, the dot-product kernel -> this (less 7.5), with the combine launch: 8 query heads on each of 8 KV heads of 128, 14413 keys 34.8 -> 18.3 (17.3), 5 on 8 at 32768
+// 41.5 -> 26.3 (25.4), 5 on 8 of 64 at 9000 15.9 -> 10.5 (10.3), 3 on 4 of 64 at 5200 10.1 -> 9.1 (9.0).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct __attribute__((packed, aligned(8))) U4A8 { u32x4 v; };
@@ -1074,11 +1076,11 @@ union Frag { uint32_t w[4]; bf16x8 v; };
 // the upper halves of two f32: two bf16 (exact where the lower halves are zero)
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
 
-// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16. 4-bit formats: less 8 (Q4_1: 7.5), and a sixteenth (v_cvt_off_f32_i4 makes that of a two's complement nibble in one
+// Eight dims (8 g .. 8 g + 7 of a block of 32) of a key: its codes as bf16. 4-bit formats: less 8, and a sixteenth (Q4_1: `off` more) (v_cvt_off_f32_i4 makes that of a two's complement nibble in one
 // instruction, where the byte, its conversion and the 8 were three; the scales carry the 16, so every bit is the same). 128 x 8 KV heads of 5, 32768 keys, with the combine launch 23.1 -> 21.2 us,
 // 4 KV heads of 8 16.5 -> 15.6, heads of 64 16.4 -> 15.3: 804 -> 613 vector instructions a round beside its softmax.
 template <int FMT>
-__device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) {
+__device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift, float off) {
     Frag f;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -1089,7 +1091,7 @@ __device__ __forceinline__ bf16x8 codes_bf16(const uint32_t (&w)[2], int shift) 
         } else {
             const uint32_t x = (w[i] ^ 0x88888888u) >> shift;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_cvt_off_f32_i4((int)(j % 3 ? (x >> (8 * j)) & 255u : x >> (8 * j))) + (FMT == FHIP_KVQ_Q4_1 ? 0.03125f : 0.f);
+            for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_cvt_off_f32_i4((int)(j % 3 ? (x >> (8 * j)) & 255u : x >> (8 * j))) + (FMT == FHIP_KVQ_Q4_1 ? off : 0.f);
         }
         f.w[2 * i] = upper_halves(v[0], v[1]);
         f.w[2 * i + 1] = upper_halves(v[2], v[3]);
@@ -1109,13 +1111,13 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
     constexpr int LR = NB * CW / 4, KL = LONG_KEYS * LR / 64;           // lanes that request a row's key codes, 16 bytes each; requests of a round
     constexpr int KROW = 16 * LR + 16;                                  // bytes of a row in LDS: sixteen rows' same 8 bytes lie in different banks
     constexpr bool MIN = FMT == FHIP_KVQ_Q4_1;
-    constexpr float HALF = MIN ? 0.03125f : 0.f;                        // half a step, in sixteenths
     constexpr int SW = MIN ? NB : NB / 2;                               // words of a row's scales (Q4_1: scale and minimum a word)
     __shared__ float sm_m[LONG_WAVES][8], sm_l[LONG_WAVES][8];
     constexpr int COLS = SPL ? 16 : 8;
     __shared__ __attribute__((aligned(16))) float sm_acc[LONG_WAVES][COLS][HD + 4];    // rows four banks apart
     __shared__ __attribute__((aligned(16))) float sm_d[LONG_WAVES][NB][64];   // rows 0 .. 31 the keys' scales, 32 .. 63 the values'
-    __shared__ __attribute__((aligned(16))) float sm_min[MIN ? LONG_WAVES : 1][NB][64];   // MIN: what code 7.5 stands for, the minimum and as many steps
+    __shared__ __attribute__((aligned(16))) float sm_min[MIN ? LONG_WAVES : 1][NB][64];   // MIN: what the block's code next to zero stands for, ...
+    __shared__ __attribute__((aligned(16))) float sm_off[MIN ? LONG_WAVES : 1][NB][64];   // ... and 8 less that code, in sixteenths
     __shared__ float sm_qs[NB][16];                                     // MIN: the sum of block j's dims of column n's query
     __shared__ __attribute__((aligned(16))) uint8_t sm_k[LONG_WAVES][LONG_KEYS * KROW];   // a round's key codes, row by row
     __shared__ uint4 sm_q[NB][3][64];                                   // dims 32 j + 8 g .. + 7 of column n's query at lane n + 16 g, three bf16 each
@@ -1273,7 +1275,9 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             const float lo = __half2float(__ushort_as_half((uint16_t)R.sc[i])), hi = __half2float(__ushort_as_half((uint16_t)(R.sc[i] >> 16)));
             if constexpr (MIN) {
                 sm_d[wave][i][lane] = 16.0f * lo;
-                sm_min[wave][i][lane] = fmaf(7.5f, lo, hi);
+                const float zero = fminf(fmaxf(rintf(-hi * __builtin_amdgcn_rcpf(lo)), 0.f), 15.f);   // (any whole number does, the rest is exact for each)
+                sm_min[wave][i][lane] = fmaf(zero, lo, hi);
+                sm_off[wave][i][lane] = 0.0625f * (8.0f - zero);
             } else {
                 sm_d[wave][2 * i][lane] = Q8 ? lo : 16.0f * lo;         // (4-bit codes are sixteenths)
                 sm_d[wave][2 * i + 1][lane] = Q8 ? hi : 16.0f * hi;
@@ -1308,7 +1312,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
             for (int t = 0; t < NT; t++) {
                 const uint2 w = *(const uint2*)&sm_k[wave][(16 * t + n) * KROW + 4 * CW * j + 8 * (g & (CW / 2 - 1))];
                 const uint32_t kw[2] = {w.x, w.y};
-                const bf16x8 c = codes_bf16<FMT>(kw, 4 * (g >> 1));
+                const bf16x8 c = codes_bf16<FMT>(kw, 4 * (g >> 1), MIN ? sm_off[wave][j][16 * t + n] : 0.f);
                 f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int i = 2; i >= 0; i--) a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, qf[i].v, a, 0, 0, 0);
@@ -1376,6 +1380,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             float x[2 * 4];                     // probability times the block's scale, key 16 t + 4 g + r at 4 t + r
+            f32x4 off[NT];
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 const f32x4 d = *(const f32x4*)&sm_d[wave][j][32 + 16 * t + 4 * g];
@@ -1384,6 +1389,7 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                 if constexpr (MIN) {
                     const f32x4 least = *(const f32x4*)&sm_min[wave][j][32 + 16 * t + 4 * g];
                     floors[j] += fmaf(p[t][0], least[0], p[t][1] * least[1]) + fmaf(p[t][2], least[2], p[t][3] * least[3]);
+                    off[t] = *(const f32x4*)&sm_off[wave][j][32 + 16 * t + 4 * g];
                 }
             }
             if (j % 2 == 0)
@@ -1399,7 +1405,8 @@ __device__ __forceinline__ void attn_long_body(const float* __restrict__ q, cons
                     if constexpr (Q8) { lo = (float)(int8_t)(w >> (8 * i)); hi = (float)(int8_t)(w >> (16 + 8 * i)); }
                     else {
                         const uint32_t x = (w ^ 0x88888888u) >> (4 * i);
-                        lo = __builtin_amdgcn_cvt_off_f32_i4((int)x) + HALF; hi = __builtin_amdgcn_cvt_off_f32_i4((int)(x >> 16)) + HALF;
+                        lo = __builtin_amdgcn_cvt_off_f32_i4((int)x); hi = __builtin_amdgcn_cvt_off_f32_i4((int)(x >> 16));
+                        if constexpr (MIN) { lo += off[e >> 1][2 * (e & 1)]; hi += off[e >> 1][2 * (e & 1) + 1]; }
                     }
                     a[i].w[e] = upper_halves(lo, hi);
                 }

@@ -300,6 +300,33 @@ def test_long_caches_of_many_kv_heads_in_the_fewest_splits(F, Q, K, fmt, nkv, g,
     assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("nkv,g,n", [(171, 3, 700), (300, 3, 511), (171, 6, 257), (171, 8, 31)])
+def test_long_caches_of_many_kv_heads_of_blocks_with_a_minimum(F, Q, K, nkv, g, n):
+    test_long_caches_of_many_kv_heads_in_the_fewest_splits(F, Q, K, 2, nkv, g, n)
+
+
+@pytest.mark.parametrize("off,every", [(3.0, 1), (12.0, 16)])
+def test_blocks_with_a_minimum_whose_channels_lie_off_zero(F, Q, K, off, every):
+    """Q4_1 rows whose channels, all or one in sixteen, lie several times the spread off zero: there a block's minimum and its codes cancel, unless the codes are taken from the one
+    next to zero. At the bar above, and over all of it no further from f64 than attention over the dequantized rows."""
+    from types import SimpleNamespace
+    from ferric_amd import decode as X
+    from oracle import decode_oracle as D
+    rows, squares = 5200, np.zeros(2)
+    for nh, nkv, hd in ((3, 1, 64), (5, 1, 128), (8, 1, 128)):
+        for seed in range(6):
+            rng, width = np.random.default_rng(seed), nkv * hd
+            k, v = ((rng.standard_normal((rows, width)) + off * rng.standard_normal(width) * (rng.integers(0, every, width) == 0)).astype(np.float32) for _ in range(2))
+            q = (rng.standard_normal((1, nh * hd)) * (4.0 if seed % 2 else 1.0)).astype(np.float32)
+            kq, vq = (Q.QKvCache.from_tensor(F.Tensor.from_vec(x, x.shape), Q.Q4_1) for x in (k, v))
+            plain, qt = SimpleNamespace(k=kq.dequantize(), v=vq.dequantize(), cap=rows, width=width, len=rows), F.Tensor.from_vec(q, q.shape)
+            want = D.decode_attention(q[0], K.roundtrip(k, rows, width, Q.Q4_1), K.roundtrip(v, rows, width, Q.Q4_1), nh, nkv, 0, 0.0).reshape(-1)
+            errors = [t.to_vec().reshape(-1) - want for t in (X.decode_attention_kvq(qt, kq, vq, nh, nkv), X.decode_attention(qt, plain, nh, nkv))]
+            assert np.abs(errors[0]).max() <= 1e-5 * np.abs(want).max(), (nh, hd, seed)
+            squares += [(e.astype(np.float64) ** 2).sum() / (want.astype(np.float64) ** 2).sum() for e in errors]
+    assert squares[0] <= squares[1], np.sqrt(squares)
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("nkv,g,hd,n", [(8, 5, 128, 33), (8, 3, 64, 1), (5, 8, 128, 8340), (171, 3, 64, 514), (171, 5, 128, 514), (171, 8, 128, 258), (300, 6, 128, 31)])
 def test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, fmt, nkv, g, hd, n):
