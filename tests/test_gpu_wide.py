@@ -65,8 +65,8 @@ def test_more_waves_than_items(F, ty, rows, cols):
     x[3, -32:] = np.float32(1e30)
     one = singles_of(F, qm, x)
     xt = F.Tensor.from_vec(x, x.shape)
-    # (four rows of this few weights: at 24 bits where the dot-product kernel needs two passes; else they are its own, and it promises no row's bits beside the run of 1e30)
-    four = qm.matvec_precision(0) == 24 and ty in (Q4_1, IQ4_NL)
+    # (four rows of this few weights: at 24 bits, Q8_0 apart; else they are the dot-product kernel's, which promises no row's bits beside the run of 1e30)
+    four = qm.matvec_precision(0) == 24 and ty != Q8_0
     for m in (4, 5, 8, 9, 14, 16) if four else (5, 8, 9, 14, 16):
         assert route(F, qm, xt, m) == [(ROUTES["WIDE"], m)]
         assert same(F.Tensor.from_vec(x[:m], (m, cols)).matmul_q(qm).to_vec().reshape(m, rows), one[:m]), m
@@ -93,14 +93,8 @@ def test_the_rows_behind_the_last_sixteen_go_where_a_batch_of_them_would(F, ty, 
     assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
 
 
-# four rows: two passes of the dot-product kernel or one (1536 and 2048 columns | 1504, 2080, 4608), and the widths at which one pass is behind and ahead at 24 bits; three: the sizes from which on
-@pytest.mark.parametrize("ty,rows,cols,m,at24,at16", [
-    (Q4_0, 520, 1600, 4, "WIDE", "WIDE"), (MXFP4, 300, 2048, 4, "WIDE", "WIDE"), (Q5_0, 33, 3616, 4, "WIDE", "WIDE"), (Q5_1, 17, 6144, 4, "WIDE", "WIDE"), (Q5_1, 17, 7648, 4, "WIDE", "DOT"),
-    (MXFP4, 20, 352, 4, "DOT", "DOT"), (Q5_0, 793, 928, 4, "DOT", "DOT"), (IQ4_NL, 64, 1024, 4, "DOT", "DOT"), (IQ4_NL, 64, 1056, 4, "WIDE", "DOT"), (Q4_1, 50, 1536, 4, "DOT", "DOT"),
-    (Q4_1, 50, 2080, 4, "WIDE", "DOT"), (Q5_0, 50, 2080, 4, "DOT", "DOT"), (Q4_0, 40, 3072, 4, "WIDE", "DOT"), (Q5_1, 326, 4896, 4, "DOT", "DOT"), (MXFP4, 399, 4256, 4, "DOT", "DOT"),
-    (MXFP4, 30, 6656, 4, "DOT", "DOT"), (MXFP4, 300, 7168, 4, "WIDE", "DOT"), (Q5_0, 30, 7168, 4, "DOT", "DOT"), (IQ4_XS, 30, 1024, 4, "DOT", "DOT"), (IQ4_XS, 30, 4608, 4, "WIDE", "DOT"),
-    (Q5_0, 20, 12288, 4, "WIDE", "DOT"), (Q5_0, 20, 12320, 4, "DOT", "DOT"), (Q5_0, 1728, 4864, 4, "WIDE", "WIDE"),
-    (IQ4_NL, 1600, 8192, 3, "WIDE", "DOT"), (Q5_0, 1600, 8192, 3, "DOT", "DOT"), (IQ4_NL, 1500, 8192, 3, "DOT", "DOT"), (Q5_1, 1400, 9216, 3, "DOT", "DOT")])
+@pytest.mark.parametrize("ty,rows,cols,m,at24,at16", [(Q4_0, 520, 1600, 4, "WIDE", "WIDE"), (MXFP4, 20, 352, 4, "WIDE", "WIDE"), (MXFP4, 300, 7168, 4, "WIDE", "DOT"), (IQ4_NL, 1600, 8192, 3, "WIDE", "DOT"),
+                                                       (IQ4_NL, 1500, 8192, 3, "DOT", "DOT"), (Q5_1, 1400, 9216, 3, "DOT", "DOT")])
 def test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16):
     from ferric_amd.synth import synth_weights
     qm = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
@@ -112,6 +106,18 @@ def test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16):
     xt = F.Tensor.from_vec(x, x.shape)
     assert route(F, qm, xt, m) == [(ROUTES[kernel], m)]
     assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
+
+
+# four rows: up to 256 weight rows from a group of blocks on, two passes of the dot-product kernel or one (over 1568 .. 2048, 3104 .. 4096, 5152 .. 6144 columns, from 7200 on | else), long rows at 24 bits; three: Q5_0
+@pytest.mark.parametrize("ty,rows,cols,m,at24,at16", [
+    (Q4_0, 40, 480, 4, "DOT", "DOT"), (Q4_0, 256, 512, 4, "WIDE", "WIDE"), (Q4_0, 257, 512, 4, "DOT", "DOT"), (Q4_0, 40, 3072, 4, "WIDE", "WIDE"), (Q4_0, 257, 3072, 4, "WIDE", "DOT"),
+    (Q5_0, 256, 1536, 4, "WIDE", "WIDE"), (Q5_0, 257, 1536, 4, "DOT", "DOT"), (Q5_0, 50, 2080, 4, "DOT", "DOT"), (MXFP4, 20, 256, 4, "DOT", "DOT"), (MXFP4, 256, 288, 4, "WIDE", "WIDE"),
+    (MXFP4, 257, 288, 4, "DOT", "DOT"), (MXFP4, 300, 2048, 4, "WIDE", "WIDE"), (Q5_0, 33, 3616, 4, "WIDE", "WIDE"), (Q5_1, 17, 6144, 4, "WIDE", "WIDE"), (Q5_1, 17, 7648, 4, "WIDE", "DOT"),
+    (Q5_0, 793, 928, 4, "DOT", "DOT"), (IQ4_NL, 300, 1024, 4, "DOT", "DOT"), (IQ4_NL, 300, 1056, 4, "WIDE", "DOT"), (Q4_1, 300, 1536, 4, "DOT", "DOT"), (Q4_1, 300, 2080, 4, "WIDE", "DOT"),
+    (IQ4_XS, 300, 1024, 4, "DOT", "DOT"), (IQ4_XS, 30, 4608, 4, "WIDE", "DOT"), (Q5_1, 326, 4896, 4, "WIDE", "DOT"), (Q5_0, 326, 4896, 4, "DOT", "DOT"), (Q5_0, 20, 12288, 4, "WIDE", "DOT"),
+    (Q5_0, 20, 12320, 4, "DOT", "DOT"), (Q5_0, 1728, 4864, 4, "WIDE", "WIDE"), (Q5_0, 1600, 8192, 3, "DOT", "DOT")])
+def test_where_three_and_four_rows_of_small_weights_change_kernels(F, ty, rows, cols, m, at24, at16):
+    test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16)
 
 
 def test_mxfp4_blocks_that_may_overflow(F):
