@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from .qmatrix import DeviceBuffer, Graph, Tensor, _stream_handle, _upload
+from .qmatrix import Q4_K, Q5_K, Q6_K, Q8_0, DeviceBuffer, Graph, Tensor, _stream_handle, _upload
 
 
 def _check(rc):
@@ -243,9 +243,11 @@ class Qwen3Decoder:
         # a default-arm layer; short caches, whose attention splits nothing, need no combine launch behind it
         short = self.ws is None
         self.launches_per_layer = (7 if self.fuse_norm else 9) - (1 if self.fuse_attn else 0) - (1 if short else 0)
-        # per token beside the layers, at most: the head and the final norm, which takes the position word's increment with it and is inside the head's mat-vec but for
-        # a head of 128 MB and more (there a launch of its own costs less than the wider workgroups the fused norm needs)
-        self.launches_per_token_extra = (2 if self.fuse_norm else 3) if lm_head is not None else 1
+        # per token beside the layers: the head and the final norm, which takes the position word's increment with it and is inside the head's mat-vec but for formats without
+        # that and heads of 128 MB and more (a launch of its own costs less than the wider workgroups the fused norm needs). Without a head the last residual add takes the
+        # word; a head whose workgroups leave no CU free has one launch more for it.
+        inside = lm_head is not None and lm_head.ggml_type in (Q4_K, Q5_K, Q6_K, Q8_0) and lm_head.nbytes() < (128 << 20)
+        self.launches_per_token_extra = 1 if lm_head is None else 3 if not self.fuse_norm else 1 if inside else 2
         self._graph = None
 
     # -- state ------------------------------------------------------------------------------------

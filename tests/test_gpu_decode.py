@@ -497,6 +497,27 @@ def test_decoder_steps_match_the_oracle_layer_by_layer_and_replay_as_a_graph(F, 
     assert close(dec2.logits.to_vec(stream), D.rmsnorm(want[0], onorm, 1e-6) @ head.T, dot_bar(20))
 
 
+@pytest.mark.parametrize("head,fuse_norm", [(None, True), (Q6_K, True), (2, True), (Q6_K, False)])
+def test_the_launches_of_a_step_are_as_many_as_it_says(F, X, O, head, fuse_norm):
+    import ctypes as C
+    from ferric_amd.synth import synth_weights
+    d, n_layer, stream = 1024, 2, F.Stream()
+    layers, _ = _tiny_model(F, X, O, np.random.default_rng(3), n_layer, d, 8, 2, 128, 1536, True)
+    w = F.QMatrix.from_bytes(synth_weights(head, 300, d, 77), head, 300, d) if head is not None else None
+    dec = X.Qwen3Decoder(X.Qwen3Cfg(d, 8, 2, 128, 1536), layers, max_len=4, stream=stream, output_norm=F.Tensor.from_vec(np.ones(d, np.float32), (d,)) if head is not None else None,
+                         lm_head=w, fuse_norm=fuse_norm)
+    dec.set_input(np.ones(d, np.float32))
+    dec.step()
+    hip, graph, nodes = C.CDLL("libamdhip64.so.7"), C.c_void_p(), C.c_size_t()
+    stream.synchronize()
+    assert hip.hipStreamBeginCapture(stream.handle, 2) == 0
+    dec.step()
+    assert hip.hipStreamEndCapture(stream.handle, C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+    hip.hipGraphDestroy(graph)
+    assert nodes.value == n_layer * dec.launches_per_layer + dec.launches_per_token_extra
+
+
 # ---------------------------------------------------------------- the other arms of the layer (qwen3.rs:857-863, 917-938, 953-958, 1015-1020)
 
 def test_mul_sigmoid_and_geglu(F, X, D):
