@@ -379,6 +379,29 @@ def test_the_position_word_goes_along(F, ty, cols, resid):
     assert lib.fhip_add_count(x.buf.ptr, r.buf.ptr, 4, total.buf.ptr, None, 1, None) != 0
 
 
+# workgroups that take every CU (the word is a launch of its own); rows dealt in turn to all CUs, or to all but one, which has the word; short of that
+@pytest.mark.parametrize("ty", [Q4_K, 13, Q6_K, Q8_0])
+@pytest.mark.parametrize("rows", [255, 256, 512, 513, 4096, 66001])
+@pytest.mark.parametrize("resid", [False, True])
+def test_the_position_word_goes_along_with_full_launches(F, ty, rows, resid):
+    """Once, and beside the same bits."""
+    from ferric_amd.synth import synth_weights
+    lib, cols, rng = F._lib.load(), 768, np.random.default_rng(rows)
+    T = lambda a: F.Tensor.from_vec(a, a.shape)
+    x, r, nw = (T(rng.standard_normal(cols).astype(np.float32)) for _ in range(3))
+    w = F.QMatrix.from_bytes(synth_weights(ty, rows, cols, 3), ty, rows, cols)
+    word = T(np.array([5, 9], np.uint32).view(np.float32))
+    got = []
+    for count in (False, True):
+        y, xo, hs = (F.Tensor.empty((n,)) for n in (rows, cols, cols))
+        args = (w.handle, x.buf.ptr, r.buf.ptr if resid else None, nw.buf.ptr, 1e-6, xo.buf.ptr if resid else None, hs.buf.ptr, 0, y.buf.ptr)
+        F._lib.check(lib.fhip_norm_matmul_q_count(*args, word.buf.ptr, 3, None) if count else lib.fhip_norm_matmul_q(*args, None))
+        got.append([bits(t.to_vec()) for t in ((y, xo) if resid else (y,))])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    assert word.to_vec().view(np.uint32).tolist() == [8, 9]
+
+
 def test_norm_fused_into_the_matvec(F, X, D, O, precision):
     """fhip_norm_matmul_q against rmsnorm / add_rmsnorm followed by the mat-vec: the residual sum bit-exact, the product
     within the dot-product bound of the unfused pair (the sum of squares is added in another order: ~1e-7 on the scale),

@@ -359,6 +359,12 @@ def test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, fmt, nkv, g, hd, n
     assert np.abs(got[1][0] - want).max() <= 1e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("nkv,g,hd,n", [(8, 5, 128, 33), (8, 3, 64, 1), (5, 8, 128, 8340), (171, 3, 64, 514), (171, 8, 128, 258)])
+def test_the_token_s_row_of_blocks_with_a_minimum(F, Q, K, nkv, g, hd, n):
+    test_the_token_s_row_at_the_edges_of_long_caches(F, Q, K, 2, nkv, g, hd, n)
+
+
+
 @pytest.mark.parametrize("nkv,g,hd,n", [(8, 5, 128, 33), (8, 3, 64, 1), (5, 8, 128, 8340), (171, 8, 128, 258), (300, 6, 128, 31)])
 def test_the_token_s_row_of_blocks_with_a_minimum(F, Q, K, nkv, g, hd, n):
     """The same on a Q4_1 cache, fused and not."""
