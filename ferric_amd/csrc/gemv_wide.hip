@@ -263,7 +263,7 @@ __global__ void __launch_bounds__((64 * max_waves<F, E>())) gemv_wide_kernel(Wid
     const int tid = threadIdx.x, lane = tid & 63, W = (int)(blockDim.x >> 6);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g4 = lane >> 4, c = lane & 15;
-    {                                                     // the workgroup's activation rows
+    if constexpr (E < 4) {                                // the workgroup's activation rows (of more than eight a workgroup has all: these lines cost it 0.4 us)
         const int first = (int)blockIdx.y * p.R;
         p.T = p.T - first < p.R ? p.T - first : p.R;
         p.x += (size_t)first * p.cols;
@@ -551,6 +551,7 @@ size_t lds_of(int E, int P, int tiles, int passes, int W, int image, WideParams*
 // How a launch of t rows is laid out with R of them a workgroup.
 struct WidePlan { int R, E, tiles, P, passes, W; unsigned grid, row_groups; };
 constexpr int pairs_of(int R) { return R <= 4 ? 1 : R <= 8 ? 2 : 4; }
+static_assert(pairs_of((16 + 1) / 2) < 4, "four pairs a lane: one workgroup has all rows of a launch");
 WidePlan wide_plan(int rows, int NG, int t, int R, int image, bool big, int cus, size_t lds_max) {
     WidePlan q;
     q.R = R; q.E = pairs_of(R);
@@ -575,8 +576,10 @@ WidePlan wide_plan(int rows, int NG, int t, int R, int image, bool big, int cus,
     // More waves than items, as many as there may be, where each has two pieces to quantise and their images fit: the quantiser is what a workgroup of few tiles
     // does longest. us, a wave an item | all: Q5_1 993 x 4320 at 8 rows 13.6 | 12.1, Q4_0 1458 x 17248 at 7 41.8 | 37.2, 1312 x 13280 at 14 33.1 | 29.4. With
     // fewer pieces the barriers of more waves cost as much (IQ4_XS 1029 x 1792 at 4 rows 5.5 | 6.1), and where the images take a pass's room it has more of
-    // them (Q5_1 949 x 2368 at 10 rows 12.6 | 15.7).
-    if (q.W < most && R * q.P >= 2 * q.W && lds_of(q.E, q.P, q.tiles, q.passes, most, image, nullptr) <= lds_max) q.W = most;
+    // them (Q5_1 949 x 2368 at 10 rows 12.6 | 15.7). Not for Q8_0, whose images are twice as large, at more than eight rows: 9238 x 512 at 16 7.9 | 8.7, 4914 x 1120 at 11 11.6 | 12.4; of 501
+    // products 20 were longer by more than 3 %.
+    const bool large = image > 2048 && q.E == 4;
+    if (!large && q.W < most && R * q.P >= 2 * q.W && lds_of(q.E, q.P, q.tiles, q.passes, most, image, nullptr) <= lds_max) q.W = most;
     return q;
 }
 

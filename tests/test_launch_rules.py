@@ -55,6 +55,34 @@ def test_when_a_norm_requests_its_weights_with_the_row(decode):
         assert bool(decode.h_norm_ahead(C.c_size_t(grid))) == (with_row < behind), grid
 
 
+@pytest.fixture(scope="module")
+def wide(tmp_path_factory):
+    c = C.CDLL(build(tmp_path_factory.mktemp("wide"), "wide_rules_harness.cpp", ["-DFHIP_GEMV_PLANES=3"], ["-shared", "-Wl,-Bsymbolic"]))
+
+    def ask(ty, rows, cols, t, each):
+        out = (C.c_int64 * 7)()
+        c.h_wide_plan(C.c_uint32(ty), *(C.c_size_t(n) for n in (rows, cols, t, each)), out)
+        return tuple(out)
+    return ask
+
+
+def test_more_waves_than_items_of_a_batch_where_they_were_the_faster(wide):
+    """Q8_0 at more than eight rows keeps a wave an item, eight at least: us with those | with all waves."""
+    q5_0 = 6
+    for ty, rows, cols, t, few, all_waves in ((Q8_0, 9238, 512, 16, 7.9, 8.7), (Q8_0, 4914, 1120, 11, 11.6, 12.4), (Q8_0, 7482, 1088, 11, 11.7, 12.4), (q5_0, 1458, 17248, 7, 41.8, 37.2),
+                                              (q5_0, 1312, 13280, 14, 33.1, 29.4)):
+        pairs, tiles, groups, _, waves, _, _ = wide(ty, rows, cols, t, t)
+        assert (waves > max(8, tiles * groups)) == (all_waves < few), (ty, rows, cols, t)
+
+
+def test_four_pairs_a_lane_are_one_workgroup_s_only(wide):
+    """The kernel of four pairs does not look for rows of its own: whatever a batch is dealt out to, it never shares one."""
+    for t in range(1, 17):
+        for shares in range(1, min(t, 4) + 1):
+            pairs, *_, n = wide(Q8_0, 5000, 2048, t, -(-t // shares))
+            assert n <= shares and n * 4 * pairs >= t and (pairs < 4 or n == 1), (t, shares)
+
+
 @pytest.mark.parametrize("width", [64, 256])      # columns of a step (unpacked weights shared) and of a chunk (waves that unpack for themselves)
 def test_no_activation_is_read_from_behind_the_last(gemm, width):
     """Threads stage 16-byte pieces of whole steps or chunks of columns: rows and columns that do not exist are read from x all the same, those that do from where they are."""
