@@ -113,24 +113,33 @@ size_t device_lds_bytes() { return g_lds; }
 // plus the weight once; the dot-product kernel's is a launch and the weight per pass, of one to four rows by how many of them its registers hold at that width. us, dot-product |
 // wide, each by itself and the weights in the Infinity Cache, three rows at 24 bits: IQ4_NL 1024 x 5120 7.4 | 9.0, 1024 x 16384 20.3 | 22.0, 2000 x 8192 16.6 | 12.2, 3000 x 5632
 // 10.7 | 9.5, 4096 x 4096 8.7 | 8.3, 8000 x 1600 7.7 | 7.1, 12000 x 1600 10.1 | 8.2 (at 16 bits 2048 x 8192 9.1 | 11.3, 9000 x 2048 7.8 | 8.1; Q5_0
-// 4124 x 5024 11.1 | 14.4, 2579 x 7296 11.6 | 13.5, 12677 x 1920 10.1 | 10.9: the dot-product kernel's up to 24 M weights). Four, of small weights: up to 256 rows are one a CU or
-// none, and the dot-product kernel is behind by 0.7 .. 0.95 from a whole group of blocks to 3072 columns (Q5_0, whose fifth bits cost the quantiser's kernel more, to 1536), at both precisions; beyond, where it needs
-// two passes for four rows, Q4_0 560 x 1792 9.2 | 6.4, Q5_0 260 x 3616 9.8 | 8.9, MXFP4 258 x 3520 10.7 | 7.8, at 16 bits IQ4_XS 1498 x 2048 8.6 | 5.6
-// (but Q5_0 412 x 14336 19.6 | 21.8). Where it has them in one it is ahead at 16 bits, MXFP4 399 x 4256 7.1 | 8.3, and of Q5_0, 793 x 928 5.3 | 6.2, 696 x 4896 8.9 | 10.7; at 24 bits of
-// short rows, Q4_0 900 x 352 4.5 | 5.1 (formats with a minimum a block to 1536 columns: Q5_1 842 x 1376 5.6 | 6.2), and behind by 0.93 over the longer ones (Q4_0 1024 x 7168 11.1 | 9.5, but IQ4_NL 428 x
-// 4352 7.9 | 8.4). MXFP4 of up to 256 rows and less than a group is level at 24 bits (20 x 352 5.07 | 5.01), behind at 16 (4.40 | 4.78). Over 3640 drawn products of four rows and up to 8 M weights, both
-// precisions, 0.87 of the dot-product kernel's time, 29 of them longer by more than 3 %, at most 1.09 times (this kernel for all of them 0.87, and 871 longer, up to 1.41 times; the better of both each time 0.85).
+// 4124 x 5024 11.1 | 14.4, 2579 x 7296 11.6 | 13.5, 12677 x 1920 10.1 | 10.9: the dot-product kernel's up to 24 M weights). Four, of small weights, ahead is: this kernel
+// over a whole number of its groups of 512 columns, Q5_0 2706 x 1536 6.8 | 5.6, Q4_0 1432 x 1024 at 16 bits 4.9 | 4.3; with two passes of the dot-product kernel, Q4_0 560 x 1792 9.2 | 6.4,
+// MXFP4 258 x 3520 10.7 | 7.8, IQ4_XS 1498 x 2048 at 16 bits 8.6 | 5.6 (but Q5_0, whose fifth bits cost this one's items more, 412 x 14336 19.6 | 21.8); with one pass of it, up to 256 rows, which leave its CUs a row each
+// or none, 0.7 .. 0.95, and from 4097 on, where a CU has its second tile, 0.83 .. 1.0 (Q5_0 at 16 bits 1.03); between these at 24 bits, IQ4_NL 300 x 1056 0.84, Q4_0 1024 x 7168 11.1 | 9.5, and at 16 over 1568 .. 3072 columns, 0.95. The
+// dot-product kernel is: of Q5_0, 793 x 928 5.3 | 6.2, 696 x 4896 8.9 | 10.7; of 513 .. 1024 rows to 1536 columns, 842 x 1376 Q5_1 5.6 | 6.2; of formats with a minimum a block to 1024, 900 x 800 1.08; at 16 bits to 1536, MXFP4 1.03, and over
+// the longer rows, MXFP4 399 x 4256 7.1 | 8.3; and of rows short of a group, Q4_0 900 x 352 4.5 | 5.1, unless very many, 26545 x 288 at 24 bits 0.83 (MXFP4 of up to 256 is level at 24 bits, 20 x 352 5.07 | 5.01,
+// and behind at 16, 4.40 | 4.78). Over 3640 drawn products, both precisions, 0.88 of the dot-product kernel's time, 46 of them longer by more than 3 %, at most 1.08 times (this kernel for all of them 0.89, and 927
+// longer, up to 1.42 times; the better of both each time 0.865).
 // At 16 bits and more than 6144 columns two passes
 // are ahead too: 1024 x 7168 9.2 | 10.3, 500 x 16000 15.6 | 17.4. Cold: Q4_0 34816 x 5120 at four rows 42.3 | 32.6, at five 62.9 | 38.9; sixteen: IQ4_NL 1467 x 1760 37.1 | 12.1, Q4_0
 // 34816 x 5120 169 | 64. Q8_0 has the others at three and four rows of up to 5120 columns: three, dot-product |
 // wide, 4096 x 4096 9.6 | 10.7; four, four-row | wide, 34816 x 5120 48.4 | 57.5, 5120 x 5120 15.1 | 17.5, 2048 x 4096 10.1 | 10.8 (but 4096 x 4096 12.5 | 11.0, 12288 x 4096 22.8 | 19.6).
 static bool wide_for_four(const fhip_weight* w, bool whole) {      // of up to 8 M weights
+    const size_t rows = w->rows, cols = w->cols;
     const bool q5 = w->type == FHIP_Q5_0;
-    if (w->rows <= 256 && ((w->cols >= 512 && w->cols <= (q5 ? 1536 : 3072)) || (w->type == FHIP_MXFP4 && w->cols > 256 && w->cols < 512))) return true;
+    if (cols < 512) return cols >= 256 && (rows > 20480 || (whole && !q5 && rows > 10240) || (w->type == FHIP_MXFP4 && cols > 256 && rows <= 256));
+    if (cols % 512 == 0 && cols <= 3072) return true;
     const bool one_pass = (w->planes == 3 ? gemv_pass_rows_p3(w, 4, 0) : gemv_pass_rows_p2(w, 4, 0)) == 4;
-    if (!whole) return w->cols <= 6144 && !one_pass;
-    if (q5) return w->cols <= 12288 && !one_pass;
-    return !one_pass || w->cols > (w->type == FHIP_Q4_1 || w->type == FHIP_Q5_1 ? 1536 : 1024);
+    if (one_pass && cols <= 3072) {
+        if (rows <= 256) return !q5 || cols <= 1536;
+        if (rows > 4096) return whole || !q5;
+        if (q5) return whole && cols > 1536 && rows > 1536;
+        if (rows > 512 && rows <= 1024 && cols <= 1536) return false;
+        return cols > 1536 || w->type == FHIP_IQ4_XS || (whole && (cols > 1024 || (w->type != FHIP_Q4_1 && w->type != FHIP_Q5_1)));
+    }
+    if (!whole) return cols <= 6144 && !one_pass;
+    return !q5 || (cols <= 12288 && !one_pass);
 }
 bool takes_wide(const fhip_weight* w, size_t t) {
     const size_t weights = w->rows * w->cols;

@@ -108,14 +108,16 @@ def test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16):
     assert same(xt.matmul_q(qm).to_vec().reshape(m, rows), singles_of(F, qm, x))
 
 
-# four rows: up to 256 weight rows from a group of blocks on, two passes of the dot-product kernel or one (over 1568 .. 2048, 3104 .. 4096, 5152 .. 6144 columns, from 7200 on | else), long rows at 24 bits; three: Q5_0
+# four rows: short of a group; whole groups; one pass of the dot-product kernel by rows and columns; two (over 1568 .. 2048, 3104 .. 4096, 5152 .. 6144 columns, from 7200 on); three: Q5_0
 @pytest.mark.parametrize("ty,rows,cols,m,at24,at16", [
-    (Q4_0, 40, 480, 4, "DOT", "DOT"), (Q4_0, 256, 512, 4, "WIDE", "WIDE"), (Q4_0, 257, 512, 4, "DOT", "DOT"), (Q4_0, 40, 3072, 4, "WIDE", "WIDE"), (Q4_0, 257, 3072, 4, "WIDE", "DOT"),
-    (Q5_0, 256, 1536, 4, "WIDE", "WIDE"), (Q5_0, 257, 1536, 4, "DOT", "DOT"), (Q5_0, 50, 2080, 4, "DOT", "DOT"), (MXFP4, 20, 256, 4, "DOT", "DOT"), (MXFP4, 256, 288, 4, "WIDE", "WIDE"),
-    (MXFP4, 257, 288, 4, "DOT", "DOT"), (MXFP4, 300, 2048, 4, "WIDE", "WIDE"), (Q5_0, 33, 3616, 4, "WIDE", "WIDE"), (Q5_1, 17, 6144, 4, "WIDE", "WIDE"), (Q5_1, 17, 7648, 4, "WIDE", "DOT"),
-    (Q5_0, 793, 928, 4, "DOT", "DOT"), (IQ4_NL, 300, 1024, 4, "DOT", "DOT"), (IQ4_NL, 300, 1056, 4, "WIDE", "DOT"), (Q4_1, 300, 1536, 4, "DOT", "DOT"), (Q4_1, 300, 2080, 4, "WIDE", "DOT"),
-    (IQ4_XS, 300, 1024, 4, "DOT", "DOT"), (IQ4_XS, 30, 4608, 4, "WIDE", "DOT"), (Q5_1, 326, 4896, 4, "WIDE", "DOT"), (Q5_0, 326, 4896, 4, "DOT", "DOT"), (Q5_0, 20, 12288, 4, "WIDE", "DOT"),
-    (Q5_0, 20, 12320, 4, "DOT", "DOT"), (Q5_0, 1728, 4864, 4, "WIDE", "WIDE"), (Q5_0, 1600, 8192, 3, "DOT", "DOT")])
+    (Q4_0, 40, 480, 4, "DOT", "DOT"), (MXFP4, 20, 256, 4, "DOT", "DOT"), (MXFP4, 256, 288, 4, "WIDE", "WIDE"), (MXFP4, 257, 288, 4, "DOT", "DOT"), (Q4_0, 10241, 256, 4, "WIDE", "DOT"),
+    (Q4_0, 10240, 256, 4, "DOT", "DOT"), (Q5_0, 20481, 288, 4, "WIDE", "WIDE"), (Q5_0, 20480, 288, 4, "DOT", "DOT"), (Q5_0, 700, 512, 4, "WIDE", "WIDE"), (Q5_0, 600, 3072, 4, "WIDE", "WIDE"),
+    (Q4_0, 256, 544, 4, "WIDE", "WIDE"), (Q4_0, 257, 544, 4, "WIDE", "DOT"), (Q5_1, 257, 544, 4, "DOT", "DOT"), (Q5_1, 257, 1056, 4, "WIDE", "DOT"), (IQ4_XS, 300, 768, 4, "WIDE", "WIDE"),
+    (IQ4_XS, 513, 768, 4, "DOT", "DOT"), (IQ4_NL, 1024, 1056, 4, "DOT", "DOT"), (IQ4_NL, 1025, 1056, 4, "WIDE", "DOT"), (Q4_1, 4097, 544, 4, "WIDE", "WIDE"), (Q5_0, 4097, 544, 4, "WIDE", "DOT"),
+    (Q5_0, 4096, 544, 4, "DOT", "DOT"), (Q4_1, 600, 2080, 4, "WIDE", "WIDE"), (Q5_0, 256, 1504, 4, "WIDE", "WIDE"), (Q5_0, 50, 2080, 4, "DOT", "DOT"), (Q5_0, 1537, 2080, 4, "WIDE", "DOT"),
+    (MXFP4, 300, 2048, 4, "WIDE", "WIDE"), (Q5_0, 33, 3616, 4, "WIDE", "WIDE"), (Q5_1, 17, 6144, 4, "WIDE", "WIDE"), (Q5_1, 17, 7648, 4, "WIDE", "DOT"), (IQ4_XS, 30, 4608, 4, "WIDE", "DOT"),
+    (Q5_1, 326, 4896, 4, "WIDE", "DOT"), (Q5_0, 326, 4896, 4, "DOT", "DOT"), (Q5_0, 20, 12288, 4, "WIDE", "DOT"), (Q5_0, 20, 12320, 4, "DOT", "DOT"), (Q5_0, 1728, 4864, 4, "WIDE", "WIDE"),
+    (Q5_0, 1600, 8192, 3, "DOT", "DOT")])
 def test_where_three_and_four_rows_of_small_weights_change_kernels(F, ty, rows, cols, m, at24, at16):
     test_three_and_four_rows_of_small_weights(F, ty, rows, cols, m, at24, at16)
 
