@@ -616,8 +616,8 @@ int launch_wide(const fhip_weight* w, const float* d_x, size_t t, const WidePlan
 // tiles too few for the CUs meet more of these, for the weight once more a group. Dealt out where the estimate is 8 % under that of one group. us, one | two | three |
 // four groups, 24 bits: IQ4_XS 1636 x 13824 at 16 rows 55.2 | 32.7 | 31.6 | 25.0, MXFP4 1145 x 8160 at 8 20.3 | 13.7 | 13.2 | 16.2, 5433 x 14048 at 16 78.8 | 54.5 | 57.4 | 60.0,
 // Q4_0 918 x 3680 at 5 9.6 | 8.2 | 7.7 | 7.7; not: Q4_1 29831 x 2688 at 16 41.0 | 45.6 | 60.7 | 56.2, MXFP4 22048 x 2592 at 7 (16 bits) 19.2 | 22.2 | 34.6 | 39.6. Over
-// 1173 products of 3 .. 16 rows 0.83 of the time of one group with a wave an item (or of the dot-product kernel, where that had them), ten 3 .. 10 % slower; over 633 of them 0.80, and
-// the best of all layouts would give 0.78. (At 5 % and a wave an item these 633 take 0.80 too, but seventeen are 3 .. 15 % slower: Q4_0 2057 x 4096 at four rows 8.4 -> 9.9, whose 129
+// 1000 products of 3 .. 16 rows 0.77 of the time of one group with a wave an item (or of the dot-product kernel, where that had them), seven 3 .. 14 % slower, most where half the
+// CUs for a group make two tiles of one (IQ4_XS 2642 x 15872 at 5 rows and 16 bits 20.2 | 24.0); the best of all layouts would give 0.98 of that. (At 5 % and a wave an item as good on average, but more are slower: Q4_0 2057 x 4096 at four rows 8.4 -> 9.9, whose 129
 // tiles are one more than half the CUs.)
 template <class F>
 int launch_wide_fmt(const fhip_weight* w, const float* d_x, size_t t, float* d_y, hipStream_t s) {

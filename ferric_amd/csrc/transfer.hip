@@ -474,9 +474,8 @@ static int upload_chunks(Ring* r, uint8_t* d, const uint8_t* h, size_t n, hipStr
     return rc;
 }
 
-// Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime (10 MB in 285 us;
-// chunks of it copied into slots by workers and pulled over the bus by kernels took 300 - 360), and it returns when the source has
-// been read or is known to be pinned. A copy in a stream capture stays a copy node; on another stream than the captured one it goes
+// Up to a slot's IN_BYTES: the source has been copied when the call returns. Longer sources go through the runtime, which returns when the source has
+// been read or is known to be pinned (upload(), which may wait, sends those of up to IN_CHUNKS_TO through slots). A copy in a stream capture stays a copy node; on another stream than the captured one it goes
 // through the runtime too, since a slot may have to be made.
 int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     int rc;
@@ -493,7 +492,7 @@ int copy_h2d(void* d, const void* h, size_t n, hipStream_t s) {
     memcpy(q->host, h, n);
     int wgs = 0;
     // One unit a thread while there are workgroups for it: a thread that has three makes three trips over the bus, one after the other. With the wait behind it, us, four units
-    // a thread | one: 20 KB 17.8 | 15.8, 64 KB 18.1 | 17.1, 192 KB 21.6 | 20.7, 426 KB 31.2 | 29.3, 593 KB 37.3 | 37.0.
+    // a thread | one: 20 KB 17.8 | 15.8, 64 KB 18.1 | 17.1, 192 KB 21.6 | 20.7, 426 KB 31.2 | 29.3, 608 KB 34.3 | 35.4.
     if (!(rc = launch_copy(q->host, d, n, 1, q->done, q->seq + 1, s, &wgs))) { q->seq++; q->wgs = wgs; }
     r->release(q);
     return rc;
